@@ -124,6 +124,16 @@ void fill_linear_args(mi355_linear_args& a, const mi355_model* m, const mi355_we
     a.ldy = ldy;
 }
 
+// Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per 5-13 rows.  BF16: eight layers of a 7B
+// model, 10 rows 1139 us (rows) / 1159 us (tiled), 12 rows 1181 / 1162, 24 rows 2172 / 1223.  int4: 31 rows 1906 / 737 us, but its sums of
+// (128 + level) x run over a whole K-slice in one accumulator, where the row kernel's eight waves sum a part each: with single activations 10^4 times the
+// others (the full-depth fixture with a trained model's statistics) that took the logits from 0.05 to 0.08 of their spread, so short chunks stay there.
+int wide_rows(const mi355_weight& w) {
+#ifdef MI355_GEMM_SWEEP
+    if (const char* e = getenv("MI355_WIDE_ROWS")) return atoi(e);
+#endif
+    return w.fmt == MI355_W_BF16 ? 11 : 32;
+}
 bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: int4 / bf16 stream, one scale per row
     return (w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && (w.group_cols == 0 || w.group_cols >= w.K) && w.N % 4 == 0 &&
            w.K % 128 == 0;
@@ -132,7 +142,7 @@ bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: i
 FuseCtx plan_fusion(const mi355_model* m, int T) {
     FuseCtx z;
     memset(&z, 0, sizeof(z));
-    if (T < 32) return z;  // (decode steps and short chunks: the streaming kernels, nothing to plan)
+    if (m->n_layer < 1 || T < 32) return z;  // (shorter chunks keep the row attention, f32 queries and weights; their products may still be tiled: wide_rows)
     // (read once per mi355_forward call, here, and nowhere on the launch path: the plan this returns is what every launch of the
     // call follows; tests/test_prefill_gpu.py toggles the variable between two calls of one process)
     const char* env = getenv("MI355_GEMM_FUSE");
@@ -147,6 +157,8 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
         if (L.attn.N != 3 * C || L.attn.K != C || L.proj.N != C || L.proj.K != C || L.fc.N != H || L.fc.K != C || L.fc.R != 2 ||
             L.mproj.N != C || L.mproj.K != H || L.kcache == nullptr || L.vcache == nullptr)
             return z;
+        // (one plan for all layers: it depends on the format)
+        if (L.proj.fmt != m->layers[0].proj.fmt || L.fc.fmt != m->layers[0].fc.fmt || L.mproj.fmt != m->layers[0].mproj.fmt) return z;
     }
     if (C % 128 != 0 || H % 128 != 0) return z;
     int ks, n, ppu;
@@ -157,8 +169,8 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
     if ((size_t)m->gemm_ws_bytes < mi355_linear_gemm_workspace_bytes(T, kmax)) return z;
     float* cur = (float*)((char*)m->gemm_ws + (((size_t)m->gemm_ws_bytes - tail) & ~(size_t)15));
     float* const end = (float*)((char*)m->gemm_ws + (size_t)m->gemm_ws_bytes);
-    auto edge = [&](FuseEdge& e, int N, int K, int R, bool with_ss) {
-        mi355_linear_gemm_plan(T, N, K, R, &ks, &n, &ppu);
+    auto edge = [&](FuseEdge& e, const mi355_weight& w, bool with_ss) {
+        mi355_linear_gemm_plan(T, w.N, w.K, w.R, w.fmt == MI355_W_BF16, &ks, &n, &ppu);
         e.n = n;
         e.ppu = ppu;
         e.sx = cur;
@@ -166,9 +178,9 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
         e.ss = with_ss ? cur : nullptr;
         if (with_ss) cur += (size_t)n * Ts;
     };
-    edge(z.proj, C, C, 1, true);
-    edge(z.mproj, C, H, 1, true);
-    edge(z.fc, H, C, 2, false);
+    edge(z.proj, m->layers[0].proj, true);
+    edge(z.mproj, m->layers[0].mproj, true);
+    edge(z.fc, m->layers[0].fc, false);
     z.att.n = m->n_head;
     z.att.ppu = 1;
     z.att.sx = cur;
@@ -186,9 +198,8 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
 int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x_dtype, int M, int64_t ldx,
                const void* norm_scale, int epi, void* y, int y_dtype, int64_t ldy, hipStream_t s,
                const float* attn_partials = nullptr) {
-    // wide inputs (prompt chunks of >= 32 tokens) of an int4 model: the LDS-tiled MFMA GEMM over the same stream
-    // (per-row or grouped scales)
-    if ((w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && M >= 32 && m->gemm_ws != nullptr &&
+    // wide inputs of an int4 or bf16 model: the LDS-tiled MFMA GEMM over the same stream (per-row or grouped scales)
+    if ((w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && M >= wide_rows(w) && m->gemm_ws != nullptr &&
         attn_partials == nullptr && w.N % 4 == 0 && ldy % 4 == 0 && (w.group_cols == 0 || w.K % 128 == 0)) {
         mi355_linear_args a;
         fill_linear_args(a, m, w, x, x_dtype, M, ldx, norm_scale, epi, y, y_dtype, ldy);

@@ -70,32 +70,15 @@ constexpr int kTPW = MI355_GEMM_TPW;
 #ifndef MI355_GEMM_PIN_W
 #define MI355_GEMM_PIN_W 0
 #endif
-#ifndef MI355_GEMM_BF16_REFILL
-#define MI355_GEMM_BF16_REFILL 1
-#endif
 #ifndef MI355_GEMM_BF16_ROWMAJOR
 // workgroup order of the BF16 streams: row block major (an XCD runs every token block of a few row blocks side by side).  Token block major
 // (the int4 order) carried every weight piece across the fabric once per token block: 16 x 13.5 GB = 216 GB per 2048-token pass of the 7B
 // model, 6.3 TB/s of its 34 ms.  2048 tokens 34.0 -> 28.5 ms, 512 tokens 16.5 -> 10.6 ms (profiles/r06_ab_bf16_block_order.txt)
 #define MI355_GEMM_BF16_ROWMAJOR 1
 #endif
-#ifndef MI355_GEMM_ONE_PER_CU
-#define MI355_GEMM_ONE_PER_CU 1
-#endif
 #ifndef MI355_GEMM_Q4_ROWMAJOR
 #define MI355_GEMM_Q4_ROWMAJOR 0
 #endif
-#ifndef MI355_GEMM_BF16_OCC
-// 1 held the BF16-stream kernels at 128 VGPRs (two workgroups per CU) since round 3 — with 100-112 bytes of scratch per lane in the 128-token
-// blocks, inside the unit loop.  Round 6 measured it: a 2048-token prompt of the bf16 7B model 69.3 ms with it, 37.5 ms without (130-136 VGPRs,
-// one workgroup per CU, no scratch); 64-token blocks (118 VGPRs either way) and prompts up to 512 tokens are unchanged
-// (profiles/r06_prefill_bf16_occupancy.txt).
-#define MI355_GEMM_BF16_OCC 0
-#endif  // 16-row tile slots per wave: one B fragment read from LDS feeds kTPW MFMAs
-// Waves per workgroup: 8 (a block = 16 row tiles x 128 tokens) for prompts that fill the chip; 2 (4 row tiles) when the
-// launch would otherwise be a few dozen workgroups — a 128-token prompt of a 7B model is ONE token block, i.e. 16 workgroups
-// for attn.c_proj / mlp.c_proj (N = 4096) on 256 CUs, each streaming its 0.5-1.4 MB of weights alone: ~96 us per launch.
-
 struct GemmParams {
     const uint8_t* w;
     unsigned w_bytes;
@@ -148,8 +131,7 @@ struct GemmParams {
 
 // c_attn's q rows as the prompt attention multiplies them (flash_prefill.hip's own prologue, moved to the producer: the same f32
 // arithmetic and the one rounding, so the same bits): four outputs = two interleaved pairs at row m, column n < C
-__device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n, int posm, float o0, float o1, float o2, float o3) {
-    const f32x4 cs = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : posm) * 128 + (n & 127));
+__device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n, const f32x4& cs, float o0, float o1, float o2, float o3) {
     const float qs = p.q_scale;
     typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
     const bf2 a = {(__bf16)(qs * (o0 * cs[0] - o1 * cs[1])), (__bf16)(qs * (o1 * cs[0] + o0 * cs[1]))};
@@ -161,7 +143,8 @@ __device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n,
 }
 
 constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials a workspace holds
-constexpr int kMaxSplit = 8;
+constexpr int kMaxSplit = 16;
+constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
 __host__ __device__ __forceinline__ int slice_lo(int s, int units, int ksplit) { return (int)((int64_t)s * units / ksplit); }
@@ -175,6 +158,13 @@ __device__ __forceinline__ int swz(int tok) { return (tok & 3) ^ (((tok >> 2) & 
 
 __device__ __forceinline__ float ldsz(const void* p, int i, int dtype) {
     return dtype == MI355_F32 ? ((const float*)p)[i] : bf16_to_f32(((const bf16_t*)p)[i]);
+}
+
+// four entries from i on (each at its own element: a table may start anywhere)
+__device__ __forceinline__ f32x4 ldsz4(const void* p, int i, int dtype) {
+    if (dtype == MI355_F32) return f32x4{((const float*)p)[i], ((const float*)p)[i + 1], ((const float*)p)[i + 2], ((const float*)p)[i + 3]};
+    const bf16_t* b = (const bf16_t*)p + i;
+    return f32x4{bf16_to_f32(b[0]), bf16_to_f32(b[1]), bf16_to_f32(b[2]), bf16_to_f32(b[3])};
 }
 
 // one row per workgroup: xb = bf16(norm_scale * x), rinv = alpha rsqrt(mean(x^2) + eps) (alpha without norm), sx[m][s] = sum of xb over
@@ -262,6 +252,24 @@ __global__ __launch_bounds__(256) void group_table_kernel(const bf16_t* s0, cons
     }
 }
 
+// o += the K-slices' four values at row[0 .. 3], `stride` floats apart, in slice order.  All slices are requested before the first one is added: a
+// loop over a runtime number of them was one memory round trip per slice, most of the 5-6 us such a launch took.
+template <int N>
+__device__ __forceinline__ void add_slices_n(const float* row, int64_t stride, int ksplit, f32x4& o) {
+    f32x4 v[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) v[s] = *(const f32x4*)(row + (s < ksplit ? s : 0) * stride);
+#pragma unroll
+    for (int s = 0; s < N; ++s)
+        if (s < ksplit) o += v[s];
+}
+__device__ __forceinline__ void add_slices(const float* row, int64_t stride, int ksplit, f32x4& o) {
+    if (ksplit <= 2) return add_slices_n<2>(row, stride, ksplit, o);
+    if (ksplit <= 4) return add_slices_n<4>(row, stride, ksplit, o);
+    if (ksplit <= 8) return add_slices_n<8>(row, stride, ksplit, o);
+    add_slices_n<kMaxSplit>(row, stride, ksplit, o);
+}
+
 // y[m][n] (+)= sum over the K-slices, in slice order (deterministic)
 template <int EPI>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, int ksplit, int M, int N, void* y, int y_dtype,
@@ -272,11 +280,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
         if constexpr (is_pair_epi(EPI)) {
             f32x4 b = {0.f, 0.f, 0.f, 0.f};
-            for (int s = 0; s < ksplit; ++s) {
-                const float* row = part + ((int64_t)s * M + m) * (2 * (int64_t)N);
-                o += *(const f32x4*)(row + n);
-                b += *(const f32x4*)(row + N + n);
-            }
+            const float* row = part + (int64_t)m * (2 * (int64_t)N) + n;
+            add_slices(row, (int64_t)M * 2 * N, ksplit, o);
+            add_slices(row + N, (int64_t)M * 2 * N, ksplit, b);
             bf16_t* dst = (bf16_t*)y + (int64_t)m * ldy + n;
             u32x2 pk;
             pk[0] = (uint32_t)bf16_hw(pair_act_fast<EPI>(o[0], b[0], limit)) | ((uint32_t)bf16_hw(pair_act_fast<EPI>(o[1], b[1], limit)) << 16);
@@ -285,7 +291,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
         } else if (y_dtype == MI355_F32) {
             float* dst = (float*)y + (int64_t)m * ldy + n;
             if constexpr (EPI == MI355_EPI_ACCUM) o = *(const f32x4*)dst;
-            for (int s = 0; s < ksplit; ++s) o += *(const f32x4*)(part + ((int64_t)s * M + m) * N + n);
+            add_slices(part + (int64_t)m * N + n, (int64_t)M * N, ksplit, o);
             if (EPI == MI355_EPI_STORE && bias != nullptr) o += *(const f32x4*)(bias + n);
             if (EPI == MI355_EPI_STORE && relu2) o = f32x4{relu2_f32(o[0]), relu2_f32(o[1]), relu2_f32(o[2]), relu2_f32(o[3])};
             *(f32x4*)dst = o;
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
 #pragma unroll
                 for (int r = 0; r < 4; ++r) o[r] = bf16_to_f32(dst[r]);
             }
-            for (int s = 0; s < ksplit; ++s) o += *(const f32x4*)(part + ((int64_t)s * M + m) * N + n);
+            add_slices(part + (int64_t)m * N + n, (int64_t)M * N, ksplit, o);
             if (EPI == MI355_EPI_STORE && bias != nullptr) o += *(const f32x4*)(bias + n);
             if (EPI == MI355_EPI_STORE && relu2) o = f32x4{relu2_f32(o[0]), relu2_f32(o[1]), relu2_f32(o[2]), relu2_f32(o[3])};
             u32x2 pk;
@@ -320,11 +326,9 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
         const int n = un * 128 + l32 * 4;
         if constexpr (is_pair_epi(EPI)) {
             f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-            for (int sl = 0; sl < p.ksplit; ++sl) {
-                const float* row = p.part + ((int64_t)sl * p.M + m) * (2 * (int64_t)p.N);
-                a += *(const f32x4*)(row + n);
-                b += *(const f32x4*)(row + p.N + n);
-            }
+            const float* row = p.part + (int64_t)m * (2 * (int64_t)p.N) + n;
+            add_slices(row, (int64_t)p.M * 2 * p.N, p.ksplit, a);
+            add_slices(row + p.N, (int64_t)p.M * 2 * p.N, p.ksplit, b);
             bf16_t ob[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(pair_act_fast<EPI>(a[r], b[r], p.limit));
@@ -340,14 +344,20 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
             float* dst = (float*)p.y + (int64_t)m * p.ldy + n;  // (f32 outputs only: host check)
             f32x4 o = {0.f, 0.f, 0.f, 0.f};
             if constexpr (EPI == MI355_EPI_ACCUM) o = *(const f32x4*)dst;
-            for (int sl = 0; sl < p.ksplit; ++sl) o += *(const f32x4*)(p.part + ((int64_t)sl * p.M + m) * p.N + n);
+            [[maybe_unused]] f32x4 ns = {0.f, 0.f, 0.f, 0.f}, cs = {0.f, 0.f, 0.f, 0.f};
+            [[maybe_unused]] int posm = 0;
+            if constexpr (EPI == MI355_EPI_ACCUM) {
+                if (p.out_xb != nullptr) ns = ldsz4(p.next_norm, n, p.next_norm_dtype);
+            } else if (p.rope != nullptr) {
+                posm = p.pos[m];
+                cs = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : posm) * 128 + (n & 127));
+            }
+            add_slices(p.part + (int64_t)m * p.N + n, (int64_t)p.M * p.N, p.ksplit, o);
             if constexpr (EPI == MI355_EPI_STORE) {
                 const int sec = p.rope != nullptr ? (n >= p.C) + (n >= 2 * p.C) : 0;
                 if (sec != 0) {  // as the whole-K epilogue: k rotated in f32, K / V rows to the bf16 cache
                     const int cn = n - sec * p.C, h = cn >> 7, d = cn & 127;
-                    const int posm = p.pos[m];
                     if (sec == 1) {
-                        const f32x4 cs = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : posm) * 128 + d);
                         const float k0 = o[0] * cs[0] - o[1] * cs[1], k1 = o[1] * cs[0] + o[0] * cs[1];
                         const float k2 = o[2] * cs[2] - o[3] * cs[3], k3 = o[3] * cs[2] + o[2] * cs[3];
                         o = f32x4{k0, k1, k2, k3};
@@ -360,7 +370,7 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
                     continue;
                 }
                 if (p.rope != nullptr && p.q_scale != 0.f) {
-                    store_q_ready(p, m, n, p.pos[m], o[0], o[1], o[2], o[3]);
+                    store_q_ready(p, m, n, cs, o[0], o[1], o[2], o[3]);
                     continue;
                 }
             }
@@ -369,7 +379,7 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
                 if (p.out_xb != nullptr) {
                     bf16_t ob[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(o[r] * ldsz(p.next_norm, n + r, p.next_norm_dtype));
+                    for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(o[r] * ns[r]);
                     u32x2 pk;
                     pk[0] = (uint32_t)ob[0] | ((uint32_t)ob[1] << 16);
                     pk[1] = (uint32_t)ob[2] | ((uint32_t)ob[3] << 16);
@@ -380,6 +390,215 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
                         p.out_sx[(int64_t)un * p.M + m] = s1;
                         p.out_ss[(int64_t)un * p.M + m] = s2;
                     }
+                }
+            }
+        }
+    }
+}
+
+// LDS of gemm_q4_kernel behind the two activation buffers: the tokens' factors (2 x BM floats), FUSE: the shares they are summed from (4 KiB), the
+// tokens' positions, the rows' tables
+template <int BM, int NB = 2>
+constexpr int kPosAt = NB * BM * 256 + 2 * BM * 4 + 4096;
+template <int BM, bool FUSE, int NB = 2>
+constexpr int kRowAt = NB * BM * 256 + 2 * BM * 4 + (FUSE ? 4096 + BM * 4 : 0);
+
+// The end of a block: lane (g, c) of a wave holds rows 4 g .. 4 g + 3 of the wave's tiles for token tt * 16 + c (acc: what the MFMAs summed, GRP: the scaled
+// sums).  The tables `fr` (1/rms, operand sums of the tokens), `postab` and `rowtab` (scale, 128 + zero, next norm) stand in LDS; every wave has passed
+// its last read of the activation buffers and no request into them is under way.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP, bool FUSE>
+__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[kTPW][BM / 16], char* smem, const float* fr, const int* postab,
+                                              const float* rowtab, const int (&tile)[kTPW], int m0, int nb, int ks, int wave, int lane) {
+    constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
+    const int g = lane >> 4, c = lane & 15;
+    // old residual rows and rotations are requested for kEB token tiles at a time, without a branch between them (columns and tokens past the end read
+    // entry 0): a load behind a branch of its own is waited for alone
+    constexpr int kEB = BM == 64 ? 2 : 1;
+    const bool emit = FUSE && EPI == MI355_EPI_ACCUM && p.out_xb != nullptr;
+    const bool sums = FUSE && EPI != MI355_EPI_STORE && p.out_sx != nullptr;
+    auto rows4 = [&](int table, int t) { return *(const f32x4*)(rowtab + (table * kSlots + kTPW * wave + t) * 16 + 4 * g); };
+    int nn[kTPW];
+#pragma unroll
+    for (int t = 0; t < kTPW; ++t) nn[t] = tile[t] * 16 + 4 * g;
+#pragma unroll
+    for (int t = 0; t < kTPW; ++t) {
+        [[maybe_unused]] f32x4 sc, zp;
+        if constexpr (FMT == MI355_W_Q4 && GRP == 0) sc = rows4(0, t), zp = rows4(1, t);
+#pragma unroll
+        for (int tt = 0; tt < kTT; ++tt) {
+            const float ri = fr[tt * 16 + c];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (GRP != 0 || FMT == MI355_W_BF16)
+                    acc[t][tt][r] *= ri;
+                else
+                    acc[t][tt][r] = sc[r] * (acc[t][tt][r] - zp[r] * fr[BM + tt * 16 + c]) * ri;
+            }
+        }
+    }
+    if (p.ksplit > 1) {  // partial sums of this K-slice; the SwiGLU pair keeps c_fc1 at column n, c_fc2 at N + n
+        const int64_t ldp = PAIR ? 2 * (int64_t)p.N : (int64_t)p.N;
+#pragma unroll
+        for (int tt = 0; tt < kTT; ++tt) {
+            const int m = m0 + tt * 16 + c;
+#pragma unroll
+            for (int t = 0; t < kTPW; ++t)
+                if (m < p.M && nn[t] < p.N) *(f32x4*)(p.part + ((int64_t)ks * p.M + m) * ldp + (PAIR && (t & 1) ? p.N : 0) + nn[t]) = acc[t][tt];
+        }
+        return;
+    }
+    [[maybe_unused]] float es1[kTT], es2[kTT];  // FUSE: this lane's share of the rows' partial sums (operand values, squares)
+#pragma unroll
+    for (int tb = 0; tb < kTT; tb += kEB) {
+        [[maybe_unused]] f32x4 got[kEB][kTPW];  // ACCUM: the old rows; STORE of c_attn: rotations
+        if constexpr (EPI == MI355_EPI_ACCUM) {
+            if (p.y_dtype == MI355_F32) {
+#pragma unroll
+                for (int i = 0; i < kEB; ++i)
+#pragma unroll
+                    for (int t = 0; t < kTPW; ++t) {
+                        const int m = m0 + (tb + i) * 16 + c;
+                        got[i][t] = *(const f32x4*)((const float*)p.y + (m < p.M && nn[t] < p.N ? (int64_t)m * p.ldy + nn[t] : 0));
+                    }
+            } else {
+#pragma unroll
+                for (int i = 0; i < kEB; ++i)
+#pragma unroll
+                    for (int t = 0; t < kTPW; ++t) {
+                        const int m = m0 + (tb + i) * 16 + c;
+                        const u32x2 w = *(const u32x2*)((const bf16_t*)p.y + (m < p.M && nn[t] < p.N ? (int64_t)m * p.ldy + nn[t] : 0));
+                        got[i][t] = f32x4{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16),
+                                          __uint_as_float(w[1] & 0xffff0000u)};
+                    }
+            }
+        }
+        if constexpr (FUSE && EPI == MI355_EPI_STORE) {
+            if (p.rope != nullptr) {
+#pragma unroll
+                for (int i = 0; i < kEB; ++i) {
+                    const int t16 = (tb + i) * 16 + c;
+                    const int m = m0 + t16 < p.M ? m0 + t16 : p.M - 1;
+#pragma unroll
+                    for (int t = 0; t < kTPW; ++t)
+                        got[i][t] = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : postab[t16]) * 128 + (nn[t] & 127));
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kEB; ++i) {
+            const int tt = tb + i, m = m0 + tt * 16 + c;
+            if constexpr (FUSE) es1[tt] = es2[tt] = 0.f;
+            if (m >= p.M) continue;
+            if constexpr (is_pair_epi(EPI)) {
+#pragma unroll
+                for (int t = 0; t < kTPW; t += 2) {
+                    if (nn[t] >= p.N) continue;  // N % 4 == 0 (host check)
+                    bf16_t ob[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(pair_act_fast<EPI>(acc[t][tt][r], acc[t + 1][tt][r], p.limit));
+                    u32x2 o;
+                    o[0] = (uint32_t)ob[0] | ((uint32_t)ob[1] << 16);
+                    o[1] = (uint32_t)ob[2] | ((uint32_t)ob[3] << 16);
+                    *(u32x2*)((bf16_t*)p.y + (int64_t)m * p.ldy + nn[t]) = o;
+                    if constexpr (FUSE) es1[tt] += (bf16_to_f32(ob[0]) + bf16_to_f32(ob[1])) + (bf16_to_f32(ob[2]) + bf16_to_f32(ob[3]));
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t) {
+                    const int n = nn[t];
+                    if (n >= p.N) continue;
+                    f32x4 o = acc[t][tt];
+                    if constexpr (FUSE && EPI == MI355_EPI_STORE) {
+                        // c_attn (model.py:197-221): rows [C, 2C) are k — rotated in f32 (model.py:306-323; the lane's four rows
+                        // are two interleaved pairs) — rows [2C, 3C) are v; both go to their bf16 cache rows, q goes to y
+                        const int sec = p.rope != nullptr ? (n >= p.C) + (n >= 2 * p.C) : 0;
+                        if (sec != 0) {
+                            const int cn = n - sec * p.C, h = cn >> 7, d = cn & 127;
+                            if (sec == 1) {
+                                const f32x4 cs = got[i][t];
+                                const float k0 = o[0] * cs[0] - o[1] * cs[1], k1 = o[1] * cs[0] + o[0] * cs[1];
+                                const float k2 = o[2] * cs[2] - o[3] * cs[3], k3 = o[3] * cs[2] + o[2] * cs[3];
+                                o = f32x4{k0, k1, k2, k3};
+                            }
+                            const int posm = postab[tt * 16 + c];
+                            const int slot = posm < p.S - 1 ? posm : p.S - 1;
+                            bf16_t* dst = (sec == 1 ? p.kcache : p.vcache) + ((int64_t)h * p.S + slot) * 128 + d;
+                            u32x2 pk;
+                            pk[0] = (uint32_t)bf16_hw(o[0]) | ((uint32_t)bf16_hw(o[1]) << 16);
+                            pk[1] = (uint32_t)bf16_hw(o[2]) | ((uint32_t)bf16_hw(o[3]) << 16);
+                            *(u32x2*)dst = pk;
+                            continue;
+                        }
+                        if (p.rope != nullptr && p.q_scale != 0.f) {
+                            store_q_ready(p, m, n, got[i][t], o[0], o[1], o[2], o[3]);
+                            continue;
+                        }
+                    }
+                    if constexpr (!FUSE && EPI == MI355_EPI_STORE && FMT == MI355_W_BF16) {
+                        if (p.bias != nullptr) o += *(const f32x4*)(p.bias + n);
+                    }
+                    if constexpr (EPI == MI355_EPI_ACCUM) o += got[i][t];
+                    if (!FUSE && EPI == MI355_EPI_STORE && p.relu2) o = f32x4{relu2_f32(o[0]), relu2_f32(o[1]), relu2_f32(o[2]), relu2_f32(o[3])};
+                    if (p.y_dtype == MI355_F32) {
+                        *(f32x4*)((float*)p.y + (int64_t)m * p.ldy + n) = o;
+                        if constexpr (FUSE && EPI == MI355_EPI_ACCUM) {
+                            if (emit) {  // the next linear's operand: bf16(norm scale * x), as stage_rows_kernel rounds it
+                                const f32x4 ns = rows4(2, t);
+                                bf16_t ob[4];
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(o[r] * ns[r]);
+                                u32x2 pk;
+                                pk[0] = (uint32_t)ob[0] | ((uint32_t)ob[1] << 16);
+                                pk[1] = (uint32_t)ob[2] | ((uint32_t)ob[3] << 16);
+                                *(u32x2*)(p.out_xb + (int64_t)m * p.out_ld + n) = pk;
+                                es1[tt] += (bf16_to_f32(ob[0]) + bf16_to_f32(ob[1])) + (bf16_to_f32(ob[2]) + bf16_to_f32(ob[3]));
+                                es2[tt] += (o[0] * o[0] + o[1] * o[1]) + (o[2] * o[2] + o[3] * o[3]);
+                            }
+                        }
+                    } else {
+                        u32x2 pk;
+                        pk[0] = (uint32_t)bf16_hw(o[0]) | ((uint32_t)bf16_hw(o[1]) << 16);
+                        pk[1] = (uint32_t)bf16_hw(o[2]) | ((uint32_t)bf16_hw(o[3]) << 16);
+                        *(u32x2*)((bf16_t*)p.y + (int64_t)m * p.ldy + n) = pk;
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (FUSE && EPI != MI355_EPI_STORE) {
+        // partial sums of the block's rows per token: lane groups (permlane swaps), then the waves through LDS in wave
+        // order (the activation buffers are free: every wave is past its last unit's barrier), one entry per row block
+        if (sums) {
+            // (a block of 256 rows — 8 waves, no pair — writes one share per 128 rows: the granularity a K-split consumer's
+            // slices are cut at; smaller blocks are shares of their own)
+            constexpr int kHalves = (!PAIR && kSlots == 16) ? 2 : 1;
+            float* red = (float*)smem;  // [kWaves][2][BM]
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) {
+                float a = es1[tt], b = es2[tt];
+                a += lane_xor16(a);
+                a += lane_xor32(a);
+                b += lane_xor16(b);
+                b += lane_xor32(b);
+                if (g == 0) {
+                    red[(wave * 2 + 0) * BM + tt * 16 + c] = a;
+                    red[(wave * 2 + 1) * BM + tt * 16 + c] = b;
+                }
+            }
+            __syncthreads();
+            for (int idx = threadIdx.x; idx < kHalves * BM; idx += kThreads) {
+                const int t = idx % BM, half = idx / BM;
+                const int m = m0 + t;
+                const int share = nb * kHalves + half;
+                if (m < p.M && share * (kHalves == 2 ? 128 : (PAIR ? kSlots / 2 : kSlots) * 16) < p.N) {
+                    float a = 0.f, b = 0.f;
+#pragma unroll
+                    for (int w = 0; w < kWaves / kHalves; ++w) {
+                        a += red[((half * (kWaves / kHalves) + w) * 2 + 0) * BM + t];
+                        b += red[((half * (kWaves / kHalves) + w) * 2 + 1) * BM + t];
+                    }
+                    p.out_sx[(int64_t)share * p.M + m] = a;
+                    if (p.out_ss != nullptr) p.out_ss[(int64_t)share * p.M + m] = b;
                 }
             }
         }
@@ -399,10 +618,10 @@ __global__ __launch_bounds__(256) void splitk_fused_reduce_kernel(const GemmPara
 // FUSE: the producer / consumer fusion of gemm_fuse.h (ungrouped launches without a K split): operand sums and 1/rms from
 // partial sums instead of the staging pass; the residual epilogue emits the next linear's bf16 operand and its partial
 // sums, the SwiGLU epilogue the partial operand sums of its output, the c_attn epilogue rotates k and writes the K / V cache
-// (BF16 streams, 8 waves: four pieces per (tile, unit) in flight took the kernel to 130-136 VGPRs, i.e. ONE workgroup per CU;
-// the second launch-bound argument — waves per SIMD — holds it at 128)
+// (second launch-bound argument, waves per SIMD: BF16 streams at 128 VGPRs keep two workgroups per CU, at 132-138 the 2048-token c_fc1/c_fc2 product took
+// 300 us instead of 256; grouped scales at 168 keep three)
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
-__global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 && MI355_GEMM_BF16_OCC) ? 4 : 1) void gemm_q4_kernel(const GemmParams p) {
+__global__ __launch_bounds__(64 * kWaves, GRP == 1 && kWaves == 4 ? 3 : (FMT == MI355_W_BF16 && BM == 128) ? 4 : 1) void gemm_q4_kernel(const GemmParams p) {
     static_assert(GRP == 0 || FMT == MI355_W_Q4, "grouped scales are a Q4 feature");
     static_assert(!FUSE || GRP == 0, "the fused chain runs over per-row scales");
     constexpr int kTT = BM / 16;                   // 16-token tiles per block
@@ -433,7 +652,9 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
         nb = L - mb * n_blocks;
     }
     const int m0 = mb * BM;
-    [[maybe_unused]] float* fr = (float*)(smem + 2 * BM * 256);  // FUSE: [BM] 1/rms, [BM] operand sums of the block's rows
+    float* fr = (float*)(smem + 2 * BM * 256);  // [BM] 1/rms, [BM] operand sums of the block's tokens
+    [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM>);            // FUSE, STORE: [BM] positions
+    [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE>);  // [scale, 128 + zero, next norm's scale][rows of the block]
     // K-slice: units [u_lo, u_hi); GRP 1 cuts at group boundaries (groups [g_lo, g_hi) of upg units each)
     const int g_lo = GRP == 1 ? slice_lo(ks, p.n_groups, p.ksplit) : 0, g_hi = GRP == 1 ? slice_lo(ks + 1, p.n_groups, p.ksplit) : 0;
     const int u_lo = GRP == 1 ? g_lo * p.upg : slice_lo(ks, p.units, p.ksplit);
@@ -471,7 +692,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
     };
     // BF16 streams (round 6): piece d of the NEXT unit is requested into the registers piece d of this unit just left (behind its MFMAs):
     // no second register set — 32 registers less, two workgroups per CU without the scratch the occupancy hint had bought them with
-    constexpr bool kRefill = FMT == MI355_W_BF16 && GRP == 0 && MI355_GEMM_BF16_REFILL;
+    constexpr bool kRefill = FMT == MI355_W_BF16 && GRP == 0;
     [[maybe_unused]] auto wload1 = [&](int t, int u, int d, u32x4& dst) {
         const bool ok = tile[t] < p.n_tiles && u < u_hi;
         const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + rr[t]) * (1024u * kWP);
@@ -531,7 +752,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
     if constexpr (FUSE) {
         if (p.f_in) {
             // (behind the first unit's operand requests, in front of its barrier)
-            // partial sums -> per-row factors.  Every thread takes a row and every kP-th partial, four loads in flight
+            // partial sums -> per-row factors.  Every thread takes a row and every kP-th partial, eight loads in flight
             // (a plain loop over the partials is one memory round trip per partial: 13-15 us per launch, measured), the
             // kP shares are added in share order through LDS: a fixed order, deterministic
             constexpr int kP = kThreads >= BM ? kThreads / BM : 1;
@@ -539,36 +760,67 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
             for (int idx = threadIdx.x; idx < kP * BM; idx += kThreads) {
                 const int t = idx % BM, part = idx / BM;
                 const int64_t m = m0 + t < p.M ? m0 + t : p.M - 1;
-                float sxs = 0.f, sss = 0.f;
                 // (a K-slice of a split launch takes the shares of its own units: the operand sum of ITS columns)
                 const int jlo = p.ksplit > 1 ? slice_lo(ks, p.units, p.ksplit) * p.in_ppu : 0;
                 const int jhi = p.ksplit > 1 ? slice_lo(ks + 1, p.units, p.ksplit) * p.in_ppu : p.in_sx_n;
-                for (int j0 = jlo + part; j0 < jhi; j0 += 4 * kP) {
-                    const int j1 = j0 + kP, j2 = j0 + 2 * kP, j3 = j0 + 3 * kP;
-                    const float v0 = p.in_sx[j0 * (int64_t)p.M + m];
-                    const float v1 = p.in_sx[(j1 < jhi ? j1 : j0) * (int64_t)p.M + m];
-                    const float v2 = p.in_sx[(j2 < jhi ? j2 : j0) * (int64_t)p.M + m];
-                    const float v3 = p.in_sx[(j3 < jhi ? j3 : j0) * (int64_t)p.M + m];
-                    sxs += v0;
-                    sxs += j1 < jhi ? v1 : 0.f;
-                    sxs += j2 < jhi ? v2 : 0.f;
-                    sxs += j3 < jhi ? v3 : 0.f;
-                }
-                for (int j0 = part; j0 < p.in_ss_n; j0 += 4 * kP) {
-                    const int j1 = j0 + kP, j2 = j0 + 2 * kP, j3 = j0 + 3 * kP;
-                    const float v0 = p.in_ss[j0 * (int64_t)p.M + m];
-                    const float v1 = p.in_ss[(j1 < p.in_ss_n ? j1 : j0) * (int64_t)p.M + m];
-                    const float v2 = p.in_ss[(j2 < p.in_ss_n ? j2 : j0) * (int64_t)p.M + m];
-                    const float v3 = p.in_ss[(j3 < p.in_ss_n ? j3 : j0) * (int64_t)p.M + m];
-                    sss += v0;
-                    sss += j1 < p.in_ss_n ? v1 : 0.f;
-                    sss += j2 < p.in_ss_n ? v2 : 0.f;
-                    sss += j3 < p.in_ss_n ? v3 : 0.f;
-                }
+                auto add_shares = [&](const float* in, int lo, int hi) {
+                    constexpr int kIn = 8;  // in flight
+                    float sum = 0.f;
+                    for (int j0 = lo + part; j0 < hi; j0 += kIn * kP) {
+                        float v[kIn];
+#pragma unroll
+                        for (int i = 0; i < kIn; ++i) v[i] = in[(j0 + i * kP < hi ? j0 + i * kP : j0) * (int64_t)p.M + m];
+#pragma unroll
+                        for (int i = 0; i < kIn; ++i) sum += j0 + i * kP < hi ? v[i] : 0.f;
+                    }
+                    return sum;
+                };
+                const float sxs = add_shares(p.in_sx, jlo, jhi), sss = add_shares(p.in_ss, 0, p.in_ss_n);
                 frp[(part * 2 + 0) * BM + t] = sss;
                 frp[(part * 2 + 1) * BM + t] = sxs;
             }
         }
+    }
+    // what the epilogue needs of the block's rows and tokens, fetched behind the first unit's operands: there each of these loads, behind a branch of
+    // its own, was waited for alone (24 memory round trips per launch)
+    if constexpr (FMT == MI355_W_Q4 && GRP == 0) {
+        for (int i = threadIdx.x; i < kSlots * 16; i += kThreads) {
+            const int slot = i >> 4;
+            const int n = (PAIR ? nb * (kSlots / 2) + (slot >> 1) : nb * kSlots + slot) * 16 + (i & 15);
+            const bool ok = n < p.N, second = PAIR && (slot & 1);
+            const void* sp = second ? p.scales2 : p.scales;
+            const void* zq = second ? p.zeros2 : p.zeros;
+            float sv, zv;
+            if (p.sz_dtype == MI355_F32) {
+                sv = ((const float*)sp)[ok ? n : 0];
+                zv = ((const float*)zq)[ok ? n : 0];
+            } else {
+                sv = bf16_to_f32(((const bf16_t*)sp)[ok ? n : 0]);
+                zv = bf16_to_f32(((const bf16_t*)zq)[ok ? n : 0]);
+            }
+            rowtab[i] = ok ? sv : 0.f;
+            rowtab[kSlots * 16 + i] = ok ? 128.f + zv : 0.f;
+        }
+    }
+    if constexpr (FUSE && EPI == MI355_EPI_ACCUM) {
+        if (p.out_xb != nullptr) {
+            for (int i = threadIdx.x; i < kSlots * 16; i += kThreads) {
+                const int n = nb * kSlots * 16 + i;
+                const float v = ldsz(p.next_norm, n < p.N ? n : 0, p.next_norm_dtype);
+                rowtab[2 * kSlots * 16 + i] = n < p.N ? v : 0.f;
+            }
+        }
+    }
+    if (!(FUSE && p.f_in)) {
+        for (int t = threadIdx.x; t < BM; t += kThreads) {
+            const int m = m0 + t < p.M ? m0 + t : p.M - 1;
+            fr[t] = p.rinv != nullptr ? p.rinv[m] : p.alpha;
+            fr[BM + t] = (GRP || FMT == MI355_W_BF16) ? 0.f : p.sx[(int64_t)m * p.ksplit + ks];  // (BF16 weights have no zero point)
+        }
+    }
+    if constexpr (FUSE && EPI == MI355_EPI_STORE) {
+        if (p.rope != nullptr)
+            for (int t = threadIdx.x; t < BM; t += kThreads) postab[t] = p.pos[m0 + t < p.M ? m0 + t : p.M - 1];
     }
     xstore(u_lo & 1);
     __syncthreads();
@@ -633,7 +885,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
     asm volatile("" : "+s"(cmask));
     asm volatile("" : "+v"(cmagic));
 #endif
-    constexpr int kBPipe = (GRP == 0 && FMT == MI355_W_Q4 && BM == 128) ? MI355_GEMM_BPIPE : 0;
+    constexpr int kBPipe = (GRP == 0 && BM == 128 && FMT == MI355_W_Q4) ? MI355_GEMM_BPIPE : 0;
     auto bread = [&](const char* xs, int d, int tt, bool mine) {
         const int tok = tt * 16 + c;
         u32x4 braw = *(const u32x4*)(xs + tok * 256 + (((4 * g + d) ^ swz(tok)) << 4));
@@ -810,208 +1062,299 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && kWaves == 8 &&
         }
     }
 
-    // ---- epilogue: lane (g, c) holds rows 4 g .. 4 g + 3 of its tiles for token tt * 16 + c
-    float sc[kTPW][4], zp[kTPW][4];
-    [[maybe_unused]] float ns[kTPW][4];  // FUSE, residual epilogue: the next RMSNorm's scales of this lane's rows
-    const bool emit = FUSE && EPI == MI355_EPI_ACCUM && p.out_xb != nullptr;
-    const bool sums = FUSE && EPI != MI355_EPI_STORE && p.out_sx != nullptr;
-#pragma unroll
-    for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int n = tile[t] * 16 + 4 * g + r;
-            const bool ok = n < p.N;
-            const void* sp = (PAIR && rr[t] == 1) ? p.scales2 : p.scales;
-            const void* zq = (PAIR && rr[t] == 1) ? p.zeros2 : p.zeros;
-            if constexpr (FMT == MI355_W_BF16 || GRP != 0) {
-                sc[t][r] = ok ? 1.f : 0.f;
-                zp[t][r] = 0.f;
-            } else {
-                sc[t][r] = ok ? ldsz(sp, n, p.sz_dtype) : 0.f;
-                zp[t][r] = ok ? 128.f + ldsz(zq, n, p.sz_dtype) : 0.f;
-            }
-            if constexpr (FUSE && EPI == MI355_EPI_ACCUM) ns[t][r] = (emit && ok) ? ldsz(p.next_norm, n, p.next_norm_dtype) : 0.f;
-        }
-    [[maybe_unused]] float es1[kTT], es2[kTT];  // FUSE: this lane's share of the rows' partial sums (operand values, squares)
-#pragma unroll
-    for (int tt = 0; tt < kTT; ++tt) {
-        if constexpr (FUSE) es1[tt] = es2[tt] = 0.f;
-        const int m = m0 + tt * 16 + c;
-        if (m >= p.M) continue;
-        float sxm, ri;
-        if (FUSE && p.f_in) {
-            ri = fr[tt * 16 + c];
-            sxm = fr[BM + tt * 16 + c];
-        } else {
-            sxm = (GRP || FMT == MI355_W_BF16) ? 0.f : p.sx[(int64_t)m * p.ksplit + ks];  // (BF16 weights have no zero point)
-            ri = p.rinv != nullptr ? p.rinv[m] : p.alpha;
-        }
-        float v[kTPW][4];
+    if constexpr (GRP != 0) {
 #pragma unroll
         for (int t = 0; t < kTPW; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if constexpr (GRP != 0)
-                    v[t][r] = accf[t][tt][r] * ri;
-                else
-                    v[t][r] = sc[t][r] * (acc[t][tt][r] - zp[t][r] * sxm) * ri;
-            }
-        if (p.ksplit > 1) {  // partial sums of this K-slice; the SwiGLU pair keeps c_fc1 at column n, c_fc2 at N + n
-            const int64_t ldp = PAIR ? 2 * (int64_t)p.N : (int64_t)p.N;
-#pragma unroll
-            for (int t = 0; t < kTPW; ++t) {
-                const int n = tile[t] * 16 + 4 * g;
-                if (n < p.N)
-                    *(f32x4*)(p.part + ((int64_t)ks * p.M + m) * ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n) =
-                        f32x4{v[t][0], v[t][1], v[t][2], v[t][3]};
-            }
-            continue;
-        }
-        if constexpr (is_pair_epi(EPI)) {
-#pragma unroll
-            for (int t = 0; t < kTPW; t += 2) {
-                const int n = tile[t] * 16 + 4 * g;
-                if (n < p.N) {  // N % 4 == 0 (host check)
-                    bf16_t* dst = (bf16_t*)p.y + (int64_t)m * p.ldy + n;
-                    bf16_t ob[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(pair_act_fast<EPI>(v[t][r], v[t + 1][r], p.limit));
-                    u32x2 o;
-                    o[0] = (uint32_t)ob[0] | ((uint32_t)ob[1] << 16);
-                    o[1] = (uint32_t)ob[2] | ((uint32_t)ob[3] << 16);
-                    *(u32x2*)dst = o;
-                    if constexpr (FUSE) es1[tt] += (bf16_to_f32(ob[0]) + bf16_to_f32(ob[1])) + (bf16_to_f32(ob[2]) + bf16_to_f32(ob[3]));
-                }
-            }
-        } else {
-            [[maybe_unused]] int posm = 0;
-            if constexpr (FUSE && EPI == MI355_EPI_STORE) {
-                if (p.rope != nullptr) posm = p.pos[m];
-            }
-#pragma unroll
-            for (int t = 0; t < kTPW; ++t) {
-                const int n = tile[t] * 16 + 4 * g;
-                if (n >= p.N) continue;
-                if constexpr (FUSE && EPI == MI355_EPI_STORE) {
-                    // c_attn (model.py:197-221): rows [C, 2C) are k — rotated in f32 (model.py:306-323; the lane's four rows
-                    // are two interleaved pairs) — rows [2C, 3C) are v; both go to their bf16 cache rows, q goes to y
-                    const int sec = p.rope != nullptr ? (n >= p.C) + (n >= 2 * p.C) : 0;
-                    if (sec != 0) {
-                        const int cn = n - sec * p.C, h = cn >> 7, d = cn & 127;
-                        float o0 = v[t][0], o1 = v[t][1], o2 = v[t][2], o3 = v[t][3];
-                        if (sec == 1) {
-                            const f32x4 cs = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : posm) * 128 + d);
-                            const float k0 = o0 * cs[0] - o1 * cs[1], k1 = o1 * cs[0] + o0 * cs[1];
-                            const float k2 = o2 * cs[2] - o3 * cs[3], k3 = o3 * cs[2] + o2 * cs[3];
-                            o0 = k0, o1 = k1, o2 = k2, o3 = k3;
-                        }
-                        const int slot = posm < p.S - 1 ? posm : p.S - 1;
-                        bf16_t* dst = (sec == 1 ? p.kcache : p.vcache) + ((int64_t)h * p.S + slot) * 128 + d;
-                        u32x2 pk;
-                        pk[0] = (uint32_t)bf16_hw(o0) | ((uint32_t)bf16_hw(o1) << 16);
-                        pk[1] = (uint32_t)bf16_hw(o2) | ((uint32_t)bf16_hw(o3) << 16);
-                        *(u32x2*)dst = pk;
-                        continue;
-                    }
-                    if (p.rope != nullptr && p.q_scale != 0.f) {
-                        store_q_ready(p, m, n, posm, v[t][0], v[t][1], v[t][2], v[t][3]);
-                        continue;
-                    }
-                }
-                if constexpr (!FUSE && EPI == MI355_EPI_STORE && FMT == MI355_W_BF16) {
-                    if (p.bias != nullptr) {
-                        const f32x4 b = *(const f32x4*)(p.bias + n);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) v[t][r] += b[r];
-                    }
-                }
-                if (p.y_dtype == MI355_F32) {
-                    float* dst = (float*)p.y + (int64_t)m * p.ldy + n;
-                    f32x4 o = {v[t][0], v[t][1], v[t][2], v[t][3]};
-                    if constexpr (EPI == MI355_EPI_ACCUM) o += *(const f32x4*)dst;
-                    if (!FUSE && EPI == MI355_EPI_STORE && p.relu2) o = f32x4{relu2_f32(o[0]), relu2_f32(o[1]), relu2_f32(o[2]), relu2_f32(o[3])};
-                    *(f32x4*)dst = o;
-                    if constexpr (FUSE && EPI == MI355_EPI_ACCUM) {
-                        if (emit) {  // the next linear's operand: bf16(norm scale * x), as stage_rows_kernel rounds it
-                            bf16_t ob[4];
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) ob[r] = bf16_hw(o[r] * ns[t][r]);
-                            u32x2 pk;
-                            pk[0] = (uint32_t)ob[0] | ((uint32_t)ob[1] << 16);
-                            pk[1] = (uint32_t)ob[2] | ((uint32_t)ob[3] << 16);
-                            *(u32x2*)(p.out_xb + (int64_t)m * p.out_ld + n) = pk;
-                            es1[tt] += (bf16_to_f32(ob[0]) + bf16_to_f32(ob[1])) + (bf16_to_f32(ob[2]) + bf16_to_f32(ob[3]));
-                            es2[tt] += (o[0] * o[0] + o[1] * o[1]) + (o[2] * o[2] + o[3] * o[3]);
-                        }
-                    }
-                } else {
-                    bf16_t* dst = (bf16_t*)p.y + (int64_t)m * p.ldy + n;
-                    float o[4] = {v[t][0], v[t][1], v[t][2], v[t][3]};
-                    if constexpr (EPI == MI355_EPI_ACCUM) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) o[r] += bf16_to_f32(dst[r]);
-                    }
-                    if (!FUSE && EPI == MI355_EPI_STORE && p.relu2) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) o[r] = relu2_f32(o[r]);
-                    }
-                    u32x2 pk;
-                    pk[0] = (uint32_t)bf16_hw(o[0]) | ((uint32_t)bf16_hw(o[1]) << 16);
-                    pk[1] = (uint32_t)bf16_hw(o[2]) | ((uint32_t)bf16_hw(o[3]) << 16);
-                    *(u32x2*)dst = pk;
-                }
-            }
-        }
+            for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = accf[t][tt];
     }
-    if constexpr (FUSE && EPI != MI355_EPI_STORE) {
-        // partial sums of the block's rows per token: lane groups (permlane swaps), then the waves through LDS in wave
-        // order (the activation buffers are free: every wave is past its last unit's barrier), one entry per row block
-        if (sums) {
-            // (a block of 256 rows — 8 waves, no pair — writes one share per 128 rows: the granularity a K-split consumer's
-            // slices are cut at; smaller blocks are shares of their own)
-            constexpr int kHalves = (!PAIR && kWaves == 8) ? 2 : 1;
-            float* red = (float*)smem;  // [kWaves][2][BM]
-#pragma unroll
-            for (int tt = 0; tt < kTT; ++tt) {
-                float a = es1[tt], b = es2[tt];
-                a += lane_xor16(a);
-                a += lane_xor32(a);
-                b += lane_xor16(b);
-                b += lane_xor32(b);
-                if (g == 0) {
-                    red[(wave * 2 + 0) * BM + tt * 16 + c] = a;
-                    red[(wave * 2 + 1) * BM + tt * 16 + c] = b;
-                }
-            }
-            __syncthreads();
-            for (int idx = threadIdx.x; idx < kHalves * BM; idx += kThreads) {
-                const int t = idx % BM, half = idx / BM;
-                const int m = m0 + t;
-                const int share = nb * kHalves + half;
-                if (m < p.M && share * (kHalves == 2 ? 128 : (PAIR ? kSlots / 2 : kSlots) * 16) < p.N) {
-                    float a = 0.f, b = 0.f;
-#pragma unroll
-                    for (int w = 0; w < kWaves / kHalves; ++w) {
-                        a += red[((half * (kWaves / kHalves) + w) * 2 + 0) * BM + t];
-                        b += red[((half * (kWaves / kHalves) + w) * 2 + 1) * BM + t];
-                    }
-                    p.out_sx[(int64_t)share * p.M + m] = a;
-                    if (p.out_ss != nullptr) p.out_ss[(int64_t)share * p.M + m] = b;
-                }
-            }
-        }
-    }
+    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
-int launch_gemm_w(const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row tiles (pair tiles for the SwiGLU stream)
-    constexpr int kLdsW = 2 * BM * 256 + (FUSE ? 2 * BM * 4 + 4096 : 0);  // two activation buffers (+ the rows' factors and the shares they are summed from)
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsW);
-    if (attr_err != hipSuccess) {
-        mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
-        return (int)attr_err;
+// 16 B per lane from `off` of a buffer to 1 KiB of LDS (lane i's bytes at 16 i); out of range: zeros
+__device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, unsigned off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+}
+
+// The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of any prompt):
+// there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
+// of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
+// alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
+// BM: 16 / 32 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
+    constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
+    constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
+    constexpr int kXI = BM / 4 > kWaves ? BM / 4 / kWaves : 1;  // activation requests (1 KiB: four tokens) per wave and unit
+    constexpr int kUnit = kXI + kTPW * kWP;                     // requests per wave and unit
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int n_blocks = p.n_blocks;
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int L2 = xcd * p.per_xcd + j;
+    if (j >= p.per_xcd || L2 >= p.total_blocks * p.ksplit) return;
+    const int L = L2 / p.ksplit, ks = L2 - L * p.ksplit;
+    const int m_blocks = p.total_blocks / n_blocks;
+    int mb, nb;
+    if constexpr (FMT == MI355_W_BF16) {  // (orders: see gemm_q4_kernel)
+        nb = L / m_blocks;
+        mb = L - nb * m_blocks;
+    } else {
+        mb = L / n_blocks;
+        nb = L - mb * n_blocks;
     }
+    const int m0 = mb * BM;
+    const int u_lo = slice_lo(ks, p.units, p.ksplit), u_hi = slice_lo(ks + 1, p.units, p.ksplit);
+    float* fr = (float*)(smem + DEPTH * BM * 256);
+    [[maybe_unused]] float* frp = fr + 2 * BM;
+    [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM, DEPTH>);
+    [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE, DEPTH>);
+    int tile[kTPW];
+#pragma unroll
+    for (int t = 0; t < kTPW; ++t)
+        tile[t] = PAIR ? nb * (kSlots / 2) + (kTPW / 2) * wave + (t >> 1) : nb * kSlots + kTPW * wave + t;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (int)p.w_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw0 = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, 0, 0x00020000);
+    const bf16_t* xbase = p.xb;
+    if constexpr (EPI == MI355_EPI_STORE && FMT == MI355_W_BF16 && !FUSE) {
+        if (p.slice_blocks != 0) xbase += (int64_t)(nb / p.slice_blocks) * p.slice_stride;
+    }
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)(unsigned)((int64_t)p.M * p.ldxb * 2), 0x00020000);
+    const unsigned lane_off = lane * 16;
+    // this lane's token and column of its activation requests (waves beyond the block's BM / 4 requests repeat one: the same bytes to the same place)
+    unsigned xoff[kXI];
+    int xdst[kXI];
+#pragma unroll
+    for (int i = 0; i < kXI; ++i) {
+        const int q = (i * kWaves + wave) % (BM / 4);
+        const int tok = q * 4 + (lane >> 4), slot = lane & 15;
+        xoff[i] = m0 + tok < p.M ? (unsigned)((int64_t)(m0 + tok) * p.ldxb * 2) + (unsigned)((slot ^ swz(tok)) * 16) : 0xFFFFFFF0u;
+        xdst[i] = q * 1024;
+    }
+    u32x4 wr[DEPTH][kTPW][kWP];
+    // request i of unit u: activations first.  Past the slice: nothing is read, zeros go to a buffer that nobody reads
+    auto request = [&](int i, int u, int slot) {
+        const bool in = u < u_hi;
+        if (i < kXI) {
+            lds_from(rx, smem + slot * (BM * 256) + xdst[i < kXI ? i : 0], in && xoff[i < kXI ? i : 0] != 0xFFFFFFF0u ? xoff[i < kXI ? i : 0] + (unsigned)u * 256u : 0xFFFFFFF0u);
+        } else {
+            const int t = (i - kXI) / kWP, d = (i - kXI) % kWP;
+            const bool ok = tile[t] < p.n_tiles && in;
+            const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * (1024u * kWP) + d * 1024u;
+            wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off : 0u, 0));
+        }
+    };
+
+    // ---- tables of the epilogue: requested ahead of the units, written to LDS behind their requests
+    constexpr bool kScales = FMT == MI355_W_Q4;
+    constexpr int kRT = (kSlots * 16 + kThreads - 1) / kThreads;
+    [[maybe_unused]] float t_sc[kRT], t_zp[kRT], t_ns[kRT];
+    if constexpr (kScales) {
+        const bool f32 = p.sz_dtype == MI355_F32;
+#pragma unroll
+        for (int i = 0; i < kRT; ++i) {
+            const int r = i * kThreads + threadIdx.x, slot = r >> 4;
+            const int n = (PAIR ? nb * (kSlots / 2) + (slot >> 1) : nb * kSlots + slot) * 16 + (r & 15);
+            const int at = n < p.N ? n : 0;
+            const void* sp = PAIR && (slot & 1) ? p.scales2 : p.scales;
+            const void* zq = PAIR && (slot & 1) ? p.zeros2 : p.zeros;
+            float sv, zv;
+            if (f32) {
+                sv = ((const float*)sp)[at];
+                zv = ((const float*)zq)[at];
+            } else {
+                sv = bf16_to_f32(((const bf16_t*)sp)[at]);
+                zv = bf16_to_f32(((const bf16_t*)zq)[at]);
+            }
+            t_sc[i] = n < p.N ? sv : 0.f;
+            t_zp[i] = n < p.N ? 128.f + zv : 0.f;
+        }
+    }
+    const bool norm_tab = FUSE && EPI == MI355_EPI_ACCUM && p.out_xb != nullptr;
+    if constexpr (FUSE && EPI == MI355_EPI_ACCUM) {
+        if (norm_tab) {
+#pragma unroll
+            for (int i = 0; i < kRT; ++i) {
+                const int n = nb * kSlots * 16 + i * kThreads + (int)threadIdx.x;
+                t_ns[i] = n < p.N ? ldsz(p.next_norm, n, p.next_norm_dtype) : 0.f;
+            }
+        }
+    }
+    const int mt = (int)threadIdx.x < BM ? (m0 + (int)threadIdx.x < p.M ? m0 + (int)threadIdx.x : p.M - 1) : p.M - 1;
+    const bool own = !(FUSE && p.f_in);  // factors of the tokens as they are, not as shares
+    float t_ri = p.alpha, t_sx = 0.f;
+    if (own) {
+        if (p.rinv != nullptr) t_ri = p.rinv[mt];
+        if constexpr (kScales) t_sx = p.sx[(int64_t)mt * p.ksplit + ks];
+    }
+    [[maybe_unused]] int t_pos = 0;
+    if constexpr (FUSE && EPI == MI355_EPI_STORE) {
+        if (p.rope != nullptr) t_pos = p.pos[mt];
+    }
+    // shares of the tokens' factors (gemm_fuse.h): every thread a token and every kP-th share, in share order; the first kIn of them now
+    constexpr int kP = kThreads / BM < 8 ? kThreads / BM : 8, kIn = kSharesAhead;
+    const int s_tok = threadIdx.x % BM, s_part = threadIdx.x / BM;
+    [[maybe_unused]] const int64_t s_m = m0 + s_tok < p.M ? m0 + s_tok : p.M - 1;
+    [[maybe_unused]] const int s_lo = FUSE && p.ksplit > 1 ? u_lo * p.in_ppu : 0, s_hi = FUSE && p.ksplit > 1 ? u_hi * p.in_ppu : p.in_sx_n;
+    [[maybe_unused]] float vx[kIn], vs[kIn];
+    auto shares = [&](const float* in, int j0, int hi, float (&v)[kSharesAhead]) {
+#pragma unroll
+        for (int i = 0; i < kIn; ++i) v[i] = in[(j0 + i * kP < hi ? j0 + i * kP : 0) * (int64_t)p.M + s_m];
+    };
+    auto add_shares = [&](int j0, int hi, const float (&v)[kSharesAhead], float sum) {
+#pragma unroll
+        for (int i = 0; i < kIn; ++i) sum += j0 + i * kP < hi ? v[i] : 0.f;
+        return sum;
+    };
+    if constexpr (FUSE) {
+        if (!own && s_part < kP) {
+            shares(p.in_sx, s_lo + s_part, s_hi, vx);
+            if (p.in_ss_n > 0) shares(p.in_ss, s_part, p.in_ss_n, vs);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < DEPTH - 1; ++s) {
+#pragma unroll
+        for (int i = 0; i < kUnit; ++i) request(i, u_lo + s, s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    [[maybe_unused]] float sxs = 0.f, sss = 0.f;
+    if constexpr (FUSE) {
+        if (!own && s_part < kP) {
+            sxs = add_shares(s_lo + s_part, s_hi, vx, 0.f);
+            if (p.in_ss_n > 0) sss = add_shares(s_part, p.in_ss_n, vs, 0.f);
+        }
+    }
+    if constexpr (kScales) {
+#pragma unroll
+        for (int i = 0; i < kRT; ++i) {
+            const int r = i * kThreads + (int)threadIdx.x;
+            if (kSlots * 16 % kThreads == 0 || r < kSlots * 16) rowtab[r] = t_sc[i], rowtab[kSlots * 16 + r] = t_zp[i];
+        }
+    }
+    if constexpr (FUSE && EPI == MI355_EPI_ACCUM) {
+        if (norm_tab) {
+#pragma unroll
+            for (int i = 0; i < kRT; ++i) {
+                const int r = i * kThreads + (int)threadIdx.x;
+                if (kSlots * 16 % kThreads == 0 || r < kSlots * 16) rowtab[2 * kSlots * 16 + r] = t_ns[i];
+            }
+        }
+    }
+    if ((int)threadIdx.x < BM) {
+        if (own) fr[threadIdx.x] = t_ri, fr[BM + threadIdx.x] = t_sx;
+        if constexpr (FUSE && EPI == MI355_EPI_STORE) postab[threadIdx.x] = t_pos;
+    }
+
+    f32x4 acc[kTPW][kTT];
+#pragma unroll
+    for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+        for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint32_t cmask = 0x000F000Fu, cmagic = 0x43004300u;  // (opaque: see gemm_q4_kernel)
+    asm volatile("" : "+s"(cmask));
+    asm volatile("" : "+v"(cmagic));
+    constexpr int kFrags = 4 * kTT, kPipe = 4;
+    // the requests of unit `ahead` go out between the products: a request takes the CU's memory pipeline 16 cycles, and in one burst behind the barrier
+    // the waves of a workgroup stood in line for it with no product under way
+    constexpr int kEvery = kFrags >= 2 * kUnit ? kFrags / (2 * kUnit) : 1;  // fragments from one request to the next (all in the first half if it holds them)
+    constexpr int kPer = (kUnit + kFrags - 1) / kFrags;                      // requests behind one fragment
+    auto mfmas = [&](int slot, u32x4 (&w)[kTPW][kWP], int ahead, int ahead_slot) {
+        const char* xs = smem + slot * (BM * 256);
+        auto bread = [&](int f) {  // fragment f = d * kTT + tt
+            const int tok = (f % kTT) * 16 + c;
+            return *(const u32x4*)(xs + tok * 256 + (((4 * g + f / kTT) ^ swz(tok)) << 4));
+        };
+        u32x4 bq[kPipe];
+#pragma unroll
+        for (int q = 0; q < kPipe; ++q) bq[q] = bread(q);
+        __builtin_amdgcn_sched_group_barrier(0x100, kPipe, 0);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            bf16x8 a[kTPW];
+#pragma unroll
+            for (int t = 0; t < kTPW; ++t) {
+                if constexpr (FMT == MI355_W_BF16) {
+                    a[t] = __builtin_bit_cast(bf16x8, w[t][d]);
+                } else {
+                    const uint32_t v = w[t][0][d];
+                    u32x4 f;
+                    f[0] = (v & cmask) | cmagic;
+                    f[1] = ((v >> 4) & cmask) | cmagic;
+                    f[2] = ((v >> 8) & cmask) | cmagic;
+                    f[3] = ((v >> 12) & cmask) | cmagic;
+                    a[t] = __builtin_bit_cast(bf16x8, f);
+                }
+            }
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) {
+                const int f = d * kTT + tt;
+                const bf16x8 b = __builtin_bit_cast(bf16x8, bq[f % kPipe]);
+                if (f + kPipe < kFrags) bq[f % kPipe] = bread(f + kPipe);
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[t][tt], 0, 0, 0);
+                if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
+                if (f % kEvery == 0) {
+#pragma unroll
+                    for (int i = 0; i < kPer; ++i) {
+                        const int r = f / kEvery * kPer + i;
+                        if (r >= kUnit) continue;
+                        request(r, ahead, ahead_slot);
+                        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int u = u_lo; u < u_hi; u += DEPTH) {
+#pragma unroll
+        for (int s = 0; s < DEPTH; ++s) {
+            if (s > 0 && u + s >= u_hi) break;
+            // own requests of this unit have landed (DEPTH - 2 units are newer); every wave's have, and every wave is done with the unit before: its
+            // buffer and registers take the unit DEPTH - 1 ahead
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((DEPTH - 2) * kUnit) : "memory");
+            mfmas(s, wr[s], u + s + DEPTH - 1, (s + DEPTH - 1) % DEPTH);
+        }
+    }
+    if constexpr (FUSE) {
+        if (p.f_in) {  // the rest of the shares
+            if (s_part < kP) {
+                for (int j0 = s_lo + s_part + kIn * kP; j0 < s_hi; j0 += kIn * kP) {
+                    shares(p.in_sx, j0, s_hi, vx);
+                    sxs = add_shares(j0, s_hi, vx, sxs);
+                }
+                for (int j0 = s_part + kIn * kP; j0 < p.in_ss_n; j0 += kIn * kP) {
+                    shares(p.in_ss, j0, p.in_ss_n, vs);
+                    sss = add_shares(j0, p.in_ss_n, vs, sss);
+                }
+                frp[(s_part * 2 + 1) * BM + s_tok] = sxs;
+                frp[(s_part * 2 + 0) * BM + s_tok] = sss;
+            }
+            __syncthreads();
+            if ((int)threadIdx.x < BM) {
+                sss = sxs = 0.f;
+#pragma unroll
+                for (int q = 0; q < kP; ++q) {
+                    sss += frp[(q * 2 + 0) * BM + threadIdx.x];
+                    sxs += frp[(q * 2 + 1) * BM + threadIdx.x];
+                }
+                fr[threadIdx.x] = p.in_ss_n > 0 ? rsqrtf(sss / (float)p.K + p.eps) : 1.0f;
+                fr[BM + threadIdx.x] = sxs;
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests past the slice wrote zeros: none may land in what the epilogue keeps there)
+    __syncthreads();
+    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, 0, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
+}
+
+template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, typename Kernel>
+int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row tiles (pair tiles for the SwiGLU stream)
     constexpr int kSlots = kWaves * kTPW;
     const int per_block = PAIR ? kSlots / 2 : kSlots;
     GemmParams q = p;
@@ -1026,7 +1369,7 @@ int launch_gemm_w(const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row ti
             q.rope = nullptr;
         }
     }
-    hipLaunchKernelGGL((gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>), dim3(8 * q.per_xcd), dim3(64 * kWaves), kLdsW, s, q);
+    hipLaunchKernelGGL(kernel, dim3(8 * q.per_xcd), dim3(64 * kWaves), lds, s, q);
     MI355_LAUNCH_CHECK();
     if constexpr (FUSE) {
         if (q.ksplit > 1) {
@@ -1046,77 +1389,97 @@ int launch_gemm_w(const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row ti
     }
     return 0;
 }
-// The shape of an ungrouped launch: blocks of 16 row tiles x 128 tokens when that fills the chip (256 CUs x 2 workgroups);
-// anything smaller — the N = 4096 outputs of a long prompt (16 row blocks: at T = 2048 one workgroup per CU, matrix pipes
-// 37 % busy against 53 % for the c_fc1 / c_fc2 pair), and every launch of a short prompt, K-split or not — takes 64-token
-// blocks: twice the workgroups, half the LDS each.  Sweep over (waves, tokens per block, K-slices) at 128 / 256 / 512 tokens
-// (scripts/sweep_gemm_shapes.sh, profiles/r04_gemm_shape_sweep.txt): 64-token blocks win every linear (one layer's linears
-// 216 -> 183 / 269 -> 226 / 361 -> 320 us), the 2-wave blocks of round 3 never do; those stay for launches too small to split.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE>
+int launch_deep(const GemmParams& p, hipStream_t s) {
+    constexpr int kDepth = BM == 128 && FMT == MI355_W_BF16 ? 3 : 4;
+    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64;
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (attr_err != hipSuccess) {
+        mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
+        return (int)attr_err;
+    }
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth>, kLds, p, s);
+}
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
+int launch_gemm_w(const GemmParams& p, hipStream_t s) {
+    constexpr int kLdsW = kRowAt<BM, FUSE> + 3 * kWaves * kTPW * 64;
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsW);
+    if (attr_err != hipSuccess) {
+        mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
+        return (int)attr_err;
+    }
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
+}
 struct GemmShape {
     int waves, bm;
+    bool deep;
 };
-// tuning override for sweeps (scripts/sweep_gemm_shapes.sh): MI355_GEMM_FORCE="waves:bm:ksplit[:bf16_blocks[:q4_blocks]]", 0 = the rule's choice
-// (fields 4 / 5: the block counts below which the BF16 / int4 streams take 64-token blocks)
+// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep", 0 = the rule's choice
 struct GemmForce {
-    int waves, bm, ksplit, bf16_blocks, q4_blocks;  // *_blocks: the 64-token-block thresholds of the two formats (sweeps)
+    int waves, bm, ksplit, deep;
 };
 GemmForce gemm_force() {
-    // parsed ONCE per process (a getenv + sscanf per launch sat on the production path, and a change of the variable
-    // between mi355_linear_gemm_plan and the launch would have desynchronised the share layout of the fused chain; the sweep starts
-    // one process per setting)
-    static const GemmForce f = [] {
-        GemmForce g = {0, 0, 0, 0, 0};
-        if (const char* e = getenv("MI355_GEMM_FORCE")) sscanf(e, "%d:%d:%d:%d:%d", &g.waves, &g.bm, &g.ksplit, &g.bf16_blocks, &g.q4_blocks);
+    // parsed ONCE per process (a change of the variable between mi355_linear_gemm_plan and the launch would desynchronise the share layout of
+    // the fused chain)
+#ifndef MI355_GEMM_SWEEP
+    static
+#endif
+    const GemmForce f = [] {
+        GemmForce g = {0, 0, 0, 0};
+        if (const char* e = getenv("MI355_GEMM_FORCE")) sscanf(e, "%d:%d:%d:%d", &g.waves, &g.bm, &g.ksplit, &g.deep);
         return g;
     }();
     return f;
 }
-GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16 = false) {
+// Waves of a block (what the share layout of mi355_linear_gemm_plan depends on).  Up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them,
+// which 4-5 K-slices bring to a workgroup for two CUs of three; 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, int4 with staging:
+// 20.5 us against 22.7).
+int gemm_waves(int M) { return gemm_force().waves ? gemm_force().waves : M <= 64 ? 4 : 8; }
+// Tokens per block and kernel.  Blocks of 128 tokens x 256 rows with two workgroups per CU (gemm_q4_kernel) when a launch has a few of them per CU: 2048
+// tokens, int4, c_fc1/c_fc2 271 us against 303 (gemm_deep_kernel, one workgroup per CU), c_attn 158 / 174.  Fewer: 64-token blocks, twice as many, of the
+// deep kernel: 128 tokens, int4, c_fc1/c_fc2 49.6 -> 39.9 us, 777 tokens N = 4096 47.8 -> 42.1 us.  An int4 launch of exactly one 128-token block per CU (N = 4096
+// at 2048 tokens) keeps those.  BF16 streams are bound by the weight bytes a CU requests per product (a 64-token block requests twice a 128-token block's), so
+// they keep 128 tokens as long as those blocks cover 5/8 of the CUs: 512 tokens, c_fc1/c_fc2 134 / 106 us; up to one block per CU through the deep
+// kernel: 2048 tokens, N = 4096, K = 11008 174 -> 158 us.
+GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16) {
     const GemmForce fo = gemm_force();
-    if ((fo.waves == 8 && (fo.bm == 64 || fo.bm == kBM)) || ((fo.waves == 2 || fo.waves == 1) && (fo.bm == 0 || fo.bm == kBM)))
-        return {fo.waves, fo.bm ? fo.bm : kBM};
+    GemmShape sh = {gemm_waves(M), M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
     const int per_block8 = pair ? 8 * kTPW / 2 : 8 * kTPW;
-    const int blocks8 = ((n_tiles + per_block8 - 1) / per_block8) * ((M + kBM - 1) / kBM);
-    if (ksplit == 1 && blocks8 < 96) {  // (K < 1024: nothing to split)
-        if (blocks8 * 4 >= 128) return {2, kBM};
-        return {1, kBM};
-    }
-    // (only the WAVES of the answer enter mi355_linear_gemm_plan's share layout: the format may pick its own token block)
-    // BF16 streams are bound by the weight bytes a CU requests per MFMA (pieces four times an int4 one's, a 64-token block requests twice
-    // a 128-token block's): they keep 128 tokens as long as those blocks cover 5/8 of the CUs, K-slices or not (7B: 2048 tokens 28.5 -> 25.6 ms, 1536 23.2 -> 22.0,
-    // 512 10.6 -> 9.8; at 128 blocks — N = 4096 at 1024 tokens — 64 tokens win, 15.2 vs 16.7 ms; profiles/r06_bf16_gemm_tilings.txt)
-#ifndef MI355_GEMM_NO_BM64
-    // int4 streams: 64-token blocks below 384 blocks — unless the 128-token blocks are exactly one per CU (N = 4096 at 2048 tokens:
-    // no tail; 2048-token prompt 21.85 -> 21.5 ms, where a plain threshold of 256 cost 2 % at 384 / 512 tokens: profiles/r06_q4_gemm_tilings.txt)
-    const bool one_per_cu = blocks8 * ksplit == 256 && MI355_GEMM_ONE_PER_CU;
-    if (bf16 ? blocks8 < (fo.bf16_blocks ? fo.bf16_blocks : 160) : (blocks8 * ksplit < (fo.q4_blocks ? fo.q4_blocks : 384) && !one_per_cu)) return {8, 64};
-#endif
-    return {8, kBM};
+    const int blocks8 = ((n_tiles + per_block8 - 1) / per_block8) * ((M + kBM - 1) / kBM) * ksplit;  // of 128 tokens
+    if (bf16 ? M > 128 && blocks8 >= 160 : blocks8 >= 384 || blocks8 == 256) sh.bm = 128, sh.deep = bf16 && blocks8 <= 256;
+    if (fo.bm) sh.bm = fo.bm;
+    if (fo.deep) sh.deep = fo.deep == 1;
+    return sh;
 }
-// split-K of an ungrouped launch: fewer than 96 blocks (a 128-token prompt against N = 4096 is 16) cut K into up to 8
-// slices, as many as bring the launch to ~128 workgroups and fit the partial buffer
-int gemm_ksplit(int M, int N, int K, bool swiglu) {
+// Split-K of an ungrouped launch: as many slices as bring it to the workgroups wanted, none below 6 units (BF16: 4) or past the partial buffer.  BF16, whose
+// weights are four times the bytes, gains from more of them up to 64 tokens (16 rows, 4096 x 11008: 66 / 39 / 31 / 27 / 23.4 us with 1 / 2 / 3 / 4 / 8 slices);
+// int4 pays the reduction instead (37 tokens, 12288 x 4096: 29.8 / 28.2 / 30.4 / 34.2 us with 1 / 2 / 3 / 8).
+int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
     const int units = (K + 127) / 128;
+    const size_t row_floats = (size_t)N * (pair ? 2 : 1);
     if (const int fk = gemm_force().ksplit) {
-        if (fk >= 1 && fk <= kMaxSplit && units >= fk && (size_t)2 * fk * M * (size_t)N * (swiglu ? 2 : 1) * 4 <= kSplitBudget) return fk;
+        if (fk >= 1 && fk <= kMaxSplit && units >= fk && (size_t)2 * fk * M * row_floats * 4 <= kSplitBudget) return fk;
     }
-    const int rows_per_block = swiglu ? 16 * 8 * kTPW / 2 : 16 * 8 * kTPW;
-    const int blocks8 = ((N + rows_per_block - 1) / rows_per_block) * ((M + kBM - 1) / kBM);
-    const size_t row_floats = (size_t)N * (swiglu ? 2 : 1);
+    const int waves = gemm_waves(M);
+    const int rows_per_block = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
+    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), want = waves == 8 ? 192 : bf16 ? 400 : 160;
     int ksplit = 1;
-    while (ksplit < kMaxSplit && blocks8 * ksplit < 96 && units >= 8 * ksplit && (size_t)2 * ksplit * M * row_floats * 4 <= kSplitBudget)
-        ksplit *= 2;
+    while (ksplit < (bf16 ? kMaxSplit : 8) && blocks * ksplit < want && units >= (bf16 ? 4 : 6) * (ksplit + 1) && (size_t)2 * (ksplit + 1) * M * row_floats * 4 <= kSplitBudget) ++ksplit;
     return ksplit;
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
     const GemmShape sh = gemm_shape(p.n_tiles, p.M, PAIR, p.ksplit, FMT == MI355_W_BF16);
-    if (sh.waves == 8) {
-        if (sh.bm == 64) return launch_gemm_w<EPI, PAIR, FMT, 8, 64, 0, FUSE>(p, s);
-        return launch_gemm_w<EPI, PAIR, FMT, 8, kBM, 0, FUSE>(p, s);
+    if (sh.waves == 4) {
+        if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE>(p, s);
+        if (sh.bm == 32) return launch_deep<EPI, PAIR, FMT, 4, 32, FUSE>(p, s);
+        return launch_deep<EPI, PAIR, FMT, 4, 64, FUSE>(p, s);
     }
-    if (sh.waves == 2) return launch_gemm_w<EPI, PAIR, FMT, 2, kBM, 0, FUSE>(p, s);
-    return launch_gemm_w<EPI, PAIR, FMT, 1, kBM, 0, FUSE>(p, s);
+    if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 8, 64, FUSE>(p, s);
+    if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
+    return launch_gemm_w<EPI, PAIR, FMT, 8, kBM, 0, FUSE>(p, s);
 }
 // grouped scales: blocks of 64 tokens x 4 waves (the second accumulator set costs the registers of more tokens or waves);
 // from kGrpWideM tokens on, 128 tokens x 8 waves (2048-token g128 prompt 41.9 -> 39.4 ms; at 512 tokens it is the slower
@@ -1169,13 +1532,12 @@ extern "C" int mi355_linear_gemm(const mi355_linear_args* a, void* workspace, si
     return mi355_linear_gemm_fused(a, nullptr, workspace, workspace_bytes, stream);
 }
 
-void mi355_linear_gemm_plan(int M, int N, int K, int R, int* ksplit, int* shares, int* shares_per_unit) {
+void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
     const bool pair = R == 2;
-    const int ks = gemm_ksplit(M, N, K, pair);
-    const GemmShape sh = gemm_shape((N + 15) / 16, M, pair, ks);
+    const int ks = gemm_ksplit(M, N, K, pair, bf16);
     // rows (hidden rows of a pair stream) behind one share of a producer's partial sums: a 128-column unit when the K-slices'
     // reduction writes them or a block holds 256 rows, else the block's rows
-    int rows = (pair ? sh.waves * kTPW / 2 : sh.waves * kTPW) * 16;
+    int rows = (pair ? gemm_waves(M) * kTPW / 2 : gemm_waves(M) * kTPW) * 16;
     if (ks > 1 || rows > 128) rows = 128;
     *ksplit = ks;
     *shares = (N + rows - 1) / rows;
@@ -1243,7 +1605,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
                (size_t)2 * ksplit * a->M * row_floats * 4 <= kSplitBudget / 2)
             ksplit *= 2;
     } else {
-        ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu);
+        ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, !q4);
     }
     // producer / consumer fusion (gemm_fuse.h): whole-K launches over per-row scales only — the caller plans with
     // mi355_linear_gemm_plan

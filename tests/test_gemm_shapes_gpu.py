@@ -1,0 +1,73 @@
+"""The tiled products at the sizes where their blocks, K-slices and pipelines end: every number of tokens per block, odd rows and columns, slices of
+few units, launches that are cut and launches that are not."""
+import pytest
+import torch
+
+from lit_llama_amd import _native as nat
+from lit_llama_amd import ops, synth
+from lit_llama_amd.model import LLaMA, LLaMAConfig
+from lit_llama_amd.utils import EmptyInitOnDevice
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # M, N, K
+    (1, 16, 128), (9, 144, 300), (15, 4096, 4096), (16, 1000, 640), (17, 4096, 1024), (31, 528, 2048), (32, 272, 4224), (33, 4096, 4096),
+    (48, 12288, 512), (64, 128, 11008), (65, 4096, 4096), (127, 2064, 896), (128, 11008, 384), (129, 4096, 1664), (200, 260, 1024),
+    (300, 12288, 256), (1030, 4096, 384), (2048, 4096, 256), (2050, 8200, 128),
+]
+
+
+@pytest.mark.parametrize("epi", ["store", "accum", "pair"])
+@pytest.mark.parametrize("fmt", ["q4", "bf16"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_tiled_product_against_64_bits(dev, fmt, M, N, K, epi):
+    """The operands are exact in bf16 and summed in f32: the bf16 stream within sqrt(K) roundings of its terms, the int4 stream within those of terms 30
+    times the result's (levels enter as 128 + q, the offset is taken off at the end): 1e-3 of the result covers both at K = 11008."""
+    g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    n_mats = 2 if epi == "pair" else 1
+    if fmt == "q4":
+        qs = [torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8) for _ in range(n_mats)]
+        ss = [(torch.rand((N,), generator=g, device=dev) * 0.02 + 0.005).to(torch.bfloat16) for _ in range(n_mats)]
+        zs = [torch.randint(5, 11, (N,), generator=g, device=dev).to(torch.bfloat16) for _ in range(n_mats)]
+        pk = [synth.pack_colblock(q, 4) for q in qs] if K % 2 == 0 else None
+        stream = ops.repack_q4(pk[0], pk[1] if n_mats == 2 else None, N, K, n_mats)
+        kw = dict(scales=ss[0], zeros=zs[0])
+        if n_mats == 2:
+            kw.update(scales2=ss[1], zeros2=zs[1])
+        ws = [(q.double() - z.double()[:, None]) * s.double()[:, None] for q, s, z in zip(qs, ss, zs)]
+    else:
+        mats = [(torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16) for _ in range(n_mats)]
+        stream = ops.repack_bf16(mats[0], mats[1] if n_mats == 2 else None, n_mats)
+        kw, ws = dict(fmt=nat.W_BF16), [m.double() for m in mats]
+    prods = [x.double() @ w.T for w in ws]
+    if epi == "pair":
+        ref = torch.nn.functional.silu(prods[0]) * prods[1]
+        got = ops.linear_gemm(x, stream, 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, **kw).double()
+        assert (got - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 2e-3 * ref.square().mean().sqrt()  # one rounding to bf16
+        return
+    if epi == "accum":
+        base = torch.randn((M, N), generator=g, device=dev)
+        ref = prods[0] + base.double()
+        got = ops.linear_gemm(x, stream, 1, N, K, epi=nat.EPI_ACCUM, out=base.clone(), **kw).double()
+    else:
+        ref = prods[0]
+        got = ops.linear_gemm(x, stream, 1, N, K, out_dtype=torch.float32, **kw).double()
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
+@pytest.mark.parametrize("mode", ["gptq.int4", None])
+@pytest.mark.parametrize("T", [2, 8, 9, 10, 11, 16, 17, 31, 33, 64, 65, 130, 257])
+def test_prompt_pass_of_any_length_matches_single_tokens(dev, mode, T):
+    """A prompt in one pass against the same tokens one by one (the row kernels): logits of every position within the spread of bf16 operands."""
+    cfg = LLaMAConfig(block_size=288, n_layer=2, n_head=8, n_embd=1024, vocab_size=512)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=mode):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=1, mode=mode, device="cuda", dtype=torch.bfloat16))
+    model.eval()
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    with torch.no_grad():
+        one = model(idx.view(1, -1), 288, torch.arange(T, device=dev))[0]
+        model.reset_cache()
+        rows = torch.cat([model(idx[t:t + 1].view(1, 1), 288, torch.tensor([t], device=dev))[0] for t in range(T)])
+    assert (one - rows).abs().max() <= 0.05 * rows.std()
