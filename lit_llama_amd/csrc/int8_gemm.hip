@@ -8,14 +8,19 @@
 //   1. i8_stage_kernel   (one workgroup per row) — xh = f16(norm_scale * x * 1/rms) (or f16(x)), the row's absmax over its
 //                        sub-threshold entries, and the column mask |xh| >= threshold OR-ed over all rows (atomicOr: order
 //                        does not matter);
-//   2. i8_quant_kernel   — CA = rint(xh * 127 / absmax) with the masked columns zeroed, int8; workgroup 0 also writes the
-//                        ascending list of outlier columns;
+//   2. i8_quant_kernel   — CA = rint(xh * 127 / absmax) with the masked columns zeroed, int8; the ascending list of outlier columns; and those columns by
+//                        themselves, f16: xo (rows) and so = f16(CB * SCB / 127) (weights; workgroups behind the rows');
 //   3. i8_gemm_kernel    — the int8 weight stream of int8.hip ([tile][unit][r][piece e][lane][16 x int8], one piece = one
-//                        MFMA A operand) against CA staged through LDS (128 tokens x 128 k, XOR-swizzled), two row tiles per
-//                        wave, 8 waves; epilogue with the arithmetic of int8.hip, rounding for rounding:
+//                        MFMA A operand) against CA through LDS (128 tokens x 128 k, XOR-swizzled), two row tiles per
+//                        wave, 8 waves; then so x xo in the same loop on the f16 MFMA (of a launch cut along K: a slice of its own); epilogue with the arithmetic
+//                        of int8.hip, rounding for rounding:
 //                            d = f16((acc * 6.200012e-05 * absmax[m]) * SCB[n]);   o = sum over outlier columns k (ascending) of
 //                            xh[m, k] * f16(CB[n, k] * SCB[n] / 127);   y = f16(d + f16(o))   (the last step only with outliers)
-//                        the outlier operands of the block (128 tokens x n_out, 256 rows x n_out) are staged in LDS first.
+//                        More outlier columns than `so` has room for are staged through LDS 64 at a time, as all of them once were.
+// 512 tokens, 7B, two layers (2000 of mlp.c_proj's 11008 columns hold an outlier): 1950 -> 976 us.  A launch: quantise 30 -> 12 us, stage 16.4 -> 7.5, c_fc1/c_fc2
+// 108 -> 83, attn.c_proj / mlp.c_proj slices 48 -> 35 and their sum 151 -> 15 us on average.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -27,7 +32,8 @@ constexpr int kSlots = kWaves * kTPW;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kXTile = kBM * 128;        // bytes of one activation tile (int8)
 constexpr int kOutChunk = 64;            // outlier columns staged per pass of the epilogue
-constexpr int kLdsMain = 2 * kXTile;
+constexpr int kDepth = 4;                // units of operands in LDS and registers
+constexpr int kLdsMain = kDepth * kXTile;
 constexpr int kSoLd = kOutChunk + 8;     // row pitch of the staged outlier weights (halves): 144 B, so that 16 rows written side by side fall into 16 banks
 constexpr int kLdsEpi = (kBM * kOutChunk + kSlots * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [256 rows][kSoLd]
 constexpr int kLds = kLdsMain > kLdsEpi ? kLdsMain : kLdsEpi;
@@ -39,6 +45,10 @@ __device__ __forceinline__ float f16r(float v) { return f16_to_f32(f32_to_f16(v)
 __device__ __forceinline__ float f16r_of_f32(float v) {
     asm volatile("" : "+v"(v));
     return f16r(v);
+}
+// 16 B per lane from `off` of a buffer to 1 KiB of LDS; out of range: zeros
+__device__ __forceinline__ void i8_lds_from(__amdgpu_buffer_rsrc_t r, char* lds, unsigned off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
 }
 // 16-B chunk swizzle of a 128-B activation row in LDS: rows alternate bank halves (128-B pitch), pairs of rows rotate the
 // 8 chunks — the 16 lanes a ds_read_b128 serves together (tokens {0-3, 12-15} with one k-group, {4-11} with the next)
@@ -64,8 +74,18 @@ struct I8GemmParams {
     int ksplit;
     int64_t ldp;
     int* part;
+    // the outlier columns by themselves (i8_quant_kernel): xo[m][ld], so[(tile R + r) 16 + row][ld] = f16(CB SCB / 127), ld = compact_ld(n_out) (whole units of 64), columns past
+    // n_out zero.  They exist where so fits its region
+    f16_t* xo;
+    f16_t* so;
 };
-constexpr size_t kSplitBudget = (size_t)32 << 20;
+constexpr size_t kSplitBudget = (size_t)32 << 20;             // bytes of the int32 partial tiles of all K-slices,
+constexpr size_t kPartBytes = kSplitBudget + kSplitBudget / 2;  // next to the f32 tiles of the outlier columns (2 slices at least)
+constexpr size_t kOutlierBudget = (size_t)32 << 20;  // bytes of `so`
+__device__ __forceinline__ int compact_ld(int n_out) { return (n_out + 63) & ~63; }
+__device__ __forceinline__ bool is_compact(int n_out, int n_tiles, int R, int M) {
+    return n_out > 0 && (size_t)n_tiles * R * 16 * compact_ld(n_out) * 2 <= kOutlierBudget && (size_t)M * compact_ld(n_out) * 2 < 0x7fffffffu;
+}
 constexpr int kMaxSplit = 8;
 
 // ---- 1. rows: f16 operand, absmax over the sub-threshold entries, outlier column mask
@@ -74,69 +94,191 @@ __global__ void i8_clear_mask_kernel(unsigned* mask, int n) {
     if (i < n) mask[i] = 0u;
 }
 
-__global__ __launch_bounds__(256) void i8_stage_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale,
-                                                       int norm_dtype, float eps, float threshold, int K, int Kp, f16_t* xh,
-                                                       float* sca, unsigned* mask) {
+// (a thread's elements are 256 apart, 16 of them requested at a time: one at a time behind a switch over the type, a row of 11008 took 25 us)
+template <typename T>
+__device__ __forceinline__ float i8_row_value(T v);
+template <>
+__device__ __forceinline__ float i8_row_value<float>(float v) { return v; }
+template <>
+__device__ __forceinline__ float i8_row_value<bf16_t>(bf16_t v) { return bf16_to_f32(v); }
+struct f16_raw { f16_t v; };
+template <>
+__device__ __forceinline__ float i8_row_value<f16_raw>(f16_raw v) { return f16_to_f32(v.v); }
+
+template <typename T>
+__global__ __launch_bounds__(256) void i8_stage_kernel(const T* x, int64_t ldx, const void* norm_scale, int norm_dtype, float eps, float threshold, int K,
+                                                       int Kp, f16_t* xh, float* sca, unsigned* mask) {
+    constexpr int kAhead = 16;
     __shared__ float red[32];
     const int m = blockIdx.x;
+    const T* row = x + (int64_t)m * ldx;
     float rinv = 1.f;
     if (norm_scale != nullptr) {
         float ss = 0.f;
-        for (int k = threadIdx.x; k < K; k += blockDim.x) {
-            const float v = ld_as_f32(x, (int64_t)m * ldx + k, x_dtype);
-            ss += v * v;
+        for (int k0 = threadIdx.x; k0 < K; k0 += 256 * kAhead) {
+            T raw[kAhead];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) raw[i] = row[k0 + 256 * i < K ? k0 + 256 * i : k0];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+                if (k0 + 256 * i < K) {
+                    const float v = i8_row_value(raw[i]);
+                    ss += v * v;
+                }
         }
         rinv = rsqrtf(block_sum(ss, red) / (float)K + eps);
     }
     float amax = 0.f;
-    for (int k = threadIdx.x; k < Kp; k += blockDim.x) {
-        f16_t h = 0;
-        if (k < K) {
-            float v = ld_as_f32(x, (int64_t)m * ldx + k, x_dtype);
-            if (norm_scale != nullptr) v = ld_as_f32(norm_scale, k, norm_dtype) * (v * rinv);
-            h = f32_to_f16(v);
-            const float a = fabsf(f16_to_f32(h));
-            if (threshold > 0.f && a >= threshold)
-                atomicOr(mask + (k >> 5), 1u << (k & 31));
-            else
-                amax = fmaxf(amax, a);
+    for (int k0 = threadIdx.x; k0 < Kp; k0 += 256 * kAhead) {
+        T raw[kAhead];
+        float ns[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) raw[i] = row[k0 + 256 * i < K ? k0 + 256 * i : 0];
+        if (norm_scale != nullptr) {
+            if (norm_dtype == MI355_BF16) {
+#pragma unroll
+                for (int i = 0; i < kAhead; ++i) ns[i] = bf16_to_f32(((const bf16_t*)norm_scale)[k0 + 256 * i < K ? k0 + 256 * i : 0]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kAhead; ++i) ns[i] = ld_as_f32(norm_scale, k0 + 256 * i < K ? k0 + 256 * i : 0, norm_dtype);
+            }
         }
-        xh[(int64_t)m * Kp + k] = h;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int k = k0 + 256 * i;
+            f16_t h = 0;
+            if (k < K) {
+                float v = i8_row_value(raw[i]);
+                if (norm_scale != nullptr) v = ns[i] * (v * rinv);
+                h = f32_to_f16(v);
+                const float a = fabsf(f16_to_f32(h));
+                if (threshold > 0.f && a >= threshold)
+                    atomicOr(mask + (k >> 5), 1u << (k & 31));
+                else
+                    amax = fmaxf(amax, a);
+            }
+            if (k < Kp) xh[(int64_t)m * Kp + k] = h;
+        }
     }
     amax = block_max(amax, red);
     if (threadIdx.x == 0) sca[m] = amax;
 }
 
-// ---- 2. rows: int8 operand; workgroup 0: the outlier list
-__global__ __launch_bounds__(256) void i8_quant_kernel(const f16_t* xh, const float* sca, const unsigned* mask, int Kp, int8_t* ca,
-                                                       int* olist) {
-    const int m = blockIdx.x;
-    const float a = sca[m];
-    const float inv = a > 0.f ? __fdiv_rn(127.0f, a) : 0.f;  // IEEE division: parity with the oracle
-    for (int k4 = threadIdx.x; k4 < Kp / 4; k4 += blockDim.x) {
-        const int k = 4 * k4;
-        const unsigned mw = mask[k >> 5] >> (k & 31);
-        const u32x2 hv = *(const u32x2*)(xh + (int64_t)m * Kp + k);
-        uint32_t q4 = 0u;
+// ---- 2. the int8 operand, the list of outlier columns (workgroup 0) and, by themselves, the outlier columns of the rows and of the weights: the
+// epilogue then multiplies dense f16 matrices.  (It used to gather both per block of the product, a weight byte, a division and an f16 activation per element
+// and token block: 295 us of a 512-token mlp.c_proj; and the list was one thread's chain of dependent loads: 25 of this launch's 30 us.)
+// Workgroups 0 .. M - 1: a row each; the others: the weights, 16 rows x 32 columns per wave and turn.
+constexpr int kMaskWords = 512;  // of the mask per turn: 16 384 columns
+__global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int8_t* ca, int* olist, const I8GemmParams p, int R) {
+    __shared__ unsigned words[kMaskWords];
+    __shared__ int before[kMaskWords];  // outlier columns in front of a word
+    __shared__ uint16_t cols[kMaskWords * 32];  // the outlier columns of this turn, from its first word on
+    __shared__ int wave_tot[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int Kp = p.Kp, nw = Kp >> 5, m = blockIdx.x;
+    int n_out;
+    {
+        int c = 0;
+        for (int w = threadIdx.x; w < nw; w += 256) c += __popc(mask[w]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f16_t h = (f16_t)((j & 1) ? (hv[j >> 1] >> 16) : (hv[j >> 1] & 0xffffu));
-            const float q = ((mw >> j) & 1u) ? 0.f : rintf(f16_to_f32(h) * inv);
-            q4 |= ((uint32_t)(int)q & 0xffu) << (8 * j);
-        }
-        *(uint32_t*)(ca + (int64_t)m * Kp + k) = q4;
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+        if (lane == 0) wave_tot[wave] = c;
+        __syncthreads();
+        n_out = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
     }
-    if (m == 0 && threadIdx.x == 0) {
-        int n = 0;
-        for (int w = 0; w < Kp / 32; ++w) {
-            unsigned bits = mask[w];
-            while (bits != 0u) {
-                const int b = __builtin_ctz(bits);
-                olist[1 + n++] = w * 32 + b;
-                bits &= bits - 1u;
+    const bool compact = is_compact(n_out, p.n_tiles, R, p.M);
+    const int ld = compact_ld(n_out);
+    const bool of_row = m < p.M;
+    if (!of_row && !compact) return;
+    const float a = of_row ? p.sca[m] : 0.f;
+    const float inv = a > 0.f ? __fdiv_rn(127.0f, a) : 0.f;  // IEEE division: parity with the oracle
+    if (m == 0 && threadIdx.x == 0) olist[0] = n_out;
+    if (of_row && compact)
+        for (int j = n_out + (int)threadIdx.x; j < ld; j += 256) p.xo[(int64_t)m * ld + j] = 0;
+    int carry = 0;
+    for (int w0 = 0; w0 < nw; w0 += kMaskWords) {
+        const int cnt = nw - w0 < kMaskWords ? nw - w0 : kMaskWords;
+        const int per = (cnt + 255) / 256, lo = threadIdx.x * per, hi = lo + per < cnt ? lo + per : cnt;
+        __syncthreads();  // (the last turn is done with words, before and wave_tot)
+        int c = 0;
+        for (int w = lo; w < hi; ++w) {
+            words[w] = mask[w0 + w];
+            c += __popc(words[w]);
+        }
+        int incl = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(incl, o);
+            if (lane >= o) incl += up;
+        }
+        if (lane == 63) wave_tot[wave] = incl;
+        __syncthreads();
+        int at = carry + incl - c;
+        for (int w = 0; w < wave; ++w) at += wave_tot[w];
+        const int j_lo = carry, j_hi = carry + wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];  // outlier columns of this turn
+        carry = j_hi;
+        for (int w = lo; w < hi; ++w) {
+            before[w] = at;
+            for (unsigned bits = words[w]; bits != 0u; ++at, bits &= bits - 1u) cols[at - j_lo] = (uint16_t)(w * 32 + __builtin_ctz(bits));
+        }
+        __syncthreads();
+        if (m == 0)
+            for (int j = j_lo + (int)threadIdx.x; j < j_hi; j += 256) olist[1 + j] = w0 * 32 + cols[j - j_lo];
+        if (of_row) {
+            const f16_t* row = p.xh + (int64_t)m * Kp;
+            constexpr int kAhead = 4;
+            const int e4 = (w0 + cnt) * 8;
+            for (int k0 = w0 * 8 + (int)threadIdx.x; k0 < e4; k0 += 256 * kAhead) {
+                u32x2 hv[kAhead];
+#pragma unroll
+                for (int i = 0; i < kAhead; ++i) hv[i] = *(const u32x2*)(row + 4 * (k0 + 256 * i < e4 ? k0 + 256 * i : k0));
+#pragma unroll
+                for (int i = 0; i < kAhead; ++i) {
+                    const int k4 = k0 + 256 * i;
+                    if (k4 >= e4) continue;
+                    const int k = 4 * k4, w = (k >> 5) - w0;
+                    const unsigned bits = words[w] >> (k & 31);
+                    uint32_t q4 = 0u;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const f16_t h = (f16_t)((j & 1) ? (hv[i][j >> 1] >> 16) : (hv[i][j >> 1] & 0xffffu));
+                        const bool out = (bits >> j) & 1u;
+                        const float q = out ? 0.f : rintf(f16_to_f32(h) * inv);
+                        q4 |= ((uint32_t)(int)q & 0xffu) << (8 * j);
+                        if (out && compact) p.xo[(int64_t)m * ld + before[w] + __popc(words[w] & ((1u << ((k & 31) + j)) - 1u))] = h;
+                    }
+                    *(uint32_t*)(ca + (int64_t)m * Kp + k) = q4;
+                }
+            }
+        } else {
+            const int row = lane & 15, total = p.n_tiles * R;
+            const bool last = w0 + cnt >= nw;
+            const int jb0 = j_lo >> 5, jb1 = last ? ld >> 5 : (j_hi + 31) >> 5;
+            const int64_t items = (int64_t)(jb1 - jb0) * total;
+            for (int64_t it = (int64_t)(m - p.M) * 4 + wave; it < items; it += (int64_t)(gridDim.x - p.M) * 4) {
+                const int jb = jb0 + (int)(it / total), tr = (int)(it - (int64_t)(jb - jb0) * total);
+                const int tl = tr / R, r1 = tr - tl * R, n = tl * 16 + row;
+                const float sc = (r1 == 1 ? p.scb2 : p.scb)[n < p.N ? n : 0];
+                f16_t* dst = p.so + ((int64_t)tr * 16 + row) * ld;
+                const int j0 = jb * 32 + (lane >> 4) * 8;
+                int64_t off[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int j = j0 + i;
+                    const int k = j >= j_lo && j < j_hi ? w0 * 32 + cols[j - j_lo] : 0;
+                    off[i] = ((((int64_t)tl * p.units + (k >> 7)) * R + r1) * 2 + ((k >> 6) & 1)) * 1024 + (((k >> 4) & 3) * 16 + row) * 16 + (k & 15);
+                }
+                int8_t cb[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) cb[i] = (int8_t)p.w[off[i]];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int j = j0 + i;
+                    if (j >= j_lo && j < j_hi) dst[j] = n < p.N ? f32_to_f16(__fdiv_rn((float)cb[i] * sc, 127.0f)) : (f16_t)0;
+                    else if (last && j >= j_hi && j < ld) dst[j] = 0;
+                }
             }
         }
-        olist[0] = n;
     }
 }
 
@@ -152,13 +294,13 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
     const int L2 = xcd * p.per_xcd + j0;
     // MODE 1: a workgroup per (block, K-slice); MODE 2: a workgroup per (block, 16-token tile) — 8 x the workgroups of the
     // product launch, so that summing the slices and the epilogue are not left to a dozen workgroups
-    const int nsplit = MODE == 1 ? p.ksplit : MODE == 2 ? 8 : 1;
+    const int nsplit = MODE == 1 ? p.ksplit + 1 : MODE == 2 ? 8 : 1;
     if (j0 >= p.per_xcd || L2 >= p.total_blocks * nsplit) return;
     const int L = L2 / nsplit, ks = L2 - L * nsplit;
     // MODE 2: workgroup ks of a block finishes the rows of slot group ks (the rows wave ks owns in the product launch) for all 128
-    // tokens, wave w its token tile w — so the outlier columns' weights (the expensive side of the staging: byte gathers and an IEEE
-    // division each) are staged once per block, not once per token tile
-    const int tt_lo = MODE == 2 ? wave : 0, tt_hi = MODE == 2 ? wave + 1 : 8;  // token tiles this wave finishes
+    // tokens, wave w its token tile w
+    constexpr int kTT = MODE == 2 ? 1 : 8;                                     // token tiles a wave finishes, from tt0 on
+    const int tt0 = MODE == 2 ? wave : 0;
     const int wslot = MODE == 2 ? ks : wave;                                   // slot group of this wave's row tiles
     const int mb = L / p.n_blocks, nb = L - mb * p.n_blocks;
     const int m0 = mb * kBM;
@@ -182,73 +324,124 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
     const __amdgpu_buffer_rsrc_t rx =
         __builtin_amdgcn_make_buffer_rsrc((void*)p.ca, 0, (int)((int64_t)p.M * p.Kp), 0x00020000);
     const unsigned lane_off = lane * 16;
-    auto wload = [&](int t, int u, u32x4 (&dst)[2]) {
-        const bool ok = tile[t] < p.n_tiles && u < u_hi;
-        const unsigned off = (unsigned)((tile[t] * p.units + u) * R + rr[t]) * 2048u;
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-            dst[e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off + e * 1024u : 0u, 0));
-    };
-    // activation tile of unit u: 1024 chunks of 16 B, two per thread; chunk = (token, 16-B column)
-    u32x4 stage[2];
-    auto xload = [&](int u) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int ch = i * kThreads + threadIdx.x;
-            const int tok = ch >> 3, col = ch & 7;
-            const unsigned off = (unsigned)((int64_t)(m0 + tok) * p.Kp) + (unsigned)u * 128u + (unsigned)col * 16u;
-            stage[i] = __builtin_bit_cast(
-                u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, ((m0 + tok) < p.M && u < u_hi) ? off : 0xFFFFFFF0u, 0, 0));
-        }
-    };
-    auto xstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int ch = i * kThreads + threadIdx.x;
-            const int tok = ch >> 3, col = ch & 7;
-            *(u32x4*)(smem + buf * kXTile + tok * 128 + ((col ^ swz8(tok)) << 4)) = stage[i];
-        }
-    };
-
-    i32x4 acc[kTPW][8];
+    i32x4 acc[kTPW][kTT];
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt) acc[t][tt] = i32x4{0, 0, 0, 0};
+        for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = i32x4{0, 0, 0, 0};
 
-    if constexpr (MODE != 2) {
-        u32x4 wcur[kTPW][2], wnext[kTPW][2];
+    // The units of a product: int8 units of 128 columns, or (F16) units of 64 compact outlier columns — 128 B of a token either way.  The weights (registers) and
+    // the activations (LDS, by DMA, the swizzle on the source's side) of the next kDepth - 1 units are under way; a unit waits for its own requests by
+    // count, and the requests go out between the products (as gemm_deep_kernel: csrc/gemm.hip).  One unit ahead, waited for in front of its LDS stores, a unit
+    // took 1.56 us at one workgroup per CU
+    constexpr int kXI = kBM / 8 / kWaves, kUnit = kXI + 2 * kTPW;  // requests per wave and unit: 1 KiB = 8 tokens of activations; weight pieces
+    auto run_units = [&](auto f16, auto& sum, int lo, int hi, __amdgpu_buffer_rsrc_t rwt, __amdgpu_buffer_rsrc_t rxt, int64_t ldb) {
+        constexpr bool F16 = decltype(f16)::value;
+        typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_l;
+        unsigned xoff[kXI];
+        int xdst[kXI];
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t) wload(t, u_lo, wcur[t]);
-        xload(u_lo);
-        xstore(u_lo & 1);
-        __syncthreads();
-        for (int u = u_lo; u < u_hi; ++u) {
-            const int buf = u & 1;
-            xload(u + 1);  // unconditional: past the last unit the offsets are out of the descriptor (zeros, no traffic)
+        for (int i = 0; i < kXI; ++i) {
+            const int q = i * kWaves + wave, tok = q * 8 + (lane >> 3), slot = lane & 7;
+            xoff[i] = m0 + tok < p.M ? (unsigned)((int64_t)(m0 + tok) * ldb) + (unsigned)((slot ^ swz8(tok)) * 16) : 0xFFFFFFF0u;
+            xdst[i] = q * 1024;
+        }
+        const unsigned w_lane = F16 ? (unsigned)(c * ldb + g * 16) : lane_off;
+        u32x4 wr[kDepth][kTPW][2];
+        auto request = [&](int i, int u, int slot) {
+            const bool in = u < hi;
+            if (i < kXI) {
+                const unsigned off = in && xoff[i < kXI ? i : 0] != 0xFFFFFFF0u ? xoff[i < kXI ? i : 0] + (unsigned)u * 128u : 0xFFFFFFF0u;
+                i8_lds_from(rxt, smem + slot * kXTile + xdst[i < kXI ? i : 0], off);
+            } else {
+                const int t = (i - kXI) / 2, e = (i - kXI) % 2;
+                const bool ok = tile[t] < p.n_tiles && in;
+                const unsigned off = F16 ? (unsigned)((int64_t)(tile[t] * R + rr[t]) * 16 * ldb) + (unsigned)u * 128u + e * 64u
+                                         : (unsigned)((tile[t] * p.units + u) * R + rr[t]) * 2048u + e * 1024u;
+                wr[slot][t][e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rwt : rw0, w_lane, ok ? off : 0u, 0));
+            }
+        };
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t) wload(t, u + 1, wnext[t]);
-            const char* xs = smem + buf * kXTile;
+        for (int d = 0; d < kDepth - 1; ++d) {
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
+            for (int i = 0; i < kUnit; ++i) request(i, lo + d, d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto products = [&](int slot, int ahead, int ahead_slot) {
+            const char* xs = smem + slot * kXTile;
+            constexpr int kFrags = 16, kPipe = 4;  // fragment f = e * 8 + tt
+            auto bread = [&](int f) {
+                const int tok = (f & 7) * 16 + c;
+                return *(const i32x4*)(xs + tok * 128 + (((4 * (f >> 3) + g) ^ swz8(tok)) << 4));
+            };
+            i32x4 bq[kPipe];
 #pragma unroll
-                for (int tt = 0; tt < 8; ++tt) {
-                    const int tok = tt * 16 + c;
-                    const i32x4 b = *(const i32x4*)(xs + tok * 128 + (((4 * e + g) ^ swz8(tok)) << 4));
+            for (int q = 0; q < kPipe; ++q) bq[q] = bread(q);
+            __builtin_amdgcn_sched_group_barrier(0x100, kPipe, 0);
 #pragma unroll
-                    for (int t = 0; t < kTPW; ++t)
-                        acc[t][tt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, wcur[t][e]), b, acc[t][tt], 0, 0, 0);
+            for (int f = 0; f < kFrags; ++f) {
+                const i32x4 b = bq[f % kPipe];
+                if (f + kPipe < kFrags) bq[f % kPipe] = bread(f + kPipe);
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t) {
+                    if constexpr (F16)
+                        sum[t][f & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_l, wr[slot][t][f >> 3]),
+                                                                               __builtin_bit_cast(f16x8_l, b), sum[t][f & 7], 0, 0, 0);
+                    else
+                        sum[t][f & 7] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, wr[slot][t][f >> 3]), b, sum[t][f & 7], 0, 0, 0);
+                }
+                if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
+                if (f < kUnit) {
+                    request(f, ahead, ahead_slot);
+                    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
                 }
             }
-            xstore(buf ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int u = lo; u < hi; u += kDepth) {
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t) {
-                wcur[t][0] = wnext[t][0];
-                wcur[t][1] = wnext[t][1];
+            for (int d = 0; d < kDepth; ++d) {
+                if (d > 0 && u + d >= hi) break;
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kDepth - 2) * kUnit) : "memory");
+                products(d, u + d + kDepth - 1, (d + kDepth - 1) % kDepth);
             }
-            __syncthreads();
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests past the end wrote zeros: none may land in what follows)
+        __syncthreads();
+    };
+    const int n_out = MODE == 1 && ks < p.ksplit ? 0 : p.olist[0];
+    const bool compact = is_compact(n_out, p.n_tiles, R, p.M);
+    [[maybe_unused]] f32x4 o[kTPW][kTT];  // the compact outlier columns' share
+    auto outliers = [&]() {
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) o[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int ld = compact_ld(n_out);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.so, 0, p.n_tiles * R * 16 * ld * 2, 0x00020000);
+        const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void*)p.xo, 0, p.M * ld * 2, 0x00020000);
+        run_units(std::true_type{}, o, 0, ld / 64, rs, ro, (int64_t)ld * 2);
+    };
+    if constexpr (MODE == 1) {
+        if (ks == p.ksplit) {  // the launch's last slice: the outlier columns
+            if (!compact) return;
+            outliers();
+#pragma unroll
+            for (int tt = 0; tt < 8; ++tt) {
+                const int m = m0 + tt * 16 + c;
+                if (m >= p.M) continue;
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t) {
+                    const int n = tile[t] * 16 + 4 * g;
+                    if (tile[t] < p.n_tiles && n < p.N)
+                        *(f32x4*)((float*)p.part + ((int64_t)ks * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n) = o[t][tt];
+                }
+            }
+            return;
         }
     }
+    if constexpr (MODE != 2) run_units(std::false_type{}, acc, u_lo, u_hi, rw, rx, (int64_t)p.Kp);
     // partial tiles of a K-slice: column n of c_fc2 sits at N + n
     if constexpr (MODE == 1) {
 #pragma unroll
@@ -264,42 +457,58 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         }
         return;
     }
-    if constexpr (MODE == 2) {
+    if constexpr (MODE == 2) {  // all slices requested before the first is added (one at a time was a memory round trip each)
+        const int m = m0 + tt0 * 16 + c;
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt) {
-            const int m = m0 + tt * 16 + c;
-            if (m >= p.M || tt < tt_lo || tt >= tt_hi) continue;
+        for (int t = 0; t < kTPW; ++t) {
+            const int n = tile[t] * 16 + 4 * g;
+            const int* at = p.part + (m < p.M && tile[t] < p.n_tiles && n < p.N ? (int64_t)m * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n : 0);
+            i32x4 v[kMaxSplit];
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t) {
-                const int n = tile[t] * 16 + 4 * g;
-                if (tile[t] < p.n_tiles && n < p.N)
-                    for (int s2 = 0; s2 < p.ksplit; ++s2)
-                        acc[t][tt] += *(const i32x4*)(p.part + ((int64_t)s2 * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n);
-            }
+            for (int s2 = 0; s2 < kMaxSplit; ++s2) v[s2] = *(const i32x4*)(at + (s2 < p.ksplit ? s2 : 0) * ((int64_t)p.M * p.ldp));
+#pragma unroll
+            for (int s2 = 0; s2 < kMaxSplit; ++s2)
+                if (s2 < p.ksplit) acc[t][0] += v[s2];
+            if (compact) o[t][0] = *(const f32x4*)((const float*)at + p.ksplit * ((int64_t)p.M * p.ldp));
         }
     }
 
-    // ---- epilogue.  lane (g, c) holds rows 4 g .. 4 g + 3 of its tiles for token tt * 16 + c
-    float scb[kTPW][4];
+    // ---- epilogue.  lane (g, c) holds rows 4 g .. 4 g + 3 of its tiles for token tt * 16 + c.  Loads without a branch between them
+    float scb[kTPW][4], sa[kTT];
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = tile[t] * 16 + 4 * g + r;
-            scb[t][r] = n < p.N ? ((PAIR && rr[t] == 1) ? p.scb2 : p.scb)[n] : 0.f;
+            scb[t][r] = ((PAIR && rr[t] == 1) ? p.scb2 : p.scb)[n < p.N ? n : 0];
         }
-    float d[kTPW][8][4];
 #pragma unroll
-    for (int tt = 0; tt < 8; ++tt) {
-        const int m = m0 + tt * 16 + c;
-        const float sa = m < p.M ? p.sca[m] : 0.f;
+    for (int tt = 0; tt < kTT; ++tt) {
+        const int m = m0 + (tt0 + tt) * 16 + c;
+        sa[tt] = p.sca[m < p.M ? m : 0];
+    }
+    float d[kTPW][kTT][4];
+    auto dequant = [&]() {
+#pragma unroll
+        for (int tt = 0; tt < kTT; ++tt)
+#pragma unroll
+            for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r_of_f32((((float)acc[t][tt][r] * 6.200012e-05f) * sa[tt]) * scb[t][r]);
+    };
+    typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+    if (compact) {
+        // mixed-precision decomposition over the compact columns, ascending k
+        if constexpr (MODE == 0) outliers();
+        dequant();
 #pragma unroll
         for (int t = 0; t < kTPW; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r_of_f32((((float)acc[t][tt][r] * 6.200012e-05f) * sa) * scb[t][r]);
-    }
-    const int n_out = p.olist[0];
-    if (n_out > 0) {
+            for (int tt = 0; tt < kTT; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r(d[t][tt][r] + f16r(o[t][tt][r]));
+    } else if (n_out > 0) {  // (too many for their region)
+        dequant();
         // mixed-precision decomposition: the outlier columns in f16, ascending k, kOutChunk columns per pass through LDS
         f16_t* xo = (f16_t*)smem;                     // [128 tokens][kOutChunk]
         f16_t* so = xo + kBM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
@@ -309,12 +518,11 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         // ascending k — bitsandbytes' own f16 GEMM promises no order either, and the tests allow the one f16 ulp this can move.  The scalar
         // loop it replaces (64 FMAs per lane and outlier column) took 1.4 ms per attn.c_proj / mlp.c_proj launch at T = 2048, where ~10 % of
         // the columns of a 2048-token call hold an outlier: profiles/r06_prefill_int8_outliers.txt.)
-        typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-        f32x4 o[kTPW][8];
+        f32x4 o[kTPW][kTT];
 #pragma unroll
         for (int t = 0; t < kTPW; ++t)
 #pragma unroll
-            for (int tt = 0; tt < 8; ++tt) o[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int tt = 0; tt < kTT; ++tt) o[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int base = 0; base < n_out; base += kOutChunk) {
             const int nc = n_out - base < kOutChunk ? n_out - base : kOutChunk;
             __syncthreads();  // (the main loop / the previous pass is done with the LDS)
@@ -370,9 +578,8 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
 #pragma unroll
                 for (int t = 0; t < kTPW; ++t) a[t] = *(const f16x8_t*)(so + ((wslot * kTPW + t) * 16 + c) * kSoLd + kb * 32 + 8 * g);
 #pragma unroll
-                for (int tt = 0; tt < 8; ++tt) {
-                    if (MODE == 2 && (tt < tt_lo || tt >= tt_hi)) continue;
-                    const f16x8_t b = *(const f16x8_t*)(xo + (tt * 16 + c) * kOutChunk + kb * 32 + 8 * g);
+                for (int tt = 0; tt < kTT; ++tt) {
+                    const f16x8_t b = *(const f16x8_t*)(xo + ((tt0 + tt) * 16 + c) * kOutChunk + kb * 32 + 8 * g);
 #pragma unroll
                     for (int t = 0; t < kTPW; ++t) o[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b, o[t][tt], 0, 0, 0);
                 }
@@ -381,16 +588,31 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
 #pragma unroll
         for (int t = 0; t < kTPW; ++t)
 #pragma unroll
-            for (int tt = 0; tt < 8; ++tt)
+            for (int tt = 0; tt < kTT; ++tt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r(d[t][tt][r] + f16r(o[t][tt][r]));
+    } else {
+        dequant();
     }
+    // four consecutive output columns per lane and tile: one 16-B (f32) / 8-B (bf16, f16) access when the row allows it
+    const bool vec = (p.N & 3) == 0 && (p.ldy & 3) == 0 && ((uintptr_t)p.y & 15) == 0;
+    constexpr int kOld = kTT < 2 ? kTT : 2;
+    [[maybe_unused]] f32x4 old[kTPW][kOld];  // ACCUM, f32 rows: of kOld token tiles at a time
 #pragma unroll
-    for (int tt = 0; tt < 8; ++tt) {
-        const int m = m0 + tt * 16 + c;
-        if (m >= p.M || tt < tt_lo || tt >= tt_hi) continue;
-        // four consecutive output columns per lane and tile: one 16-B (f32) / 8-B (bf16, f16) access when the row allows it
-        const bool vec = (p.N & 3) == 0 && (p.ldy & 3) == 0 && ((uintptr_t)p.y & 15) == 0;
+    for (int tt = 0; tt < kTT; ++tt) {
+        const int m = m0 + (tt0 + tt) * 16 + c;
+        if constexpr (EPI == MI355_EPI_ACCUM) {
+            if (tt % kOld == 0 && vec && p.y_dtype == MI355_F32) {
+#pragma unroll
+                for (int i = 0; i < kOld; ++i)
+#pragma unroll
+                    for (int t = 0; t < kTPW; ++t) {
+                        const int mi = m + 16 * i, n = tile[t] * 16 + 4 * g;
+                        old[t][i] = *(const f32x4*)((const float*)p.y + (mi < p.M && tile[t] < p.n_tiles && n < p.N ? (int64_t)mi * p.ldy + n : 0));
+                    }
+            }
+        }
+        if (m >= p.M) continue;
         if constexpr (EPI == MI355_EPI_SWIGLU) {
 #pragma unroll
             for (int t = 0; t < kTPW; t += 2) {
@@ -418,7 +640,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                 const int64_t yi = (int64_t)m * p.ldy + n;
                 if (vec && p.y_dtype == MI355_F32) {
                     f32x4 o = {d[t][tt][0], d[t][tt][1], d[t][tt][2], d[t][tt][3]};
-                    if constexpr (EPI == MI355_EPI_ACCUM) o += *(const f32x4*)((const float*)p.y + yi);
+                    if constexpr (EPI == MI355_EPI_ACCUM) o += old[t][tt % kOld];
                     *(f32x4*)((float*)p.y + yi) = o;
                 } else if (vec && p.y_dtype == MI355_BF16) {
                     float o[4] = {d[t][tt][0], d[t][tt][1], d[t][tt][2], d[t][tt][3]};
@@ -456,7 +678,7 @@ int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
         return (int)attr_err;
     }
     I8GemmParams r = q;
-    r.per_xcd = (q.total_blocks * (MODE == 1 ? q.ksplit : MODE == 2 ? 8 : 1) + 7) / 8;
+    r.per_xcd = (q.total_blocks * (MODE == 1 ? q.ksplit + 1 : MODE == 2 ? 8 : 1) + 7) / 8;
     hipLaunchKernelGGL((i8_gemm_kernel<EPI, PAIR, MODE>), dim3(8 * r.per_xcd), dim3(kThreads), kLds, s, r);
     MI355_LAUNCH_CHECK();
     return 0;
@@ -481,7 +703,8 @@ extern "C" size_t mi355_linear_int8_gemm_workspace_bytes(int M, int K) {
     const size_t kp = ((size_t)K + 127) / 128 * 128;
     // xh f16 [M, Kp], CA int8 [M, Kp], absmax [M], column mask [Kp / 32], outlier list [1 + Kp]
     return pad16((size_t)M * kp * 2) + pad16((size_t)M * kp) + pad16((size_t)M * 4) + pad16(kp / 8) + pad16((1 + kp) * 4) + 256 +
-           kSplitBudget;  // int32 partial tiles of the split-K launches (short prompts)
+           kPartBytes +                                      // partial tiles of the split-K launches (short prompts)
+           pad16((size_t)M * kp * 2) + kOutlierBudget;       // outlier columns by themselves: of the rows, of the weights
 }
 
 extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace, size_t workspace_bytes, mi355_stream_t stream) {
@@ -514,6 +737,10 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     int* olist = (int*)ws;
     ws += pad16((size_t)(1 + kp) * 4);
     int* part = (int*)ws;
+    ws += kPartBytes;
+    f16_t* xo = (f16_t*)ws;
+    ws += pad16((size_t)a->M * kp * 2);
+    f16_t* so = (f16_t*)ws;
     // split-K: launches of fewer than 96 blocks are cut into up to 8 K-slices (as many as fit the partial buffer)
     int ksplit = 1;
     const int64_t ldp = (int64_t)a->N * (swiglu ? 2 : 1);
@@ -527,10 +754,14 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     // (a kernel, not hipMemsetAsync: a caller may capture this launch, and memset nodes have replayed wrongly)
     hipLaunchKernelGGL(i8_clear_mask_kernel, dim3((kp / 32 + 255) / 256), dim3(256), 0, s, mask, kp / 32);
     MI355_LAUNCH_CHECK();
-    hipLaunchKernelGGL(i8_stage_kernel, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype, a->eps,
-                       a->threshold, a->K, kp, xh, sca, mask);
-    MI355_LAUNCH_CHECK();
-    hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M), dim3(256), 0, s, xh, sca, mask, kp, ca, olist);
+    auto stage = [&](auto type) {
+        using T = decltype(type);
+        hipLaunchKernelGGL(i8_stage_kernel<T>, dim3(a->M), dim3(256), 0, s, (const T*)a->x, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->threshold, a->K, kp,
+                           xh, sca, mask);
+    };
+    if (a->x_dtype == MI355_F32) stage(float{});
+    else if (a->x_dtype == MI355_BF16) stage(bf16_t{});
+    else stage(f16_raw{});
     MI355_LAUNCH_CHECK();
     I8GemmParams p;
     memset(&p, 0, sizeof(p));
@@ -558,6 +789,10 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     p.ksplit = ksplit;
     p.ldp = ldp;
     p.part = part;
+    p.xo = xo;
+    p.so = so;
+    hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), 0, s, mask, ca, olist, p, a->R);
+    MI355_LAUNCH_CHECK();
     if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, s);
     if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, s);
     return launch_i8_gemm<MI355_EPI_STORE, false>(p, s);

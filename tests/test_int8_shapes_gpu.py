@@ -1,0 +1,58 @@
+"""LLM.int8 products of many rows where their outlier columns begin and end: none, one, a block of 64 and its neighbours, columns past the first 16 384, more
+than their region holds; cut into K-slices and not."""
+import pytest
+import torch
+
+from lit_llama_amd import _native as nat
+from lit_llama_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(x, cb, scb):
+    """The restated algorithm in 64 bits but for its own roundings: int8 part, outlier part, the latter's terms by size."""
+    xh = x.half().double()
+    big = xh.abs() >= 6
+    cols = big.any(0)
+    sca = xh.masked_fill(big, 0).abs().amax(1)
+    inv = torch.where(sca > 0, torch.full_like(sca, 127.0, dtype=torch.float32) / sca.float(), torch.zeros_like(sca, dtype=torch.float32))
+    ca = torch.round(xh.float() * inv[:, None]).double()
+    ca[:, cols] = 0
+    acc = ca @ cb.double().T
+    main = ((acc.float() * 6.200012e-05) * sca.float()[:, None]) * scb[None, :]
+    w = ((cb[:, cols].float() * scb[:, None]) / torch.full_like(scb, 127.0)[:, None]).half().double()
+    return main.half().float(), xh[:, cols] @ w.T, xh[:, cols].abs() @ w.abs().T
+
+
+@pytest.mark.parametrize("M,N,K,outliers", [
+    (33, 72, 200, 1), (64, 4096, 4096, 63), (200, 4096, 4096, 64), (130, 1000, 1024, 65), (257, 4096, 11008, 700), (48, 4096, 22016, 300),
+    (1030, 4096, 640, 129), (2050, 1040, 512, 33), (40, 11008, 4096, 4096), (512, 4096, 1024, 0),
+])
+@pytest.mark.parametrize("epi", ["store", "accum", "pair"])
+def test_outlier_columns(dev, M, N, K, outliers, epi):
+    """Integer sums are exact; the outlier part is an f32 sum of exact products, so its f16 rounding may fall on either side: one f16 step of that part,
+    and one of the sum that it moves; 2^-22 of its terms' sizes for the sum itself."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K + outliers)
+    x = torch.randn((M, K), generator=g, device=dev).clamp_(-5.9, 5.9)
+    at = torch.randperm(K, generator=g, device=dev)[:outliers]
+    x[torch.randint(0, M, (outliers,), generator=g, device=dev), at] = 6.0 + 2 * torch.rand(outliers, generator=g, device=dev)
+    x = x.to(torch.bfloat16)
+    mats = [ops.int8_quant_rows(torch.randn((N, K), generator=g, device=dev) * K ** -0.5) for _ in range(2 if epi == "pair" else 1)]
+    stream = ops.repack_i8(mats[0][0], mats[1][0] if epi == "pair" else None, len(mats))
+    parts = [_reference(x, *m) for m in mats]
+    refs = [(a + b.half().float()).half().float() for a, b, _ in parts]
+    tols = [2.0 ** -10 * (b.abs().float() + r.abs()) + 2.0 ** -24 + 2.0 ** -22 * s.float() for (_, b, s), r in zip(parts, refs)]
+    if epi == "pair":
+        got = ops.linear_int8_gemm(x, stream, mats[0][1], 2, N, K, scb2=mats[1][1], epi=nat.EPI_SWIGLU, out_dtype=torch.float32)
+        ref = torch.nn.functional.silu(refs[0]) * refs[1]
+        tol = 1.1 * (tols[0] * refs[1].abs() + tols[1] * refs[0].abs()) + 1e-6 + 1e-6 * ref.abs()
+    elif epi == "accum":
+        base = torch.randn((M, N), generator=g, device=dev)
+        got = ops.linear_int8_gemm(x, stream, mats[0][1], 1, N, K, epi=nat.EPI_ACCUM, out=base.clone())
+        ref, tol = base + refs[0], tols[0] + 2.0 ** -22 * (base.abs() + refs[0].abs())
+    else:
+        got = ops.linear_int8_gemm(x, stream, mats[0][1], 1, N, K, out_dtype=torch.float32)
+        ref, tol = refs[0], tols[0]
+    assert bool(((got - ref).abs() <= tol).all())
+    if outliers == 0 and epi == "store":
+        assert torch.equal(got, ref)
