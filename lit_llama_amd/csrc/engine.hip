@@ -129,9 +129,6 @@ void fill_linear_args(mi355_linear_args& a, const mi355_model* m, const mi355_we
 // (128 + level) x run over a whole K-slice in one accumulator, where the row kernel's eight waves sum a part each: with single activations 10^4 times the
 // others (the full-depth fixture with a trained model's statistics) that took the logits from 0.05 to 0.08 of their spread, so short chunks stay there.
 int wide_rows(const mi355_weight& w) {
-#ifdef MI355_GEMM_SWEEP
-    if (const char* e = getenv("MI355_WIDE_ROWS")) return atoi(e);
-#endif
     return w.fmt == MI355_W_BF16 ? 11 : 32;
 }
 bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: int4 / bf16 stream, one scale per row

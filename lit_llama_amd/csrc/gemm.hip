@@ -24,6 +24,8 @@
 //  * operands are staged once per linear by stage_rows_kernel: bf16(norm_scale * x) with RMSNorm's 1/rms kept as a
 //    per-row factor for the epilogue, and the per-row operand sum that undoes the +128 / zero-point offset:
 //        y[m, n] = scale[n] * (acc[m, n] - (128 + zero[n]) * sum_k xb[m, k]) * rinv[m]      (same arithmetic as gemv.hip).
+#include <type_traits>
+
 #include <stdlib.h>
 
 #include "common.h"
@@ -105,10 +107,10 @@ struct GemmParams {
     int slice_blocks;      // != 0: row blocks [i slice_blocks, (i + 1) slice_blocks) read the operand at xb + i slice_stride
     int64_t slice_stride;
     // grouped scales (GRP kernels): gtab[group 0..n_groups][r][tab_ld rows] = bf16 scale | bf16 zero << 16 (row n_groups
-    // is all zero), sxt[group][M] = operand sums per group; upg = 128-column units per group (groups of >= 128 columns)
+    // is all zero).  Groups of 2^gq_shift units: sxt[unit][M] = operand sums per unit; of 32 << gq_shift columns (GRP 2): sxt[group][M]
     const uint32_t* gtab;
     const float* sxt;
-    int n_groups, gq_shift, upg, tab_ld;
+    int n_groups, gq_shift, tab_ld;
     // producer / consumer fusion (gemm_fuse.h; FUSE kernels only).  f_in: xb is the caller's operand, 1/rms and the operand
     // sums of the block's rows are rebuilt from the partial sums in_ss / in_sx ([partial][M])
     int f_in, in_sx_n, in_ss_n, in_ppu;  // in_ppu: partial operand sums per 128-column unit (a K-slice sums its own units' shares)
@@ -199,57 +201,85 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dt
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
 }
 
-// grouped scales: as stage_rows_kernel, but sxt[grp][m] = sum of xb over the group's input columns.  A wave per group
-// (wave reductions only); one row per workgroup
-__global__ __launch_bounds__(256) void stage_rows_grouped_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale,
-                                                                 int norm_dtype, float eps, int K, int Kp, bf16_t* xb,
-                                                                 int64_t ldxb, float* rinv, float* sxt, int M, int group_cols,
-                                                                 int n_groups) {
-    __shared__ float red[32];
-    const int m = blockIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float ss = 0.f;
-    for (int grp = wave; grp < n_groups; grp += 4) {
-        const int k_lo = grp * group_cols;
-        const int k_hi = k_lo + group_cols < Kp ? k_lo + group_cols : Kp;
-        float sum = 0.f;
-        for (int k = k_lo + lane; k < k_hi; k += 64) {
-            bf16_t o = 0;
-            if (k < K) {
-                float v = ld_as_f32(x, (int64_t)m * ldx + k, x_dtype);
-                if (norm_scale != nullptr) {
-                    ss += v * v;
-                    v *= ld_as_f32(norm_scale, k, norm_dtype);
-                }
-                o = bf16_hw(v);
-                sum += bf16_to_f32(o);
-            }
-            xb[(int64_t)m * ldxb + k] = o;
-        }
-        sum = wave_sum(sum);
-        if (lane == 0) sxt[(int64_t)grp * M + m] = sum;
+// grouped scales: as stage_rows_kernel, but sxt[i][m] = sum of xb over columns [i * cols, (i + 1) * cols), cols = 32, 64 or 128 (K: whole 128-column units);
+// four columns per lane, one row per workgroup.  The workgroups behind the M rows lay out the tables, [N][n_groups] bf16 scales / zeros -> gtab[grp][r][n]
+// dwords (n fastest: the four rows a lane holds are one 16-B load; row n_groups and the rows past N are zero), a 64 x 64 piece each through LDS.
+// A lane per column and wave per group took 17 us for 1000 x 4096 f32, the tables 5 us in a launch of their own; together they take 9.
+struct GroupTables {
+    const bf16_t *s0, *z0, *s1, *z1;
+    int N, tab_ld, n_groups, R;
+    uint32_t* out;
+    __host__ __device__ int row_pieces() const { return (tab_ld + 63) / 64; }
+    __host__ __device__ int pieces() const { return R * row_pieces() * ((n_groups + 64) / 64); }
+};
+__device__ __forceinline__ void group_table_piece(const GroupTables& t, int piece, uint32_t* lds) {  // lds: 64 x 65
+    const int rp = t.row_pieces(), r = piece % t.R, n0 = piece / t.R % rp * 64, g0 = piece / t.R / rp * 64;
+    const bf16_t* s = r == 1 ? t.s1 : t.s0;
+    const bf16_t* z = r == 1 ? t.z1 : t.z0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int row = i * 4 + ((int)threadIdx.x >> 6), col = threadIdx.x & 63;
+        const bool in = n0 + row < t.N && g0 + col < t.n_groups;
+        const int64_t at = in ? (int64_t)(n0 + row) * t.n_groups + g0 + col : 0;
+        const uint32_t v = s[at] | ((uint32_t)z[at] << 16);
+        lds[row * 65 + col] = in ? v : 0u;
     }
-    for (int k = n_groups * group_cols + (int)threadIdx.x; k < Kp; k += 256) xb[(int64_t)m * ldxb + k] = 0;
-    const float tss = block_sum(ss, red);
-    if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) : 1.0f;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int grp = g0 + i * 4 + ((int)threadIdx.x >> 6), n = n0 + (threadIdx.x & 63);
+        if (grp <= t.n_groups && n < t.tab_ld) t.out[((int64_t)grp * t.R + r) * t.tab_ld + n] = lds[(threadIdx.x & 63) * 65 + (grp - g0)];
+    }
 }
-
-// the reference's [N, n_groups] bf16 scale / zero tables -> gtab[grp][r][n] dwords (n fastest: the four rows a lane holds
-// are one 16-B load); row n_groups and the rows past N are zero
-__global__ __launch_bounds__(256) void group_table_kernel(const bf16_t* s0, const bf16_t* z0, const bf16_t* s1, const bf16_t* z1,
-                                                          int N, int tab_ld, int n_groups, int R, uint32_t* gtab) {
-    const int64_t total = (int64_t)(n_groups + 1) * R * tab_ld;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int n = (int)(i % tab_ld);
-        const int64_t gr = i / tab_ld;
-        const int r = (int)(gr % R), grp = (int)(gr / R);
-        uint32_t v = 0;
-        if (n < N && grp < n_groups) {
-            const int64_t src = (int64_t)n * n_groups + grp;
-            v = (uint32_t)(r == 1 ? s1 : s0)[src] | ((uint32_t)(r == 1 ? z1 : z0)[src] << 16);
+template <bool WIDE>  // rows and norm scale in whole aligned groups of four
+__global__ __launch_bounds__(256) void stage_rows_grouped_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale, int norm_dtype, float eps,
+                                                                 int K, bf16_t* xb, float* rinv, float* sxt, int M, int cols, const GroupTables tables) {
+    __shared__ uint32_t lds[64 * 65];
+    if ((int)blockIdx.x >= M) return group_table_piece(tables, blockIdx.x - M, lds);
+    const int m = blockIdx.x;
+    auto load4 = [&](const void* src, int64_t at, int dtype) {
+        f32x4 v;
+        if constexpr (WIDE) {
+            if (dtype == MI355_F32) return *(const f32x4*)((const float*)src + at);
+            const u32x2 w = *(const u32x2*)((const bf16_t*)src + at);
+            return f32x4{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u)};
         }
-        gtab[i] = v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ld_as_f32(src, at + j, dtype);
+        return v;
+    };
+    constexpr int kAhead = 4;
+    float ss = 0.f;
+    for (int k0 = threadIdx.x * 4; k0 < K; k0 += 1024 * kAhead) {
+        f32x4 v[kAhead], ns[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) v[i] = load4(x, (int64_t)m * ldx + (k0 + i * 1024 < K ? k0 + i * 1024 : k0), x_dtype);
+        if (norm_scale != nullptr) {
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) ns[i] = load4(norm_scale, k0 + i * 1024 < K ? k0 + i * 1024 : k0, norm_dtype);
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            const int k = k0 + i * 1024;
+            if (k >= K) break;  // (whole 128-column units: the 32 lanes of one leave together)
+            if (norm_scale != nullptr) {
+                ss += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
+                v[i] *= ns[i];
+            }
+            bf16_t o[4];
+            float sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                o[j] = bf16_hw(v[i][j]);
+                sum += bf16_to_f32(o[j]);
+            }
+            *(u32x2*)(xb + (int64_t)m * K + k) = u32x2{o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16)};
+            sum = group_sum(sum, cols >> 2);
+            if (k % cols == 0) sxt[(int64_t)(k / cols) * M + m] = sum;
+        }
     }
+    const float tss = block_sum(ss, (float*)lds);
+    if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) : 1.0f;
 }
 
 // o += the K-slices' four values at row[0 .. 3], `stride` floats apart, in slice order.  All slices are requested before the first one is added: a
@@ -608,20 +638,20 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 // FMT = MI355_W_Q4: int4 stream, one 1-KiB piece per (tile, unit), converted below; MI355_W_BF16: unquantised weights
 // four 1-KiB pieces per (tile, unit) whose piece d IS the A fragment of k-quarter d — same k
 // order as the int4 conversion produces, no conversion, scale 1 / zero-point 0 in the epilogue
-// GRP (Q4): 0 one (scale, zero) pair per output row; 1 / 2: one pair per row and group of input columns (GPTQ "groupsize",
-// /root/reference lit_llama/quantization.py:284-333 with tile_cols > 0), groups of whole 128-column units (1) or of 32 / 64
-// columns (2).  The MFMA accumulators keep running over K (cum_g = columns up to the end of group g) and at every group
+// GRP (Q4): 0 one (scale, zero) pair per output row; 2: one pair per row and group of 32 or 64 input columns (GPTQ "groupsize",
+// /root/reference lit_llama/quantization.py:284-333 with tile_cols > 0; groups of whole units: gemm_deep_kernel).  The MFMA accumulators keep running over K (cum_g =
+// columns up to the end of group g) and at every group
 // end     accf += (s_g - s_{g+1}) cum_g - s_g (128 + z_g) X_g      (Abel summation of sum_g s_g (A_g - (128 + z_g) X_g),
 // s past the last group = 0; X_g = the group's operand sum from stage_rows_grouped_kernel): two FMAs per output element
 // and group, no accumulator reset.  The k columns of ONE MFMA are spread over the unit (lane group g holds columns
-// 32 g + 8 d ..), so sub-unit groups take one pass per group with the other lane groups' activations zeroed, as in gemv.hip.
+// 32 g + 8 d ..), so a unit takes one pass per group with the other lane groups' activations zeroed, as in gemv.hip.
 // FUSE: the producer / consumer fusion of gemm_fuse.h (ungrouped launches without a K split): operand sums and 1/rms from
 // partial sums instead of the staging pass; the residual epilogue emits the next linear's bf16 operand and its partial
 // sums, the SwiGLU epilogue the partial operand sums of its output, the c_attn epilogue rotates k and writes the K / V cache
 // (second launch-bound argument, waves per SIMD: BF16 streams at 128 VGPRs keep two workgroups per CU, at 132-138 the 2048-token c_fc1/c_fc2 product took
-// 300 us instead of 256; grouped scales at 168 keep three)
+// 300 us instead of 256)
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
-__global__ __launch_bounds__(64 * kWaves, GRP == 1 && kWaves == 4 ? 3 : (FMT == MI355_W_BF16 && BM == 128) ? 4 : 1) void gemm_q4_kernel(const GemmParams p) {
+__global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4 : 1) void gemm_q4_kernel(const GemmParams p) {
     static_assert(GRP == 0 || FMT == MI355_W_Q4, "grouped scales are a Q4 feature");
     static_assert(!FUSE || GRP == 0, "the fused chain runs over per-row scales");
     constexpr int kTT = BM / 16;                   // 16-token tiles per block
@@ -655,10 +685,7 @@ __global__ __launch_bounds__(64 * kWaves, GRP == 1 && kWaves == 4 ? 3 : (FMT == 
     float* fr = (float*)(smem + 2 * BM * 256);  // [BM] 1/rms, [BM] operand sums of the block's tokens
     [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM>);            // FUSE, STORE: [BM] positions
     [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE>);  // [scale, 128 + zero, next norm's scale][rows of the block]
-    // K-slice: units [u_lo, u_hi); GRP 1 cuts at group boundaries (groups [g_lo, g_hi) of upg units each)
-    const int g_lo = GRP == 1 ? slice_lo(ks, p.n_groups, p.ksplit) : 0, g_hi = GRP == 1 ? slice_lo(ks + 1, p.n_groups, p.ksplit) : 0;
-    const int u_lo = GRP == 1 ? g_lo * p.upg : slice_lo(ks, p.units, p.ksplit);
-    const int u_hi = GRP == 1 ? (g_hi * p.upg < p.units ? g_hi * p.upg : p.units) : slice_lo(ks + 1, p.units, p.ksplit);
+    const int u_lo = slice_lo(ks, p.units, p.ksplit), u_hi = slice_lo(ks + 1, p.units, p.ksplit);  // K-slice
 
     // this wave's row tiles
     int tile[kTPW], rr[kTPW];
@@ -1029,36 +1056,20 @@ __global__ __launch_bounds__(64 * kWaves, GRP == 1 && kWaves == 4 ? 3 : (FMT == 
             for (int t = 0; t < kTPW; ++t) tabc[t] = tabn[t];
         };
         // (a K-slice is a sum of its own: past its last group the scale is 0 — table row n_groups)
-        if constexpr (GRP == 1) {
-            tload(g_lo, tabc);
-            int u = u_lo;
-            for (int grp = g_lo; grp < g_hi; ++grp) {
-                tload(grp + 1 < g_hi ? grp + 1 : p.n_groups, tabn);
+        const int sub_shift = p.gq_shift;  // lane groups per sub-group = 1 << gq_shift (0: 32 columns, 1: 64)
+        const int nsub = 4 >> sub_shift;
+        tload(u_lo * nsub, tabc);
+        for (int u = u_lo; u < u_hi; ++u) {
+            prefetch(u);
+#pragma unroll 1
+            for (int sub = 0; sub < nsub; ++sub) {
+                const int grp = u * nsub + sub < p.n_groups ? u * nsub + sub : p.n_groups - 1;
+                tload((u == u_hi - 1 && sub == nsub - 1) ? p.n_groups : grp + 1, tabn);
                 sxload(grp);
-                const int u_end = (grp + 1) * p.upg < u_hi ? (grp + 1) * p.upg : u_hi;
-                for (; u < u_end; ++u) {
-                    prefetch(u);
-                    mfmas(u & 1, 0, 0);
-                    rotate(u & 1);
-                }
+                mfmas(u & 1, sub, sub_shift);
                 apply();
             }
-        } else {
-            const int sub_shift = p.gq_shift;  // lane groups per sub-group = 1 << gq_shift (0: 32 columns, 1: 64)
-            const int nsub = 4 >> sub_shift;
-            tload(u_lo * nsub, tabc);
-            for (int u = u_lo; u < u_hi; ++u) {
-                prefetch(u);
-#pragma unroll 1
-                for (int sub = 0; sub < nsub; ++sub) {
-                    const int grp = u * nsub + sub < p.n_groups ? u * nsub + sub : p.n_groups - 1;
-                    tload((u == u_hi - 1 && sub == nsub - 1) ? p.n_groups : grp + 1, tabn);
-                    sxload(grp);
-                    mfmas(u & 1, sub, sub_shift);
-                    apply();
-                }
-                rotate(u & 1);
-            }
+            rotate(u & 1);
         }
     }
 
@@ -1071,9 +1082,9 @@ __global__ __launch_bounds__(64 * kWaves, GRP == 1 && kWaves == 4 ? 3 : (FMT == 
     gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
-// 16 B per lane from `off` of a buffer to 1 KiB of LDS (lane i's bytes at 16 i); out of range: zeros
-__device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, unsigned off) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+// 16 B per lane from `off` + `scalar_off` of a buffer to 1 KiB of LDS (lane i's bytes at 16 i); out of range: zeros
+__device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, unsigned off, int scalar_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, scalar_off, 0, 0);
 }
 
 // The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of any prompt):
@@ -1081,12 +1092,17 @@ __device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, un
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
 // BM: 16 / 32 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH>
+// GRP (Q4, groups of whole 128-column units): the products of a unit start from 0, and accf += s_unit * them, one FMA per output element and unit on the
+// VALU beside the next unit's products; the zero points, accf -= sum over units of s (128 + z) X_unit (X: the unit's operand sums), are a product with K =
+// units / 4 of their own on the f32 MFMA in front of the loop.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
+    static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1 && !FUSE), "grouped scales are a Q4 feature");
+    static_assert(DEPTH == 3 || DEPTH == 4, "units under way + 1");
     constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
     constexpr int kXI = BM / 4 > kWaves ? BM / 4 / kWaves : 1;  // activation requests (1 KiB: four tokens) per wave and unit
-    constexpr int kUnit = kXI + kTPW * kWP;                     // requests per wave and unit
+    constexpr int kUnit = kXI + kTPW * kWP + (GRP ? kTPW : 0);  // requests per wave and unit
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1115,13 +1131,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
         tile[t] = PAIR ? nb * (kSlots / 2) + (kTPW / 2) * wave + (t >> 1) : nb * kSlots + kTPW * wave + t;
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (int)p.w_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rw0 = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, 0, 0x00020000);
     const bf16_t* xbase = p.xb;
     if constexpr (EPI == MI355_EPI_STORE && FMT == MI355_W_BF16 && !FUSE) {
         if (p.slice_blocks != 0) xbase += (int64_t)(nb / p.slice_blocks) * p.slice_stride;
     }
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)(unsigned)((int64_t)p.M * p.ldxb * 2), 0x00020000);
+    const int x_bytes = (int)(unsigned)((int64_t)p.M * p.ldxb * 2);
     const unsigned lane_off = lane * 16;
     // this lane's token and column of its activation requests (waves beyond the block's BM / 4 requests repeat one: the same bytes to the same place)
     unsigned xoff[kXI];
@@ -1134,21 +1148,34 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         xdst[i] = q * 1024;
     }
     u32x4 wr[DEPTH][kTPW][kWP];
-    // request i of unit u: activations first.  Past the slice: nothing is read, zeros go to a buffer that nobody reads
-    auto request = [&](int i, int u, int slot) {
+    [[maybe_unused]] u32x4 tb[GRP ? DEPTH : 1][kTPW];  // (scale, zero) of rows 4 g .. 4 g + 3 in the unit's group
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc((void*)p.gtab, 0, GRP ? (p.n_groups + 1) * (PAIR ? 2 : 1) * p.tab_ld * 4 : 0, 0x00020000);
+    [[maybe_unused]] const int tbstep = (PAIR ? 2 : 1) * p.tab_ld * 4;
+    [[maybe_unused]] int tboff[kTPW];  // (tiles past the last read the first one's)
+#pragma unroll
+    for (int t = 0; t < kTPW; ++t) tboff[t] = ((PAIR ? t & 1 : 0) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + 4 * g) * 4;
+    // request i of unit u: activations first.  What tells the units apart is scalar (offsets, and the size in the descriptor): no address
+    // instruction on the VALU.  Past the slice or the tiles: a size of 0, nothing is read (the scalar offset is not range-checked), zeros go to a buffer that
+    // nobody reads
+    auto request = [&](int i, int u, int slot) __attribute__((always_inline)) {
         const bool in = u < u_hi;
         if (i < kXI) {
-            lds_from(rx, smem + slot * (BM * 256) + xdst[i < kXI ? i : 0], in && xoff[i < kXI ? i : 0] != 0xFFFFFFF0u ? xoff[i < kXI ? i : 0] + (unsigned)u * 256u : 0xFFFFFFF0u);
+            const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, in ? x_bytes : 0, 0x00020000);
+            lds_from(rx, smem + slot * (BM * 256) + xdst[i < kXI ? i : 0], xoff[i < kXI ? i : 0], in ? u * 256 : 0);
+        } else if (i >= kXI + kTPW * kWP) {
+            const int t = i - (kXI + kTPW * kWP) < kTPW ? i - (kXI + kTPW * kWP) : 0;
+            tb[GRP ? slot : 0][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rt, tboff[t], ((in ? u : u_hi - 1) >> p.gq_shift) * tbstep, 0));
         } else {
             const int t = (i - kXI) / kWP, d = (i - kXI) % kWP;
             const bool ok = tile[t] < p.n_tiles && in;
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, ok ? (int)p.w_bytes : 0, 0x00020000);
             const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * (1024u * kWP) + d * 1024u;
-            wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off : 0u, 0));
+            wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane_off, ok ? off : 0u, 0));
         }
     };
 
     // ---- tables of the epilogue: requested ahead of the units, written to LDS behind their requests
-    constexpr bool kScales = FMT == MI355_W_Q4;
+    constexpr bool kScales = FMT == MI355_W_Q4 && GRP == 0;
     constexpr int kRT = (kSlots * 16 + kThreads - 1) / kThreads;
     [[maybe_unused]] float t_sc[kRT], t_zp[kRT], t_ns[kRT];
     if constexpr (kScales) {
@@ -1257,12 +1284,107 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     uint32_t cmask = 0x000F000Fu, cmagic = 0x43004300u;  // (opaque: see gemm_q4_kernel)
     asm volatile("" : "+s"(cmask));
     asm volatile("" : "+v"(cmagic));
+    auto levels = [&](uint32_t v) __attribute__((always_inline)) {  // eight int4 levels as bf16 128 + q
+        return __builtin_bit_cast(bf16x8, u32x4{(v & cmask) | cmagic, ((v >> 4) & cmask) | cmagic, ((v >> 8) & cmask) | cmagic, ((v >> 12) & cmask) | cmagic});
+    };
+    if constexpr (GRP != 0) {
+        // lane (g, c): units u0 + 4 g + i of product i; a chunk's factors are requested while the one before is multiplied
+        struct Chunk { uint32_t sz[4][kTPW]; float x[4][kTT]; };
+        auto fetch = [&](int u0, Chunk& k) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int u = u0 + 4 * g + i < u_hi ? u0 + 4 * g + i : u_hi - 1;
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t)
+                    k.sz[i][t] = p.gtab[((int64_t)(u >> p.gq_shift) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + c];
+#pragma unroll
+                for (int tt = 0; tt < kTT; ++tt) k.x[i][tt] = p.sxt[(int64_t)u * p.M + (m0 + tt * 16 + c < p.M ? m0 + tt * 16 + c : p.M - 1)];
+            }
+        };
+        Chunk cur, nxt;
+        fetch(u_lo, cur);
+        for (int u0 = u_lo; u0 < u_hi; u0 += 16) {
+            fetch(u0 + 16 < u_hi ? u0 + 16 : u0, nxt);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool in = u0 + 4 * g + i < u_hi;
+                float a[kTPW];
+#pragma unroll
+                for (int t = 0; t < kTPW; ++t)
+                    a[t] = in ? -__uint_as_float(cur.sz[i][t] << 16) * (128.f + __uint_as_float(cur.sz[i][t] & 0xffff0000u)) : 0.f;
+#pragma unroll
+                for (int tt = 0; tt < kTT; ++tt) {
+                    const float x = in ? cur.x[i][tt] : 0.f;
+#pragma unroll
+                    for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], x, acc[t][tt], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): registers of a load whose result nobody takes are waited for where they are used next, in the loop
+    }
     constexpr int kFrags = 4 * kTT, kPipe = 4;
     // the requests of unit `ahead` go out between the products: a request takes the CU's memory pipeline 16 cycles, and in one burst behind the barrier
     // the waves of a workgroup stood in line for it with no product under way
     constexpr int kEvery = kFrags >= 2 * kUnit ? kFrags / (2 * kUnit) : 1;  // fragments from one request to the next (all in the first half if it holds them)
     constexpr int kPer = (kUnit + kFrags - 1) / kFrags;                      // requests behind one fragment
-    auto mfmas = [&](int slot, u32x4 (&w)[kTPW][kWP], int ahead, int ahead_slot) {
+    // GRP: token tile by token tile, so the sums of one unit live in two token tiles' registers: those being summed, and those being scaled
+    auto mfmas_grouped = [&](int slot, u32x4 (&w)[kTPW][kWP], u32x4 (&sz)[kTPW], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
+        const char* xs = smem + slot * (BM * 256);
+        auto bread = [&](int f) {  // fragment f = tt * 4 + d
+            const int tok = (f >> 2) * 16 + c;
+            return *(const u32x4*)(xs + tok * 256 + (((4 * g + (f & 3)) ^ swz(tok)) << 4));
+        };
+        u32x4 bq[kPipe];
+#pragma unroll
+        for (int q = 0; q < kPipe; ++q) bq[q] = bread(q);
+        __builtin_amdgcn_sched_group_barrier(0x100, kPipe, 0);
+        bf16x8 a[4][kTPW];
+        f32x4 sc[kTPW];
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                a[d][t] = levels(w[t][0][d]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[t][r] = __uint_as_float(sz[t][r] << 16);
+        }
+        f32x4 un[2][kTPW];
+#pragma unroll
+        for (int f = 0; f < kFrags; ++f) {
+            const int tt = f >> 2, d = f & 3;
+            const bf16x8 b = __builtin_bit_cast(bf16x8, bq[f % kPipe]);
+            if (f + kPipe < kFrags) bq[f % kPipe] = bread(f + kPipe);
+#pragma unroll
+            for (int t = 0; t < kTPW; ++t)
+                un[tt & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b, d == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : un[tt & 1][t], 0, 0, 0);
+            if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
+            if (more && f % kEvery == 0) {
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const int r = f / kEvery * kPer + i;
+                    if (r >= kUnit) continue;
+                    request(r, ahead, ahead_slot);
+                    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+                }
+            }
+            if (tt > 0 && d > 0 && d <= kTPW) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[d - 1][tt - 1][r] = __builtin_fmaf(sc[d - 1][r], un[(tt - 1) & 1][d - 1][r], acc[d - 1][tt - 1][r]);
+                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][kTT - 1][r] = __builtin_fmaf(sc[t][r], un[(kTT - 1) & 1][t][r], acc[t][kTT - 1][r]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mfmas = [&](int slot, u32x4 (&w)[kTPW][kWP], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
         const char* xs = smem + slot * (BM * 256);
         auto bread = [&](int f) {  // fragment f = d * kTT + tt
             const int tok = (f % kTT) * 16 + c;
@@ -1277,17 +1399,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             bf16x8 a[kTPW];
 #pragma unroll
             for (int t = 0; t < kTPW; ++t) {
-                if constexpr (FMT == MI355_W_BF16) {
+                if constexpr (FMT == MI355_W_BF16)
                     a[t] = __builtin_bit_cast(bf16x8, w[t][d]);
-                } else {
-                    const uint32_t v = w[t][0][d];
-                    u32x4 f;
-                    f[0] = (v & cmask) | cmagic;
-                    f[1] = ((v >> 4) & cmask) | cmagic;
-                    f[2] = ((v >> 8) & cmask) | cmagic;
-                    f[3] = ((v >> 12) & cmask) | cmagic;
-                    a[t] = __builtin_bit_cast(bf16x8, f);
-                }
+                else
+                    a[t] = levels(w[t][0][d]);
             }
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) {
@@ -1298,7 +1413,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
                 for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[t][tt], 0, 0, 0);
                 if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
-                if (f % kEvery == 0) {
+                if (more && f % kEvery == 0) {
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) {
                         const int r = f / kEvery * kPer + i;
@@ -1311,14 +1426,32 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    for (int u = u_lo; u < u_hi; u += DEPTH) {
-#pragma unroll
-        for (int s = 0; s < DEPTH; ++s) {
-            if (s > 0 && u + s >= u_hi) break;
-            // own requests of this unit have landed (DEPTH - 2 units are newer); every wave's have, and every wave is done with the unit before: its
-            // buffer and registers take the unit DEPTH - 1 ahead
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((DEPTH - 2) * kUnit) : "memory");
-            mfmas(s, wr[s], u + s + DEPTH - 1, (s + DEPTH - 1) % DEPTH);
+    // DEPTH units a round: own requests of a unit have landed (those of the DEPTH - 2 units behind it may be under way); every wave's have, and every wave is
+    // done with the unit before: its buffer and registers take the unit DEPTH - 1 ahead.  The last, shorter round stands behind the loop and requests nothing:
+    // with a way out between the units hipcc joins all of them in front of the loop's head and waits there for every request under way, once a round.
+    auto unit = [&](auto slot, int u, auto more) __attribute__((always_inline)) {
+        constexpr int s = slot, kNewer = more ? (DEPTH - 2) * kUnit : (DEPTH - 2 - s) * kUnit;
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kNewer) : "memory");
+        if constexpr (GRP != 0)
+            mfmas_grouped(s, wr[s], tb[s], u + DEPTH - 1, (s + DEPTH - 1) % DEPTH, more);
+        else
+            mfmas(s, wr[s], u + DEPTH - 1, (s + DEPTH - 1) % DEPTH, more);
+    };
+    using std::integral_constant;
+    int u = u_lo;
+    for (; u + DEPTH <= u_hi; u += DEPTH) {
+        unit(integral_constant<int, 0>{}, u, std::true_type{});
+        unit(integral_constant<int, 1>{}, u + 1, std::true_type{});
+        unit(integral_constant<int, 2>{}, u + 2, std::true_type{});
+        if constexpr (DEPTH == 4) unit(integral_constant<int, 3>{}, u + 3, std::true_type{});
+    }
+    if (u < u_hi) {
+        unit(integral_constant<int, 0>{}, u, std::false_type{});
+        if (u + 1 < u_hi) {
+            unit(integral_constant<int, 1>{}, u + 1, std::false_type{});
+            if constexpr (DEPTH == 4) {
+                if (u + 2 < u_hi) unit(integral_constant<int, 2>{}, u + 2, std::false_type{});
+            }
         }
     }
     if constexpr (FUSE) {
@@ -1350,7 +1483,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests past the slice wrote zeros: none may land in what the epilogue keeps there)
     __syncthreads();
-    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, 0, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
+    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
 template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, typename Kernel>
@@ -1389,17 +1522,17 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     }
     return 0;
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0>
 int launch_deep(const GemmParams& p, hipStream_t s) {
     constexpr int kDepth = BM == 128 && FMT == MI355_W_BF16 ? 3 : 4;
     constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64;
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth>,
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth>, kLds, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP>, kLds, p, s);
 }
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
 int launch_gemm_w(const GemmParams& p, hipStream_t s) {
@@ -1435,8 +1568,14 @@ GemmForce gemm_force() {
 }
 // Waves of a block (what the share layout of mi355_linear_gemm_plan depends on).  Up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them,
 // which 4-5 K-slices bring to a workgroup for two CUs of three; 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, int4 with staging:
-// 20.5 us against 22.7).
-int gemm_waves(int M) { return gemm_force().waves ? gemm_force().waves : M <= 64 ? 4 : 8; }
+// 20.5 us against 22.7).  Longer int4 prompts likewise while the 256-row blocks leave half of the CUs idle, except where the 128-row blocks of a launch without
+// slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096, 128 tokens 29.3 / 24.5 us, 512 38.9 / 32.0; N = 12288, 128 tokens 34.6 / 29.6;
+// K = 11008, 300 tokens 57.5 / 64.0, 512 71.2 / 66.7).  The SwiGLU pair does not gain (128 tokens 36.5 / 39.4).
+int gemm_waves(int M, int N, bool pair, bool bf16) {
+    if (gemm_force().waves) return gemm_force().waves;
+    const int blocks8 = (N + 255) / 256 * ((M + 63) / 64);
+    return M <= 64 || (!bf16 && !pair && (blocks8 <= 64 || (blocks8 >= 96 && blocks8 <= 128))) ? 4 : 8;
+}
 // Tokens per block and kernel.  Blocks of 128 tokens x 256 rows with two workgroups per CU (gemm_q4_kernel) when a launch has a few of them per CU: 2048
 // tokens, int4, c_fc1/c_fc2 271 us against 303 (gemm_deep_kernel, one workgroup per CU), c_attn 158 / 174.  Fewer: 64-token blocks, twice as many, of the
 // deep kernel: 128 tokens, int4, c_fc1/c_fc2 49.6 -> 39.9 us, 777 tokens N = 4096 47.8 -> 42.1 us.  An int4 launch of exactly one 128-token block per CU (N = 4096
@@ -1445,12 +1584,35 @@ int gemm_waves(int M) { return gemm_force().waves ? gemm_force().waves : M <= 64
 // kernel: 2048 tokens, N = 4096, K = 11008 174 -> 158 us.
 GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16) {
     const GemmForce fo = gemm_force();
-    GemmShape sh = {gemm_waves(M), M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
+    GemmShape sh = {gemm_waves(M, n_tiles * 16, pair, bf16), M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
     const int per_block8 = pair ? 8 * kTPW / 2 : 8 * kTPW;
     const int blocks8 = ((n_tiles + per_block8 - 1) / per_block8) * ((M + kBM - 1) / kBM) * ksplit;  // of 128 tokens
     if (bf16 ? M > 128 && blocks8 >= 160 : blocks8 >= 384 || blocks8 == 256) sh.bm = 128, sh.deep = bf16 && blocks8 <= 256;
     if (fo.bm) sh.bm = fo.bm;
     if (fo.deep) sh.deep = fo.deep == 1;
+    return sh;
+}
+// Grouped scales, groups of whole units.  Blocks of 256 rows x 64 tokens and of 256 x 128 fill a CU alone, two of 128 x 64 share one; per round of the chip
+// they take 1 : 1.75 : 1, a round of at most one 128 x 64 block per CU 0.75 (N = 4096, K = 11008: 256 x 64 blocks 104 us at 512 tokens, 106 at 777, 108 at 1000;
+// 256 x 128 165 / 168 / 169; 128 x 64 78 / 106 / 114): the fewest.  1000 tokens, 7B: 235 / 101 / 137 us for c_fc1 / c_fc2, c_proj on average, c_attn with blocks
+// of 64 x 128 one unit ahead -> 185 / 75 / 120.
+GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
+    const GemmForce fo = gemm_force();
+    GemmShape sh = {4, M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
+    if (M > 64) {
+        auto blocks = [&](int waves, int bm) {
+            const int per_block = pair ? waves * kTPW / 2 : waves * kTPW;
+            return (n_tiles + per_block - 1) / per_block * ksplit * ((M + bm - 1) / bm);
+        };
+        const int half = blocks(4, 64), full = blocks(8, 64), wide = blocks(8, 128);
+        const int t_half = half / 512 * 4 + (half % 512 == 0 ? 0 : half % 512 <= 256 ? 3 : 4), t_full = (full + 255) / 256 * 4, t_wide = (wide + 255) / 256 * 7;
+        if (t_wide < t_half && t_wide <= t_full)
+            sh = {8, 128, true};
+        else if (t_full <= t_half)
+            sh.waves = 8;
+    }
+    if (fo.waves) sh.waves = fo.waves;
+    if (fo.bm) sh.bm = fo.bm;
     return sh;
 }
 // Split-K of an ungrouped launch: as many slices as bring it to the workgroups wanted, none below 6 units (BF16: 4) or past the partial buffer.  BF16, whose
@@ -1462,7 +1624,7 @@ int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
     if (const int fk = gemm_force().ksplit) {
         if (fk >= 1 && fk <= kMaxSplit && units >= fk && (size_t)2 * fk * M * row_floats * 4 <= kSplitBudget) return fk;
     }
-    const int waves = gemm_waves(M);
+    const int waves = gemm_waves(M, N, pair, bf16);
     const int rows_per_block = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
     const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), want = waves == 8 ? 192 : bf16 ? 400 : 160;
     int ksplit = 1;
@@ -1481,28 +1643,31 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
     if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
     return launch_gemm_w<EPI, PAIR, FMT, 8, kBM, 0, FUSE>(p, s);
 }
-// grouped scales: blocks of 64 tokens x 4 waves (the second accumulator set costs the registers of more tokens or waves);
-// from kGrpWideM tokens on, 128 tokens x 8 waves (2048-token g128 prompt 41.9 -> 39.4 ms; at 512 tokens it is the slower
-// one, 16.3 -> 17.6 ms, at 1024 22.5 -> 27.3 ms, and 64 x 8 / 128 x 4 lose everywhere: profiles/r06_ab_grouped_prompt.txt)
-constexpr int kGrpBM = 64;
-constexpr int kGrpWideM = 2048;
-template <int EPI, bool PAIR, int GRP>
-int launch_gemm_grouped(const GemmParams& p, hipStream_t s) {
+// grouped scales.  Groups of 32 or 64 columns: blocks of 64 tokens x 4 waves (the second accumulator set costs the registers of more tokens or waves).
+template <int EPI, bool PAIR>
+int launch_gemm_subgroups(const GemmParams& p, hipStream_t s) {
     const int per_block8 = PAIR ? 8 * kTPW / 2 : 8 * kTPW;
-    const int blocks8 = ((p.n_tiles + per_block8 - 1) / per_block8) * ((p.M + kGrpBM - 1) / kGrpBM);
-    if (p.ksplit > 1) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 4, 64, GRP>(p, s);
-    if constexpr (GRP == 1) {  // groups below a unit (GRP 2) carry masked passes: 128 x 8 does not fit their registers
-        if (blocks8 >= 128 && p.M >= kGrpWideM) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 8, 128, GRP>(p, s);
-    }
-    if (blocks8 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 4, kGrpBM, GRP>(p, s);
-    if (blocks8 * 4 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 2, 64, GRP>(p, s);
-    return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 1, 64, GRP>(p, s);
+    const int blocks8 = ((p.n_tiles + per_block8 - 1) / per_block8) * ((p.M + 63) / 64);
+    if (p.ksplit > 1 || blocks8 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 4, 64, 2>(p, s);
+    if (blocks8 * 4 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 2, 64, 2>(p, s);
+    return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 1, 64, 2>(p, s);
 }
-template <int GRP>
-int launch_gemm_grouped_epi(const GemmParams& p, int epi, hipStream_t s) {
-    if (epi == MI355_EPI_SWIGLU) return launch_gemm_grouped<MI355_EPI_SWIGLU, true, GRP>(p, s);
-    if (epi == MI355_EPI_ACCUM) return launch_gemm_grouped<MI355_EPI_ACCUM, false, GRP>(p, s);
-    return launch_gemm_grouped<MI355_EPI_STORE, false, GRP>(p, s);
+template <int EPI, bool PAIR>
+int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
+    if (subgroups) return launch_gemm_subgroups<EPI, PAIR>(p, s);
+    const GemmShape sh = gemm_shape_grouped(p.n_tiles, p.M, PAIR, p.ksplit);
+    if (sh.waves == 4) {
+        if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, false, 1>(p, s);
+        if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, false, 1>(p, s);
+        return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 64, false, 1>(p, s);
+    }
+    if (sh.bm == 64) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 64, false, 1>(p, s);
+    return launch_deep<EPI, PAIR, MI355_W_Q4, 8, kBM, false, 1>(p, s);
+}
+int launch_gemm_grouped_epi(const GemmParams& p, int epi, bool subgroups, hipStream_t s) {
+    if (epi == MI355_EPI_SWIGLU) return launch_gemm_grouped<MI355_EPI_SWIGLU, true>(p, subgroups, s);
+    if (epi == MI355_EPI_ACCUM) return launch_gemm_grouped<MI355_EPI_ACCUM, false>(p, subgroups, s);
+    return launch_gemm_grouped<MI355_EPI_STORE, false>(p, subgroups, s);
 }
 template <int FMT, bool FUSE>
 int launch_gemm_epi(const GemmParams& p, int epi, hipStream_t s) {
@@ -1515,14 +1680,17 @@ int launch_gemm_epi(const GemmParams& p, int epi, hipStream_t s) {
     return launch_gemm<MI355_EPI_STORE, false, FMT, FUSE>(p, s);
 }
 
+// floats from the 1/rms of the staged rows to their operand sums per unit
+size_t unit_sums_at(int M) { return (size_t)M * (1 + kMaxSplit); }
+
 }  // namespace
 
 extern "C" size_t mi355_linear_gemm_workspace_bytes(int M, int K) {
     if (M <= 0 || K <= 0) return 0;
     const size_t kp = ((size_t)K + 127) / 128 * 128;
-    // staged operands, 1/rms, per-slice operand sums, split-K partials (used when a launch would be a few dozen blocks)
+    // staged operands, 1/rms, per-slice operand sums, operand sums per unit, split-K partials (used when a launch would be a few dozen blocks)
     // ... and, at the very end, the partial sums of the fused prompt chain (gemm_fuse.h)
-    return (size_t)M * kp * 2 + (size_t)M * 4 * (1 + kMaxSplit) + 256 + kSplitBudget + kFuseScratch;
+    return (size_t)M * kp * 2 + unit_sums_at(M) * 4 + (size_t)M * (kp / 128) * 4 + 256 + kSplitBudget + kFuseScratch;
 }
 
 size_t mi355_linear_gemm_fuse_scratch_bytes() { return kFuseScratch; }
@@ -1537,7 +1705,8 @@ void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, 
     const int ks = gemm_ksplit(M, N, K, pair, bf16);
     // rows (hidden rows of a pair stream) behind one share of a producer's partial sums: a 128-column unit when the K-slices'
     // reduction writes them or a block holds 256 rows, else the block's rows
-    int rows = (pair ? gemm_waves(M) * kTPW / 2 : gemm_waves(M) * kTPW) * 16;
+    const int waves = gemm_waves(M, N, pair, bf16);
+    int rows = (pair ? waves * kTPW / 2 : waves * kTPW) * 16;
     if (ks > 1 || rows > 128) rows = 128;
     *ksplit = ks;
     *shares = (N + rows - 1) / rows;
@@ -1592,7 +1761,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
         n_groups = (a->K + a->group_cols - 1) / a->group_cols;
         tab_ld = (a->N + 15) / 16 * 16;
         tab_bytes = ((size_t)(n_groups + 1) * a->R * tab_ld * 4 + 15) & ~(size_t)15;
-        sxt_bytes = (size_t)n_groups * a->M * 4;
+        sxt_bytes = (size_t)n_groups * a->M * 4;  // (of groups of whole units: in a place of their own)
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
         // blocks of 8 row tiles x 64 tokens; slices of whole groups (>= 4 per slice), partials in the first half of the
@@ -1632,7 +1801,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
                                                a->N == 3 * f->n_head * f->hs),
                         MI355_E_ARG, "linear_gemm: the K / V cache epilogue is c_attn's (N = 3 n_head x 128, STORE)");
     }
-    float* part = (float*)((char*)workspace + (size_t)a->M * kp * 2 + (size_t)a->M * 4 * (1 + kMaxSplit) + 256);
+    float* part = (float*)((char*)(rinv + unit_sums_at(a->M) + (size_t)a->M * units) + 256);
     part = (float*)(((uintptr_t)part + 15) & ~(uintptr_t)15);
     // a bf16 operand in front of BF16 weights, whole units of it and no norm: multiplied where it lies
     const bool direct = !fused && !q4 && a->norm_scale == nullptr && a->x_dtype == MI355_BF16 && a->K % 128 == 0 && a->ldx % 8 == 0 &&
@@ -1642,22 +1811,18 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     if (grouped) {
         // the group tables live in the split-K region of the workspace (its second half when the launch is split)
         uint32_t* gtab = (uint32_t*)((char*)part + (ksplit > 1 ? kSplitBudget / 2 : 0));
-        float* sxt = (float*)((char*)gtab + tab_bytes);
-        {
-            const int64_t total = (int64_t)(n_groups + 1) * a->R * tab_ld;
-            const int grid = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-            hipLaunchKernelGGL(group_table_kernel, dim3(grid), dim3(256), 0, s, (const bf16_t*)a->scales, (const bf16_t*)a->zeros,
-                               (const bf16_t*)a->scales2, (const bf16_t*)a->zeros2, a->N, tab_ld, n_groups, a->R, gtab);
-            MI355_LAUNCH_CHECK();
-        }
-        hipLaunchKernelGGL(stage_rows_grouped_kernel, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale,
-                           a->norm_dtype, a->eps, a->K, kp, xb, (int64_t)kp, rinv, sxt, a->M, a->group_cols, n_groups);
+        const int cols = a->group_cols >= 128 ? 128 : a->group_cols;
+        float* sxt = cols == 128 ? rinv + unit_sums_at(a->M) : (float*)((char*)gtab + tab_bytes);
+        const GroupTables tables = {(const bf16_t*)a->scales, (const bf16_t*)a->zeros, (const bf16_t*)a->scales2, (const bf16_t*)a->zeros2, a->N, tab_ld, n_groups, a->R, gtab};
+        const bool wide = ((uintptr_t)a->x | (uintptr_t)a->norm_scale) % 16 == 0 && a->ldx % 4 == 0;
+        auto stage = wide ? stage_rows_grouped_kernel<true> : stage_rows_grouped_kernel<false>;
+        hipLaunchKernelGGL(stage, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv,
+                           sxt, a->M, cols, tables);
         MI355_LAUNCH_CHECK();
         p.gtab = gtab;
         p.sxt = sxt;
         p.n_groups = n_groups;
-        p.gq_shift = gq_shift;
-        p.upg = a->group_cols >= 128 ? a->group_cols / 128 : 1;
+        p.gq_shift = a->group_cols >= 128 ? gq_shift - 2 : gq_shift;
         p.tab_ld = tab_ld;
     } else if (!f_in && !direct) {
         hipLaunchKernelGGL(stage_rows_kernel, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype,
@@ -1703,7 +1868,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     p.y_dtype = a->y_dtype;
     p.ksplit = ksplit;
     p.part = part;
-    if (grouped) return a->group_cols >= 128 ? launch_gemm_grouped_epi<1>(p, a->epi, s) : launch_gemm_grouped_epi<2>(p, a->epi, s);
+    if (grouped) return launch_gemm_grouped_epi(p, a->epi, a->group_cols < 128, s);
     if (fused) {
         p.f_in = f_in ? 1 : 0;
         p.in_sx = f->in_sx;

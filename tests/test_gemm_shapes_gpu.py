@@ -56,6 +56,26 @@ def test_tiled_product_against_64_bits(dev, fmt, M, N, K, epi):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
+@pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,cols", [(1, 16, 256, 128), (16, 144, 2176, 128), (17, 4096, 1280, 256), (33, 12288, 512, 128), (64, 128, 11008, 512), (65, 4096, 4096, 128),
+                                        (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128)])
+def test_tiled_product_of_grouped_scales_against_64_bits(dev, M, N, K, cols, x_dtype):
+    """Groups of whole units: the products of a unit are sums of 128 terms of up to 143 x, the zero points a sum of their own: 1e-3 of the result as above.
+    Rows whose addresses are no multiple of 16 B take the staging pass of single loads."""
+    g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
+    ld = K + (4 if M % 2 else 3)
+    x = torch.randn((M, ld), generator=g, device=dev).to(x_dtype)[:, :K]
+    ng = -(-K // cols)
+    q = torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand((N, ng), generator=g, device=dev) * 0.02 + 0.005).to(torch.bfloat16)
+    z = torch.randint(5, 11, (N, ng), generator=g, device=dev).to(torch.bfloat16)
+    wide = lambda t: t.double().repeat_interleave(cols, 1)[:, :K]  # noqa: E731
+    ref = x.to(torch.bfloat16).double() @ ((q.double() - wide(z)) * wide(s)).T
+    stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
+    got = ops.linear_gemm(x, stream, 1, N, K, scales=s.reshape(-1), zeros=z.reshape(-1), group_cols=cols, out_dtype=torch.float32).double()
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
 @pytest.mark.parametrize("mode", ["gptq.int4", None])
 @pytest.mark.parametrize("T", [2, 8, 9, 10, 11, 16, 17, 31, 33, 64, 65, 130, 257])
 def test_prompt_pass_of_any_length_matches_single_tokens(dev, mode, T):
