@@ -124,12 +124,29 @@ void fill_linear_args(mi355_linear_args& a, const mi355_model* m, const mi355_we
     a.ldy = ldy;
 }
 
-// Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per 5-13 rows.  BF16: eight layers of a 7B
-// model, 10 rows 1139 us (rows) / 1159 us (tiled), 12 rows 1181 / 1162, 24 rows 2172 / 1223.  int4: 31 rows 1906 / 737 us, but its sums of
-// (128 + level) x run over a whole K-slice in one accumulator, where the row kernel's eight waves sum a part each: with single activations 10^4 times the
-// others (the full-depth fixture with a trained model's statistics) that took the logits from 0.05 to 0.08 of their spread, so short chunks stay there.
+// rows of one launch of the row kernel: what fits the LDS
+int row_cap(const mi355_weight& w) {
+    int cap = mi355_linear_max_rows(w.fmt, w.K, w.R, w.waves);
+    if (w.fmt == MI355_W_Q4 && w.group_cols > 0 && w.group_cols < w.K) {
+        // the tile's (scale, zero) table shares the LDS with the activation rows: 2 x 16 R x groups dwords
+        const int groups = (w.K + w.group_cols - 1) / w.group_cols;
+        const int row_bytes = ((w.K + 127) / 128 + 1) * 256 + 16;
+        cap -= (2 * 16 * w.R * groups * 4 + 16 + row_bytes - 1) / row_bytes;
+        if (cap < 1) cap = 1;
+    }
+    return cap;
+}
+// Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per row_cap() rows (7B: 13 at K = 4096, 5 at
+// 11008): from the second reading on, and 8 rows (int4 of one scale per row, the cheapest to read again: 11).  Eight layers of a 7B model, all by rows / by
+// this rule: bf16 6 rows 896 / 896 us (926 with the tiled kernel from row 6 on), 8 1057 / 968, 12 1163 / 1056, 16 1614 / 1188, 31 2824 / 1339; int4 8 rows 652 / 652
+// (689), 11 802 / 771, 16 1146 / 869, 31 1877 / 1002; groups of 128 columns 8 rows 752 / 744, 10 896 / 808, 16 1362 / 1028, 31 2318 / 1166.  Int4 scales that the
+// tiled kernel cannot apply unit by unit (mi355_linear_gemm): 32 rows, their sums over a whole K-slice in one accumulator cost a short chunk precision.
 int wide_rows(const mi355_weight& w) {
-    return w.fmt == MI355_W_BF16 ? 11 : 32;
+    const bool by_unit = w.sz_dtype == MI355_BF16 && w.K % 128 == 0 && (w.group_cols == 0 || w.group_cols >= 128);
+    if (w.fmt == MI355_W_Q4 && !by_unit) return 32;
+    const int cap = row_cap(w);
+    const int from = w.fmt == MI355_W_Q4 && (w.group_cols == 0 || w.group_cols >= w.K) ? 11 : 8;
+    return cap < from ? from : cap < 31 ? cap + 1 : 32;
 }
 bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: int4 / bf16 stream, one scale per row
     return (w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && (w.group_cols == 0 || w.group_cols >= w.K) && w.N % 4 == 0 &&
@@ -227,14 +244,7 @@ int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x
         a.ldy = ldy;
         return mi355_linear_int8_gemm(&a, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
     }
-    int cap = mi355_linear_max_rows(w.fmt, w.K, w.R, w.waves);
-    if (w.fmt == MI355_W_Q4 && w.group_cols > 0 && w.group_cols < w.K) {
-        // the tile's (scale, zero) table shares the LDS with the activation rows: 2 x 16 R x groups dwords
-        const int groups = (w.K + w.group_cols - 1) / w.group_cols;
-        const int row_bytes = ((w.K + 127) / 128 + 1) * 256 + 16;
-        cap -= (2 * 16 * w.R * groups * 4 + 16 + row_bytes - 1) / row_bytes;
-        if (cap < 1) cap = 1;
-    }
+    const int cap = row_cap(w);
     MI355_CHECK_ARG(cap >= 1, MI355_E_SHAPE, "forward: a row of K=%d does not fit LDS", w.K);
     if (M <= cap) return run_linear_rows(m, w, x, x_dtype, M, ldx, norm_scale, epi, y, y_dtype, ldy, s, attn_partials);
     const int n_sub = (M + cap - 1) / cap, step = (M + n_sub - 1) / n_sub;

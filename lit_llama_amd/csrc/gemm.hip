@@ -170,7 +170,7 @@ __device__ __forceinline__ f32x4 ldsz4(const void* p, int i, int dtype) {
 }
 
 // one row per workgroup: xb = bf16(norm_scale * x), rinv = alpha rsqrt(mean(x^2) + eps) (alpha without norm), sx[m][s] = sum of xb over
-// K-slice s (ksplit = 1: the whole row)
+// K-slice s (ksplit = 1: the whole row).  Rows of any length at any address; whole aligned ones: stage_units_kernel
 __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale,
                                                          int norm_dtype, float eps, int K, int Kp, bf16_t* xb, int64_t ldxb,
                                                          float* rinv, float* sx, int ksplit, float alpha, float norm_add) {
@@ -201,10 +201,12 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dt
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
 }
 
-// grouped scales: as stage_rows_kernel, but sxt[i][m] = sum of xb over columns [i * cols, (i + 1) * cols), cols = 32, 64 or 128 (K: whole 128-column units);
-// four columns per lane, one row per workgroup.  The workgroups behind the M rows lay out the tables, [N][n_groups] bf16 scales / zeros -> gtab[grp][r][n]
-// dwords (n fastest: the four rows a lane holds are one 16-B load; row n_groups and the rows past N are zero), a 64 x 64 piece each through LDS.
-// A lane per column and wave per group took 17 us for 1000 x 4096 f32, the tables 5 us in a launch of their own; together they take 9.
+// As stage_rows_kernel for rows of whole 128-column units, four columns per lane and four loads ahead: 12 rows of 4096 f32 columns 13 -> 5 us (a load, a
+// multiplication and a store at a time, and a sum of the block per K-slice).  Grouped scales: sxt[i][m] = sum of xb over columns [i * cols, (i + 1) * cols),
+// cols = 32, 64 or 128, in place of the sums per slice; the workgroups behind the M rows then lay out the tables, [N][n_groups] bf16 scales / zeros ->
+// gtab[grp][r][n] dwords (n fastest: the four rows a lane holds are one 16-B load; row n_groups and the rows past N are zero), a 64 x 64 piece each through
+// LDS: 1000 x 4096 f32 and the tables of 12288 rows 17 us and 5 in a launch of their own -> 9 together.
+constexpr int kStageLds = 64 * 65;  // dwords: a piece of the tables, or a sum per unit
 struct GroupTables {
     const bf16_t *s0, *z0, *s1, *z1;
     int N, tab_ld, n_groups, R;
@@ -232,11 +234,13 @@ __device__ __forceinline__ void group_table_piece(const GroupTables& t, int piec
     }
 }
 template <bool WIDE>  // rows and norm scale in whole aligned groups of four
-__global__ __launch_bounds__(256) void stage_rows_grouped_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale, int norm_dtype, float eps,
-                                                                 int K, bf16_t* xb, float* rinv, float* sxt, int M, int cols, const GroupTables tables) {
-    __shared__ uint32_t lds[64 * 65];
+__global__ __launch_bounds__(256) void stage_units_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale, int norm_dtype, float eps, int K,
+                                                          bf16_t* xb, float* rinv, float* sx, int ksplit, float alpha, float norm_add, float* sxt, int M,
+                                                          int cols, const GroupTables tables) {
+    __shared__ uint32_t lds[kStageLds];
     if ((int)blockIdx.x >= M) return group_table_piece(tables, blockIdx.x - M, lds);
     const int m = blockIdx.x;
+    float* per_unit = (float*)lds + 32;
     auto load4 = [&](const void* src, int64_t at, int dtype) {
         f32x4 v;
         if constexpr (WIDE) {
@@ -264,7 +268,7 @@ __global__ __launch_bounds__(256) void stage_rows_grouped_kernel(const void* x, 
             if (k >= K) break;  // (whole 128-column units: the 32 lanes of one leave together)
             if (norm_scale != nullptr) {
                 ss += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
-                v[i] *= ns[i];
+                v[i] *= ns[i] + norm_add;
             }
             bf16_t o[4];
             float sum = 0.f;
@@ -275,11 +279,23 @@ __global__ __launch_bounds__(256) void stage_rows_grouped_kernel(const void* x, 
             }
             *(u32x2*)(xb + (int64_t)m * K + k) = u32x2{o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16)};
             sum = group_sum(sum, cols >> 2);
-            if (k % cols == 0) sxt[(int64_t)(k / cols) * M + m] = sum;
+            if (k % cols == 0) {
+                if (sxt != nullptr)
+                    sxt[(int64_t)(k / cols) * M + m] = sum;
+                else
+                    per_unit[k >> 7] = sum;
+            }
         }
     }
     const float tss = block_sum(ss, (float*)lds);
-    if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) : 1.0f;
+    if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
+    if (sxt == nullptr) {  // (every wave has passed the block sum's barriers: the units' sums stand in LDS)
+        for (int s = threadIdx.x; s < ksplit; s += 256) {
+            float sum = 0.f;
+            for (int u = slice_lo(s, K >> 7, ksplit); u < slice_lo(s + 1, K >> 7, ksplit); ++u) sum += per_unit[u];
+            sx[(int64_t)m * ksplit + s] = sum;
+        }
+    }
 }
 
 // o += the K-slices' four values at row[0 .. 3], `stride` floats apart, in slice order.  All slices are requested before the first one is added: a
@@ -642,7 +658,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 // /root/reference lit_llama/quantization.py:284-333 with tile_cols > 0; groups of whole units: gemm_deep_kernel).  The MFMA accumulators keep running over K (cum_g =
 // columns up to the end of group g) and at every group
 // end     accf += (s_g - s_{g+1}) cum_g - s_g (128 + z_g) X_g      (Abel summation of sum_g s_g (A_g - (128 + z_g) X_g),
-// s past the last group = 0; X_g = the group's operand sum from stage_rows_grouped_kernel): two FMAs per output element
+// s past the last group = 0; X_g = the group's operand sum from stage_units_kernel): two FMAs per output element
 // and group, no accumulator reset.  The k columns of ONE MFMA are spread over the unit (lane group g holds columns
 // 32 g + 8 d ..), so a unit takes one pass per group with the other lane groups' activations zeroed, as in gemv.hip.
 // FUSE: the producer / consumer fusion of gemm_fuse.h (ungrouped launches without a K split): operand sums and 1/rms from
@@ -1721,9 +1737,15 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     const bool q4 = a->fmt == MI355_W_Q4;
     MI355_CHECK_ARG(a->w && a->x && a->y && (!q4 || (a->scales && a->zeros)), MI355_E_ARG, "linear_gemm: null w/x/y/scales/zeros");
     // grouped scales: group_cols = input columns per (scale, zero) pair; 0 or >= K: one pair per output row
-    const bool grouped = q4 && a->group_cols > 0 && a->group_cols < a->K;
+    const bool scale_groups = q4 && a->group_cols > 0 && a->group_cols < a->K;
+    // Few rows of one pair per output row: as one group, unit by unit.  The levels enter as 128 + q, and with single activations 10^4 times the others a sum of
+    // those over a whole K-slice in one accumulator loses what the row kernel, whose eight waves sum a part each, keeps (logits of a full-depth model with a
+    // trained model's statistics, 14 tokens: off by 0.05 of their spread there, 0.08 here, unit by unit 0.03).
+    const bool unit_sums = q4 && !scale_groups && f == nullptr && a->M < 32 && a->K % 128 == 0 && a->sz_dtype == MI355_BF16 && (a->alpha == 0.f || a->alpha == 1.f) &&
+                           !(a->flags & MI355_LF_NORM_ONE);
+    const bool grouped = scale_groups || unit_sums;
     int gq_shift = 0;
-    if (grouped) {
+    if (scale_groups) {
         while ((32 << gq_shift) < a->group_cols) ++gq_shift;
         MI355_CHECK_ARG((32 << gq_shift) == a->group_cols && a->K % 128 == 0, MI355_E_SHAPE,
                         "linear_gemm: group size %d is not 32 * 2^n or K %% 128 != 0 (use the generic kernel)", a->group_cols);
@@ -1758,7 +1780,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     size_t tab_bytes = 0, sxt_bytes = 0;
     int n_groups = 0, tab_ld = 0;
     if (grouped) {
-        n_groups = (a->K + a->group_cols - 1) / a->group_cols;
+        n_groups = unit_sums ? 1 : (a->K + a->group_cols - 1) / a->group_cols;
         tab_ld = (a->N + 15) / 16 * 16;
         tab_bytes = ((size_t)(n_groups + 1) * a->R * tab_ld * 4 + 15) & ~(size_t)15;
         sxt_bytes = (size_t)n_groups * a->M * 4;  // (of groups of whole units: in a place of their own)
@@ -1769,10 +1791,13 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
         const int rows_per_block = swiglu ? 16 * 4 * kTPW / 2 : 16 * 4 * kTPW;
         const int blocks = ((a->N + rows_per_block - 1) / rows_per_block) * ((a->M + 63) / 64);
         const size_t row_floats = (size_t)a->N * (swiglu ? 2 : 1);
-        const int cuts = a->group_cols >= 128 ? n_groups : units;
-        while (ksplit < kMaxSplit && blocks * ksplit < 256 && cuts >= 8 * ksplit && tab_bytes + sxt_bytes <= kSplitBudget / 2 &&
-               (size_t)2 * ksplit * a->M * row_floats * 4 <= kSplitBudget / 2)
-            ksplit *= 2;
+        const int cuts = scale_groups && a->group_cols >= 128 ? n_groups : units;
+        if (unit_sums)
+            ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, false);
+        else
+            while (ksplit < kMaxSplit && blocks * ksplit < 256 && cuts >= 8 * ksplit && tab_bytes + sxt_bytes <= kSplitBudget / 2 &&
+                   (size_t)2 * ksplit * a->M * row_floats * 4 <= kSplitBudget / 2)
+                ksplit *= 2;
     } else {
         ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, !q4);
     }
@@ -1806,24 +1831,27 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     // a bf16 operand in front of BF16 weights, whole units of it and no norm: multiplied where it lies
     const bool direct = !fused && !q4 && a->norm_scale == nullptr && a->x_dtype == MI355_BF16 && a->K % 128 == 0 && a->ldx % 8 == 0 &&
                         (uintptr_t)a->x % 16 == 0;
+    const bool aligned = ((uintptr_t)a->x | (uintptr_t)a->norm_scale) % 16 == 0 && a->ldx % 4 == 0;
     GemmParams p;
     memset(&p, 0, sizeof(p));
     if (grouped) {
         // the group tables live in the split-K region of the workspace (its second half when the launch is split)
         uint32_t* gtab = (uint32_t*)((char*)part + (ksplit > 1 ? kSplitBudget / 2 : 0));
-        const int cols = a->group_cols >= 128 ? 128 : a->group_cols;
+        const int cols = unit_sums || a->group_cols >= 128 ? 128 : a->group_cols;
         float* sxt = cols == 128 ? rinv + unit_sums_at(a->M) : (float*)((char*)gtab + tab_bytes);
         const GroupTables tables = {(const bf16_t*)a->scales, (const bf16_t*)a->zeros, (const bf16_t*)a->scales2, (const bf16_t*)a->zeros2, a->N, tab_ld, n_groups, a->R, gtab};
-        const bool wide = ((uintptr_t)a->x | (uintptr_t)a->norm_scale) % 16 == 0 && a->ldx % 4 == 0;
-        auto stage = wide ? stage_rows_grouped_kernel<true> : stage_rows_grouped_kernel<false>;
-        hipLaunchKernelGGL(stage, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv,
-                           sxt, a->M, cols, tables);
+        hipLaunchKernelGGL(aligned ? stage_units_kernel<true> : stage_units_kernel<false>, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx,
+                           a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv, (float*)nullptr, 1, 1.f, 0.f, sxt, a->M, cols, tables);
         MI355_LAUNCH_CHECK();
         p.gtab = gtab;
         p.sxt = sxt;
         p.n_groups = n_groups;
-        p.gq_shift = a->group_cols >= 128 ? gq_shift - 2 : gq_shift;
+        p.gq_shift = unit_sums ? 30 : a->group_cols >= 128 ? gq_shift - 2 : gq_shift;
         p.tab_ld = tab_ld;
+    } else if (!f_in && !direct && aligned && a->K % 128 == 0 && units <= kStageLds - 32) {
+        hipLaunchKernelGGL(stage_units_kernel<true>, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv,
+                           sx, ksplit, a->alpha == 0.f ? 1.f : a->alpha, (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f, (float*)nullptr, a->M, 128, GroupTables{});
+        MI355_LAUNCH_CHECK();
     } else if (!f_in && !direct) {
         hipLaunchKernelGGL(stage_rows_kernel, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype,
                            a->eps, a->K, kp, xb, (int64_t)kp, rinv, sx, ksplit, a->alpha == 0.f ? 1.f : a->alpha,
@@ -1868,7 +1896,7 @@ int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f
     p.y_dtype = a->y_dtype;
     p.ksplit = ksplit;
     p.part = part;
-    if (grouped) return launch_gemm_grouped_epi(p, a->epi, a->group_cols < 128, s);
+    if (grouped) return launch_gemm_grouped_epi(p, a->epi, scale_groups && a->group_cols < 128, s);
     if (fused) {
         p.f_in = f_in ? 1 : 0;
         p.in_sx = f->in_sx;
