@@ -741,9 +741,7 @@ class DecodeEngine:
             self._cache_pool = {S: pool}  # one cache geometry at a time
             self._kv_arena = arena
         else:
-            for k, v in pool:
-                k.zero_()
-                v.zero_()
+            self._kv_arena.zero_()  # (one launch: the pool's tensors are its views)
         for i, (k, v) in enumerate(pool):
             self.layers[i].kcache, self.layers[i].vcache = ptr(k), ptr(v)
         self.model.kv_caches = list(pool)
