@@ -49,6 +49,16 @@ struct mi355_gemm_fuse {
 void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
 // bytes mi355_linear_gemm_workspace_bytes reserves at the END of a workspace for the chain's partial sums
 size_t mi355_linear_gemm_fuse_scratch_bytes();
+// The RMSNorm of the rows that a residual product (MI355_EPI_ACCUM, f32 y without gaps up to N) leaves: xb[m] = bf16(norm(y[m]) (scale + add)), rows of N.
+// Taken up by the sum of its K-slices, if there is one (`done`): the caller's own norm is a launch of its own, 4.6 us and a gap for 16 rows.
+struct mi355_reduce_norm {
+    const void* scale;
+    int scale_dtype;
+    float eps, add;
+    bf16_t* xb;
+    bool done;  // out
+};
+int mi355_linear_gemm_norm(const mi355_linear_args* a, mi355_reduce_norm* norm, void* workspace, size_t workspace_bytes, mi355_stream_t stream);
 // as mi355_linear_gemm, with the fusion described by `f` (NULL: none)
 int mi355_linear_gemm_fused(const mi355_linear_args* a, const mi355_gemm_fuse* f, void* workspace, size_t workspace_bytes,
                             mi355_stream_t stream);

@@ -3,6 +3,7 @@
 // experts (experts.hip).  RMSNorm rides in the consuming linear and the residual sum in the producing one; the residual stream is f32.
 // A parallel layer normalises its row once (by groups, with the token shift of its mixer), and its mixer's output and hidden row leave
 // through one product.  A sandwich layer's sublayers read rows that the pass behind the sublayer in front (join.hip) has normalised.
+#include "gemm_fuse.h"
 #include "product.h"
 
 namespace {
@@ -360,9 +361,12 @@ int ew_blocks(int64_t n) {
 
 enum { kStore = 0, kRelu2 = 1, kResidual = 2, kGeglu = 3, kLogits = 4 };
 
-// y[M, N] (+)= alpha * W norm(x), or what a feed-forward makes of it; alpha: residual_mult (kResidual), logit_scale (kLogits), 1.  x f32 with `norm`, or dtype without
+// y[M, N] (+)= alpha * W norm(x), or what a feed-forward makes of it; alpha: residual_mult (kResidual), logit_scale (kLogits), 1.  x f32 with `norm`, or dtype without.
+// kResidual: *ready = the norm `next` of the new rows stands in m->xb (if it could be had with the product); with `norm`: whether this one does
 int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int64_t ldx, const void* norm, int what, void* y, int64_t ldy,
-           int y_dtype, int M, hipStream_t s) {
+           int y_dtype, int M, hipStream_t s, bool* ready = nullptr, const void* next = nullptr) {
+    const bool normed = norm != nullptr && ready != nullptr && *ready;
+    if (ready != nullptr) *ready = false;
     if (m->dtype == MI355_F32) {
         const float* in = (const float*)x;
         int64_t ld_in = ldx;
@@ -417,9 +421,17 @@ int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int6
         a.x = x;
         a.y = y;
         a.M = M;
+        if (what == kResidual && next != nullptr && w.N == m->width && w.N % 128 == 0 && ldy % 4 == 0) {
+            mi355_reduce_norm rn = {next, m->norm_dtype, m->eps, m->norm_add, (bf16_t*)m->xb, false};
+            const int rc = mi355_linear_gemm_norm(&a, &rn, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
+            *ready = rn.done;
+            return rc;
+        }
         if (norm != nullptr && w.K % 128 == 0 && ldx % 4 == 0) {
-            hipLaunchKernelGGL(norm_rows_kernel, dim3(M), dim3(512), 0, s, (const float*)x, ldx, norm, m->norm_dtype, m->eps, w.K, m->norm_add, m->xb);
-            MI355_LAUNCH_CHECK();
+            if (!normed) {
+                hipLaunchKernelGGL(norm_rows_kernel, dim3(M), dim3(512), 0, s, (const float*)x, ldx, norm, m->norm_dtype, m->eps, w.K, m->norm_add, m->xb);
+                MI355_LAUNCH_CHECK();
+            }
             a.x = m->xb;
             a.x_dtype = MI355_BF16;
             a.ldx = w.K;
@@ -691,6 +703,11 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
         MI355_LAUNCH_CHECK();
     }
     const int runs = run_end < m->n_runs ? run_end : m->n_runs;
+    bool ready = false;  // the norm that the next product takes stands in m->xb
+    auto norm_behind = [&](int r) -> const void* {  // ... of the rows that layer r leaves, where the product behind it reads nothing else
+        if (r + 1 < runs) return m->layers[r + 1].parallel || m->layers[r + 1].sandwich ? nullptr : m->layers[r + 1].norm1;
+        return runs == m->n_runs && n_want > 0 && want == nullptr && m->norm_groups == 0 ? m->final_norm : nullptr;
+    };
     for (int r = 0; r < runs; ++r) {
         const mi355_hybrid_layer& l = m->layers[r];
         const int64_t ldp = l.in.N;
@@ -703,7 +720,7 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
         } else if (l.parallel) {
             if (int rc = norm_groups(m, l.norm1, &l, b, nullptr, M, s)) return rc;
             if (int rc = parallel_in(m, l, M, s)) return rc;
-        } else if (int rc = linear(m, l.in, m->x, m->ldx, l.norm1, kStore, m->proj, ldp, m->dtype, M, s)) return rc;
+        } else if (int rc = linear(m, l.in, m->x, m->ldx, l.norm1, kStore, m->proj, ldp, m->dtype, M, s, &ready)) return rc;
         if (l.mixer == MI355_MIX_ATTENTION) {
             mi355_window_attn_args a = l.attn;
             a.proj = proj;
@@ -753,7 +770,8 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
             if (int rc = parallel_out(m, l, M, s)) return rc;
             continue;
         }
-        if (int rc = linear(m, l.out, m->att, m->ld_att, nullptr, kResidual, m->x, m->ldx, MI355_F32, M, s)) return rc;
+        const void* after = l.mlp == MI355_MLP_EXPERTS ? nullptr : l.mlp != MI355_MLP_NONE ? l.norm2 : norm_behind(r);
+        if (int rc = linear(m, l.out, m->att, m->ld_att, nullptr, kResidual, m->x, m->ldx, MI355_F32, M, s, &ready, after)) return rc;
         if (l.mlp == MI355_MLP_EXPERTS) {
             mi355_experts_args e = l.moe;
             e.dtype = m->dtype;
@@ -770,8 +788,8 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
             if (int rc = mi355_experts(&e, stream)) return rc;
         } else if (l.mlp != MI355_MLP_NONE) {
             const int what = l.mlp == MI355_MLP_GEGLU ? kGeglu : kRelu2;
-            if (int rc = linear(m, l.up, m->x, m->ldx, l.norm2, what, m->hid, l.up.N, m->dtype, M, s)) return rc;
-            if (int rc = linear(m, l.down, m->hid, l.up.N, nullptr, kResidual, m->x, m->ldx, MI355_F32, M, s)) return rc;
+            if (int rc = linear(m, l.up, m->x, m->ldx, l.norm2, what, m->hid, l.up.N, m->dtype, M, s, &ready)) return rc;
+            if (int rc = linear(m, l.down, m->hid, l.up.N, nullptr, kResidual, m->x, m->ldx, MI355_F32, M, s, &ready, norm_behind(r))) return rc;
         }
     }
     if (run_end < m->n_runs || n_want == 0) return 0;
@@ -788,7 +806,7 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
         MI355_LAUNCH_CHECK();
         xh = m->xw;
     }
-    return linear(m, m->head, xh, m->ldx, m->final_norm, kLogits, logits, m->ld_logits, MI355_F32, n_want, s);
+    return linear(m, m->head, xh, m->ldx, m->final_norm, kLogits, logits, m->ld_logits, MI355_F32, n_want, s, &ready);
 }
 
 extern "C" int mi355_hybrid_reset_slots(const mi355_hybrid_model* m, const int32_t* slots, int n, mi355_stream_t stream) {

@@ -453,3 +453,29 @@ def test_trace_replay_and_command_line(dev, tmp_path, capsys, monkeypatch):
                      "--max-new-tokens", "5"]) == 0
     lines = capsys.readouterr().out.strip().split("\n")
     assert len(lines) == 2 and lines[0].startswith(",".join(map(str, a))) and len(lines[0].split(",")) == 30
+
+
+@pytest.mark.parametrize("width,batch", [(1024, 9), (1152, 16), (4096, 33), (8192, 10), (8320, 10)])
+def test_norm_behind_the_slices_of_a_residual_product(dev, width, batch):
+    """Batches whose residual products are cut along K, the norm of the next product taken with their sum (rows of up to 8192) or by itself, in front of
+    products of either kind of layer, the next layer's and the head: the logits of each sequence alone, whose norms are taken in the row kernel."""
+    from lit_llama_amd.hybrid_engine import Entry
+
+    att = {"type": "attention", "mixer": {"heads": 9, "kv_heads": 3, "dim": 128, "vdim": 128, "scale": 0.09, "mask": {"size": 19}}}
+    config = small_config(layers=[{**att, "mlp": {"kind": "dense", "ff": 1280}}, {**att, "mlp": None}], loop=None, width=width)
+    m, _ = build(config, torch.bfloat16, dev)
+    eng = m.engine()
+    eng.ensure(batch + 1, 64)
+    seqs = [tokens_of(3, seed=i) for i in range(batch)]
+
+    def steps(group):
+        slots = [eng.acquire() for _ in group]
+        out = [eng.step([Entry(s, j, t[j:j + 1], [0]) for s, t in zip(slots, group)]).clone() for j in range(3)]
+        for s in slots:
+            eng.release(s)
+        return torch.stack(out)
+
+    got = steps(seqs)
+    for i, t in enumerate(seqs):
+        # (both sides round the same values to bf16; a value at the edge of a rounding falls either way: a few 2^-9 of the terms over four products)
+        assert rel(got[:, i].float(), steps([t])[:, 0].float()) < 4e-2, i
