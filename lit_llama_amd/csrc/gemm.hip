@@ -1668,9 +1668,10 @@ GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
     if (fo.bm) sh.bm = fo.bm;
     return sh;
 }
-// Split-K of an ungrouped launch: as many slices as bring it to the workgroups wanted, none below 6 units (BF16: 4) or past the partial buffer.  BF16, whose
-// weights are four times the bytes, gains from more of them up to 64 tokens (16 rows, 4096 x 11008: 66 / 39 / 31 / 27 / 23.4 us with 1 / 2 / 3 / 4 / 8 slices);
-// int4 pays the reduction instead (37 tokens, 12288 x 4096: 29.8 / 28.2 / 30.4 / 34.2 us with 1 / 2 / 3 / 8).
+// Split-K of an ungrouped launch: as many slices as bring it to the workgroups wanted, none below 6 units (BF16: 4) or past the partial buffer.  Blocks of 4
+// waves stop at one workgroup per CU: a few more than 256 leave the chip to those few (bf16, 16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us
+// with 1 / 2 / 3 / 4 slices; the c_fc1 / c_fc2 pair of 172 blocks 34.5 with 1, 42.8 with 3), and three quarters of them are as good for BF16 and cheaper to
+// sum (K = 11008, N = 4096, 32 blocks: 24.2 / 21.9 / 21.3 / 21.9 / 23.2 us with 4 / 5 / 6 / 8 / 13; int4, 37 rows: 28.4 / 26.7 / 25.6 / 24.7 with 4 / 5 / 6 / 8).
 int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
     const int units = (K + 127) / 128;
     const size_t row_floats = (size_t)N * (pair ? 2 : 1);
@@ -1679,9 +1680,11 @@ int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
     }
     const int waves = gemm_waves(M, N, pair, bf16);
     const int rows_per_block = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
-    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), want = waves == 8 ? 192 : bf16 ? 400 : 160;
+    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), want = bf16 || waves == 8 ? 192 : 256, most = waves == 8 ? 1 << 20 : 256;
     int ksplit = 1;
-    while (ksplit < (bf16 ? kMaxSplit : 8) && blocks * ksplit < want && units >= (bf16 ? 4 : 6) * (ksplit + 1) && (size_t)2 * (ksplit + 1) * M * row_floats * 4 <= kSplitBudget) ++ksplit;
+    while (ksplit < (bf16 ? kMaxSplit : 8) && blocks * ksplit < want && blocks * (ksplit + 1) <= most && units >= (bf16 ? 4 : 6) * (ksplit + 1) &&
+           (size_t)2 * (ksplit + 1) * M * row_floats * 4 <= kSplitBudget)
+        ++ksplit;
     return ksplit;
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
