@@ -1239,7 +1239,10 @@ int gemv_prepare(const mi355_linear_args* a, GemvParams& p, int& grid, int& wave
     p.relu2 = (a->flags & MI355_LF_RELU2) ? 1 : 0;
     p.norm_add = (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f;
     MI355_CHECK_ARG(!p.relu2 || a->epi == MI355_EPI_STORE, MI355_E_ARG, "linear_fast: RELU2 belongs to the STORE epilogue");
-    waves = a->waves > 0 ? a->waves : 8;
+    // rows of at most four units: four waves, one unit each as with eight, and twice the workgroups (of eight, four had nothing to do: N = 32000,
+    // K = 256 11.3 -> 8.1 us, N = K = 256 3.6 -> 3.3; the same bits)
+    const bool few = a->waves <= 0 && p.units <= 4;
+    waves = a->waves > 0 ? a->waves : few ? 4 : 8;
     if (waves > 16) waves = 16;
     if ((a->fmt != MI355_W_Q4 || (a->group_cols > 0 && a->group_cols < a->K)) && waves > 8) waves = 8;  // see kMaxThreads
     if (waves < 4) waves = 4;  // the combine step needs 256 owner threads
@@ -1299,7 +1302,7 @@ int gemv_prepare(const mi355_linear_args* a, GemvParams& p, int& grid, int& wave
     grid = a->grid;
     if (grid <= 0) {
         const int cus = mi355_num_cus() > 0 ? mi355_num_cus() : 256;
-        grid = cus * 2;
+        grid = cus * (few ? 4 : 2);
     }
     if (grid > p.n_tiles) grid = p.n_tiles;
     p.u_q = p.units / waves;

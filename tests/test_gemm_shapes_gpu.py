@@ -91,3 +91,16 @@ def test_prompt_pass_of_any_length_matches_single_tokens(dev, mode, T):
         model.reset_cache()
         rows = torch.cat([model(idx[t:t + 1].view(1, 1), 288, torch.tensor([t], device=dev))[0] for t in range(T)])
     assert (one - rows).abs().max() <= 0.05 * rows.std()
+
+
+@pytest.mark.parametrize("M", [1, 5])
+@pytest.mark.parametrize("N,K", [(16, 64), (32000, 128), (33000, 384), (260, 512)])
+def test_short_rows_in_four_waves_give_the_bits_of_eight(dev, N, K, M):
+    """Rows of at most four units: a wave has one unit or none with four waves as with eight, so the sums are the same."""
+    g = torch.Generator(device=dev).manual_seed(N + K + M)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    q = torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8)
+    kw = dict(scales=(torch.rand((N,), generator=g, device=dev) * 0.02).to(torch.bfloat16), zeros=torch.full((N,), 7.0, device=dev).to(torch.bfloat16),
+              out_dtype=torch.float32)
+    stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
+    assert torch.equal(ops.linear_fast(x, stream, nat.W_Q4, 1, N, K, **kw), ops.linear_fast(x, stream, nat.W_Q4, 1, N, K, waves=8, **kw))
