@@ -1,11 +1,11 @@
-// Wide (M >= 32 tokens) linear over the int4 or the bf16 weight stream for gfx950: prompt prefill and no-cache evaluation.
+// Wide (several tokens) linear over the int4 or the bf16 weight stream for gfx950: prompt prefill, no-cache evaluation, batches of decoding sequences.
 //
 // Replaces the reference's Triton `linear_kernel_4bit_weight` (/root/reference lit_llama/quantization.py:187-333,
 // reached from ColBlockQuantizedLinear.forward :413-421) at the shapes of evaluate/full.py:120-129 (T = 2048, no cache)
 // and of generate.py's prompt pass — where the skinny weight-streaming kernel (gemv.hip) re-reads the whole weight
 // stream once per 13 tokens.
 //
-// Design:
+// Design (gemm_q4_kernel; launches of about one workgroup per CU and grouped scales: gemm_deep_kernel, three units of operands under way):
 //  * the weights stay in the decode path's stream layout [tile of 16 rows][unit of 128 k][r][lane][16 B]: a wave reads
 //    a (tile, unit) piece with ONE coalesced 1-KiB load straight into registers (no LDS for weights: a piece is
 //    private to its wave) and turns it into four MFMA A fragments with 7 VALU ops per 8 weights — amortised over the
@@ -21,7 +21,7 @@
 //  * XCD-aware block order: workgroup b runs on XCD b % 8 (each XCD has its own 4 MiB L2).  The (token block, row
 //    block) pairs are cut, token-block major, into 8 contiguous ranges, one per XCD: the workgroups an XCD runs side by
 //    side share one or two token blocks (1 MiB of activations each), fetched into that L2 once;
-//  * operands are staged once per linear by stage_rows_kernel: bf16(norm_scale * x) with RMSNorm's 1/rms kept as a
+//  * operands are staged once per linear by stage_units_kernel (odd rows: stage_rows_kernel): bf16(norm_scale * x) with RMSNorm's 1/rms kept as a
 //    per-row factor for the epilogue, and the per-row operand sum that undoes the +128 / zero-point offset:
 //        y[m, n] = scale[n] * (acc[m, n] - (128 + zero[n]) * sum_k xb[m, k]) * rinv[m]      (same arithmetic as gemv.hip).
 #include <type_traits>
@@ -62,9 +62,6 @@ constexpr int kTPW = MI355_GEMM_TPW;
 #define MI355_GEMM_BPIPE 4   // 128-token blocks: B fragments requested this many LDS reads ahead of the MFMAs that take them (0: hipcc's
                              // order, which waits for every pair of reads right behind their issue); 2 / 3 / 4: -1.4 / -1.9 / -2.0 % per 2048-token
                              // prompt (profiles/r06_prefill_gemm_ab.txt); 124-127 VGPRs at 4, still two workgroups per CU
-#endif
-#ifndef MI355_GEMM_PIN_LOADS
-#define MI355_GEMM_PIN_LOADS 1
 #endif
 #ifndef MI355_GEMM_AND_OR
 #define MI355_GEMM_AND_OR 1
@@ -948,11 +945,6 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
 #pragma unroll
             for (int t = 0; t < kTPW; ++t) wload(t, u + 1, wnext[t]);
         }
-        // hipcc sinks these requests to the END of the unit, right in front of the LDS stores that wait for them (the
-        // 24 registers they land in would otherwise be live across the MFMAs): a unit pays the memory latency in front
-        // of its barrier, covered by the other waves of the SIMD.  Pinned here they fly under the unit's MFMAs — at
-        // 141-145 VGPRs for 128-token blocks (one workgroup per CU), so only the 64-token blocks (95) can take it.
-        if constexpr (MI355_GEMM_PIN_LOADS && BM <= 64 && GRP == 0) __builtin_amdgcn_sched_barrier(0);
     };
     // the 4 x kTT x kTPW MFMAs of a unit; sub >= 0 (GRP 2): only the lane groups of sub-group `sub` contribute
     // (explicitly software-pipelined B-fragment reads — 16 fragments in registers, pinned with sched_barrier —
