@@ -1133,7 +1133,7 @@ __device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, un
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
-// BM: 16 / 32 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel.
+// BM: 16 / 32 / 48 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel.
 // GRP (Q4, groups of whole 128-column units): the products of a unit start from 0, and accf += s_unit * them, one FMA per output element and unit on the
 // VALU beside the next unit's products; the zero points, accf -= sum over units of s (128 + z) X_unit (X: the unit's operand sums), are a product with K =
 // units / 4 of their own on the f32 MFMA in front of the loop.
@@ -1621,6 +1621,9 @@ int gemm_waves(int M, int N, bool pair, bool bf16) {
     const int blocks8 = (N + 255) / 256 * ((M + 63) / 64);
     return M <= 64 || (!bf16 && !pair && (blocks8 <= 64 || (blocks8 >= 96 && blocks8 <= 128))) ? 4 : 8;
 }
+// (blocks of 48 tokens, int4: N = 12288 / 11008 pair, K = 4096, 37 tokens 22.9 / 25.1 us with blocks of 64, 21.7 / 23.3 with 48, groups of 128 columns 29.5 / 36.0 and
+// 27.4 / 33.6; BF16, bound by the weights, the same either way)
+int short_block(int M, bool bf16) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 48 && !bf16 ? 48 : 64; }
 // Tokens per block and kernel.  Blocks of 128 tokens x 256 rows with two workgroups per CU (gemm_q4_kernel) when a launch has a few of them per CU: 2048
 // tokens, int4, c_fc1/c_fc2 271 us against 303 (gemm_deep_kernel, one workgroup per CU), c_attn 158 / 174.  Fewer: 64-token blocks, twice as many, of the
 // deep kernel: 128 tokens, int4, c_fc1/c_fc2 49.6 -> 39.9 us, 777 tokens N = 4096 47.8 -> 42.1 us.  An int4 launch of exactly one 128-token block per CU (N = 4096
@@ -1629,7 +1632,7 @@ int gemm_waves(int M, int N, bool pair, bool bf16) {
 // kernel: 2048 tokens, N = 4096, K = 11008 174 -> 158 us.
 GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16) {
     const GemmForce fo = gemm_force();
-    GemmShape sh = {gemm_waves(M, n_tiles * 16, pair, bf16), M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
+    GemmShape sh = {gemm_waves(M, n_tiles * 16, pair, bf16), short_block(M, bf16), true};
     const int per_block8 = pair ? 8 * kTPW / 2 : 8 * kTPW;
     const int blocks8 = ((n_tiles + per_block8 - 1) / per_block8) * ((M + kBM - 1) / kBM) * ksplit;  // of 128 tokens
     if (bf16 ? M > 128 && blocks8 >= 160 : blocks8 >= 384 || blocks8 == 256) sh.bm = 128, sh.deep = bf16 && blocks8 <= 256;
@@ -1643,7 +1646,7 @@ GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16) {
 // of 64 x 128 one unit ahead -> 185 / 75 / 120.
 GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
     const GemmForce fo = gemm_force();
-    GemmShape sh = {4, M <= 16 ? 16 : M <= 32 ? 32 : 64, true};
+    GemmShape sh = {4, short_block(M, false), true};
     if (M > 64) {
         auto blocks = [&](int waves, int bm) {
             const int per_block = pair ? waves * kTPW / 2 : waves * kTPW;
@@ -1685,6 +1688,9 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, FMT, 4, 32, FUSE>(p, s);
+        if constexpr (FMT == MI355_W_Q4) {
+            if (sh.bm == 48) return launch_deep<EPI, PAIR, FMT, 4, 48, FUSE>(p, s);
+        }
         return launch_deep<EPI, PAIR, FMT, 4, 64, FUSE>(p, s);
     }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 8, 64, FUSE>(p, s);
@@ -1707,6 +1713,7 @@ int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, false, 1>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, false, 1>(p, s);
+        if (sh.bm == 48) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 48, false, 1>(p, s);
         return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 64, false, 1>(p, s);
     }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 64, false, 1>(p, s);
