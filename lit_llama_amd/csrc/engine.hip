@@ -138,8 +138,8 @@ int row_cap(const mi355_weight& w) {
 }
 // Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per row_cap() rows (7B: 13 at K = 4096, 5 at
 // 11008): from the second reading on, and 8 rows (int4 of one scale per row, the cheapest to read again: 11).  Eight layers of a 7B model, all by rows / by
-// this rule: bf16 6 rows 896 / 896 us (926 with the tiled kernel from row 6 on), 8 1057 / 968, 12 1163 / 1056, 16 1614 / 1188, 31 2824 / 1339; int4 8 rows 652 / 652
-// (689), 11 802 / 771, 16 1146 / 869, 31 1877 / 1002; groups of 128 columns 8 rows 752 / 744, 10 896 / 808, 16 1362 / 1028, 31 2318 / 1166.  Int4 scales that the
+// this rule: bf16 6 rows 896 / 896 us (926 with the tiled kernel from row 6 on), 8 1057 / 963, 12 1163 / 1056, 16 1614 / 1136, 31 2824 / 1236; int4 8 rows 652 / 652
+// (689), 11 802 / 737, 16 1146 / 839, 31 1877 / 965; groups of 128 columns 8 rows 752 / 749, 10 896 / 813, 16 1362 / 1030, 31 2318 / 1164.  Int4 scales that the
 // tiled kernel cannot apply unit by unit (mi355_linear_gemm): 32 rows, their sums over a whole K-slice in one accumulator cost a short chunk precision.
 int wide_rows(const mi355_weight& w) {
     const bool by_unit = w.sz_dtype == MI355_BF16 && w.K % 128 == 0 && (w.group_cols == 0 || w.group_cols >= 128);
