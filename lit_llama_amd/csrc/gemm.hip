@@ -94,8 +94,11 @@ struct GemmParams {
     int M, N, K, units, n_tiles, n_blocks, per_xcd, total_blocks;
     int sz_dtype, y_dtype;
     // split-K (few blocks: short prompts against N = 4096): slice ks of the units -> part[ks][M][N] f32, summed in order
-    // by splitk_reduce_kernel; sx then holds [M][ksplit] per-slice operand sums
+    // by splitk_reduce_kernel
     int ksplit;
+    // Q4, gemm_deep_kernel: a slice's units go through the accumulators in up to `runs` runs of run_units (runs = 1: all its units), whose sums are added up beside
+    // them (gemm_runs()).  sx: [M][ksplit][runs] operand sums
+    int runs, run_units;
     float* part;
     int relu2;             // STORE: max(y, 0)^2
     float alpha;           // factor of the product where rinv is NULL (an operand that needed no staging)
@@ -144,10 +147,16 @@ __device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n,
 
 constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials a workspace holds
 constexpr int kMaxSplit = 16;
+constexpr int kMaxRuns = 8;
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
 __host__ __device__ __forceinline__ int slice_lo(int s, int units, int ksplit) { return (int)((int64_t)s * units / ksplit); }
+// first unit of run i = slice * runs + run of a row cut into `ksplit` slices of `runs` runs (run i = units [run_lo(i), run_lo(i + 1)), possibly none)
+__device__ __forceinline__ int run_lo(int i, int units, int ksplit, int runs, int run_units) {
+    const int ks = i / runs, lo = slice_lo(ks, units, ksplit) + (i - ks * runs) * run_units, hi = slice_lo(ks + 1, units, ksplit);
+    return lo < hi ? lo : hi;
+}
 
 // 16-B chunk swizzle of an activation row in LDS (see the header): bits 0, 1 of the token stay, bit 2 -> 8, bit 3 -> 12
 #ifdef MI355_NO_SWZ
@@ -167,17 +176,17 @@ __device__ __forceinline__ f32x4 ldsz4(const void* p, int i, int dtype) {
     return f32x4{bf16_to_f32(b[0]), bf16_to_f32(b[1]), bf16_to_f32(b[2]), bf16_to_f32(b[3])};
 }
 
-// one row per workgroup: xb = bf16(norm_scale * x), rinv = alpha rsqrt(mean(x^2) + eps) (alpha without norm), sx[m][s] = sum of xb over
-// K-slice s (ksplit = 1: the whole row).  Rows of any length at any address; whole aligned ones: stage_units_kernel
+// one row per workgroup: xb = bf16(norm_scale * x), rinv = alpha rsqrt(mean(x^2) + eps) (alpha without norm), sx[m][i] = sum of xb over
+// run i (ksplit = runs = 1: the whole row).  Rows of any length at any address; whole aligned ones: stage_units_kernel
 __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale,
                                                          int norm_dtype, float eps, int K, int Kp, bf16_t* xb, int64_t ldxb,
-                                                         float* rinv, float* sx, int ksplit, float alpha, float norm_add) {
+                                                         float* rinv, float* sx, int ksplit, int runs, int run_units, float alpha, float norm_add) {
     __shared__ float red[32];
     const int m = blockIdx.x;
     const int units = Kp >> 7;
     float ss = 0.f;
-    for (int s = 0; s < ksplit; ++s) {
-        const int k_lo = slice_lo(s, units, ksplit) << 7, k_hi = slice_lo(s + 1, units, ksplit) << 7;
+    for (int s = 0; s < ksplit * runs; ++s) {
+        const int k_lo = run_lo(s, units, ksplit, runs, run_units) << 7, k_hi = run_lo(s + 1, units, ksplit, runs, run_units) << 7;
         float sum = 0.f;
         for (int k = k_lo + threadIdx.x; k < k_hi; k += blockDim.x) {
             bf16_t o = 0;
@@ -193,7 +202,7 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dt
             xb[(int64_t)m * ldxb + k] = o;
         }
         const float tot = block_sum(sum, red);
-        if (threadIdx.x == 0) sx[(int64_t)m * ksplit + s] = tot;
+        if (threadIdx.x == 0) sx[(int64_t)m * (ksplit * runs) + s] = tot;
     }
     const float tss = block_sum(ss, red);
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
@@ -233,8 +242,8 @@ __device__ __forceinline__ void group_table_piece(const GroupTables& t, int piec
 }
 template <bool WIDE>  // rows and norm scale in whole aligned groups of four
 __global__ __launch_bounds__(256) void stage_units_kernel(const void* x, int x_dtype, int64_t ldx, const void* norm_scale, int norm_dtype, float eps, int K,
-                                                          bf16_t* xb, float* rinv, float* sx, int ksplit, float alpha, float norm_add, float* sxt, int M,
-                                                          int cols, const GroupTables tables) {
+                                                          bf16_t* xb, float* rinv, float* sx, int ksplit, int runs, int run_units, float alpha, float norm_add,
+                                                          float* sxt, int M, int cols, const GroupTables tables) {
     __shared__ uint32_t lds[kStageLds];
     if ((int)blockIdx.x >= M) return group_table_piece(tables, blockIdx.x - M, lds);
     const int m = blockIdx.x;
@@ -288,10 +297,10 @@ __global__ __launch_bounds__(256) void stage_units_kernel(const void* x, int x_d
     const float tss = block_sum(ss, (float*)lds);
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
     if (sxt == nullptr) {  // (every wave has passed the block sum's barriers: the units' sums stand in LDS)
-        for (int s = threadIdx.x; s < ksplit; s += 256) {
-            float sum = 0.f;
-            for (int u = slice_lo(s, K >> 7, ksplit); u < slice_lo(s + 1, K >> 7, ksplit); ++u) sum += per_unit[u];
-            sx[(int64_t)m * ksplit + s] = sum;
+        for (int s = threadIdx.x; s < ksplit * runs; s += 256) {
+            double sum = 0.;  // (one rounding beside a large unit, not one per unit)
+            for (int u = run_lo(s, K >> 7, ksplit, runs, run_units); u < run_lo(s + 1, K >> 7, ksplit, runs, run_units); ++u) sum += per_unit[u];
+            sx[(int64_t)m * (ksplit * runs) + s] = (float)sum;
         }
     }
 }
@@ -1133,13 +1142,16 @@ __device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, un
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
-// BM: 16 / 32 / 48 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel.
+// BM: 16 / 32 / 48 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
 // GRP (Q4, groups of whole 128-column units): the products of a unit start from 0, and accf += s_unit * them, one FMA per output element and unit on the
 // VALU beside the next unit's products; the zero points, accf -= sum over units of s (128 + z) X_unit (X: the unit's operand sums), are a product with K =
 // units / 4 of their own on the f32 MFMA in front of the loop.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0>
+// RUNS (Q4): a slice of several runs (gemm_runs()).  The second set of sums is 32 registers, with which two workgroups of 8 waves no longer share a CU: kernels of
+// their own.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
     static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1 && !FUSE), "grouped scales are a Q4 feature");
+    static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
     static_assert(DEPTH == 3 || DEPTH == 4, "units under way + 1");
     constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
@@ -1169,6 +1181,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] float* frp = fr + 2 * BM;
     [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM, DEPTH>);
     [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE, DEPTH>);
+    [[maybe_unused]] float* runtab = rowtab + 3 * kSlots * 16;  // [run][BM] operand sums
     int tile[kTPW];
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
@@ -1253,34 +1266,49 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     }
     const int mt = (int)threadIdx.x < BM ? (m0 + (int)threadIdx.x < p.M ? m0 + (int)threadIdx.x : p.M - 1) : p.M - 1;
     const bool own = !(FUSE && p.f_in);  // factors of the tokens as they are, not as shares
-    float t_ri = p.alpha, t_sx = 0.f;
-    if (own) {
-        if (p.rinv != nullptr) t_ri = p.rinv[mt];
-        if constexpr (kScales) t_sx = p.sx[(int64_t)mt * p.ksplit + ks];
+    float t_ri = p.alpha;
+    if (own && p.rinv != nullptr) t_ri = p.rinv[mt];
+    constexpr int kSX = RUNS ? (kMaxRuns * BM + kThreads - 1) / kThreads : 1;
+    [[maybe_unused]] float t_sx[kSX];  // operand sum of token (i kThreads + thread) % BM in run (...) / BM
+    if constexpr (kScales) {
+        if (own) {
+            if constexpr (!RUNS) {
+                t_sx[0] = p.sx[(int64_t)mt * p.ksplit + ks];
+            } else {
+#pragma unroll
+                for (int i = 0; i < kSX; ++i) {
+                    const int at = i * kThreads + (int)threadIdx.x, run = at / BM < p.runs ? at / BM : 0, m = m0 + at % BM;
+                    t_sx[i] = p.sx[((int64_t)(m < p.M ? m : p.M - 1) * p.ksplit + ks) * p.runs + run];
+                }
+            }
+        }
     }
     [[maybe_unused]] int t_pos = 0;
     if constexpr (FUSE && EPI == MI355_EPI_STORE) {
         if (p.rope != nullptr) t_pos = p.pos[mt];
     }
-    // shares of the tokens' factors (gemm_fuse.h): every thread a token and every kP-th share, in share order; the first kIn of them now
+    // shares of the tokens' factors (gemm_fuse.h): every thread a token and every kP-th share (operand sums of several runs: every share of every kP-th run), in
+    // share order; the first kIn of them now
     constexpr int kP = kThreads / BM < 8 ? kThreads / BM : 8, kIn = kSharesAhead;
     const int s_tok = threadIdx.x % BM, s_part = threadIdx.x / BM;
     [[maybe_unused]] const int64_t s_m = m0 + s_tok < p.M ? m0 + s_tok : p.M - 1;
     [[maybe_unused]] const int s_lo = FUSE && p.ksplit > 1 ? u_lo * p.in_ppu : 0, s_hi = FUSE && p.ksplit > 1 ? u_hi * p.in_ppu : p.in_sx_n;
+    [[maybe_unused]] const int s_first = s_lo + (RUNS ? s_part * p.run_units * p.in_ppu : s_part);
+    [[maybe_unused]] auto run_end = [&](int run) { return (u_lo + (run + 1) * p.run_units < u_hi ? u_lo + (run + 1) * p.run_units : u_hi) * p.in_ppu; };
     [[maybe_unused]] float vx[kIn], vs[kIn];
-    auto shares = [&](const float* in, int j0, int hi, float (&v)[kSharesAhead]) {
+    auto shares = [&](const float* in, int j0, int step, int hi, float (&v)[kSharesAhead]) {
 #pragma unroll
-        for (int i = 0; i < kIn; ++i) v[i] = in[(j0 + i * kP < hi ? j0 + i * kP : 0) * (int64_t)p.M + s_m];
+        for (int i = 0; i < kIn; ++i) v[i] = in[(j0 + i * step < hi ? j0 + i * step : 0) * (int64_t)p.M + s_m];
     };
-    auto add_shares = [&](int j0, int hi, const float (&v)[kSharesAhead], float sum) {
+    auto add_shares = [&](int j0, int step, int hi, const float (&v)[kSharesAhead], float sum) {
 #pragma unroll
-        for (int i = 0; i < kIn; ++i) sum += j0 + i * kP < hi ? v[i] : 0.f;
+        for (int i = 0; i < kIn; ++i) sum += j0 + i * step < hi ? v[i] : 0.f;
         return sum;
     };
     if constexpr (FUSE) {
         if (!own && s_part < kP) {
-            shares(p.in_sx, s_lo + s_part, s_hi, vx);
-            if (p.in_ss_n > 0) shares(p.in_ss, s_part, p.in_ss_n, vs);
+            shares(p.in_sx, s_first, RUNS ? 1 : kP, RUNS ? run_end(s_part) : s_hi, vx);
+            if (p.in_ss_n > 0) shares(p.in_ss, s_part, kP, p.in_ss_n, vs);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1293,8 +1321,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] float sxs = 0.f, sss = 0.f;
     if constexpr (FUSE) {
         if (!own && s_part < kP) {
-            sxs = add_shares(s_lo + s_part, s_hi, vx, 0.f);
-            if (p.in_ss_n > 0) sss = add_shares(s_part, p.in_ss_n, vs, 0.f);
+            if constexpr (RUNS) {
+                for (int run = s_part; run < p.runs; run += kP) {
+                    float sum = 0.f;
+                    for (int j0 = s_lo + run * p.run_units * p.in_ppu, hi = run_end(run); j0 < hi; j0 += kIn) {
+                        if (run != s_part || j0 != s_first) shares(p.in_sx, j0, 1, hi, vx);
+                        sum = add_shares(j0, 1, hi, vx, sum);
+                    }
+                    runtab[run * BM + s_tok] = sum;
+                }
+            } else {
+                sxs = add_shares(s_first, kP, s_hi, vx, 0.f);
+            }
+            if (p.in_ss_n > 0) sss = add_shares(s_part, kP, p.in_ss_n, vs, 0.f);
         }
     }
     if constexpr (kScales) {
@@ -1313,8 +1352,18 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             }
         }
     }
+    if constexpr (kScales) {
+        if (own) {
+#pragma unroll
+            for (int i = 0; i < kSX; ++i) {
+                const int at = i * kThreads + (int)threadIdx.x;
+                if (RUNS && at < p.runs * BM) runtab[at] = t_sx[i];
+                if (at < BM) fr[BM + at] = RUNS ? 0.f : t_sx[i];
+            }
+        }
+    }
     if ((int)threadIdx.x < BM) {
-        if (own) fr[threadIdx.x] = t_ri, fr[BM + threadIdx.x] = t_sx;
+        if (own) fr[threadIdx.x] = t_ri;
         if constexpr (FUSE && EPI == MI355_EPI_STORE) postab[threadIdx.x] = t_pos;
     }
 
@@ -1480,13 +1529,44 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             mfmas(s, wr[s], u + DEPTH - 1, (s + DEPTH - 1) % DEPTH, more);
     };
     using std::integral_constant;
+    // the sum of a run, its levels' offset and zero points taken off, leaves the accumulators
+    [[maybe_unused]] f32x4 of_runs[RUNS ? kTPW : 1][RUNS ? kTT : 1];
+    [[maybe_unused]] int run = 0, left = p.run_units;
+    [[maybe_unused]] auto end_run = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t) {
+            const f32x4 zp = *(const f32x4*)(rowtab + (kSlots + kTPW * wave + t) * 16 + 4 * g);
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) {
+                const float x = runtab[run * BM + tt * 16 + c];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    of_runs[t][tt][r] += acc[t][tt][r] - zp[r] * x;
+                    acc[t][tt][r] = 0.f;
+                }
+            }
+        }
+        ++run;
+        left = p.run_units;
+    };
+    if constexpr (RUNS) {
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) of_runs[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     int u = u_lo;
     for (; u + DEPTH <= u_hi; u += DEPTH) {
         unit(integral_constant<int, 0>{}, u, std::true_type{});
         unit(integral_constant<int, 1>{}, u + 1, std::true_type{});
         unit(integral_constant<int, 2>{}, u + 2, std::true_type{});
         if constexpr (DEPTH == 4) unit(integral_constant<int, 3>{}, u + 3, std::true_type{});
+        if constexpr (RUNS) {
+            left -= DEPTH;
+            if (left == 0) end_run();
+        }
     }
+    [[maybe_unused]] const bool open = u < u_hi || left != p.run_units;  // the last run has units
     if (u < u_hi) {
         unit(integral_constant<int, 0>{}, u, std::false_type{});
         if (u + 1 < u_hi) {
@@ -1496,16 +1576,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             }
         }
     }
+    if constexpr (RUNS) {
+        if (open) end_run();
+#pragma unroll
+        for (int t = 0; t < kTPW; ++t)
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = of_runs[t][tt];
+    }
     if constexpr (FUSE) {
         if (p.f_in) {  // the rest of the shares
             if (s_part < kP) {
-                for (int j0 = s_lo + s_part + kIn * kP; j0 < s_hi; j0 += kIn * kP) {
-                    shares(p.in_sx, j0, s_hi, vx);
-                    sxs = add_shares(j0, s_hi, vx, sxs);
+                for (int j0 = s_first + kIn * kP; !RUNS && j0 < s_hi; j0 += kIn * kP) {
+                    shares(p.in_sx, j0, kP, s_hi, vx);
+                    sxs = add_shares(j0, kP, s_hi, vx, sxs);
                 }
                 for (int j0 = s_part + kIn * kP; j0 < p.in_ss_n; j0 += kIn * kP) {
-                    shares(p.in_ss, j0, p.in_ss_n, vs);
-                    sss = add_shares(j0, p.in_ss_n, vs, sss);
+                    shares(p.in_ss, j0, kP, p.in_ss_n, vs);
+                    sss = add_shares(j0, kP, p.in_ss_n, vs, sss);
                 }
                 frp[(s_part * 2 + 1) * BM + s_tok] = sxs;
                 frp[(s_part * 2 + 0) * BM + s_tok] = sss;
@@ -1567,17 +1654,20 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     }
     return 0;
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, bool RUNS = false>
 int launch_deep(const GemmParams& p, hipStream_t s) {
+    if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM < kBM && !RUNS) {
+        if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, true>(p, s);
+    }
     constexpr int kDepth = BM == 128 && FMT == MI355_W_BF16 ? 3 : 4;
-    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64;
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP>,
+    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0);
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP>, kLds, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>, kLds, p, s);
 }
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
 int launch_gemm_w(const GemmParams& p, hipStream_t s) {
@@ -1681,6 +1771,24 @@ int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
            (size_t)2 * (ksplit + 1) * M * row_floats * 4 <= kSplitBudget)
         ++ksplit;
     return ksplit;
+}
+// Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
+// product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows
+// number less than 96 / cuts and a run keeps 4 units; a K-slice that is longer takes several runs, each with its own operand sum.  Error beside one activation of
+// 2^17 (rms, in units of its product's last bit), N = K = 4096 / N = 4096, K = 11008 / N = 12288, K = 4096, a run per slice -> runs: 40 tokens 3.0 / 3.9 / 4.8 -> 2.6 /
+// 3.9 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.5 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.6 / 6.8; it takes a layer's products from 84.7 to 86.0 us at 37 tokens,
+// from 114 to 117 at 100 and leaves 512 as they were.  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
+void gemm_runs(int M, int N, int K, bool pair, int ksplit, int* runs, int* run_units) {
+    const int units = (K + 127) / 128, longest = (units + ksplit - 1) / ksplit;
+    const int rows_per_block = 16 * (pair ? 8 * kTPW / 2 : 8 * kTPW);
+    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + kBM - 1) / kBM);
+    int cuts = 1;
+    while (cuts < 8 && blocks * cuts < 96 && units >= 8 * cuts) cuts *= 2;
+    *runs = 1, *run_units = units;
+    const GemmShape sh = gemm_shape((N + 15) / 16, M, pair, ksplit, false);
+    if (longest <= (units + cuts - 1) / cuts || !sh.deep || sh.bm == kBM) return;
+    *run_units = units / cuts / 4 * 4;
+    *runs = (longest + *run_units - 1) / *run_units;
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
@@ -1849,6 +1957,8 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     } else {
         ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, !q4);
     }
+    int runs = 1, run_units = units;
+    if (q4 && !grouped) gemm_runs(a->M, a->N, a->K, swiglu, ksplit, &runs, &run_units);
     // producer / consumer fusion (gemm_fuse.h): whole-K launches over per-row scales only — the caller plans with
     // mi355_linear_gemm_plan
     const bool fused = f != nullptr;
@@ -1859,8 +1969,8 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         MI355_CHECK_ARG(!produces || a->N % 128 == 0, MI355_E_SHAPE, "linear_gemm: a producer of the fused chain has N %% 128 == 0 (N=%d)", a->N);
         MI355_CHECK_ARG(ksplit == 1 || !produces || a->epi == MI355_EPI_SWIGLU || a->y_dtype == MI355_F32, MI355_E_DTYPE,
                         "linear_gemm: the fused reduction of a K-split launch writes f32 rows (or the SwiGLU pair's bf16)");
-        MI355_CHECK_ARG(!f_in || ksplit == 1 || (f->in_ppu >= 1 && f->in_sx_n == units * f->in_ppu), MI355_E_ARG,
-                        "linear_gemm: a K-split consumer needs %d x in_ppu partial operand sums (got %d, in_ppu %d)", units, f->in_sx_n, f->in_ppu);
+        MI355_CHECK_ARG(!f_in || (ksplit == 1 && runs == 1) || (f->in_ppu >= 1 && f->in_sx_n == units * f->in_ppu), MI355_E_ARG,
+                        "linear_gemm: a consumer of K-slices or runs needs %d x in_ppu partial operand sums (got %d, in_ppu %d)", units, f->in_sx_n, f->in_ppu);
         MI355_CHECK_ARG(!f_in || (a->x_dtype == MI355_BF16 && a->norm_scale == nullptr && a->K % 128 == 0 && a->ldx % 8 == 0 &&
                                   (uintptr_t)a->x % 16 == 0 && f->in_sx != nullptr && f->in_sx_n > 0 && (f->in_ss == nullptr || f->in_ss_n > 0)),
                         MI355_E_ARG, "linear_gemm: a pre-staged operand is bf16 [M, ldx] with K %% 128 == 0 and partial operand sums");
@@ -1889,7 +1999,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         float* sxt = cols == 128 ? rinv + unit_sums_at(a->M) : (float*)((char*)gtab + tab_bytes);
         const GroupTables tables = {(const bf16_t*)a->scales, (const bf16_t*)a->zeros, (const bf16_t*)a->scales2, (const bf16_t*)a->zeros2, a->N, tab_ld, n_groups, a->R, gtab};
         hipLaunchKernelGGL(aligned ? stage_units_kernel<true> : stage_units_kernel<false>, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx,
-                           a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv, (float*)nullptr, 1, 1.f, 0.f, sxt, a->M, cols, tables);
+                           a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv, (float*)nullptr, 1, 1, units, 1.f, 0.f, sxt, a->M, cols, tables);
         MI355_LAUNCH_CHECK();
         p.gtab = gtab;
         p.sxt = sxt;
@@ -1898,11 +2008,12 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         p.tab_ld = tab_ld;
     } else if (!f_in && !direct && aligned && a->K % 128 == 0 && units <= kStageLds - 32) {
         hipLaunchKernelGGL(stage_units_kernel<true>, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv,
-                           sx, ksplit, a->alpha == 0.f ? 1.f : a->alpha, (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f, (float*)nullptr, a->M, 128, GroupTables{});
+                           sx, ksplit, runs, run_units, a->alpha == 0.f ? 1.f : a->alpha, (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f, (float*)nullptr, a->M, 128,
+                           GroupTables{});
         MI355_LAUNCH_CHECK();
     } else if (!f_in && !direct) {
         hipLaunchKernelGGL(stage_rows_kernel, dim3(a->M), dim3(256), 0, s, a->x, a->x_dtype, a->ldx, a->norm_scale, a->norm_dtype,
-                           a->eps, a->K, kp, xb, (int64_t)kp, rinv, sx, ksplit, a->alpha == 0.f ? 1.f : a->alpha,
+                           a->eps, a->K, kp, xb, (int64_t)kp, rinv, sx, ksplit, runs, run_units, a->alpha == 0.f ? 1.f : a->alpha,
                            (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f);
         MI355_LAUNCH_CHECK();
     }
@@ -1943,6 +2054,8 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     p.sz_dtype = a->sz_dtype;
     p.y_dtype = a->y_dtype;
     p.ksplit = ksplit;
+    p.runs = runs;
+    p.run_units = run_units;
     p.part = part;
     if (norm != nullptr) {
         norm->done = ksplit > 1 && a->epi == MI355_EPI_ACCUM && a->y_dtype == MI355_F32 && a->N <= kNormHeld * 4096;

@@ -56,6 +56,29 @@ def test_tiled_product_against_64_bits(dev, fmt, M, N, K, epi):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
+@pytest.mark.parametrize("M,N,K,run", [
+    (33, 4096, 4096, 4), (64, 4096, 4096, 4), (65, 4096, 4096, 4), (128, 4096, 11008, 11), (129, 4096, 4096, 8), (256, 4096, 11008, 22), (321, 4096, 4096, 16),
+    (512, 4096, 11008, 43), (100, 12288, 4096, 16), (40, 5120, 13824, 14), (24, 4096, 4032, 4), (50, 4096, 4000, 4),
+])
+def test_int4_sums_beside_a_large_activation(dev, M, N, K, run):
+    """Levels are summed as 128 + q: beside an activation of 2^17 an f32 sum is 2^24 and more, and each product of 32 columns costs it a rounding of that size.
+    An accumulator sums `run` units of four such products (of the N = 12288 products 1 / 2 of K, of the others 1 / 8 up to 128 tokens, 1 / 4 up to 256, 1 / 2 up to
+    640), and only the one with that activation is so large.  A product adds its 32 terms in a few steps, five roundings to the nearest at most: 5 / 12 of a squared
+    last bit each, so the rms is sqrt(4 run 5 / 12) last bits (the operand sum's own roundings and the sample: 6 %).  The activation's own levels are its rows' zero points: its share of the result is 0."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    q = torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8)
+    z = torch.randint(5, 11, (N,), generator=g, device=dev)
+    q[:, 0] = z.to(torch.uint8)
+    s = torch.full((N,), 2.0 ** -6, device=dev).to(torch.float32 if M < 32 else torch.bfloat16)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    x[:, 0] = 2.0 ** 17
+    ref = x.double() @ ((q.double() - z.double()[:, None]) * 2.0 ** -6).T
+    stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
+    got = ops.linear_gemm(x, stream, 1, N, K, scales=s, zeros=z.to(s.dtype), out_dtype=torch.float32).double()
+    last_bit = 2.0 ** -6 * 2.0  # 128 x 2^17 = 2^24 and up to 2^24.2
+    assert (got - ref).square().mean().sqrt() <= 1.06 * (4 * run * 5 / 12) ** 0.5 * last_bit
+
+
 @pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K,cols", [(1, 16, 256, 128), (16, 144, 2176, 128), (17, 4096, 1280, 256), (33, 12288, 512, 128), (64, 128, 11008, 512), (65, 4096, 4096, 128),
                                         (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128)])
@@ -104,3 +127,24 @@ def test_short_rows_in_four_waves_give_the_bits_of_eight(dev, N, K, M):
               out_dtype=torch.float32)
     stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
     assert torch.equal(ops.linear_fast(x, stream, nat.W_Q4, 1, N, K, **kw), ops.linear_fast(x, stream, nat.W_Q4, 1, N, K, waves=8, **kw))
+
+
+@pytest.mark.parametrize("T", [33, 64, 100])
+def test_runs_of_shares_in_the_fused_prompt_chain(dev, monkeypatch, T):
+    """Slices of several runs whose operand sums come as shares of the producer: one per unit, or two (c_fc1 / c_fc2 in blocks of 64 rows, up to 64 tokens).  The
+    chain with staging passes in place of shares rounds the same operands and sums in another order, as does the rotation of q and k: 0.02 of the logits' spread, the
+    bound of the chain at 7B width; a run that took another one's sum would be off by the spread of 135 operands."""
+    cfg = LLaMAConfig(block_size=128, n_layer=2, n_head=15, n_embd=1920, vocab_size=512)  # hidden rows of 5120: 40 units
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode="gptq.int4"):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode="gptq.int4", device="cuda", dtype=torch.bfloat16))
+    model.eval()
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
+        model.reset_cache()
+        with torch.no_grad():
+            out.append(model(idx.view(1, -1), 128, torch.arange(T, device=dev))[0].float())
+    assert not torch.equal(*out)  # (the chain was on)
+    assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
