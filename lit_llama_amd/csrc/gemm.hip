@@ -151,10 +151,12 @@ constexpr int kMaxRuns = 8;
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
-__host__ __device__ __forceinline__ int slice_lo(int s, int units, int ksplit) { return (int)((int64_t)s * units / ksplit); }
+__host__ __device__ __forceinline__ int slice_lo(int s, int units, int ksplit) { return (int)((unsigned)(s * units) / (unsigned)ksplit); }  // (s <= 16: 32 bits do)
 // first unit of run i = slice * runs + run of a row cut into `ksplit` slices of `runs` runs (run i = units [run_lo(i), run_lo(i + 1)), possibly none)
 __device__ __forceinline__ int run_lo(int i, int units, int ksplit, int runs, int run_units) {
-    const int ks = i / runs, lo = slice_lo(ks, units, ksplit) + (i - ks * runs) * run_units, hi = slice_lo(ks + 1, units, ksplit);
+    if (runs == 1) return slice_lo(i, units, ksplit);
+    const unsigned ks = (unsigned)i / (unsigned)runs;
+    const int lo = slice_lo(ks, units, ksplit) + (i - (int)ks * runs) * run_units, hi = slice_lo(ks + 1, units, ksplit);
     return lo < hi ? lo : hi;
 }
 
@@ -298,8 +300,9 @@ __global__ __launch_bounds__(256) void stage_units_kernel(const void* x, int x_d
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
     if (sxt == nullptr) {  // (every wave has passed the block sum's barriers: the units' sums stand in LDS)
         for (int s = threadIdx.x; s < ksplit * runs; s += 256) {
+            const int u_lo = run_lo(s, K >> 7, ksplit, runs, run_units), u_hi = run_lo(s + 1, K >> 7, ksplit, runs, run_units);
             double sum = 0.;  // (one rounding beside a large unit, not one per unit)
-            for (int u = run_lo(s, K >> 7, ksplit, runs, run_units); u < run_lo(s + 1, K >> 7, ksplit, runs, run_units); ++u) sum += per_unit[u];
+            for (int u = u_lo; u < u_hi; ++u) sum += per_unit[u];
             sx[(int64_t)m * (ksplit * runs) + s] = (float)sum;
         }
     }
