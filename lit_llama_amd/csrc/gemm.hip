@@ -1683,9 +1683,11 @@ int launch_gemm_w(const GemmParams& p, hipStream_t s) {
     }
     return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
 }
-struct GemmShape {
+// How a launch of one scale per row is cut: waves and tokens of a block, gemm_deep_kernel (or gemm_q4_kernel), K-slices
+struct GemmCut {
     int waves, bm;
     bool deep;
+    int ksplit;
 };
 // tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep", 0 = the rule's choice
 struct GemmForce {
@@ -1704,42 +1706,96 @@ GemmForce gemm_force() {
     }();
     return f;
 }
-// Waves of a block (what the share layout of mi355_linear_gemm_plan depends on).  Up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them,
-// which 4-5 K-slices bring to a workgroup for two CUs of three; 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, int4 with staging:
-// 20.5 us against 22.7).  Longer int4 prompts likewise while the 256-row blocks leave half of the CUs idle, except where the 128-row blocks of a launch without
-// slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096, 128 tokens 29.3 / 24.5 us, 512 38.9 / 32.0; N = 12288, 128 tokens 34.6 / 29.6;
-// K = 11008, 300 tokens 57.5 / 64.0, 512 71.2 / 66.7).  The SwiGLU pair does not gain (128 tokens 36.5 / 39.4).
-int gemm_waves(int M, int N, bool pair, bool bf16) {
-    if (gemm_force().waves) return gemm_force().waves;
-    const int blocks8 = (N + 255) / 256 * ((M + 63) / 64);
-    return M <= 64 || (!bf16 && !pair && (blocks8 <= 64 || (blocks8 >= 96 && blocks8 <= 128))) ? 4 : 8;
+// blocks of `waves` waves and `bm` tokens
+int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
+    const int rows = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
+    return (N + rows - 1) / rows * ((M + bm - 1) / bm);
 }
+// bytes of the K-slices' partial sums
+size_t gemm_part_bytes(int M, int N, bool pair, int ksplit) { return (size_t)ksplit * M * N * (pair ? 2 : 1) * 4; }
 // (blocks of 48 tokens, int4: N = 12288 / 11008 pair, K = 4096, 37 tokens 22.9 / 25.1 us with blocks of 64, 21.7 / 23.3 with 48, groups of 128 columns 29.5 / 36.0 and
 // 27.4 / 33.6; BF16, bound by the weights, the same either way)
 int short_block(int M, bool bf16) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 48 && !bf16 ? 48 : 64; }
-// Tokens per block and kernel.  Blocks of 128 tokens x 256 rows with two workgroups per CU (gemm_q4_kernel) when a launch has a few of them per CU: 2048
-// tokens, int4, c_fc1/c_fc2 271 us against 303 (gemm_deep_kernel, one workgroup per CU), c_attn 158 / 174.  Fewer: 64-token blocks, twice as many, of the
-// deep kernel: 128 tokens, int4, c_fc1/c_fc2 49.6 -> 39.9 us, 777 tokens N = 4096 47.8 -> 42.1 us.  An int4 launch of exactly one 128-token block per CU (N = 4096
-// at 2048 tokens) keeps those.  BF16 streams are bound by the weight bytes a CU requests per product (a 64-token block requests twice a 128-token block's), so
-// they keep 128 tokens as long as those blocks cover 5/8 of the CUs: 512 tokens, c_fc1/c_fc2 134 / 106 us; up to one block per CU through the deep
-// kernel: 2048 tokens, N = 4096, K = 11008 174 -> 158 us.
-GemmShape gemm_shape(int n_tiles, int M, bool pair, int ksplit, bool bf16) {
+
+// Int4.  Waves of a block: up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them, which 4-5 K-slices bring to a workgroup for two CUs of three;
+// 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, with staging: 20.5 us against 22.7).  Longer prompts likewise while the 256-row
+// blocks leave half of the CUs idle, except where the 128-row blocks of a launch without slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096,
+// 128 tokens 29.3 / 24.5 us, 512 38.9 / 32.0; N = 12288, 128 tokens 34.6 / 29.6; K = 11008, 300 tokens 57.5 / 64.0, 512 71.2 / 66.7).  The SwiGLU pair does
+// not gain (128 tokens 36.5 / 39.4).
+// Slices: as many as bring the launch to the workgroups wanted, none below 6 units.  Their sums, written and read again, take at most half the partial buffer,
+// 16 MB: past that a slice costs more than the CUs that it fills (1 / 2 slices, 600 tokens, N = 4096: K = 4096 38.1 / 45.6 us, 11008 77 / 84; 120, N = 11008 pair 35.4 /
+// 42.1).  Blocks of 4 waves stop at one workgroup per CU: a few more than 256 leave the chip to those few (37 rows, K = 11008, N = 4096: 28.4 / 26.7 / 25.6 /
+// 24.7 with 4 / 5 / 6 / 8).
+// Tokens: blocks of 128 x 256 rows with two workgroups per CU (gemm_q4_kernel) when a launch has a few of them per CU: 2048 tokens, c_fc1/c_fc2 271 us against
+// 303 (gemm_deep_kernel, one workgroup per CU), c_attn 158 / 174.  Fewer: 64-token blocks, twice as many, of the deep kernel: 128 tokens, c_fc1/c_fc2 49.6 -> 39.9
+// us, 777 tokens N = 4096 47.8 -> 42.1 us.  A launch of exactly one 128-token block per CU (N = 4096 at 2048 tokens) keeps those.
+GemmCut q4_cut(int M, int N, int K, bool pair) {
+    const int units = (K + 127) / 128, blocks8 = (N + 255) / 256 * ((M + 63) / 64);
+    GemmCut cut = {M <= 64 || (!pair && (blocks8 <= 64 || (blocks8 >= 96 && blocks8 <= 128))) ? 4 : 8, short_block(M, false), true, 1};
+    const int blocks = gemm_blocks(M, N, pair, cut.waves, 64), want = cut.waves == 8 ? 192 : 256, most = cut.waves == 8 ? 1 << 20 : 256;
+    while (cut.ksplit < 8 && blocks * cut.ksplit < want && blocks * (cut.ksplit + 1) <= most && units >= 6 * (cut.ksplit + 1) &&
+           gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
+        ++cut.ksplit;
+    const int wide = gemm_blocks(M, N, pair, 8, kBM) * cut.ksplit;
+    if (wide >= 384 || wide == 256) cut.bm = kBM, cut.deep = false;
+    return cut;
+}
+// BF16 streams.  From 192 blocks of 128 tokens x 256 rows on those, one per CU of the deep kernel, more of gemm_q4_kernel (2048 tokens, N = 4096, K = 11008 174 -> 158 us;
+// 512 tokens, c_fc1/c_fc2 134 / 106 us with blocks of 64 / 128).  Up to 64 tokens blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
+// none to a few more than all (16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 /
+// 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13).  In between, and where those blocks are more than the CUs, what an estimate takes for the fastest: the busiest CU's workgroups one behind the
+// other, `start` and `unit` us for each of their units; the weights from HBM at 6.6 TB/s behind 4.3 us, both at once; and with slices 1.6 us and 1 us per
+// 2.3 MB of partial sums.  Fitted to 17 000 launches (28 products of 1024 to 32000 rows, 8 to 2000 tokens, weights not in any cache: the next layer's never are)
+// within 8 % rms; its choice is 1 % behind the fastest on average.  Blocks of 8 waves throughout, from 65 tokens on, with slices
+// to three quarters of the CUs, a rule from weights that the cache held, took 31.5 us for 160 tokens of N = K = 5120 (now 27.1), 52 / 116 for 256 / 640 of
+// N = 4096, K = 11008 (43 / 83), 107 for 128 of N = 8192, K = 22016 (87); 280 blocks of 4 waves 115 for 48 of the N = 17920 pair, K = 6656 (101).
+GemmCut bf16_cut(int M, int N, int K, bool pair) {
+    const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
+    if (M > 128 && wide >= 192) return {8, kBM, wide <= 256, 1};
+    GemmCut cut = {4, short_block(M, true), true, 1};
+    if (M <= 64 && few <= 256) {
+        while (cut.ksplit < kMaxSplit && few * cut.ksplit < 192 && few * (cut.ksplit + 1) <= 256 && units >= 4 * (cut.ksplit + 1) &&
+               gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
+            ++cut.ksplit;
+        return cut;
+    }
+    struct Kind {
+        int waves, bm;
+        bool deep;
+        float start, unit;
+    };
+    const Kind kinds[] = {{4, cut.bm, true, cut.bm == 16 ? 0.9f : cut.bm == 32 ? 1.3f : 3.0f, cut.bm == 16 ? 0.67f : cut.bm == 32 ? 0.71f : 0.75f},
+                          {8, 64, true, 4.2f, 1.27f}, {8, 64, false, 3.4f, 1.23f}, {8, kBM, true, 6.6f, 1.48f}};
+    const float bytes = 2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N, hbm = 4.3f + bytes / 6.6e6f;
+    float best = 0.f;
+    for (const Kind& k : kinds)
+        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || units >= 4 * ks); ++ks) {
+            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks;
+            const size_t part = gemm_part_bytes(M, N, pair, ks);
+            // (128-token blocks: no two on a CU, and with slices the last CUs slow the others: 300 tokens, K = 11008, N = 4096 49.7 us with 192, 58.5 with 240)
+            if ((ks > 1 && part > kSplitBudget) || (k.bm == kBM && (M <= 64 || blocks > (ks == 1 ? 256 : 208)))) continue;
+            const float work = k.start + (float)((blocks + 255) / 256 * ((units + ks - 1) / ks)) * k.unit;
+            const float us = sqrtf(work * work + hbm * hbm) + (ks == 1 ? 0.f : 1.6f + (float)part / 2.3e6f);
+            if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, k.deep, ks};
+        }
+    return cut;
+}
+GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16) {
     const GemmForce fo = gemm_force();
-    GemmShape sh = {gemm_waves(M, n_tiles * 16, pair, bf16), short_block(M, bf16), true};
-    const int per_block8 = pair ? 8 * kTPW / 2 : 8 * kTPW;
-    const int blocks8 = ((n_tiles + per_block8 - 1) / per_block8) * ((M + kBM - 1) / kBM) * ksplit;  // of 128 tokens
-    if (bf16 ? M > 128 && blocks8 >= 160 : blocks8 >= 384 || blocks8 == 256) sh.bm = 128, sh.deep = bf16 && blocks8 <= 256;
-    if (fo.bm) sh.bm = fo.bm;
-    if (fo.deep) sh.deep = fo.deep == 1;
-    return sh;
+    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair) : q4_cut(M, N, K, pair);
+    if (fo.waves) cut.waves = fo.waves;
+    if (fo.bm) cut.bm = fo.bm;
+    if (fo.deep) cut.deep = fo.deep == 1;
+    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= kSplitBudget / 2) cut.ksplit = fo.ksplit;
+    return cut;
 }
 // Grouped scales, groups of whole units.  Blocks of 256 rows x 64 tokens and of 256 x 128 fill a CU alone, two of 128 x 64 share one; per round of the chip
 // they take 1 : 1.75 : 1, a round of at most one 128 x 64 block per CU 0.75 (N = 4096, K = 11008: 256 x 64 blocks 104 us at 512 tokens, 106 at 777, 108 at 1000;
 // 256 x 128 165 / 168 / 169; 128 x 64 78 / 106 / 114): the fewest.  1000 tokens, 7B: 235 / 101 / 137 us for c_fc1 / c_fc2, c_proj on average, c_attn with blocks
 // of 64 x 128 one unit ahead -> 185 / 75 / 120.
-GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
+GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
     const GemmForce fo = gemm_force();
-    GemmShape sh = {4, short_block(M, false), true};
+    GemmCut sh = {4, short_block(M, false), true, ksplit};
     if (M > 64) {
         auto blocks = [&](int waves, int bm) {
             const int per_block = pair ? waves * kTPW / 2 : waves * kTPW;
@@ -1748,7 +1804,7 @@ GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
         const int half = blocks(4, 64), full = blocks(8, 64), wide = blocks(8, 128);
         const int t_half = half / 512 * 4 + (half % 512 == 0 ? 0 : half % 512 <= 256 ? 3 : 4), t_full = (full + 255) / 256 * 4, t_wide = (wide + 255) / 256 * 7;
         if (t_wide < t_half && t_wide <= t_full)
-            sh = {8, 128, true};
+            sh = {8, 128, true, ksplit};
         else if (t_full <= t_half)
             sh.waves = 8;
     }
@@ -1756,46 +1812,24 @@ GemmShape gemm_shape_grouped(int n_tiles, int M, bool pair, int ksplit) {
     if (fo.bm) sh.bm = fo.bm;
     return sh;
 }
-// Split-K of an ungrouped launch: as many slices as bring it to the workgroups wanted, none below 6 units (BF16: 4) or past the partial buffer.  Blocks of 4
-// waves stop at one workgroup per CU: a few more than 256 leave the chip to those few (bf16, 16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us
-// with 1 / 2 / 3 / 4 slices; the c_fc1 / c_fc2 pair of 172 blocks 34.5 with 1, 42.8 with 3), and three quarters of them are as good for BF16 and cheaper to
-// sum (K = 11008, N = 4096, 32 blocks: 24.2 / 21.9 / 21.3 / 21.9 / 23.2 us with 4 / 5 / 6 / 8 / 13; int4, 37 rows: 28.4 / 26.7 / 25.6 / 24.7 with 4 / 5 / 6 / 8).
-int gemm_ksplit(int M, int N, int K, bool pair, bool bf16) {
-    const int units = (K + 127) / 128;
-    const size_t row_floats = (size_t)N * (pair ? 2 : 1);
-    if (const int fk = gemm_force().ksplit) {
-        if (fk >= 1 && fk <= kMaxSplit && units >= fk && (size_t)2 * fk * M * row_floats * 4 <= kSplitBudget) return fk;
-    }
-    const int waves = gemm_waves(M, N, pair, bf16);
-    const int rows_per_block = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
-    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), want = bf16 || waves == 8 ? 192 : 256, most = waves == 8 ? 1 << 20 : 256;
-    int ksplit = 1;
-    while (ksplit < (bf16 ? kMaxSplit : 8) && blocks * ksplit < want && blocks * (ksplit + 1) <= most && units >= (bf16 ? 4 : 6) * (ksplit + 1) &&
-           (size_t)2 * (ksplit + 1) * M * row_floats * 4 <= kSplitBudget)
-        ++ksplit;
-    return ksplit;
-}
 // Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
 // product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows
 // number less than 96 / cuts and a run keeps 4 units; a K-slice that is longer takes several runs, each with its own operand sum.  Error beside one activation of
 // 2^17 (rms, in units of its product's last bit), N = K = 4096 / N = 4096, K = 11008 / N = 12288, K = 4096, a run per slice -> runs: 40 tokens 3.0 / 3.9 / 4.8 -> 2.6 /
 // 3.9 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.5 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.6 / 6.8; it takes a layer's products from 84.7 to 86.0 us at 37 tokens,
 // from 114 to 117 at 100 and leaves 512 as they were.  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
-void gemm_runs(int M, int N, int K, bool pair, int ksplit, int* runs, int* run_units) {
-    const int units = (K + 127) / 128, longest = (units + ksplit - 1) / ksplit;
-    const int rows_per_block = 16 * (pair ? 8 * kTPW / 2 : 8 * kTPW);
-    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + kBM - 1) / kBM);
+void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, int* run_units) {
+    const int units = (K + 127) / 128, longest = (units + cut.ksplit - 1) / cut.ksplit, blocks = gemm_blocks(M, N, pair, 8, kBM);
     int cuts = 1;
     while (cuts < 8 && blocks * cuts < 96 && units >= 8 * cuts) cuts *= 2;
     *runs = 1, *run_units = units;
-    const GemmShape sh = gemm_shape((N + 15) / 16, M, pair, ksplit, false);
-    if (longest <= (units + cuts - 1) / cuts || !sh.deep || sh.bm == kBM) return;
+    if (longest <= (units + cuts - 1) / cuts || !cut.deep || cut.bm == kBM) return;
     *run_units = units / cuts / 4 * 4;
     *runs = (longest + *run_units - 1) / *run_units;
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
-    const GemmShape sh = gemm_shape(p.n_tiles, p.M, PAIR, p.ksplit, FMT == MI355_W_BF16);
+    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16);
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, FMT, 4, 32, FUSE>(p, s);
@@ -1803,6 +1837,9 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
             if (sh.bm == 48) return launch_deep<EPI, PAIR, FMT, 4, 48, FUSE>(p, s);
         }
         return launch_deep<EPI, PAIR, FMT, 4, 64, FUSE>(p, s);
+    }
+    if constexpr (FMT == MI355_W_BF16) {
+        if (sh.bm == 64 && !sh.deep) return launch_gemm_w<EPI, PAIR, FMT, 8, 64, 0, FUSE>(p, s);
     }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 8, 64, FUSE>(p, s);
     if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
@@ -1820,7 +1857,7 @@ int launch_gemm_subgroups(const GemmParams& p, hipStream_t s) {
 template <int EPI, bool PAIR>
 int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
     if (subgroups) return launch_gemm_subgroups<EPI, PAIR>(p, s);
-    const GemmShape sh = gemm_shape_grouped(p.n_tiles, p.M, PAIR, p.ksplit);
+    const GemmCut sh = gemm_cut_grouped(p.n_tiles, p.M, PAIR, p.ksplit);
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, false, 1>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, false, 1>(p, s);
@@ -1866,15 +1903,14 @@ extern "C" int mi355_linear_gemm(const mi355_linear_args* a, void* workspace, si
     return mi355_linear_gemm_fused(a, nullptr, workspace, workspace_bytes, stream);
 }
 
-void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
+extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
     const bool pair = R == 2;
-    const int ks = gemm_ksplit(M, N, K, pair, bf16);
+    const GemmCut cut = gemm_cut(M, N, K, pair, bf16);
     // rows (hidden rows of a pair stream) behind one share of a producer's partial sums: a 128-column unit when the K-slices'
     // reduction writes them or a block holds 256 rows, else the block's rows
-    const int waves = gemm_waves(M, N, pair, bf16);
-    int rows = (pair ? waves * kTPW / 2 : waves * kTPW) * 16;
-    if (ks > 1 || rows > 128) rows = 128;
-    *ksplit = ks;
+    int rows = (pair ? cut.waves * kTPW / 2 : cut.waves * kTPW) * 16;
+    if (cut.ksplit > 1 || rows > 128) rows = 128;
+    *ksplit = cut.ksplit;
     *shares = (N + rows - 1) / rows;
     *shares_per_unit = 128 / rows;
 }
@@ -1952,16 +1988,18 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         const size_t row_floats = (size_t)a->N * (swiglu ? 2 : 1);
         const int cuts = scale_groups && a->group_cols >= 128 ? n_groups : units;
         if (unit_sums)
-            ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, false);
+            ksplit = gemm_cut(a->M, a->N, a->K, swiglu, false).ksplit;  // (partial sums: at most half the region, the tables lie in the other)
         else
             while (ksplit < kMaxSplit && blocks * ksplit < 256 && cuts >= 8 * ksplit && tab_bytes + sxt_bytes <= kSplitBudget / 2 &&
                    (size_t)2 * ksplit * a->M * row_floats * 4 <= kSplitBudget / 2)
                 ksplit *= 2;
-    } else {
-        ksplit = gemm_ksplit(a->M, a->N, a->K, swiglu, !q4);
     }
     int runs = 1, run_units = units;
-    if (q4 && !grouped) gemm_runs(a->M, a->N, a->K, swiglu, ksplit, &runs, &run_units);
+    if (!grouped) {
+        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4);
+        ksplit = cut.ksplit;
+        if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
+    }
     // producer / consumer fusion (gemm_fuse.h): whole-K launches over per-row scales only — the caller plans with
     // mi355_linear_gemm_plan
     const bool fused = f != nullptr;

@@ -46,7 +46,7 @@ struct mi355_gemm_fuse {
 // how a launch of the wide GEMM is cut: K-slices (1 = none), the partial sums ("shares") a producer writes per row and how
 // many of them make a 128-column unit.  A launch split over K produces through the reduction of its slices
 // (splitk_fused_reduce_kernel), one share per unit.
-void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
+extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
 // bytes mi355_linear_gemm_workspace_bytes reserves at the END of a workspace for the chain's partial sums
 size_t mi355_linear_gemm_fuse_scratch_bytes();
 // The RMSNorm of the rows that a residual product (MI355_EPI_ACCUM, f32 y without gaps up to N) leaves: xb[m] = bf16(norm(y[m]) (scale + add)), rows of N.

@@ -622,3 +622,32 @@ def test_int8_row_absmax_from_the_largest_staged_magnitude_statement():
         q1 = np.rint(xh.astype(np.float32) * inv).astype(np.int8)
         q2 = np.where(outl, 0, np.rint(xh.astype(np.float32) * (np.float32(127.0) / amax2))).astype(np.int8)
         assert np.array_equal(q1, q2)
+
+
+def _gemm_plan(M, N, K, R, bf16):
+    """K-slices, shares and shares per 128 columns of a launch of the tiled product (csrc/gemm_fuse.h)."""
+    import ctypes as C
+
+    out = [C.c_int(0) for _ in range(3)]
+    nat.lib().mi355_linear_gemm_plan(M, N, K, R, C.c_bool(bf16), *[C.byref(o) for o in out])
+    return tuple(o.value for o in out)
+
+
+@pytest.mark.parametrize("M,N,K,R,slices", [
+    # slices of bf16 rows: as many as an estimate of the busiest CU, of HBM and of the partial sums takes for the fastest, not as many as reach a number of workgroups
+    (256, 4096, 11008, 1, 4), (640, 4096, 11008, 1, 2), (160, 5120, 5120, 1, 2), (128, 8192, 22016, 1, 6), (330, 6656, 17920, 1, 2), (200, 2816, 1024, 2, 1), (16, 17920, 6656, 2, 4),
+    # up to 64 tokens and with a launch of many blocks: rules of their own
+    (16, 4096, 4096, 1, 6), (64, 4096, 11008, 1, 6), (16, 11008, 4096, 2, 1), (777, 12288, 4096, 1, 1), (2048, 4096, 11008, 1, 1),
+])
+def test_slices_of_bf16_rows(M, N, K, R, slices):
+    assert _gemm_plan(M, N, K, R, True)[0] == slices
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_partial_sums_of_slices_fit_their_buffer(bf16):
+    """Of int4 they stay in the half of the region that group tables leave."""
+    for N, K, R in [(4096, 4096, 1), (12288, 4096, 1), (11008, 4096, 2), (4096, 11008, 1), (8192, 22016, 1), (2048, 8192, 1), (768, 23000, 1), (128, 65536, 1)]:
+        for M in list(range(1, 70)) + list(range(70, 2049, 13)):
+            ks, shares, ppu = _gemm_plan(M, N, K, R, bf16)
+            assert 1 <= ks <= 16 and ks * M * N * R * 4 <= (32 if bf16 else 16) << 20 or ks == 1
+            assert (ks == 1 or ppu == 1) and shares * 128 >= N * ppu
