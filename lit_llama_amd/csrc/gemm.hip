@@ -1689,22 +1689,24 @@ struct GemmCut {
     bool deep;
     int ksplit;
 };
-// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep", 0 = the rule's choice
+// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel), 0 = the rule's choice.  A cut that no kernel is
+// instantiated for is ignored as a whole, a number of slices that does not fit by itself
 struct GemmForce {
     int waves, bm, ksplit, deep;
 };
 GemmForce gemm_force() {
     // parsed ONCE per process (a change of the variable between mi355_linear_gemm_plan and the launch would desynchronise the share layout of
     // the fused chain)
-#ifndef MI355_GEMM_SWEEP
-    static
-#endif
-    const GemmForce f = [] {
+    static const GemmForce f = [] {
         GemmForce g = {0, 0, 0, 0};
         if (const char* e = getenv("MI355_GEMM_FORCE")) sscanf(e, "%d:%d:%d:%d", &g.waves, &g.bm, &g.ksplit, &g.deep);
         return g;
     }();
     return f;
+}
+bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (the kernels of launch_gemm())
+    if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
+    return c.waves == 8 && (c.bm == kBM || (c.bm == 64 && (c.deep || bf16)));
 }
 // blocks of `waves` waves and `bm` tokens
 int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
@@ -1783,9 +1785,8 @@ GemmCut bf16_cut(int M, int N, int K, bool pair) {
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16) {
     const GemmForce fo = gemm_force();
     GemmCut cut = bf16 ? bf16_cut(M, N, K, pair) : q4_cut(M, N, K, pair);
-    if (fo.waves) cut.waves = fo.waves;
-    if (fo.bm) cut.bm = fo.bm;
-    if (fo.deep) cut.deep = fo.deep == 1;
+    const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep == 1 : cut.deep, cut.ksplit};
+    if (launch_gemm_has(forced, bf16)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= kSplitBudget / 2) cut.ksplit = fo.ksplit;
     return cut;
 }
@@ -1808,9 +1809,8 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
         else if (t_full <= t_half)
             sh.waves = 8;
     }
-    if (fo.waves) sh.waves = fo.waves;
-    if (fo.bm) sh.bm = fo.bm;
-    return sh;
+    const GemmCut forced = {fo.waves ? fo.waves : sh.waves, fo.bm ? fo.bm : sh.bm, true, ksplit};
+    return launch_gemm_has(forced, false) ? forced : sh;
 }
 // Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
 // product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows

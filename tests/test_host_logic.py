@@ -651,3 +651,30 @@ def test_partial_sums_of_slices_fit_their_buffer(bf16):
             ks, shares, ppu = _gemm_plan(M, N, K, R, bf16)
             assert 1 <= ks <= 16 and ks * M * N * R * 4 <= (32 if bf16 else 16) << 20 or ks == 1
             assert (ks == 1 or ppu == 1) and shares * 128 >= N * ppu
+
+
+def _forced_plans(value):
+    """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
+    import os
+    import subprocess
+    import sys
+
+    code = ("import ctypes as C, sys\n"
+            "plan = C.CDLL(sys.argv[1]).mi355_linear_gemm_plan\n"
+            "for M in (20, 40, 100, 300, 700, 2000):\n"
+            "    for N, K, R in ((4096, 4096, 1), (12288, 4096, 1), (11008, 4096, 2), (4096, 11008, 1)):\n"
+            "        for bf16 in (True, False):\n"
+            "            o = [C.c_int(0) for _ in range(3)]\n"
+            "            plan(M, N, K, R, C.c_bool(bf16), *[C.byref(v) for v in o])\n"
+            "            print(M, N, K, R, bf16, *[v.value for v in o])\n")
+    out = subprocess.run([sys.executable, "-c", code, str(nat.LIB_PATH)], env={**os.environ, "MI355_GEMM_FORCE": value}, capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    return out.stdout
+
+
+def test_a_forced_cut_without_a_kernel_changes_nothing():
+    """What a launch writes as shares, what the next one adds up and the slices come from one cut: one that no kernel is instantiated for must reach none of them."""
+    rule = _forced_plans("")
+    for force in ("2:128:0", "1:0:0", "16:64:0", "8:32:0", "4:128:0", "8:16:0", "8:96:0", "0:7:0", "4:64:0:2"):
+        assert _forced_plans(force) == rule, force
+    assert _forced_plans("8:128:0") != rule
