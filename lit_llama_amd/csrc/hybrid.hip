@@ -361,6 +361,13 @@ int ew_blocks(int64_t n) {
 
 enum { kStore = 0, kRelu2 = 1, kResidual = 2, kGeglu = 3, kLogits = 4 };
 
+// A bf16 product of M rows by tiles.  The weight-streaming kernel takes up to 8 rows; from there on, and for operands that leave its LDS room for a few rows only, the tiled
+// product (split over K, the operand read in place) moves the weights faster: 4096 x 16512 at 4 / 8 / 16 rows 57 / 118 / 251 us against
+// 28 / 28 / 30, 16512 x 4096 with the norm at 8 / 16 rows 31 / 41 against 35 / 36
+bool tiled(const mi355_proj& w, int M, int R, bool norm) {
+    return M > 8 || mi355_linear_max_rows(MI355_W_BF16, w.K, R, 0) < M || (M > 2 && !norm && w.K > 12288 && w.K % 128 == 0);
+}
+
 // y[M, N] (+)= alpha * W norm(x), or what a feed-forward makes of it; alpha: residual_mult (kResidual), logit_scale (kLogits), 1.  x f32 with `norm`, or dtype without.
 // kResidual: *ready = the norm `next` of the new rows stands in m->xb (if it could be had with the product); with `norm`: whether this one does
 int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int64_t ldx, const void* norm, int what, void* y, int64_t ldy,
@@ -412,12 +419,7 @@ int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int6
     a.alpha = what == kResidual ? m->residual_mult : what == kLogits ? m->logit_scale : 1.f;
     a.y_dtype = y_dtype;
     a.ldy = ldy;
-    const int most = mi355_linear_max_rows(MI355_W_BF16, w.K, a.R, 0);
-    // The weight-streaming kernel up to 8 rows; from there on, and for operands that leave its LDS room for a few rows only, the tiled
-    // product (split over K, the operand read in place) moves the weights faster: 4096 x 16512 at 4 / 8 / 16 rows 57 / 118 / 251 us against
-    // 28 / 28 / 30, 16512 x 4096 with the norm at 8 / 16 rows 31 / 41 against 35 / 36
-    const bool wide = M > 8 || most < M || (M > 2 && norm == nullptr && w.K > 12288 && w.K % 128 == 0);
-    if (wide) {
+    if (tiled(w, M, a.R, norm != nullptr)) {
         a.x = x;
         a.y = y;
         a.M = M;
@@ -704,9 +706,12 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
     }
     const int runs = run_end < m->n_runs ? run_end : m->n_runs;
     bool ready = false;  // the norm that the next product takes stands in m->xb
+    // ... of rows in front of a product that takes them from there: one of tiles (the row kernel norms its rows itself; with 4 rows of a hidden layer of 16512 the
+    // norm was a launch of 4 workgroups for nothing)
+    auto norm_of = [&](const void* norm, const mi355_proj& w, int R) { return tiled(w, M, R, true) ? norm : nullptr; };
     auto norm_behind = [&](int r) -> const void* {  // ... of the rows that layer r leaves, where the product behind it reads nothing else
-        if (r + 1 < runs) return m->layers[r + 1].parallel || m->layers[r + 1].sandwich ? nullptr : m->layers[r + 1].norm1;
-        return runs == m->n_runs && n_want > 0 && want == nullptr && m->norm_groups == 0 ? m->final_norm : nullptr;
+        if (r + 1 < runs) return m->layers[r + 1].parallel || m->layers[r + 1].sandwich ? nullptr : norm_of(m->layers[r + 1].norm1, m->layers[r + 1].in, 1);
+        return runs == m->n_runs && n_want > 0 && want == nullptr && m->norm_groups == 0 ? norm_of(m->final_norm, m->head, 1) : nullptr;
     };
     for (int r = 0; r < runs; ++r) {
         const mi355_hybrid_layer& l = m->layers[r];
@@ -770,7 +775,7 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
             if (int rc = parallel_out(m, l, M, s)) return rc;
             continue;
         }
-        const void* after = l.mlp == MI355_MLP_EXPERTS ? nullptr : l.mlp != MI355_MLP_NONE ? l.norm2 : norm_behind(r);
+        const void* after = l.mlp == MI355_MLP_EXPERTS ? nullptr : l.mlp != MI355_MLP_NONE ? norm_of(l.norm2, l.up, l.mlp == MI355_MLP_GEGLU ? 2 : 1) : norm_behind(r);
         if (int rc = linear(m, l.out, m->att, m->ld_att, nullptr, kResidual, m->x, m->ldx, MI355_F32, M, s, &ready, after)) return rc;
         if (l.mlp == MI355_MLP_EXPERTS) {
             mi355_experts_args e = l.moe;

@@ -479,3 +479,32 @@ def test_norm_behind_the_slices_of_a_residual_product(dev, width, batch):
     for i, t in enumerate(seqs):
         # (both sides round the same values to bf16; a value at the edge of a rounding falls either way: a few 2^-9 of the terms over four products)
         assert rel(got[:, i].float(), steps([t])[:, 0].float()) < 4e-2, i
+
+
+@pytest.mark.parametrize("batch,taken", [(4, False), (8, False), (9, True)])
+def test_norm_of_rows_only_in_front_of_a_product_that_takes_it(dev, batch, taken):
+    """Hidden rows of more than 12288 leave through the tiled product from 3 rows on, with its K-slices' sum; what stands behind them takes rows that are normed
+    already only if it is tiled too, from 9 rows on.  Before that nobody writes (or reads) normed rows."""
+    from lit_llama_amd.hybrid_engine import Entry
+
+    att = {"type": "attention", "mixer": {"heads": 9, "kv_heads": 3, "dim": 128, "vdim": 128, "scale": 0.09, "mask": {"size": 19}}}
+    config = small_config(layers=[{**att, "mlp": {"kind": "dense", "ff": 12416}}, {**att, "mlp": None}], loop=None, width=1024)
+    m, _ = build(config, torch.bfloat16, dev)
+    eng = m.engine()
+    eng.ensure(batch + 1, 64)
+    seqs = [tokens_of(3, seed=i) for i in range(batch)]
+    normed = next(t for t in eng._keep if t.data_ptr() == eng.m.xb)
+
+    def steps(group):
+        slots = [eng.acquire() for _ in group]
+        out = [eng.step([Entry(s, j, t[j:j + 1], [0]) for s, t in zip(slots, group)]).clone() for j in range(3)]
+        for s in slots:
+            eng.release(s)
+        return torch.stack(out)
+
+    normed.fill_(7.0)
+    got = steps(seqs)
+    assert bool((normed != 7.0).any()) == taken
+    for i, t in enumerate(seqs):
+        # (the same values rounded to bf16 on both sides, a value at the edge of a rounding either way: a few 2^-9 of the terms over four products)
+        assert rel(got[:, i].float(), steps([t])[:, 0].float()) < 4e-2, i
