@@ -298,6 +298,15 @@ def group_table(scales: torch.Tensor, zeros: torch.Tensor) -> torch.Tensor:
     return word.view(N // 16, 16, G).permute(0, 2, 1).contiguous().reshape(-1)
 
 
+def prompt_workspace_bytes(kinds, rows: int, K: int) -> int:
+    """Scratch of the products of `rows` rows of up to K columns over streams of these kinds ("q4", "bf16", "i8"): of 2048 x 11008 87 MB for int4 and bf16, 190 for
+    LLM.int8, whose outlier columns have regions of their own."""
+    need = [lib().mi355_linear_int8_gemm_workspace_bytes] if "i8" in kinds else []
+    if kinds - {"i8"}:
+        need.append(lib().mi355_linear_gemm_workspace_bytes)
+    return max(int(f(rows, K)) for f in need)
+
+
 class DecodeEngine:
     """Owns everything `mi355_forward` / `mi355_fused_step` need for one `LLaMA` instance."""
 
@@ -410,16 +419,14 @@ class DecodeEngine:
                 max_T = 0
             if max_T < 1:
                 raise EngineUnavailable("hidden size does not fit LDS")
-            # int4 and bf16 models: prompt chunks of >= 32 tokens go through the wide MFMA GEMM + flash attention (csrc/gemm.hip,
-            # flash_prefill.hip), so the chunk is bounded by scratch memory only (0.5 GB at 2048 tokens of a 7B model,
-            # most of it the f32 logits rows).  Large chunks matter: the [n_embd]-wide outputs (c_proj, mlp.c_proj) are
+            # prompt chunks of >= 32 tokens go through the wide MFMA GEMM (csrc/gemm.hip, int8_gemm.hip; int4 and bf16 products from 8 to 32 rows on:
+            # engine.hip wide_rows) and flash attention (flash_prefill.hip), so the chunk is bounded by scratch memory only (0.5 GB at 2048 tokens
+            # of a 7B model, most of it the f32 logits rows).  Large chunks matter: the [n_embd]-wide outputs (c_proj, mlp.c_proj) are
             # 16 row blocks, so 512 tokens fill only a quarter of the chip (9 % vs 27-36 % of the MFMA peak at 2048)
             self.gemm_ws = None
             if kinds <= {"q4", "bf16", "i8"} and _env_int("MI355_PREFILL_GEMM", 1):
                 max_T = max(max_T, min(_env_int("MI355_PREFILL_T", 2048), cfg.block_size))
-                need = max(int(lib().mi355_linear_gemm_workspace_bytes(max_T, max(C_, self.n_hidden))),
-                           int(lib().mi355_linear_int8_gemm_workspace_bytes(max_T, max(C_, self.n_hidden))))
-                self.gemm_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+                self.gemm_ws = torch.empty(prompt_workspace_bytes(kinds, max_T, max(C_, self.n_hidden)), dtype=torch.uint8, device=self.device)
             self.max_T = max_T
 
             local_heads = first.attn.c_attn.out_features // (3 * hs)

@@ -148,3 +148,12 @@ def test_runs_of_shares_in_the_fused_prompt_chain(dev, monkeypatch, T):
             out.append(model(idx.view(1, -1), 128, torch.arange(T, device=dev))[0].float())
     assert not torch.equal(*out)  # (the chain was on)
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
+
+
+def test_an_int4_engine_holds_no_scratch_of_int8_products(dev):
+    cfg = LLaMAConfig(block_size=128, n_layer=1, n_head=2, n_embd=256, vocab_size=512)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode="gptq.int4"):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode="gptq.int4", device="cuda", dtype=torch.bfloat16))
+    eng = model.eval().engine()
+    assert eng.gemm_ws.numel() == nat.lib().mi355_linear_gemm_workspace_bytes(eng.max_T, eng.n_hidden)

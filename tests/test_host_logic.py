@@ -678,3 +678,14 @@ def test_a_forced_cut_without_a_kernel_changes_nothing():
     for force in ("2:128:0", "1:0:0", "16:64:0", "8:32:0", "4:128:0", "8:16:0", "8:96:0", "0:7:0", "4:64:0:2"):
         assert _forced_plans(force) == rule, force
     assert _forced_plans("8:128:0") != rule
+
+
+def test_prompt_scratch_holds_what_the_formats_need():
+    from lit_llama_amd.engine import prompt_workspace_bytes
+
+    gemm, i8 = nat.lib().mi355_linear_gemm_workspace_bytes(2048, 11008), nat.lib().mi355_linear_int8_gemm_workspace_bytes(2048, 11008)
+    assert gemm < 90 << 20 < i8
+    for kinds in ({"q4"}, {"bf16"}, {"q4", "bf16"}):
+        assert prompt_workspace_bytes(kinds, 2048, 11008) == gemm
+    assert prompt_workspace_bytes({"i8"}, 2048, 11008) == i8
+    assert prompt_workspace_bytes({"i8", "bf16"}, 2048, 11008) == max(gemm, i8)
