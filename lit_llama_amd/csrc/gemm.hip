@@ -1896,6 +1896,17 @@ extern "C" size_t mi355_linear_gemm_workspace_bytes(int M, int K) {
     return (size_t)M * kp * 2 + unit_sums_at(M) * 4 + (size_t)M * (kp / 128) * 4 + 256 + kSplitBudget + kFuseScratch;
 }
 
+namespace {
+struct TableBytes {
+    size_t tables, sums;  // [n_groups + 1][R][tab_ld] dwords; operand sums per group
+};
+TableBytes table_bytes(int M, int N, int R, int n_groups) { return {((size_t)(n_groups + 1) * R * ((N + 15) / 16 * 16) * 4 + 15) & ~(size_t)15, (size_t)n_groups * M * 4}; }
+}  // namespace
+bool mi355_linear_gemm_tables_fit(int M, int N, int K, int R, int group_cols) {
+    const TableBytes t = table_bytes(M, N, R, (K + group_cols - 1) / group_cols);
+    return t.tables + t.sums <= kSplitBudget;
+}
+
 size_t mi355_linear_gemm_fuse_scratch_bytes() { return kFuseScratch; }
 
 extern "C" int mi355_linear_gemm(const mi355_linear_args* a, void* workspace, size_t workspace_bytes,
@@ -1937,7 +1948,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     // those over a whole K-slice in one accumulator loses what the row kernel, whose eight waves sum a part each, keeps (logits of a full-depth model with a
     // trained model's statistics, 14 tokens: off by 0.05 of their spread there, 0.08 here, unit by unit 0.03).
     const bool unit_sums = q4 && !scale_groups && f == nullptr && a->M < 32 && a->K % 128 == 0 && a->sz_dtype == MI355_BF16 && (a->alpha == 0.f || a->alpha == 1.f) &&
-                           !(a->flags & MI355_LF_NORM_ONE);
+                           !(a->flags & MI355_LF_NORM_ONE) && mi355_linear_gemm_tables_fit(a->M, a->N, a->K, a->R, a->K);
     const bool grouped = scale_groups || unit_sums;
     int gq_shift = 0;
     if (scale_groups) {
@@ -1977,8 +1988,9 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     if (grouped) {
         n_groups = unit_sums ? 1 : (a->K + a->group_cols - 1) / a->group_cols;
         tab_ld = (a->N + 15) / 16 * 16;
-        tab_bytes = ((size_t)(n_groups + 1) * a->R * tab_ld * 4 + 15) & ~(size_t)15;
-        sxt_bytes = (size_t)n_groups * a->M * 4;  // (of groups of whole units: in a place of their own)
+        const TableBytes t = table_bytes(a->M, a->N, a->R, n_groups);
+        tab_bytes = t.tables;
+        sxt_bytes = t.sums;  // (of groups of whole units: in a place of their own)
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
         // blocks of 8 row tiles x 64 tokens; slices of whole groups (>= 4 per slice), partials in the first half of the

@@ -49,6 +49,8 @@ struct mi355_gemm_fuse {
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
 // bytes mi355_linear_gemm_workspace_bytes reserves at the END of a workspace for the chain's partial sums
 size_t mi355_linear_gemm_fuse_scratch_bytes();
+// whether the tables of a product's (scale, zero) pairs per row and group of `group_cols` columns fit their region of a workspace (a launch refuses those that do not)
+bool mi355_linear_gemm_tables_fit(int M, int N, int K, int R, int group_cols);
 // The RMSNorm of the rows that a residual product (MI355_EPI_ACCUM, f32 y without gaps up to N) leaves: xb[m] = bf16(norm(y[m]) (scale + add)), rows of N.
 // Taken up by the sum of its K-slices, if there is one (`done`): the caller's own norm is a launch of its own, 4.6 us and a gap for 16 rows.
 struct mi355_reduce_norm {

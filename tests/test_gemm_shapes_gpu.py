@@ -157,3 +157,17 @@ def test_an_int4_engine_holds_no_scratch_of_int8_products(dev):
     model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode="gptq.int4", device="cuda", dtype=torch.bfloat16))
     eng = model.eval().engine()
     assert eng.gemm_ws.numel() == nat.lib().mi355_linear_gemm_workspace_bytes(eng.max_T, eng.n_hidden)
+
+
+def test_few_rows_of_more_outputs_than_a_table_holds(dev):
+    """Few int4 rows of one scale per row are summed as one group, whose table has a region of 32 MB: beyond 4.19 million rows of the matrix without it."""
+    M, N, K = 8, (1 << 22) + 16, 128
+    g = torch.Generator(device=dev).manual_seed(5)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    q = torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand((N,), generator=g, device=dev) * 0.02 + 0.005).to(torch.bfloat16)
+    z = torch.randint(5, 11, (N,), generator=g, device=dev).to(torch.bfloat16)
+    got = ops.linear_gemm(x, ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1), 1, N, K, scales=s, zeros=z, out_dtype=torch.float32)
+    for rows in (slice(0, 4096), slice(N - 4096, N)):
+        ref = x.double() @ ((q[rows].double() - z[rows].double()[:, None]) * s[rows].double()[:, None]).T
+        assert (got[:, rows].double() - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
