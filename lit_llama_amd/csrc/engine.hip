@@ -148,6 +148,12 @@ int wide_rows(const mi355_weight& w) {
     const int from = w.fmt == MI355_W_Q4 && (w.group_cols == 0 || w.group_cols >= w.K) ? 11 : 8;
     return cap < from ? from : cap < 31 ? cap + 1 : 32;
 }
+// Chunks of fewer than 32 rows were the row kernel's before they could be tiled: what the tiled kernel does not take stays there
+bool short_chunk_fits(const mi355_model* m, const mi355_weight& w, int M, int epi) {
+    const bool scale_groups = w.fmt == MI355_W_Q4 && w.group_cols > 0 && w.group_cols < w.K;
+    return w.R == (epi == MI355_EPI_SWIGLU ? 2 : 1) && (uintptr_t)m->gemm_ws % 16 == 0 && (size_t)m->gemm_ws_bytes >= mi355_linear_gemm_workspace_bytes(M, w.K) &&
+           (!scale_groups || mi355_linear_gemm_tables_fit(M, w.N, w.K, w.R, w.group_cols));
+}
 bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: int4 / bf16 stream, one scale per row
     return (w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && (w.group_cols == 0 || w.group_cols >= w.K) && w.N % 4 == 0 &&
            w.K % 128 == 0;
@@ -214,7 +220,7 @@ int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x
                const float* attn_partials = nullptr) {
     // wide inputs of an int4 or bf16 model: the LDS-tiled MFMA GEMM over the same stream (per-row or grouped scales)
     if ((w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && M >= wide_rows(w) && m->gemm_ws != nullptr &&
-        attn_partials == nullptr && w.N % 4 == 0 && ldy % 4 == 0 && (w.group_cols == 0 || w.K % 128 == 0)) {
+        attn_partials == nullptr && w.N % 4 == 0 && ldy % 4 == 0 && (w.group_cols == 0 || w.K % 128 == 0) && (M >= 32 || short_chunk_fits(m, w, M, epi))) {
         mi355_linear_args a;
         fill_linear_args(a, m, w, x, x_dtype, M, ldx, norm_scale, epi, y, y_dtype, ldy);
         return mi355_linear_gemm(&a, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);

@@ -171,3 +171,35 @@ def test_few_rows_of_more_outputs_than_a_table_holds(dev):
     for rows in (slice(0, 4096), slice(N - 4096, N)):
         ref = x.double() @ ((q[rows].double() - z[rows].double()[:, None]) * s[rows].double()[:, None]).T
         assert (got[:, rows].double() - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
+@pytest.mark.parametrize("case", ["tables", "workspace", "stream"])
+def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev, case):
+    """24 tokens at a width where the row kernel reads the weights twice: with group tables of a vocabulary that exceeds their region, a workspace sized for less,
+    a head in tiles of 32 rows: as the tokens one by one."""
+    cfg = LLaMAConfig(block_size=32, n_layer=1, n_head=32, n_embd=4096, vocab_size=260_000 if case == "tables" else 512)
+    cols = 128 if case == "tables" else 0
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=None if case == "stream" else "gptq.int4"):
+        model = LLaMA(cfg)
+    if cols:
+        from lit_llama_amd.quantization import ColBlockQuantizedLinear
+
+        for mod in model.modules():
+            if isinstance(mod, ColBlockQuantizedLinear):
+                mod.tile_cols = cols
+                mod.scales, mod.zeros = (torch.empty((mod.out_features, mod.in_features // cols), device=dev, dtype=torch.bfloat16) for _ in range(2))
+    model.load_state_dict(synth.make_state_dict(cfg, seed=2, mode=None if case == "stream" else "gptq.int4", device="cuda", dtype=torch.bfloat16, group_cols=cols))
+    model.eval()
+    eng = model.engine()
+    assert eng is not None, model._engine_failed
+    if case == "workspace":
+        eng.m.gemm_ws_bytes = 4096
+    if case == "stream":
+        head = ops.repack_bf16(model.lm_head.weight, None, 2)
+        eng.m.lm_head.w, eng.m.lm_head.R = head.data_ptr(), 2
+    idx = synth.make_prompt(24, vocab=512).to(dev)
+    with torch.no_grad():
+        one = model(idx.view(1, -1), 32, torch.arange(24, device=dev))[0].float()
+        model.reset_cache()
+        rows = torch.cat([model(idx[t:t + 1].view(1, 1), 32, torch.tensor([t], device=dev))[0].float() for t in range(24)])
+    assert (one - rows).abs().max() <= 0.05 * rows.std()
