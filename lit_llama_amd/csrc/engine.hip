@@ -85,7 +85,11 @@ int run_linear_rows(const mi355_model* m, const mi355_weight& w, const void* x, 
 struct FuseEdge {      // partial sums ("shares") a producer leaves per row, [share][T] f32
     float* ss;         // sums of squares of the f32 residual row (residual epilogues only)
     float* sx;         // operand sums
-    int n, ppu;        // shares, shares per 128-column unit (mi355_linear_gemm_plan of the producer's launch)
+    struct Cut {
+        int n, ppu;    // shares, shares per 128-column unit (mi355_linear_gemm_plan of the producer's launch)
+    } of[2];           // by the producer's stream: int4, bf16
+    int n, ppu;        // what the last producer has left
+    void left_by(const mi355_weight& w) { n = of[w.fmt == MI355_W_BF16].n, ppu = of[w.fmt == MI355_W_BF16].ppu; }
 };
 struct FuseCtx {
     bool on;
@@ -177,11 +181,8 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
         if (L.attn.N != 3 * C || L.attn.K != C || L.proj.N != C || L.proj.K != C || L.fc.N != H || L.fc.K != C || L.fc.R != 2 ||
             L.mproj.N != C || L.mproj.K != H || L.kcache == nullptr || L.vcache == nullptr)
             return z;
-        // (one plan for all layers: it depends on the format)
-        if (L.proj.fmt != m->layers[0].proj.fmt || L.fc.fmt != m->layers[0].fc.fmt || L.mproj.fmt != m->layers[0].mproj.fmt) return z;
     }
     if (C % 128 != 0 || H % 128 != 0) return z;
-    int ks, n, ppu;
     const size_t Ts = (size_t)T;
     // scratch: the tail of the workspace (mi355_linear_gemm_workspace_bytes reserves it behind the split-K partials)
     const int kmax = H > C ? H : C;
@@ -189,10 +190,10 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
     if ((size_t)m->gemm_ws_bytes < mi355_linear_gemm_workspace_bytes(T, kmax)) return z;
     float* cur = (float*)((char*)m->gemm_ws + (((size_t)m->gemm_ws_bytes - tail) & ~(size_t)15));
     float* const end = (float*)((char*)m->gemm_ws + (size_t)m->gemm_ws_bytes);
-    auto edge = [&](FuseEdge& e, const mi355_weight& w, bool with_ss) {
-        mi355_linear_gemm_plan(T, w.N, w.K, w.R, w.fmt == MI355_W_BF16, &ks, &n, &ppu);
-        e.n = n;
-        e.ppu = ppu;
+    auto edge = [&](FuseEdge& e, const mi355_weight& w, bool with_ss) {  // (the layers may differ in their formats)
+        int ks;
+        for (int b = 0; b < 2; ++b) mi355_linear_gemm_plan(T, w.N, w.K, w.R, b == 1, &ks, &e.of[b].n, &e.of[b].ppu);
+        const int n = e.of[0].n > e.of[1].n ? e.of[0].n : e.of[1].n;
         e.sx = cur;
         cur += (size_t)n * Ts;
         e.ss = with_ss ? cur : nullptr;
@@ -409,6 +410,7 @@ static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStr
             f.next_norm_dtype = m->param_dtype;
             f.out_ss = fz->proj.ss;
             f.out_sx = fz->proj.sx;
+            fz->proj.left_by(L.proj);
             fz->have_x = true;
             return mi355_linear_gemm_fused(&a, &f, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
         case 2:  // c_fc1 / c_fc2 + SwiGLU over the emitted operand; partial operand sums of the hidden vector
@@ -420,6 +422,7 @@ static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStr
             f.in_sx_n = f.in_ss_n = fz->proj.n;
             f.in_ppu = fz->proj.ppu;
             f.out_sx = fz->fc.sx;
+            fz->fc.left_by(L.fc);
             fz->have_x = false;
             return mi355_linear_gemm_fused(&a, &f, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
         default:  // mlp.c_proj; the residual epilogue emits the next layer's c_attn operand
@@ -435,6 +438,7 @@ static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStr
                 f.next_norm_dtype = m->param_dtype;
                 f.out_ss = fz->mproj.ss;
                 f.out_sx = fz->mproj.sx;
+                fz->mproj.left_by(L.mproj);
                 fz->have_x = true;
             }
             return mi355_linear_gemm_fused(&a, &f, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);

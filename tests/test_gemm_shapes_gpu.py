@@ -203,3 +203,33 @@ def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev,
         model.reset_cache()
         rows = torch.cat([model(idx[t:t + 1].view(1, 1), 32, torch.tensor([t], device=dev))[0].float() for t in range(24)])
     assert (one - rows).abs().max() <= 0.05 * rows.std()
+
+
+@pytest.mark.parametrize("T", [40, 150, 700])
+def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T):
+    """Int4 and bf16 layers in turn: what a producer leaves is cut by its own format, and the chain holds over both.  0.02 of the logits' spread as for one format
+    (other orders of f32 sums in front of bf16 roundings)."""
+    cfg = LLaMAConfig(block_size=704, n_layer=3, n_head=15, n_embd=1920, vocab_size=512)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode="gptq.int4"):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode="gptq.int4", device="cuda", dtype=torch.bfloat16))
+    g = torch.Generator(device=dev).manual_seed(4)
+    for layer, names in ((0, ["attn.c_proj"]), (1, ["attn.c_attn", "attn.c_proj", "mlp.c_fc1", "mlp.c_fc2", "mlp.c_proj"]), (2, ["mlp.c_proj"])):
+        for name in names:
+            part, attr = name.split(".")
+            owner = getattr(model.transformer.h[layer], part)
+            q = getattr(owner, attr)
+            dense = torch.nn.Linear(q.in_features, q.out_features, bias=False, device=dev, dtype=torch.bfloat16)
+            dense.weight.data = (torch.randn(dense.weight.shape, generator=g, device=dev) * q.in_features ** -0.5).to(torch.bfloat16)
+            setattr(owner, attr, dense)
+    model.eval()
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
+        model.reset_cache()
+        with torch.no_grad():
+            out.append(model(idx.view(1, -1), 704, torch.arange(T, device=dev))[0].float())
+    assert model.engine() is not None, model._engine_failed
+    assert not torch.equal(*out)  # (the chain was on)
+    assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
