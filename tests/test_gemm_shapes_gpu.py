@@ -173,13 +173,8 @@ def test_few_rows_of_more_outputs_than_a_table_holds(dev):
         assert (got[:, rows].double() - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
-@pytest.mark.parametrize("case", ["tables", "workspace", "stream"])
-def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev, case):
-    """24 tokens at a width where the row kernel reads the weights twice: with group tables of a vocabulary that exceeds their region, a workspace sized for less,
-    a head in tiles of 32 rows: as the tokens one by one."""
-    cfg = LLaMAConfig(block_size=32, n_layer=1, n_head=32, n_embd=4096, vocab_size=260_000 if case == "tables" else 512)
-    cols = 128 if case == "tables" else 0
-    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=None if case == "stream" else "gptq.int4"):
+def _wide_model(dev, cfg, mode, cols):
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=mode):
         model = LLaMA(cfg)
     if cols:
         from lit_llama_amd.quantization import ColBlockQuantizedLinear
@@ -188,8 +183,39 @@ def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev,
             if isinstance(mod, ColBlockQuantizedLinear):
                 mod.tile_cols = cols
                 mod.scales, mod.zeros = (torch.empty((mod.out_features, mod.in_features // cols), device=dev, dtype=torch.bfloat16) for _ in range(2))
-    model.load_state_dict(synth.make_state_dict(cfg, seed=2, mode=None if case == "stream" else "gptq.int4", device="cuda", dtype=torch.bfloat16, group_cols=cols))
-    model.eval()
+    model.load_state_dict(synth.make_state_dict(cfg, seed=2, mode=mode, device="cuda", dtype=torch.bfloat16, group_cols=cols))
+    return model.eval()
+
+
+def _chunk_and_rows(dev, model, T):
+    """Logits of T tokens in one pass and one by one (the row kernels)."""
+    S = model.config.block_size
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    with torch.no_grad():
+        one = model(idx.view(1, -1), S, torch.arange(T, device=dev))[0].float()
+        model.reset_cache()
+        rows = torch.cat([model(idx[t:t + 1].view(1, 1), S, torch.tensor([t], device=dev))[0].float() for t in range(T)])
+    model.reset_cache()
+    return one, rows
+
+
+@pytest.mark.parametrize("mode,cols", [("gptq.int4", 0), ("gptq.int4", 128), ("gptq.int4", 256), (None, 0)])
+def test_chunks_of_8_to_31_rows_at_a_width_that_tiles_them(dev, mode, cols):
+    """7B width, where the row kernel would read the weights of 8 to 14 rows and more twice (mlp.c_proj's: of 8): on both sides of each product's change of kernel,
+    single scales, groups of 128 and 256 columns, bf16."""
+    model = _wide_model(dev, LLaMAConfig(block_size=32, n_layer=1, n_head=32, n_embd=4096, vocab_size=512), mode, cols)
+    assert model.engine() is not None, model._engine_failed
+    for T in (7, 8, 10, 11, 12, 13, 14, 16, 17, 31):
+        one, rows = _chunk_and_rows(dev, model, T)
+        assert (one - rows).abs().max() <= 0.05 * rows.std(), T
+
+
+@pytest.mark.parametrize("case", ["tables", "workspace", "stream"])
+def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev, case):
+    """24 tokens at a width where the row kernel reads the weights twice: with group tables of a vocabulary that exceeds their region, a workspace sized for less,
+    a head in tiles of 32 rows: as the tokens one by one."""
+    cfg = LLaMAConfig(block_size=32, n_layer=1, n_head=32, n_embd=4096, vocab_size=260_000 if case == "tables" else 512)
+    model = _wide_model(dev, cfg, None if case == "stream" else "gptq.int4", 128 if case == "tables" else 0)
     eng = model.engine()
     assert eng is not None, model._engine_failed
     if case == "workspace":
@@ -197,11 +223,7 @@ def test_short_chunks_that_the_tiled_product_refuses_stay_in_the_row_kernel(dev,
     if case == "stream":
         head = ops.repack_bf16(model.lm_head.weight, None, 2)
         eng.m.lm_head.w, eng.m.lm_head.R = head.data_ptr(), 2
-    idx = synth.make_prompt(24, vocab=512).to(dev)
-    with torch.no_grad():
-        one = model(idx.view(1, -1), 32, torch.arange(24, device=dev))[0].float()
-        model.reset_cache()
-        rows = torch.cat([model(idx[t:t + 1].view(1, 1), 32, torch.tensor([t], device=dev))[0].float() for t in range(24)])
+    one, rows = _chunk_and_rows(dev, model, 24)
     assert (one - rows).abs().max() <= 0.05 * rows.std()
 
 
@@ -233,3 +255,35 @@ def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T
     assert model.engine() is not None, model._engine_failed
     assert not torch.equal(*out)  # (the chain was on)
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
+
+
+@pytest.mark.parametrize("M", [9, 40, 100, 300, 600])
+@pytest.mark.parametrize("fmt", ["q4", "g128", "g32", "bf16", "i8"])
+def test_rows_that_are_not_finite_stay_by_themselves(dev, fmt, M):
+    """NaN and infinities in two rows (LLM.int8: NaN alone, an infinity makes its columns everyone's outliers): the other rows keep their bits, in blocks with and
+    without empty rows, slices, runs and groups."""
+    N, K = 4096, 4096
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    bad = x.clone()
+    bad[2], bad[M - 1, 100:300] = float("nan"), float("nan") if fmt == "i8" else float("inf")
+    if fmt == "i8":
+        cb, scb = ops.int8_quant_rows(torch.randn((N, K), generator=g, device=dev) * K ** -0.5)
+        stream = ops.repack_i8(cb, None, 1)
+        run = lambda v: ops.linear_int8_gemm(v, stream, scb, 1, N, K, out_dtype=torch.float32)  # noqa: E731
+    elif fmt == "bf16":
+        stream = ops.repack_bf16((torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16), None, 1)
+        run = lambda v: ops.linear_gemm(v, stream, 1, N, K, fmt=nat.W_BF16, out_dtype=torch.float32)  # noqa: E731
+    else:
+        cols = int(fmt[1:]) if fmt != "q4" else 0
+        ng = K // cols if cols else 1
+        stream = ops.repack_q4(synth.pack_colblock(torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8), 4), None, N, K, 1)
+        s = (torch.rand((N * ng,), generator=g, device=dev) * 0.02 + 0.005).to(torch.bfloat16)
+        z = torch.randint(5, 11, (N * ng,), generator=g, device=dev).to(torch.bfloat16)
+        run = lambda v: ops.linear_gemm(v, stream, 1, N, K, scales=s, zeros=z, group_cols=cols, out_dtype=torch.float32)  # noqa: E731
+    clean, got = run(x).clone(), run(bad)
+    others = torch.ones(M, dtype=torch.bool, device=dev)
+    others[2] = others[M - 1] = False
+    assert torch.equal(got[others], clean[others]) and bool(clean.isfinite().all())
+    if fmt != "i8":
+        assert not bool(got[2].isfinite().any()) and not bool(got[M - 1].isfinite().any())

@@ -508,3 +508,22 @@ def test_norm_of_rows_only_in_front_of_a_product_that_takes_it(dev, batch, taken
     for i, t in enumerate(seqs):
         # (the same values rounded to bf16 on both sides, a value at the edge of a rounding either way: a few 2^-9 of the terms over four products)
         assert rel(got[:, i].float(), steps([t])[:, 0].float()) < 4e-2, i
+
+
+@pytest.mark.parametrize("width,batch", [(128, 9), (1024, 16), (1152, 33), (4096, 20), (8192, 12)])
+def test_norm_taken_with_a_sum_of_slices(dev, width, batch):
+    """What the sum of the last residual product's slices leaves for the head: bf16(x rinv scale) of the rows that it writes, to one step of bf16 (its own rounding;
+    the factors in front of it are f32)."""
+    from lit_llama_amd.hybrid_engine import Entry
+
+    att = {"type": "attention", "mixer": {"heads": 9, "kv_heads": 3, "dim": 128, "vdim": 128, "scale": 0.09, "mask": {"size": 19}}}
+    m, sd = build(small_config(layers=[{**att, "mlp": None}, {**att, "mlp": {"kind": "dense", "ff": 1280}}], loop=None, width=width), torch.bfloat16, dev)
+    eng = m.engine()
+    eng.ensure(batch, 64)
+    normed = next(t for t in eng._keep if t.data_ptr() == eng.m.xb)
+    normed.fill_(7.0)
+    eng.step([Entry(eng.acquire(), 0, tokens_of(1, seed=i), [0]) for i in range(batch)])
+    got = normed[:batch * width].view(batch, width).double()
+    x = eng.x.view(-1, eng.m.ldx)[:batch, :width].double()
+    ref = x * (x.square().mean(1, keepdim=True) + 3e-5).rsqrt() * sd["final.norm"].to(torch.bfloat16).to(dev).double()
+    assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-6).all()
