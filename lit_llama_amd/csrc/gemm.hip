@@ -66,9 +66,6 @@ constexpr int kTPW = MI355_GEMM_TPW;
 #ifndef MI355_GEMM_AND_OR
 #define MI355_GEMM_AND_OR 1
 #endif
-#ifndef MI355_GEMM_PIN_W
-#define MI355_GEMM_PIN_W 0
-#endif
 #ifndef MI355_GEMM_BF16_ROWMAJOR
 // workgroup order of the BF16 streams: row block major (an XCD runs every token block of a few row blocks side by side).  Token block major
 // (the int4 order) carried every weight piece across the fabric once per token block: 16 x 13.5 GB = 216 GB per 2048-token pass of the 7B
@@ -214,7 +211,8 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(const void* x, int x_dt
 // multiplication and a store at a time, and a sum of the block per K-slice).  Grouped scales: sxt[i][m] = sum of xb over columns [i * cols, (i + 1) * cols),
 // cols = 32, 64 or 128, in place of the sums per slice; the workgroups behind the M rows then lay out the tables, [N][n_groups] bf16 scales / zeros ->
 // gtab[grp][r][n] dwords (n fastest: the four rows a lane holds are one 16-B load; row n_groups and the rows past N are zero), a 64 x 64 piece each through
-// LDS: 1000 x 4096 f32 and the tables of 12288 rows 17 us and 5 in a launch of their own -> 9 together.
+// LDS: 1000 x 4096 f32 rows 17 us, and the tables of 12288 rows 5 in a launch of their own -> 9 together by themselves, 14.7 within a prompt, whose rows the product
+// before has just written (profiles/prompt_and_batch_kernels.txt).
 constexpr int kStageLds = 64 * 65;  // dwords: a piece of the tables, or a sum per unit
 struct GroupTables {
     const bf16_t *s0, *z0, *s1, *z1;
@@ -931,17 +929,6 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     // i.e. wait for these very loads before the first MFMA): past the last unit the offsets fall into the next row /
     // tile or out of the descriptors (zeros) and the values are never used
     auto prefetch = [&](int u) {
-#if MI355_GEMM_PIN_W
-        // (A / B knob, off: 128-token blocks with only the WEIGHT requests — HBM latency — pinned at the unit's start, the
-        // activation requests, L2 hits, free to sink: 116-124 VGPRs, measured neutral — profiles/r04_prefill_fused_chain_ab.txt)
-        if constexpr (BM > 64 && GRP == 0 && FMT == MI355_W_Q4) {
-#pragma unroll
-            for (int t = 0; t < kTPW; ++t) wload(t, u + 1, wnext[t]);
-            __builtin_amdgcn_sched_barrier(0);
-            xload(u + 1);
-            return;
-        }
-#endif
         if constexpr (kXDma) {
             // (weights first: HBM latency; both pinned at the unit's start — they cost 8 registers now, not 40)
             if constexpr (!kRefill) {
@@ -1141,7 +1128,7 @@ __device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, un
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, scalar_off, 0, 0);
 }
 
-// The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of any prompt):
+// The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of longer ones):
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
@@ -1715,11 +1702,13 @@ int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
 }
 // bytes of the K-slices' partial sums
 size_t gemm_part_bytes(int M, int N, bool pair, int ksplit) { return (size_t)ksplit * M * N * (pair ? 2 : 1) * 4; }
-// (blocks of 48 tokens, int4: N = 12288 / 11008 pair, K = 4096, 37 tokens 22.9 / 25.1 us with blocks of 64, 21.7 / 23.3 with 48, groups of 128 columns 29.5 / 36.0 and
-// 27.4 / 33.6; BF16, bound by the weights, the same either way)
+// (blocks of 48 tokens, int4: of eight products of 2048 to 13824 rows at 33 / 40 / 48 tokens 2-10 / 2-9 / 2-7 % less than blocks of 64, groups of 128 columns 3-9 / 3-8 /
+// 3-7 % (N = 12288, K = 4096: 22.2 -> 20.9, 22.1 -> 21.0, 22.4 -> 21.3 us).  BF16, bound by the weights, the same either way)
 int short_block(int M, bool bf16) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 48 && !bf16 ? 48 : 64; }
 
-// Int4.  Waves of a block: up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them, which 4-5 K-slices bring to a workgroup for two CUs of three;
+// Int4.  (Of 18 products of 2048 to 32000 rows at 72 to 700 tokens, weights not in any cache, this choice is within 5 % of the fastest instantiated one for two in three
+// and 4 % behind on average; at most 1.4 times as long, for narrow SwiGLU pairs: 5632 rows, K = 2048, 128 tokens 24.5 us against 17.4 in blocks of 4 waves.)
+// Waves of a block: up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them, which 4-5 K-slices bring to a workgroup for two CUs of three;
 // 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, with staging: 20.5 us against 22.7).  Longer prompts likewise while the 256-row
 // blocks leave half of the CUs idle, except where the 128-row blocks of a launch without slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096,
 // 128 tokens 29.3 / 24.5 us, 512 38.9 / 32.0; N = 12288, 128 tokens 34.6 / 29.6; K = 11008, 300 tokens 57.5 / 64.0, 512 71.2 / 66.7).  The SwiGLU pair does
@@ -1980,9 +1969,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     bf16_t* xb = (bf16_t*)workspace;
     float* rinv = (float*)((char*)workspace + (size_t)a->M * kp * 2);
     float* sx = rinv + a->M;
-    // split-K: launches of fewer than 96 blocks (a 128-token prompt against N = 4096 is 16) cut K into up to 8
-    // slices, as many as bring the launch to ~128 workgroups and fit the partial buffer
-    int ksplit = 1;
+    int ksplit = 1;  // K-slices: gemm_cut(); grouped scales: here
     size_t tab_bytes = 0, sxt_bytes = 0;
     int n_groups = 0, tab_ld = 0;
     if (grouped) {
@@ -1993,8 +1980,8 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         sxt_bytes = t.sums;  // (of groups of whole units: in a place of their own)
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
-        // blocks of 8 row tiles x 64 tokens; slices of whole groups (>= 4 per slice), partials in the first half of the
-        // region, the tables in the second
+        // grouped scales: blocks of 8 row tiles x 64 tokens, doubled to 256 by slices of at least 4 cuts (groups; units where a group holds several: a slice may end within
+        // a group, whose products are scaled unit by unit).  Partial sums in the first half of the region, the tables in the second
         const int rows_per_block = swiglu ? 16 * 4 * kTPW / 2 : 16 * 4 * kTPW;
         const int blocks = ((a->N + rows_per_block - 1) / rows_per_block) * ((a->M + 63) / 64);
         const size_t row_floats = (size_t)a->N * (swiglu ? 2 : 1);
@@ -2012,8 +1999,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
     }
-    // producer / consumer fusion (gemm_fuse.h): whole-K launches over per-row scales only — the caller plans with
-    // mi355_linear_gemm_plan
+    // producer / consumer fusion (gemm_fuse.h): launches over per-row scales only — the caller plans with mi355_linear_gemm_plan
     const bool fused = f != nullptr;
     const bool f_in = fused && f->prestaged;
     if (fused) {
