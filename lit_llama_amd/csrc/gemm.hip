@@ -297,11 +297,14 @@ __global__ __launch_bounds__(256) void stage_units_kernel(const void* x, int x_d
     const float tss = block_sum(ss, (float*)lds);
     if (threadIdx.x == 0) rinv[m] = norm_scale != nullptr ? rsqrtf(tss / (float)K + eps) * alpha : alpha;
     if (sxt == nullptr) {  // (every wave has passed the block sum's barriers: the units' sums stand in LDS)
-        for (int s = threadIdx.x; s < ksplit * runs; s += 256) {
-            const int u_lo = run_lo(s, K >> 7, ksplit, runs, run_units), u_hi = run_lo(s + 1, K >> 7, ksplit, runs, run_units);
-            double sum = 0.;  // (one rounding beside a large unit, not one per unit)
-            for (int u = u_lo; u < u_hi; ++u) sum += per_unit[u];
-            sx[(int64_t)m * (ksplit * runs) + s] = (float)sum;
+        // 16 lanes a sum: beside a large unit four roundings, not one per unit (and a thread's chain of 32 units took 1 us)
+        for (int s0 = 0; s0 < ksplit * runs; s0 += 16) {
+            const int s = s0 + (threadIdx.x >> 4), i = s < ksplit * runs ? s : 0;
+            const int u_lo = run_lo(i, K >> 7, ksplit, runs, run_units), u_hi = run_lo(i + 1, K >> 7, ksplit, runs, run_units);
+            float sum = 0.f;
+            for (int u = u_lo + (threadIdx.x & 15); u < u_hi; u += 16) sum += per_unit[u];
+            sum = group_sum(sum, 16);
+            if ((threadIdx.x & 15) == 0 && s < ksplit * runs) sx[(int64_t)m * (ksplit * runs) + s] = sum;
         }
     }
 }
@@ -1171,7 +1174,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] float* frp = fr + 2 * BM;
     [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM, DEPTH>);
     [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE, DEPTH>);
-    [[maybe_unused]] float* runtab = rowtab + 3 * kSlots * 16;  // [run][BM] operand sums
+    [[maybe_unused]] float* runtab = rowtab + 3 * kSlots * 16;  // [part of a run's sum][run][BM] operand sums
     int tile[kTPW];
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
@@ -1277,13 +1280,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     if constexpr (FUSE && EPI == MI355_EPI_STORE) {
         if (p.rope != nullptr) t_pos = p.pos[mt];
     }
-    // shares of the tokens' factors (gemm_fuse.h): every thread a token and every kP-th share (operand sums of several runs: every share of every kP-th run), in
-    // share order; the first kIn of them now
+    // shares of the tokens' factors (gemm_fuse.h): every thread a token and every kP-th share, in share order; the first kIn of them now.  Operand sums of several
+    // runs: kP / runs threads take a run's shares in turn, and end_run() adds their sums
     constexpr int kP = kThreads / BM < 8 ? kThreads / BM : 8, kIn = kSharesAhead;
     const int s_tok = threadIdx.x % BM, s_part = threadIdx.x / BM;
     [[maybe_unused]] const int64_t s_m = m0 + s_tok < p.M ? m0 + s_tok : p.M - 1;
     [[maybe_unused]] const int s_lo = FUSE && p.ksplit > 1 ? u_lo * p.in_ppu : 0, s_hi = FUSE && p.ksplit > 1 ? u_hi * p.in_ppu : p.in_sx_n;
-    [[maybe_unused]] const int s_first = s_lo + (RUNS ? s_part * p.run_units * p.in_ppu : s_part);
+    // (kP <= 8 and two runs at least: quotients of up to 4, without a division in front of the first request)
+    auto over_runs = [&](int v) { return (v >= p.runs) + (v >= 2 * p.runs) + (v >= 3 * p.runs) + (v >= 4 * p.runs); };
+    [[maybe_unused]] const int subs = RUNS && !own && kP >= 2 * p.runs ? over_runs(kP) : 1;
+    [[maybe_unused]] const int s_sub = subs > 1 ? over_runs(s_part) : 0, s_run = s_part - s_sub * p.runs;
+    [[maybe_unused]] const int s_first = s_lo + (RUNS ? s_run * p.run_units * p.in_ppu + s_sub : s_part);
     [[maybe_unused]] auto run_end = [&](int run) { return (u_lo + (run + 1) * p.run_units < u_hi ? u_lo + (run + 1) * p.run_units : u_hi) * p.in_ppu; };
     [[maybe_unused]] float vx[kIn], vs[kIn];
     auto shares = [&](const float* in, int j0, int step, int hi, float (&v)[kSharesAhead]) {
@@ -1297,7 +1304,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     };
     if constexpr (FUSE) {
         if (!own && s_part < kP) {
-            shares(p.in_sx, s_first, RUNS ? 1 : kP, RUNS ? run_end(s_part) : s_hi, vx);
+            shares(p.in_sx, s_first, RUNS ? subs : kP, RUNS ? run_end(s_run) : s_hi, vx);
             if (p.in_ss_n > 0) shares(p.in_ss, s_part, kP, p.in_ss_n, vs);
         }
     }
@@ -1312,13 +1319,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     if constexpr (FUSE) {
         if (!own && s_part < kP) {
             if constexpr (RUNS) {
-                for (int run = s_part; run < p.runs; run += kP) {
+                for (int run = s_run; run < p.runs && s_sub < subs; run += kP) {
                     float sum = 0.f;
-                    for (int j0 = s_lo + run * p.run_units * p.in_ppu, hi = run_end(run); j0 < hi; j0 += kIn) {
-                        if (run != s_part || j0 != s_first) shares(p.in_sx, j0, 1, hi, vx);
-                        sum = add_shares(j0, 1, hi, vx, sum);
+                    for (int j0 = s_lo + run * p.run_units * p.in_ppu + s_sub, hi = run_end(run); j0 < hi; j0 += kIn * subs) {
+                        if (run != s_run || j0 != s_first) shares(p.in_sx, j0, subs, hi, vx);
+                        sum = add_shares(j0, subs, hi, vx, sum);
                     }
-                    runtab[run * BM + s_tok] = sum;
+                    runtab[(run + s_sub * p.runs) * BM + s_tok] = sum;
                 }
             } else {
                 sxs = add_shares(s_first, kP, s_hi, vx, 0.f);
@@ -1523,15 +1530,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] f32x4 of_runs[RUNS ? kTPW : 1][RUNS ? kTT : 1];
     [[maybe_unused]] int run = 0, left = p.run_units;
     [[maybe_unused]] auto end_run = [&]() __attribute__((always_inline)) {
+        float x[kTT];
+#pragma unroll
+        for (int tt = 0; tt < kTT; ++tt) x[tt] = runtab[run * BM + tt * 16 + c];
+        for (int q = 1; q < subs; ++q)
+#pragma unroll
+            for (int tt = 0; tt < kTT; ++tt) x[tt] += runtab[(run + q * p.runs) * BM + tt * 16 + c];
 #pragma unroll
         for (int t = 0; t < kTPW; ++t) {
             const f32x4 zp = *(const f32x4*)(rowtab + (kSlots + kTPW * wave + t) * 16 + 4 * g);
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) {
-                const float x = runtab[run * BM + tt * 16 + c];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    of_runs[t][tt][r] += acc[t][tt][r] - zp[r] * x;
+                    of_runs[t][tt][r] += acc[t][tt][r] - zp[r] * x[tt];
                     acc[t][tt][r] = 0.f;
                 }
             }
@@ -1713,7 +1725,8 @@ int short_block(int M, bool bf16) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 48
 // blocks leave half of the CUs idle, except where the 128-row blocks of a launch without slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096,
 // 128 tokens 29.3 / 24.5 us, 512 38.9 / 32.0; N = 12288, 128 tokens 34.6 / 29.6; K = 11008, 300 tokens 57.5 / 64.0, 512 71.2 / 66.7).  The SwiGLU pair does
 // not gain (128 tokens 36.5 / 39.4).
-// Slices: as many as bring the launch to the workgroups wanted, none below 6 units.  Their sums, written and read again, take at most half the partial buffer,
+// Slices: as many as bring the launch to the workgroups wanted, none below 6 units, from the third on of blocks of 4 waves 4 (each is one run then, gemm_runs(): 40
+// tokens, N = K = 4096, 15.8 us with 8 slices, 16.4 with 5; 2048, 12.5 with 4, 14.3 with 2; but N = 2816 pair, K = 1024, 12.5 with 2, 10.6 with 1).  Their sums, written and read again, take at most half the partial buffer,
 // 16 MB: past that a slice costs more than the CUs that it fills (1 / 2 slices, 600 tokens, N = 4096: K = 4096 38.1 / 45.6 us, 11008 77 / 84; 120, N = 11008 pair 35.4 /
 // 42.1).  Blocks of 4 waves stop at one workgroup per CU: a few more than 256 leave the chip to those few (37 rows, K = 11008, N = 4096: 28.4 / 26.7 / 25.6 /
 // 24.7 with 4 / 5 / 6 / 8).
@@ -1724,7 +1737,7 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
     const int units = (K + 127) / 128, blocks8 = (N + 255) / 256 * ((M + 63) / 64);
     GemmCut cut = {M <= 64 || (!pair && (blocks8 <= 64 || (blocks8 >= 96 && blocks8 <= 128))) ? 4 : 8, short_block(M, false), true, 1};
     const int blocks = gemm_blocks(M, N, pair, cut.waves, 64), want = cut.waves == 8 ? 192 : 256, most = cut.waves == 8 ? 1 << 20 : 256;
-    while (cut.ksplit < 8 && blocks * cut.ksplit < want && blocks * (cut.ksplit + 1) <= most && units >= 6 * (cut.ksplit + 1) &&
+    while (cut.ksplit < 8 && blocks * cut.ksplit < want && blocks * (cut.ksplit + 1) <= most && units >= (cut.waves == 4 && cut.ksplit > 1 ? 4 : 6) * (cut.ksplit + 1) &&
            gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
         ++cut.ksplit;
     const int wide = gemm_blocks(M, N, pair, 8, kBM) * cut.ksplit;
@@ -1805,8 +1818,8 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
 // product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows
 // number less than 96 / cuts and a run keeps 4 units; a K-slice that is longer takes several runs, each with its own operand sum.  Error beside one activation of
 // 2^17 (rms, in units of its product's last bit), N = K = 4096 / N = 4096, K = 11008 / N = 12288, K = 4096, a run per slice -> runs: 40 tokens 3.0 / 3.9 / 4.8 -> 2.6 /
-// 3.9 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.5 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.6 / 6.8; it takes a layer's products from 84.7 to 86.0 us at 37 tokens,
-// from 114 to 117 at 100 and leaves 512 as they were.  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
+// 3.8 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.6 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.5 / 6.7.  A second run takes a launch 0.5-0.7 us (a prompt of 37
+// tokens, 7B: 2.48 -> 2.49 ms).  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
 void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, int* run_units) {
     const int units = (K + 127) / 128, longest = (units + cut.ksplit - 1) / cut.ksplit, blocks = gemm_blocks(M, N, pair, 8, kBM);
     int cuts = 1;
