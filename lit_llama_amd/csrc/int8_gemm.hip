@@ -94,7 +94,8 @@ __global__ void i8_clear_mask_kernel(unsigned* mask, int n) {
     if (i < n) mask[i] = 0u;
 }
 
-// (a thread's elements are 256 apart, 16 of them requested at a time: one at a time behind a switch over the type, a row of 11008 took 25 us)
+// (a thread's elements are 256 apart, kAhead of them requested at a time: one at a time behind a switch over the type, a row of 11008 took 25 us.  Of short rows as many
+// as there are: 2000 rows of 512 7.8 us with 16 ahead, 5.9 one at a time, 5.1 with 4)
 template <typename T>
 __device__ __forceinline__ float i8_row_value(T v);
 template <>
@@ -105,10 +106,9 @@ struct f16_raw { f16_t v; };
 template <>
 __device__ __forceinline__ float i8_row_value<f16_raw>(f16_raw v) { return f16_to_f32(v.v); }
 
-template <typename T>
+template <typename T, int kAhead>
 __global__ __launch_bounds__(256) void i8_stage_kernel(const T* x, int64_t ldx, const void* norm_scale, int norm_dtype, float eps, float threshold, int K,
                                                        int Kp, f16_t* xh, float* sca, unsigned* mask) {
-    constexpr int kAhead = 16;
     __shared__ float red[32];
     const int m = blockIdx.x;
     const T* row = x + (int64_t)m * ldx;
@@ -167,15 +167,17 @@ __global__ __launch_bounds__(256) void i8_stage_kernel(const T* x, int64_t ldx, 
 // ---- 2. the int8 operand, the list of outlier columns (workgroup 0) and, by themselves, the outlier columns of the rows and of the weights: the
 // epilogue then multiplies dense f16 matrices.  (It used to gather both per block of the product, a weight byte, a division and an f16 activation per element
 // and token block: 295 us of a 512-token mlp.c_proj; and the list was one thread's chain of dependent loads: 25 of this launch's 30 us.)
-// Workgroups 0 .. M - 1: a row each; the others: the weights, 16 rows x 32 columns per wave and turn.
+// Workgroups 0 .. M - 1: a row each; the others: the weights, 16 rows x 32 columns per wave and turn.  Tables of the columns there are, and none of a
+// call without outliers (2000 rows, N = K = 512, all launches of the product: 26.2 us with tables of 16 384 columns and 16 requests ahead above, 22.5 now; N = K = 1024 40.9, 37.1).
 constexpr int kMaskWords = 512;  // of the mask per turn: 16 384 columns
+constexpr int kQuantLds = 4 + 4 + 64;
 __global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int8_t* ca, int* olist, const I8GemmParams p, int R) {
-    __shared__ unsigned words[kMaskWords];
-    __shared__ int before[kMaskWords];  // outlier columns in front of a word
-    __shared__ uint16_t cols[kMaskWords * 32];  // the outlier columns of this turn, from its first word on
+    extern __shared__ unsigned words[];  // kQuantLds bytes per word
     __shared__ int wave_tot[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int Kp = p.Kp, nw = Kp >> 5, m = blockIdx.x;
+    const int Kp = p.Kp, nw = Kp >> 5, m = blockIdx.x, held = nw < kMaskWords ? nw : kMaskWords;
+    int* before = (int*)words + held;               // outlier columns in front of a word
+    uint16_t* cols = (uint16_t*)(before + held);    // the outlier columns of this turn, from its first word on
     int n_out;
     {
         int c = 0;
@@ -199,29 +201,33 @@ __global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int
     for (int w0 = 0; w0 < nw; w0 += kMaskWords) {
         const int cnt = nw - w0 < kMaskWords ? nw - w0 : kMaskWords;
         const int per = (cnt + 255) / 256, lo = threadIdx.x * per, hi = lo + per < cnt ? lo + per : cnt;
-        __syncthreads();  // (the last turn is done with words, before and wave_tot)
-        int c = 0;
-        for (int w = lo; w < hi; ++w) {
-            words[w] = mask[w0 + w];
-            c += __popc(words[w]);
-        }
-        int incl = c;
+        const int j_lo = carry;  // outlier columns of this turn: j_lo .. j_hi - 1
+        int j_hi = carry;
+        if (n_out > 0) {
+            __syncthreads();  // (the last turn is done with words, before and wave_tot)
+            int c = 0;
+            for (int w = lo; w < hi; ++w) {
+                words[w] = mask[w0 + w];
+                c += __popc(words[w]);
+            }
+            int incl = c;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int up = __shfl_up(incl, o);
+                if (lane >= o) incl += up;
+            }
+            if (lane == 63) wave_tot[wave] = incl;
+            __syncthreads();
+            int at = carry + incl - c;
+            for (int w = 0; w < wave; ++w) at += wave_tot[w];
+            j_hi = carry + wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
+            carry = j_hi;
+            for (int w = lo; w < hi; ++w) {
+                before[w] = at;
+                for (unsigned bits = words[w]; bits != 0u; ++at, bits &= bits - 1u) cols[at - j_lo] = (uint16_t)(w * 32 + __builtin_ctz(bits));
+            }
+            __syncthreads();
         }
-        if (lane == 63) wave_tot[wave] = incl;
-        __syncthreads();
-        int at = carry + incl - c;
-        for (int w = 0; w < wave; ++w) at += wave_tot[w];
-        const int j_lo = carry, j_hi = carry + wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];  // outlier columns of this turn
-        carry = j_hi;
-        for (int w = lo; w < hi; ++w) {
-            before[w] = at;
-            for (unsigned bits = words[w]; bits != 0u; ++at, bits &= bits - 1u) cols[at - j_lo] = (uint16_t)(w * 32 + __builtin_ctz(bits));
-        }
-        __syncthreads();
         if (m == 0)
             for (int j = j_lo + (int)threadIdx.x; j < j_hi; j += 256) olist[1 + j] = w0 * 32 + cols[j - j_lo];
         if (of_row) {
@@ -237,7 +243,7 @@ __global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int
                     const int k4 = k0 + 256 * i;
                     if (k4 >= e4) continue;
                     const int k = 4 * k4, w = (k >> 5) - w0;
-                    const unsigned bits = words[w] >> (k & 31);
+                    const unsigned bits = n_out > 0 ? words[w] >> (k & 31) : 0u;
                     uint32_t q4 = 0u;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
@@ -756,8 +762,8 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     MI355_LAUNCH_CHECK();
     auto stage = [&](auto type) {
         using T = decltype(type);
-        hipLaunchKernelGGL(i8_stage_kernel<T>, dim3(a->M), dim3(256), 0, s, (const T*)a->x, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->threshold, a->K, kp,
-                           xh, sca, mask);
+        auto kernel = kp <= 1024 ? i8_stage_kernel<T, 4> : kp <= 2048 ? i8_stage_kernel<T, 8> : i8_stage_kernel<T, 16>;
+        hipLaunchKernelGGL(kernel, dim3(a->M), dim3(256), 0, s, (const T*)a->x, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->threshold, a->K, kp, xh, sca, mask);
     };
     if (a->x_dtype == MI355_F32) stage(float{});
     else if (a->x_dtype == MI355_BF16) stage(bf16_t{});
@@ -791,7 +797,7 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     p.part = part;
     p.xo = xo;
     p.so = so;
-    hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), 0, s, mask, ca, olist, p, a->R);
+    hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), (kp / 32 < kMaskWords ? kp / 32 : kMaskWords) * kQuantLds, s, mask, ca, olist, p, a->R);
     MI355_LAUNCH_CHECK();
     if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, s);
     if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, s);
