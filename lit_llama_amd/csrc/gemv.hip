@@ -1240,8 +1240,9 @@ int gemv_prepare(const mi355_linear_args* a, GemvParams& p, int& grid, int& wave
     p.norm_add = (a->flags & MI355_LF_NORM_ONE) ? 1.f : 0.f;
     MI355_CHECK_ARG(!p.relu2 || a->epi == MI355_EPI_STORE, MI355_E_ARG, "linear_fast: RELU2 belongs to the STORE epilogue");
     // rows of at most four units: four waves, one unit each as with eight, and twice the workgroups (of eight, four had nothing to do: N = 32000,
-    // K = 256 11.3 -> 8.1 us, N = K = 256 3.6 -> 3.3; the same bits)
-    const bool few = a->waves <= 0 && p.units <= 4;
+    // K = 256 11.3 -> 8.1 us, N = K = 256 3.6 -> 3.3; the same bits).  Pairs of more than four rows of three or four units keep eight, whose combining step is the longer
+    // part (N = 4096, K = 512, 8 / 16 rows 7.7 / 10.6 us with eight waves, 8.4 / 12.9 with four; N = 32000, K = 256, 8 rows 18.4 / 13.7)
+    const bool few = a->waves <= 0 && p.units <= (a->R == 1 || a->M <= 4 ? 4 : 2);
     waves = a->waves > 0 ? a->waves : few ? 4 : 8;
     if (waves > 16) waves = 16;
     if ((a->fmt != MI355_W_Q4 || (a->group_cols > 0 && a->group_cols < a->K)) && waves > 8) waves = 8;  // see kMaxThreads
