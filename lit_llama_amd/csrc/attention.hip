@@ -1,7 +1,7 @@
 // RoPE + KV-cache write + causal attention for gfx950.
 //
 // Replaces the body of CausalSelfAttention.forward between the two linears
-// (/root/reference lit_llama/model.py:199-232): q/k/v split, apply_rope (:306-323), the out-of-place
+// (lit_llama/model.py:199-232): q/k/v split, apply_rope (:306-323), the out-of-place
 // cache index_copy (:219-220, here an in-place row write), and F.scaled_dot_product_attention with the
 // boolean causal mask (:230) — which the reference evaluates over all S cache rows; here only rows
 // [0, slot] are read.
@@ -684,7 +684,7 @@ extern "C" int mi355_attn_combine(const float* partials, int n_split, int rows, 
 }
 
 // ------------------------------------------------------------------------------------ LLaMA-Adapter prefix term
-// y[row, h, :] += gate[h] * softmax(rope(q[row, h]) . ak[h]^T / sqrt(hs)) av[h]      (/root/reference lit_llama/adapter.py:134-151:
+// y[row, h, :] += gate[h] * softmax(rope(q[row, h]) . ak[h]^T / sqrt(hs)) av[h]      (lit_llama/adapter.py:134-151:
 // the adaption prompt's keys / values carry no RoPE and no mask, the softmax is its own, the gate is per head).
 // One wave per (row, head): a lane holds the interleaved pairs lane, lane + 64 of the query (RoPE is lane-local), the
 // aT (ten) prefix rows are walked with a running (max, sum, weighted values) — f32 throughout.

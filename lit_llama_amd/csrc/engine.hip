@@ -1,4 +1,4 @@
-// Whole-forward entry of libmi355llama: LLaMA.forward (/root/reference lit_llama/model.py:76-122) for
+// Whole-forward entry of libmi355llama: LLaMA.forward (lit_llama/model.py:76-122) for
 // B = 1 and T <= max_T tokens with KV cache, entered ONCE per call from the host and, for the T = 1
 // decode step, captured in a hipGraph and replayed.
 //

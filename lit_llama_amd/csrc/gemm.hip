@@ -1,6 +1,6 @@
 // Wide (several tokens) linear over the int4 or the bf16 weight stream for gfx950: prompt prefill, no-cache evaluation, batches of decoding sequences.
 //
-// Replaces the reference's Triton `linear_kernel_4bit_weight` (/root/reference lit_llama/quantization.py:187-333,
+// Replaces the reference's Triton `linear_kernel_4bit_weight` (lit_llama/quantization.py:187-333,
 // reached from ColBlockQuantizedLinear.forward :413-421) at the shapes of evaluate/full.py:120-129 (T = 2048, no cache)
 // and of generate.py's prompt pass — where the skinny weight-streaming kernel (gemv.hip) re-reads the whole weight
 // stream once per 13 tokens.
@@ -31,7 +31,7 @@
 #include "common.h"
 #include "gemm_fuse.h"
 
-// The epilogues' conversions on the hardware paths (round 6: with IEEE division + expf in SiLU and the six-instruction software rounding
+// The epilogues' conversions on the hardware paths (with IEEE division + expf in SiLU and the six-instruction software rounding
 // the c_fc1 / c_fc2 epilogue was VALU-bound — 33 us of a 269-us launch at T = 2048 against 9 us for its 45 MB of stores,
 // profiles/r06_prefill_epilogue_cost.txt): v_cvt_pk_bf16_f32 rounds to nearest even exactly as f32_to_bf16 does (finite inputs),
 // v_exp_f32 / v_rcp_f32 are within 1 ulp of f32 — 2^-15 of the bf16 step the result is rounded to.
@@ -695,11 +695,11 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
     }
 }
 
-// FMT = MI355_W_Q4: int4 stream, one 1-KiB piece per (tile, unit), converted below; MI355_W_BF16: unquantised weights
-// (BASELINE configs[1]), four 1-KiB pieces per (tile, unit) whose piece d IS the A fragment of k-quarter d — same k
+// FMT = MI355_W_Q4: int4 stream, one 1-KiB piece per (tile, unit), converted below; MI355_W_BF16: unquantised weights,
+// four 1-KiB pieces per (tile, unit) whose piece d IS the A fragment of k-quarter d — same k
 // order as the int4 conversion produces, no conversion, scale 1 / zero-point 0 in the epilogue
 // GRP (Q4): 0 one (scale, zero) pair per output row; 2: one pair per row and group of 32 or 64 input columns (GPTQ "groupsize",
-// /root/reference lit_llama/quantization.py:284-333 with tile_cols > 0; groups of whole units: gemm_deep_kernel).  The MFMA accumulators keep running over K (cum_g =
+// lit_llama/quantization.py:284-333 with tile_cols > 0; groups of whole units: gemm_deep_kernel).  The MFMA accumulators keep running over K (cum_g =
 // columns up to the end of group g) and at every group
 // end     accf += (s_g - s_{g+1}) cum_g - s_g (128 + z_g) X_g      (Abel summation of sum_g s_g (A_g - (128 + z_g) X_g),
 // s past the last group = 0; X_g = the group's operand sum from stage_units_kernel): two FMAs per output element
@@ -777,7 +777,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
         for (int d = 0; d < kWP; ++d)
             dst[d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off + d * 1024u : 0u, 0));
     };
-    // BF16 streams (round 6): piece d of the NEXT unit is requested into the registers piece d of this unit just left (behind its MFMAs):
+    // BF16 streams: piece d of the NEXT unit is requested into the registers piece d of this unit just left (behind its MFMAs):
     // no second register set — 32 registers less, two workgroups per CU without the scratch the occupancy hint had bought them with
     constexpr bool kRefill = FMT == MI355_W_BF16 && GRP == 0;
     [[maybe_unused]] auto wload1 = [&](int t, int u, int d, u32x4& dst) {
@@ -786,7 +786,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
         dst = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off + d * 1024u : 0u, 0));
     };
     // activation block of unit u: 2048 chunks of 16 B, kXChunks per thread; chunk = (token, 16-B column)
-    // Round 6: the activation block of the NEXT unit goes global -> LDS by LDS-DMA (buffer_load ... lds, 16 B per lane: one instruction
+    // The activation block of the NEXT unit goes global -> LDS by LDS-DMA (buffer_load ... lds, 16 B per lane: one instruction
     // fills 1 KiB = four token rows of the buffer; the XOR swizzle is applied on the SOURCE side — LDS slot c of token t takes column
     // c ^ swz(t)), requested at the unit's start.  The staged version held the block in 32 registers per thread, which hipcc could only
     // afford by sinking the requests to the unit's END, right in front of the LDS stores that wait for them: every unit paid the memory

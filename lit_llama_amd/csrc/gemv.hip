@@ -1,7 +1,7 @@
 // Skinny (M <= 16) weight-streaming linear for gfx950: the decode hot kernel.
 //
 // Replaces, for decode shapes, the reference's Triton `linear_kernel_4bit_weight`
-// (/root/reference lit_llama/quantization.py:187-333, reached from
+// (lit_llama/quantization.py:187-333, reached from
 // ColBlockQuantizedLinear.forward :413-421) and the dense F.linear of lit_llama/model.py.
 //
 // Design:
@@ -422,7 +422,7 @@ constexpr int kMaxThreads = (FMT == MI355_W_Q4 && P <= 4 && !GRP) ? 1024 : 512;
 // tiles that reach the epilogue are then plain sums.
 constexpr int kGrpLoadsMax = 12; // GRP = (scale, zero) pairs per thread, matrix and tile: 16 n_groups <= GRP x threads (1, 4 or 12;
                                  // every pair is an issued buffer load whether it fetches or not: 32 groups over 512 threads need one).
-                                 // 12 (round 6) admits 384 groups per row: groupsize 32 against K = 11008 (344), which the cap of 4 x 512 / 16
+                                 // 12 admits 384 groups per row: groupsize 32 against K = 11008 (344), which the cap of 4 x 512 / 16
                                  // = 128 groups had kept — with groupsize 64 (172) — off the engine altogether
 constexpr int kGrpLoadsMid = 4;
 

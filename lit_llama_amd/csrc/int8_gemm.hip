@@ -1,7 +1,7 @@
 // Wide (M >= 32 tokens) LLM.int8 linear for gfx950: prompt prefill / no-cache evaluation of a `--quantize llm.int8` model.
 //
 // Replaces, for B * T >= 32 rows, bitsandbytes' MatMul8bitLt forward as Linear8bitLt reaches it
-// (/root/reference lit_llama/quantization.py:38-77; the algorithm is restated in oracle/oracle.py::llm_int8_linear — PARITY
+// (lit_llama/quantization.py:38-77; the algorithm is restated in oracle/oracle.py::llm_int8_linear — PARITY
 // UNPINNED: bitsandbytes is not vendored).  The skinny kernel (int8.hip) feeds such inputs in chunks
 // of <= 16 rows and determines the outlier COLUMN set per chunk; this path determines it over all rows of the call, as the
 // algorithm does, and runs the int8 product on v_mfma_i32_16x16x64_i8 over 128-token blocks:
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         // mixed-precision decomposition: the outlier columns in f16, ascending k, kOutChunk columns per pass through LDS
         f16_t* xo = (f16_t*)smem;                     // [128 tokens][kOutChunk]
         f16_t* so = xo + kBM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
-        // (round 6: the side product runs on v_mfma_f32_16x16x32_f16 — A = 16 rows x 32 outlier columns of `so`, B = 16 tokens x the same
+        // (the side product runs on v_mfma_f32_16x16x32_f16 — A = 16 rows x 32 outlier columns of `so`, B = 16 tokens x the same
         // columns of `xo`, result in the accumulators' own layout: lane (g, c) holds rows 4 g .. 4 g + 3 for token c.  The products of two f16
         // values are exact in f32 and the sum is f32 as before; its ORDER inside a block of 32 columns is the hardware's instead of
         // ascending k — bitsandbytes' own f16 GEMM promises no order either, and the tests allow the one f16 ulp this can move.  The scalar
