@@ -5,7 +5,7 @@
 // and of generate.py's prompt pass — where the skinny weight-streaming kernel (gemv.hip) re-reads the whole weight
 // stream once per 13 tokens.
 //
-// Design (gemm_q4_kernel; launches of about one workgroup per CU and grouped scales: gemm_deep_kernel, three units of operands under way):
+// Design (gemm_q4_kernel, the int4 stream; BF16, launches of about one workgroup per CU and grouped scales: gemm_deep_kernel, up to three units of operands under way):
 //  * the weights stay in the decode path's stream layout [tile of 16 rows][unit of 128 k][r][lane][16 B]: a wave reads
 //    a (tile, unit) piece with ONE coalesced 1-KiB load straight into registers (no LDS for weights: a piece is
 //    private to its wave) and turns it into four MFMA A fragments with 7 VALU ops per 8 weights — amortised over the
@@ -65,15 +65,6 @@ constexpr int kTPW = MI355_GEMM_TPW;
 #endif
 #ifndef MI355_GEMM_AND_OR
 #define MI355_GEMM_AND_OR 1
-#endif
-#ifndef MI355_GEMM_BF16_ROWMAJOR
-// workgroup order of the BF16 streams: row block major (an XCD runs every token block of a few row blocks side by side).  Token block major
-// (the int4 order) carried every weight piece across the fabric once per token block: 16 x 13.5 GB = 216 GB per 2048-token pass of the 7B
-// model, 6.3 TB/s of its 34 ms.  2048 tokens 34.0 -> 28.5 ms, 512 tokens 16.5 -> 10.6 ms (profiles/r06_ab_bf16_block_order.txt)
-#define MI355_GEMM_BF16_ROWMAJOR 1
-#endif
-#ifndef MI355_GEMM_Q4_ROWMAJOR
-#define MI355_GEMM_Q4_ROWMAJOR 0
 #endif
 struct GemmParams {
     const uint8_t* w;
@@ -695,10 +686,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
     }
 }
 
-// FMT = MI355_W_Q4: int4 stream, one 1-KiB piece per (tile, unit), converted below; MI355_W_BF16: unquantised weights,
-// four 1-KiB pieces per (tile, unit) whose piece d IS the A fragment of k-quarter d — same k
-// order as the int4 conversion produces, no conversion, scale 1 / zero-point 0 in the epilogue
-// GRP (Q4): 0 one (scale, zero) pair per output row; 2: one pair per row and group of 32 or 64 input columns (GPTQ "groupsize",
+// The int4 stream, one 1-KiB piece per (tile, unit).
+// GRP: 0 one (scale, zero) pair per output row; 2: one pair per row and group of 32 or 64 input columns (GPTQ "groupsize",
 // lit_llama/quantization.py:284-333 with tile_cols > 0; groups of whole units: gemm_deep_kernel).  The MFMA accumulators keep running over K (cum_g =
 // columns up to the end of group g) and at every group
 // end     accf += (s_g - s_{g+1}) cum_g - s_g (128 + z_g) X_g      (Abel summation of sum_g s_g (A_g - (128 + z_g) X_g),
@@ -708,17 +697,13 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 // FUSE: the producer / consumer fusion of gemm_fuse.h (ungrouped launches without a K split): operand sums and 1/rms from
 // partial sums instead of the staging pass; the residual epilogue emits the next linear's bf16 operand and its partial
 // sums, the SwiGLU epilogue the partial operand sums of its output, the c_attn epilogue rotates k and writes the K / V cache
-// (second launch-bound argument, waves per SIMD: BF16 streams at 128 VGPRs keep two workgroups per CU, at 132-138 the 2048-token c_fc1/c_fc2 product took
-// 300 us instead of 256)
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
-__global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4 : 1) void gemm_q4_kernel(const GemmParams p) {
-    static_assert(GRP == 0 || FMT == MI355_W_Q4, "grouped scales are a Q4 feature");
+template <int EPI, bool PAIR, int kWaves, int BM, int GRP = 0, bool FUSE = false>
+__global__ __launch_bounds__(64 * kWaves) void gemm_q4_kernel(const GemmParams p) {
     static_assert(!FUSE || GRP == 0, "the fused chain runs over per-row scales");
     constexpr int kTT = BM / 16;                   // 16-token tiles per block
     constexpr int kSlots = kWaves * kTPW;          // tile slots per block
     constexpr int kThreads = 64 * kWaves;
     constexpr int kXChunks = BM * 16 / kThreads;   // 16-B activation chunks per thread and unit
-    constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;  // pieces per (tile, unit)
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -730,17 +715,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     const int L2 = xcd * p.per_xcd + j;
     if (j >= p.per_xcd || L2 >= p.total_blocks * p.ksplit) return;
     const int L = L2 / p.ksplit, ks = L2 - L * p.ksplit;  // (ksplit = 1: ks = 0, all units)
-    int mb, nb;
-    if constexpr (FMT == MI355_W_BF16 ? MI355_GEMM_BF16_ROWMAJOR != 0 : MI355_GEMM_Q4_ROWMAJOR != 0) {
-        // row block major — an XCD runs every token block of a few row blocks side by side, so a weight piece (BF16: 4 x the
-        // bytes of an int4 one) crosses the fabric once per XCD instead of once per token block
-        const int m_blocks = p.total_blocks / n_blocks;
-        nb = L / m_blocks;
-        mb = L - nb * m_blocks;
-    } else {
-        mb = L / n_blocks;
-        nb = L - mb * n_blocks;
-    }
+    const int mb = L / n_blocks, nb = L - mb * n_blocks;
     const int m0 = mb * BM;
     float* fr = (float*)(smem + 2 * BM * 256);  // [BM] 1/rms, [BM] operand sums of the block's tokens
     [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM>);            // FUSE, STORE: [BM] positions
@@ -762,28 +737,14 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (int)p.w_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw0 = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, 0, 0x00020000);
     const unsigned xbytes = (unsigned)((int64_t)p.M * p.ldxb * 2);
-    const bf16_t* xbase = p.xb;
-    if constexpr (EPI == MI355_EPI_STORE && FMT == MI355_W_BF16 && !FUSE) {
-        if (p.slice_blocks != 0) xbase += (int64_t)(nb / p.slice_blocks) * p.slice_stride;
-    }
-    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)xbytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)p.xb, 0, (int)xbytes, 0x00020000);
     const unsigned lane_off = lane * 16;
-    auto wload = [&](int t, int u, u32x4 (&dst)[kWP]) {
+    auto wload = [&](int t, int u) {
         // past the last unit / tile the load goes through a zero-sized descriptor: the scalar offset operand of a raw
         // buffer load is NOT range-checked (an unconditional prefetch of unit `units` of the last tile faulted)
         const bool ok = tile[t] < p.n_tiles && u < u_hi;
-        const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + rr[t]) * (1024u * kWP);
-#pragma unroll
-        for (int d = 0; d < kWP; ++d)
-            dst[d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off + d * 1024u : 0u, 0));
-    };
-    // BF16 streams: piece d of the NEXT unit is requested into the registers piece d of this unit just left (behind its MFMAs):
-    // no second register set — 32 registers less, two workgroups per CU without the scratch the occupancy hint had bought them with
-    constexpr bool kRefill = FMT == MI355_W_BF16 && GRP == 0;
-    [[maybe_unused]] auto wload1 = [&](int t, int u, int d, u32x4& dst) {
-        const bool ok = tile[t] < p.n_tiles && u < u_hi;
-        const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + rr[t]) * (1024u * kWP);
-        dst = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off + d * 1024u : 0u, 0));
+        const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + rr[t]) * 1024u;
+        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ok ? rw : rw0, lane_off, ok ? off : 0u, 0));
     };
     // activation block of unit u: 2048 chunks of 16 B, kXChunks per thread; chunk = (token, 16-B column)
     // The activation block of the NEXT unit goes global -> LDS by LDS-DMA (buffer_load ... lds, 16 B per lane: one instruction
@@ -831,9 +792,9 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
 #pragma unroll
         for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    u32x4 wcur[kTPW][kWP], wnext[kRefill ? 1 : kTPW][kRefill ? 1 : kWP];
+    u32x4 wcur[kTPW], wnext[kTPW];
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t) wload(t, u_lo, wcur[t]);
+    for (int t = 0; t < kTPW; ++t) wcur[t] = wload(t, u_lo);
     if constexpr (kXDma) xdma(u_lo, u_lo & 1);
     xload(u_lo);
     if constexpr (FUSE) {
@@ -870,7 +831,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     }
     // what the epilogue needs of the block's rows and tokens, fetched behind the first unit's operands: there each of these loads, behind a branch of
     // its own, was waited for alone (24 memory round trips per launch)
-    if constexpr (FMT == MI355_W_Q4 && GRP == 0) {
+    if constexpr (GRP == 0) {
         for (int i = threadIdx.x; i < kSlots * 16; i += kThreads) {
             const int slot = i >> 4;
             const int n = (PAIR ? nb * (kSlots / 2) + (slot >> 1) : nb * kSlots + slot) * 16 + (i & 15);
@@ -902,7 +863,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
         for (int t = threadIdx.x; t < BM; t += kThreads) {
             const int m = m0 + t < p.M ? m0 + t : p.M - 1;
             fr[t] = p.rinv != nullptr ? p.rinv[m] : p.alpha;
-            fr[BM + t] = (GRP || FMT == MI355_W_BF16) ? 0.f : p.sx[(int64_t)m * p.ksplit + ks];  // (BF16 weights have no zero point)
+            fr[BM + t] = GRP ? 0.f : p.sx[(int64_t)m * p.ksplit + ks];
         }
     }
     if constexpr (FUSE && EPI == MI355_EPI_STORE) {
@@ -934,19 +895,15 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     auto prefetch = [&](int u) {
         if constexpr (kXDma) {
             // (weights first: HBM latency; both pinned at the unit's start — they cost 8 registers now, not 40)
-            if constexpr (!kRefill) {
 #pragma unroll
-                for (int t = 0; t < kTPW; ++t) wload(t, u + 1, wnext[t]);
-            }
+            for (int t = 0; t < kTPW; ++t) wnext[t] = wload(t, u + 1);
             xdma(u + 1, (u & 1) ^ 1);
             __builtin_amdgcn_sched_barrier(0);
             return;
         }
         xload(u + 1);
-        if constexpr (!kRefill) {
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t) wload(t, u + 1, wnext[t]);
-        }
+        for (int t = 0; t < kTPW; ++t) wnext[t] = wload(t, u + 1);
     };
     // the 4 x kTT x kTPW MFMAs of a unit; sub >= 0 (GRP 2): only the lane groups of sub-group `sub` contribute
     // (explicitly software-pipelined B-fragment reads — 16 fragments in registers, pinned with sched_barrier —
@@ -956,14 +913,13 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     asm volatile("" : "+s"(cmask));
     asm volatile("" : "+v"(cmagic));
 #endif
-    constexpr int kBPipe = (GRP == 0 && BM == 128 && FMT == MI355_W_Q4) ? MI355_GEMM_BPIPE : 0;
+    constexpr int kBPipe = (GRP == 0 && BM == 128) ? MI355_GEMM_BPIPE : 0;
     auto bread = [&](const char* xs, int d, int tt, bool mine) {
         const int tok = tt * 16 + c;
         u32x4 braw = *(const u32x4*)(xs + tok * 256 + (((4 * g + d) ^ swz(tok)) << 4));
         if constexpr (GRP == 2) braw = mine ? braw : u32x4{0u, 0u, 0u, 0u};
         return braw;
     };
-    [[maybe_unused]] int u_refill = 0;  // kRefill: the unit whose pieces mfmas() requests
     auto mfmas = [&](int buf, int sub, int sub_shift) {
         const char* xs = smem + buf * (BM * 256);
         const bool mine = GRP != 2 || (g >> sub_shift) == sub;
@@ -974,27 +930,23 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
             bf16x8 a[kTPW];
 #pragma unroll
             for (int t = 0; t < kTPW; ++t) {
-                if constexpr (FMT == MI355_W_BF16) {
-                    a[t] = __builtin_bit_cast(bf16x8, wcur[t][d]);
-                } else {
-                    const uint32_t v = wcur[t][0][d];
-                    u32x4 f;
+                const uint32_t v = wcur[t][d];
+                u32x4 f;
 #if MI355_GEMM_AND_OR
-                    // (mask and exponent pattern as OPAQUE register values: hipcc then selects one v_and_or_b32 per field
-                    // — from literals it emits v_and + v_or, 11 instead of 7 VALU per dword — and pads the VALU -> MFMA
-                    // hazard itself, which an inline-asm v_and_or_b32 does not get: csrc/fused_step_ring.hip nib2f16)
-                    f[0] = (v & cmask) | cmagic;
-                    f[1] = ((v >> 4) & cmask) | cmagic;
-                    f[2] = ((v >> 8) & cmask) | cmagic;
-                    f[3] = ((v >> 12) & cmask) | cmagic;
+                // (mask and exponent pattern as OPAQUE register values: hipcc then selects one v_and_or_b32 per field
+                // — from literals it emits v_and + v_or, 11 instead of 7 VALU per dword — and pads the VALU -> MFMA
+                // hazard itself, which an inline-asm v_and_or_b32 does not get: csrc/fused_step_ring.hip nib2f16)
+                f[0] = (v & cmask) | cmagic;
+                f[1] = ((v >> 4) & cmask) | cmagic;
+                f[2] = ((v >> 8) & cmask) | cmagic;
+                f[3] = ((v >> 12) & cmask) | cmagic;
 #else
-                    f[0] = (v & 0x000F000Fu) | 0x43004300u;
-                    f[1] = ((v >> 4) & 0x000F000Fu) | 0x43004300u;
-                    f[2] = ((v >> 8) & 0x000F000Fu) | 0x43004300u;
-                    f[3] = ((v >> 12) & 0x000F000Fu) | 0x43004300u;
+                f[0] = (v & 0x000F000Fu) | 0x43004300u;
+                f[1] = ((v >> 4) & 0x000F000Fu) | 0x43004300u;
+                f[2] = ((v >> 8) & 0x000F000Fu) | 0x43004300u;
+                f[3] = ((v >> 12) & 0x000F000Fu) | 0x43004300u;
 #endif
-                    a[t] = __builtin_bit_cast(bf16x8, f);
-                }
+                a[t] = __builtin_bit_cast(bf16x8, f);
             }
             if constexpr (kBPipe > 0) {
                 // fragment s = d * kTT + tt of the unit; bq holds the next kBPipe of them.  The group barriers pin "one LDS read (of
@@ -1022,20 +974,12 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
                     for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[t][tt], 0, 0, 0);
                 }
             }
-            if constexpr (kRefill) {
-#pragma unroll
-                for (int t = 0; t < kTPW; ++t) wload1(t, u_refill, d, wcur[t][d]);
-            }
         }
     };
     auto rotate = [&](int buf) {
         xstore(buf ^ 1);
-        if constexpr (!kRefill) {
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-                for (int d = 0; d < kWP; ++d) wcur[t][d] = wnext[t][d];
-        }
+        for (int t = 0; t < kTPW; ++t) wcur[t] = wnext[t];
         __syncthreads();
     };
 
@@ -1043,7 +987,6 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
     if constexpr (GRP == 0) {
         for (int u = u_lo; u < u_hi; ++u) {
             prefetch(u);
-            u_refill = u + 1;
             mfmas(u & 1, 0, 0);
             rotate(u & 1);
         }
@@ -1123,7 +1066,7 @@ __global__ __launch_bounds__(64 * kWaves, (FMT == MI355_W_BF16 && BM == 128) ? 4
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = accf[t][tt];
     }
-    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
+    gemm_epilogue<EPI, PAIR, MI355_W_Q4, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
 // 16 B per lane from `off` + `scalar_off` of a buffer to 1 KiB of LDS (lane i's bytes at 16 i); out of range: zeros
@@ -1131,11 +1074,23 @@ __device__ __forceinline__ void lds_from(__amdgpu_buffer_rsrc_t r, char* lds, un
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, scalar_off, 0, 0);
 }
 
+// Four bytes per lane, each lane's from its own place, to 256 B of LDS that nobody reads: what this is for are the cache lines
+__device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, unsigned off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, off, 0, 0, 0);
+}
+
 // The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of longer ones):
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
-// BM: 16 / 32 / 48 / 64 / 128 tokens.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
+// BM: 16 / 32 / 48 / 64 / 128 tokens, BF16 also 96 / 192 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
+// BF16: what bounds it is the CU's memory pipeline, which returns data in the order of the requests and holds some 50 KB of them: with nothing but its requests (no
+// products) a block of 128 tokens x 256 rows took 1.67 us for the 96 KB of a unit, 0.95 when all of it lay in L2.  So the requests of a unit are spread over all of its
+// products (in the first half of them, as before, the waves stood at requests that the pipeline had no room for: N = 4096, K = 16512, 2048 tokens 248 -> 226 us with what follows,
+// N = 12288, K = 4096 214 -> 186); large blocks ask for fewer bytes per product; and where four blocks or more of a row block run on an XCD, they bring its weights to
+// the XCD's L2 a round ahead, each a share, one lane per cache line: a block then waits for HBM once per round for its share and not for every line behind
+// every other (N = 4096, K = 11008, 777 tokens in blocks of 64 x 256 102 -> 90 us; blocks of 64 x 128 7 % less on average, of 128 x 128 4 %; 8 waves from 128 tokens on nothing).  The
+// activations likewise: 5-25 % slower, few blocks of an XCD share them.  A last block of few tokens runs ahead of the others and does it for them.
 // GRP (Q4, groups of whole 128-column units): the products of a unit start from 0, and accf += s_unit * them, one FMA per output element and unit on the
 // VALU beside the next unit's products; the zero points, accf -= sum over units of s (128 + z) X_unit (X: the unit's operand sums), are a product with K =
 // units / 4 of their own on the f32 MFMA in front of the loop.
@@ -1145,7 +1100,7 @@ template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH,
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
     static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1 && !FUSE), "grouped scales are a Q4 feature");
     static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
-    static_assert(DEPTH == 3 || DEPTH == 4, "units under way + 1");
+    static_assert(DEPTH >= 2 && DEPTH <= 4, "units under way + 1");
     constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
     constexpr int kXI = BM / 4 > kWaves ? BM / 4 / kWaves : 1;  // activation requests (1 KiB: four tokens) per wave and unit
@@ -1179,6 +1134,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
     for (int t = 0; t < kTPW; ++t)
         tile[t] = PAIR ? nb * (kSlots / 2) + (kTPW / 2) * wave + (t >> 1) : nb * kSlots + kTPW * wave + t;
+    // this block's share of its row block's weights (see above): thread i's line of every round of DEPTH units, at touch_off from the round's first unit
+    constexpr bool kTouch = FMT == MI355_W_BF16 && (BM == 64 || (BM > 64 && kWaves == 4));
+    constexpr int kTouchAhead = 2 * DEPTH - 1, kStreams = PAIR ? kSlots / 2 : kSlots, kRun = DEPTH * (PAIR ? 64 : 32);  // kRun: lines of DEPTH units of a tile
+    constexpr unsigned kNone = 0xFFFFFFF0u;
+    [[maybe_unused]] unsigned touch_off = kNone;
+    if constexpr (kTouch) {
+        const int first = xcd * p.per_xcd, last = first + p.per_xcd - 1;
+        const int lo = nb * m_blocks > first ? nb * m_blocks : first, hi = (nb + 1) * m_blocks - 1 < last ? (nb + 1) * m_blocks - 1 : last;
+        const int touch_n = hi - lo + 1, share = (kStreams * kRun + touch_n - 1) / touch_n;
+        const int line = (L - lo) * share + (int)threadIdx.x, stream = line / kRun, at = line - stream * kRun;
+        if (p.ksplit == 1 && touch_n >= 4 && (p.M - 1) % BM >= BM / 2 && (int)threadIdx.x < share && line < kStreams * kRun && nb * kStreams + stream < p.n_tiles)
+            touch_off = (unsigned)((nb * kStreams + stream) * p.units) * (PAIR ? 8192u : 4096u) + at * 128u;
+    }
+    [[maybe_unused]] const bool touching = __builtin_amdgcn_ballot_w64(touch_off != kNone) != 0;
     const bf16_t* xbase = p.xb;
     if constexpr (EPI == MI355_EPI_STORE && FMT == MI355_W_BF16 && !FUSE) {
         if (p.slice_blocks != 0) xbase += (int64_t)(nb / p.slice_blocks) * p.slice_stride;
@@ -1220,6 +1189,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * (1024u * kWP) + d * 1024u;
             wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane_off, ok ? off : 0u, 0));
         }
+    };
+
+    [[maybe_unused]] auto touch = [&](int u) __attribute__((always_inline)) {  // (a round that is not whole: a size of 0)
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, u + DEPTH <= u_hi ? (int)p.w_bytes : 0, 0x00020000);
+        lds_touch(rw, smem + kRowAt<BM, FUSE, DEPTH> + 3 * kSlots * 64, touch_off == kNone ? kNone : touch_off + (unsigned)u * (PAIR ? 8192u : 4096u));
     };
 
     // ---- tables of the epilogue: requested ahead of the units, written to LDS behind their requests
@@ -1314,6 +1288,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
         for (int i = 0; i < kUnit; ++i) request(i, u_lo + s, s);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kTouch) {
+            if (s == 0 && touching) touch(u_lo + DEPTH - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     [[maybe_unused]] float sxs = 0.f, sss = 0.f;
     if constexpr (FUSE) {
@@ -1416,7 +1394,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     constexpr int kFrags = 4 * kTT, kPipe = 4;
     // the requests of unit `ahead` go out between the products: a request takes the CU's memory pipeline 16 cycles, and in one burst behind the barrier
     // the waves of a workgroup stood in line for it with no product under way
-    constexpr int kEvery = kFrags >= 2 * kUnit ? kFrags / (2 * kUnit) : 1;  // fragments from one request to the next (all in the first half if it holds them)
+    constexpr int kEvery = kFrags >= kUnit ? kFrags / kUnit : 1;  // fragments from one request to the next
     constexpr int kPer = (kUnit + kFrags - 1) / kFrags;                      // requests behind one fragment
     // GRP: token tile by token tile, so the sums of one unit live in two token tiles' registers: those being summed, and those being scaled
     auto mfmas_grouped = [&](int slot, u32x4 (&w)[kTPW][kWP], u32x4 (&sz)[kTPW], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
@@ -1519,7 +1497,18 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     // with a way out between the units hipcc joins all of them in front of the loop's head and waits there for every request under way, once a round.
     auto unit = [&](auto slot, int u, auto more) __attribute__((always_inline)) {
         constexpr int s = slot, kNewer = more ? (DEPTH - 2) * kUnit : (DEPTH - 2 - s) * kUnit;
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kNewer) : "memory");
+        if constexpr (kTouch && s > 0 && s < DEPTH - 1 && more) {
+            if (touching)
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNewer + 1) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNewer) : "memory");
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kNewer) : "memory");
+        }
+        if constexpr (kTouch && s == 0 && more) {
+            if (touching) touch(u + kTouchAhead);
+        }
         if constexpr (GRP != 0)
             mfmas_grouped(s, wr[s], tb[s], u + DEPTH - 1, (s + DEPTH - 1) % DEPTH, more);
         else
@@ -1561,7 +1550,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     for (; u + DEPTH <= u_hi; u += DEPTH) {
         unit(integral_constant<int, 0>{}, u, std::true_type{});
         unit(integral_constant<int, 1>{}, u + 1, std::true_type{});
-        unit(integral_constant<int, 2>{}, u + 2, std::true_type{});
+        if constexpr (DEPTH > 2) unit(integral_constant<int, 2>{}, u + 2, std::true_type{});
         if constexpr (DEPTH == 4) unit(integral_constant<int, 3>{}, u + 3, std::true_type{});
         if constexpr (RUNS) {
             left -= DEPTH;
@@ -1571,10 +1560,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] const bool open = u < u_hi || left != p.run_units;  // the last run has units
     if (u < u_hi) {
         unit(integral_constant<int, 0>{}, u, std::false_type{});
-        if (u + 1 < u_hi) {
-            unit(integral_constant<int, 1>{}, u + 1, std::false_type{});
-            if constexpr (DEPTH == 4) {
-                if (u + 2 < u_hi) unit(integral_constant<int, 2>{}, u + 2, std::false_type{});
+        if constexpr (DEPTH > 2) {
+            if (u + 1 < u_hi) {
+                unit(integral_constant<int, 1>{}, u + 1, std::false_type{});
+                if constexpr (DEPTH == 4) {
+                    if (u + 2 < u_hi) unit(integral_constant<int, 2>{}, u + 2, std::false_type{});
+                }
             }
         }
     }
@@ -1661,8 +1652,8 @@ int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM < kBM && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, true>(p, s);
     }
-    constexpr int kDepth = BM == 128 && FMT == MI355_W_BF16 ? 3 : 4;
-    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0);
+    constexpr int kDepth = BM == 256 ? 2 : BM >= 96 && FMT == MI355_W_BF16 ? 3 : 4;
+    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
     static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr_err != hipSuccess) {
@@ -1671,16 +1662,16 @@ int launch_deep(const GemmParams& p, hipStream_t s) {
     }
     return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>, kLds, p, s);
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP = 0, bool FUSE = false>
+template <int EPI, bool PAIR, int kWaves, int BM, int GRP = 0, bool FUSE = false>
 int launch_gemm_w(const GemmParams& p, hipStream_t s) {
     constexpr int kLdsW = kRowAt<BM, FUSE> + 3 * kWaves * kTPW * 64;
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>,
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_q4_kernel<EPI, PAIR, kWaves, BM, GRP, FUSE>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLdsW);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_q4_kernel<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_q4_kernel<EPI, PAIR, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
 }
 // How a launch of one scale per row is cut: waves and tokens of a block, gemm_deep_kernel (or gemm_q4_kernel), K-slices
 struct GemmCut {
@@ -1688,7 +1679,7 @@ struct GemmCut {
     bool deep;
     int ksplit;
 };
-// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel), 0 = the rule's choice.  A cut that no kernel is
+// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep, int4: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel), 0 = the rule's choice.  A cut that no kernel is
 // instantiated for is ignored as a whole, a number of slices that does not fit by itself
 struct GemmForce {
     int waves, bm, ksplit, deep;
@@ -1704,8 +1695,9 @@ GemmForce gemm_force() {
     return f;
 }
 bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (the kernels of launch_gemm())
-    if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
-    return c.waves == 8 && (c.bm == kBM || (c.bm == 64 && (c.deep || bf16)));
+    if (bf16) return c.deep && (c.waves == 4 ? c.bm == 16 || c.bm == 32 || c.bm == 64 || c.bm == 96 || c.bm == 128 : c.waves == 8 && (c.bm == 64 || c.bm == 128 || c.bm == 192 || c.bm == 256));
+    if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 48 || c.bm == 64);
+    return c.waves == 8 && (c.bm == kBM || (c.bm == 64 && c.deep));
 }
 // blocks of `waves` waves and `bm` tokens
 int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
@@ -1744,43 +1736,48 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
     if (wide >= 384 || wide == 256) cut.bm = kBM, cut.deep = false;
     return cut;
 }
-// BF16 streams.  From 192 blocks of 128 tokens x 256 rows on those, one per CU of the deep kernel, more of gemm_q4_kernel (2048 tokens, N = 4096, K = 11008 174 -> 158 us;
-// 512 tokens, c_fc1/c_fc2 134 / 106 us with blocks of 64 / 128).  Up to 64 tokens blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
+// BF16 streams.  Up to 64 tokens blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
 // none to a few more than all (16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 /
-// 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13).  In between, and where those blocks are more than the CUs, what an estimate takes for the fastest: the busiest CU's workgroups one behind the
-// other, `start` and `unit` us for each of their units; the weights from HBM at 6.6 TB/s behind 4.3 us, both at once; and with slices 1.6 us and 1 us per
-// 2.3 MB of partial sums.  Fitted to 17 000 launches (28 products of 1024 to 32000 rows, 8 to 2000 tokens, weights not in any cache: the next layer's never are)
-// within 8 % rms; its choice is 1 % behind the fastest on average.  Blocks of 8 waves throughout, from 65 tokens on, with slices
-// to three quarters of the CUs, a rule from weights that the cache held, took 31.5 us for 160 tokens of N = K = 5120 (now 27.1), 52 / 116 for 256 / 640 of
-// N = 4096, K = 11008 (43 / 83), 107 for 128 of N = 8192, K = 22016 (87); 280 blocks of 4 waves 115 for 48 of the N = 17920 pair, K = 6656 (101).
+// 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13); where those blocks are more than the CUs, blocks of 8 (48 tokens of the N = 17920 pair, K = 6656: 104 / 95 us with 4 / 8 waves).
+// Longer: 192 to 256 blocks of 128 tokens x 256 rows, one round of the chip, take those (3-5 % less than what the estimate takes).  Else what an estimate takes for the
+// fastest: the rounds of the chip one behind the other, each the busiest CU's units (`unit` us when it is alone, `crowd` more when every CU has a block, whatever of the
+// block is padding) and its share of the bytes from HBM at once; slices cost a launch, and their sums' way to memory and back.  Blocks of 192 and 256 tokens x 256 rows ask
+// for 75 and 64 KB per 8.4 MFLOP instead of the 96 of 128 x 256, and give the rounds more sizes to fit: 2048 tokens, N = 16512, K = 4096, 4.1 rounds of 128 tokens 278 us, 2.8 of
+// 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  Fitted to 15 000
+// launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are) within 8 % rms; its choice takes 0.8 % longer than the
+// fastest on average, 2.4 % at the 90th percentile.
 GemmCut bf16_cut(int M, int N, int K, bool pair) {
-    const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
-    if (M > 128 && wide >= 192) return {8, kBM, wide <= 256, 1};
-    GemmCut cut = {4, short_block(M, true), true, 1};
-    if (M <= 64 && few <= 256) {
+    const int units = (K + 127) / 128;
+    if (M <= 64) {
+        const int few = gemm_blocks(M, N, pair, 4, 64);
+        if (few > 256) return {8, 64, true, 1};
+        GemmCut cut = {4, short_block(M, true), true, 1};
         while (cut.ksplit < kMaxSplit && few * cut.ksplit < 192 && few * (cut.ksplit + 1) <= 256 && units >= 4 * (cut.ksplit + 1) &&
                gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
             ++cut.ksplit;
         return cut;
     }
+    if (const int wide = gemm_blocks(M, N, pair, 8, kBM); wide >= 192 && wide <= 256) return {8, kBM, true, 1};
     struct Kind {
         int waves, bm;
-        bool deep;
-        float start, unit;
+        float start, unit, crowd;
     };
-    const Kind kinds[] = {{4, cut.bm, true, cut.bm == 16 ? 0.9f : cut.bm == 32 ? 1.3f : 3.0f, cut.bm == 16 ? 0.67f : cut.bm == 32 ? 0.71f : 0.75f},
-                          {8, 64, true, 4.2f, 1.27f}, {8, 64, false, 3.4f, 1.23f}, {8, kBM, true, 6.6f, 1.48f}};
-    const float bytes = 2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N, hbm = 4.3f + bytes / 6.6e6f;
+    constexpr Kind kinds[] = {{4, 64, 5.3f, 0.50f, 0.16f},  {4, 96, 5.1f, 0.68f, 0.12f},  {4, kBM, 5.0f, 0.78f, 0.22f}, {8, 64, 6.5f, 0.97f, 0.18f},
+                              {8, kBM, 6.6f, 1.29f, 0.35f}, {8, 192, 8.3f, 1.44f, 0.76f}, {8, 256, 8.8f, 2.23f, 0.86f}};
+    const float hbm = (2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N) / 7.83e6f;
+    GemmCut cut = {4, 64, true, 1};
     float best = 0.f;
     for (const Kind& k : kinds)
         for (int ks = 1; ks <= kMaxSplit && (ks == 1 || units >= 4 * ks); ++ks) {
-            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks;
             const size_t part = gemm_part_bytes(M, N, pair, ks);
-            // (128-token blocks: no two on a CU, and with slices the last CUs slow the others: 300 tokens, K = 11008, N = 4096 49.7 us with 192, 58.5 with 240)
-            if ((ks > 1 && part > kSplitBudget) || (k.bm == kBM && (M <= 64 || blocks > (ks == 1 ? 256 : 208)))) continue;
-            const float work = k.start + (float)((blocks + 255) / 256 * ((units + ks - 1) / ks)) * k.unit;
-            const float us = sqrtf(work * work + hbm * hbm) + (ks == 1 ? 0.f : 1.6f + (float)part / 2.3e6f);
-            if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, k.deep, ks};
+            if (ks > 1 && part > kSplitBudget / 2) break;
+            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks, units_of = (units + ks - 1) / ks;
+            auto round = [&](int of) {  // a round of `of` blocks
+                const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), bytes = 0.6f + hbm * (float)of / (float)blocks;
+                return sqrtf(work * work + bytes * bytes);
+            };
+            const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 1.6f + (float)part / 2.8e6f);
+            if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, true, ks};
         }
     return cut;
 }
@@ -1838,23 +1835,30 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
         if constexpr (FMT == MI355_W_Q4) {
             if (sh.bm == 48) return launch_deep<EPI, PAIR, FMT, 4, 48, FUSE>(p, s);
         }
+        if constexpr (FMT == MI355_W_BF16) {
+            if (sh.bm == 96) return launch_deep<EPI, PAIR, FMT, 4, 96, FUSE>(p, s);
+            if (sh.bm == kBM) return launch_deep<EPI, PAIR, FMT, 4, kBM, FUSE>(p, s);
+        }
         return launch_deep<EPI, PAIR, FMT, 4, 64, FUSE>(p, s);
     }
-    if constexpr (FMT == MI355_W_BF16) {
-        if (sh.bm == 64 && !sh.deep) return launch_gemm_w<EPI, PAIR, FMT, 8, 64, 0, FUSE>(p, s);
-    }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 8, 64, FUSE>(p, s);
-    if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
-    return launch_gemm_w<EPI, PAIR, FMT, 8, kBM, 0, FUSE>(p, s);
+    if constexpr (FMT == MI355_W_BF16) {
+        if (sh.bm == 192) return launch_deep<EPI, PAIR, FMT, 8, 192, FUSE>(p, s);
+        if (sh.bm == 256) return launch_deep<EPI, PAIR, FMT, 8, 256, FUSE>(p, s);
+        return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
+    } else {
+        if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
+        return launch_gemm_w<EPI, PAIR, 8, kBM, 0, FUSE>(p, s);
+    }
 }
 // grouped scales.  Groups of 32 or 64 columns: blocks of 64 tokens x 4 waves (the second accumulator set costs the registers of more tokens or waves).
 template <int EPI, bool PAIR>
 int launch_gemm_subgroups(const GemmParams& p, hipStream_t s) {
     const int per_block8 = PAIR ? 8 * kTPW / 2 : 8 * kTPW;
     const int blocks8 = ((p.n_tiles + per_block8 - 1) / per_block8) * ((p.M + 63) / 64);
-    if (p.ksplit > 1 || blocks8 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 4, 64, 2>(p, s);
-    if (blocks8 * 4 >= 128) return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 2, 64, 2>(p, s);
-    return launch_gemm_w<EPI, PAIR, MI355_W_Q4, 1, 64, 2>(p, s);
+    if (p.ksplit > 1 || blocks8 >= 128) return launch_gemm_w<EPI, PAIR, 4, 64, 2>(p, s);
+    if (blocks8 * 4 >= 128) return launch_gemm_w<EPI, PAIR, 2, 64, 2>(p, s);
+    return launch_gemm_w<EPI, PAIR, 1, 64, 2>(p, s);
 }
 template <int EPI, bool PAIR>
 int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {

@@ -79,6 +79,49 @@ def test_int4_sums_beside_a_large_activation(dev, M, N, K, run):
     assert (got - ref).square().mean().sqrt() <= 1.06 * (4 * run * 5 / 12) ** 0.5 * last_bit
 
 
+@pytest.mark.parametrize("M,N,K,pair", [
+    (512, 4096, 1664, 0), (128, 6160, 640, 0), (449, 4112, 1664, 0), (1281, 6160, 640, 0), (128, 4096, 128, 0), (193, 12288, 2176, 0), (500, 6160, 640, 0),
+    (320, 12288, 2176, 0), (257, 12288, 1664, 0), (512, 12288, 640, 0), (1025, 6160, 256, 0), (769, 12288, 1664, 0), (1281, 8200, 640, 0), (1025, 12288, 2048, 0),
+    (512, 1000, 2176, 1), (193, 4112, 1664, 1), (449, 12288, 2048, 1), (320, 6160, 2048, 1), (641, 4112, 384, 1), (1281, 6160, 2176, 1), (641, 8200, 1664, 1),
+])
+def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
+    """Blocks of 64 / 96 / 128 tokens x 4 waves and 64 / 128 / 192 / 256 x 8 (in this order above, pairs behind), a few tokens or rows more than whole blocks, rounds of units that end
+    early, row blocks that share an XCD and such that are cut between two.  Bounds: as in test_tiled_product_against_64_bits."""
+    g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    mats = [(torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16) for _ in range(1 + pair)]
+    stream = ops.repack_bf16(mats[0], mats[1] if pair else None, 1 + pair)
+    prods = [x.double() @ m.double().T for m in mats]
+    if pair:
+        ref = torch.nn.functional.silu(prods[0]) * prods[1]
+        got = ops.linear_gemm(x, stream, 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, fmt=nat.W_BF16).double()
+        assert (got - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 2e-3 * ref.square().mean().sqrt()
+        return
+    base = torch.randn((M, N), generator=g, device=dev)
+    ref = prods[0] + base.double()
+    got = ops.linear_gemm(x, stream, 1, N, K, epi=nat.EPI_ACCUM, out=base.clone(), fmt=nat.W_BF16).double()
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
+@pytest.mark.parametrize("T", [300, 777, 1300])
+def test_fused_prompt_chain_of_bf16_layers_at_7b_width(dev, monkeypatch, T):
+    """The chain's shares and rotations in blocks of 64 to 256 tokens.  0.02 of the logits' spread as in test_runs_of_shares_in_the_fused_prompt_chain."""
+    cfg = LLaMAConfig(block_size=1304, n_layer=2, n_head=32, n_embd=4096, vocab_size=512)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode=None, device="cuda", dtype=torch.bfloat16))
+    model.eval()
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
+        model.reset_cache()
+        with torch.no_grad():
+            out.append(model(idx.view(1, -1), 1304, torch.arange(T, device=dev))[0].float())
+    assert not torch.equal(*out)  # (the chain was on)
+    assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
+
+
 @pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K,cols", [(1, 16, 256, 128), (16, 144, 2176, 128), (17, 4096, 1280, 256), (33, 12288, 512, 128), (64, 128, 11008, 512), (65, 4096, 4096, 128),
                                         (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128)])
