@@ -1694,10 +1694,9 @@ GemmForce gemm_force() {
     }();
     return f;
 }
-bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (the kernels of launch_gemm())
-    if (bf16) return c.deep && (c.waves == 4 ? c.bm == 16 || c.bm == 32 || c.bm == 64 || c.bm == 96 || c.bm == 128 : c.waves == 8 && (c.bm == 64 || c.bm == 128 || c.bm == 192 || c.bm == 256));
-    if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 48 || c.bm == 64);
-    return c.waves == 8 && (c.bm == kBM || (c.bm == 64 && c.deep));
+bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (what a sweep may force of the kernels of launch_gemm(); the other blocks of BF16 streams are the estimate's)
+    if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
+    return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
 }
 // blocks of `waves` waves and `bm` tokens
 int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
@@ -1741,44 +1740,54 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
 // 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13); where those blocks are more than the CUs, blocks of 8 (48 tokens of the N = 17920 pair, K = 6656: 104 / 95 us with 4 / 8 waves).
 // Longer: 192 to 256 blocks of 128 tokens x 256 rows, one round of the chip, take those (3-5 % less than what the estimate takes).  Else what an estimate takes for the
 // fastest: the rounds of the chip one behind the other, each the busiest CU's units (`unit` us when it is alone, `crowd` more when every CU has a block, whatever of the
-// block is padding) and its share of the bytes from HBM at once; slices cost a launch, and their sums' way to memory and back.  Blocks of 192 and 256 tokens x 256 rows ask
+// block is padding) and its share of the bytes at once; slices cost a launch, and their sums' way to memory and back.  Blocks of 192 and 256 tokens x 256 rows ask
 // for 75 and 64 KB per 8.4 MFLOP instead of the 96 of 128 x 256, and give the rounds more sizes to fit: 2048 tokens, N = 16512, K = 4096, 4.1 rounds of 128 tokens 278 us, 2.8 of
-// 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  Fitted to 15 000
-// launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are) within 8 % rms; its choice takes 0.8 % longer than the
-// fastest on average, 2.4 % at the 90th percentile.
+// 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  The constants
+// are those whose choice is best over 19 500 launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are): 1.7 % behind the
+// fastest of them on average, 6 % at the 90th percentile.
 GemmCut bf16_cut(int M, int N, int K, bool pair) {
-    const int units = (K + 127) / 128;
-    if (M <= 64) {
-        const int few = gemm_blocks(M, N, pair, 4, 64);
-        if (few > 256) return {8, 64, true, 1};
-        GemmCut cut = {4, short_block(M, true), true, 1};
+    const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
+    GemmCut cut = {4, short_block(M, true), true, 1};
+    if (M <= 64 && few <= 256) {
         while (cut.ksplit < kMaxSplit && few * cut.ksplit < 192 && few * (cut.ksplit + 1) <= 256 && units >= 4 * (cut.ksplit + 1) &&
                gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
             ++cut.ksplit;
         return cut;
     }
-    if (const int wide = gemm_blocks(M, N, pair, 8, kBM); wide >= 192 && wide <= 256) return {8, kBM, true, 1};
+    if (M > 64 && wide >= 192 && wide <= 256) return {8, kBM, true, 1};
     struct Kind {
         int waves, bm;
         float start, unit, crowd;
     };
-    constexpr Kind kinds[] = {{4, 64, 5.3f, 0.50f, 0.16f},  {4, 96, 5.1f, 0.68f, 0.12f},  {4, kBM, 5.0f, 0.78f, 0.22f}, {8, 64, 6.5f, 0.97f, 0.18f},
-                              {8, kBM, 6.6f, 1.29f, 0.35f}, {8, 192, 8.3f, 1.44f, 0.76f}, {8, 256, 8.8f, 2.23f, 0.86f}};
-    const float hbm = (2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N) / 7.83e6f;
-    GemmCut cut = {4, 64, true, 1};
+    // (up to 64 tokens, more blocks than CUs: the weights bound them)
+    const Kind few_tokens[] = {{4, cut.bm, cut.bm == 16 ? 0.9f : cut.bm == 32 ? 1.3f : 3.0f, cut.bm == 16 ? 0.67f : cut.bm == 32 ? 0.71f : 0.75f, 0.f}, {8, 64, 3.4f, 1.23f, 0.f}};
+    static constexpr Kind kinds[] = {{4, 64, 1.8f, 0.539f, 0.147f},   {4, 96, 4.2f, 0.507f, 0.237f},   {4, kBM, 3.1f, 0.746f, 0.237f}, {8, 64, 7.8f, 0.766f, 0.219f},
+                                     {8, kBM, 6.4f, 0.988f, 0.321f}, {8, 192, 9.7f, 1.274f, 0.424f}, {8, 256, 4.2f, 1.52f, 0.871f}};
+    const float bytes = 2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N;
     float best = 0.f;
-    for (const Kind& k : kinds)
-        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || units >= 4 * ks); ++ks) {
-            const size_t part = gemm_part_bytes(M, N, pair, ks);
-            if (ks > 1 && part > kSplitBudget / 2) break;
-            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks, units_of = (units + ks - 1) / ks;
-            auto round = [&](int of) {  // a round of `of` blocks
-                const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), bytes = 0.6f + hbm * (float)of / (float)blocks;
-                return sqrtf(work * work + bytes * bytes);
-            };
-            const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 1.6f + (float)part / 2.8e6f);
+    auto estimate = [&](const Kind& k, int ks) {
+        const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks, units_of = (units + ks - 1) / ks;
+        const float part = ks == 1 ? 0.f : (float)gemm_part_bytes(M, N, pair, ks);
+        if (M <= 64) {
+            const float work = k.start + (float)((blocks + 255) / 256 * units_of) * k.unit, hbm = 4.3f + bytes / 6.6e6f;
+            return sqrtf(work * work + hbm * hbm) + (ks == 1 ? 0.f : 1.6f + part / 2.3e6f);
+        }
+        auto round = [&](int of) {  // a round of `of` blocks
+            const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), hbm = 0.16f + bytes / 23.8e6f * (float)of / (float)blocks;
+            return sqrtf(work * work + hbm * hbm);
+        };
+        return k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 0.8f + part / 3.38e6f);
+    };
+    auto consider = [&](const Kind& k) {
+        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget * 3 / 4)); ++ks) {
+            const float us = estimate(k, ks);
             if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, true, ks};
         }
+    };
+    if (M <= 64)
+        for (const Kind& k : few_tokens) consider(k);
+    else
+        for (const Kind& k : kinds) consider(k);
     return cut;
 }
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16) {

@@ -12,7 +12,7 @@
 //                        themselves, f16: xo (rows) and so = f16(CB * SCB / 127) (weights; workgroups behind the rows');
 //   3. i8_gemm_kernel    — the int8 weight stream of int8.hip ([tile][unit][r][piece e][lane][16 x int8], one piece = one
 //                        MFMA A operand) against CA through LDS (128 tokens x 128 k, XOR-swizzled), two row tiles per
-//                        wave, 8 waves; then so x xo in the same loop on the f16 MFMA (of a launch cut along K: a slice of its own); epilogue with the arithmetic
+//                        wave, 8 or 4 waves; then so x xo in the same loop on the f16 MFMA (of a launch cut along K: a slice of its own); epilogue with the arithmetic
 //                        of int8.hip, rounding for rounding:
 //                            d = f16((acc * 6.200012e-05 * absmax[m]) * SCB[n]);   o = sum over outlier columns k (ascending) of
 //                            xh[m, k] * f16(CB[n, k] * SCB[n] / 127);   y = f16(d + f16(o))   (the last step only with outliers)
@@ -27,16 +27,15 @@ namespace {
 
 constexpr int kBM = 128;      // tokens per block
 constexpr int kTPW = 2;       // 16-row tile slots per wave
-constexpr int kWaves = 8;
-constexpr int kSlots = kWaves * kTPW;
-constexpr int kThreads = 64 * kWaves;
 constexpr int kXTile = kBM * 128;        // bytes of one activation tile (int8)
 constexpr int kOutChunk = 64;            // outlier columns staged per pass of the epilogue
 constexpr int kDepth = 4;                // units of operands in LDS and registers
 constexpr int kLdsMain = kDepth * kXTile;
 constexpr int kSoLd = kOutChunk + 8;     // row pitch of the staged outlier weights (halves): 144 B, so that 16 rows written side by side fall into 16 banks
-constexpr int kLdsEpi = (kBM * kOutChunk + kSlots * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [256 rows][kSoLd]
-constexpr int kLds = kLdsMain > kLdsEpi ? kLdsMain : kLdsEpi;
+template <int kWaves>
+constexpr int kLdsEpi = (kBM * kOutChunk + kWaves * kTPW * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [rows][kSoLd]
+template <int kWaves>
+constexpr int kLds = kLdsMain > kLdsEpi<kWaves> ? kLdsMain : kLdsEpi<kWaves>;
 
 __device__ __forceinline__ float f16r(float v) { return f16_to_f32(f32_to_f16(v)); }
 // the same for a value that must be an f32 PRODUCT rounded to f32 first (MatMul8bitLt's dequantisation multiplies in f32 and converts): hipcc
@@ -81,7 +80,7 @@ struct I8GemmParams {
 };
 constexpr size_t kSplitBudget = (size_t)32 << 20;             // bytes of the int32 partial tiles of all K-slices,
 constexpr size_t kPartBytes = kSplitBudget + kSplitBudget / 2;  // next to the f32 tiles of the outlier columns (2 slices at least)
-constexpr size_t kOutlierBudget = (size_t)32 << 20;  // bytes of `so`
+constexpr size_t kOutlierBudget = (size_t)128 << 20;  // bytes of `so`
 __device__ __forceinline__ int compact_ld(int n_out) { return (n_out + 63) & ~63; }
 __device__ __forceinline__ bool is_compact(int n_out, int n_tiles, int R, int M) {
     return n_out > 0 && (size_t)n_tiles * R * 16 * compact_ld(n_out) * 2 <= kOutlierBudget && (size_t)M * compact_ld(n_out) * 2 < 0x7fffffffu;
@@ -290,8 +289,10 @@ __global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int
 
 // ---- 3. the product
 // MODE 0: product + epilogue; 1: product of one K-slice -> partial tiles; 2: sum of the partial tiles + epilogue
-template <int EPI, bool PAIR, int MODE>
-__global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p) {
+template <int EPI, bool PAIR, int MODE, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmParams p) {
+    static_assert(MODE != 2 || kWaves == 8, "a wave per token tile");
+    constexpr int kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -308,7 +309,8 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
     constexpr int kTT = MODE == 2 ? 1 : 8;                                     // token tiles a wave finishes, from tt0 on
     const int tt0 = MODE == 2 ? wave : 0;
     const int wslot = MODE == 2 ? ks : wave;                                   // slot group of this wave's row tiles
-    const int mb = L / p.n_blocks, nb = L - mb * p.n_blocks;
+    // row block major: an XCD runs every token block of a few row blocks side by side, so their weights cross to its L2 once
+    const int m_blocks = p.total_blocks / p.n_blocks, nb = L / m_blocks, mb = L - nb * m_blocks;
     const int m0 = mb * kBM;
     const int u_lo = MODE == 1 ? (int)((int64_t)ks * p.units / p.ksplit) : 0;
     const int u_hi = MODE == 1 ? (int)((int64_t)(ks + 1) * p.units / p.ksplit) : p.units;
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         }
         const unsigned w_lane = F16 ? (unsigned)(c * ldb + g * 16) : lane_off;
         u32x4 wr[kDepth][kTPW][2];
-        auto request = [&](int i, int u, int slot) {
+        auto request = [&](int i, int u, int slot) __attribute__((always_inline)) {
             const bool in = u < hi;
             if (i < kXI) {
                 const unsigned off = in && xoff[i < kXI ? i : 0] != 0xFFFFFFF0u ? xoff[i < kXI ? i : 0] + (unsigned)u * 128u : 0xFFFFFFF0u;
@@ -373,7 +375,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
             for (int i = 0; i < kUnit; ++i) request(i, lo + d, d);
             __builtin_amdgcn_sched_barrier(0);
         }
-        auto products = [&](int slot, int ahead, int ahead_slot) {
+        auto products = [&](int slot, int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
             const char* xs = smem + slot * kXTile;
             constexpr int kFrags = 16, kPipe = 4;  // fragment f = e * 8 + tt
             auto bread = [&](int f) {
@@ -398,19 +400,33 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                 }
                 if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
-                if (f < kUnit) {
-                    request(f, ahead, ahead_slot);
+                constexpr int kEvery = kFrags / kUnit;  // (spread over the unit: csrc/gemm.hip)
+                if (more && f % kEvery == 0 && f / kEvery < kUnit) {
+                    request(f / kEvery, ahead, ahead_slot);
                     __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        for (int u = lo; u < hi; u += kDepth) {
-#pragma unroll
-            for (int d = 0; d < kDepth; ++d) {
-                if (d > 0 && u + d >= hi) break;
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kDepth - 2) * kUnit) : "memory");
-                products(d, u + d + kDepth - 1, (d + kDepth - 1) % kDepth);
+        // (the last, shorter round stands behind the loop and requests nothing: with a way out between the units hipcc waited for every request once a round)
+        auto unit = [&](auto slot, int u, auto more) __attribute__((always_inline)) {
+            constexpr int d = slot, kNewer = more ? (kDepth - 2) * kUnit : (kDepth - 2 - d) * kUnit;
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kNewer) : "memory");
+            products(d, u + kDepth - 1, (d + kDepth - 1) % kDepth, more);
+        };
+        using std::integral_constant;
+        int u = lo;
+        for (; u + kDepth <= hi; u += kDepth) {
+            unit(integral_constant<int, 0>{}, u, std::true_type{});
+            unit(integral_constant<int, 1>{}, u + 1, std::true_type{});
+            unit(integral_constant<int, 2>{}, u + 2, std::true_type{});
+            unit(integral_constant<int, 3>{}, u + 3, std::true_type{});
+        }
+        if (u < hi) {
+            unit(integral_constant<int, 0>{}, u, std::false_type{});
+            if (u + 1 < hi) {
+                unit(integral_constant<int, 1>{}, u + 1, std::false_type{});
+                if (u + 2 < hi) unit(integral_constant<int, 2>{}, u + 2, std::false_type{});
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests past the end wrote zeros: none may land in what follows)
@@ -418,12 +434,15 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
     };
     const int n_out = MODE == 1 && ks < p.ksplit ? 0 : p.olist[0];
     const bool compact = is_compact(n_out, p.n_tiles, R, p.M);
-    [[maybe_unused]] f32x4 o[kTPW][kTT];  // the compact outlier columns' share
-    auto outliers = [&]() {
+    f32x4 o[kTPW][kTT];  // the outlier columns' share
+    auto no_outliers = [&]() {
 #pragma unroll
         for (int t = 0; t < kTPW; ++t)
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) o[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto outliers = [&]() {
+        no_outliers();
         const int ld = compact_ld(n_out);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.so, 0, p.n_tiles * R * 16 * ld * 2, 0x00020000);
         const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void*)p.xo, 0, p.M * ld * 2, 0x00020000);
@@ -493,28 +512,10 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         const int m = m0 + (tt0 + tt) * 16 + c;
         sa[tt] = p.sca[m < p.M ? m : 0];
     }
-    float d[kTPW][kTT][4];
-    auto dequant = [&]() {
-#pragma unroll
-        for (int tt = 0; tt < kTT; ++tt)
-#pragma unroll
-            for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r_of_f32((((float)acc[t][tt][r] * 6.200012e-05f) * sa[tt]) * scb[t][r]);
-    };
     typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
     if (compact) {
-        // mixed-precision decomposition over the compact columns, ascending k
         if constexpr (MODE == 0) outliers();
-        dequant();
-#pragma unroll
-        for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-            for (int tt = 0; tt < kTT; ++tt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r(d[t][tt][r] + f16r(o[t][tt][r]));
     } else if (n_out > 0) {  // (too many for their region)
-        dequant();
         // mixed-precision decomposition: the outlier columns in f16, ascending k, kOutChunk columns per pass through LDS
         f16_t* xo = (f16_t*)smem;                     // [128 tokens][kOutChunk]
         f16_t* so = xo + kBM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
@@ -524,11 +525,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
         // ascending k — bitsandbytes' own f16 GEMM promises no order either, and the tests allow the one f16 ulp this can move.  The scalar
         // loop it replaces (64 FMAs per lane and outlier column) took 1.4 ms per attn.c_proj / mlp.c_proj launch at T = 2048, where ~10 % of
         // the columns of a 2048-token call hold an outlier: profiles/r06_prefill_int8_outliers.txt.)
-        f32x4 o[kTPW][kTT];
-#pragma unroll
-        for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-            for (int tt = 0; tt < kTT; ++tt) o[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        no_outliers();
         for (int base = 0; base < n_out; base += kOutChunk) {
             const int nc = n_out - base < kOutChunk ? n_out - base : kOutChunk;
             __syncthreads();  // (the main loop / the previous pass is done with the LDS)
@@ -546,15 +543,15 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                 xo[idx] = (m < p.M && col_ok) ? p.xh[(int64_t)m * p.Kp + k] : (f16_t)0;
             }
             // weights: ROW fastest — 16 lanes = the 16 rows of a tile at one outlier column (16 B apart in the stream: two cache lines),
-            // four columns per wave (the column-fastest order touched 64 lines per wave load); a thread sees two columns, oc and oc + 32
-            static_assert(kThreads == 512 && kOutChunk == 64, "element e = j * 512 + thread: row e & 15, column (e >> 4) & 63, slot e >> 10 = j >> 1");
+            // four columns per wave (the column-fastest order touched 64 lines per wave load); a thread sees kCols columns, kStep apart
+            constexpr int kStep = kThreads / 16, kCols = kOutChunk / kStep;
             const int oc = threadIdx.x >> 4, row = threadIdx.x & 15;
-            const bool c_ok[2] = {oc < nc, oc + 32 < nc};
-            const int k2[2] = {c_ok[0] ? p.olist[1 + base + oc] : 0, c_ok[1] ? p.olist[1 + base + oc + 32] : 0};
-            const int j_lo = MODE == 2 ? 2 * ks * kTPW : 0, j_hi = MODE == 2 ? j_lo + 2 * kTPW : 2 * kSlots;  // MODE 2: the rows of slot group ks only
-#pragma unroll 8
-            for (int j = j_lo; j < j_hi; ++j) {
-                const int slot = j >> 1, h = j & 1;
+            int k2[kCols];
+#pragma unroll
+            for (int h = 0; h < kCols; ++h) k2[h] = oc + kStep * h < nc ? p.olist[1 + base + oc + kStep * h] : -1;
+            const int s_lo = MODE == 2 ? ks * kTPW : 0, s_hi = MODE == 2 ? s_lo + kTPW : kSlots;  // MODE 2: the rows of slot group ks only
+#pragma unroll 4
+            for (int slot = s_lo; slot < s_hi; ++slot) {
                 const int wv = slot / kTPW, t = slot - wv * kTPW;
                 int tl, r1;
                 if (PAIR) {
@@ -565,16 +562,19 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                     r1 = 0;
                 }
                 const int n = tl * 16 + row;
-                const int kk = h ? k2[1] : k2[0];
-                f16_t sub = 0;
-                if ((h ? c_ok[1] : c_ok[0]) && tl < p.n_tiles && n < p.N) {
-                    const int ku = kk >> 7, ke = (kk >> 6) & 1, kgg = (kk >> 4) & 3, kjj = kk & 15;
-                    const int64_t off = ((((int64_t)tl * p.units + ku) * R + r1) * 2 + ke) * 1024 + (kgg * 16 + row) * 16 + kjj;
-                    const float cb = (float)(int8_t)p.w[off];
-                    const float s = ((PAIR && r1 == 1) ? p.scb2 : p.scb)[n];
-                    sub = f32_to_f16(__fdiv_rn(cb * s, 127.0f));
+#pragma unroll
+                for (int h = 0; h < kCols; ++h) {
+                    const int kk = k2[h];
+                    f16_t sub = 0;
+                    if (kk >= 0 && tl < p.n_tiles && n < p.N) {
+                        const int ku = kk >> 7, ke = (kk >> 6) & 1, kgg = (kk >> 4) & 3, kjj = kk & 15;
+                        const int64_t off = ((((int64_t)tl * p.units + ku) * R + r1) * 2 + ke) * 1024 + (kgg * 16 + row) * 16 + kjj;
+                        const float cb = (float)(int8_t)p.w[off];
+                        const float s = ((PAIR && r1 == 1) ? p.scb2 : p.scb)[n];
+                        sub = f32_to_f16(__fdiv_rn(cb * s, 127.0f));
+                    }
+                    so[(slot * 16 + row) * kSoLd + oc + kStep * h] = sub;
                 }
-                so[(slot * 16 + row) * kSoLd + oc + 32 * h] = sub;
             }
             __syncthreads();
 #pragma unroll
@@ -591,15 +591,17 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                 }
             }
         }
-#pragma unroll
-        for (int t = 0; t < kTPW; ++t)
-#pragma unroll
-            for (int tt = 0; tt < kTT; ++tt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) d[t][tt][r] = f16r(d[t][tt][r] + f16r(o[t][tt][r]));
-    } else {
-        dequant();
     }
+    // the result at row r of tile t, token tile tt; with outliers the mixed-precision decomposition over them, ascending k, comes on top
+    auto value = [&](int t, int tt) {
+        f32x4 d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = f16r_of_f32((((float)acc[t][tt][r] * 6.200012e-05f) * sa[tt]) * scb[t][r]);
+        if (n_out > 0)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) d[r] = f16r(d[r] + f16r(o[t][tt][r]));
+        return d;
+    };
     // four consecutive output columns per lane and tile: one 16-B (f32) / 8-B (bf16, f16) access when the row allows it
     const bool vec = (p.N & 3) == 0 && (p.ldy & 3) == 0 && ((uintptr_t)p.y & 15) == 0;
     constexpr int kOld = kTT < 2 ? kTT : 2;
@@ -624,9 +626,10 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
             for (int t = 0; t < kTPW; t += 2) {
                 const int n = tile[t] * 16 + 4 * g;
                 if (tile[t] >= p.n_tiles || n >= p.N) continue;
+                const f32x4 a = value(t, tt), b = value(t + 1, tt);
                 float v[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = swiglu_f32(d[t][tt][r], d[t + 1][tt][r]);
+                for (int r = 0; r < 4; ++r) v[r] = swiglu_f32(a[r], b[r]);
                 if (vec && p.y_dtype == MI355_BF16) {
                     u32x2 pk;
                     pk[0] = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
@@ -644,12 +647,13 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
                 const int n = tile[t] * 16 + 4 * g;
                 if (tile[t] >= p.n_tiles || n >= p.N) continue;
                 const int64_t yi = (int64_t)m * p.ldy + n;
+                const f32x4 d = value(t, tt);
                 if (vec && p.y_dtype == MI355_F32) {
-                    f32x4 o = {d[t][tt][0], d[t][tt][1], d[t][tt][2], d[t][tt][3]};
+                    f32x4 o = d;
                     if constexpr (EPI == MI355_EPI_ACCUM) o += old[t][tt % kOld];
                     *(f32x4*)((float*)p.y + yi) = o;
                 } else if (vec && p.y_dtype == MI355_BF16) {
-                    float o[4] = {d[t][tt][0], d[t][tt][1], d[t][tt][2], d[t][tt][3]};
+                    float o[4] = {d[0], d[1], d[2], d[3]};
                     if constexpr (EPI == MI355_EPI_ACCUM) {
                         const u32x2 old = *(const u32x2*)((const bf16_t*)p.y + yi);
                         o[0] += __uint_as_float(old[0] << 16);
@@ -665,7 +669,7 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         if (n + r >= p.N) continue;
-                        float v = d[t][tt][r];
+                        float v = d[r];
                         if constexpr (EPI == MI355_EPI_ACCUM) v += ld_as_f32(p.y, yi + r, p.y_dtype);
                         st_from_f32(p.y, yi + r, p.y_dtype, v);
                     }
@@ -675,29 +679,55 @@ __global__ __launch_bounds__(kThreads) void i8_gemm_kernel(const I8GemmParams p)
     }
 }
 
-template <int EPI, bool PAIR, int MODE>
+template <int EPI, bool PAIR, int MODE, int kWaves>
 int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
     static hipError_t attr_err =
-        hipFuncSetAttribute((const void*)i8_gemm_kernel<EPI, PAIR, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        hipFuncSetAttribute((const void*)i8_gemm_kernel<EPI, PAIR, MODE, kWaves>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds<kWaves>);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(i8_gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
     I8GemmParams r = q;
-    r.per_xcd = (q.total_blocks * (MODE == 1 ? q.ksplit + 1 : MODE == 2 ? 8 : 1) + 7) / 8;
-    hipLaunchKernelGGL((i8_gemm_kernel<EPI, PAIR, MODE>), dim3(8 * r.per_xcd), dim3(kThreads), kLds, s, r);
+    r.n_blocks = (q.n_tiles + kWaves * kTPW / (PAIR ? 2 : 1) - 1) / (kWaves * kTPW / (PAIR ? 2 : 1));
+    r.total_blocks = r.n_blocks * ((q.M + kBM - 1) / kBM);
+    r.per_xcd = (r.total_blocks * (MODE == 1 ? q.ksplit + 1 : MODE == 2 ? 8 : 1) + 7) / 8;
+    hipLaunchKernelGGL((i8_gemm_kernel<EPI, PAIR, MODE, kWaves>), dim3(8 * r.per_xcd), dim3(64 * kWaves), kLds<kWaves>, s, r);
     MI355_LAUNCH_CHECK();
     return 0;
 }
+// How a launch is cut: blocks of 128 tokens x 256 rows (8 waves, a CU each) or x 128 (4 waves, two to a CU), and K-slices, which are a sum and its launch more; what an
+// estimate takes for the fastest, as for the bf16 stream (csrc/gemm.hip: bf16_cut()).  Its constants are those whose choice is best over 1700 launches (18 products
+// of 2048 to 32000 rows, 33 to 2048 tokens, weights not in any cache): 1.1 % behind the fastest of them on average, 3 % at the 90th percentile.  Blocks of 8 waves throughout and
+// slices for launches of less than 96 of them: N = K = 4096, 128 tokens 31.0 us (now 28.3), 512 44.8 (34.3); N = 12288, 128 tokens 46.5 (37.6)
+struct I8Cut {
+    int waves, ksplit;
+};
+I8Cut i8_cut(int M, int N, int units, bool pair) {
+    struct Kind {
+        int waves;
+        float start, unit, crowd;
+    };
+    static constexpr Kind kinds[] = {{4, 2.9f, 0.513f, 0.036f}, {8, 2.9f, 0.626f, 0.381f}};
+    const size_t part = (size_t)M * N * (pair ? 2 : 1) * 4;  // bytes of one slice's sums
+    I8Cut cut = {8, 1};
+    float best = 0.f;
+    for (const Kind& k : kinds)
+        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && part * ks <= kSplitBudget)); ++ks) {
+            const int rows = 16 * k.waves * kTPW / (pair ? 2 : 1), blocks = (N + rows - 1) / rows * ((M + kBM - 1) / kBM) * ks, units_of = (units + ks - 1) / ks;
+            auto round = [&](int of) {
+                const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), hbm = 128.f * units * N * (pair ? 2 : 1) / 1.63e6f * (float)of / (float)blocks;
+                return sqrtf(work * work + hbm * hbm);
+            };
+            const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 3.1f + (float)(part * ks) / 1.61e6f);
+            if (best == 0.f || us < best) best = us, cut = {k.waves, ks};
+        }
+    return cut;
+}
 template <int EPI, bool PAIR>
-int launch_i8_gemm(const I8GemmParams& p, hipStream_t s) {
-    const int per_block = PAIR ? kSlots / 2 : kSlots;
-    I8GemmParams q = p;
-    q.n_blocks = (p.n_tiles + per_block - 1) / per_block;
-    q.total_blocks = q.n_blocks * ((p.M + kBM - 1) / kBM);
-    if (q.ksplit <= 1) return launch_i8_mode<EPI, PAIR, 0>(q, s);
-    if (int rc = launch_i8_mode<EPI, PAIR, 1>(q, s)) return rc;
-    return launch_i8_mode<EPI, PAIR, 2>(q, s);
+int launch_i8_gemm(const I8GemmParams& p, int waves, hipStream_t s) {
+    if (p.ksplit <= 1) return waves == 4 ? launch_i8_mode<EPI, PAIR, 0, 4>(p, s) : launch_i8_mode<EPI, PAIR, 0, 8>(p, s);
+    if (int rc = waves == 4 ? launch_i8_mode<EPI, PAIR, 1, 4>(p, s) : launch_i8_mode<EPI, PAIR, 1, 8>(p, s)) return rc;
+    return launch_i8_mode<EPI, PAIR, 2, 8>(p, s);
 }
 
 size_t pad16(size_t v) { return (v + 15) & ~(size_t)15; }
@@ -747,16 +777,9 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     f16_t* xo = (f16_t*)ws;
     ws += pad16((size_t)a->M * kp * 2);
     f16_t* so = (f16_t*)ws;
-    // split-K: launches of fewer than 96 blocks are cut into up to 8 K-slices (as many as fit the partial buffer)
-    int ksplit = 1;
+    const I8Cut cut = i8_cut(a->M, a->N, units, swiglu);
+    const int ksplit = cut.ksplit;
     const int64_t ldp = (int64_t)a->N * (swiglu ? 2 : 1);
-    {
-        const int rows_per_block = swiglu ? 16 * kSlots / 2 : 16 * kSlots;
-        const int blocks = ((a->N + rows_per_block - 1) / rows_per_block) * ((a->M + kBM - 1) / kBM);
-        while (ksplit < kMaxSplit && blocks * ksplit < 96 && units >= 8 * ksplit &&
-               (size_t)2 * ksplit * a->M * ldp * 4 <= kSplitBudget)
-            ksplit *= 2;
-    }
     // (a kernel, not hipMemsetAsync: a caller may capture this launch, and memset nodes have replayed wrongly)
     hipLaunchKernelGGL(i8_clear_mask_kernel, dim3((kp / 32 + 255) / 256), dim3(256), 0, s, mask, kp / 32);
     MI355_LAUNCH_CHECK();
@@ -799,7 +822,7 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     p.so = so;
     hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), (kp / 32 < kMaskWords ? kp / 32 : kMaskWords) * kQuantLds, s, mask, ca, olist, p, a->R);
     MI355_LAUNCH_CHECK();
-    if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, s);
-    if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, s);
-    return launch_i8_gemm<MI355_EPI_STORE, false>(p, s);
+    if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, cut.waves, s);
+    if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, cut.waves, s);
+    return launch_i8_gemm<MI355_EPI_STORE, false>(p, cut.waves, s);
 }
