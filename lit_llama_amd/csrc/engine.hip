@@ -80,16 +80,20 @@ int run_linear_rows(const mi355_model* m, const mi355_weight& w, const void* x, 
                     const float* attn_partials);
 
 // The wide-GEMM chain of one prompt pass with the staging passes and the K / V cache write folded into the producers'
-// epilogues (gemm_fuse.h).  Decided once per mi355_forward call: every layer linear on the wide path over per-row scales,
+// epilogues (gemm_fuse.h).  Decided once per mi355_forward call: every layer linear on the wide path over per-row scales or groups of whole units,
 // widths of whole 128-column units, a bf16 cache at head size 128, no adapter prefix, one GPU.
+bool in_groups(const mi355_weight& w) { return w.fmt == MI355_W_Q4 && w.group_cols > 0 && w.group_cols < w.K; }
 struct FuseEdge {      // partial sums ("shares") a producer leaves per row, [share][T] f32
     float* ss;         // sums of squares of the f32 residual row (residual epilogues only)
     float* sx;         // operand sums
     struct Cut {
         int n, ppu;    // shares, shares per 128-column unit (mi355_linear_gemm_plan of the producer's launch)
-    } of[2];           // by the producer's stream: int4, bf16
+    } of[3];           // by the producer's stream: int4, bf16, int4 with grouped scales
     int n, ppu;        // what the last producer has left
-    void left_by(const mi355_weight& w) { n = of[w.fmt == MI355_W_BF16].n, ppu = of[w.fmt == MI355_W_BF16].ppu; }
+    void left_by(const mi355_weight& w) {
+        const Cut& cut = of[w.fmt == MI355_W_BF16 ? 1 : in_groups(w) ? 2 : 0];
+        n = cut.n, ppu = cut.ppu;
+    }
 };
 struct FuseCtx {
     bool on;
@@ -99,6 +103,10 @@ struct FuseCtx {
     FuseEdge fc;       // SwiGLU output -> mlp.c_proj
     FuseEdge att;      // attention output -> attn.c_proj (one share per head)
     bool have_x;       // xb and the mproj edge hold the input of the next c_attn
+    // tables of grouped scales: those of products [tab_first, tab_first + tab_n) (4 layer + segment) lie at tab[0 ..], in the room at tab_at
+    char* tab_at;
+    int tab_first, tab_n;
+    uint32_t* tab[MI355_TABLE_PRODUCTS];
 };
 
 void fill_linear_args(mi355_linear_args& a, const mi355_model* m, const mi355_weight& w, const void* x, int x_dtype, int M,
@@ -158,9 +166,12 @@ bool short_chunk_fits(const mi355_model* m, const mi355_weight& w, int M, int ep
     return w.R == (epi == MI355_EPI_SWIGLU ? 2 : 1) && (uintptr_t)m->gemm_ws % 16 == 0 && (size_t)m->gemm_ws_bytes >= mi355_linear_gemm_workspace_bytes(M, w.K) &&
            (!scale_groups || mi355_linear_gemm_tables_fit(M, w.N, w.K, w.R, w.group_cols));
 }
-bool wide_plain(const mi355_weight& w) {  // a linear the fused chain can run: int4 / bf16 stream, one scale per row
-    return (w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && (w.group_cols == 0 || w.group_cols >= w.K) && w.N % 4 == 0 &&
-           w.K % 128 == 0;
+// a linear the fused chain can run: int4 / bf16 stream, one scale per row or per group of whole units
+bool wide_plain(const mi355_weight& w) {
+    const bool groups = in_groups(w);
+    return (w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && w.N % 4 == 0 && w.K % 128 == 0 &&
+           (!groups || (w.group_cols >= 128 && (w.group_cols & (w.group_cols - 1)) == 0 && w.sz_dtype == MI355_BF16 &&
+                        mi355_linear_gemm_table_bytes(w.N, w.K, w.R, w.group_cols) <= mi355_linear_gemm_table_room()));
 }
 
 FuseCtx plan_fusion(const mi355_model* m, int T) {
@@ -175,8 +186,14 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
         (int64_t)m->S * 256 >= 0x7fffffffLL || m->n_head * m->hs != m->n_embd)
         return z;
     const int C = m->n_embd, H = m->n_hidden;
+    int groups = 0;  // columns of a group, wherever there are groups
     for (int l = 0; l < m->n_layer; ++l) {
         const mi355_layer& L = m->layers[l];
+        for (const mi355_weight* w : {&L.attn, &L.proj, &L.fc, &L.mproj}) {
+            if (!in_groups(*w)) continue;
+            if (groups == 0) groups = w->group_cols;
+            if (w->group_cols != groups || !mi355_linear_gemm_tables_fit(T, w->N, w->K, w->R, groups)) return z;
+        }
         if (L.adapter_len > 0 || !wide_plain(L.attn) || !wide_plain(L.proj) || !wide_plain(L.fc) || !wide_plain(L.mproj)) return z;
         if (L.attn.N != 3 * C || L.attn.K != C || L.proj.N != C || L.proj.K != C || L.fc.N != H || L.fc.K != C || L.fc.R != 2 ||
             L.mproj.N != C || L.mproj.K != H || L.kcache == nullptr || L.vcache == nullptr)
@@ -189,11 +206,14 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
     const size_t tail = mi355_linear_gemm_fuse_scratch_bytes();
     if ((size_t)m->gemm_ws_bytes < mi355_linear_gemm_workspace_bytes(T, kmax)) return z;
     float* cur = (float*)((char*)m->gemm_ws + (((size_t)m->gemm_ws_bytes - tail) & ~(size_t)15));
+    z.tab_at = (char*)cur - mi355_linear_gemm_table_room();
     float* const end = (float*)((char*)m->gemm_ws + (size_t)m->gemm_ws_bytes);
     auto edge = [&](FuseEdge& e, const mi355_weight& w, bool with_ss) {  // (the layers may differ in their formats)
         int ks;
         for (int b = 0; b < 2; ++b) mi355_linear_gemm_plan(T, w.N, w.K, w.R, b == 1, &ks, &e.of[b].n, &e.of[b].ppu);
-        const int n = e.of[0].n > e.of[1].n ? e.of[0].n : e.of[1].n;
+        if (groups != 0) mi355_linear_gemm_plan_grouped(T, w.N, w.K, w.R, groups, &ks, &e.of[2].n, &e.of[2].ppu);
+        int n = 0;
+        for (const FuseEdge::Cut& cut : e.of) n = cut.n > n ? cut.n : n;
         e.sx = cur;
         cur += (size_t)n * Ts;
         e.ss = with_ss ? cur : nullptr;
@@ -363,6 +383,32 @@ extern "C" int mi355_forward_segment(const mi355_model* m, int T, int layer, int
     return forward_segment_impl(m, T, layer, seg_begin, seg_end, stream, nullptr);
 }
 
+// The tables of a product over grouped scales, laid out with those of the products behind it, as many as there is room for: up to the first one of another kind, whose
+// K-slice sums may take the room
+static int group_tables_of(const mi355_model* m, int layer, int seg, hipStream_t s, FuseCtx* fz, const uint32_t** out) {
+    const int at = 4 * layer + seg;
+    if (at < fz->tab_first || at >= fz->tab_first + fz->tab_n) {
+        mi355_linear_args of[MI355_TABLE_PRODUCTS];
+        size_t room = mi355_linear_gemm_table_room();
+        char* to = fz->tab_at;
+        int n = 0;
+        for (; n < MI355_TABLE_PRODUCTS && at + n < 4 * m->n_layer; ++n) {
+            const mi355_layer& L = m->layers[(at + n) / 4];
+            const mi355_weight& w = *(const mi355_weight* const[]){&L.attn, &L.proj, &L.fc, &L.mproj}[(at + n) % 4];
+            const size_t bytes = in_groups(w) ? mi355_linear_gemm_table_bytes(w.N, w.K, w.R, w.group_cols) : 0;
+            if (bytes == 0 || bytes > room) break;
+            fill_linear_args(of[n], m, w, nullptr, MI355_BF16, 0, 0, nullptr, MI355_EPI_STORE, nullptr, MI355_F32, 0);
+            fz->tab[n] = (uint32_t*)to;
+            to += bytes;
+            room -= bytes;
+        }
+        if (int rc = mi355_linear_gemm_tables(of, fz->tab, n, s)) return rc;
+        fz->tab_first = at, fz->tab_n = n;
+    }
+    *out = fz->tab[at - fz->tab_first];
+    return 0;
+}
+
 // the fused chain of a prompt pass (FuseCtx above): one segment with its producer / consumer roles
 static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStream_t s, FuseCtx* fz) {
     const mi355_layer& L = m->layers[layer];
@@ -370,6 +416,10 @@ static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStr
     mi355_linear_args a;
     mi355_gemm_fuse f;
     memset(&f, 0, sizeof(f));
+    const mi355_weight& w = seg == 0 ? L.attn : seg == 1 ? L.proj : seg == 2 ? L.fc : L.mproj;
+    if (in_groups(w) && (seg != 0 || fz->have_x)) {  // (rows that are staged: so are their product's tables)
+        if (int rc = group_tables_of(m, layer, seg, s, fz, &f.tables)) return rc;
+    }
     switch (seg) {
         case 0: {
             // RMSNorm + c_attn; the epilogue rotates k and writes the K / V cache rows, q goes to qkv; then causal attention

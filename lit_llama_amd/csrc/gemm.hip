@@ -136,6 +136,7 @@ __device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n,
 constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials a workspace holds
 constexpr int kMaxSplit = 16;
 constexpr int kMaxRuns = 8;
+constexpr int kTableProducts = MI355_TABLE_PRODUCTS;
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
@@ -1098,7 +1099,7 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // their own.
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
-    static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1 && !FUSE), "grouped scales are a Q4 feature");
+    static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1), "grouped scales are a Q4 feature");
     static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
     static_assert(DEPTH >= 2 && DEPTH <= 4, "units under way + 1");
     constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
@@ -1278,7 +1279,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     };
     if constexpr (FUSE) {
         if (!own && s_part < kP) {
-            shares(p.in_sx, s_first, RUNS ? subs : kP, RUNS ? run_end(s_run) : s_hi, vx);
+            if constexpr (GRP == 0) shares(p.in_sx, s_first, RUNS ? subs : kP, RUNS ? run_end(s_run) : s_hi, vx);  // (GRP takes them unit by unit, below)
             if (p.in_ss_n > 0) shares(p.in_ss, s_part, kP, p.in_ss_n, vs);
         }
     }
@@ -1305,10 +1306,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
                     }
                     runtab[(run + s_sub * p.runs) * BM + s_tok] = sum;
                 }
-            } else {
+            } else if constexpr (GRP == 0) {
                 sxs = add_shares(s_first, kP, s_hi, vx, 0.f);
             }
             if (p.in_ss_n > 0) sss = add_shares(s_part, kP, p.in_ss_n, vs, 0.f);
+            if constexpr (GRP != 0) {  // (all of them now: the zero points' product in front of the loop waits for its loads anyway, and the loop has no register to spare)
+                for (int j0 = s_part + kIn * kP; j0 < p.in_ss_n; j0 += kIn * kP) {
+                    shares(p.in_ss, j0, kP, p.in_ss_n, vs);
+                    sss = add_shares(j0, kP, p.in_ss_n, vs, sss);
+                }
+                frp[(s_part * 2 + 0) * BM + s_tok] = sss;
+            }
         }
     }
     if constexpr (kScales) {
@@ -1356,6 +1364,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     if constexpr (GRP != 0) {
         // lane (g, c): units u0 + 4 g + i of product i; a chunk's factors are requested while the one before is multiplied
         struct Chunk { uint32_t sz[4][kTPW]; float x[4][kTT]; };
+        const bool halves = FUSE && p.in_ppu == 2;  // a producer in blocks of 64 hidden rows leaves two shares a unit
+        const int64_t x_step = halves ? 2 * (int64_t)p.M : p.M;
         auto fetch = [&](int u0, Chunk& k) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1364,7 +1374,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
                 for (int t = 0; t < kTPW; ++t)
                     k.sz[i][t] = p.gtab[((int64_t)(u >> p.gq_shift) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + c];
 #pragma unroll
-                for (int tt = 0; tt < kTT; ++tt) k.x[i][tt] = p.sxt[(int64_t)u * p.M + (m0 + tt * 16 + c < p.M ? m0 + tt * 16 + c : p.M - 1)];
+                for (int tt = 0; tt < kTT; ++tt) k.x[i][tt] = p.sxt[(int64_t)u * x_step + (m0 + tt * 16 + c < p.M ? m0 + tt * 16 + c : p.M - 1)];
+                if constexpr (FUSE) {
+                    if (halves) {
+#pragma unroll
+                        for (int tt = 0; tt < kTT; ++tt) k.x[i][tt] += p.sxt[(int64_t)u * x_step + p.M + (m0 + tt * 16 + c < p.M ? m0 + tt * 16 + c : p.M - 1)];
+                    }
+                }
             }
         };
         Chunk cur, nxt;
@@ -1578,7 +1594,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     }
     if constexpr (FUSE) {
         if (p.f_in) {  // the rest of the shares
-            if (s_part < kP) {
+            if (GRP == 0 && s_part < kP) {
                 for (int j0 = s_first + kIn * kP; !RUNS && j0 < s_hi; j0 += kIn * kP) {
                     shares(p.in_sx, j0, kP, s_hi, vx);
                     sxs = add_shares(j0, kP, s_hi, vx, sxs);
@@ -1596,7 +1612,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
                 for (int q = 0; q < kP; ++q) {
                     sss += frp[(q * 2 + 0) * BM + threadIdx.x];
-                    sxs += frp[(q * 2 + 1) * BM + threadIdx.x];
+                    if constexpr (GRP == 0) sxs += frp[(q * 2 + 1) * BM + threadIdx.x];
                 }
                 fr[threadIdx.x] = p.in_ss_n > 0 ? rsqrtf(sss / (float)p.K + p.eps) : 1.0f;
                 fr[BM + threadIdx.x] = sxs;
@@ -1869,23 +1885,26 @@ int launch_gemm_subgroups(const GemmParams& p, hipStream_t s) {
     if (blocks8 * 4 >= 128) return launch_gemm_w<EPI, PAIR, 2, 64, 2>(p, s);
     return launch_gemm_w<EPI, PAIR, 1, 64, 2>(p, s);
 }
-template <int EPI, bool PAIR>
+template <int EPI, bool PAIR, bool FUSE>
 int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
-    if (subgroups) return launch_gemm_subgroups<EPI, PAIR>(p, s);
+    if constexpr (!FUSE) {
+        if (subgroups) return launch_gemm_subgroups<EPI, PAIR>(p, s);
+    }
     const GemmCut sh = gemm_cut_grouped(p.n_tiles, p.M, PAIR, p.ksplit);
     if (sh.waves == 4) {
-        if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, false, 1>(p, s);
-        if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, false, 1>(p, s);
-        if (sh.bm == 48) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 48, false, 1>(p, s);
-        return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 64, false, 1>(p, s);
+        if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, FUSE, 1>(p, s);
+        if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, FUSE, 1>(p, s);
+        if (sh.bm == 48) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 48, FUSE, 1>(p, s);
+        return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 64, FUSE, 1>(p, s);
     }
-    if (sh.bm == 64) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 64, false, 1>(p, s);
-    return launch_deep<EPI, PAIR, MI355_W_Q4, 8, kBM, false, 1>(p, s);
+    if (sh.bm == 64) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 64, FUSE, 1>(p, s);
+    return launch_deep<EPI, PAIR, MI355_W_Q4, 8, kBM, FUSE, 1>(p, s);
 }
+template <bool FUSE>
 int launch_gemm_grouped_epi(const GemmParams& p, int epi, bool subgroups, hipStream_t s) {
-    if (epi == MI355_EPI_SWIGLU) return launch_gemm_grouped<MI355_EPI_SWIGLU, true>(p, subgroups, s);
-    if (epi == MI355_EPI_ACCUM) return launch_gemm_grouped<MI355_EPI_ACCUM, false>(p, subgroups, s);
-    return launch_gemm_grouped<MI355_EPI_STORE, false>(p, subgroups, s);
+    if (epi == MI355_EPI_SWIGLU) return launch_gemm_grouped<MI355_EPI_SWIGLU, true, FUSE>(p, subgroups, s);
+    if (epi == MI355_EPI_ACCUM) return launch_gemm_grouped<MI355_EPI_ACCUM, false, FUSE>(p, subgroups, s);
+    return launch_gemm_grouped<MI355_EPI_STORE, false, FUSE>(p, subgroups, s);
 }
 template <int FMT, bool FUSE>
 int launch_gemm_epi(const GemmParams& p, int epi, hipStream_t s) {
@@ -1929,9 +1948,20 @@ extern "C" int mi355_linear_gemm(const mi355_linear_args* a, void* workspace, si
     return mi355_linear_gemm_fused(a, nullptr, workspace, workspace_bytes, stream);
 }
 
-extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
-    const bool pair = R == 2;
-    const GemmCut cut = gemm_cut(M, N, K, pair, bf16);
+namespace {
+// K-slices of grouped scales: blocks of 8 row tiles x 64 tokens, doubled to 256 by slices of at least 4 cuts (groups; units where a group holds several: a slice may end
+// within a group, whose products are scaled unit by unit).  Partial sums in the first half of the region, the tables in the second
+int grouped_split(int M, int N, int K, bool pair, int group_cols) {
+    const int rows_per_block = pair ? 16 * 4 * kTPW / 2 : 16 * 4 * kTPW, n_groups = (K + group_cols - 1) / group_cols;
+    const int blocks = ((N + rows_per_block - 1) / rows_per_block) * ((M + 63) / 64), cuts = group_cols >= 128 ? n_groups : (K + 127) / 128;
+    const TableBytes t = table_bytes(M, N, pair ? 2 : 1, n_groups);
+    int ksplit = 1;
+    while (ksplit < kMaxSplit && blocks * ksplit < 256 && cuts >= 8 * ksplit && t.tables + t.sums <= kSplitBudget / 2 &&
+           gemm_part_bytes(M, N, pair, 2 * ksplit) <= kSplitBudget / 2)
+        ksplit *= 2;
+    return ksplit;
+}
+void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares, int* shares_per_unit) {
     // rows (hidden rows of a pair stream) behind one share of a producer's partial sums: a 128-column unit when the K-slices'
     // reduction writes them or a block holds 256 rows, else the block's rows
     int rows = (pair ? cut.waves * kTPW / 2 : cut.waves * kTPW) * 16;
@@ -1939,6 +1969,48 @@ extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, in
     *ksplit = cut.ksplit;
     *shares = (N + rows - 1) / rows;
     *shares_per_unit = 128 / rows;
+}
+}  // namespace
+extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
+    plan_shares(gemm_cut(M, N, K, R == 2, bf16), N, R == 2, ksplit, shares, shares_per_unit);
+}
+void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
+    plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
+}
+
+// The tables of several products in one launch: a prompt's layers take theirs 10 at a time (7B), 9 us, instead of 5 us and a gap in front of each
+namespace {
+struct TableSet {
+    GroupTables of[kTableProducts];
+    int end[kTableProducts];  // pieces up to the end of each product's
+};
+__global__ __launch_bounds__(256) void group_tables_kernel(const TableSet set) {
+    __shared__ uint32_t lds[kStageLds];
+    int i = 0, from = 0;
+    while (i < kTableProducts - 1 && (int)blockIdx.x >= set.end[i]) from = set.end[i++];
+    group_table_piece(set.of[i], (int)blockIdx.x - from, lds);
+}
+GroupTables group_tables(const mi355_linear_args& a, int cols, uint32_t* out) {
+    return {(const bf16_t*)a.scales, (const bf16_t*)a.zeros, (const bf16_t*)a.scales2, (const bf16_t*)a.zeros2, a.N, (a.N + 15) / 16 * 16, (a.K + cols - 1) / cols, a.R, out};
+}
+}  // namespace
+size_t mi355_linear_gemm_table_bytes(int N, int K, int R, int group_cols) { return table_bytes(0, N, R, (K + group_cols - 1) / group_cols).tables; }
+size_t mi355_linear_gemm_table_room() { return kSplitBudget / 2 - 256; }  // (the region itself starts up to 15 bytes past its place)
+int mi355_linear_gemm_tables(const mi355_linear_args* products, uint32_t* const* out, int n, mi355_stream_t stream) {
+    MI355_CHECK_ARG(n >= 1 && n <= kTableProducts, MI355_E_ARG, "linear_gemm: tables of %d products", n);
+    TableSet set;
+    memset(&set, 0, sizeof(set));
+    int pieces = 0;
+    for (int i = 0; i < kTableProducts; ++i) {
+        if (i < n) {
+            set.of[i] = group_tables(products[i], products[i].group_cols, out[i]);
+            pieces += set.of[i].pieces();
+        }
+        set.end[i] = pieces;
+    }
+    hipLaunchKernelGGL(group_tables_kernel, dim3(pieces), dim3(256), 0, (hipStream_t)stream, set);
+    MI355_LAUNCH_CHECK();
+    return 0;
 }
 
 static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f, mi355_reduce_norm* norm, void* workspace, size_t workspace_bytes, mi355_stream_t stream);
@@ -2006,18 +2078,8 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         sxt_bytes = t.sums;  // (of groups of whole units: in a place of their own)
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
-        // grouped scales: blocks of 8 row tiles x 64 tokens, doubled to 256 by slices of at least 4 cuts (groups; units where a group holds several: a slice may end within
-        // a group, whose products are scaled unit by unit).  Partial sums in the first half of the region, the tables in the second
-        const int rows_per_block = swiglu ? 16 * 4 * kTPW / 2 : 16 * 4 * kTPW;
-        const int blocks = ((a->N + rows_per_block - 1) / rows_per_block) * ((a->M + 63) / 64);
-        const size_t row_floats = (size_t)a->N * (swiglu ? 2 : 1);
-        const int cuts = scale_groups && a->group_cols >= 128 ? n_groups : units;
-        if (unit_sums)
-            ksplit = gemm_cut(a->M, a->N, a->K, swiglu, false).ksplit;  // (partial sums: at most half the region, the tables lie in the other)
-        else
-            while (ksplit < kMaxSplit && blocks * ksplit < 256 && cuts >= 8 * ksplit && tab_bytes + sxt_bytes <= kSplitBudget / 2 &&
-                   (size_t)2 * ksplit * a->M * row_floats * 4 <= kSplitBudget / 2)
-                ksplit *= 2;
+        // (partial sums: at most half the region, the tables lie in the other)
+        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
     }
     int runs = 1, run_units = units;
     if (!grouped) {
@@ -2025,17 +2087,18 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
     }
-    // producer / consumer fusion (gemm_fuse.h): launches over per-row scales only — the caller plans with mi355_linear_gemm_plan
+    // producer / consumer fusion (gemm_fuse.h): one scale per row, or groups of whole units — the caller plans with mi355_linear_gemm_plan or ..._grouped
     const bool fused = f != nullptr;
     const bool f_in = fused && f->prestaged;
     if (fused) {
-        MI355_CHECK_ARG(!grouped, MI355_E_STATE, "linear_gemm: fusion over a grouped launch (M=%d N=%d K=%d)", a->M, a->N, a->K);
+        MI355_CHECK_ARG(!grouped || (a->group_cols >= 128 && (!f_in || f->tables != nullptr)), MI355_E_STATE,
+                        "linear_gemm: fusion over a launch of small groups or without its tables (M=%d N=%d K=%d)", a->M, a->N, a->K);
         const bool produces = f->out_xb != nullptr || f->out_sx != nullptr || f->rope != nullptr;
         MI355_CHECK_ARG(!produces || a->N % 128 == 0, MI355_E_SHAPE, "linear_gemm: a producer of the fused chain has N %% 128 == 0 (N=%d)", a->N);
         MI355_CHECK_ARG(ksplit == 1 || !produces || a->epi == MI355_EPI_SWIGLU || a->y_dtype == MI355_F32, MI355_E_DTYPE,
                         "linear_gemm: the fused reduction of a K-split launch writes f32 rows (or the SwiGLU pair's bf16)");
-        MI355_CHECK_ARG(!f_in || (ksplit == 1 && runs == 1) || (f->in_ppu >= 1 && f->in_sx_n == units * f->in_ppu), MI355_E_ARG,
-                        "linear_gemm: a consumer of K-slices or runs needs %d x in_ppu partial operand sums (got %d, in_ppu %d)", units, f->in_sx_n, f->in_ppu);
+        MI355_CHECK_ARG(!f_in || (ksplit == 1 && runs == 1 && !grouped) || (f->in_ppu >= 1 && (!grouped || f->in_ppu <= 2) && f->in_sx_n == units * f->in_ppu), MI355_E_ARG,
+                        "linear_gemm: a consumer of K-slices, runs or groups needs %d x in_ppu partial operand sums (got %d, in_ppu %d)", units, f->in_sx_n, f->in_ppu);
         MI355_CHECK_ARG(!f_in || (a->x_dtype == MI355_BF16 && a->norm_scale == nullptr && a->K % 128 == 0 && a->ldx % 8 == 0 &&
                                   (uintptr_t)a->x % 16 == 0 && f->in_sx != nullptr && f->in_sx_n > 0 && (f->in_ss == nullptr || f->in_ss_n > 0)),
                         MI355_E_ARG, "linear_gemm: a pre-staged operand is bf16 [M, ldx] with K %% 128 == 0 and partial operand sums");
@@ -2059,13 +2122,18 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     memset(&p, 0, sizeof(p));
     if (grouped) {
         // the group tables live in the split-K region of the workspace (its second half when the launch is split)
-        uint32_t* gtab = (uint32_t*)((char*)part + (ksplit > 1 ? kSplitBudget / 2 : 0));
+        const uint32_t* gtab = (uint32_t*)((char*)part + (ksplit > 1 ? kSplitBudget / 2 : 0));
         const int cols = unit_sums || a->group_cols >= 128 ? 128 : a->group_cols;
-        float* sxt = cols == 128 ? rinv + unit_sums_at(a->M) : (float*)((char*)gtab + tab_bytes);
-        const GroupTables tables = {(const bf16_t*)a->scales, (const bf16_t*)a->zeros, (const bf16_t*)a->scales2, (const bf16_t*)a->zeros2, a->N, tab_ld, n_groups, a->R, gtab};
-        hipLaunchKernelGGL(aligned ? stage_units_kernel<true> : stage_units_kernel<false>, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx,
-                           a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv, (float*)nullptr, 1, 1, units, 1.f, 0.f, sxt, a->M, cols, tables);
-        MI355_LAUNCH_CHECK();
+        const float* sxt = cols == 128 ? rinv + unit_sums_at(a->M) : (const float*)((const char*)gtab + tab_bytes);
+        if (f_in) {
+            gtab = f->tables;
+            sxt = f->in_sx;
+        } else {
+            const GroupTables tables = group_tables(*a, unit_sums ? a->K : a->group_cols, (uint32_t*)gtab);
+            hipLaunchKernelGGL(aligned ? stage_units_kernel<true> : stage_units_kernel<false>, dim3(a->M + tables.pieces()), dim3(256), 0, s, a->x, a->x_dtype, a->ldx,
+                               a->norm_scale, a->norm_dtype, a->eps, a->K, xb, rinv, (float*)nullptr, 1, 1, units, 1.f, 0.f, (float*)sxt, a->M, cols, tables);
+            MI355_LAUNCH_CHECK();
+        }
         p.gtab = gtab;
         p.sxt = sxt;
         p.n_groups = n_groups;
@@ -2126,7 +2194,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         norm->done = ksplit > 1 && a->epi == MI355_EPI_ACCUM && a->y_dtype == MI355_F32 && a->N <= kNormHeld * 4096;
         p.rn = *norm;
     }
-    if (grouped) return launch_gemm_grouped_epi(p, a->epi, scale_groups && a->group_cols < 128, s);
+    if (grouped && !fused) return launch_gemm_grouped_epi<false>(p, a->epi, scale_groups && a->group_cols < 128, s);
     if (fused) {
         p.f_in = f_in ? 1 : 0;
         p.in_sx = f->in_sx;
@@ -2149,6 +2217,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         p.C = f->n_head * f->hs;
         p.rope_gathered = f->rope_gathered;
         p.q_scale = f->rope != nullptr ? f->q_scale : 0.f;
+        if (grouped) return launch_gemm_grouped_epi<true>(p, a->epi, false, s);
         if (q4) return launch_gemm_epi<MI355_W_Q4, true>(p, a->epi, s);
         return launch_gemm_epi<MI355_W_BF16, true>(p, a->epi, s);
     }

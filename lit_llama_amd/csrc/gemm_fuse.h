@@ -22,6 +22,7 @@ struct mi355_gemm_fuse {
     int in_ppu;           // shares per 128-column unit (a K-split consumer's slice adds the shares of its own units)
     const float* in_ss;   // [in_ss_n][M] partial sums of squares of the f32 row behind the operand, or NULL (1/rms = 1)
     int in_ss_n;
+    const uint32_t* tables;  // grouped scales: this product's tables (mi355_linear_gemm_tables)
     // ---- producer side, MI355_EPI_ACCUM with f32 y: also emit the next linear's operand
     bf16_t* out_xb;       // [M, out_ld] = bf16(next_norm[n] * y_new[m, n]), or NULL
     int64_t out_ld;
@@ -47,6 +48,15 @@ struct mi355_gemm_fuse {
 // many of them make a 128-column unit.  A launch split over K produces through the reduction of its slices
 // (splitk_fused_reduce_kernel), one share per unit.
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
+// the same for scales in groups of group_cols columns (whole units)
+void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit);
+// Tables of the (scale, zero) pairs of up to MI355_TABLE_PRODUCTS products over grouped scales, laid out ahead of them in one launch: fmt, N, K, R, group_cols and the
+// scales and zeros of products[i] count; out[i] takes mi355_linear_gemm_table_bytes.  table_room: bytes at the end of the region of K-slice sums (in front of the fuse
+// scratch) that no grouped launch's own sums reach.
+#define MI355_TABLE_PRODUCTS 16
+size_t mi355_linear_gemm_table_bytes(int N, int K, int R, int group_cols);
+size_t mi355_linear_gemm_table_room();
+int mi355_linear_gemm_tables(const mi355_linear_args* products, uint32_t* const* out, int n, mi355_stream_t stream);
 // bytes mi355_linear_gemm_workspace_bytes reserves at the END of a workspace for the chain's partial sums
 size_t mi355_linear_gemm_fuse_scratch_bytes();
 // whether the tables of a product's (scale, zero) pairs per row and group of `group_cols` columns fit their region of a workspace (a launch refuses those that do not)

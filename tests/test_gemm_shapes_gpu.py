@@ -300,6 +300,54 @@ def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
 
 
+@pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600)])
+def test_fused_prompt_chain_over_grouped_scales(dev, monkeypatch, cols, heads, T):
+    """Groups of whole units in the chain: one share per unit, or two (c_fc1 / c_fc2 in blocks of 64 hidden rows); slices and whole sums; tables of several layers from one
+    launch and the next.  Against the same layers with staging passes, 0.02 of the logits' spread as for one scale per row."""
+    model = _wide_model(dev, LLaMAConfig(block_size=784, n_layer=5 if heads == 15 else 3, n_head=heads, n_embd=128 * heads, vocab_size=512), "gptq.int4", cols)
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
+        model.reset_cache()
+        with torch.no_grad():
+            out.append(model(idx.view(1, -1), 784, torch.arange(T, device=dev))[0].float())
+    assert model.engine() is not None, model._engine_failed
+    assert not torch.equal(*out)  # (the chain was on)
+    assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
+
+
+@pytest.mark.parametrize("T", [40, 150, 700])
+def test_fused_prompt_chain_over_groups_rows_and_bf16(dev, monkeypatch, T):
+    """Layers of groups of 128 columns, of one scale per row and of bf16 in one chain: K-slices of the latter take the room of the former's tables, which are laid out
+    again behind them.  The bound as above."""
+    cfg = LLaMAConfig(block_size=704, n_layer=4, n_head=15, n_embd=1920, vocab_size=512)
+    model = _wide_model(dev, cfg, "gptq.int4", 128)
+    rows = _wide_model(dev, cfg, "gptq.int4", 0)
+    g = torch.Generator(device=dev).manual_seed(4)
+    for layer, name, kind in ((0, "attn.c_proj", "rows"), (1, "attn.c_attn", "bf16"), (1, "mlp.c_proj", "bf16"), (2, "mlp.c_fc1", "rows"), (2, "mlp.c_fc2", "rows"), (2, "attn.c_proj", "bf16"),
+                              (3, "attn.c_attn", "rows")):
+        part, attr = name.split(".")
+        owner = getattr(model.transformer.h[layer], part)
+        q = getattr(owner, attr)
+        if kind == "rows":
+            new = getattr(getattr(rows.transformer.h[layer], part), attr)
+        else:
+            new = torch.nn.Linear(q.in_features, q.out_features, bias=False, device=dev, dtype=torch.bfloat16)
+            new.weight.data = (torch.randn(new.weight.shape, generator=g, device=dev) * q.in_features ** -0.5).to(torch.bfloat16)
+        setattr(owner, attr, new)
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
+        model.reset_cache()
+        with torch.no_grad():
+            out.append(model(idx.view(1, -1), 704, torch.arange(T, device=dev))[0].float())
+    assert model.engine() is not None, model._engine_failed
+    assert not torch.equal(*out)  # (the chain was on)
+    assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
+
+
 @pytest.mark.parametrize("M", [9, 40, 100, 300, 600])
 @pytest.mark.parametrize("fmt", ["q4", "g128", "g32", "bf16", "i8"])
 def test_rows_that_are_not_finite_stay_by_themselves(dev, fmt, M):
