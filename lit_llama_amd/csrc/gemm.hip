@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     static_assert(DEPTH >= 2 && DEPTH <= 4, "units under way + 1");
     constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
-    constexpr int kXI = BM / 4 > kWaves ? BM / 4 / kWaves : 1;  // activation requests (1 KiB: four tokens) per wave and unit
+    constexpr int kXI = (BM / 4 + kWaves - 1) / kWaves;  // activation requests (1 KiB: four tokens) per wave and unit
     constexpr int kUnit = kXI + kTPW * kWP + (GRP ? kTPW : 0);  // requests per wave and unit
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
@@ -1711,6 +1711,7 @@ GemmForce gemm_force() {
     return f;
 }
 bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (what a sweep may force of the kernels of launch_gemm(); the other blocks of BF16 streams are the estimate's)
+    if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
 }
@@ -1751,7 +1752,26 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
     if (wide >= 384 || wide == 256) cut.bm = kBM, cut.deep = false;
     return cut;
 }
-// BF16 streams.  Up to 64 tokens blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
+// Up to 32 tokens, outside the fused chain (whose shares are 64 or 128 rows), where blocks of 4 waves do not fill the chip: blocks of 2, 3 or 4 waves (64, 96, 128 rows).  A CU
+// asks for no more than its memory pipeline holds, so 129 blocks of 128 rows leave half of what HBM gives, and a slice that would fill the other CUs costs a launch; smaller
+// blocks cost their activations again.  16 tokens, 4 / 3 / 2 waves without slices: N = 16512, K = 4096 29.7 / 26.1 / 35.0 us (129, 172, 258 blocks), 12416 33.2 (24.9 in two
+// slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, a block's unit
+// taking its share of HBM too, and a launch for the slices: over 72 launches (36 products of 1024 to 32000 rows, 16 and 32 tokens, weights not in any cache) its choice
+// is 0.4 % behind the fastest, 0.909 times what blocks of 4 waves took, none slower.
+GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
+    const int units = (K + 127) / 128;
+    GemmCut cut = {4, short_block(M, true), true, 1};
+    float best = 0.f;
+    for (int waves = 2; waves <= 4; ++waves)
+        for (int ks = 1; ks <= 8 && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget / 2)); ++ks) {
+            const int blocks = gemm_blocks(M, N, pair, waves, cut.bm) * ks;
+            auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (0.007f + (float)waves * (0.066f + 0.193f * (float)of / 256.f)); };
+            const float us = (float)(blocks / 256) * round(256) + round(blocks % 256) + (ks == 1 ? 0.f : 1.5f + (float)gemm_part_bytes(M, N, pair, ks) / 2.7e6f);
+            if (best == 0.f || us < best) best = us, cut.waves = waves, cut.ksplit = ks;
+        }
+    return cut;
+}
+// BF16 streams.  33 to 64 tokens (and fewer of the chain): blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
 // none to a few more than all (16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 /
 // 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13); where those blocks are more than the CUs, blocks of 8 (48 tokens of the N = 17920 pair, K = 6656: 104 / 95 us with 4 / 8 waves).
 // Longer: 192 to 256 blocks of 128 tokens x 256 rows, one round of the chip, take those (3-5 % less than what the estimate takes).  Else what an estimate takes for the
@@ -1761,7 +1781,8 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
 // 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  The constants
 // are those whose choice is best over 19 500 launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are): 1.7 % behind the
 // fastest of them on average, 6 % at the 90th percentile.
-GemmCut bf16_cut(int M, int N, int K, bool pair) {
+GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain) {
+    if (!chain && M <= 32 && gemm_blocks(M, N, pair, 4, 32) <= 256) return bf16_cut_few(M, N, K, pair);
     const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
     GemmCut cut = {4, short_block(M, true), true, 1};
     if (M <= 64 && few <= 256) {
@@ -1806,11 +1827,12 @@ GemmCut bf16_cut(int M, int N, int K, bool pair) {
         for (const Kind& k : kinds) consider(k);
     return cut;
 }
-GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16) {
+// chain: a launch of the fused prompt chain (gemm_fuse.h)
+GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain) {
     const GemmForce fo = gemm_force();
-    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair) : q4_cut(M, N, K, pair);
+    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain) : q4_cut(M, N, K, pair);
     const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep == 1 : cut.deep, cut.ksplit};
-    if (launch_gemm_has(forced, bf16)) cut = forced;
+    if (launch_gemm_has(forced, bf16) && (!chain || forced.waves >= 4)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= kSplitBudget / 2) cut.ksplit = fo.ksplit;
     return cut;
 }
@@ -1853,7 +1875,12 @@ void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, in
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
-    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16);
+    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE);
+    if constexpr (FMT == MI355_W_BF16 && !FUSE) {
+        // (operand slices start at multiples of 256 rows: blocks of 64 divide them, of 96 not)
+        if (sh.waves == 3 && p.slice_blocks == 0) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
+        if (sh.waves <= 3) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
+    }
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, FMT, 4, 32, FUSE>(p, s);
@@ -1972,7 +1999,7 @@ void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares,
 }
 }  // namespace
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
-    plan_shares(gemm_cut(M, N, K, R == 2, bf16), N, R == 2, ksplit, shares, shares_per_unit);
+    plan_shares(gemm_cut(M, N, K, R == 2, bf16, true), N, R == 2, ksplit, shares, shares_per_unit);
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
     plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
@@ -2079,11 +2106,11 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
         // (partial sums: at most half the region, the tables lie in the other)
-        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
+        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
     }
     int runs = 1, run_units = units;
     if (!grouped) {
-        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4);
+        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr);
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
     }

@@ -300,6 +300,26 @@ def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
 
 
+@pytest.mark.parametrize("epi", ["store", "pair", "accum"])
+@pytest.mark.parametrize("M", [5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(64, 128), (68, 1000), (96, 4096), (100, 640), (4096, 2048), (8200, 384), (12352, 1024), (16512, 512)])
+def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
+    """Block edges at 64, 96 and 128 rows, slices, a last unit that is not whole.  The bound of the tiled product."""
+    g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    ws = [(torch.randn((N, K), generator=g, device=dev) * K ** -0.5).to(torch.bfloat16) for _ in range(2)]
+    prods = [x.double() @ w.double().T for w in ws]
+    if epi == "pair":
+        ref = torch.nn.functional.silu(prods[0]) * prods[1]
+        got = ops.linear_gemm(x, ops.repack_bf16(ws[0], ws[1], 2), 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, fmt=nat.W_BF16).double()
+        assert (got - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 2e-3 * ref.square().mean().sqrt()
+        return
+    base = torch.randn((M, N), generator=g, device=dev) if epi == "accum" else torch.zeros((M, N), device=dev)
+    ref = prods[0] + base.double()
+    got = ops.linear_gemm(x, ops.repack_bf16(ws[0], None, 1), 1, N, K, epi=nat.EPI_ACCUM if epi == "accum" else nat.EPI_STORE, out=base.clone(), fmt=nat.W_BF16).double()
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
 @pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600)])
 def test_fused_prompt_chain_over_grouped_scales(dev, monkeypatch, cols, heads, T):
     """Groups of whole units in the chain: one share per unit, or two (c_fc1 / c_fc2 in blocks of 64 hidden rows); slices and whole sums; tables of several layers from one
