@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "gemm_fuse.h"
+#include "int8_chain.h"
 
 // implemented in int8.hip: the LLM.int8 linear driven from a mi355_weight descriptor
 int mi355_linear_int8_from_weight(const mi355_weight* w, const mi355_model* m, const void* x, int x_dtype, int M,
@@ -233,12 +234,26 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
     return z;
 }
 
+// The chain of a forward call's LLM.int8 products.  Its mask ends the workspace, behind what any product of T rows uses there (an int4 or bf16 product without the fused chain
+// leaves the fused chain's partial sums alone, which are longer); no mask if the workspace was sized for less.
+mi355_i8_chain plan_i8_chain(const mi355_model* m, int T) {
+    mi355_i8_chain c = {nullptr, 0, false};
+    int K = m->lm_head.K;
+    for (int l = 0; l < m->n_layer; ++l)
+        for (const mi355_weight* w : {&m->layers[l].attn, &m->layers[l].proj, &m->layers[l].fc, &m->layers[l].mproj}) K = w->K > K ? w->K : K;
+    const size_t bytes = mi355_i8_chain_bytes(K);
+    if (T < 32 || m->gemm_ws == nullptr || (size_t)m->gemm_ws_bytes < mi355_linear_int8_gemm_workspace_bytes(T, K)) return c;
+    c.mask = (unsigned*)((char*)m->gemm_ws + (((size_t)m->gemm_ws_bytes - bytes) & ~(size_t)15));
+    c.words = (int)(bytes / 4);
+    return c;
+}
+
 // One linear over M <= max_T rows.  The rows of one launch must fit the workgroup's LDS next to the combine
 // buffers (7B: 13 rows at K = 4096, 5 at K = 11008), so wide inputs are fed in equal sub-chunks of rows: the
 // prompt chunk size is set by the NARROW linears and only mlp.c_proj pays extra launches.
 int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x_dtype, int M, int64_t ldx,
                const void* norm_scale, int epi, void* y, int y_dtype, int64_t ldy, hipStream_t s,
-               const float* attn_partials = nullptr) {
+               const float* attn_partials = nullptr, mi355_i8_chain* chain = nullptr) {
     // wide inputs of an int4 or bf16 model: the LDS-tiled MFMA GEMM over the same stream (per-row or grouped scales)
     if ((w.fmt == MI355_W_Q4 || w.fmt == MI355_W_BF16) && M >= wide_rows(w) && m->gemm_ws != nullptr &&
         attn_partials == nullptr && w.N % 4 == 0 && ldy % 4 == 0 && (w.group_cols == 0 || w.K % 128 == 0) && (M >= 32 || short_chunk_fits(m, w, M, epi))) {
@@ -269,7 +284,7 @@ int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x
         a.y = y;
         a.y_dtype = y_dtype;
         a.ldy = ldy;
-        return mi355_linear_int8_gemm(&a, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
+        return mi355_linear_int8_gemm_chained(&a, chain, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
     }
     const int cap = row_cap(w);
     MI355_CHECK_ARG(cap >= 1, MI355_E_SHAPE, "forward: a row of K=%d does not fit LDS", w.K);
@@ -346,7 +361,8 @@ extern "C" int mi355_set_step(const mi355_model* m, const void* idx, int idx_is_
 }
 
 static int forward_segment_impl(const mi355_model* m, int T, int layer, int seg_begin, int seg_end, mi355_stream_t stream,
-                                FuseCtx* fz);
+                                FuseCtx* fz, mi355_i8_chain* chain);
+static int forward_head_impl(const mi355_model* m, int T, int logits_mode, int argmax, mi355_stream_t stream, mi355_i8_chain* chain);
 
 extern "C" int mi355_forward(const mi355_model* m, int T, int logits_mode, int argmax, mi355_stream_t stream) {
     MI355_CHECK_ARG(m != nullptr && m->layers != nullptr, MI355_E_ARG, "forward: null model");
@@ -369,10 +385,12 @@ extern "C" int mi355_forward(const mi355_model* m, int T, int logits_mode, int a
     }
 
     FuseCtx fz = plan_fusion(m, T);
+    mi355_i8_chain masks = plan_i8_chain(m, T);
+    mi355_i8_chain* const chain = masks.mask != nullptr ? &masks : nullptr;
     for (int l = 0; l < m->n_layer; ++l) {
-        if (int rc = forward_segment_impl(m, T, l, 0, 4, s, fz.on ? &fz : nullptr)) return rc;
+        if (int rc = forward_segment_impl(m, T, l, 0, 4, s, fz.on ? &fz : nullptr, chain)) return rc;
     }
-    return mi355_forward_head(m, T, logits_mode, argmax, s);
+    return forward_head_impl(m, T, logits_mode, argmax, s, chain);
 }
 
 // segments of layer l: 0 = RMSNorm + c_attn + attention, 1 = attn.c_proj, 2 = RMSNorm + fc + SwiGLU, 3 = mlp.c_proj.
@@ -380,7 +398,7 @@ extern "C" int mi355_forward(const mi355_model* m, int T, int logits_mode, int a
 // calls mi355_residual_add); with tp_world == 1 they accumulate into the residual stream directly.
 extern "C" int mi355_forward_segment(const mi355_model* m, int T, int layer, int seg_begin, int seg_end,
                                      mi355_stream_t stream) {
-    return forward_segment_impl(m, T, layer, seg_begin, seg_end, stream, nullptr);
+    return forward_segment_impl(m, T, layer, seg_begin, seg_end, stream, nullptr, nullptr);
 }
 
 // The tables of a product over grouped scales, laid out with those of the products behind it, as many as there is room for: up to the first one of another kind, whose
@@ -496,7 +514,7 @@ static int fused_segment(const mi355_model* m, int T, int layer, int seg, hipStr
 }
 
 static int forward_segment_impl(const mi355_model* m, int T, int layer, int seg_begin, int seg_end, mi355_stream_t stream,
-                                FuseCtx* fz) {
+                                FuseCtx* fz, mi355_i8_chain* chain) {
     MI355_CHECK_ARG(m != nullptr && m->layers != nullptr, MI355_E_ARG, "forward_segment: null model");
     MI355_CHECK_ARG(layer >= 0 && layer < m->n_layer, MI355_E_ARG, "forward_segment: bad layer %d", layer);
     MI355_CHECK_ARG(seg_begin >= 0 && seg_end <= 4 && seg_begin < seg_end, MI355_E_ARG, "forward_segment: bad range");
@@ -516,7 +534,7 @@ static int forward_segment_impl(const mi355_model* m, int T, int layer, int seg_
         switch (seg) {
             case 0: {
                 if (int rc = run_linear(m, L.attn, m->x, MI355_F32, T, C, L.rms1, MI355_EPI_STORE, m->qkv, MI355_F32,
-                                        3 * Cl, s))
+                                        3 * Cl, s, nullptr, chain))
                     return rc;
                 mi355_attn_args a;
                 memset(&a, 0, sizeof(a));
@@ -562,18 +580,18 @@ static int forward_segment_impl(const mi355_model* m, int T, int layer, int seg_
                 }
                 if (int rc = run_linear(m, L.proj, m->att, MI355_BF16, T, Cl, nullptr,
                                         tp ? MI355_EPI_STORE : MI355_EPI_ACCUM, tp ? m->partial : m->x, MI355_F32, C, s,
-                                        fused ? m->attn_part : nullptr))
+                                        fused ? m->attn_part : nullptr, chain))
                     return rc;
                 break;
             }
             case 2:
                 if (int rc = run_linear(m, L.fc, m->x, MI355_F32, T, C, L.rms2, MI355_EPI_SWIGLU, m->hbuf, MI355_BF16,
-                                        m->n_hidden, s))
+                                        m->n_hidden, s, nullptr, chain))
                     return rc;
                 break;
             case 3:
                 if (int rc = run_linear(m, L.mproj, m->hbuf, MI355_BF16, T, m->n_hidden, nullptr,
-                                        tp ? MI355_EPI_STORE : MI355_EPI_ACCUM, tp ? m->partial : m->x, MI355_F32, C, s))
+                                        tp ? MI355_EPI_STORE : MI355_EPI_ACCUM, tp ? m->partial : m->x, MI355_F32, C, s, nullptr, chain))
                     return rc;
                 break;
         }
@@ -598,6 +616,10 @@ extern "C" int mi355_residual_add(const mi355_model* m, int T, mi355_stream_t st
 }
 
 extern "C" int mi355_forward_head(const mi355_model* m, int T, int logits_mode, int argmax, mi355_stream_t stream) {
+    return forward_head_impl(m, T, logits_mode, argmax, stream, nullptr);
+}
+
+static int forward_head_impl(const mi355_model* m, int T, int logits_mode, int argmax, mi355_stream_t stream, mi355_i8_chain* chain) {
     MI355_CHECK_ARG(m != nullptr, MI355_E_ARG, "forward_head: null model");
     MI355_CHECK_ARG(T >= 1 && T <= m->max_T, MI355_E_SHAPE, "forward_head: T=%d outside 1..%d", T, m->max_T);
     if (logits_mode == 0) return 0;
@@ -612,7 +634,7 @@ extern "C" int mi355_forward_head(const mi355_model* m, int T, int logits_mode, 
             return rc;
     } else {
         if (int rc = run_linear(m, m->lm_head, m->x, MI355_F32, T, C, m->ln_f, MI355_EPI_STORE, m->logits, MI355_F32, V,
-                                s))
+                                s, nullptr, chain))
             return rc;
     }
     if (argmax) {

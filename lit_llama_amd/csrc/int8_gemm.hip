@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "int8_chain.h"
 
 namespace {
 
@@ -77,6 +78,8 @@ struct I8GemmParams {
     // n_out zero.  They exist where so fits its region
     f16_t* xo;
     f16_t* so;
+    unsigned* mask_next;  // what the next product of a chain ORs into, cleared here (int8_chain.h), or NULL
+    int mask_words;
 };
 constexpr size_t kSplitBudget = (size_t)32 << 20;             // bytes of the int32 partial tiles of all K-slices,
 constexpr size_t kPartBytes = kSplitBudget + kSplitBudget / 2;  // next to the f32 tiles of the outlier columns (2 slices at least)
@@ -299,6 +302,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
     const int g = lane >> 4, c = lane & 15;
     const int xcd = blockIdx.x & 7, j0 = blockIdx.x >> 3;
     const int L2 = xcd * p.per_xcd + j0;
+    if (MODE != 2 && blockIdx.x == 0 && p.mask_next != nullptr)
+        for (int i = threadIdx.x; i < p.mask_words; i += kThreads) p.mask_next[i] = 0u;
     // MODE 1: a workgroup per (block, K-slice); MODE 2: a workgroup per (block, 16-token tile) — 8 x the workgroups of the
     // product launch, so that summing the slices and the epilogue are not left to a dozen workgroups
     const int nsplit = MODE == 1 ? p.ksplit + 1 : MODE == 2 ? 8 : 1;
@@ -740,10 +745,16 @@ extern "C" size_t mi355_linear_int8_gemm_workspace_bytes(int M, int K) {
     // xh f16 [M, Kp], CA int8 [M, Kp], absmax [M], column mask [Kp / 32], outlier list [1 + Kp]
     return pad16((size_t)M * kp * 2) + pad16((size_t)M * kp) + pad16((size_t)M * 4) + pad16(kp / 8) + pad16((1 + kp) * 4) + 256 +
            kPartBytes +                                      // partial tiles of the split-K launches (short prompts)
-           pad16((size_t)M * kp * 2) + kOutlierBudget;       // outlier columns by themselves: of the rows, of the weights
+           pad16((size_t)M * kp * 2) + kOutlierBudget +      // outlier columns by themselves: of the rows, of the weights
+           mi355_i8_chain_bytes(K);                          // the mask of a chain of products
 }
+size_t mi355_i8_chain_bytes(int K) { return pad16(((size_t)K + 127) / 128 * 16); }
 
 extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace, size_t workspace_bytes, mi355_stream_t stream) {
+    return mi355_linear_int8_gemm_chained(a, nullptr, workspace, workspace_bytes, stream);
+}
+
+int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* chain, void* workspace, size_t workspace_bytes, mi355_stream_t stream) {
     MI355_CHECK_ARG(a != nullptr && workspace != nullptr && a->w && a->scb && a->x && a->y, MI355_E_ARG, "linear_int8_gemm: null argument");
     MI355_CHECK_ARG(a->R == 1 || a->R == 2, MI355_E_ARG, "linear_int8_gemm: R must be 1 or 2");
     MI355_CHECK_ARG(a->M >= 1 && a->N > 0 && a->K > 0, MI355_E_SHAPE, "linear_int8_gemm: bad shape M=%d N=%d K=%d", a->M, a->N, a->K);
@@ -768,7 +779,8 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     ws += pad16((size_t)a->M * kp);
     float* sca = (float*)ws;
     ws += pad16((size_t)a->M * 4);
-    unsigned* mask = (unsigned*)ws;
+    MI355_CHECK_ARG(chain == nullptr || chain->words >= kp / 32, MI355_E_ARG, "linear_int8_gemm: a chain's mask of %d words for rows of %d", chain->words, a->K);
+    unsigned* mask = chain != nullptr ? chain->mask : (unsigned*)ws;
     ws += pad16((size_t)kp / 8);
     int* olist = (int*)ws;
     ws += pad16((size_t)(1 + kp) * 4);
@@ -781,8 +793,10 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     const int ksplit = cut.ksplit;
     const int64_t ldp = (int64_t)a->N * (swiglu ? 2 : 1);
     // (a kernel, not hipMemsetAsync: a caller may capture this launch, and memset nodes have replayed wrongly)
-    hipLaunchKernelGGL(i8_clear_mask_kernel, dim3((kp / 32 + 255) / 256), dim3(256), 0, s, mask, kp / 32);
-    MI355_LAUNCH_CHECK();
+    if (chain == nullptr || !chain->clear) {
+        hipLaunchKernelGGL(i8_clear_mask_kernel, dim3((kp / 32 + 255) / 256), dim3(256), 0, s, mask, kp / 32);
+        MI355_LAUNCH_CHECK();
+    }
     auto stage = [&](auto type) {
         using T = decltype(type);
         auto kernel = kp <= 1024 ? i8_stage_kernel<T, 4> : kp <= 2048 ? i8_stage_kernel<T, 8> : i8_stage_kernel<T, 16>;
@@ -820,6 +834,11 @@ extern "C" int mi355_linear_int8_gemm(const mi355_int8_args* a, void* workspace,
     p.part = part;
     p.xo = xo;
     p.so = so;
+    if (chain != nullptr) {
+        p.mask_next = chain->mask;
+        p.mask_words = chain->words;
+        chain->clear = true;
+    }
     hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), (kp / 32 < kMaskWords ? kp / 32 : kMaskWords) * kQuantLds, s, mask, ca, olist, p, a->R);
     MI355_LAUNCH_CHECK();
     if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, cut.waves, s);

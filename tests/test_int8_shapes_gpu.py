@@ -1,10 +1,12 @@
 """LLM.int8 products of many rows where their outlier columns begin and end: none, one, a block of 64 and its neighbours, columns past the first 16 384, more
 than their region holds; cut into K-slices and not."""
+import ctypes as C
+
 import pytest
 import torch
 
 from lit_llama_amd import _native as nat
-from lit_llama_amd import ops
+from lit_llama_amd import ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +58,38 @@ def test_outlier_columns(dev, M, N, K, outliers, epi):
     assert bool(((got - ref).abs() <= tol).all())
     if outliers == 0 and epi == "store":
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("T", [32, 100, 300])
+def test_a_chain_of_products_clears_the_mask_of_the_next(dev, T):
+    """A prompt's LLM.int8 products share a mask of outlier columns that each clears for the next; driven segment by segment each has its own and clears it first: the same
+    bits.  Norm scales bring some columns of every product above the threshold, others in each layer."""
+    from lit_llama_amd import LLaMA, LLaMAConfig
+    from lit_llama_amd.utils import EmptyInitOnDevice
+
+    cfg = LLaMAConfig(block_size=320, n_layer=3, n_head=4, n_embd=512, vocab_size=512)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode="llm.int8"):
+        model = LLaMA(cfg)
+    sd = synth.make_state_dict(cfg, seed=5, mode="llm.int8", device="cuda", dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(6)
+    for k in sd:
+        if k.endswith(".scale"):
+            sd[k] = (sd[k].float().cpu() * (1 + 4 * (torch.rand(512, generator=g) < 0.02))).to(torch.bfloat16).to(dev)
+    model.load_state_dict(sd)
+    model.eval()
+    eng = model.engine()
+    assert eng is not None and eng.gemm_ws is not None, model._engine_failed
+    idx = synth.make_prompt(T, vocab=512).to(dev)
+    with torch.no_grad():
+        got = [model(idx.view(1, -1), 320, torch.arange(T, device=dev))[0].clone() for _ in range(2)]
+        torch.cuda.synchronize()
+        s = eng.stream.cuda_stream
+        with torch.cuda.stream(eng.stream):
+            eng.set_step(idx.reshape(-1), T, 0)
+            nat.check(nat.lib().mi355_forward_embed(C.byref(eng.m), T, s), "embed")
+            for layer in range(cfg.n_layer):
+                nat.check(nat.lib().mi355_forward_segment(C.byref(eng.m), T, layer, 0, 4, s), "segment")
+            nat.check(nat.lib().mi355_forward_head(C.byref(eng.m), T, 2, 0, s), "head")
+        torch.cuda.synchronize()
+    want = eng.logits[:T]
+    assert torch.equal(got[0], want) and torch.equal(got[1], want)
