@@ -238,11 +238,12 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
 // leaves the fused chain's partial sums alone, which are longer); no mask if the workspace was sized for less.
 mi355_i8_chain plan_i8_chain(const mi355_model* m, int T) {
     mi355_i8_chain c = {nullptr, 0, false};
+    if (T < 32 || m->gemm_ws == nullptr) return c;
     int K = m->lm_head.K;
     for (int l = 0; l < m->n_layer; ++l)
         for (const mi355_weight* w : {&m->layers[l].attn, &m->layers[l].proj, &m->layers[l].fc, &m->layers[l].mproj}) K = w->K > K ? w->K : K;
     const size_t bytes = mi355_i8_chain_bytes(K);
-    if (T < 32 || m->gemm_ws == nullptr || (size_t)m->gemm_ws_bytes < mi355_linear_int8_gemm_workspace_bytes(T, K)) return c;
+    if ((size_t)m->gemm_ws_bytes < mi355_linear_int8_gemm_workspace_bytes(T, K)) return c;
     c.mask = (unsigned*)((char*)m->gemm_ws + (((size_t)m->gemm_ws_bytes - bytes) & ~(size_t)15));
     c.words = (int)(bytes / 4);
     return c;

@@ -1092,6 +1092,8 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // the XCD's L2 a round ahead, each a share, one lane per cache line: a block then waits for HBM once per round for its share and not for every line behind
 // every other (N = 4096, K = 11008, 777 tokens in blocks of 64 x 256 102 -> 90 us; blocks of 64 x 128 7 % less on average, of 128 x 128 4 %; 8 waves from 128 tokens on nothing).  The
 // activations likewise: 5-25 % slower, few blocks of an XCD share them.  A last block of few tokens runs ahead of the others and does it for them.
+// GRP with FUSE: a unit's operand sums are the producer's shares, the tables come from group_tables_kernel.  1000 tokens, 7B, 8 layers with a staging pass in front
+// of each product 4.59 ms, in the chain 4.31 (the products themselves 3-5 % slower: 1/rms from shares, operand and shares of the next product).
 // GRP (Q4, groups of whole 128-column units): the products of a unit start from 0, and accf += s_unit * them, one FMA per output element and unit on the
 // VALU beside the next unit's products; the zero points, accf -= sum over units of s (128 + z) X_unit (X: the unit's operand sums), are a product with K =
 // units / 4 of their own on the f32 MFMA in front of the loop.
@@ -2005,7 +2007,8 @@ void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, 
     plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
 }
 
-// The tables of several products in one launch: a prompt's layers take theirs 10 at a time (7B), 9 us, instead of 5 us and a gap in front of each
+// The tables of several products in one launch: a 7B prompt's layers take theirs 10 products at a time, 15 us (13 MB read, 13 written) instead of a launch in front of
+// each, 5 us and its gap, or with the staging pass, 10.5 to 16.6 us for rows and tables
 namespace {
 struct TableSet {
     GroupTables of[kTableProducts];

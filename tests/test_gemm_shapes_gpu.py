@@ -398,3 +398,23 @@ def test_rows_that_are_not_finite_stay_by_themselves(dev, fmt, M):
     assert torch.equal(got[others], clean[others]) and bool(clean.isfinite().all())
     if fmt != "i8":
         assert not bool(got[2].isfinite().any()) and not bool(got[M - 1].isfinite().any())
+
+
+@pytest.mark.parametrize("vocab", [512, 514])
+def test_logits_of_a_prompt_in_portions(dev, vocab):
+    """The head writes a portion's logits where they are returned; rows of 514 values put the second portion 8 bytes off a 16-byte line, which goes through the engine's
+    buffer.  A portion's products are cut by its own rows: the spread of bf16 operands against the prompt in one pass."""
+    cfg = LLaMAConfig(block_size=128, n_layer=2, n_head=4, n_embd=512, vocab_size=vocab)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16):
+        model = LLaMA(cfg)
+    model.load_state_dict(synth.make_state_dict(cfg, seed=7, mode=None, device="cuda", dtype=torch.bfloat16))
+    model.eval()
+    eng = model.engine()
+    assert eng is not None, model._engine_failed
+    idx, pos = synth.make_prompt(70, vocab=vocab).to(dev).view(1, -1), torch.arange(70, device=dev)
+    with torch.no_grad():
+        whole = model(idx, 128, pos)[0].clone()
+        model.reset_cache()
+        eng.max_T = 33
+        parts = model(idx, 128, pos)[0]
+    assert parts.shape == whole.shape and (parts - whole).abs().max() <= 0.05 * whole.std()
