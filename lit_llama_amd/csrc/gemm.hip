@@ -1713,7 +1713,7 @@ GemmForce gemm_force() {
     return f;
 }
 bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (what a sweep may force of the kernels of launch_gemm(); the other blocks of BF16 streams are the estimate's)
-    if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32);
+    if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
 }
@@ -1754,26 +1754,32 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
     if (wide >= 384 || wide == 256) cut.bm = kBM, cut.deep = false;
     return cut;
 }
-// Up to 32 tokens, outside the fused chain (whose shares are 64 or 128 rows), where blocks of 4 waves do not fill the chip: blocks of 2, 3 or 4 waves (64, 96, 128 rows).  A CU
+// Up to 64 tokens, outside the fused chain (whose shares are 64 or 128 rows), where blocks of 4 waves do not fill the chip: blocks of 2, 3 or 4 waves (64, 96, 128 rows).  A CU
 // asks for no more than its memory pipeline holds, so 129 blocks of 128 rows leave half of what HBM gives, and a slice that would fill the other CUs costs a launch; smaller
 // blocks cost their activations again.  16 tokens, 4 / 3 / 2 waves without slices: N = 16512, K = 4096 29.7 / 26.1 / 35.0 us (129, 172, 258 blocks), 12416 33.2 (24.9 in two
-// slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, a block's unit
-// taking its share of HBM too, and a launch for the slices: over 72 launches (36 products of 1024 to 32000 rows, 16 and 32 tokens, weights not in any cache) its choice
-// is 0.4 % behind the fastest, 0.909 times what blocks of 4 waves took, none slower.
+// slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, each unit of one `unit` us, `unit_wave`
+// more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Fitted to launches of 36 products of 1024 to 32000 rows, weights not in any
+// cache: 16 and 32 tokens 0.909 times what blocks of 4 waves took, 0.4 % behind the fastest, none slower; 40 and 64 tokens 0.950 times, 1.2 % behind, at most 2.6 % slower.
 GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
+    struct Cost {
+        float wave, unit, unit_wave, crowd, slices, bytes;
+    };
+    static constexpr Cost costs[] = {{0.f, 0.007f, 0.066f, 0.193f, 1.5f, 2.7e6f}, {0.25f, 0.21f, 0.023f, 0.041f, 0.3f, 2.3e6f}};  // up to 32 tokens, up to 64
+    const Cost& c = costs[M > 32];
     const int units = (K + 127) / 128;
     GemmCut cut = {4, short_block(M, true), true, 1};
     float best = 0.f;
     for (int waves = 2; waves <= 4; ++waves)
         for (int ks = 1; ks <= 8 && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget / 2)); ++ks) {
             const int blocks = gemm_blocks(M, N, pair, waves, cut.bm) * ks;
-            auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (0.007f + (float)waves * (0.066f + 0.193f * (float)of / 256.f)); };
-            const float us = (float)(blocks / 256) * round(256) + round(blocks % 256) + (ks == 1 ? 0.f : 1.5f + (float)gemm_part_bytes(M, N, pair, ks) / 2.7e6f);
+            auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (c.unit + (float)waves * (c.unit_wave + c.crowd * (float)of / 256.f)); };
+            const float us = c.wave * (float)waves + (float)(blocks / 256) * round(256) + round(blocks % 256) +
+                             (ks == 1 ? 0.f : c.slices + (float)gemm_part_bytes(M, N, pair, ks) / c.bytes);
             if (best == 0.f || us < best) best = us, cut.waves = waves, cut.ksplit = ks;
         }
     return cut;
 }
-// BF16 streams.  33 to 64 tokens (and fewer of the chain): blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
+// BF16 streams.  Up to 64 tokens of the chain: blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
 // none to a few more than all (16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 /
 // 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13); where those blocks are more than the CUs, blocks of 8 (48 tokens of the N = 17920 pair, K = 6656: 104 / 95 us with 4 / 8 waves).
 // Longer: 192 to 256 blocks of 128 tokens x 256 rows, one round of the chip, take those (3-5 % less than what the estimate takes).  Else what an estimate takes for the
@@ -1784,7 +1790,7 @@ GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
 // are those whose choice is best over 19 500 launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are): 1.7 % behind the
 // fastest of them on average, 6 % at the 90th percentile.
 GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain) {
-    if (!chain && M <= 32 && gemm_blocks(M, N, pair, 4, 32) <= 256) return bf16_cut_few(M, N, K, pair);
+    if (!chain && M <= 64 && gemm_blocks(M, N, pair, 4, 64) <= 256) return bf16_cut_few(M, N, K, pair);
     const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
     GemmCut cut = {4, short_block(M, true), true, 1};
     if (M <= 64 && few <= 256) {
@@ -1880,6 +1886,7 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
     const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE);
     if constexpr (FMT == MI355_W_BF16 && !FUSE) {
         // (operand slices start at multiples of 256 rows: blocks of 64 divide them, of 96 not)
+        if (sh.waves <= 3 && sh.bm == 64) return sh.waves == 3 && p.slice_blocks == 0 ? launch_deep<EPI, PAIR, FMT, 3, 64, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
         if (sh.waves == 3 && p.slice_blocks == 0) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
         if (sh.waves <= 3) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
     }

@@ -301,7 +301,7 @@ def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T
 
 
 @pytest.mark.parametrize("epi", ["store", "pair", "accum"])
-@pytest.mark.parametrize("M", [5, 16, 17, 32])
+@pytest.mark.parametrize("M", [5, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(64, 128), (68, 1000), (96, 4096), (100, 640), (4096, 2048), (8200, 384), (12352, 1024), (16512, 512)])
 def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
     """Block edges at 64, 96 and 128 rows, slices, a last unit that is not whole.  The bound of the tiled product."""
