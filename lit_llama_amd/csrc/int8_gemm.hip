@@ -70,8 +70,10 @@ struct I8GemmParams {
     int y_dtype;
     // split-K for short prompts (a 128-token prompt is ONE token block: 16 workgroups for N = 4096): MODE 1 launches
     // total_blocks x ksplit workgroups that store their int32 partial tiles to part[ks][M][ldp]; MODE 2 (total_blocks
-    // workgroups) sums them — integer sums: exact in any order — and runs the epilogue
+    // workgroups) sums them — integer sums: exact in any order — and runs the epilogue.  Sums move four columns at a time: a row has ldn = N rounded up to four of
+    // them, and a pair's c_fc2 starts at ldn
     int ksplit;
+    int ldn;
     int64_t ldp;
     int* part;
     // the outlier columns by themselves (i8_quant_kernel): xo[m][ld], so[(tile R + r) 16 + row][ld] = f16(CB SCB / 127), ld = compact_ld(n_out) (whole units of 64), columns past
@@ -465,14 +467,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
                 for (int t = 0; t < kTPW; ++t) {
                     const int n = tile[t] * 16 + 4 * g;
                     if (tile[t] < p.n_tiles && n < p.N)
-                        *(f32x4*)((float*)p.part + ((int64_t)ks * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n) = o[t][tt];
+                        *(f32x4*)((float*)p.part + ((int64_t)ks * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.ldn : 0) + n) = o[t][tt];
                 }
             }
             return;
         }
     }
     if constexpr (MODE != 2) run_units(std::false_type{}, acc, u_lo, u_hi, rw, rx, (int64_t)p.Kp);
-    // partial tiles of a K-slice: column n of c_fc2 sits at N + n
+    // partial tiles of a K-slice: column n of c_fc2 sits at ldn + n
     if constexpr (MODE == 1) {
 #pragma unroll
         for (int tt = 0; tt < 8; ++tt) {
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
             for (int t = 0; t < kTPW; ++t) {
                 const int n = tile[t] * 16 + 4 * g;
                 if (tile[t] < p.n_tiles && n < p.N)
-                    *(i32x4*)(p.part + ((int64_t)ks * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n) = acc[t][tt];
+                    *(i32x4*)(p.part + ((int64_t)ks * p.M + m) * p.ldp + (PAIR && rr[t] == 1 ? p.ldn : 0) + n) = acc[t][tt];
             }
         }
         return;
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
 #pragma unroll
         for (int t = 0; t < kTPW; ++t) {
             const int n = tile[t] * 16 + 4 * g;
-            const int* at = p.part + (m < p.M && tile[t] < p.n_tiles && n < p.N ? (int64_t)m * p.ldp + (PAIR && rr[t] == 1 ? p.N : 0) + n : 0);
+            const int* at = p.part + (m < p.M && tile[t] < p.n_tiles && n < p.N ? (int64_t)m * p.ldp + (PAIR && rr[t] == 1 ? p.ldn : 0) + n : 0);
             i32x4 v[kMaxSplit];
 #pragma unroll
             for (int s2 = 0; s2 < kMaxSplit; ++s2) v[s2] = *(const i32x4*)(at + (s2 < p.ksplit ? s2 : 0) * ((int64_t)p.M * p.ldp));
@@ -707,13 +709,14 @@ int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
 struct I8Cut {
     int waves, ksplit;
 };
+int i8_part_columns(int N) { return (N + 3) & ~3; }
 I8Cut i8_cut(int M, int N, int units, bool pair) {
     struct Kind {
         int waves;
         float start, unit, crowd;
     };
     static constexpr Kind kinds[] = {{4, 2.9f, 0.513f, 0.036f}, {8, 2.9f, 0.626f, 0.381f}};
-    const size_t part = (size_t)M * N * (pair ? 2 : 1) * 4;  // bytes of one slice's sums
+    const size_t part = (size_t)M * i8_part_columns(N) * (pair ? 2 : 1) * 4;  // bytes of one slice's sums
     I8Cut cut = {8, 1};
     float best = 0.f;
     for (const Kind& k : kinds)
@@ -791,7 +794,7 @@ int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* cha
     f16_t* so = (f16_t*)ws;
     const I8Cut cut = i8_cut(a->M, a->N, units, swiglu);
     const int ksplit = cut.ksplit;
-    const int64_t ldp = (int64_t)a->N * (swiglu ? 2 : 1);
+    const int ldn = i8_part_columns(a->N);
     // (a kernel, not hipMemsetAsync: a caller may capture this launch, and memset nodes have replayed wrongly)
     if (chain == nullptr || !chain->clear) {
         hipLaunchKernelGGL(i8_clear_mask_kernel, dim3((kp / 32 + 255) / 256), dim3(256), 0, s, mask, kp / 32);
@@ -830,7 +833,8 @@ int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* cha
     p.n_tiles = (a->N + 15) / 16;
     p.y_dtype = a->y_dtype;
     p.ksplit = ksplit;
-    p.ldp = ldp;
+    p.ldn = ldn;
+    p.ldp = (int64_t)ldn * (swiglu ? 2 : 1);
     p.part = part;
     p.xo = xo;
     p.so = so;
