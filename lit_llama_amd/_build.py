@@ -42,6 +42,11 @@ def _stale(target: Path, deps) -> bool:
     return any(Path(d).stat().st_mtime > t for d in deps)
 
 
+def headers_of_sources():
+    """What an object is older than counts as changed: every header of the sources (two of them that disagree about a struct would link)."""
+    return [*sorted(CSRC.glob("*.h")), PKG.parent / "include" / "mi355_llama.h"]
+
+
 def build_core(force: bool = False, verbose: bool = True) -> Path:
     """The part of the library that a layered hybrid model needs (a fresh checkout that serves one compiles no more)."""
     return build(force, verbose, CORE_SOURCES, CORE_LIB)
@@ -51,7 +56,7 @@ def build(force: bool = False, verbose: bool = True, sources=None, lib: Path = L
     sources = SOURCES if sources is None else sources
     hipcc = _hipcc()
     OBJ_DIR.mkdir(exist_ok=True)
-    headers = [CSRC / "common.h", CSRC / "fused_step_common.h", CSRC / "gemm_fuse.h", CSRC / "recurrent.h", CSRC / "product.h", PKG.parent / "include" / "mi355_llama.h"]
+    headers = headers_of_sources()
     flags = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", *NO_PACKED_F32]
 
     def compile_one(name: str):

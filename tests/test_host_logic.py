@@ -689,3 +689,14 @@ def test_prompt_scratch_holds_what_the_formats_need():
         assert prompt_workspace_bytes(kinds, 2048, 11008) == gemm
     assert prompt_workspace_bytes({"i8"}, 2048, 11008) == i8
     assert prompt_workspace_bytes({"i8", "bf16"}, 2048, 11008) == max(gemm, i8)
+
+
+def test_objects_follow_every_header_that_a_source_includes():
+    import re
+
+    from lit_llama_amd import _build
+
+    watched = {h.resolve() for h in _build.headers_of_sources()}
+    for f in [*_build.CSRC.glob("*.hip"), *_build.CSRC.glob("*.h")]:
+        for name in re.findall(r'^#include "([^"]+)"', f.read_text(), re.M):
+            assert any((d / name).resolve() in watched for d in (f.parent, _build.PKG.parent / "include")), (f.name, name)
