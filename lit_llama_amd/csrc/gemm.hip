@@ -30,6 +30,7 @@
 
 #include "common.h"
 #include "gemm_fuse.h"
+#include "l2_share.h"
 
 // The epilogues' conversions on the hardware paths (with IEEE division + expf in SiLU and the six-instruction software rounding
 // the c_fc1 / c_fc2 epilogue was VALU-bound — 33 us of a 269-us launch at T = 2048 against 9 us for its 45 MB of stores,
@@ -1143,11 +1144,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     constexpr unsigned kNone = 0xFFFFFFF0u;
     [[maybe_unused]] unsigned touch_off = kNone;
     if constexpr (kTouch) {
-        const int first = xcd * p.per_xcd, last = first + p.per_xcd - 1;
-        const int lo = nb * m_blocks > first ? nb * m_blocks : first, hi = (nb + 1) * m_blocks - 1 < last ? (nb + 1) * m_blocks - 1 : last;
-        const int touch_n = hi - lo + 1, share = (kStreams * kRun + touch_n - 1) / touch_n;
-        const int line = (L - lo) * share + (int)threadIdx.x, stream = line / kRun, at = line - stream * kRun;
-        if (p.ksplit == 1 && touch_n >= 4 && (p.M - 1) % BM >= BM / 2 && (int)threadIdx.x < share && line < kStreams * kRun && nb * kStreams + stream < p.n_tiles)
+        const L2Share mine = l2_share(kStreams * kRun, L, nb, m_blocks, p.ksplit, xcd, p.per_xcd);
+        const int line = mine.first + (int)threadIdx.x, stream = line / kRun, at = line - stream * kRun;
+        if ((p.M - 1) % BM >= BM / 2 && (int)threadIdx.x < mine.count && line < kStreams * kRun && nb * kStreams + stream < p.n_tiles)
             touch_off = (unsigned)((nb * kStreams + stream) * p.units) * (PAIR ? 8192u : 4096u) + at * 128u;
     }
     [[maybe_unused]] const bool touching = __builtin_amdgcn_ballot_w64(touch_off != kNone) != 0;

@@ -700,3 +700,44 @@ def test_objects_follow_every_header_that_a_source_includes():
     for f in [*_build.CSRC.glob("*.hip"), *_build.CSRC.glob("*.h")]:
         for name in re.findall(r'^#include "([^"]+)"', f.read_text(), re.M):
             assert any((d / name).resolve() in watched for d in (f.parent, _build.PKG.parent / "include")), (f.name, name)
+
+
+def test_shares_of_a_row_blocks_weights(tmp_path):
+    """csrc/l2_share.h, built for the host with division checked: the blocks of a row block on one XCD bring each of its lines once, no share is longer than the smallest
+    workgroup that takes one (4 waves, 1024 lines), and a launch in K-slices, whose places on an XCD count slices, asks for none."""
+    import subprocess
+
+    from lit_llama_amd import _build
+
+    (tmp_path / "t.cpp").write_text(r"""
+#define __host__
+#define __device__
+#include "l2_share.h"
+#include <cstdio>
+#include <vector>
+int main() {
+    const int lines = 1024;
+    for (int ks = 1; ks <= 16; ++ks)
+        for (int n_blocks : {1, 2, 5, 16, 33, 129})
+            for (int m_blocks : {1, 3, 4, 5, 8, 13, 31, 64}) {
+                const int total = n_blocks * m_blocks * ks, per_xcd = (total + 7) / 8;
+                for (int xcd = 0; xcd < 8; ++xcd) {
+                    std::vector<std::vector<int>> brought(n_blocks, std::vector<int>(lines));
+                    std::vector<int> here(n_blocks);
+                    for (int at = xcd * per_xcd; at < (xcd + 1) * per_xcd && at < total; ++at) {
+                        const int L = at / ks, nb = L / m_blocks;
+                        const L2Share s = l2_share(lines, L, nb, m_blocks, ks, xcd, per_xcd);
+                        if (s.count < 0 || s.count > 256 || (ks > 1 && s.count != 0)) return std::printf("share of %d lines, %d slices", s.count, ks), 1;
+                        here[nb]++;
+                        for (int i = s.first; i < s.first + s.count && i < lines; ++i) brought[nb].at(i)++;
+                    }
+                    for (int nb = 0; ks == 1 && nb < n_blocks; ++nb)
+                        for (int n : brought[nb])
+                            if (n != (here[nb] >= 4)) return std::printf("a line %d times, %d blocks", n, here[nb]), 1;
+                }
+            }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-fsanitize=integer-divide-by-zero", "-fno-sanitize-recover=all", f"-I{_build.CSRC}", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")], check=True)
+    r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
