@@ -1696,8 +1696,8 @@ struct GemmCut {
     bool deep;
     int ksplit;
 };
-// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep, int4: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel), 0 = the rule's choice.  A cut that no kernel is
-// instantiated for is ignored as a whole, a number of slices that does not fit by itself
+// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel, the latter int4 only), 0 = the rule's choice.  A cut that
+// no kernel is instantiated for is ignored as a whole, a number of slices that does not fit by itself; blocks that only BF16 streams have need the kernel named (deep = 1)
 struct GemmForce {
     int waves, bm, ksplit, deep;
 };
@@ -1711,7 +1711,8 @@ GemmForce gemm_force() {
     }();
     return f;
 }
-bool launch_gemm_has(const GemmCut& c, bool bf16) {  // (what a sweep may force of the kernels of launch_gemm(); the other blocks of BF16 streams are the estimate's)
+bool launch_gemm_has(const GemmCut& c, bool bf16, bool named) {  // (what a sweep may force of the kernels of launch_gemm())
+    if (bf16 && named && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 192 || c.bm == 256)))) return true;
     if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
@@ -1839,8 +1840,8 @@ GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain) {
     const GemmForce fo = gemm_force();
     GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain) : q4_cut(M, N, K, pair);
     const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep == 1 : cut.deep, cut.ksplit};
-    if (launch_gemm_has(forced, bf16) && (!chain || forced.waves >= 4)) cut = forced;
-    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= kSplitBudget / 2) cut.ksplit = fo.ksplit;
+    if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4)) cut = forced;
+    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) cut.ksplit = fo.ksplit;
     return cut;
 }
 // Grouped scales, groups of whole units.  Blocks of 256 rows x 64 tokens and of 256 x 128 fill a CU alone, two of 128 x 64 share one; per round of the chip
@@ -1863,7 +1864,7 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
             sh.waves = 8;
     }
     const GemmCut forced = {fo.waves ? fo.waves : sh.waves, fo.bm ? fo.bm : sh.bm, true, ksplit};
-    return launch_gemm_has(forced, false) ? forced : sh;
+    return launch_gemm_has(forced, false, false) ? forced : sh;
 }
 // Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
 // product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows

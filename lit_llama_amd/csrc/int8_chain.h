@@ -10,5 +10,7 @@ struct mi355_i8_chain {
     int words;       // of the longest row
     bool clear;      // the mask is zero once the launches so far are done
 };
+// how a launch is cut: waves of a block, K-slices
+extern "C" void mi355_linear_int8_gemm_plan(int M, int N, int K, int R, int* waves, int* ksplit);
 size_t mi355_i8_chain_bytes(int K);
 int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* chain, void* workspace, size_t workspace_bytes, mi355_stream_t stream);

@@ -21,6 +21,9 @@
 // 108 -> 83, attn.c_proj / mlp.c_proj slices 48 -> 35 and their sum 151 -> 15 us on average.
 #include <type_traits>
 
+#include <stdio.h>
+#include <stdlib.h>
+
 #include "common.h"
 #include "int8_chain.h"
 
@@ -729,6 +732,16 @@ I8Cut i8_cut(int M, int N, int units, bool pair) {
             const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 3.1f + (float)(part * ks) / 1.61e6f);
             if (best == 0.f || us < best) best = us, cut = {k.waves, ks};
         }
+    struct Force {
+        int waves, bm, ksplit;
+    };
+    static const Force fo = [] {  // (sweeps: MI355_GEMM_FORCE as in csrc/gemm.hip)
+        Force f = {0, 0, 0};
+        if (const char* e = getenv("MI355_GEMM_FORCE")) sscanf(e, "%d:%d:%d", &f.waves, &f.bm, &f.ksplit);
+        return f;
+    }();
+    if ((fo.waves == 4 || fo.waves == 8) && (fo.bm == 0 || fo.bm == kBM)) cut.waves = fo.waves;
+    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && units >= 4 * fo.ksplit && part * fo.ksplit <= kSplitBudget) cut.ksplit = fo.ksplit;
     return cut;
 }
 template <int EPI, bool PAIR>
@@ -750,6 +763,10 @@ extern "C" size_t mi355_linear_int8_gemm_workspace_bytes(int M, int K) {
            kPartBytes +                                      // partial tiles of the split-K launches (short prompts)
            pad16((size_t)M * kp * 2) + kOutlierBudget +      // outlier columns by themselves: of the rows, of the weights
            mi355_i8_chain_bytes(K);                          // the mask of a chain of products
+}
+extern "C" void mi355_linear_int8_gemm_plan(int M, int N, int K, int R, int* waves, int* ksplit) {
+    const I8Cut cut = i8_cut(M, N, (K + 127) / 128, R == 2);
+    *waves = cut.waves, *ksplit = cut.ksplit;
 }
 size_t mi355_i8_chain_bytes(int K) { return pad16(((size_t)K + 127) / 128 * 16); }
 

@@ -680,6 +680,26 @@ def test_a_forced_cut_without_a_kernel_changes_nothing():
     assert _forced_plans("8:128:0") != rule
 
 
+def test_every_block_of_the_estimates_can_be_forced():
+    """Blocks that only BF16 streams have, by their kernel's name (the last field); LLM.int8 cuts answer to the same variable."""
+    rule = _forced_plans("")
+    for block in ("4:96", "4:128", "8:192", "8:256"):
+        assert _forced_plans(block + ":3:1") != rule and _forced_plans(block + ":0") == rule, block
+        q4 = [[line for line in out.splitlines() if "False" in line] for out in (_forced_plans(block + ":0:1"), rule)]
+        assert q4[0] == q4[1], block
+    import os
+    import subprocess
+    import sys
+
+    code = ("import ctypes as C, sys\n"
+            "w, k = C.c_int(0), C.c_int(0)\n"
+            "C.CDLL(sys.argv[1]).mi355_linear_int8_gemm_plan(100, 4096, 4096, 1, C.byref(w), C.byref(k))\n"
+            "print(w.value, k.value)\n")
+    for force, want in (("8:0:5", "8 5"), ("4:128:2", "4 2"), ("4:0:1", "4 1")):
+        out = subprocess.run([sys.executable, "-c", code, str(nat.LIB_PATH)], env={**os.environ, "MI355_GEMM_FORCE": force}, capture_output=True, text=True)
+        assert out.returncode == 0 and out.stdout.strip() == want, (force, out.stdout, out.stderr)
+
+
 def test_prompt_scratch_holds_what_the_formats_need():
     from lit_llama_amd.engine import prompt_workspace_bytes
 
