@@ -705,10 +705,14 @@ int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
     MI355_LAUNCH_CHECK();
     return 0;
 }
-// How a launch is cut: blocks of 128 tokens x 256 rows (8 waves, a CU each) or x 128 (4 waves, two to a CU), and K-slices, which are a sum and its launch more; what an
-// estimate takes for the fastest, as for the bf16 stream (csrc/gemm.hip: bf16_cut()).  Its constants are those whose choice is best over 1700 launches (18 products
-// of 2048 to 32000 rows, 33 to 2048 tokens, weights not in any cache): 1.1 % behind the fastest of them on average, 3 % at the 90th percentile.  Blocks of 8 waves throughout and
-// slices for launches of less than 96 of them: N = K = 4096, 128 tokens 31.0 us (now 28.3), 512 44.8 (34.3); N = 12288, 128 tokens 46.5 (37.6)
+// How a launch is cut: blocks of 128 tokens x 256 rows (8 waves) or x 128 (4 waves), and K-slices, which are a sum and its launch more; what an estimate takes for the
+// fastest.  A launch in K-slices has one slice's workgroups more for the outlier columns, and a CU that gets one of them runs it beside or behind its other work: 64
+// blocks of 4 waves (N = K = 8192, 33 tokens) take 44.7 / 39.5 / 34.2 / 41.3 / 38.1 us with 1 / 2 / 3 / 4 / 5 slices, since 4 are 320 workgroups and not 256.  So: the
+// rounds of the chip, each the units of a slice or the launch's share of the weights from HBM, whichever is longer (a root of squares), and for slices a launch and the
+// sums' way to memory and back.  How many outlier columns there are is on the device; the constants are those whose choice is best over 2688 launches (32 products of
+// 768 to 32000 rows, 32 to 2048 tokens, 0, 0.3, 2 and 10 % of the columns, weights not in any cache: profiles/product_cuts_int8.txt): 0.5 % behind the fastest on average, 2 %
+// at the 90th percentile; with the outliers' workgroups left out 1.6 % and 5 %, and N = 5120, K = 13824, 256 tokens 79 us (now 66).  Blocks of 8 waves throughout and
+// slices for launches of less than 96 of them: 1.23 times as long on average, none more than 2.5 % shorter
 struct I8Cut {
     int waves, ksplit;
 };
@@ -716,20 +720,20 @@ int i8_part_columns(int N) { return (N + 3) & ~3; }
 I8Cut i8_cut(int M, int N, int units, bool pair) {
     struct Kind {
         int waves;
-        float start, unit, crowd;
+        float start, unit;
     };
-    static constexpr Kind kinds[] = {{4, 2.9f, 0.513f, 0.036f}, {8, 2.9f, 0.626f, 0.381f}};
+    static constexpr Kind kinds[] = {{4, 0.21f, 0.436f}, {8, 0.737f, 0.763f}};
     const size_t part = (size_t)M * i8_part_columns(N) * (pair ? 2 : 1) * 4;  // bytes of one slice's sums
     I8Cut cut = {8, 1};
     float best = 0.f;
     for (const Kind& k : kinds)
         for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && part * ks <= kSplitBudget)); ++ks) {
-            const int rows = 16 * k.waves * kTPW / (pair ? 2 : 1), blocks = (N + rows - 1) / rows * ((M + kBM - 1) / kBM) * ks, units_of = (units + ks - 1) / ks;
+            const int rows = 16 * k.waves * kTPW / (pair ? 2 : 1), blocks = (N + rows - 1) / rows * ((M + kBM - 1) / kBM) * (ks == 1 ? 1 : ks + 1);
             auto round = [&](int of) {
-                const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), hbm = 128.f * units * N * (pair ? 2 : 1) / 1.63e6f * (float)of / (float)blocks;
+                const float work = (float)((units + ks - 1) / ks) * k.unit, hbm = 0.557f + 128.f * units * N * (pair ? 2 : 1) / 2.03e6f * (float)of / (float)blocks;
                 return sqrtf(work * work + hbm * hbm);
             };
-            const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 3.1f + (float)(part * ks) / 1.61e6f);
+            const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 3.19f + (float)(part * ks) / 2.29e6f);
             if (best == 0.f || us < best) best = us, cut = {k.waves, ks};
         }
     struct Force {

@@ -1,6 +1,8 @@
 """Host-side logic on CPU: drop-in module contract (ctor signatures, buffers, state-dict keys, layouts), the
 `quantization()` selector, format utilities against the reference's golden vectors, synthetic checkpoints, and the
 rule that the product path refuses to compute off-GPU (no silent CPU fallback)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -698,6 +700,16 @@ def test_every_block_of_the_estimates_can_be_forced():
     for force, want in (("8:0:5", "8 5"), ("4:128:2", "4 2"), ("4:0:1", "4 1")):
         out = subprocess.run([sys.executable, "-c", code, str(nat.LIB_PATH)], env={**os.environ, "MI355_GEMM_FORCE": force}, capture_output=True, text=True)
         assert out.returncode == 0 and out.stdout.strip() == want, (force, out.stdout, out.stderr)
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 5120, 13824), (256, 5120, 13824), (33, 8192, 8192), (65, 6656, 17920)])
+def test_int8_slices_leave_room_for_the_outlier_columns(M, N, K):
+    """The workgroups of the outlier columns, one slice's more, are counted: slices of few blocks stay within the 256 CUs (200 tokens, N = 5120, K = 13824:
+    73 us with 320 workgroups, 62 with 240)."""
+    w, k = C.c_int(0), C.c_int(0)
+    nat.lib().mi355_linear_int8_gemm_plan(M, N, K, 1, C.byref(w), C.byref(k))
+    blocks = -(-N // (32 * w.value)) * -(-M // 128)
+    assert k.value == 1 or blocks * (k.value + 1) <= 256, (w.value, k.value)
 
 
 def test_prompt_scratch_holds_what_the_formats_need():
