@@ -1779,61 +1779,67 @@ GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
         }
     return cut;
 }
-// BF16 streams.  Up to 64 tokens of the chain: blocks of 4 waves, with as many slices as bring them to three quarters of the CUs and
-// none to a few more than all (16 rows, N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 /
-// 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13); where those blocks are more than the CUs, blocks of 8 (48 tokens of the N = 17920 pair, K = 6656: 104 / 95 us with 4 / 8 waves).
-// Longer: 192 to 256 blocks of 128 tokens x 256 rows, one round of the chip, take those (3-5 % less than what the estimate takes).  Else what an estimate takes for the
-// fastest: the rounds of the chip one behind the other, each the busiest CU's units (`unit` us when it is alone, `crowd` more when every CU has a block, whatever of the
-// block is padding) and its share of the bytes at once; slices cost a launch, and their sums' way to memory and back.  Blocks of 192 and 256 tokens x 256 rows ask
-// for 75 and 64 KB per 8.4 MFLOP instead of the 96 of 128 x 256, and give the rounds more sizes to fit: 2048 tokens, N = 16512, K = 4096, 4.1 rounds of 128 tokens 278 us, 2.8 of
-// 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  The constants
-// are those whose choice is best over 19 500 launches (34 products of 2048 to 36864 rows, 66 to 2048 tokens, weights not in any cache: the next layer's never are): 1.7 % behind the
-// fastest of them on average, 6 % at the 90th percentile.
-GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain) {
-    if (!chain && M <= 64 && gemm_blocks(M, N, pair, 4, 64) <= 256) return bf16_cut_few(M, N, K, pair);
-    const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64), wide = gemm_blocks(M, N, pair, 8, kBM);
+// Up to 64 tokens in the chain, blocks of 4 waves no more than the CUs: as many slices as bring them to three quarters of the CUs and none to a few more than all (16 rows,
+// N = 16512, K = 4096, 129 blocks: 30.1 / 38.8 / 32.2 / 36.3 us with 1 / 2 / 3 / 4; K = 11008, N = 4096, 32 blocks 24.2 / 21.9 / 21.3 / 21.9 / 23.2 with 4 / 5 / 6 / 8 / 13).
+GemmCut bf16_cut_few_chained(int M, int N, int K, bool pair) {
+    const int units = (K + 127) / 128, few = gemm_blocks(M, N, pair, 4, 64);
     GemmCut cut = {4, short_block(M, true), true, 1};
-    if (M <= 64 && few <= 256) {
-        while (cut.ksplit < kMaxSplit && few * cut.ksplit < 192 && few * (cut.ksplit + 1) <= 256 && units >= 4 * (cut.ksplit + 1) &&
-               gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
-            ++cut.ksplit;
-        return cut;
-    }
-    if (M > 64 && wide >= 192 && wide <= 256) return {8, kBM, true, 1};
+    while (cut.ksplit < kMaxSplit && few * cut.ksplit < 192 && few * (cut.ksplit + 1) <= 256 && units >= 4 * (cut.ksplit + 1) &&
+           gemm_part_bytes(M, N, pair, cut.ksplit + 1) <= kSplitBudget / 2)
+        ++cut.ksplit;
+    return cut;
+}
+// Up to 64 tokens, blocks of 4 waves more than the CUs: the weights bound them, 6.6 TB/s behind 4.3 us, beside the busiest CU's units (48 tokens of the N = 17920 pair, K = 6656: 104 /
+// 95 us with 4 / 8 waves).
+GemmCut bf16_cut_many(int M, int N, int K, bool pair) {
+    struct Kind {
+        int waves, bm;
+        float start, unit;
+    };
+    const int units = (K + 127) / 128, bm = short_block(M, true);
+    const Kind kinds[] = {{4, bm, bm == 16 ? 0.9f : bm == 32 ? 1.3f : 3.0f, bm == 16 ? 0.67f : bm == 32 ? 0.71f : 0.75f}, {8, 64, 3.4f, 1.23f}};
+    const float bytes = 2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N, hbm = 4.3f + bytes / 6.6e6f;
+    GemmCut cut = {4, bm, true, 1};
+    float best = 0.f;
+    for (const Kind& k : kinds)
+        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget * 3 / 4)); ++ks) {
+            const float work = k.start + (float)((gemm_blocks(M, N, pair, k.waves, k.bm) * ks + 255) / 256 * ((units + ks - 1) / ks)) * k.unit;
+            const float us = sqrtf(work * work + hbm * hbm) + (ks == 1 ? 0.f : 1.6f + (float)gemm_part_bytes(M, N, pair, ks) / 2.3e6f);
+            if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, true, ks};
+        }
+    return cut;
+}
+// From 65 tokens on: what an estimate takes for the fastest, a start and the rounds of the chip one behind the other, each the units of a slice, `unit` us when a CU is alone with its
+// block and `crowd` more when every CU has one, whatever of a block is padding; slices cost their sums' way to memory and back, no less than a launch.  Blocks of 192 and 256 tokens x 256
+// rows ask for 75 and 64 KB per 8.4 MFLOP instead of the 96 of 128 x 256, and give the rounds more sizes to fit: 2048 tokens, N = 16512, K = 4096, 4.1 rounds of 128 tokens 278 us, 2.8 of
+// 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  The constants are
+// those whose choice is best over 1078 launches (41 products of 512 to 32000 rows, 65 to 2048 tokens; those below 20 MB with their weights in the 256-MB cache and without, the others
+// without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.6 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
+// a launch as the least that slices cost, 1.6 % and 5.4 %: short rows were cut (512 tokens, N = K = 2048 16.1 us in two slices, 12.7 whole; 96 of the N = 2816 pair, K = 1024 11.6, 8.2).
+GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
     struct Kind {
         int waves, bm;
         float start, unit, crowd;
     };
-    // (up to 64 tokens, more blocks than CUs: the weights bound them)
-    const Kind few_tokens[] = {{4, cut.bm, cut.bm == 16 ? 0.9f : cut.bm == 32 ? 1.3f : 3.0f, cut.bm == 16 ? 0.67f : cut.bm == 32 ? 0.71f : 0.75f, 0.f}, {8, 64, 3.4f, 1.23f, 0.f}};
-    static constexpr Kind kinds[] = {{4, 64, 1.8f, 0.539f, 0.147f},   {4, 96, 4.2f, 0.507f, 0.237f},   {4, kBM, 3.1f, 0.746f, 0.237f}, {8, 64, 7.8f, 0.766f, 0.219f},
-                                     {8, kBM, 6.4f, 0.988f, 0.321f}, {8, 192, 9.7f, 1.274f, 0.424f}, {8, 256, 4.2f, 1.52f, 0.871f}};
-    const float bytes = 2.f * N * K * (pair ? 2 : 1) + 2.f * M * K + 4.f * M * N;
+    static constexpr Kind kinds[] = {{4, 64, 2.744f, 0.518f, 0.181f},  {4, 96, 4.059f, 0.484f, 0.333f},   {4, kBM, 2.751f, 0.78f, 0.272f},  {8, 64, 6.209f, 0.684f, 0.474f},
+                                     {8, kBM, 8.323f, 0.926f, 0.424f}, {8, 192, 11.38f, 1.231f, 0.501f}, {8, 256, 9.51f, 1.344f, 1.146f}};
+    const int units = (K + 127) / 128;
+    GemmCut cut = {4, 64, true, 1};
     float best = 0.f;
-    auto estimate = [&](const Kind& k, int ks) {
-        const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks, units_of = (units + ks - 1) / ks;
-        const float part = ks == 1 ? 0.f : (float)gemm_part_bytes(M, N, pair, ks);
-        if (M <= 64) {
-            const float work = k.start + (float)((blocks + 255) / 256 * units_of) * k.unit, hbm = 4.3f + bytes / 6.6e6f;
-            return sqrtf(work * work + hbm * hbm) + (ks == 1 ? 0.f : 1.6f + part / 2.3e6f);
-        }
-        auto round = [&](int of) {  // a round of `of` blocks
-            const float work = units_of * (k.unit + k.crowd * (float)of / 256.f), hbm = 0.16f + bytes / 23.8e6f * (float)of / (float)blocks;
-            return sqrtf(work * work + hbm * hbm);
-        };
-        return k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 0.8f + part / 3.38e6f);
-    };
-    auto consider = [&](const Kind& k) {
+    for (const Kind& k : kinds)
         for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget * 3 / 4)); ++ks) {
-            const float us = estimate(k, ks);
+            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks;
+            auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (k.unit + k.crowd * (float)of / 256.f); };
+            float us = k.start + (float)(blocks / 256) * round(256) + round(blocks % 256);
+            if (ks > 1) us += fmaxf(0.976f + (float)gemm_part_bytes(M, N, pair, ks) / 2.486e6f, 2.17f);
             if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, true, ks};
         }
-    };
-    if (M <= 64)
-        for (const Kind& k : few_tokens) consider(k);
-    else
-        for (const Kind& k : kinds) consider(k);
     return cut;
+}
+GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain) {
+    if (M > 64) return bf16_cut_long(M, N, K, pair);
+    if (gemm_blocks(M, N, pair, 4, 64) > 256) return bf16_cut_many(M, N, K, pair);
+    return chain ? bf16_cut_few_chained(M, N, K, pair) : bf16_cut_few(M, N, K, pair);
 }
 // chain: a launch of the fused prompt chain (gemm_fuse.h)
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain) {
@@ -2009,6 +2015,10 @@ void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares,
 }  // namespace
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
     plan_shares(gemm_cut(M, N, K, R == 2, bf16, true), N, R == 2, ksplit, shares, shares_per_unit);
+}
+extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, int* waves, int* tokens, int* ksplit) {
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain);
+    *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
     plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);

@@ -655,6 +655,19 @@ def test_partial_sums_of_slices_fit_their_buffer(bf16):
             assert (ks == 1 or ppu == 1) and shares * 128 >= N * ppu
 
 
+def _gemm_cut(M, N, K, R, chain):
+    out = [C.c_int(0) for _ in range(3)]
+    nat.lib().mi355_linear_gemm_cut(M, N, K, R, C.c_bool(True), C.c_bool(chain), *[C.byref(v) for v in out])
+    return tuple(v.value for v in out)
+
+
+@pytest.mark.parametrize("M,N,K,R", [(512, 1024, 1024, 1), (512, 2048, 2048, 1), (450, 1024, 1024, 1), (150, 3072, 1024, 1), (65, 2816, 1024, 2), (96, 2816, 1024, 2)])
+def test_short_bf16_rows_are_not_cut_along_k(M, N, K, R):
+    """Each of these took 1.15 to 1.46 times as long in two slices, whose sum is a launch more, as whole."""
+    for chain in (False, True):
+        assert _gemm_cut(M, N, K, R, chain) == (4, 64, 1)
+
+
 def _forced_plans(value):
     """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
     import os
