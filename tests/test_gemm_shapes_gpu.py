@@ -79,14 +79,19 @@ def test_int4_sums_beside_a_large_activation(dev, M, N, K, run):
     assert (got - ref).square().mean().sqrt() <= 1.06 * (4 * run * 5 / 12) ** 0.5 * last_bit
 
 
-@pytest.mark.parametrize("M,N,K,pair", [
+BF16_BLOCKS = [
     (512, 4096, 1664, 0), (257, 12288, 1664, 0), (257, 1000, 1664, 0), (449, 4112, 1664, 0), (512, 4112, 1664, 0), (193, 12288, 2176, 0), (500, 6160, 640, 0),
     (320, 12288, 2176, 0), (512, 12288, 640, 0), (1025, 6160, 256, 0), (769, 12288, 2176, 0), (1281, 6160, 2176, 0), (1281, 8200, 256, 0), (1025, 12288, 2048, 0),
     (512, 1000, 2176, 1), (193, 4112, 1664, 1), (320, 4112, 1664, 1), (320, 6160, 2176, 1), (641, 4112, 384, 1), (1281, 4096, 2176, 1), (449, 12288, 2048, 1), (1281, 12288, 128, 1),
-])
+    (600, 12288, 1152, 0), (600, 11012, 1664, 1), (70, 4100, 2176, 0), (129, 4100, 4224, 0), (66, 4100, 3200, 0), (300, 4096, 11008, 0), (135, 11012, 8448, 0),
+    (70, 2816, 1664, 1), (70, 4100, 2176, 1), (66, 2052, 3200, 1), (129, 11012, 4224, 1),
+]
+
+
+@pytest.mark.parametrize("M,N,K,pair", BF16_BLOCKS)
 def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
-    """Blocks of 64 / 96 / 128 tokens x 4 waves and 64 / 128 / 192 / 256 x 8 (in this order above, pairs behind): a few tokens or rows more than whole blocks, rounds of units that
-    end early, row blocks that share an XCD and such that are cut between two.  Bounds: as in test_tiled_product_against_64_bits."""
+    """Blocks of 64 / 96 / 128 tokens x 4 waves and 64 / 128 / 192 / 256 x 8, whole rows and K-slices, pairs too (tests/test_host_logic.py compares the list with the rule): a few
+    tokens or rows more than whole blocks, rounds of units that end early, row blocks that share an XCD and such that are cut between two.  Bounds: as in test_tiled_product_against_64_bits."""
     g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
     x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
     mats = [(torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16) for _ in range(1 + pair)]
@@ -103,10 +108,17 @@ def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
-@pytest.mark.parametrize("T", [300, 777, 1300])
-def test_fused_prompt_chain_of_bf16_layers_at_7b_width(dev, monkeypatch, T):
-    """The chain's shares and rotations in blocks of 64 to 256 tokens.  0.02 of the logits' spread as in test_runs_of_shares_in_the_fused_prompt_chain."""
-    cfg = LLaMAConfig(block_size=1304, n_layer=2, n_head=32, n_embd=4096, vocab_size=512)
+BF16_CHAIN = [
+    (640, 65), (640, 1094), (1024, 709), (1280, 65), (1280, 1731), (1920, 65), (1920, 646), (1920, 1633), (2048, 261), (2560, 65), (2560, 1542), (2560, 1605), (3072, 65),
+    (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1731),
+]
+
+
+@pytest.mark.parametrize("width,T", BF16_CHAIN)
+def test_fused_prompt_chain_of_bf16_layers(dev, monkeypatch, width, T):
+    """The chain's shares, rotations and cache rows in every block that its products take (tests/test_host_logic.py compares the list with the rule), a last block that is not
+    whole.  0.02 of the logits' spread as in test_runs_of_shares_in_the_fused_prompt_chain."""
+    cfg = LLaMAConfig(block_size=T + 4, n_layer=2, n_head=width // 128, n_embd=width, vocab_size=512)
     with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16):
         model = LLaMA(cfg)
     model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode=None, device="cuda", dtype=torch.bfloat16))
@@ -117,7 +129,7 @@ def test_fused_prompt_chain_of_bf16_layers_at_7b_width(dev, monkeypatch, T):
         monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
         model.reset_cache()
         with torch.no_grad():
-            out.append(model(idx.view(1, -1), 1304, torch.arange(T, device=dev))[0].float())
+            out.append(model(idx.view(1, -1), T + 4, torch.arange(T, device=dev))[0].float())
     assert not torch.equal(*out)  # (the chain was on)
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
 

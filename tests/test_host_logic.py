@@ -668,6 +668,31 @@ def test_short_bf16_rows_are_not_cut_along_k(M, N, K, R):
         assert _gemm_cut(M, N, K, R, chain) == (4, 64, 1)
 
 
+def test_gpu_tests_of_bf16_blocks_run_every_block():
+    """Each block that the rule takes at widths of 640 to 8192 and 65 to 2048 tokens, with whole rows and with slices, is run outside the fused chain and inside, by c_attn, by residual
+    products and by the gated pair."""
+    import importlib.util
+    import pathlib
+
+    spec = importlib.util.spec_from_file_location("gemm_shapes", pathlib.Path(__file__).parent / "test_gemm_shapes_gpu.py")
+    shapes = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(shapes)
+
+    def chain_of(width, T):
+        hidden = find_multiple(int(8 * width / 3), 256)
+        for role, N, K, R in (("c_attn", 3 * width, width, 1), ("residual", width, width, 1), ("residual", width, hidden, 1), ("pair", hidden, width, 2)):
+            waves, tokens, slices = _gemm_cut(T, N, K, R, True)
+            yield role, waves, tokens, slices > 1
+
+    taken = {c for width in (640, 1024, 1280, 1920, 2048, 2560, 3072, 4096, 5120, 6656, 8192) for T in range(65, 2049, 7) for c in chain_of(width, T)}
+    assert taken <= {c for width, T in shapes.BF16_CHAIN for c in chain_of(width, T)}
+    run = set()
+    for M, N, K, pair in shapes.BF16_BLOCKS:
+        waves, tokens, slices = _gemm_cut(M, N, K, 1 + pair, False)
+        run.add(("pair" if pair else "single", waves, tokens, slices > 1))
+    assert {("pair" if role == "pair" else "single", *c) for role, *c in taken} <= run
+
+
 def _forced_plans(value):
     """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
     import os
