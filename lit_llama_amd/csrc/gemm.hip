@@ -1629,9 +1629,10 @@ template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, typename Kernel>
 int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row tiles (pair tiles for the SwiGLU stream)
     constexpr int kSlots = kWaves * kTPW;
     const int per_block = PAIR ? kSlots / 2 : kSlots;
+    MI355_CHECK_ARG(p.slice_blocks % (16 * per_block) == 0, MI355_E_STATE, "linear_gemm: blocks of %d rows do not divide operand slices of %d", 16 * per_block, p.slice_blocks);
     GemmParams q = p;
     q.n_blocks = (p.n_tiles + per_block - 1) / per_block;
-    q.slice_blocks = p.slice_blocks / (16 * per_block);  // (in: rows; a multiple of 256, which every block divides)
+    q.slice_blocks = p.slice_blocks / (16 * per_block);  // (in: rows)
     q.total_blocks = q.n_blocks * ((p.M + BM - 1) / BM);
     q.per_xcd = (q.total_blocks * q.ksplit + 7) / 8;
     if constexpr (FUSE) {
@@ -1760,7 +1761,7 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
 // slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, each unit of one `unit` us, `unit_wave`
 // more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Fitted to launches of 36 products of 1024 to 32000 rows, weights not in any
 // cache: 16 and 32 tokens 0.909 times what blocks of 4 waves took, 0.4 % behind the fastest, none slower; 40 and 64 tokens 0.950 times, 1.2 % behind, at most 2.6 % slower.
-GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
+GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced) {
     struct Cost {
         float wave, unit, unit_wave, crowd, slices, bytes;
     };
@@ -1769,7 +1770,7 @@ GemmCut bf16_cut_few(int M, int N, int K, bool pair) {
     const int units = (K + 127) / 128;
     GemmCut cut = {4, short_block(M, true), true, 1};
     float best = 0.f;
-    for (int waves = 2; waves <= 4; ++waves)
+    for (int waves = 2; waves <= 4; waves += sliced ? 2 : 1)  // (operand slices start at multiples of 256 rows, which blocks of 96 do not divide)
         for (int ks = 1; ks <= 8 && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget / 2)); ++ks) {
             const int blocks = gemm_blocks(M, N, pair, waves, cut.bm) * ks;
             auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (c.unit + (float)waves * (c.unit_wave + c.crowd * (float)of / 256.f)); };
@@ -1836,17 +1837,17 @@ GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
         }
     return cut;
 }
-GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain) {
+GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {
     if (M > 64) return bf16_cut_long(M, N, K, pair);
     if (gemm_blocks(M, N, pair, 4, 64) > 256) return bf16_cut_many(M, N, K, pair);
-    return chain ? bf16_cut_few_chained(M, N, K, pair) : bf16_cut_few(M, N, K, pair);
+    return chain ? bf16_cut_few_chained(M, N, K, pair) : bf16_cut_few(M, N, K, pair, sliced);
 }
-// chain: a launch of the fused prompt chain (gemm_fuse.h)
-GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain) {
+// chain: a launch of the fused prompt chain (gemm_fuse.h); sliced: a launch of operand slices
+GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced) {
     const GemmForce fo = gemm_force();
-    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain) : q4_cut(M, N, K, pair);
+    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
     const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep == 1 : cut.deep, cut.ksplit};
-    if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4)) cut = forced;
+    if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) cut.ksplit = fo.ksplit;
     return cut;
 }
@@ -1889,12 +1890,16 @@ void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, in
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
-    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE);
+    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE, p.slice_blocks != 0);
     if constexpr (FMT == MI355_W_BF16 && !FUSE) {
-        // (operand slices start at multiples of 256 rows: blocks of 64 divide them, of 96 not)
-        if (sh.waves <= 3 && sh.bm == 64) return sh.waves == 3 && p.slice_blocks == 0 ? launch_deep<EPI, PAIR, FMT, 3, 64, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
-        if (sh.waves == 3 && p.slice_blocks == 0) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
-        if (sh.waves <= 3) return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
+        if (sh.waves == 3) {
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 3, 64, FUSE>(p, s);
+            return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
+        }
+        if (sh.waves == 2) {
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
+            return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
+        }
     }
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE>(p, s);
@@ -2014,10 +2019,10 @@ void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares,
 }
 }  // namespace
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
-    plan_shares(gemm_cut(M, N, K, R == 2, bf16, true), N, R == 2, ksplit, shares, shares_per_unit);
+    plan_shares(gemm_cut(M, N, K, R == 2, bf16, true, false), N, R == 2, ksplit, shares, shares_per_unit);
 }
-extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, int* waves, int* tokens, int* ksplit) {
-    const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain);
+extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, bool sliced, int* waves, int* tokens, int* ksplit) {
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain, sliced);
     *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
@@ -2126,11 +2131,11 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
         // (partial sums: at most half the region, the tables lie in the other)
-        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
+        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false, false, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
     }
     int runs = 1, run_units = units;
     if (!grouped) {
-        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr);
+        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr, a->slice_rows != 0);
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
     }

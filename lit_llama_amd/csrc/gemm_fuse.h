@@ -48,8 +48,8 @@ struct mi355_gemm_fuse {
 // many of them make a 128-column unit.  A launch split over K produces through the reduction of its slices
 // (splitk_fused_reduce_kernel), one share per unit.
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
-// how a launch of one scale per row is cut, in the chain or outside it: waves and tokens of a block, K-slices
-extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, int* waves, int* tokens, int* ksplit);
+// how a launch of one scale per row is cut, in the chain or outside it, of operand slices or not: waves and tokens of a block, K-slices
+extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, bool sliced, int* waves, int* tokens, int* ksplit);
 // the plan for scales in groups of group_cols columns (whole units)
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit);
 // Tables of the (scale, zero) pairs of up to MI355_TABLE_PRODUCTS products over grouped scales, laid out ahead of them in one launch: fmt, N, K, R, group_cols and the

@@ -1,5 +1,7 @@
 """The tiled products at the sizes where their blocks, K-slices and pipelines end: every number of tokens per block, odd rows and columns, slices of
 few units, launches that are cut and launches that are not."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -330,6 +332,27 @@ def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
     ref = prods[0] + base.double()
     got = ops.linear_gemm(x, ops.repack_bf16(ws[0], None, 1), 1, N, K, epi=nat.EPI_ACCUM if epi == "accum" else nat.EPI_STORE, out=base.clone(), fmt=nat.W_BF16).double()
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
+OPERAND_SLICES = [(9, 256, 9, 4096), (16, 512, 5, 4096), (24, 256, 22, 4096), (32, 256, 65, 128), (32, 3072, 2, 4096), (40, 256, 65, 256), (40, 256, 18, 4096), (64, 256, 66, 256), (64, 512, 11, 4096)]
+
+
+@pytest.mark.parametrize("M,rows,n,K", OPERAND_SLICES)
+def test_operand_slices_of_few_bf16_rows(dev, M, rows, n, K):
+    """Products of these rows and columns that read one operand take blocks of 3 waves, 96 rows, which do not divide the slices (tests/test_host_logic.py): one bf16 rounding of the result and
+    the sums' 1e-3 of the tiled product."""
+    g = torch.Generator(device=dev).manual_seed(M + rows + n)
+    x = torch.randn((n, M + 1, K), generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn((n * rows, K), generator=g, device=dev) * K ** -0.5).to(torch.bfloat16)
+    y = torch.zeros((M, n * rows), dtype=torch.bfloat16, device=dev)
+    stream = ops.repack_bf16(w, None, 1)
+    a = nat.LinearArgs()
+    a.fmt, a.R, a.w, a.N, a.K, a.x, a.x_dtype, a.M, a.ldx = nat.W_BF16, 1, nat.ptr(stream), n * rows, K, nat.ptr(x), nat.BF16, M, x.stride(1)
+    a.epi, a.y, a.y_dtype, a.ldy, a.alpha, a.slice_rows, a.slice_stride = nat.EPI_STORE, nat.ptr(y), nat.BF16, y.stride(0), 1.0, rows, x.stride(0)
+    ws = torch.empty(nat.lib().mi355_linear_gemm_workspace_bytes(M, K), dtype=torch.uint8, device=dev)
+    nat.check(nat.lib().mi355_linear_gemm(C.byref(a), nat.ptr(ws), ws.numel(), nat.stream_ptr()))
+    ref = torch.cat([x[i, :M].double() @ w[i * rows:(i + 1) * rows].double().T for i in range(n)], 1)
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-3 * ref.square().mean().sqrt()).all()
 
 
 @pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600)])

@@ -655,9 +655,9 @@ def test_partial_sums_of_slices_fit_their_buffer(bf16):
             assert (ks == 1 or ppu == 1) and shares * 128 >= N * ppu
 
 
-def _gemm_cut(M, N, K, R, chain):
+def _gemm_cut(M, N, K, R, chain, sliced=False):
     out = [C.c_int(0) for _ in range(3)]
-    nat.lib().mi355_linear_gemm_cut(M, N, K, R, C.c_bool(True), C.c_bool(chain), *[C.byref(v) for v in out])
+    nat.lib().mi355_linear_gemm_cut(M, N, K, R, C.c_bool(True), C.c_bool(chain), C.c_bool(sliced), *[C.byref(v) for v in out])
     return tuple(v.value for v in out)
 
 
@@ -668,15 +668,31 @@ def test_short_bf16_rows_are_not_cut_along_k(M, N, K, R):
         assert _gemm_cut(M, N, K, R, chain) == (4, 64, 1)
 
 
-def test_gpu_tests_of_bf16_blocks_run_every_block():
-    """Each block that the rule takes at widths of 640 to 8192 and 65 to 2048 tokens, with whole rows and with slices, is run outside the fused chain and inside, by c_attn, by residual
-    products and by the gated pair."""
+def _gemm_shapes():
     import importlib.util
     import pathlib
 
     spec = importlib.util.spec_from_file_location("gemm_shapes", pathlib.Path(__file__).parent / "test_gemm_shapes_gpu.py")
     shapes = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(shapes)
+    return shapes
+
+
+def test_operand_slices_are_cut_for_the_blocks_that_divide_them():
+    """Blocks of 3 waves are 96 rows: a launch of operand slices is not cut for them and then run in others (16 rows, N = 2560, K = 4096: 8 K-slices for blocks of 96 rows, 4 for
+    blocks of 64)."""
+    sizes = [(M, rows * n, K) for M, rows, n, K in _gemm_shapes().OPERAND_SLICES]
+    assert all(_gemm_cut(M, N, K, 1, False)[0] == 3 for M, N, K in sizes)
+    for M, N, K in sizes + [(M, 256 * n, K) for M in (9, 24, 33, 64) for n in range(1, 100, 7) for K in (256, 1024, 4096)]:
+        cut, whole = _gemm_cut(M, N, K, 1, False, True), _gemm_cut(M, N, K, 1, False)
+        assert cut[0] != 3 and (cut == whole or whole[0] == 3), (M, N, K)
+    assert _gemm_cut(16, 2560, 4096, 1, False, True) == (2, 16, 4)
+
+
+def test_gpu_tests_of_bf16_blocks_run_every_block():
+    """Each block that the rule takes at widths of 640 to 8192 and 65 to 2048 tokens, with whole rows and with slices, is run outside the fused chain and inside, by c_attn, by residual
+    products and by the gated pair."""
+    shapes = _gemm_shapes()
 
     def chain_of(width, T):
         hidden = find_multiple(int(8 * width / 3), 256)
