@@ -1,5 +1,5 @@
-"""LLM.int8 products of many rows where their outlier columns begin and end: none, one, a block of 64 and its neighbours, columns past the first 16 384, more
-than their region holds; cut into K-slices and not."""
+"""LLM.int8 products of many rows where their outlier columns begin and end: none, one, a block of 64 and its neighbours, columns past the first 16 384, all of
+them, more than their region holds; cut into K-slices and not."""
 import ctypes as C
 
 import pytest
@@ -35,6 +35,26 @@ def _reference(x, cb, scb):
 def test_outlier_columns(dev, M, N, K, outliers, epi):
     """Integer sums are exact; the outlier part is an f32 sum of exact products, so its f16 rounding may fall on either side: one f16 step of that part,
     and one of the sum that it moves; 2^-22 of its terms' sizes for the sum itself."""
+    _check_outlier_columns(dev, M, N, K, outliers, epi)
+
+
+@pytest.mark.parametrize("M,N,K,outliers,epi,waves,slices", [
+    (40, 32000, 4096, 2100, "store", 4, 1), (150, 32000, 4096, 2100, "store", 8, 1), (260, 32000, 4096, 2100, "accum", 4, 1), (129, 32000, 4096, 2100, "accum", 8, 1),
+    (64, 8192, 22016, 8200, "store", 4, 3), (150, 8192, 22016, 8200, "accum", 8, 3),
+    (150, 22016, 8192, 1480, "pair", 4, 1), (40, 22016, 8192, 1480, "pair", 8, 1), (64, 4096, 22016, 8200, "pair", 4, 3), (33, 5632, 12288, 6000, "pair", 8, 4),
+])
+def test_more_outlier_columns_than_their_region_holds(dev, M, N, K, outliers, epi, waves, slices):
+    """16-bit weights of the outlier columns (whole 64 of them, whole tiles of 16 rows) beyond the region's 128 MB: each is gathered in the product's own blocks, 64 columns a pass, in
+    blocks of 4 and 8 waves, of one token block and several, behind K-slices in the launch that sums them.  Bounds as above."""
+    R = 2 if epi == "pair" else 1
+    assert (N + 15) // 16 * 16 * R * ((outliers + 63) // 64 * 64) * 2 > 128 << 20
+    got = C.c_int(0), C.c_int(0)
+    nat.lib().mi355_linear_int8_gemm_plan(M, N, K, R, C.byref(got[0]), C.byref(got[1]))
+    assert (got[0].value, got[1].value) == (waves, slices)
+    _check_outlier_columns(dev, M, N, K, outliers, epi)
+
+
+def _check_outlier_columns(dev, M, N, K, outliers, epi):
     g = torch.Generator(device=dev).manual_seed(M + N + K + outliers)
     x = torch.randn((M, K), generator=g, device=dev).clamp_(-5.9, 5.9)
     at = torch.randperm(K, generator=g, device=dev)[:outliers]
