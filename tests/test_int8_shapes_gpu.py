@@ -84,7 +84,8 @@ def _check_outlier_columns(dev, M, N, K, outliers, epi):
 @pytest.mark.parametrize("T", [32, 100, 300])
 def test_a_chain_of_products_clears_the_mask_of_the_next(dev, T):
     """A prompt's LLM.int8 products share a mask of outlier columns that each clears for the next; driven segment by segment each has its own and clears it first: the same
-    bits.  Norm scales bring some columns of every product above the threshold, others in each layer."""
+    bits.  Norm scales bring some columns of c_attn, of the c_fc pair and of the head above the threshold, larger rows of the value and c_fc weights some of c_proj and mlp.c_proj, others
+    in each layer."""
     from lit_llama_amd import LLaMA, LLaMAConfig
     from lit_llama_amd.utils import EmptyInitOnDevice
 
@@ -96,6 +97,11 @@ def test_a_chain_of_products_clears_the_mask_of_the_next(dev, T):
     for k in sd:
         if k.endswith(".scale"):
             sd[k] = (sd[k].float().cpu() * (1 + 4 * (torch.rand(512, generator=g) < 0.02))).to(torch.bfloat16).to(dev)
+        if k.endswith(("c_attn.weight", "c_fc1.weight", "c_fc2.weight")):
+            larger = 1 + 7 * (torch.rand((sd[k].shape[0], 1), generator=g) < 0.02)
+            if k.endswith("c_attn.weight"):
+                larger[:1024] = 1  # (queries and keys)
+            sd[k] = (sd[k].float().cpu() * larger).to(torch.bfloat16).to(dev)
     model.load_state_dict(sd)
     model.eval()
     eng = model.engine()
@@ -108,9 +114,15 @@ def test_a_chain_of_products_clears_the_mask_of_the_next(dev, T):
         with torch.cuda.stream(eng.stream):
             eng.set_step(idx.reshape(-1), T, 0)
             nat.check(nat.lib().mi355_forward_embed(C.byref(eng.m), T, s), "embed")
+            columns = []
             for layer in range(cfg.n_layer):
-                nat.check(nat.lib().mi355_forward_segment(C.byref(eng.m), T, layer, 0, 4, s), "segment")
+                for seg in range(4):
+                    nat.check(nat.lib().mi355_forward_segment(C.byref(eng.m), T, layer, seg, seg + 1, s), "segment")
+                    if seg % 2 == 0:  # what c_proj or mlp.c_proj reads
+                        rows = (eng.att if seg == 0 else eng.hbuf)[:T]
+                        columns.append((rows.abs() >= 6).any(0))
             nat.check(nat.lib().mi355_forward_head(C.byref(eng.m), T, 2, 0, s), "head")
         torch.cuda.synchronize()
+    assert all(0 < int(c.sum()) < len(c) for c in columns)
     want = eng.logits[:T]
     assert torch.equal(got[0], want) and torch.equal(got[1], want)
