@@ -1084,7 +1084,8 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of longer ones):
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
-// alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight.
+// alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB of weights (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight; bf16 blocks of 96 to 192 tokens, whose
+// activations fill the LDS, have two units under way, of 256 one.
 // BM: 16 / 32 / 48 / 64 / 128 tokens, BF16 also 96 / 192 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
 // BF16: what bounds it is the CU's memory pipeline, which returns data in the order of the requests and holds some 50 KB of them: with nothing but its requests (no
 // products) a block of 128 tokens x 256 rows took 1.67 us for the 96 KB of a unit, 0.95 when all of it lay in L2.  So the requests of a unit are spread over all of its
@@ -1759,8 +1760,9 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
 // asks for no more than its memory pipeline holds, so 129 blocks of 128 rows leave half of what HBM gives, and a slice that would fill the other CUs costs a launch; smaller
 // blocks cost their activations again.  16 tokens, 4 / 3 / 2 waves without slices: N = 16512, K = 4096 29.7 / 26.1 / 35.0 us (129, 172, 258 blocks), 12416 33.2 (24.9 in two
 // slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, each unit of one `unit` us, `unit_wave`
-// more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Fitted to launches of 36 products of 1024 to 32000 rows, weights not in any
-// cache: 16 and 32 tokens 0.909 times what blocks of 4 waves took, 0.4 % behind the fastest, none slower; 40 and 64 tokens 0.950 times, 1.2 % behind, at most 2.6 % slower.
+// more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  36 products of 1024 to 32000 rows, weights not in any
+// cache (profiles/product_cuts_bf16_few.txt): 16 and 32 tokens 0.92 times what blocks of 4 waves took, 0.8 % behind the fastest, none more than 1 % slower; 40 and 64 tokens 0.94 times,
+// 1.5 % behind, 5 of 72 2 to 5 % slower (the same launch in two processes: up to 5 %).
 GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced) {
     struct Cost {
         float wave, unit, unit_wave, crowd, slices, bytes;
@@ -1815,7 +1817,7 @@ GemmCut bf16_cut_many(int M, int N, int K, bool pair) {
 // rows ask for 75 and 64 KB per 8.4 MFLOP instead of the 96 of 128 x 256, and give the rounds more sizes to fit: 2048 tokens, N = 16512, K = 4096, 4.1 rounds of 128 tokens 278 us, 2.8 of
 // 192 234; N = 6208, 1.6 of 128 108, 0.8 of 256 94; 777 tokens, N = 12288, 1.3 of 128 105, 0.9 of 192 79; N = 4096, K = 11008 in 128 x 128 85 (64 x 256: 104).  The constants are
 // those whose choice is best over 1078 launches (41 products of 512 to 32000 rows, 65 to 2048 tokens; those below 20 MB with their weights in the 256-MB cache and without, the others
-// without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.6 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
+// without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.7 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
 // a launch as the least that slices cost, 1.6 % and 5.4 %: short rows were cut (512 tokens, N = K = 2048 16.1 us in two slices, 12.7 whole; 96 of the N = 2816 pair, K = 1024 11.6, 8.2).
 GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
     struct Kind {

@@ -2,7 +2,7 @@
 //
 // Replaces, for B * T >= 32 rows, bitsandbytes' MatMul8bitLt forward as Linear8bitLt reaches it
 // (lit_llama/quantization.py:38-77; the algorithm is restated in oracle/oracle.py::llm_int8_linear — PARITY
-// UNPINNED: bitsandbytes is not vendored, see DESIGN.md section 3).  The skinny kernel (int8.hip) feeds such inputs in chunks
+// UNPINNED: bitsandbytes is not vendored).  The skinny kernel (int8.hip) feeds such inputs in chunks
 // of <= 16 rows and determines the outlier COLUMN set per chunk; this path determines it over all rows of the call, as the
 // algorithm does, and runs the int8 product on v_mfma_i32_16x16x64_i8 over 128-token blocks:
 //   1. i8_stage_kernel   (one workgroup per row) — xh = f16(norm_scale * x * 1/rms) (or f16(x)), the row's absmax over its

@@ -299,8 +299,8 @@ def group_table(scales: torch.Tensor, zeros: torch.Tensor) -> torch.Tensor:
 
 
 def prompt_workspace_bytes(kinds, rows: int, K: int) -> int:
-    """Scratch of the products of `rows` rows of up to K columns over streams of these kinds ("q4", "bf16", "i8"): of 2048 x 11008 87 MB for int4 and bf16, 190 for
-    LLM.int8, whose outlier columns have regions of their own."""
+    """Scratch of the products of `rows` rows of up to K columns over streams of these kinds ("q4", "bf16", "i8"): of 2048 x 11008 88 MB for int4 and bf16, 297 for
+    LLM.int8, whose outlier columns have regions of their own (of the weights 128 MB for any number of rows, K-slices' sums 48)."""
     need = [lib().mi355_linear_int8_gemm_workspace_bytes] if "i8" in kinds else []
     if kinds - {"i8"}:
         need.append(lib().mi355_linear_gemm_workspace_bytes)
@@ -420,8 +420,8 @@ class DecodeEngine:
             if max_T < 1:
                 raise EngineUnavailable("hidden size does not fit LDS")
             # prompt chunks of >= 32 tokens go through the wide MFMA GEMM (csrc/gemm.hip, int8_gemm.hip; int4 and bf16 products from 8 to 32 rows on:
-            # engine.hip wide_rows) and flash attention (flash_prefill.hip), so the chunk is bounded by scratch memory only (0.5 GB at 2048 tokens
-            # of a 7B model, most of it the f32 logits rows).  Large chunks matter: the [n_embd]-wide outputs (c_proj, mlp.c_proj) are
+            # engine.hip wide_rows) and flash attention (flash_prefill.hip), so the chunk is bounded by scratch memory only (0.6 GB at 2048 tokens
+            # of a 7B model, 0.8 as LLM.int8: 262 MB of it f32 logits rows, which prefill() uses past the first for results off a 16-byte line).  Large chunks matter: the [n_embd]-wide outputs (c_proj, mlp.c_proj) are
             # 16 row blocks, so 512 tokens fill only a quarter of the chip (9 % vs 27-36 % of the MFMA peak at 2048)
             self.gemm_ws = None
             if kinds <= {"q4", "bf16", "i8"} and _env_int("MI355_PREFILL_GEMM", 1):
