@@ -94,6 +94,7 @@ struct GemmParams {
     float limit;           // CLAMPGLU
     const float* bias;     // STORE: [N], or NULL
     mi355_reduce_norm rn;  // rn.done: the sum of the K-slices also leaves the rows' norm
+    bool squares;          // BF16, 8 waves: an XCD's blocks are kSquare row blocks by some token blocks (square_blocks())
     int slice_blocks;      // != 0: row blocks [i slice_blocks, (i + 1) slice_blocks) read the operand at xb + i slice_stride
     int64_t slice_stride;
     // grouped scales (GRP kernels): gtab[group 0..n_groups][r][tab_ld rows] = bf16 scale | bf16 zero << 16 (row n_groups
@@ -138,6 +139,7 @@ constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials 
 constexpr int kMaxSplit = 16;
 constexpr int kMaxRuns = 8;
 constexpr int kTableProducts = MI355_TABLE_PRODUCTS;
+constexpr int kSquare = 4;                        // row blocks of a square (GemmParams::squares)
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
@@ -1085,8 +1087,8 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
 // alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB of weights (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight; bf16 blocks of 96 to 192 tokens, whose
-// activations fill the LDS, have two units under way, of 256 one.
-// BM: 16 / 32 / 48 / 64 / 128 tokens, BF16 also 96 / 192 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
+// activations fill the LDS, have two units under way, of 208 and 256 one.
+// BM: 16 / 32 / 48 / 64 / 128 tokens, BF16 also 96 / 160 / 192 / 208 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
 // BF16: what bounds it is the CU's memory pipeline, which returns data in the order of the requests and holds some 50 KB of them: with nothing but its requests (no
 // products) a block of 128 tokens x 256 rows took 1.67 us for the 96 KB of a unit, 0.95 when all of it lay in L2.  So the requests of a unit are spread over all of its
 // products (in the first half of them, as before, the waves stood at requests that the pipeline had no room for: N = 4096, K = 16512, 2048 tokens 248 -> 226 us with what follows,
@@ -1124,6 +1126,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     if constexpr (FMT == MI355_W_BF16) {  // (orders: see gemm_q4_kernel)
         nb = L / m_blocks;
         mb = L - nb * m_blocks;
+        if constexpr (kWaves == 8) {
+            if (p.squares) {
+                const int first = nb / kSquare * kSquare, at = L - first * m_blocks, rows = n_blocks - first < kSquare ? n_blocks - first : kSquare;
+                mb = rows == kSquare ? at / kSquare : at / rows;
+                nb = first + at - mb * rows;
+            }
+        }
     } else {
         mb = L / n_blocks;
         nb = L - mb * n_blocks;
@@ -1626,6 +1635,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
+// BF16 blocks of 8 waves.  Row block by row block, the 32 blocks that an XCD runs side by side are all token blocks of two or three row blocks: with 16 token blocks of 128 they
+// bring 2 x 64 KB of weights and 16 x 32 of activations to its L2 per unit.  As 4 row blocks by 8 token blocks 4 x 64 + 8 x 32, a fifth less of what all of them wait for: 2048 tokens, N =
+// 4096, K = 16512 246 -> 218 us, 1800 tokens 211 -> 195.  Over 15 products, 129 to 2048 tokens: more than 12 token blocks 0.97 times (0.89 to 1.03), 9 to 12 0.97 times where K is
+// above 8192 (0.92 to 1.01) and 1.01 below, fewer 1.01 (the two divisions).
+bool square_blocks(int m_blocks, int units) { return m_blocks > 12 || (m_blocks > 8 && units > 64); }
 template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, typename Kernel>
 int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row tiles (pair tiles for the SwiGLU stream)
     constexpr int kSlots = kWaves * kTPW;
@@ -1636,6 +1650,7 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     q.slice_blocks = p.slice_blocks / (16 * per_block);  // (in: rows)
     q.total_blocks = q.n_blocks * ((p.M + BM - 1) / BM);
     q.per_xcd = (q.total_blocks * q.ksplit + 7) / 8;
+    q.squares = square_blocks((p.M + BM - 1) / BM, p.units);
     if constexpr (FUSE) {
         if (q.ksplit > 1) {  // the producer roles move to the reduction of the K-slices
             q.out_xb = nullptr;
@@ -1671,7 +1686,7 @@ int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM < kBM && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, true>(p, s);
     }
-    constexpr int kDepth = BM == 256 ? 2 : BM >= 96 && FMT == MI355_W_BF16 ? 3 : 4;
+    constexpr int kDepth = BM > 192 ? 2 : BM >= 96 && FMT == MI355_W_BF16 ? 3 : 4;
     constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
     static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -1714,7 +1729,7 @@ GemmForce gemm_force() {
     return f;
 }
 bool launch_gemm_has(const GemmCut& c, bool bf16, bool named) {  // (what a sweep may force of the kernels of launch_gemm())
-    if (bf16 && named && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 192 || c.bm == 256)))) return true;
+    if (bf16 && named && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 160 || c.bm == 192 || c.bm == 208 || c.bm == 256)))) return true;
     if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
@@ -1819,13 +1834,16 @@ GemmCut bf16_cut_many(int M, int N, int K, bool pair) {
 // those whose choice is best over 1078 launches (41 products of 512 to 32000 rows, 65 to 2048 tokens; those below 20 MB with their weights in the 256-MB cache and without, the others
 // without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.7 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
 // a launch as the least that slices cost, 1.6 % and 5.4 %: short rows were cut (512 tokens, N = K = 2048 16.1 us in two slices, 12.7 whole; 96 of the N = 2816 pair, K = 1024 11.6, 8.2).
+// Blocks of 160 and 208 tokens came later, their constants fitted to 270 launches without slices (15 products, 129 to 2048 tokens; 0.05 % behind the fastest of six blocks): the launches that they
+// take are 8 % faster on average (777 tokens, N = 15360, K = 5120 in 256 / 208 tokens 123 / 107 us; N = 12288, K = 4096 in 192 / 160 75 / 69, the N = 11008 pair 138 / 128; 2048, N = 12416 in 256 / 208 199 / 179).
 GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
     struct Kind {
         int waves, bm;
         float start, unit, crowd;
     };
-    static constexpr Kind kinds[] = {{4, 64, 2.744f, 0.518f, 0.181f},  {4, 96, 4.059f, 0.484f, 0.333f},   {4, kBM, 2.751f, 0.78f, 0.272f},  {8, 64, 6.209f, 0.684f, 0.474f},
-                                     {8, kBM, 8.323f, 0.926f, 0.424f}, {8, 192, 11.38f, 1.231f, 0.501f}, {8, 256, 9.51f, 1.344f, 1.146f}};
+    static constexpr Kind kinds[] = {{4, 64, 2.744f, 0.518f, 0.181f},  {4, 96, 4.059f, 0.484f, 0.333f}, {4, kBM, 2.751f, 0.78f, 0.272f},
+                                     {8, 64, 6.209f, 0.684f, 0.474f},  {8, kBM, 8.323f, 0.926f, 0.424f}, {8, 160, 8.129f, 1.217f, 0.283f},
+                                     {8, 192, 11.38f, 1.231f, 0.501f}, {8, 208, 8.519f, 1.703f, 0.271f}, {8, 256, 9.51f, 1.344f, 1.146f}};
     const int units = (K + 127) / 128;
     GemmCut cut = {4, 64, true, 1};
     float best = 0.f;
@@ -1917,7 +1935,9 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
     }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 8, 64, FUSE>(p, s);
     if constexpr (FMT == MI355_W_BF16) {
+        if (sh.bm == 160) return launch_deep<EPI, PAIR, FMT, 8, 160, FUSE>(p, s);
         if (sh.bm == 192) return launch_deep<EPI, PAIR, FMT, 8, 192, FUSE>(p, s);
+        if (sh.bm == 208) return launch_deep<EPI, PAIR, FMT, 8, 208, FUSE>(p, s);
         if (sh.bm == 256) return launch_deep<EPI, PAIR, FMT, 8, 256, FUSE>(p, s);
         return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
     } else {

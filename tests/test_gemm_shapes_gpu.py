@@ -87,12 +87,13 @@ BF16_BLOCKS = [
     (512, 1000, 2176, 1), (193, 4112, 1664, 1), (320, 4112, 1664, 1), (320, 6160, 2176, 1), (641, 4112, 384, 1), (1281, 4096, 2176, 1), (449, 12288, 2048, 1), (1281, 12288, 128, 1),
     (600, 12288, 1152, 0), (600, 11012, 1664, 1), (70, 4100, 2176, 0), (129, 4100, 4224, 0), (66, 4100, 3200, 0), (300, 4096, 11008, 0), (135, 11012, 8448, 0),
     (70, 2816, 1664, 1), (70, 4100, 2176, 1), (66, 2052, 3200, 1), (129, 11012, 4224, 1),
+    (482, 16400, 1664, 0), (674, 16400, 640, 0), (386, 8200, 640, 1), (962, 6160, 384, 1), (1930, 8280, 384, 0), (1165, 3340, 8448, 0),
 ]
 
 
 @pytest.mark.parametrize("M,N,K,pair", BF16_BLOCKS)
 def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
-    """Blocks of 64 / 96 / 128 tokens x 4 waves and 64 / 128 / 192 / 256 x 8, whole rows and K-slices, pairs too (tests/test_host_logic.py compares the list with the rule): a few
+    """Blocks of 64 / 96 / 128 tokens x 4 waves and 64 / 128 / 160 / 192 / 208 / 256 x 8, whole rows and K-slices, pairs too (tests/test_host_logic.py compares the list with the rule): a few
     tokens or rows more than whole blocks, rounds of units that end early, row blocks that share an XCD and such that are cut between two.  Bounds: as in test_tiled_product_against_64_bits."""
     g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
     x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
@@ -112,7 +113,7 @@ def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
 
 BF16_CHAIN = [
     (640, 65), (640, 1094), (1024, 709), (1280, 65), (1280, 1731), (1920, 65), (1920, 646), (1920, 1633), (2048, 261), (2560, 65), (2560, 1542), (2560, 1605), (3072, 65),
-    (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1731),
+    (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1542), (6656, 1731), (6656, 1878),
 ]
 
 
