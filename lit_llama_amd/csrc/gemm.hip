@@ -491,10 +491,10 @@ constexpr int kRowAt = NB * BM * 256 + 2 * BM * 4 + (FUSE ? 4096 + BM * 4 : 0);
 // The end of a block: lane (g, c) of a wave holds rows 4 g .. 4 g + 3 of the wave's tiles for token tt * 16 + c (acc: what the MFMAs summed, GRP: the scaled
 // sums).  The tables `fr` (1/rms, operand sums of the tokens), `postab` and `rowtab` (scale, 128 + zero, next norm) stand in LDS; every wave has passed
 // its last read of the activation buffers and no request into them is under way.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP, bool FUSE>
-__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[kTPW][BM / 16], char* smem, const float* fr, const int* postab,
-                                              const float* rowtab, const int (&tile)[kTPW], int m0, int nb, int ks, int wave, int lane) {
-    constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, int GRP, bool FUSE, int TPW>
+__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[TPW][BM / 16], char* smem, const float* fr, const int* postab,
+                                              const float* rowtab, const int (&tile)[TPW], int m0, int nb, int ks, int wave, int lane) {
+    constexpr int kTT = BM / 16, kSlots = kWaves * TPW, kThreads = 64 * kWaves;
     const int g = lane >> 4, c = lane & 15;
     // old residual rows and rotations are requested for kEB token tiles at a time, without a branch between them (columns and tokens past the end read
     // entry 0): a load behind a branch of its own is waited for alone.  Four at a time: a bf16 prompt of 777 tokens (7B, 8 layers) 3.37 -> 3.25 ms on one box; int4 blocks of 128 tokens,
@@ -502,12 +502,12 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
     constexpr int kEB = BM >= 128 && FMT == MI355_W_Q4 ? 1 : kTT < 4 ? kTT : 4;
     const bool emit = FUSE && EPI == MI355_EPI_ACCUM && p.out_xb != nullptr;
     const bool sums = FUSE && EPI != MI355_EPI_STORE && p.out_sx != nullptr;
-    auto rows4 = [&](int table, int t) { return *(const f32x4*)(rowtab + (table * kSlots + kTPW * wave + t) * 16 + 4 * g); };
-    int nn[kTPW];
+    auto rows4 = [&](int table, int t) { return *(const f32x4*)(rowtab + (table * kSlots + TPW * wave + t) * 16 + 4 * g); };
+    int nn[TPW];
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t) nn[t] = tile[t] * 16 + 4 * g;
+    for (int t = 0; t < TPW; ++t) nn[t] = tile[t] * 16 + 4 * g;
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t) {
+    for (int t = 0; t < TPW; ++t) {
         [[maybe_unused]] f32x4 sc, zp;
         if constexpr (FMT == MI355_W_Q4 && GRP == 0) sc = rows4(0, t), zp = rows4(1, t);
 #pragma unroll
@@ -528,7 +528,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
         for (int tt = 0; tt < kTT; ++tt) {
             const int m = m0 + tt * 16 + c;
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t)
+            for (int t = 0; t < TPW; ++t)
                 if (m < p.M && nn[t] < p.N) *(f32x4*)(p.part + ((int64_t)ks * p.M + m) * ldp + (PAIR && (t & 1) ? p.N : 0) + nn[t]) = acc[t][tt];
         }
         return;
@@ -536,13 +536,13 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
     [[maybe_unused]] float es1[kTT], es2[kTT];  // FUSE: this lane's share of the rows' partial sums (operand values, squares)
 #pragma unroll
     for (int tb = 0; tb < kTT; tb += kEB) {
-        [[maybe_unused]] f32x4 got[kEB][kTPW];  // ACCUM: the old rows; STORE of c_attn: rotations
+        [[maybe_unused]] f32x4 got[kEB][TPW];  // ACCUM: the old rows; STORE of c_attn: rotations
         if constexpr (EPI == MI355_EPI_ACCUM) {
             if (p.y_dtype == MI355_F32) {
 #pragma unroll
                 for (int i = 0; i < kEB && tb + i < kTT; ++i)
 #pragma unroll
-                    for (int t = 0; t < kTPW; ++t) {
+                    for (int t = 0; t < TPW; ++t) {
                         const int m = m0 + (tb + i) * 16 + c;
                         got[i][t] = *(const f32x4*)((const float*)p.y + (m < p.M && nn[t] < p.N ? (int64_t)m * p.ldy + nn[t] : 0));
                     }
@@ -550,7 +550,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 #pragma unroll
                 for (int i = 0; i < kEB && tb + i < kTT; ++i)
 #pragma unroll
-                    for (int t = 0; t < kTPW; ++t) {
+                    for (int t = 0; t < TPW; ++t) {
                         const int m = m0 + (tb + i) * 16 + c;
                         const u32x2 w = *(const u32x2*)((const bf16_t*)p.y + (m < p.M && nn[t] < p.N ? (int64_t)m * p.ldy + nn[t] : 0));
                         got[i][t] = f32x4{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16),
@@ -565,7 +565,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
                     const int t16 = (tb + i) * 16 + c;
                     const int m = m0 + t16 < p.M ? m0 + t16 : p.M - 1;
 #pragma unroll
-                    for (int t = 0; t < kTPW; ++t)
+                    for (int t = 0; t < TPW; ++t)
                         got[i][t] = *(const f32x4*)(p.rope + (int64_t)(p.rope_gathered ? m : postab[t16]) * 128 + (nn[t] & 127));
                 }
             }
@@ -577,7 +577,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
             if (m >= p.M) continue;
             if constexpr (is_pair_epi(EPI)) {
 #pragma unroll
-                for (int t = 0; t < kTPW; t += 2) {
+                for (int t = 0; t < TPW; t += 2) {
                     if (nn[t] >= p.N) continue;  // N % 4 == 0 (host check)
                     bf16_t ob[4];
 #pragma unroll
@@ -590,7 +590,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
                 }
             } else {
 #pragma unroll
-                for (int t = 0; t < kTPW; ++t) {
+                for (int t = 0; t < TPW; ++t) {
                     const int n = nn[t];
                     if (n >= p.N) continue;
                     f32x4 o = acc[t][tt];
@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_q4_kernel(const GemmParams p
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = accf[t][tt];
     }
-    gemm_epilogue<EPI, PAIR, MI355_W_Q4, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
+    gemm_epilogue<EPI, PAIR, MI355_W_Q4, kWaves, BM, GRP, FUSE, kTPW>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
 // 16 B per lane from `off` + `scalar_off` of a buffer to 1 KiB of LDS (lane i's bytes at 16 i); out of range: zeros
@@ -1104,15 +1104,16 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // units / 4 of their own on the f32 MFMA in front of the loop.
 // RUNS (Q4): a slice of several runs (gemm_runs()).  The second set of sums is 32 registers, with which two workgroups of 8 waves no longer share a CU: kernels of
 // their own.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
     static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1), "grouped scales are a Q4 feature");
     static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
+    static_assert(TPW == 2 || (TPW == 1 && !PAIR), "a pair is two row tiles");
     static_assert(DEPTH >= 2 && DEPTH <= 4, "units under way + 1");
-    constexpr int kTT = BM / 16, kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
+    constexpr int kTT = BM / 16, kSlots = kWaves * TPW, kThreads = 64 * kWaves;
     constexpr int kWP = FMT == MI355_W_BF16 ? 4 : 1;
     constexpr int kXI = (BM / 4 + kWaves - 1) / kWaves;  // activation requests (1 KiB: four tokens) per wave and unit
-    constexpr int kUnit = kXI + kTPW * kWP + (GRP ? kTPW : 0);  // requests per wave and unit
+    constexpr int kUnit = kXI + TPW * kWP + (GRP ? TPW : 0);  // requests per wave and unit
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1145,10 +1146,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     [[maybe_unused]] int* postab = (int*)(smem + kPosAt<BM, DEPTH>);
     [[maybe_unused]] float* rowtab = (float*)(smem + kRowAt<BM, FUSE, DEPTH>);
     [[maybe_unused]] float* runtab = rowtab + 3 * kSlots * 16;  // [part of a run's sum][run][BM] operand sums
-    int tile[kTPW];
+    int tile[TPW];
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t)
-        tile[t] = PAIR ? nb * (kSlots / 2) + (kTPW / 2) * wave + (t >> 1) : nb * kSlots + kTPW * wave + t;
+    for (int t = 0; t < TPW; ++t)
+        tile[t] = PAIR ? nb * (kSlots / 2) + (TPW / 2) * wave + (t >> 1) : nb * kSlots + TPW * wave + t;
     // this block's share of its row block's weights (see above): thread i's line of every round of DEPTH units, at touch_off from the round's first unit
     constexpr bool kTouch = FMT == MI355_W_BF16 && (BM == 64 || (BM > 64 && kWaves == 4));
     constexpr int kTouchAhead = 2 * DEPTH - 1, kStreams = PAIR ? kSlots / 2 : kSlots, kRun = DEPTH * (PAIR ? 64 : 32);  // kRun: lines of DEPTH units of a tile
@@ -1177,13 +1178,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         xoff[i] = m0 + tok < p.M ? (unsigned)((int64_t)(m0 + tok) * p.ldxb * 2) + (unsigned)((slot ^ swz(tok)) * 16) : 0xFFFFFFF0u;
         xdst[i] = q * 1024;
     }
-    u32x4 wr[DEPTH][kTPW][kWP];
-    [[maybe_unused]] u32x4 tb[GRP ? DEPTH : 1][kTPW];  // (scale, zero) of rows 4 g .. 4 g + 3 in the unit's group
+    u32x4 wr[DEPTH][TPW][kWP];
+    [[maybe_unused]] u32x4 tb[GRP ? DEPTH : 1][TPW];  // (scale, zero) of rows 4 g .. 4 g + 3 in the unit's group
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc((void*)p.gtab, 0, GRP ? (p.n_groups + 1) * (PAIR ? 2 : 1) * p.tab_ld * 4 : 0, 0x00020000);
     [[maybe_unused]] const int tbstep = (PAIR ? 2 : 1) * p.tab_ld * 4;
-    [[maybe_unused]] int tboff[kTPW];  // (tiles past the last read the first one's)
+    [[maybe_unused]] int tboff[TPW];  // (tiles past the last read the first one's)
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t) tboff[t] = ((PAIR ? t & 1 : 0) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + 4 * g) * 4;
+    for (int t = 0; t < TPW; ++t) tboff[t] = ((PAIR ? t & 1 : 0) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + 4 * g) * 4;
     // request i of unit u: activations first.  What tells the units apart is scalar (offsets, and the size in the descriptor): no address
     // instruction on the VALU.  Past the slice or the tiles: a size of 0, nothing is read (the scalar offset is not range-checked), zeros go to a buffer that
     // nobody reads
@@ -1192,8 +1193,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         if (i < kXI) {
             const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, in ? x_bytes : 0, 0x00020000);
             lds_from(rx, smem + slot * (BM * 256) + xdst[i < kXI ? i : 0], xoff[i < kXI ? i : 0], in ? u * 256 : 0);
-        } else if (i >= kXI + kTPW * kWP) {
-            const int t = i - (kXI + kTPW * kWP) < kTPW ? i - (kXI + kTPW * kWP) : 0;
+        } else if (i >= kXI + TPW * kWP) {
+            const int t = i - (kXI + TPW * kWP) < TPW ? i - (kXI + TPW * kWP) : 0;
             tb[GRP ? slot : 0][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rt, tboff[t], ((in ? u : u_hi - 1) >> p.gq_shift) * tbstep, 0));
         } else {
             const int t = (i - kXI) / kWP, d = (i - kXI) % kWP;
@@ -1362,9 +1363,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         if constexpr (FUSE && EPI == MI355_EPI_STORE) postab[threadIdx.x] = t_pos;
     }
 
-    f32x4 acc[kTPW][kTT];
+    f32x4 acc[TPW][kTT];
 #pragma unroll
-    for (int t = 0; t < kTPW; ++t)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
         for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint32_t cmask = 0x000F000Fu, cmagic = 0x43004300u;  // (opaque: see gemm_q4_kernel)
@@ -1375,7 +1376,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     };
     if constexpr (GRP != 0) {
         // lane (g, c): units u0 + 4 g + i of product i; a chunk's factors are requested while the one before is multiplied
-        struct Chunk { uint32_t sz[4][kTPW]; float x[4][kTT]; };
+        struct Chunk { uint32_t sz[4][TPW]; float x[4][kTT]; };
         const bool halves = FUSE && p.in_ppu == 2;  // a producer in blocks of 64 hidden rows leaves two shares a unit
         const int64_t x_step = halves ? 2 * (int64_t)p.M : p.M;
         auto fetch = [&](int u0, Chunk& k) {
@@ -1383,7 +1384,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             for (int i = 0; i < 4; ++i) {
                 const int u = u0 + 4 * g + i < u_hi ? u0 + 4 * g + i : u_hi - 1;
 #pragma unroll
-                for (int t = 0; t < kTPW; ++t)
+                for (int t = 0; t < TPW; ++t)
                     k.sz[i][t] = p.gtab[((int64_t)(u >> p.gq_shift) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * p.tab_ld + (tile[t] < p.n_tiles ? tile[t] * 16 : 0) + c];
 #pragma unroll
                 for (int tt = 0; tt < kTT; ++tt) k.x[i][tt] = p.sxt[(int64_t)u * x_step + (m0 + tt * 16 + c < p.M ? m0 + tt * 16 + c : p.M - 1)];
@@ -1403,15 +1404,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const bool in = u0 + 4 * g + i < u_hi;
-                float a[kTPW];
+                float a[TPW];
 #pragma unroll
-                for (int t = 0; t < kTPW; ++t)
+                for (int t = 0; t < TPW; ++t)
                     a[t] = in ? -__uint_as_float(cur.sz[i][t] << 16) * (128.f + __uint_as_float(cur.sz[i][t] & 0xffff0000u)) : 0.f;
 #pragma unroll
                 for (int tt = 0; tt < kTT; ++tt) {
                     const float x = in ? cur.x[i][tt] : 0.f;
 #pragma unroll
-                    for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], x, acc[t][tt], 0, 0, 0);
+                    for (int t = 0; t < TPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], x, acc[t][tt], 0, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1425,7 +1426,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     constexpr int kEvery = kFrags >= kUnit ? kFrags / kUnit : 1;  // fragments from one request to the next
     constexpr int kPer = (kUnit + kFrags - 1) / kFrags;                      // requests behind one fragment
     // GRP: token tile by token tile, so the sums of one unit live in two token tiles' registers: those being summed, and those being scaled
-    auto mfmas_grouped = [&](int slot, u32x4 (&w)[kTPW][kWP], u32x4 (&sz)[kTPW], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
+    auto mfmas_grouped = [&](int slot, u32x4 (&w)[TPW][kWP], u32x4 (&sz)[TPW], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
         const char* xs = smem + slot * (BM * 256);
         auto bread = [&](int f) {  // fragment f = tt * 4 + d
             const int tok = (f >> 2) * 16 + c;
@@ -1435,10 +1436,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
         for (int q = 0; q < kPipe; ++q) bq[q] = bread(q);
         __builtin_amdgcn_sched_group_barrier(0x100, kPipe, 0);
-        bf16x8 a[4][kTPW];
-        f32x4 sc[kTPW];
+        bf16x8 a[4][TPW];
+        f32x4 sc[TPW];
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t) {
+        for (int t = 0; t < TPW; ++t) {
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 a[d][t] = levels(w[t][0][d]);
@@ -1446,17 +1447,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
             for (int r = 0; r < 4; ++r) sc[t][r] = __uint_as_float(sz[t][r] << 16);
         }
-        f32x4 un[2][kTPW];
+        f32x4 un[2][TPW];
 #pragma unroll
         for (int f = 0; f < kFrags; ++f) {
             const int tt = f >> 2, d = f & 3;
             const bf16x8 b = __builtin_bit_cast(bf16x8, bq[f % kPipe]);
             if (f + kPipe < kFrags) bq[f % kPipe] = bread(f + kPipe);
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t)
+            for (int t = 0; t < TPW; ++t)
                 un[tt & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b, d == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : un[tt & 1][t], 0, 0, 0);
             if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, TPW, 0);
             if (more && f % kEvery == 0) {
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) {
@@ -1466,19 +1467,19 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
                     __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
                 }
             }
-            if (tt > 0 && d > 0 && d <= kTPW) {
+            if (tt > 0 && d > 0 && d <= TPW) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[d - 1][tt - 1][r] = __builtin_fmaf(sc[d - 1][r], un[(tt - 1) & 1][d - 1][r], acc[d - 1][tt - 1][r]);
                 __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
             }
         }
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t)
+        for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[t][kTT - 1][r] = __builtin_fmaf(sc[t][r], un[(kTT - 1) & 1][t][r], acc[t][kTT - 1][r]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto mfmas = [&](int slot, u32x4 (&w)[kTPW][kWP], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
+    auto mfmas = [&](int slot, u32x4 (&w)[TPW][kWP], int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
         const char* xs = smem + slot * (BM * 256);
         auto bread = [&](int f) {  // fragment f = d * kTT + tt
             const int tok = (f % kTT) * 16 + c;
@@ -1490,9 +1491,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
         __builtin_amdgcn_sched_group_barrier(0x100, kPipe, 0);
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            bf16x8 a[kTPW];
+            bf16x8 a[TPW];
 #pragma unroll
-            for (int t = 0; t < kTPW; ++t) {
+            for (int t = 0; t < TPW; ++t) {
                 if constexpr (FMT == MI355_W_BF16)
                     a[t] = __builtin_bit_cast(bf16x8, w[t][d]);
                 else
@@ -1504,9 +1505,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
                 const bf16x8 b = __builtin_bit_cast(bf16x8, bq[f % kPipe]);
                 if (f + kPipe < kFrags) bq[f % kPipe] = bread(f + kPipe);
 #pragma unroll
-                for (int t = 0; t < kTPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[t][tt], 0, 0, 0);
+                for (int t = 0; t < TPW; ++t) acc[t][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[t][tt], 0, 0, 0);
                 if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, TPW, 0);
                 if (more && f % kEvery == 0) {
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) {
@@ -1544,7 +1545,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     };
     using std::integral_constant;
     // the sum of a run, its levels' offset and zero points taken off, leaves the accumulators
-    [[maybe_unused]] f32x4 of_runs[RUNS ? kTPW : 1][RUNS ? kTT : 1];
+    [[maybe_unused]] f32x4 of_runs[RUNS ? TPW : 1][RUNS ? kTT : 1];
     [[maybe_unused]] int run = 0, left = p.run_units;
     [[maybe_unused]] auto end_run = [&]() __attribute__((always_inline)) {
         float x[kTT];
@@ -1554,8 +1555,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) x[tt] += runtab[(run + q * p.runs) * BM + tt * 16 + c];
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t) {
-            const f32x4 zp = *(const f32x4*)(rowtab + (kSlots + kTPW * wave + t) * 16 + 4 * g);
+        for (int t = 0; t < TPW; ++t) {
+            const f32x4 zp = *(const f32x4*)(rowtab + (kSlots + TPW * wave + t) * 16 + 4 * g);
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) {
 #pragma unroll
@@ -1570,7 +1571,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     };
     if constexpr (RUNS) {
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t)
+        for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) of_runs[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1600,7 +1601,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     if constexpr (RUNS) {
         if (open) end_run();
 #pragma unroll
-        for (int t = 0; t < kTPW; ++t)
+        for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int tt = 0; tt < kTT; ++tt) acc[t][tt] = of_runs[t][tt];
     }
@@ -1633,7 +1634,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (requests past the slice wrote zeros: none may land in what the epilogue keeps there)
     __syncthreads();
-    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
+    gemm_epilogue<EPI, PAIR, FMT, kWaves, BM, GRP, FUSE, TPW>(p, acc, smem, fr, postab, rowtab, tile, m0, nb, ks, wave, lane);
 }
 
 // BF16 blocks of 8 waves.  Row block by row block, the 32 blocks that an XCD runs side by side are all token blocks of two or three row blocks: with 16 token blocks of 128 they
@@ -1641,9 +1642,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
 // 4096, K = 16512 246 -> 218 us, 1800 tokens 211 -> 195.  Over 15 products, 129 to 2048 tokens: more than 12 token blocks 0.97 times (0.89 to 1.03), 9 to 12 0.97 times where K is
 // above 8192 (0.92 to 1.01) and 1.01 below, fewer 1.01 (the two divisions).
 bool square_blocks(int m_blocks, int units) { return m_blocks > 12 || (m_blocks > 8 && units > 64); }
-template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, typename Kernel>
+template <int EPI, bool PAIR, int kWaves, int BM, bool FUSE, int TPW, typename Kernel>
 int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) {  // p.n_tiles: 16-row tiles (pair tiles for the SwiGLU stream)
-    constexpr int kSlots = kWaves * kTPW;
+    constexpr int kSlots = kWaves * TPW;
     const int per_block = PAIR ? kSlots / 2 : kSlots;
     MI355_CHECK_ARG(p.slice_blocks % (16 * per_block) == 0, MI355_E_STATE, "linear_gemm: blocks of %d rows do not divide operand slices of %d", 16 * per_block, p.slice_blocks);
     GemmParams q = p;
@@ -1682,20 +1683,20 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     }
     return 0;
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, bool RUNS = false>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false>
 int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM < kBM && !RUNS) {
-        if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, true>(p, s);
+        if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, true>(p, s);
     }
     constexpr int kDepth = BM > 192 ? 2 : BM >= 96 && FMT == MI355_W_BF16 ? 3 : 4;
-    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * kTPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>,
+    constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * TPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS>, kLds, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE, TPW>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW>, kLds, p, s);
 }
 template <int EPI, bool PAIR, int kWaves, int BM, int GRP = 0, bool FUSE = false>
 int launch_gemm_w(const GemmParams& p, hipStream_t s) {
@@ -1706,13 +1707,14 @@ int launch_gemm_w(const GemmParams& p, hipStream_t s) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE>(gemm_q4_kernel<EPI, PAIR, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE, kTPW>(gemm_q4_kernel<EPI, PAIR, kWaves, BM, GRP, FUSE>, kLdsW, p, s);
 }
 // How a launch of one scale per row is cut: waves and tokens of a block, gemm_deep_kernel (or gemm_q4_kernel), K-slices
 struct GemmCut {
     int waves, bm;
     bool deep;
     int ksplit;
+    int tiles = kTPW;  // row tiles of a wave
 };
 // tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel, the latter int4 only), 0 = the rule's choice.  A cut that
 // no kernel is instantiated for is ignored as a whole, a number of slices that does not fit by itself; blocks that only BF16 streams have need the kernel named (deep = 1)
@@ -1730,14 +1732,15 @@ GemmForce gemm_force() {
     return f;
 }
 bool launch_gemm_has(const GemmCut& c, bool bf16, bool named) {  // (what a sweep may force of the kernels of launch_gemm())
+    if (c.tiles == 1) return !bf16 && c.waves == 4 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 48 || c.bm == 64);
     if (bf16 && named && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 160 || c.bm == 192 || c.bm == 208 || c.bm == 256)))) return true;
     if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
 }
 // blocks of `waves` waves and `bm` tokens
-int gemm_blocks(int M, int N, bool pair, int waves, int bm) {
-    const int rows = 16 * (pair ? waves * kTPW / 2 : waves * kTPW);
+int gemm_blocks(int M, int N, bool pair, int waves, int bm, int tiles = kTPW) {
+    const int rows = 16 * (pair ? waves * tiles / 2 : waves * tiles);
     return (N + rows - 1) / rows * ((M + bm - 1) / bm);
 }
 // bytes of the K-slices' partial sums
@@ -1771,6 +1774,50 @@ GemmCut q4_cut(int M, int N, int K, bool pair) {
     const int wide = gemm_blocks(M, N, pair, 8, kBM) * cut.ksplit;
     if (wide >= 384 || wide == 256) cut.bm = kBM, cut.deep = false;
     return cut;
+}
+// Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
+// product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows
+// number less than 96 / cuts and a run keeps 4 units; a K-slice that is longer takes several runs, each with its own operand sum.  Error beside one activation of
+// 2^17 (rms, in units of its product's last bit), N = K = 4096 / N = 4096, K = 11008 / N = 12288, K = 4096, a run per slice -> runs: 40 tokens 3.0 / 3.9 / 4.8 -> 2.6 /
+// 3.8 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.6 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.5 / 6.7.  A second run takes a launch 0.5-0.7 us (a prompt of 37
+// tokens, 7B: 2.48 -> 2.49 ms).  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
+void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, int* run_units) {
+    const int units = (K + 127) / 128, longest = (units + cut.ksplit - 1) / cut.ksplit, blocks = gemm_blocks(M, N, pair, 8, kBM);
+    int cuts = 1;
+    while (cuts < 8 && blocks * cuts < 96 && units >= 8 * cuts) cuts *= 2;
+    *runs = 1, *run_units = units;
+    if (longest <= (units + cuts - 1) / cuts || !cut.deep || cut.bm == kBM) return;
+    *run_units = units / cuts / 4 * 4;
+    *runs = (longest + *run_units - 1) / *run_units;
+}
+// Int4 products other than pairs, where blocks of 64 rows x 4 waves are one per CU at most: a wave of one row tile.  A wave alone on its SIMD is bound by what it issues (37 tokens: two row tiles take
+// 0.45 us a unit, one 0.31 to 0.34, with all operands in the L2 caches as well, and no barrier 0.42), so half the rows per wave on idle CUs are worth more than K-slices, whose sums are a launch more:
+// 37 tokens, N = 12288, K = 4096 20.6 us in two slices of 128-row blocks, 18.1 whole in 64-row blocks; N = K = 4096 16.2 in 8 slices, 15.4 in 4; 128 tokens, N = 6144, K = 2048 19.6 / 14.5.  The
+// estimate: per unit of a slice `unit` us and `crowd` more when every CU has a block, `slices` and `bytes` for partial sums, fitted to 1422 launches (18 products of 1024 to 32000 rows, 32 to 300
+// tokens, weights in no cache; 7 % off on average).  Where it takes these blocks or not: 0.96 / 0.95 / 0.94 / 0.93 times the time of 128-row blocks (32, to 48, to 64, more tokens), 3 % slower at worst.
+// In the chain, whose blocks add up shares first and whose sums of slices write the next ones, whole rows only (37 tokens, 7B: c_attn 12.8 + 4.2 us for the sum of its slices -> 15.9; attn.c_proj in 4
+// narrow slices 8.4 + 4.2, in 8 wide ones 7.8 + 4.4).
+void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
+    struct Cost {
+        float start, wide, wide_crowd, unit, crowd, slices, bytes;
+    };
+    static constexpr Cost costs[] = {{-0.476f, 0.369f, 0.24f, 0.288f, 0.148f, 3.485f, 1.2e6f},
+                                     {-0.67f, 0.451f, 0.158f, 0.333f, 0.116f, 3.491f, 1.167e6f},
+                                     {-0.796f, 0.539f, 0.073f, 0.383f, 0.083f, 3.592f, 1.153e6f},
+                                     {-0.872f, 0.531f, 0.027f, 0.416f, -0.021f, 3.362f, 1.555e6f}};
+    const int units = (K + 127) / 128, wide = gemm_blocks(M, N, false, 4, cut->bm) * cut->ksplit;
+    if (pair || cut->waves != 4 || !cut->deep || wide > 256) return;
+    const Cost& c = costs[M <= 32 ? 0 : M <= 48 ? 1 : M <= 64 ? 2 : 3];
+    auto slices = [&](int ks) { return ks == 1 ? 0.f : c.slices + (float)gemm_part_bytes(M, N, false, ks) / c.bytes; };
+    float best = (float)((units + cut->ksplit - 1) / cut->ksplit) * (c.wide + c.wide_crowd * (float)wide / 256.f) + slices(cut->ksplit);
+    const int bm = cut->bm, blocks = gemm_blocks(M, N, false, 4, bm, 1);
+    for (int ks = 1; ks <= (chain ? 1 : 8) && blocks * ks <= 256 && (ks == 1 || (units >= 2 * ks && gemm_part_bytes(M, N, false, ks) <= kSplitBudget / 2)); ++ks) {
+        const GemmCut narrow = {4, bm, true, ks, 1};
+        int runs, run_units;
+        gemm_runs(M, N, K, false, narrow, &runs, &run_units);
+        const float us = c.start + (float)((units + ks - 1) / ks) * (c.unit + c.crowd * (float)(blocks * ks) / 256.f) + slices(ks);
+        if (us < best && runs <= kMaxRuns && ks * runs <= kMaxSplit) best = us, *cut = narrow;
+    }
 }
 // Up to 64 tokens, outside the fused chain (whose shares are 64 or 128 rows), where blocks of 4 waves do not fill the chip: blocks of 2, 3 or 4 waves (64, 96, 128 rows).  A CU
 // asks for no more than its memory pipeline holds, so 129 blocks of 128 rows leave half of what HBM gives, and a slice that would fill the other CUs costs a launch; smaller
@@ -1867,7 +1914,8 @@ GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced) {
     const GemmForce fo = gemm_force();
     GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
-    const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep == 1 : cut.deep, cut.ksplit};
+    if (!bf16) q4_narrow(M, N, K, pair, chain, &cut);
+    const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep != 2 : cut.deep, cut.ksplit, fo.deep ? (fo.deep == 3 && !pair ? 1 : kTPW) : cut.tiles};
     if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) cut.ksplit = fo.ksplit;
     return cut;
@@ -1894,21 +1942,6 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
     const GemmCut forced = {fo.waves ? fo.waves : sh.waves, fo.bm ? fo.bm : sh.bm, true, ksplit};
     return launch_gemm_has(forced, false, false) ? forced : sh;
 }
-// Int4: the units that one accumulator sums.  Levels enter as 128 + q: beside an activation 10^5 times the others a sum is 10^7 times its other terms, and every
-// product of 32 columns costs it another rounding of that size.  So a sum ends behind 1 / cuts of K at the latest, cuts = 2, 4, 8 while 128-token blocks of 256 rows
-// number less than 96 / cuts and a run keeps 4 units; a K-slice that is longer takes several runs, each with its own operand sum.  Error beside one activation of
-// 2^17 (rms, in units of its product's last bit), N = K = 4096 / N = 4096, K = 11008 / N = 12288, K = 4096, a run per slice -> runs: 40 tokens 3.0 / 3.9 / 4.8 -> 2.6 /
-// 3.8 / 4.8, 100 tokens 3.5 / 5.6 / 6.8 -> 2.6 / 3.5 / 4.8, 512 tokens 6.8 / 11.2 / 6.8 -> 4.8 / 7.5 / 6.7.  A second run takes a launch 0.5-0.7 us (a prompt of 37
-// tokens, 7B: 2.48 -> 2.49 ms).  Runs of K / 8 for longer prompts too would cost them registers: 400 tokens 239 -> 268 us a layer.
-void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, int* run_units) {
-    const int units = (K + 127) / 128, longest = (units + cut.ksplit - 1) / cut.ksplit, blocks = gemm_blocks(M, N, pair, 8, kBM);
-    int cuts = 1;
-    while (cuts < 8 && blocks * cuts < 96 && units >= 8 * cuts) cuts *= 2;
-    *runs = 1, *run_units = units;
-    if (longest <= (units + cuts - 1) / cuts || !cut.deep || cut.bm == kBM) return;
-    *run_units = units / cuts / 4 * 4;
-    *runs = (longest + *run_units - 1) / *run_units;
-}
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
     const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE, p.slice_blocks != 0);
@@ -1920,6 +1953,14 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
         if (sh.waves == 2) {
             if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
             return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
+        }
+    }
+    if constexpr (FMT == MI355_W_Q4 && !PAIR) {
+        if (sh.tiles == 1) {
+            if (sh.bm == 16) return launch_deep<EPI, PAIR, FMT, 4, 16, FUSE, 0, 1>(p, s);
+            if (sh.bm == 32) return launch_deep<EPI, PAIR, FMT, 4, 32, FUSE, 0, 1>(p, s);
+            if (sh.bm == 48) return launch_deep<EPI, PAIR, FMT, 4, 48, FUSE, 0, 1>(p, s);
+            return launch_deep<EPI, PAIR, FMT, 4, 64, FUSE, 0, 1>(p, s);
         }
     }
     if (sh.waves == 4) {
@@ -2034,7 +2075,7 @@ int grouped_split(int M, int N, int K, bool pair, int group_cols) {
 void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares, int* shares_per_unit) {
     // rows (hidden rows of a pair stream) behind one share of a producer's partial sums: a 128-column unit when the K-slices'
     // reduction writes them or a block holds 256 rows, else the block's rows
-    int rows = (pair ? cut.waves * kTPW / 2 : cut.waves * kTPW) * 16;
+    int rows = (pair ? cut.waves * cut.tiles / 2 : cut.waves * cut.tiles) * 16;
     if (cut.ksplit > 1 || rows > 128) rows = 128;
     *ksplit = cut.ksplit;
     *shares = (N + rows - 1) / rows;
@@ -2154,7 +2195,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         MI355_CHECK_ARG(tab_bytes + sxt_bytes <= kSplitBudget, MI355_E_SHAPE,
                         "linear_gemm: group tables of %zu B exceed the workspace region (%zu B)", tab_bytes + sxt_bytes, kSplitBudget);
         // (partial sums: at most half the region, the tables lie in the other)
-        ksplit = unit_sums ? gemm_cut(a->M, a->N, a->K, swiglu, false, false, false).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
+        ksplit = unit_sums ? q4_cut(a->M, a->N, a->K, swiglu).ksplit : grouped_split(a->M, a->N, a->K, swiglu, a->group_cols);
     }
     int runs = 1, run_units = units;
     if (!grouped) {

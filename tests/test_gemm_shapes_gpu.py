@@ -16,6 +16,7 @@ SHAPES = [  # M, N, K
     (1, 16, 128), (9, 144, 300), (15, 4096, 4096), (16, 1000, 640), (17, 4096, 1024), (31, 528, 2048), (32, 272, 4224), (33, 4096, 4096),
     (48, 12288, 512), (64, 128, 11008), (65, 4096, 4096), (127, 2064, 896), (128, 11008, 384), (129, 4096, 1664), (200, 260, 1024),
     (300, 12288, 256), (1030, 4096, 384), (2048, 4096, 256), (2050, 8200, 128), (160, 5120, 5120), (330, 6656, 5120), (640, 4096, 11008), (100, 528, 2048),
+    (33, 68, 384), (40, 4100, 1024), (64, 6148, 2048), (100, 6144, 2048), (256, 2052, 640), (200, 4112, 4096),  # int4: blocks of 64 rows
 ]
 
 
