@@ -29,17 +29,15 @@
 
 namespace {
 
-constexpr int kBM = 128;      // tokens per block
+constexpr int kBM = 128;      // tokens per block (64 in launches that leave CUs idle: i8_cut())
 constexpr int kTPW = 2;       // 16-row tile slots per wave
-constexpr int kXTile = kBM * 128;        // bytes of one activation tile (int8)
 constexpr int kOutChunk = 64;            // outlier columns staged per pass of the epilogue
 constexpr int kDepth = 4;                // units of operands in LDS and registers
-constexpr int kLdsMain = kDepth * kXTile;
 constexpr int kSoLd = kOutChunk + 8;     // row pitch of the staged outlier weights (halves): 144 B, so that 16 rows written side by side fall into 16 banks
-template <int kWaves>
-constexpr int kLdsEpi = (kBM * kOutChunk + kWaves * kTPW * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [rows][kSoLd]
-template <int kWaves>
-constexpr int kLds = kLdsMain > kLdsEpi<kWaves> ? kLdsMain : kLdsEpi<kWaves>;
+template <int kWaves, int BM>
+constexpr int kLdsEpi = (BM * kOutChunk + kWaves * kTPW * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [rows][kSoLd]
+template <int kWaves, int BM>
+constexpr int kLds = kDepth * BM * 128 > kLdsEpi<kWaves, BM> ? kDepth * BM * 128 : kLdsEpi<kWaves, BM>;
 
 __device__ __forceinline__ float f16r(float v) { return f16_to_f32(f32_to_f16(v)); }
 // the same for a value that must be an f32 PRODUCT rounded to f32 first (MatMul8bitLt's dequantisation multiplies in f32 and converts): hipcc
@@ -297,9 +295,11 @@ __global__ __launch_bounds__(256) void i8_quant_kernel(const unsigned* mask, int
 
 // ---- 3. the product
 // MODE 0: product + epilogue; 1: product of one K-slice -> partial tiles; 2: sum of the partial tiles + epilogue
-template <int EPI, bool PAIR, int MODE, int kWaves>
+template <int EPI, bool PAIR, int MODE, int kWaves, int BM = kBM>
 __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmParams p) {
     static_assert(MODE != 2 || kWaves == 8, "a wave per token tile");
+    static_assert(MODE == 0 || BM == kBM, "K-slices come in blocks of 128 tokens");
+    constexpr int kXTile = BM * 128;  // bytes of one activation tile (int8)
     constexpr int kSlots = kWaves * kTPW, kThreads = 64 * kWaves;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
@@ -316,12 +316,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
     const int L = L2 / nsplit, ks = L2 - L * nsplit;
     // MODE 2: workgroup ks of a block finishes the rows of slot group ks (the rows wave ks owns in the product launch) for all 128
     // tokens, wave w its token tile w
-    constexpr int kTT = MODE == 2 ? 1 : 8;                                     // token tiles a wave finishes, from tt0 on
+    constexpr int kTT = MODE == 2 ? 1 : BM / 16;                               // token tiles a wave finishes, from tt0 on
     const int tt0 = MODE == 2 ? wave : 0;
     const int wslot = MODE == 2 ? ks : wave;                                   // slot group of this wave's row tiles
     // row block major: an XCD runs every token block of a few row blocks side by side, so their weights cross to its L2 once
     const int m_blocks = p.total_blocks / p.n_blocks, nb = L / m_blocks, mb = L - nb * m_blocks;
-    const int m0 = mb * kBM;
+    const int m0 = mb * BM;
     const int u_lo = MODE == 1 ? (int)((int64_t)ks * p.units / p.ksplit) : 0;
     const int u_hi = MODE == 1 ? (int)((int64_t)(ks + 1) * p.units / p.ksplit) : p.units;
     constexpr int R = PAIR ? 2 : 1;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
     // the activations (LDS, by DMA, the swizzle on the source's side) of the next kDepth - 1 units are under way; a unit waits for its own requests by
     // count, and the requests go out between the products (as gemm_deep_kernel: csrc/gemm.hip).  One unit ahead, waited for in front of its LDS stores, a unit
     // took 1.56 us at one workgroup per CU
-    constexpr int kXI = kBM / 8 / kWaves, kUnit = kXI + 2 * kTPW;  // requests per wave and unit: 1 KiB = 8 tokens of activations; weight pieces
+    constexpr int kXI = BM / 8 / kWaves, kUnit = kXI + 2 * kTPW;  // requests per wave and unit: 1 KiB = 8 tokens of activations; weight pieces
     auto run_units = [&](auto f16, auto& sum, int lo, int hi, __amdgpu_buffer_rsrc_t rwt, __amdgpu_buffer_rsrc_t rxt, int64_t ldb) {
         constexpr bool F16 = decltype(f16)::value;
         typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_l;
@@ -387,10 +387,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
         }
         auto products = [&](int slot, int ahead, int ahead_slot, auto more) __attribute__((always_inline)) {
             const char* xs = smem + slot * kXTile;
-            constexpr int kFrags = 16, kPipe = 4;  // fragment f = e * 8 + tt
+            constexpr int kT = BM / 16, kFrags = 2 * kT, kPipe = 4;  // fragment f = e * kT + tt
             auto bread = [&](int f) {
-                const int tok = (f & 7) * 16 + c;
-                return *(const i32x4*)(xs + tok * 128 + (((4 * (f >> 3) + g) ^ swz8(tok)) << 4));
+                const int tok = (f % kT) * 16 + c;
+                return *(const i32x4*)(xs + tok * 128 + (((4 * (f / kT) + g) ^ swz8(tok)) << 4));
             };
             i32x4 bq[kPipe];
 #pragma unroll
@@ -403,10 +403,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
 #pragma unroll
                 for (int t = 0; t < kTPW; ++t) {
                     if constexpr (F16)
-                        sum[t][f & 7] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_l, wr[slot][t][f >> 3]),
-                                                                               __builtin_bit_cast(f16x8_l, b), sum[t][f & 7], 0, 0, 0);
+                        sum[t][f % kT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_l, wr[slot][t][f / kT]),
+                                                                               __builtin_bit_cast(f16x8_l, b), sum[t][f % kT], 0, 0, 0);
                     else
-                        sum[t][f & 7] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, wr[slot][t][f >> 3]), b, sum[t][f & 7], 0, 0, 0);
+                        sum[t][f % kT] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, wr[slot][t][f / kT]), b, sum[t][f % kT], 0, 0, 0);
                 }
                 if (f + kPipe < kFrags) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, kTPW, 0);
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
     } else if (n_out > 0) {  // (too many for their region)
         // mixed-precision decomposition: the outlier columns in f16, ascending k, kOutChunk columns per pass through LDS
         f16_t* xo = (f16_t*)smem;                     // [128 tokens][kOutChunk]
-        f16_t* so = xo + kBM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
+        f16_t* so = xo + BM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
         // (the side product runs on v_mfma_f32_16x16x32_f16 — A = 16 rows x 32 outlier columns of `so`, B = 16 tokens x the same
         // columns of `xo`, result in the accumulators' own layout: lane (g, c) holds rows 4 g .. 4 g + 3 for token c.  The products of two f16
         // values are exact in f32 and the sum is f32 as before; its ORDER inside a block of 32 columns is the hardware's instead of
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
             const bool col_ok = oi < nc;
             const int k = col_ok ? p.olist[1 + base + oi] : 0;
 #pragma unroll 8
-            for (int idx = threadIdx.x; idx < kBM * kOutChunk; idx += kThreads) {
+            for (int idx = threadIdx.x; idx < BM * kOutChunk; idx += kThreads) {
                 const int tok = idx / kOutChunk;
                 const int m = m0 + tok;
                 xo[idx] = (m < p.M && col_ok) ? p.xh[(int64_t)m * p.Kp + k] : (f16_t)0;
@@ -689,19 +689,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
     }
 }
 
-template <int EPI, bool PAIR, int MODE, int kWaves>
+template <int EPI, bool PAIR, int MODE, int kWaves, int BM = kBM>
 int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
+    constexpr int lds = kLds<kWaves, BM>;
     static hipError_t attr_err =
-        hipFuncSetAttribute((const void*)i8_gemm_kernel<EPI, PAIR, MODE, kWaves>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds<kWaves>);
+        hipFuncSetAttribute((const void*)i8_gemm_kernel<EPI, PAIR, MODE, kWaves, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(i8_gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
     I8GemmParams r = q;
     r.n_blocks = (q.n_tiles + kWaves * kTPW / (PAIR ? 2 : 1) - 1) / (kWaves * kTPW / (PAIR ? 2 : 1));
-    r.total_blocks = r.n_blocks * ((q.M + kBM - 1) / kBM);
+    r.total_blocks = r.n_blocks * ((q.M + BM - 1) / BM);
     r.per_xcd = (r.total_blocks * (MODE == 1 ? q.ksplit + 1 : MODE == 2 ? 8 : 1) + 7) / 8;
-    hipLaunchKernelGGL((i8_gemm_kernel<EPI, PAIR, MODE, kWaves>), dim3(8 * r.per_xcd), dim3(64 * kWaves), kLds<kWaves>, s, r);
+    hipLaunchKernelGGL((i8_gemm_kernel<EPI, PAIR, MODE, kWaves, BM>), dim3(8 * r.per_xcd), dim3(64 * kWaves), lds, s, r);
     MI355_LAUNCH_CHECK();
     return 0;
 }
@@ -712,29 +713,31 @@ int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
 // sums' way to memory and back.  How many outlier columns there are is on the device; the constants are those whose choice is best over 2688 launches (32 products of
 // 768 to 32000 rows, 32 to 2048 tokens, 0, 0.3, 2 and 10 % of the columns, weights not in any cache: profiles/product_cuts_int8.txt): 0.5 % behind the fastest on average, 2 %
 // at the 90th percentile; with the outliers' workgroups left out 1.6 % and 5 %, and N = 5120, K = 13824, 256 tokens 79 us (now 66).  Blocks of 8 waves throughout and
-// slices for launches of less than 96 of them: 1.23 times as long on average, none more than 2.5 % shorter
+// slices for launches of less than 96 of them: 1.23 times as long on average, none more than 2.5 % shorter.
+// Blocks of 64 tokens x 128 rows (whole rows only) where they bring work to idle CUs: 512 tokens, N = 4096, K = 4096 35.8 -> 31.4 us, K = 11008 73.2 -> 59.2, with 2750 outlier columns 154 -> 136
+// (128 blocks -> 256; staging and quantisation with it); of 493 launches (13 products, 33 to 2048 tokens, 0, 2 and 25 % of the columns) the rule takes them in 167, 0.90 times as long, 2.6 % longer at worst.
 struct I8Cut {
-    int waves, ksplit;
+    int waves, ksplit, bm;
 };
 int i8_part_columns(int N) { return (N + 3) & ~3; }
 I8Cut i8_cut(int M, int N, int units, bool pair) {
     struct Kind {
-        int waves;
+        int waves, bm;
         float start, unit;
     };
-    static constexpr Kind kinds[] = {{4, 0.21f, 0.436f}, {8, 0.737f, 0.763f}};
+    static constexpr Kind kinds[] = {{4, kBM, 0.21f, 0.436f}, {8, kBM, 0.737f, 0.763f}, {4, 64, 0.f, 0.41f}};
     const size_t part = (size_t)M * i8_part_columns(N) * (pair ? 2 : 1) * 4;  // bytes of one slice's sums
-    I8Cut cut = {8, 1};
+    I8Cut cut = {8, 1, kBM};
     float best = 0.f;
     for (const Kind& k : kinds)
-        for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && part * ks <= kSplitBudget)); ++ks) {
-            const int rows = 16 * k.waves * kTPW / (pair ? 2 : 1), blocks = (N + rows - 1) / rows * ((M + kBM - 1) / kBM) * (ks == 1 ? 1 : ks + 1);
+        for (int ks = 1; ks <= (k.bm == kBM ? kMaxSplit : 1) && (ks == 1 || (units >= 4 * ks && part * ks <= kSplitBudget)); ++ks) {
+            const int rows = 16 * k.waves * kTPW / (pair ? 2 : 1), blocks = (N + rows - 1) / rows * ((M + k.bm - 1) / k.bm) * (ks == 1 ? 1 : ks + 1);
             auto round = [&](int of) {
                 const float work = (float)((units + ks - 1) / ks) * k.unit, hbm = 0.557f + 128.f * units * N * (pair ? 2 : 1) / 2.03e6f * (float)of / (float)blocks;
                 return sqrtf(work * work + hbm * hbm);
             };
             const float us = k.start + (float)(blocks / 256) * round(256) + (blocks % 256 ? round(blocks % 256) : 0.f) + (ks == 1 ? 0.f : 3.19f + (float)(part * ks) / 2.29e6f);
-            if (best == 0.f || us < best) best = us, cut = {k.waves, ks};
+            if (best == 0.f || us < best) best = us, cut = {k.waves, ks, k.bm};
         }
     struct Force {
         int waves, bm, ksplit;
@@ -744,12 +747,15 @@ I8Cut i8_cut(int M, int N, int units, bool pair) {
         if (const char* e = getenv("MI355_GEMM_FORCE")) sscanf(e, "%d:%d:%d", &f.waves, &f.bm, &f.ksplit);
         return f;
     }();
-    if ((fo.waves == 4 || fo.waves == 8) && (fo.bm == 0 || fo.bm == kBM)) cut.waves = fo.waves;
+    if ((fo.waves == 4 || fo.waves == 8) && (fo.bm == 0 || fo.bm == kBM || (fo.bm == 64 && fo.waves == 4))) cut.waves = fo.waves, cut.bm = fo.bm ? fo.bm : cut.bm;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && units >= 4 * fo.ksplit && part * fo.ksplit <= kSplitBudget) cut.ksplit = fo.ksplit;
+    if (cut.waves != 4 || cut.ksplit > 1) cut.bm = kBM;
     return cut;
 }
 template <int EPI, bool PAIR>
-int launch_i8_gemm(const I8GemmParams& p, int waves, hipStream_t s) {
+int launch_i8_gemm(const I8GemmParams& p, const I8Cut& cut, hipStream_t s) {
+    const int waves = cut.waves;
+    if (cut.bm == 64) return launch_i8_mode<EPI, PAIR, 0, 4, 64>(p, s);
     if (p.ksplit <= 1) return waves == 4 ? launch_i8_mode<EPI, PAIR, 0, 4>(p, s) : launch_i8_mode<EPI, PAIR, 0, 8>(p, s);
     if (int rc = waves == 4 ? launch_i8_mode<EPI, PAIR, 1, 4>(p, s) : launch_i8_mode<EPI, PAIR, 1, 8>(p, s)) return rc;
     return launch_i8_mode<EPI, PAIR, 2, 8>(p, s);
@@ -866,7 +872,7 @@ int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* cha
     }
     hipLaunchKernelGGL(i8_quant_kernel, dim3(a->M + 512), dim3(256), (kp / 32 < kMaskWords ? kp / 32 : kMaskWords) * kQuantLds, s, mask, ca, olist, p, a->R);
     MI355_LAUNCH_CHECK();
-    if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, cut.waves, s);
-    if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, cut.waves, s);
-    return launch_i8_gemm<MI355_EPI_STORE, false>(p, cut.waves, s);
+    if (swiglu) return launch_i8_gemm<MI355_EPI_SWIGLU, true>(p, cut, s);
+    if (a->epi == MI355_EPI_ACCUM) return launch_i8_gemm<MI355_EPI_ACCUM, false>(p, cut, s);
+    return launch_i8_gemm<MI355_EPI_STORE, false>(p, cut, s);
 }

@@ -30,6 +30,7 @@ def _reference(x, cb, scb):
     (33, 72, 200, 1), (64, 4096, 4096, 63), (200, 4096, 4096, 64), (130, 1000, 1024, 65), (257, 4096, 11008, 700), (48, 4096, 22016, 300),
     (1030, 4096, 640, 129), (2050, 1040, 512, 33), (40, 11008, 4096, 4096), (512, 4096, 1024, 0),
     (33, 1001, 4096, 3), (64, 1001, 4096, 5), (64, 4098, 4096, 70), (129, 1003, 2048, 0),  # K-slices whose rows are not whole vectors of four sums
+    (100, 12292, 1152, 20), (200, 4100, 4096, 70), (257, 4096, 1030, 9), (65, 260, 12416, 2000),  # blocks of 64 tokens; rows staged element by element, twelve fours a thread
 ])
 @pytest.mark.parametrize("epi", ["store", "accum", "pair"])
 def test_outlier_columns(dev, M, N, K, outliers, epi):
@@ -40,6 +41,7 @@ def test_outlier_columns(dev, M, N, K, outliers, epi):
 
 @pytest.mark.parametrize("M,N,K,outliers,epi,waves,slices", [
     (40, 32000, 4096, 2100, "store", 4, 1), (150, 32000, 4096, 2100, "store", 8, 1), (260, 32000, 4096, 2100, "accum", 4, 1), (129, 32000, 4096, 2100, "accum", 8, 1),
+    (100, 16384, 8192, 4200, "store", 4, 1),
     (64, 8192, 22016, 8200, "store", 4, 3), (150, 8192, 22016, 8200, "accum", 8, 3),
     (150, 22016, 8192, 1480, "pair", 4, 1), (40, 22016, 8192, 1480, "pair", 8, 1), (64, 4096, 22016, 8200, "pair", 4, 3), (33, 5632, 12288, 6000, "pair", 8, 4),
 ])
