@@ -21,6 +21,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
 
 constexpr int kRowThreads = 256;
+constexpr int kPassKeys = 4 * (kRowThreads / 16);  // keys that the row kernel scores at a time
 constexpr int kKeys = 256;        // keys per pass of the row kernel
 constexpr int kMaxSplit = 32;     // (<= 64, a lane each) workgroups over the keys of one (row, key head) in a decode step
 constexpr double kInvTwoPi = 0.15915494309189533577;
@@ -83,6 +84,7 @@ struct WinParams {
     mi355_window_attn_args a;
     mi355_seq_batch b;
     int n_split, head_tiles, fresh;  // fresh: a decode step
+    int chunk;                       // keys of a split, at least (rows of fewer than splits x chunk have splits without keys)
     int own;                         // a decode step of a layer with keys of its own: the row's k is raw and not in the cache yet
     const void *krows, *vrows;       // prepared keys and values of the step's rows, first key head
     int64_t ld_rows;
@@ -141,8 +143,15 @@ __global__ __launch_bounds__(kRowThreads, HT <= 4 ? 4 : 2) void window_rows_kern
     const int g_cur = pos0 < n_first ? pos0 : max(n_first, pos0 - w_shift);
     auto row_of = [&](int g) { return (unsigned)(g < n_first ? g : g < g_wrap ? g + row_shift : g + row_shift - a.ring); };
     auto step_row = [&](int g) { return (unsigned)((g < n_first ? g : g + w_shift) - pos0); };
-    const int step = (n_keys + p.n_split - 1) / p.n_split;
+    const int step = max((n_keys + p.n_split - 1) / p.n_split, p.chunk);
     const int k_begin = split * step, k_end = min(n_keys, k_begin + step);
+    if (FRESH && split > 0 && k_begin >= n_keys) {  // no keys: a record without weight
+        for (int i = tid; i < nh * (vdim + 2); i += kRowThreads) {
+            const int h = i / (vdim + 2), d = i - h * (vdim + 2);
+            a.partials[(((int64_t)row * a.heads + h0 + h) * p.n_split + split) * (vdim + 2) + d] = d == 0 ? -INFINITY : 0.f;
+        }
+        return;
+    }
     const bool owner = FRESH && p.own && k_begin < n_keys && k_end == n_keys;  // this split holds the row's own key
     const bool made_v = a.unit_v || a.v_first != nullptr;                      // ... whose value is not the projection's
 
@@ -242,7 +251,7 @@ __global__ __launch_bounds__(kRowThreads, HT <= 4 ? 4 : 2) void window_rows_kern
         const int nk = min(kKeys, k_end - kb);
         // ---- scores: 16 lanes per key, four keys per lane group in flight
         const int l16 = tid & 15;
-        for (int k4 = tid >> 4; k4 - (tid >> 4) < nk; k4 += 4 * (kRowThreads / 16)) {
+        for (int k4 = tid >> 4; k4 - (tid >> 4) < nk; k4 += kPassKeys) {
             float dot[4][HT];
             const T* src[4];
 #pragma unroll
@@ -957,10 +966,12 @@ template <typename T>
 int run(WinParams p, hipStream_t s) {
     const mi355_window_attn_args& a = p.a;
     if (p.fresh) {
-        // splits: enough workgroups for the chip, at least 64 keys each, as far as the scratch goes
+        // splits: enough workgroups for the chip, at least 64 keys each, as far as the scratch goes.  A row of few keys has them in its first splits, a pass of keys each, and leaves the others
+        // empty: each split prepares the row's queries again (16 sequences of 32 to 512 keys, 4 layers, 4 steps: 2588 -> 2562 us, of 96 to 1536 2638 -> 2630)
         const int per = a.heads / a.kv_heads, ht = per >= 5 ? 8 : per >= 2 ? 4 : 1;
         const int groups = p.b.rows * a.kv_heads * ((per + ht - 1) / ht);
         int n = 2048 / groups;
+        p.chunk = kPassKeys;
         const int most = (a.keep + (a.window < a.ring ? a.window : a.ring)) / 64;
         n = n < most ? n : most;
         n = n < kMaxSplit ? n : kMaxSplit;
@@ -1018,7 +1029,7 @@ int make_params(const mi355_window_attn_args* a, const mi355_seq_batch* b, WinPa
     p.b = *b;
     p.fresh = b->max_count == 1;
     p.own = p.fresh && a->role != MI355_KV_BORROWS;
-    p.n_split = p.head_tiles = 1;
+    p.n_split = p.head_tiles = p.chunk = 1;
     const int size = dtype_size(a->dtype);
     if (a->role == MI355_KV_OWN || p.own) {
         p.krows = (const char*)a->proj + (int64_t)a->off_k * size;
