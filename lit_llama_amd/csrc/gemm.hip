@@ -1685,10 +1685,10 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
 }
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false>
 int launch_deep(const GemmParams& p, hipStream_t s) {
-    if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM < kBM && !RUNS) {
+    if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM <= 64 && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, true>(p, s);
     }
-    constexpr int kDepth = BM > 192 ? 2 : BM >= 96 && FMT == MI355_W_BF16 ? 3 : 4;
+    constexpr int kDepth = BM > 192 ? 2 : BM > kBM || (BM >= 96 && FMT == MI355_W_BF16) ? 3 : 4;
     constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * TPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
     static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -1749,8 +1749,8 @@ size_t gemm_part_bytes(int M, int N, bool pair, int ksplit) { return (size_t)ksp
 // 3-7 % (N = 12288, K = 4096: 22.2 -> 20.9, 22.1 -> 21.0, 22.4 -> 21.3 us).  BF16, bound by the weights, the same either way)
 int short_block(int M, bool bf16) { return M <= 16 ? 16 : M <= 32 ? 32 : M <= 48 && !bf16 ? 48 : 64; }
 
-// Int4.  (Of 18 products of 2048 to 32000 rows at 72 to 700 tokens, weights not in any cache, this choice is within 5 % of the fastest instantiated one for two in three
-// and 4 % behind on average; at most 1.4 times as long, for narrow SwiGLU pairs: 5632 rows, K = 2048, 128 tokens 24.5 us against 17.4 in blocks of 4 waves.)
+// Int4: up to 64 tokens, and what q4_narrow() and q4_whole() start from.  (Narrow SwiGLU pairs of up to 128 tokens are left behind: 5632 rows, K = 2048, 128 tokens 24.5 us against 17.4 in blocks of
+// 4 waves.)
 // Waves of a block: up to 64 tokens blocks of 128 rows x 4 waves: N = 4096 is 32 of them, which 4-5 K-slices bring to a workgroup for two CUs of three;
 // 256-row blocks x 8 waves need twice the slices (37 tokens, N = K = 4096, with staging: 20.5 us against 22.7).  Longer prompts likewise while the 256-row
 // blocks leave half of the CUs idle, except where the 128-row blocks of a launch without slices are one for 5/8 of the CUs (8 / 4 waves, with staging: N = K = 4096,
@@ -1786,7 +1786,7 @@ void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, in
     int cuts = 1;
     while (cuts < 8 && blocks * cuts < 96 && units >= 8 * cuts) cuts *= 2;
     *runs = 1, *run_units = units;
-    if (longest <= (units + cuts - 1) / cuts || !cut.deep || cut.bm == kBM) return;
+    if (longest <= (units + cuts - 1) / cuts || !cut.deep || cut.bm > 64) return;  // (q4_whole() takes blocks of more than 64 tokens only where they need no runs)
     *run_units = units / cuts / 4 * 4;
     *runs = (longest + *run_units - 1) / *run_units;
 }
@@ -1817,6 +1817,42 @@ void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
         gemm_runs(M, N, K, false, narrow, &runs, &run_units);
         const float us = c.start + (float)((units + ks - 1) / ks) * (c.unit + c.crowd * (float)(blocks * ks) / 256.f) + slices(ks);
         if (us < best && runs <= kMaxRuns && ks * runs <= kMaxSplit) best = us, *cut = narrow;
+    }
+}
+// Int4, from 65 tokens on: whole rows in blocks of 64, 96, 160 or 192 tokens x 8 waves where an estimate takes them for 3 % faster than q4_cut()'s and q4_narrow()'s cut and no accumulator sums
+// more than there; against two workgroups per CU, whose estimate is the least certain, for 7 %, and no blocks of 64 (2048 tokens, N = K = 4096 64 us, in those 66).  Blocks of 64 and 128 tokens
+// leave the rounds of the chip two sizes to fit: 777 tokens, N = 12288, K = 4096, 624 blocks of 64 83.6 us, 240 of 160 67.2; the N = 11008 pair 131 / 112; 450, N = 19968, K = 6656 125 / 98 (160);
+// 130, the N = 11008 pair, 258 blocks of 64 51.2, 172 of 96 42.6; 1500, N = 4096, K = 11008 136 / 114 (96); 384 of the N = 13824 pair, K = 5120 94.7 / 82.7 (192).  The estimate is a start and the
+// rounds one behind the other, as in bf16_cut_long(), fitted to 3000 launches (22 products of 1024 to 24576 rows, 72 to 2048 tokens; 3 to 5 % off on average): of 506 launches a quarter take
+// these blocks, 0.87 times as long as before, none more than 2 % longer, and all together 0.5 % behind the best of each.  Whole prompts of 72 to 2048 tokens, widths 2048 to 6656, one scale per row or groups
+// of 128 columns: 0.965 times as long on average, 0.89 at best, the rest within the noise.
+void q4_whole(int M, int N, int K, bool pair, GemmCut* cut) {
+    struct Kind {
+        int waves, bm, tiles;
+        float start, unit, crowd, slices, bytes;  // (the last two: of the sums of K-slices)
+    };
+    static constexpr Kind whole[] = {{8, 64, 2, 10.63f, 0.715f, 0.054f, 4.06f, 2.86e6f}, {8, 96, 2, 11.03f, 0.981f, 0.126f}, {8, 160, 2, 12.34f, 1.37f, 0.252f}, {8, 192, 2, 13.4f, 1.55f, 0.327f}};
+    static constexpr Kind narrow = {4, 64, 1, 8.35f, 0.261f, 0.154f, 1.33f, 0.77e6f}, half = {4, 64, 2, 10.42f, 0.392f, 0.148f, 6.15f, 5.75e6f}, two_per_cu = {8, kBM, 2, 18.84f, 0.705f, 0.647f, 2.2f, 2.5e6f};
+    if (M <= 64) return;
+    const int units = (K + 127) / 128;
+    auto longest = [&](const GemmCut& c) {  // units of a sum (as good as none where there are more runs than a launch takes)
+        int runs, run_units;
+        gemm_runs(M, N, K, pair, c, &runs, &run_units);
+        return runs > kMaxRuns || c.ksplit * runs > kMaxSplit ? units + 1 : runs > 1 ? run_units : (units + c.ksplit - 1) / c.ksplit;
+    };
+    auto estimate = [&](const Kind& k, int ks) {
+        const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm, k.tiles) * ks;
+        auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (k.unit + k.crowd * (float)of / 256.f); };
+        return k.start + (float)(blocks / 256) * round(256) + round(blocks % 256) + (ks == 1 ? 0.f : k.slices + (float)gemm_part_bytes(M, N, pair, ks) / k.bytes);
+    };
+    const int most = longest(*cut);
+    const bool crowded = cut->bm == kBM;
+    float best = (crowded ? 0.93f : 0.97f) * estimate(crowded ? two_per_cu : cut->tiles == 1 ? narrow : cut->waves == 4 ? half : whole[0], cut->ksplit);
+    for (const Kind& k : whole) {
+        if (crowded && k.bm == 64) continue;
+        const GemmCut c = {k.waves, k.bm, true, 1};
+        const float us = estimate(k, 1);
+        if (us < best && longest(c) <= most) best = us, *cut = c;
     }
 }
 // Up to 64 tokens, outside the fused chain (whose shares are 64 or 128 rows), where blocks of 4 waves do not fill the chip: blocks of 2, 3 or 4 waves (64, 96, 128 rows).  A CU
@@ -1914,7 +1950,7 @@ GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced) {
     const GemmForce fo = gemm_force();
     GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
-    if (!bf16) q4_narrow(M, N, K, pair, chain, &cut);
+    if (!bf16) q4_narrow(M, N, K, pair, chain, &cut), q4_whole(M, N, K, pair, &cut);
     const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep != 2 : cut.deep, cut.ksplit, fo.deep ? (fo.deep == 3 && !pair ? 1 : kTPW) : cut.tiles};
     if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) cut.ksplit = fo.ksplit;
@@ -1924,7 +1960,17 @@ GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sli
 // they take 1 : 1.75 : 1, a round of at most one 128 x 64 block per CU 0.75 (N = 4096, K = 11008: 256 x 64 blocks 104 us at 512 tokens, 106 at 777, 108 at 1000;
 // 256 x 128 165 / 168 / 169; 128 x 64 78 / 106 / 114): the fewest.  1000 tokens, 7B: 235 / 101 / 137 us for c_fc1 / c_fc2, c_proj on average, c_attn with blocks
 // of 64 x 128 one unit ahead -> 185 / 75 / 120.
-GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
+// Blocks of 96 or 160 tokens x 8 waves where an estimate as in q4_whole(), the slices given, takes them for 2 % faster: 777 tokens, N = 12288, K = 4096 104 us in blocks of 64, 89 of 160; 130, the
+// N = 11008 pair 65.9 / 56.5 (96); 1500, N = 4096, K = 11008 170 / 145 (96); 1000, N = K = 4096 48 in blocks of 128 rows x 64 as before (96: 59).  Of 506 launches 104 take them, 0.90 times as long as before, none more
+// than 1 % longer.  (Blocks of 192 tokens would spill; those of 160 hold 24 to 36 bytes a lane of what is made once outside the registers.)
+GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int units, int ksplit) {
+    struct Kind {
+        int waves, bm;
+        float start, unit, crowd;
+        int round;  // blocks that the chip holds
+    };
+    static constexpr Kind kinds[] = {{4, 64, 12.67f, 0.481f, 0.592f, 512}, {8, 64, 13.47f, 0.868f, 0.226f, 256}, {8, kBM, 16.17f, 1.132f, 0.711f, 256}, {8, 96, 14.75f, 1.255f, 0.21f, 256},
+                                     {8, 160, 17.46f, 1.939f, 0.237f, 256}};
     const GemmForce fo = gemm_force();
     GemmCut sh = {4, short_block(M, false), true, ksplit};
     if (M > 64) {
@@ -1938,6 +1984,14 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int ksplit) {
             sh = {8, 128, true, ksplit};
         else if (t_full <= t_half)
             sh.waves = 8;
+        auto estimate = [&](const Kind& k) {
+            const int of = blocks(k.waves, k.bm), rest = of % k.round;
+            const float all = k.unit + k.crowd, part = rest == 0 ? 0.f : k.unit + k.crowd * (float)rest / (float)k.round;
+            return k.start + (float)((units + ksplit - 1) / ksplit) * ((float)(of / k.round) * all + part);
+        };
+        float best = 0.98f * estimate(kinds[sh.bm == kBM ? 2 : sh.waves == 8]);
+        for (int i = 3; i < 5; ++i)
+            if (const float us = estimate(kinds[i]); us < best) best = us, sh.waves = kinds[i].waves, sh.bm = kinds[i].bm;
     }
     const GemmCut forced = {fo.waves ? fo.waves : sh.waves, fo.bm ? fo.bm : sh.bm, true, ksplit};
     return launch_gemm_has(forced, false, false) ? forced : sh;
@@ -1983,6 +2037,9 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
         if (sh.bm == 256) return launch_deep<EPI, PAIR, FMT, 8, 256, FUSE>(p, s);
         return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
     } else {
+        if (sh.bm == 96) return launch_deep<EPI, PAIR, FMT, 8, 96, FUSE>(p, s);
+        if (sh.bm == 160) return launch_deep<EPI, PAIR, FMT, 8, 160, FUSE>(p, s);
+        if (sh.bm == 192) return launch_deep<EPI, PAIR, FMT, 8, 192, FUSE>(p, s);
         if (sh.deep) return launch_deep<EPI, PAIR, FMT, 8, kBM, FUSE>(p, s);
         return launch_gemm_w<EPI, PAIR, 8, kBM, 0, FUSE>(p, s);
     }
@@ -2001,7 +2058,7 @@ int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
     if constexpr (!FUSE) {
         if (subgroups) return launch_gemm_subgroups<EPI, PAIR>(p, s);
     }
-    const GemmCut sh = gemm_cut_grouped(p.n_tiles, p.M, PAIR, p.ksplit);
+    const GemmCut sh = gemm_cut_grouped(p.n_tiles, p.M, PAIR, (p.K + 127) / 128, p.ksplit);
     if (sh.waves == 4) {
         if (sh.bm == 16) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 16, FUSE, 1>(p, s);
         if (sh.bm == 32) return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 32, FUSE, 1>(p, s);
@@ -2009,6 +2066,8 @@ int launch_gemm_grouped(const GemmParams& p, bool subgroups, hipStream_t s) {
         return launch_deep<EPI, PAIR, MI355_W_Q4, 4, 64, FUSE, 1>(p, s);
     }
     if (sh.bm == 64) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 64, FUSE, 1>(p, s);
+    if (sh.bm == 96) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 96, FUSE, 1>(p, s);
+    if (sh.bm == 160) return launch_deep<EPI, PAIR, MI355_W_Q4, 8, 160, FUSE, 1>(p, s);
     return launch_deep<EPI, PAIR, MI355_W_Q4, 8, kBM, FUSE, 1>(p, s);
 }
 template <bool FUSE>
@@ -2090,7 +2149,7 @@ extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, boo
     *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
-    plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
+    plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, (K + 127) / 128, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
 }
 
 // The tables of several products in one launch: a 7B prompt's layers take theirs 10 products at a time, 15 us (13 MB read, 13 written) instead of a launch in front of

@@ -18,6 +18,10 @@ SHAPES = [  # M, N, K
     (300, 12288, 256), (1030, 4096, 384), (2048, 4096, 256), (2050, 8200, 128), (160, 5120, 5120), (330, 6656, 5120), (640, 4096, 11008), (100, 528, 2048),
     (33, 68, 384), (40, 4100, 1024), (64, 6148, 2048), (100, 6144, 2048), (256, 2052, 640), (200, 4112, 4096),  # int4: blocks of 64 rows
 ]
+INT4_WHOLE = [  # M, N, K, pair: blocks of 64, 96, 160 and 192 tokens x 8 waves, whole rows
+    (65, 1028, 1024, 1), (500, 2756, 3328, 0), (193, 2752, 3840, 1), (300, 12292, 4096, 0), (130, 12292, 300, 1), (700, 6148, 2048, 0), (390, 5124, 256, 1), (1300, 4100, 1664, 0), (257, 16388, 512, 1),
+    (770, 12292, 640, 0), (785, 6148, 512, 1), (450, 16388, 1664, 0), (330, 12292, 1024, 1), (385, 16388, 1280, 1), (810, 12292, 4096, 0),
+]
 
 
 @pytest.mark.parametrize("epi", ["store", "accum", "pair"])
@@ -82,6 +86,12 @@ def test_int4_sums_beside_a_large_activation(dev, M, N, K, run):
     assert (got - ref).square().mean().sqrt() <= 1.06 * (4 * run * 5 / 12) ** 0.5 * last_bit
 
 
+@pytest.mark.parametrize("M,N,K,pair", INT4_WHOLE)
+def test_int4_blocks_of_whole_rows_against_64_bits(dev, M, N, K, pair):
+    """A few tokens or rows more than whole blocks, rows shorter than the pipeline and ends of it, runs and none (tests/test_host_logic.py compares the list with the rule)."""
+    test_tiled_product_against_64_bits(dev, "q4", M, N, K, "pair" if pair else "accum")
+
+
 BF16_BLOCKS = [
     (512, 4096, 1664, 0), (257, 12288, 1664, 0), (257, 1000, 1664, 0), (449, 4112, 1664, 0), (512, 4112, 1664, 0), (193, 12288, 2176, 0), (500, 6160, 640, 0),
     (320, 12288, 2176, 0), (512, 12288, 640, 0), (1025, 6160, 256, 0), (769, 12288, 2176, 0), (1281, 6160, 2176, 0), (1281, 8200, 256, 0), (1025, 12288, 2048, 0),
@@ -112,20 +122,11 @@ def test_bf16_blocks_of_every_size_against_64_bits(dev, M, N, K, pair):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
-BF16_CHAIN = [
-    (640, 65), (640, 1094), (1024, 709), (1280, 65), (1280, 1731), (1920, 65), (1920, 646), (1920, 1633), (2048, 261), (2560, 65), (2560, 1542), (2560, 1605), (3072, 65),
-    (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1542), (6656, 1731), (6656, 1878),
-]
-
-
-@pytest.mark.parametrize("width,T", BF16_CHAIN)
-def test_fused_prompt_chain_of_bf16_layers(dev, monkeypatch, width, T):
-    """The chain's shares, rotations and cache rows in every block that its products take (tests/test_host_logic.py compares the list with the rule), a last block that is not
-    whole.  0.02 of the logits' spread as in test_runs_of_shares_in_the_fused_prompt_chain."""
+def _chain_against_staging(dev, monkeypatch, width, T, mode):
     cfg = LLaMAConfig(block_size=T + 4, n_layer=2, n_head=width // 128, n_embd=width, vocab_size=512)
-    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16):
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=mode):
         model = LLaMA(cfg)
-    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode=None, device="cuda", dtype=torch.bfloat16))
+    model.load_state_dict(synth.make_state_dict(cfg, seed=3, mode=mode, device="cuda", dtype=torch.bfloat16))
     model.eval()
     idx = synth.make_prompt(T, vocab=512).to(dev)
     out = []
@@ -138,9 +139,32 @@ def test_fused_prompt_chain_of_bf16_layers(dev, monkeypatch, width, T):
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
 
 
+INT4_CHAIN = [(2048, 400), (2048, 730), (2048, 850), (4096, 180), (4096, 450), (4096, 700), (4096, 777), (4096, 850)]
+
+
+@pytest.mark.parametrize("width,T", INT4_CHAIN)
+def test_fused_prompt_chain_of_int4_layers_in_blocks_of_whole_rows(dev, monkeypatch, width, T):
+    """As test_fused_prompt_chain_of_bf16_layers, for the blocks of 64, 96, 160 and 192 tokens x 8 waves of one scale per row."""
+    _chain_against_staging(dev, monkeypatch, width, T, "gptq.int4")
+
+
+BF16_CHAIN = [
+    (640, 65), (640, 1094), (1024, 709), (1280, 65), (1280, 1731), (1920, 65), (1920, 646), (1920, 1633), (2048, 261), (2560, 65), (2560, 1542), (2560, 1605), (3072, 65),
+    (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1542), (6656, 1731), (6656, 1878),
+]
+
+
+@pytest.mark.parametrize("width,T", BF16_CHAIN)
+def test_fused_prompt_chain_of_bf16_layers(dev, monkeypatch, width, T):
+    """The chain's shares, rotations and cache rows in every block that its products take (tests/test_host_logic.py compares the list with the rule), a last block that is not
+    whole.  0.02 of the logits' spread as in test_runs_of_shares_in_the_fused_prompt_chain."""
+    _chain_against_staging(dev, monkeypatch, width, T, None)
+
+
 @pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K,cols", [(1, 16, 256, 128), (16, 144, 2176, 128), (17, 4096, 1280, 256), (33, 12288, 512, 128), (64, 128, 11008, 512), (65, 4096, 4096, 128),
-                                        (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128)])
+                                        (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128),
+                                        (385, 15364, 1280, 128), (1300, 4100, 256, 128), (770, 12292, 640, 256), (1500, 6148, 128, 128), (450, 16388, 1664, 128)])  # blocks of 96 and 160 tokens
 def test_tiled_product_of_grouped_scales_against_64_bits(dev, M, N, K, cols, x_dtype):
     """Groups of whole units: the products of a unit are sums of 128 terms of up to 143 x, the zero points a sum of their own: 1e-3 of the result as above.
     Rows whose addresses are no multiple of 16 B take the staging pass of single loads."""
@@ -357,7 +381,8 @@ def test_operand_slices_of_few_bf16_rows(dev, M, rows, n, K):
     assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-3 * ref.square().mean().sqrt()).all()
 
 
-@pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600)])
+@pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600),
+                                            (128, 32, 180), (256, 32, 450), (128, 32, 650)])
 def test_fused_prompt_chain_over_grouped_scales(dev, monkeypatch, cols, heads, T):
     """Groups of whole units in the chain: one share per unit, or two (c_fc1 / c_fc2 in blocks of 64 hidden rows); slices and whole sums; tables of several layers from one
     launch and the next.  Against the same layers with staging passes, 0.02 of the logits' spread as for one scale per row."""

@@ -655,9 +655,9 @@ def test_partial_sums_of_slices_fit_their_buffer(bf16):
             assert (ks == 1 or ppu == 1) and shares * 128 >= N * ppu
 
 
-def _gemm_cut(M, N, K, R, chain, sliced=False):
+def _gemm_cut(M, N, K, R, chain, sliced=False, bf16=True):
     out = [C.c_int(0) for _ in range(3)]
-    nat.lib().mi355_linear_gemm_cut(M, N, K, R, C.c_bool(True), C.c_bool(chain), C.c_bool(sliced), *[C.byref(v) for v in out])
+    nat.lib().mi355_linear_gemm_cut(M, N, K, R, C.c_bool(bf16), C.c_bool(chain), C.c_bool(sliced), *[C.byref(v) for v in out])
     return tuple(v.value for v in out)
 
 
@@ -707,6 +707,39 @@ def test_gpu_tests_of_bf16_blocks_run_every_block():
         waves, tokens, slices = _gemm_cut(M, N, K, 1 + pair, False)
         run.add(("pair" if pair else "single", waves, tokens, slices > 1))
     assert {("pair" if role == "pair" else "single", *c) for role, *c in taken} <= run
+
+
+def test_gpu_tests_of_int4_blocks_run_every_block_of_whole_rows():
+    """Blocks of 8 waves, each number of tokens, of single products and pairs, outside the chain; inside it those that layers of 2048 and 4096 columns take."""
+    shapes = _gemm_shapes()
+    cuts = lambda sizes, chain: {(R, *_gemm_cut(M, N, K, R, chain, bf16=False)) for M, N, K, R in sizes}  # noqa: E731
+    blocks = {(R, 8, tokens, 1) for R in (1, 2) for tokens in (64, 96, 160, 192)}
+    assert cuts([(M, N, K, 1 + pair) for M, N, K, pair in shapes.INT4_WHOLE], False) == blocks
+
+    def layer(width, T):
+        hidden = find_multiple(int(8 * width / 3), 256)
+        return [(T, 3 * width, width, 1), (T, width, width, 1), (T, width, hidden, 1), (T, hidden, width, 2)]
+
+    run = cuts([p for width, T in shapes.INT4_CHAIN for p in layer(width, T)], True)
+    assert {c for width in (2048, 4096) for T in range(65, 1000) for c in cuts(layer(width, T), True)} & blocks <= run
+
+
+def test_int4_blocks_of_whole_rows_sum_no_more_than_a_launch_holds():
+    """A slice of several runs has at most 8 of them, a row 16 sums: no launch is cut into more, and blocks of more than 64 tokens, which take no runs, are left where sums end within a row."""
+    for K in list(range(128, 4353, 128)) + [11008, 13824]:
+        units = -(-K // 128)
+        for N in (64, 256, 1000, 1796, 2752, 4096, 6144, 11008, 16384):
+            for M in (65, 96, 130, 193, 385, 500, 700, 1300):
+                for R in (1, 2):
+                    waves, tokens, slices = _gemm_cut(M, N, K, R, False, bf16=False)
+                    if waves != 8 or slices != 1 or tokens == 128:
+                        continue
+                    blocks, cuts = -(-N // (256 // R)) * -(-M // 128), 1
+                    while cuts < 8 and blocks * cuts < 96 and units >= 8 * cuts:
+                        cuts *= 2
+                    run = units // cuts // 4 * 4
+                    runs = 1 if cuts == 1 or units <= -(-units // cuts) else -(-units // run)
+                    assert runs <= (8 if tokens == 64 else 1), (M, N, K, R, waves, tokens)
 
 
 def _forced_plans(value):
