@@ -139,7 +139,7 @@ def _chain_against_staging(dev, monkeypatch, width, T, mode):
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()
 
 
-INT4_CHAIN = [(2048, 400), (2048, 730), (2048, 850), (4096, 180), (4096, 450), (4096, 700), (4096, 777), (4096, 850)]
+INT4_CHAIN = [(2048, 130), (2048, 400), (2048, 730), (2048, 850), (4096, 180), (4096, 300), (4096, 450), (4096, 700), (4096, 777), (4096, 850)]
 
 
 @pytest.mark.parametrize("width,T", INT4_CHAIN)
