@@ -1823,7 +1823,7 @@ void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
 // more than there; against two workgroups per CU, whose estimate is the least certain, for 7 %, and no blocks of 64 (2048 tokens, N = K = 4096 64 us, in those 66).  Blocks of 64 and 128 tokens
 // leave the rounds of the chip two sizes to fit: 777 tokens, N = 12288, K = 4096, 624 blocks of 64 83.6 us, 240 of 160 67.2; the N = 11008 pair 131 / 112; 450, N = 19968, K = 6656 125 / 98 (160);
 // 130, the N = 11008 pair, 258 blocks of 64 51.2, 172 of 96 42.6; 1500, N = 4096, K = 11008 136 / 114 (96); 384 of the N = 13824 pair, K = 5120 94.7 / 82.7 (192).  The estimate is a start and the
-// rounds one behind the other, as in bf16_cut_long(), fitted to 3000 launches (22 products of 1024 to 24576 rows, 72 to 2048 tokens; 3 to 5 % off on average): of 506 launches a quarter take
+// rounds one behind the other, as in bf16_cut_long(), fitted to 3000 launches (profiles/product_cuts_int4.txt: 22 products of 1024 to 24576 rows, 72 to 2048 tokens; 3 to 5 % off on average): of 506 launches a quarter take
 // these blocks, 0.87 times as long as before, none more than 2 % longer, and all together 0.5 % behind the best of each.  Whole prompts of 72 to 2048 tokens, widths 2048 to 6656, one scale per row or groups
 // of 128 columns: 0.965 times as long on average, 0.89 at best, the rest within the noise.
 void q4_whole(int M, int N, int K, bool pair, GemmCut* cut) {
