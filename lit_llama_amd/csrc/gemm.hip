@@ -94,7 +94,7 @@ struct GemmParams {
     float limit;           // CLAMPGLU
     const float* bias;     // STORE: [N], or NULL
     mi355_reduce_norm rn;  // rn.done: the sum of the K-slices also leaves the rows' norm
-    bool squares;          // BF16, 8 waves: an XCD's blocks are kSquare row blocks by some token blocks (square_blocks())
+    bool squares;          // BF16 blocks that may_run_in_squares(): an XCD's blocks are kSquare row blocks by some token blocks (square_blocks())
     int slice_blocks;      // != 0: row blocks [i slice_blocks, (i + 1) slice_blocks) read the operand at xb + i slice_stride
     int64_t slice_stride;
     // grouped scales (GRP kernels): gtab[group 0..n_groups][r][tab_ld rows] = bf16 scale | bf16 zero << 16 (row n_groups
@@ -139,7 +139,6 @@ constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials 
 constexpr int kMaxSplit = 16;
 constexpr int kMaxRuns = 8;
 constexpr int kTableProducts = MI355_TABLE_PRODUCTS;
-constexpr int kSquare = 4;                        // row blocks of a square (GemmParams::squares)
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
 // first unit of K-slice s of `ksplit` (slice s = units [lo(s), lo(s + 1)))
@@ -1126,15 +1125,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     const int m_blocks = p.total_blocks / n_blocks;
     int mb, nb;
     if constexpr (FMT == MI355_W_BF16) {  // (orders: see gemm_q4_kernel)
-        nb = L / m_blocks;
-        mb = L - nb * m_blocks;
-        if constexpr (kWaves == 8) {
-            if (p.squares) {
-                const int first = nb / kSquare * kSquare, at = L - first * m_blocks, rows = n_blocks - first < kSquare ? n_blocks - first : kSquare;
-                mb = rows == kSquare ? at / kSquare : at / rows;
-                nb = first + at - mb * rows;
-            }
-        }
+        const BlockAt at = block_at(L, n_blocks, m_blocks, may_run_in_squares(kWaves, BM) && p.squares);
+        nb = at.nb, mb = at.mb;
     } else {
         mb = L / n_blocks;
         nb = L - mb * n_blocks;
@@ -1151,7 +1143,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     for (int t = 0; t < TPW; ++t)
         tile[t] = PAIR ? nb * (kSlots / 2) + (TPW / 2) * wave + (t >> 1) : nb * kSlots + TPW * wave + t;
     // this block's share of its row block's weights (see above): thread i's line of every round of DEPTH units, at touch_off from the round's first unit
-    constexpr bool kTouch = FMT == MI355_W_BF16 && (BM == 64 || (BM > 64 && kWaves == 4));
+    constexpr bool kTouch = FMT == MI355_W_BF16 && shares_weights(kWaves, BM);
     constexpr int kTouchAhead = 2 * DEPTH - 1, kStreams = PAIR ? kSlots / 2 : kSlots, kRun = DEPTH * (PAIR ? 64 : 32);  // kRun: lines of DEPTH units of a tile
     constexpr unsigned kNone = 0xFFFFFFF0u;
     [[maybe_unused]] unsigned touch_off = kNone;

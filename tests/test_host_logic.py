@@ -821,6 +821,57 @@ def test_objects_follow_every_header_that_a_source_includes():
             assert any((d / name).resolve() in watched for d in (f.parent, _build.PKG.parent / "include")), (f.name, name)
 
 
+def test_blocks_that_share_out_weights_run_in_the_order_of_their_shares(tmp_path):
+    """csrc/l2_share.h in the order that gemm_deep_kernel walks, with and without squares: every block of every kind runs once, and where blocks share out a row block's weights each line is
+    brought once, none twice and none of another row block's (64 tokens x 8 waves in squares: 1300 tokens of N = K = 3072 asked for 2645 lines in front of their row block)."""
+    import subprocess
+
+    from lit_llama_amd import _build
+
+    (tmp_path / "t.cpp").write_text(r"""
+#define __host__
+#define __device__
+#include "l2_share.h"
+#include <cstdio>
+#include <vector>
+int main() {
+    const int lines = 1024, waves[] = {2, 3, 4, 8}, tokens[] = {16, 32, 64, 96, 128, 160, 192, 208, 256};
+    for (int w : waves)
+        for (int t : tokens)
+            for (bool squares : {false, true})
+                for (int n_blocks : {1, 2, 3, 4, 5, 7, 12, 26, 33})
+                    for (int m_blocks : {1, 3, 4, 9, 13, 21, 31}) {
+                        const int total = n_blocks * m_blocks, per_xcd = (total + 7) / 8;
+                        std::vector<int> ran(total);
+                        for (int xcd = 0; xcd < 8; ++xcd) {
+                            std::vector<std::vector<int>> brought(n_blocks, std::vector<int>(lines));
+                            std::vector<int> here(n_blocks);
+                            for (int L = xcd * per_xcd; L < (xcd + 1) * per_xcd && L < total; ++L) {
+                                const BlockAt at = block_at(L, n_blocks, m_blocks, squares && may_run_in_squares(w, t));
+                                if (at.nb < 0 || at.nb >= n_blocks || at.mb < 0 || at.mb >= m_blocks) return std::printf("block %d runs as %d, %d", L, at.nb, at.mb), 1;
+                                ran[at.nb * m_blocks + at.mb]++, here[at.nb]++;
+                                if (!shares_weights(w, t)) continue;
+                                const L2Share s = l2_share(lines, L, at.nb, m_blocks, 1, xcd, per_xcd);
+                                for (int i = s.first; i < s.first + s.count && i < lines; ++i) {
+                                    if (i < 0) return std::printf("%d waves x %d tokens: a line in front of the row block's", w, t), 1;
+                                    brought[at.nb][i]++;
+                                }
+                            }
+                            for (int nb = 0; shares_weights(w, t) && nb < n_blocks; ++nb)
+                                for (int n : brought[nb])
+                                    if (n != (here[nb] >= 4)) return std::printf("%d waves x %d tokens: a line %d times, %d blocks", w, t, n, here[nb]), 1;
+                        }
+                        for (int n : ran)
+                            if (n != 1) return std::printf("a block runs %d times", n), 1;
+                    }
+    return shares_weights(8, 64) && shares_weights(4, 128) && may_run_in_squares(8, 128) ? 0 : 2;
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=all", f"-I{_build.CSRC}", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")], check=True)
+    r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
 def test_shares_of_a_row_blocks_weights(tmp_path):
     """csrc/l2_share.h, built for the host with division checked: the blocks of a row block on one XCD bring each of its lines once, no share is longer than the smallest
     workgroup that takes one (4 waves, 1024 lines), and a launch in K-slices, whose places on an XCD count slices, asks for none."""
