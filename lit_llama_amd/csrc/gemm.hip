@@ -1782,13 +1782,20 @@ void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, in
     *run_units = units / cuts / 4 * 4;
     *runs = (longest + *run_units - 1) / *run_units;
 }
+// ... and how many of them that are in this cut
+int gemm_longest(int M, int N, int K, bool pair, const GemmCut& cut) {
+    int runs, run_units;
+    gemm_runs(M, N, K, pair, cut, &runs, &run_units);
+    return runs > 1 ? run_units : ((K + 127) / 128 + cut.ksplit - 1) / cut.ksplit;
+}
 // Int4 products other than pairs, where blocks of 64 rows x 4 waves are one per CU at most: a wave of one row tile.  A wave alone on its SIMD is bound by what it issues (37 tokens: two row tiles take
 // 0.45 us a unit, one 0.31 to 0.34, with all operands in the L2 caches as well, and no barrier 0.42), so half the rows per wave on idle CUs are worth more than K-slices, whose sums are a launch more:
 // 37 tokens, N = 12288, K = 4096 20.6 us in two slices of 128-row blocks, 18.1 whole in 64-row blocks; N = K = 4096 16.2 in 8 slices, 15.4 in 4; 128 tokens, N = 6144, K = 2048 19.6 / 14.5.  The
 // estimate: per unit of a slice `unit` us and `crowd` more when every CU has a block, `slices` and `bytes` for partial sums, fitted to 1422 launches (18 products of 1024 to 32000 rows, 32 to 300
 // tokens, weights in no cache; 7 % off on average).  Where it takes these blocks or not: 0.96 / 0.95 / 0.94 / 0.93 times the time of 128-row blocks (32, to 48, to 64, more tokens), 3 % slower at worst.
 // In the chain, whose blocks add up shares first and whose sums of slices write the next ones, whole rows only (37 tokens, 7B: c_attn 12.8 + 4.2 us for the sum of its slices -> 15.9; attn.c_proj in 4
-// narrow slices 8.4 + 4.2, in 8 wide ones 7.8 + 4.4).
+// narrow slices 8.4 + 4.2, in 8 wide ones 7.8 + 4.4).  No accumulator sums more than in the cut that they replace: N = 1024, K = 3584 in 4 slices of 7 units for 7 of 4 rounds beside an activation of
+// 2^17 by 2.1 last bits rms for 1.7.
 void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
     struct Cost {
         float start, wide, wide_crowd, unit, crowd, slices, bytes;
@@ -1802,13 +1809,13 @@ void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
     const Cost& c = costs[M <= 32 ? 0 : M <= 48 ? 1 : M <= 64 ? 2 : 3];
     auto slices = [&](int ks) { return ks == 1 ? 0.f : c.slices + (float)gemm_part_bytes(M, N, false, ks) / c.bytes; };
     float best = (float)((units + cut->ksplit - 1) / cut->ksplit) * (c.wide + c.wide_crowd * (float)wide / 256.f) + slices(cut->ksplit);
-    const int bm = cut->bm, blocks = gemm_blocks(M, N, false, 4, bm, 1);
+    const int bm = cut->bm, blocks = gemm_blocks(M, N, false, 4, bm, 1), most = gemm_longest(M, N, K, false, *cut);
     for (int ks = 1; ks <= (chain ? 1 : 8) && blocks * ks <= 256 && (ks == 1 || (units >= 2 * ks && gemm_part_bytes(M, N, false, ks) <= kSplitBudget / 2)); ++ks) {
         const GemmCut narrow = {4, bm, true, ks, 1};
         int runs, run_units;
         gemm_runs(M, N, K, false, narrow, &runs, &run_units);
         const float us = c.start + (float)((units + ks - 1) / ks) * (c.unit + c.crowd * (float)(blocks * ks) / 256.f) + slices(ks);
-        if (us < best && runs <= kMaxRuns && ks * runs <= kMaxSplit) best = us, *cut = narrow;
+        if (us < best && runs <= kMaxRuns && ks * runs <= kMaxSplit && gemm_longest(M, N, K, false, narrow) <= most) best = us, *cut = narrow;
     }
 }
 // Int4, from 65 tokens on: whole rows in blocks of 64, 96, 160 or 192 tokens x 8 waves where an estimate takes them for 3 % faster than q4_cut()'s and q4_narrow()'s cut and no accumulator sums
@@ -2139,6 +2146,12 @@ extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, in
 extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, bool sliced, int* waves, int* tokens, int* ksplit) {
     const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain, sliced);
     *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
+}
+extern "C" void mi355_linear_gemm_sums(int M, int N, int K, int R, bool chain, int* tiles, int* ksplit, int* runs, int* longest, int* longest_of_wide) {
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, false, chain, false);
+    int run_units;
+    gemm_runs(M, N, K, R == 2, cut, runs, &run_units);
+    *tiles = cut.tiles, *ksplit = cut.ksplit, *longest = gemm_longest(M, N, K, R == 2, cut), *longest_of_wide = gemm_longest(M, N, K, R == 2, q4_cut(M, N, K, R == 2));
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
     plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, (K + 127) / 128, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);

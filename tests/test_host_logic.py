@@ -742,6 +742,29 @@ def test_int4_blocks_of_whole_rows_sum_no_more_than_a_launch_holds():
                     assert runs <= (8 if tokens == 64 else 1), (M, N, K, R, waves, tokens)
 
 
+def _int4_sums(M, N, K, R, chain):
+    """Row tiles of a wave, K-slices, runs of a slice, units of one sum, units of one in the blocks that the rule starts from."""
+    out = [C.c_int(0) for _ in range(5)]
+    nat.lib().mi355_linear_gemm_sums(M, N, K, R, C.c_bool(chain), *[C.byref(v) for v in out])
+    return tuple(v.value for v in out)
+
+
+def _int4_products():
+    for K in list(range(128, 8193, 128)) + [11008, 13824, 17920, 22016]:
+        for N in (64, 320, 576, 704, 1024, 1472, 1792, 2176, 2368, 2752, 3072, 4096, 6528, 12288):
+            for M in (1, 16, 33, 64, 65, 97, 160, 200, 256, 384, 512, 777):
+                yield from ((M, N, K, R) for R in (1, 2))
+
+
+def test_int4_sums_are_no_longer_than_in_the_blocks_that_the_rule_starts_from():
+    """256 tokens, N = 1024, K = 3584: blocks of 64 rows in 4 slices would sum 7 units where blocks of 128 rows in 7 slices sum 4, and round by 2.1 last bits for 1.7 beside a large activation."""
+    assert _int4_sums(256, 1024, 3584, 1, False)[3] == 4
+    for M, N, K, R in _int4_products():
+        for chain in (False, True):
+            *_, longest, wide = _int4_sums(M, N, K, R, chain)
+            assert longest <= wide, (M, N, K, R, chain)
+
+
 def _forced_plans(value):
     """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
     import os
