@@ -138,6 +138,7 @@ __device__ __forceinline__ void store_q_ready(const GemmParams& p, int m, int n,
 constexpr size_t kSplitBudget = (size_t)32 << 20;  // bytes of split-K partials a workspace holds
 constexpr int kMaxSplit = 16;
 constexpr int kMaxRuns = 8;
+constexpr int kMaxSums = 32;                       // operand sums of a row: K-slices x runs.  Slices are 7 at most where they have several runs (gemm_runs()): below units / run_units + 9
 constexpr int kTableProducts = MI355_TABLE_PRODUCTS;
 constexpr int kSharesAhead = 8;                   // partial sums that a thread of gemm_deep_kernel requests at a time
 constexpr size_t kFuseScratch = (size_t)8 << 20;  // partial sums of the fused prompt chain: <= 2048 tokens x ~500 shares x 4 B
@@ -1782,7 +1783,12 @@ void gemm_runs(int M, int N, int K, bool pair, const GemmCut& cut, int* runs, in
     *run_units = units / cuts / 4 * 4;
     *runs = (longest + *run_units - 1) / *run_units;
 }
-// ... and how many of them that are in this cut
+// ... whether a launch holds the sums of its rows (the rules' cuts do: at most 8 runs, 21 sums), and how many units one is in this cut
+bool gemm_sums_fit(int M, int N, int K, bool pair, const GemmCut& cut) {
+    int runs, run_units;
+    gemm_runs(M, N, K, pair, cut, &runs, &run_units);
+    return runs <= kMaxRuns && cut.ksplit * runs <= kMaxSums;
+}
 int gemm_longest(int M, int N, int K, bool pair, const GemmCut& cut) {
     int runs, run_units;
     gemm_runs(M, N, K, pair, cut, &runs, &run_units);
@@ -1952,7 +1958,11 @@ GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sli
     if (!bf16) q4_narrow(M, N, K, pair, chain, &cut), q4_whole(M, N, K, pair, &cut);
     const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep != 2 : cut.deep, cut.ksplit, fo.deep ? (fo.deep == 3 && !pair ? 1 : kTPW) : cut.tiles};
     if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
-    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) cut.ksplit = fo.ksplit;
+    if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) {
+        GemmCut sliced_so = cut;
+        sliced_so.ksplit = fo.ksplit;
+        if (bf16 || gemm_sums_fit(M, N, K, pair, sliced_so)) cut = sliced_so;
+    }
     return cut;
 }
 // Grouped scales, groups of whole units.  Blocks of 256 rows x 64 tokens and of 256 x 128 fill a CU alone, two of 128 x 64 share one; per round of the chip
@@ -2087,7 +2097,7 @@ int launch_gemm_epi(const GemmParams& p, int epi, hipStream_t s) {
 }
 
 // floats from the 1/rms of the staged rows to their operand sums per unit
-size_t unit_sums_at(int M) { return (size_t)M * (1 + kMaxSplit); }
+size_t unit_sums_at(int M) { return (size_t)M * (1 + kMaxSums); }
 
 }  // namespace
 
@@ -2266,6 +2276,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
         const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr, a->slice_rows != 0);
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
+        MI355_CHECK_ARG(runs <= kMaxRuns && ksplit * runs <= kMaxSums, MI355_E_STATE, "linear_gemm: %d slices of %d runs (M=%d N=%d K=%d)", ksplit, runs, a->M, a->N, a->K);
     }
     // producer / consumer fusion (gemm_fuse.h): one scale per row, or groups of whole units — the caller plans with mi355_linear_gemm_plan or ..._grouped
     const bool fused = f != nullptr;

@@ -765,6 +765,49 @@ def test_int4_sums_are_no_longer_than_in_the_blocks_that_the_rule_starts_from():
             assert longest <= wide, (M, N, K, R, chain)
 
 
+def _sums_of_a_row(K):
+    """Operand sums that the scratch of a launch holds a row: what is left of it beside the staged row, its 1/rms and its sums per unit."""
+    size, units = nat.lib().mi355_linear_gemm_workspace_bytes, -(-K // 128)
+    return (size(1001, K) - size(1000, K) - units * 256 - units * 4 - 4) // 4
+
+
+def test_operand_sums_of_int4_slices_fit_their_place():
+    """A slice has 8 runs at most (a workgroup keeps their operand sums in LDS), and slices x runs of a row have a place of their own in the scratch (777 tokens, N = 320, K = 6272:
+    6 slices of 3 runs)."""
+    for M, N, K, R in _int4_products():
+        for chain in (False, True):
+            _, slices, runs, *_ = _int4_sums(M, N, K, R, chain)
+            assert runs <= 8 and slices * runs <= _sums_of_a_row(K), (M, N, K, R, chain)
+
+
+def _in_a_process_with(force, code):
+    import os
+    import subprocess
+    import sys
+
+    out = subprocess.run([sys.executable, "-c", code, str(nat.LIB_PATH)], env={**os.environ, "MI355_GEMM_FORCE": force}, capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    return [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
+
+
+CUTS = """
+import ctypes as C, sys
+lib = C.CDLL(sys.argv[1])
+for M, N, K, R in ((37, 12288, 4096, 1), (100, 6144, 2048, 1), (40, 1024, 4480, 1), (777, 12288, 4096, 1), (450, 4096, 4096, 1), (700, 11008, 4096, 2)):
+    o, q = [C.c_int(0) for _ in range(3)], [C.c_int(0) for _ in range(5)]
+    lib.mi355_linear_gemm_cut(M, N, K, R, C.c_bool(False), C.c_bool(False), C.c_bool(False), *[C.byref(v) for v in o])
+    lib.mi355_linear_gemm_sums(M, N, K, R, C.c_bool(False), *[C.byref(v) for v in q])
+    print(M, R, *[v.value for v in o], q[0].value, q[2].value)
+"""
+
+
+def test_forced_slices_of_more_runs_than_a_launch_holds_are_ignored():
+    """40 tokens, N = 1024, K = 4480 in one slice would be 9 runs of 4 units."""
+    for rule, forced in zip(_in_a_process_with("", CUTS), _in_a_process_with("0:0:1", CUTS)):
+        assert forced[-1] <= 8 and (forced[4] == 1 or forced == rule), forced
+    assert _in_a_process_with("0:0:1", CUTS)[2] == _in_a_process_with("", CUTS)[2]
+
+
 def _forced_plans(value):
     """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
     import os
