@@ -1709,8 +1709,9 @@ struct GemmCut {
     int ksplit;
     int tiles = kTPW;  // row tiles of a wave
 };
-// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep" (deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel, the latter int4 only), 0 = the rule's choice.  A cut that
-// no kernel is instantiated for is ignored as a whole, a number of slices that does not fit by itself; blocks that only BF16 streams have need the kernel named (deep = 1)
+// tuning override for sweeps: MI355_GEMM_FORCE="waves:bm:ksplit:deep", 0 = the rule's choice.  deep: 1 / 2 for gemm_deep_kernel / gemm_q4_kernel (the latter int4 only), of int4 3 for waves of
+// one row tile (q4_narrow()) and 4 for blocks of 96 to 192 tokens x 8 waves (q4_whole(), grouped scales of whole units 96 and 160).  Where waves, tokens or 1 / 2 are given, the rest is
+// q4_cut()'s, with 3 and 4 the rule's as a whole.  A cut that no kernel is instantiated for is ignored as a whole, a number of slices that does not fit by itself; blocks that only BF16 streams have need the kernel named (deep = 1)
 struct GemmForce {
     int waves, bm, ksplit, deep;
 };
@@ -1724,9 +1725,10 @@ GemmForce gemm_force() {
     }();
     return f;
 }
-bool launch_gemm_has(const GemmCut& c, bool bf16, bool named) {  // (what a sweep may force of the kernels of launch_gemm())
+bool launch_gemm_has(const GemmCut& c, bool bf16, int kernel, bool grouped = false) {  // (what a sweep may force of the kernels of launch_gemm(); kernel: GemmForce::deep)
     if (c.tiles == 1) return !bf16 && c.waves == 4 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 48 || c.bm == 64);
-    if (bf16 && named && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 160 || c.bm == 192 || c.bm == 208 || c.bm == 256)))) return true;
+    if (kernel == 4) return !bf16 && c.waves == 8 && (c.bm == 96 || c.bm == 160 || (c.bm == 192 && !grouped));
+    if (bf16 && kernel == 1 && ((c.waves == 4 && (c.bm == 96 || c.bm == kBM)) || (c.waves == 8 && (c.bm == 160 || c.bm == 192 || c.bm == 208 || c.bm == 256)))) return true;
     if (c.waves == 2 || c.waves == 3) return bf16 && c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64);
     if (c.waves == 4) return c.deep && (c.bm == 16 || c.bm == 32 || c.bm == 64 || (c.bm == 48 && !bf16));
     return c.waves == 8 && (c.bm == kBM || c.bm == 64) && (c.deep || (!bf16 && c.bm == kBM));
@@ -1954,10 +1956,12 @@ GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {
 // chain: a launch of the fused prompt chain (gemm_fuse.h); sliced: a launch of operand slices
 GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced) {
     const GemmForce fo = gemm_force();
-    GemmCut cut = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
+    const GemmCut first = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
+    GemmCut cut = first;
     if (!bf16) q4_narrow(M, N, K, pair, chain, &cut), q4_whole(M, N, K, pair, &cut);
-    const GemmCut forced = {fo.waves ? fo.waves : cut.waves, fo.bm ? fo.bm : cut.bm, fo.deep ? fo.deep != 2 : cut.deep, cut.ksplit, fo.deep ? (fo.deep == 3 && !pair ? 1 : kTPW) : cut.tiles};
-    if (launch_gemm_has(forced, bf16, fo.deep == 1) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
+    const GemmCut& from = fo.deep >= 3 || (fo.waves == 0 && fo.bm == 0 && fo.deep == 0) ? cut : first;
+    const GemmCut forced = {fo.waves ? fo.waves : from.waves, fo.bm ? fo.bm : from.bm, fo.deep ? fo.deep != 2 : from.deep, from.ksplit, fo.deep == 3 && !pair ? 1 : fo.deep ? kTPW : from.tiles};
+    if (launch_gemm_has(forced, bf16, fo.deep) && (!chain || forced.waves >= 4) && (!sliced || forced.waves != 3)) cut = forced;
     if (fo.ksplit >= 1 && fo.ksplit <= kMaxSplit && (K + 127) / 128 >= fo.ksplit && gemm_part_bytes(M, N, pair, fo.ksplit) <= (bf16 ? kSplitBudget : kSplitBudget / 2)) {
         GemmCut sliced_so = cut;
         sliced_so.ksplit = fo.ksplit;
@@ -2003,7 +2007,7 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int units, int ksplit) {
             if (const float us = estimate(kinds[i]); us < best) best = us, sh.waves = kinds[i].waves, sh.bm = kinds[i].bm;
     }
     const GemmCut forced = {fo.waves ? fo.waves : sh.waves, fo.bm ? fo.bm : sh.bm, true, ksplit};
-    return launch_gemm_has(forced, false, false) ? forced : sh;
+    return launch_gemm_has(forced, false, fo.deep == 4 ? 4 : 0, true) ? forced : sh;
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {

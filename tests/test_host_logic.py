@@ -808,6 +808,22 @@ def test_forced_slices_of_more_runs_than_a_launch_holds_are_ignored():
     assert _in_a_process_with("0:0:1", CUTS)[2] == _in_a_process_with("", CUTS)[2]
 
 
+def test_int4_blocks_are_forced_whatever_the_rule_takes():
+    """Also where it takes waves of one row tile (37 x 12288 x 4096) or blocks of 160 tokens (777 x 12288 x 4096); those two by numbers of their own."""
+    rule = _in_a_process_with("", CUTS)
+    assert {tiles for *_, tiles, _ in rule} == {1, 2} and any(tokens > 64 and tokens != 128 for _, _, _, tokens, *_ in rule)
+    for waves, tokens in ((8, 64), (4, 64), (8, 128), (4, 32)):
+        for kernel in ("", ":0", ":1"):
+            for M, R, w, t, _, tiles, _ in _in_a_process_with(f"{waves}:{tokens}:0{kernel}", CUTS):
+                if kernel == ":1" or R == 1:  # (the pair's kernel, if none is named, is the one of 128 tokens x 8 waves alone)
+                    assert (w, t, tiles) == (waves, tokens, 2), (M, R)
+    for M, R, w, t, ks, tiles, _ in _in_a_process_with("4:64:1:3", CUTS):
+        assert (w, t, tiles) == (4, 64, 2 if R == 2 else 1), (M, R)
+    for tokens in (96, 160, 192):
+        for M, R, w, t, ks, tiles, _ in _in_a_process_with(f"8:{tokens}:1:4", CUTS):
+            assert (w, t, tiles) == (8, tokens, 2) and (ks == 1 or M == 40), (M, R)
+
+
 def _forced_plans(value):
     """Plans of a process in which MI355_GEMM_FORCE (read once) has this value."""
     import os
