@@ -1087,9 +1087,9 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // The same product for launches that leave a CU one or two workgroups (short prompts, batches of decoding sequences, the N = 4096 products of longer ones):
 // there nothing else covers a unit's memory latency, and gemm_q4_kernel, one unit ahead, paid it per unit (1.3-1.5 us a unit at T = 777, 16 rows: 1 TB/s
 // of weights).  Here the weights (registers) and the activations (LDS, by DMA) of the next DEPTH - 1 units are under way; a unit waits for its own requests
-// alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB of weights (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight; bf16 blocks of 96 to 192 tokens, whose
-// activations fill the LDS, have two units under way, of 208 and 256 one.
-// BM: 16 / 32 / 48 / 64 / 128 tokens, BF16 also 96 / 160 / 192 / 208 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
+// alone (a counted vmcnt, then the workgroup's barrier), so 3 x 16 KiB of weights (int4) or 3 x 64 KiB (bf16) per 8 waves are always in flight; bf16 blocks of 96 to 192 tokens and int4 ones of 160
+// and 192, whose activations fill the LDS, have two units under way, bf16 ones of 208 and 256 one.
+// BM: 16 / 32 / 48 / 64 / 128 tokens, int4 also 96 / 160 / 192 (groups not 192), BF16 96 / 160 / 192 / 208 / 256.  Sums run in the order of gemm_q4_kernel (RUNS: within a run).
 // BF16: what bounds it is the CU's memory pipeline, which returns data in the order of the requests and holds some 50 KB of them: with nothing but its requests (no
 // products) a block of 128 tokens x 256 rows took 1.67 us for the 96 KB of a unit, 0.95 when all of it lay in L2.  So the requests of a unit are spread over all of its
 // products (in the first half of them, as before, the waves stood at requests that the pipeline had no room for: N = 4096, K = 16512, 2048 tokens 248 -> 226 us with what follows,
@@ -2169,6 +2169,11 @@ extern "C" void mi355_linear_gemm_sums(int M, int N, int K, int R, bool chain, i
 }
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit) {
     plan_shares(gemm_cut_grouped((N + 15) / 16, M, R == 2, (K + 127) / 128, grouped_split(M, N, K, R == 2, group_cols)), N, R == 2, ksplit, shares, shares_per_unit);
+}
+
+extern "C" void mi355_linear_gemm_cut_grouped(int M, int N, int K, int R, int group_cols, int* waves, int* tokens, int* ksplit) {
+    const GemmCut cut = gemm_cut_grouped((N + 15) / 16, M, R == 2, (K + 127) / 128, grouped_split(M, N, K, R == 2, group_cols));
+    *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
 }
 
 // The tables of several products in one launch: a 7B prompt's layers take theirs 10 products at a time, 15 us (13 MB read, 13 written) instead of a launch in front of

@@ -54,6 +54,8 @@ extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, boo
 extern "C" void mi355_linear_gemm_sums(int M, int N, int K, int R, bool chain, int* tiles, int* ksplit, int* runs, int* longest, int* longest_of_wide);
 // the plan for scales in groups of group_cols columns (whole units)
 void mi355_linear_gemm_plan_grouped(int M, int N, int K, int R, int group_cols, int* ksplit, int* shares, int* shares_per_unit);
+// ... and the cut behind it
+extern "C" void mi355_linear_gemm_cut_grouped(int M, int N, int K, int R, int group_cols, int* waves, int* tokens, int* ksplit);
 // Tables of the (scale, zero) pairs of up to MI355_TABLE_PRODUCTS products over grouped scales, laid out ahead of them in one launch: fmt, N, K, R, group_cols and the
 // scales and zeros of products[i] count; out[i] takes mi355_linear_gemm_table_bytes.  table_room: bytes at the end of the region of K-slice sums (in front of the fuse
 // scratch) that no grouped launch's own sums reach.

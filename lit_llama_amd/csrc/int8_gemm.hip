@@ -35,7 +35,7 @@ constexpr int kOutChunk = 64;            // outlier columns staged per pass of t
 constexpr int kDepth = 4;                // units of operands in LDS and registers
 constexpr int kSoLd = kOutChunk + 8;     // row pitch of the staged outlier weights (halves): 144 B, so that 16 rows written side by side fall into 16 banks
 template <int kWaves, int BM>
-constexpr int kLdsEpi = (BM * kOutChunk + kWaves * kTPW * 16 * kSoLd) * 2;  // f16 [128 tokens][kOutChunk] + [rows][kSoLd]
+constexpr int kLdsEpi = (BM * kOutChunk + kWaves * kTPW * 16 * kSoLd) * 2;  // f16 [BM tokens][kOutChunk] + [rows][kSoLd]
 template <int kWaves, int BM>
 constexpr int kLds = kDepth * BM * 128 > kLdsEpi<kWaves, BM> ? kDepth * BM * 128 : kLdsEpi<kWaves, BM>;
 
@@ -620,8 +620,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void i8_gemm_kernel(const I8GemmPar
         if constexpr (MODE == 0) outliers();
     } else if (n_out > 0) {  // (too many for their region)
         // mixed-precision decomposition: the outlier columns in f16, ascending k, kOutChunk columns per pass through LDS
-        f16_t* xo = (f16_t*)smem;                     // [128 tokens][kOutChunk]
-        f16_t* so = xo + BM * kOutChunk;             // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
+        f16_t* xo = (f16_t*)smem;                     // [BM tokens][kOutChunk]
+        f16_t* so = xo + BM * kOutChunk;              // [kSlots x 16 rows][kOutChunk]: f16(CB[n, k] * SCB[n] / 127)
         // (the side product runs on v_mfma_f32_16x16x32_f16 — A = 16 rows x 32 outlier columns of `so`, B = 16 tokens x the same
         // columns of `xo`, result in the accumulators' own layout: lane (g, c) holds rows 4 g .. 4 g + 3 for token c.  The products of two f16
         // values are exact in f32 and the sum is f32 as before; its ORDER inside a block of 32 columns is the hardware's instead of

@@ -148,6 +148,15 @@ def test_fused_prompt_chain_of_int4_layers_in_blocks_of_whole_rows(dev, monkeypa
     _chain_against_staging(dev, monkeypatch, width, T, "gptq.int4")
 
 
+INT4_NARROW_CHAIN = [(640, 32), (640, 40), (640, 60), (2048, 32), (2048, 40), (2048, 64)]
+
+
+@pytest.mark.parametrize("width,T", INT4_NARROW_CHAIN)
+def test_fused_prompt_chain_of_int4_layers_in_blocks_of_64_rows(dev, monkeypatch, width, T):
+    """As test_fused_prompt_chain_of_bf16_layers, for c_attn and residual products in waves of one row tile: shares of 64 rows, slices of one run and of several."""
+    _chain_against_staging(dev, monkeypatch, width, T, "gptq.int4")
+
+
 BF16_CHAIN = [
     (640, 65), (640, 1094), (1024, 709), (1280, 65), (1280, 1731), (1920, 65), (1920, 646), (1920, 1633), (2048, 261), (2560, 65), (2560, 1542), (2560, 1605), (3072, 65),
     (4096, 135), (4096, 300), (4096, 400), (4096, 777), (4096, 1100), (4096, 1300), (5120, 1542), (6656, 100), (6656, 135), (6656, 1542), (6656, 1731), (6656, 1878),
@@ -164,7 +173,7 @@ def test_fused_prompt_chain_of_bf16_layers(dev, monkeypatch, width, T):
 @pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K,cols", [(1, 16, 256, 128), (16, 144, 2176, 128), (17, 4096, 1280, 256), (33, 12288, 512, 128), (64, 128, 11008, 512), (65, 4096, 4096, 128),
                                         (129, 1000, 896, 256), (257, 2064, 2560, 1024), (700, 11008, 384, 128), (1030, 4100, 512, 64), (2050, 8200, 256, 128),
-                                        (385, 15364, 1280, 128), (1300, 4100, 256, 128), (770, 12292, 640, 256), (1500, 6148, 128, 128), (450, 16388, 1664, 128)])  # blocks of 96 and 160 tokens
+                                        (385, 15364, 1280, 128), (1300, 4100, 256, 128), (770, 12292, 640, 256), (1500, 6148, 128, 128), (450, 16388, 1664, 128)])
 def test_tiled_product_of_grouped_scales_against_64_bits(dev, M, N, K, cols, x_dtype):
     """Groups of whole units: the products of a unit are sums of 128 terms of up to 143 x, the zero points a sum of their own: 1e-3 of the result as above.
     Rows whose addresses are no multiple of 16 B take the staging pass of single loads."""
@@ -179,6 +188,42 @@ def test_tiled_product_of_grouped_scales_against_64_bits(dev, M, N, K, cols, x_d
     ref = x.to(torch.bfloat16).double() @ ((q.double() - wide(z)) * wide(s)).T
     stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
     got = ops.linear_gemm(x, stream, 1, N, K, scales=s.reshape(-1), zeros=z.reshape(-1), group_cols=cols, out_dtype=torch.float32).double()
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
+GROUPED_BLOCKS = [  # M, N, K, columns of a group, pair: blocks of 96 and 160 tokens x 8 waves
+    (321, 12292, 1664, 128, 0), (577, 8196, 1664, 256, 0), (1025, 4100, 2176, 128, 0), (641, 12292, 2176, 256, 0), (450, 16388, 1664, 128, 0),
+    (67, 16388, 2176, 128, 1), (385, 6148, 2176, 256, 1), (482, 12292, 128, 256, 1), (450, 8196, 1664, 128, 1), (641, 6148, 2176, 256, 1),
+]
+
+
+@pytest.mark.parametrize("M,N,K,cols,epi", [(*shape[:4], epi) for shape in GROUPED_BLOCKS for epi in (["pair"] if shape[4] else ["store", "accum"])])
+def test_grouped_blocks_of_96_and_160_tokens_against_64_bits(dev, M, N, K, cols, epi):
+    """A few tokens and rows more than whole blocks, in each epilogue (tests/test_host_logic.py compares the list with the rule).  Bounds: as in test_tiled_product_against_64_bits."""
+    g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    mats, ng = 2 if epi == "pair" else 1, -(-K // cols)
+    qs = [torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8) for _ in range(mats)]
+    ss = [(torch.rand((N, ng), generator=g, device=dev) * 0.02 + 0.005).to(torch.bfloat16) for _ in range(mats)]
+    zs = [torch.randint(5, 11, (N, ng), generator=g, device=dev).to(torch.bfloat16) for _ in range(mats)]
+    wide = lambda t: t.double().repeat_interleave(cols, 1)[:, :K]  # noqa: E731
+    prods = [x.double() @ ((q.double() - wide(z)) * wide(s)).T for q, s, z in zip(qs, ss, zs)]
+    pk = [synth.pack_colblock(q, 4) for q in qs]
+    stream = ops.repack_q4(pk[0], pk[1] if mats == 2 else None, N, K, mats)
+    kw = dict(scales=ss[0].reshape(-1), zeros=zs[0].reshape(-1), group_cols=cols)
+    if epi == "pair":
+        kw.update(scales2=ss[1].reshape(-1), zeros2=zs[1].reshape(-1))
+        ref = torch.nn.functional.silu(prods[0]) * prods[1]
+        got = ops.linear_gemm(x, stream, 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, **kw).double()
+        assert (got - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 2e-3 * ref.square().mean().sqrt()  # one rounding to bf16
+        return
+    ref = prods[0]
+    if epi == "accum":
+        base = torch.randn((M, N), generator=g, device=dev)
+        ref = ref + base.double()
+        got = ops.linear_gemm(x, stream, 1, N, K, epi=nat.EPI_ACCUM, out=base.clone(), **kw).double()
+    else:
+        got = ops.linear_gemm(x, stream, 1, N, K, out_dtype=torch.float32, **kw).double()
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
@@ -381,19 +426,23 @@ def test_operand_slices_of_few_bf16_rows(dev, M, rows, n, K):
     assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-3 * ref.square().mean().sqrt()).all()
 
 
-@pytest.mark.parametrize("cols,heads,T", [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600),
-                                            (128, 32, 180), (256, 32, 450), (128, 32, 650)])
+GROUPED_CHAIN = [(128, 15, 33), (128, 15, 64), (128, 15, 65), (128, 15, 500), (128, 32, 40), (128, 32, 300), (128, 32, 777), (256, 32, 130), (256, 32, 600),
+                 (128, 32, 180), (256, 32, 450), (128, 32, 650), (128, 32, 1100), (256, 32, 1250), (128, 40, 1650)]
+
+
+@pytest.mark.parametrize("cols,heads,T", GROUPED_CHAIN)
 def test_fused_prompt_chain_over_grouped_scales(dev, monkeypatch, cols, heads, T):
     """Groups of whole units in the chain: one share per unit, or two (c_fc1 / c_fc2 in blocks of 64 hidden rows); slices and whole sums; tables of several layers from one
     launch and the next.  Against the same layers with staging passes, 0.02 of the logits' spread as for one scale per row."""
-    model = _wide_model(dev, LLaMAConfig(block_size=784, n_layer=5 if heads == 15 else 3, n_head=heads, n_embd=128 * heads, vocab_size=512), "gptq.int4", cols)
+    size = 784 if T < 784 else T + 4
+    model = _wide_model(dev, LLaMAConfig(block_size=size, n_layer=5 if heads == 15 else 3, n_head=heads, n_embd=128 * heads, vocab_size=512), "gptq.int4", cols)
     idx = synth.make_prompt(T, vocab=512).to(dev)
     out = []
     for fuse in ("1", "0"):
         monkeypatch.setenv("MI355_GEMM_FUSE", fuse)
         model.reset_cache()
         with torch.no_grad():
-            out.append(model(idx.view(1, -1), 784, torch.arange(T, device=dev))[0].float())
+            out.append(model(idx.view(1, -1), size, torch.arange(T, device=dev))[0].float())
     assert model.engine() is not None, model._engine_failed
     assert not torch.equal(*out)  # (the chain was on)
     assert (out[0] - out[1]).abs().max() <= 0.02 * out[1].std()

@@ -724,8 +724,51 @@ def test_gpu_tests_of_int4_blocks_run_every_block_of_whole_rows():
     assert {c for width in (2048, 4096) for T in range(65, 1000) for c in cuts(layer(width, T), True)} & blocks <= run
 
 
+def _chain_products(width):
+    hidden = find_multiple(int(8 * width / 3), 256)
+    return ("c_attn", 3 * width, width, 1), ("residual", width, width, 1), ("residual", width, hidden, 1), ("pair", hidden, width, 2)
+
+
+def test_gpu_tests_of_int4_blocks_of_64_rows_run_every_kernel():
+    """Each number of tokens, with one run of a slice and several: outside the chain (every shape there runs each epilogue) with whole rows and slices, inside it by c_attn and residual products."""
+    shapes = _gemm_shapes()
+
+    def narrow(sizes, chain):
+        for role, M, N, K in sizes:
+            tiles, slices, runs, *_ = _int4_sums(M, N, K, 1, chain)
+            if tiles == 1:
+                yield role, _gemm_cut(M, N, K, 1, chain, bf16=False)[1], runs > 1, slices > 1
+
+    run = set(narrow([("any", *shape) for shape in shapes.SHAPES], False))
+    assert {c[1:3] for c in run} == {(tokens, runs) for tokens in (16, 32, 48, 64) for runs in (False, True)}
+    assert {(c[1], c[3]) for c in run} == {(tokens, sliced) for tokens in (16, 32, 48, 64) for sliced in (False, True)}
+    chained = lambda width, T: [(role, T, N, K) for role, N, K, R in _chain_products(width) if R == 1]  # noqa: E731
+    taken = set(narrow([p for width in (640, 1024, 1920, 2048, 2560, 3072, 4096, 5120, 6656, 8192) for T in range(32, 2049) for p in chained(width, T)], True))
+    assert taken <= set(narrow([p for width, T in shapes.INT4_NARROW_CHAIN for p in chained(width, T)], True)) and len(taken) == 12
+
+
+def _grouped_cut(M, N, K, R, cols):
+    out = [C.c_int(0) for _ in range(3)]
+    nat.lib().mi355_linear_gemm_cut_grouped(M, N, K, R, cols, *[C.byref(v) for v in out])
+    return tuple(v.value for v in out)
+
+
+def test_gpu_tests_of_grouped_blocks_run_96_and_160_tokens_in_every_role():
+    shapes = _gemm_shapes()
+    blocks = {(R, 8, tokens, 1) for R in (1, 2) for tokens in (96, 160)}
+    assert {(1 + pair, *_grouped_cut(M, N, K, 1 + pair, cols)) for M, N, K, cols, pair in shapes.GROUPED_BLOCKS} == blocks
+
+    def large(width, T, cols):
+        return {(role, tokens) for role, N, K, R in _chain_products(width) for _, tokens, _ in [_grouped_cut(T, N, K, R, cols)] if tokens in (96, 160)}
+
+    taken = {c for width in (1920, 2048, 3072, 4096, 5120, 6656, 8192) for T in range(65, 2049, 7) for c in large(width, T, 128)}
+    assert taken == {(role, tokens) for role in ("c_attn", "residual", "pair") for tokens in (96, 160)}
+    assert taken <= {c for cols, heads, T in shapes.GROUPED_CHAIN for c in large(128 * heads, T, cols)}
+
+
 def test_int4_blocks_of_whole_rows_sum_no_more_than_a_launch_holds():
-    """A slice of several runs has at most 8 of them, a row 16 sums: no launch is cut into more, and blocks of more than 64 tokens, which take no runs, are left where sums end within a row."""
+    """Whole rows in blocks of 64 tokens x 8 waves have 8 runs at most, and blocks of more than 64 tokens, which take no runs, are left where sums end within a row (other cuts:
+    test_operand_sums_of_int4_slices_fit_their_place)."""
     for K in list(range(128, 4353, 128)) + [11008, 13824]:
         units = -(-K // 128)
         for N in (64, 256, 1000, 1796, 2752, 4096, 6144, 11008, 16384):

@@ -30,13 +30,19 @@ def _reference(x, cb, scb):
     (33, 72, 200, 1), (64, 4096, 4096, 63), (200, 4096, 4096, 64), (130, 1000, 1024, 65), (257, 4096, 11008, 700), (48, 4096, 22016, 300),
     (1030, 4096, 640, 129), (2050, 1040, 512, 33), (40, 11008, 4096, 4096), (512, 4096, 1024, 0),
     (33, 1001, 4096, 3), (64, 1001, 4096, 5), (64, 4098, 4096, 70), (129, 1003, 2048, 0),  # K-slices whose rows are not whole vectors of four sums
-    (100, 12292, 1152, 20), (200, 4100, 4096, 70), (257, 4096, 1030, 9), (65, 260, 12416, 2000),  # blocks of 64 tokens; rows staged element by element, twelve fours a thread
+    (100, 12292, 1152, 20), (200, 4100, 4096, 70), (257, 4096, 1030, 9), (65, 260, 12416, 2000),  # blocks of 64 tokens; rows staged element by element, up to 24 fours a thread
 ])
 @pytest.mark.parametrize("epi", ["store", "accum", "pair"])
 def test_outlier_columns(dev, M, N, K, outliers, epi):
     """Integer sums are exact; the outlier part is an f32 sum of exact products, so its f16 rounding may fall on either side: one f16 step of that part,
     and one of the sum that it moves; 2^-22 of its terms' sizes for the sum itself."""
     _check_outlier_columns(dev, M, N, K, outliers, epi)
+
+
+@pytest.mark.parametrize("K", [4096, 4100, 8192, 8196, 12288, 12292, 24576, 24580])
+def test_rows_at_the_ends_of_what_a_staging_thread_holds(dev, K):
+    """4, 8, 12 or 24 groups of four columns a thread, longer rows element by element: outliers in the last four columns, bounds as above."""
+    _check_outlier_columns(dev, 40, 132, K, 4, "store", last=True)
 
 
 @pytest.mark.parametrize("M,N,K,outliers,epi,waves,slices", [
@@ -56,10 +62,10 @@ def test_more_outlier_columns_than_their_region_holds(dev, M, N, K, outliers, ep
     _check_outlier_columns(dev, M, N, K, outliers, epi)
 
 
-def _check_outlier_columns(dev, M, N, K, outliers, epi):
+def _check_outlier_columns(dev, M, N, K, outliers, epi, last=False):
     g = torch.Generator(device=dev).manual_seed(M + N + K + outliers)
     x = torch.randn((M, K), generator=g, device=dev).clamp_(-5.9, 5.9)
-    at = torch.randperm(K, generator=g, device=dev)[:outliers]
+    at = torch.arange(K - outliers, K, device=dev) if last else torch.randperm(K, generator=g, device=dev)[:outliers]
     x[torch.randint(0, M, (outliers,), generator=g, device=dev), at] = 6.0 + 2 * torch.rand(outliers, generator=g, device=dev)
     x = x.to(torch.bfloat16)
     mats = [ops.int8_quant_rows(torch.randn((N, K), generator=g, device=dev) * K ** -0.5) for _ in range(2 if epi == "pair" else 1)]
