@@ -170,7 +170,9 @@ __global__ __launch_bounds__(256) void i8_stage_kernel(const T* x, int64_t ldx, 
 }
 
 // The same for rows in whole aligned groups of four columns, up to kHeld groups a thread: read once, four columns to a request and a store, and the mask a word of 32 columns at a time.
-// 512 rows: 11 008 columns of bf16, some 3000 with an outlier, 11.8 -> 8.9 us; 4096 of f32 with a norm 7.3 -> 7.1, 4096 of bf16 5.4 -> 5.1.
+// 512 rows: 11 008 columns of bf16, some 3000 with an outlier, 11.8 -> 8.9 us; 4096 of f32 with a norm 7.4 -> 6.6, 4096 of bf16 5.6 -> 4.4.  kHeld is the least that does: with more a thread
+// requests and stores what its row has not (2048 rows of bf16, element by element / 4 or 24 groups / the least: 512 columns 4.5 / 6.3 / 4.1, 2048 7.5 / 7.9 / 6.4, 13 824 34 / 34 / 24, 17 920
+// 45 / 38 / 34; 1024 rows of 13 824 16.3 / 19.4 / 15.1, of 17 920 19.5 / 20.8 / 19.6).
 template <typename T>
 __device__ __forceinline__ f32x4 i8_row_four(const T* p) {
     if constexpr (sizeof(T) == 4) {
@@ -924,8 +926,15 @@ int mi355_linear_int8_gemm_chained(const mi355_int8_args* a, mi355_i8_chain* cha
         using T = decltype(type);
         const size_t norm_four = a->norm_dtype == MI355_F32 ? 16 : 8;
         const bool fours = a->K % 4 == 0 && a->ldx % 4 == 0 && (uintptr_t)a->x % (4 * sizeof(T)) == 0 && (uintptr_t)a->norm_scale % norm_four == 0 && kp <= 24 * 1024;
-        auto kernel = fours ? (kp <= 4096 ? i8_stage_fours_kernel<T, 4> : kp <= 8192 ? i8_stage_fours_kernel<T, 8> : kp <= 12288 ? i8_stage_fours_kernel<T, 12> : i8_stage_fours_kernel<T, 24>)
-                            : kp <= 1024 ? i8_stage_kernel<T, 4> : kp <= 2048 ? i8_stage_kernel<T, 8> : i8_stage_kernel<T, 16>;
+        auto held = kp <= 1024    ? i8_stage_fours_kernel<T, 1>
+                    : kp <= 2048  ? i8_stage_fours_kernel<T, 2>
+                    : kp <= 4096  ? i8_stage_fours_kernel<T, 4>
+                    : kp <= 8192  ? i8_stage_fours_kernel<T, 8>
+                    : kp <= 12288 ? i8_stage_fours_kernel<T, 12>
+                    : kp <= 16384 ? i8_stage_fours_kernel<T, 16>
+                    : kp <= 20480 ? i8_stage_fours_kernel<T, 20>
+                                  : i8_stage_fours_kernel<T, 24>;
+        auto kernel = fours ? held : kp <= 1024 ? i8_stage_kernel<T, 4> : kp <= 2048 ? i8_stage_kernel<T, 8> : i8_stage_kernel<T, 16>;
         hipLaunchKernelGGL(kernel, dim3(a->M), dim3(256), 0, s, (const T*)a->x, a->ldx, a->norm_scale, a->norm_dtype, a->eps, a->threshold, a->K, kp, xh, sca, mask);
     };
     if (a->x_dtype == MI355_F32) stage(float{});

@@ -39,9 +39,9 @@ def test_outlier_columns(dev, M, N, K, outliers, epi):
     _check_outlier_columns(dev, M, N, K, outliers, epi)
 
 
-@pytest.mark.parametrize("K", [4096, 4100, 8192, 8196, 12288, 12292, 24576, 24580])
+@pytest.mark.parametrize("K", [1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 12288, 12292, 16384, 16388, 20480, 20484, 24576, 24580])
 def test_rows_at_the_ends_of_what_a_staging_thread_holds(dev, K):
-    """4, 8, 12 or 24 groups of four columns a thread, longer rows element by element: outliers in the last four columns, bounds as above."""
+    """1, 2, 4, 8, 12, 16, 20 or 24 groups of four columns a thread, longer rows element by element: outliers in the last four columns, bounds as above."""
     _check_outlier_columns(dev, 40, 132, K, 4, "store", last=True)
 
 
