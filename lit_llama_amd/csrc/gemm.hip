@@ -1925,27 +1925,36 @@ GemmCut bf16_cut_many(int M, int N, int K, bool pair) {
 // those whose choice is best over 1078 launches (41 products of 512 to 32000 rows, 65 to 2048 tokens; those below 20 MB with their weights in the 256-MB cache and without, the others
 // without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.7 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
 // a launch as the least that slices cost, 1.6 % and 5.4 %: short rows were cut (512 tokens, N = K = 2048 16.1 us in two slices, 12.7 whole; 96 of the N = 2816 pair, K = 1024 11.6, 8.2).
-// Blocks of 160 and 208 tokens came later, their constants fitted to 270 launches without slices (15 products, 129 to 2048 tokens; 0.05 % behind the fastest of six blocks): the launches that they
-// take are 8 % faster on average (777 tokens, N = 15360, K = 5120 in 256 / 208 tokens 123 / 107 us; N = 12288, K = 4096 in 192 / 160 75 / 69, the N = 11008 pair 138 / 128; 2048, N = 12416 in 256 / 208 199 / 179).
+// Blocks of 160 and 208 tokens came later, their constants fitted to 270 launches without slices (15 products, 129 to 2048 tokens): whole rows only, and where the estimate takes them for 4 %
+// faster than the others.  288 of 355 launches (40 products) that they would take by the lower estimate are 0.935 times as long then, two of them more than 2 % longer (777 tokens, N = 15360, K = 5120
+// in 256 / 208 tokens 123 / 107 us; N = 12288, K = 4096 in 192 / 160 75 / 69, the N = 11008 pair 138 / 128; 2048, N = 12416 in 256 / 208 199 / 179).  The 32 within 4 % are 1.3 % faster in the other blocks, up to
+// 10 % (2048 tokens, N = 32000 in 208 / 256: K = 2048 282 / 258 us, 4096 474 / 450; 1772 of the N = 2816 pair, K = 1024 in 208 / 192 26.8 / 25.0), the 35 in slices 0.4 %, up to 9 % (129 tokens, N = 4096,
+// K = 16512 11 slices of 160 tokens 46.3 us, 4 of 96 42.4; 146, N = 8192, K = 22016 100.3 / 96.0): profiles/product_cuts_bf16.txt.
 GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
     struct Kind {
         int waves, bm;
         float start, unit, crowd;
     };
-    static constexpr Kind kinds[] = {{4, 64, 2.744f, 0.518f, 0.181f},  {4, 96, 4.059f, 0.484f, 0.333f}, {4, kBM, 2.751f, 0.78f, 0.272f},
-                                     {8, 64, 6.209f, 0.684f, 0.474f},  {8, kBM, 8.323f, 0.926f, 0.424f}, {8, 160, 8.129f, 1.217f, 0.283f},
-                                     {8, 192, 11.38f, 1.231f, 0.501f}, {8, 208, 8.519f, 1.703f, 0.271f}, {8, 256, 9.51f, 1.344f, 1.146f}};
+    static constexpr Kind kinds[] = {{4, 64, 2.744f, 0.518f, 0.181f},  {4, 96, 4.059f, 0.484f, 0.333f}, {4, kBM, 2.751f, 0.78f, 0.272f}, {8, 64, 6.209f, 0.684f, 0.474f},
+                                     {8, kBM, 8.323f, 0.926f, 0.424f}, {8, 192, 11.38f, 1.231f, 0.501f}, {8, 256, 9.51f, 1.344f, 1.146f}};
+    static constexpr Kind whole[] = {{8, 160, 8.129f, 1.217f, 0.283f}, {8, 208, 8.519f, 1.703f, 0.271f}};
     const int units = (K + 127) / 128;
+    auto estimate = [&](const Kind& k, int ks) {
+        const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks;
+        auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (k.unit + k.crowd * (float)of / 256.f); };
+        return k.start + (float)(blocks / 256) * round(256) + round(blocks % 256);
+    };
     GemmCut cut = {4, 64, true, 1};
     float best = 0.f;
     for (const Kind& k : kinds)
         for (int ks = 1; ks <= kMaxSplit && (ks == 1 || (units >= 4 * ks && gemm_part_bytes(M, N, pair, ks) <= kSplitBudget * 3 / 4)); ++ks) {
-            const int blocks = gemm_blocks(M, N, pair, k.waves, k.bm) * ks;
-            auto round = [&](int of) { return of == 0 ? 0.f : (float)((units + ks - 1) / ks) * (k.unit + k.crowd * (float)of / 256.f); };
-            float us = k.start + (float)(blocks / 256) * round(256) + round(blocks % 256);
+            float us = estimate(k, ks);
             if (ks > 1) us += fmaxf(0.976f + (float)gemm_part_bytes(M, N, pair, ks) / 2.486e6f, 2.17f);
             if (best == 0.f || us < best) best = us, cut = {k.waves, k.bm, true, ks};
         }
+    best *= 0.96f;
+    for (const Kind& k : whole)
+        if (const float us = estimate(k, 1); us < best) best = us, cut = {k.waves, k.bm, true, 1};
     return cut;
 }
 GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {

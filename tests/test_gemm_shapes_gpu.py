@@ -99,6 +99,7 @@ BF16_BLOCKS = [
     (600, 12288, 1152, 0), (600, 11012, 1664, 1), (70, 4100, 2176, 0), (129, 4100, 4224, 0), (66, 4100, 3200, 0), (300, 4096, 11008, 0), (135, 11012, 8448, 0),
     (70, 2816, 1664, 1), (70, 4100, 2176, 1), (66, 2052, 3200, 1), (129, 11012, 4224, 1),
     (482, 16400, 1664, 0), (674, 16400, 640, 0), (386, 8200, 640, 1), (962, 6160, 384, 1), (1930, 8280, 384, 0), (1165, 3340, 8448, 0),
+    (770, 6148, 640, 1), (390, 13124, 640, 1), (785, 13124, 1152, 0),
 ]
 
 
