@@ -11,7 +11,7 @@
 //   2. i8_quant_kernel   — CA = rint(xh * 127 / absmax) with the masked columns zeroed, int8; the ascending list of outlier columns; and those columns by
 //                        themselves, f16: xo (rows) and so = f16(CB * SCB / 127) (weights; workgroups behind the rows');
 //   3. i8_gemm_kernel    — the int8 weight stream of int8.hip ([tile][unit][r][piece e][lane][16 x int8], one piece = one
-//                        MFMA A operand) against CA through LDS (128 tokens x 128 k, XOR-swizzled), two row tiles per
+//                        MFMA A operand) against CA through LDS (128 or 64 tokens x 128 k, XOR-swizzled), two row tiles per
 //                        wave, 8 or 4 waves; then so x xo in the same loop on the f16 MFMA (of a launch cut along K: a slice of its own); epilogue with the arithmetic
 //                        of int8.hip, rounding for rounding:
 //                            d = f16((acc * 6.200012e-05 * absmax[m]) * SCB[n]);   o = sum over outlier columns k (ascending) of
@@ -810,7 +810,8 @@ int launch_i8_mode(const I8GemmParams& q, hipStream_t s) {
 // at the 90th percentile; with the outliers' workgroups left out 1.6 % and 5 %, and N = 5120, K = 13824, 256 tokens 79 us (now 66).  Blocks of 8 waves throughout and
 // slices for launches of less than 96 of them: 1.23 times as long on average, none more than 2.5 % shorter.
 // Blocks of 64 tokens x 128 rows (whole rows only) where they bring work to idle CUs: 512 tokens, N = 4096, K = 4096 35.8 -> 31.4 us, K = 11008 73.2 -> 59.2, with 2750 outlier columns 154 -> 136
-// (128 blocks -> 256; staging and quantisation with it); of 493 launches (13 products, 33 to 2048 tokens, 0, 2 and 25 % of the columns) the rule takes them in 167, 0.90 times as long, 2.6 % longer at worst.
+// (128 blocks -> 256; staging and quantisation with it); of 493 launches (13 products, 33 to 2048 tokens, 0, 2 and 25 % of the columns) the rule takes them in 167, 0.90 times as long, 2.6 % longer at worst
+// (profiles/product_cuts_int8.txt has 585 of that kind).
 struct I8Cut {
     int waves, ksplit, bm;
 };

@@ -726,6 +726,14 @@ def test_gpu_tests_of_bf16_blocks_run_every_block():
     assert {("pair" if role == "pair" else "single", *c) for role, *c in taken} <= run
 
 
+@pytest.mark.parametrize("M,N,K,R", [(860, 32000, 2048, 1), (1195, 32000, 2048, 1), (1307, 32000, 2048, 1), (1518, 32000, 2048, 1), (1988, 5632, 2048, 2)])
+def test_short_int4_rows_keep_two_workgroups_per_cu(M, N, K, R):
+    """Each of these took 1.01 to 1.05 times as long in blocks of 160 or 192 tokens, one to a CU."""
+    for chain in (False, True):
+        assert _gemm_cut(M, N, K, R, chain, bf16=False) == (8, 128, 1)
+    assert _gemm_cut(1500, 5632, 2048, 2, False, bf16=False) == (8, 160, 1) and _gemm_cut(1500, 12288, 4096, 1, False, bf16=False)[1] != 128
+
+
 def test_gpu_tests_of_int4_blocks_run_every_block_of_whole_rows():
     """Blocks of 8 waves, each number of tokens, of single products and pairs, outside the chain; inside it those that layers of 2048 and 4096 columns take."""
     shapes = _gemm_shapes()
