@@ -1800,7 +1800,8 @@ int gemm_longest(int M, int N, int K, bool pair, const GemmCut& cut) {
 // 0.45 us a unit, one 0.31 to 0.34, with all operands in the L2 caches as well, and no barrier 0.42), so half the rows per wave on idle CUs are worth more than K-slices, whose sums are a launch more:
 // 37 tokens, N = 12288, K = 4096 20.6 us in two slices of 128-row blocks, 18.1 whole in 64-row blocks; N = K = 4096 16.2 in 8 slices, 15.4 in 4; 128 tokens, N = 6144, K = 2048 19.6 / 14.5.  The
 // estimate: per unit of a slice `unit` us and `crowd` more when every CU has a block, `slices` and `bytes` for partial sums, fitted to 1422 launches (18 products of 1024 to 32000 rows, 32 to 300
-// tokens, weights in no cache; 7 % off on average; those of 18 products again in profiles/product_cuts_int4.txt).  Where it takes these blocks or not: 0.96 / 0.95 / 0.94 / 0.93 times the time of 128-row blocks (32, to 48, to 64, more tokens), 3 % slower at worst.
+// tokens, weights in no cache; 7 % off on average; those of 18 products again in profiles/product_cuts_int4.txt).  Where it takes these blocks or not: 0.96 / 0.95 / 0.94 / 0.93 times the time of 128-row blocks (32, to 48, to 64, more tokens), 3 % slower at worst but for one (72 tokens,
+// N = 6656, K = 17920 in two slices 5 %).
 // In the chain, whose blocks add up shares first and whose sums of slices write the next ones, whole rows only (37 tokens, 7B: c_attn 12.8 + 4.2 us for the sum of its slices -> 15.9; attn.c_proj in 4
 // narrow slices 8.4 + 4.2, in 8 wide ones 7.8 + 4.4).  No accumulator sums more than in the cut that they replace: N = 1024, K = 3584 in 4 slices of 7 units for 7 of 4 rounds beside an activation of
 // 2^17 by 2.1 last bits rms for 1.7.
@@ -1831,8 +1832,8 @@ void q4_narrow(int M, int N, int K, bool pair, bool chain, GemmCut* cut) {
 // is the more of a launch the shorter its rows are (K = 2048, two per CU / one: N = 32000, 1195 tokens 139 us / 146, 1518 167 / 172).  Blocks of 64 and 128 tokens
 // leave the rounds of the chip two sizes to fit: 777 tokens, N = 12288, K = 4096, 624 blocks of 64 83.6 us, 240 of 160 67.2; the N = 11008 pair 131 / 112; 450, N = 19968, K = 6656 125 / 98 (160);
 // 130, the N = 11008 pair, 258 blocks of 64 51.2, 172 of 96 42.6; 1500, N = 4096, K = 11008 136 / 114 (96); 384 of the N = 13824 pair, K = 5120 94.7 / 82.7 (192).  The estimate is a start and the
-// rounds one behind the other, as in bf16_cut_long(), fitted to 3000 launches (profiles/product_cuts_int4.txt: 22 products of 1024 to 24576 rows, 72 to 2048 tokens; 3 to 5 % off on average): of 506 launches 171 take
-// other blocks than before these and q4_narrow(), 0.88 times as long, none more than 1.1 % longer, and all together 0.8 % behind the best of each; of 544 between and beside them (N = 32000 too) one is more than 2 %.  Whole prompts of 72 to 2048 tokens, widths 2048 to 6656, one scale per row or groups
+// rounds one behind the other, as in bf16_cut_long(), fitted to 3000 launches (profiles/product_cuts_int4.txt: 22 products of 1024 to 24576 rows, 72 to 2048 tokens; 3 to 5 % off on average): of 506 launches 169 take
+// other blocks than before these and q4_narrow(), 0.87 times as long, none more than 0.8 % longer, and all together 0.6 % behind the best of each; of 533 between and beside them (N = 32000 too) three are 2 % longer.  Whole prompts of 72 to 2048 tokens, widths 2048 to 6656, one scale per row or groups
 // of 128 columns: 0.965 times as long on average, 0.89 at best, the rest within the noise.
 void q4_whole(int M, int N, int K, bool pair, GemmCut* cut) {
     struct Kind {
@@ -1927,7 +1928,7 @@ GemmCut bf16_cut_many(int M, int N, int K, bool pair) {
 // without: profiles/product_cuts_bf16.txt): 0.8 % behind the fastest of 25 000 cuts on average, 2.7 % at the 90th percentile.  Fitted to rows of 2048 columns and more, without
 // a launch as the least that slices cost, 1.6 % and 5.4 %: short rows were cut (512 tokens, N = K = 2048 16.1 us in two slices, 12.7 whole; 96 of the N = 2816 pair, K = 1024 11.6, 8.2).
 // Blocks of 160 and 208 tokens came later, their constants fitted to 270 launches without slices (15 products, 129 to 2048 tokens): whole rows only, and where the estimate takes them for 4 %
-// faster than the others.  288 of 355 launches (40 products) that they would take by the lower estimate are 0.935 times as long then, two to six of them, run by run, more than 2 % longer, 5 % at most (777 tokens, N = 15360, K = 5120
+// faster than the others.  288 of 355 launches (40 products) that they would take by the lower estimate are 0.94 times as long then, two to six of them, run by run, more than 2 % longer, 5 % at most (777 tokens, N = 15360, K = 5120
 // in 256 / 208 tokens 123 / 107 us; N = 12288, K = 4096 in 192 / 160 75 / 69, the N = 11008 pair 138 / 128; 2048, N = 12416 in 256 / 208 199 / 179).  The 32 within 4 % are 1.3 % faster in the other blocks, up to
 // 10 % (2048 tokens, N = 32000 in 208 / 256: K = 2048 282 / 258 us, 4096 474 / 450; 1772 of the N = 2816 pair, K = 1024 in 208 / 192 26.8 / 25.0), the 35 in slices 0.4 %, up to 9 % (129 tokens, N = 4096,
 // K = 16512 11 slices of 160 tokens 46.3 us, 4 of 96 42.4; 146, N = 8192, K = 22016 100.3 / 96.0): profiles/product_cuts_bf16.txt.
