@@ -1104,7 +1104,10 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // units / 4 of their own on the f32 MFMA in front of the loop.
 // RUNS (Q4): a slice of several runs (gemm_runs()).  The second set of sums is 32 registers, with which two workgroups of 8 waves no longer share a CU: kernels of
 // their own.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW>
+// ONCE: one token block (BM tokens at most), so nothing reads a piece of the weights again: they are requested non-temporal and push no activations out of the L2 caches.
+// BF16, 16 products of 2048 to 32000 rows, weights in no cache: 16 tokens 0.89 times as long (0.86 to 0.94; N = 4096, K = 16512 30.9 -> 26.8 us, N = 32000, K = 4096 52.0 -> 46.0), 24 tokens
+// 0.91, 40 0.93, 64 0.95 (two of 16 up to 1.01).  Int4 of one scale per row, which its own work bounds, the same either way; groups of 128 columns, 16 and 24 tokens, 0.95.
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW, bool ONCE = BM <= 48>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
     static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1), "grouped scales are a Q4 feature");
     static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
@@ -1144,7 +1147,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
     for (int t = 0; t < TPW; ++t)
         tile[t] = PAIR ? nb * (kSlots / 2) + (TPW / 2) * wave + (t >> 1) : nb * kSlots + TPW * wave + t;
     // this block's share of its row block's weights (see above): thread i's line of every round of DEPTH units, at touch_off from the round's first unit
-    constexpr bool kTouch = FMT == MI355_W_BF16 && shares_weights(kWaves, BM);
+    constexpr bool kTouch = FMT == MI355_W_BF16 && shares_weights(kWaves, BM) && !ONCE;
     constexpr int kTouchAhead = 2 * DEPTH - 1, kStreams = PAIR ? kSlots / 2 : kSlots, kRun = DEPTH * (PAIR ? 64 : 32);  // kRun: lines of DEPTH units of a tile
     constexpr unsigned kNone = 0xFFFFFFF0u;
     [[maybe_unused]] unsigned touch_off = kNone;
@@ -1194,7 +1197,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmPar
             const bool ok = tile[t] < p.n_tiles && in;
             const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, ok ? (int)p.w_bytes : 0, 0x00020000);
             const unsigned off = (unsigned)((tile[t] * p.units + u) * (PAIR ? 2 : 1) + (PAIR ? t & 1 : 0)) * (1024u * kWP) + d * 1024u;
-            wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane_off, ok ? off : 0u, 0));
+            wr[slot][t][d] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, lane_off, ok ? off : 0u, ONCE ? 2 : 0));
         }
     };
 
@@ -1676,20 +1679,23 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     }
     return 0;
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false, bool ONCE = BM <= 48>
 int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM <= 64 && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, true>(p, s);
     }
+    if constexpr (FMT == MI355_W_BF16 && BM == 64 && !ONCE) {
+        if (p.M <= BM) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, RUNS, true>(p, s);
+    }
     constexpr int kDepth = BM > 192 ? 2 : BM > kBM || (BM >= 96 && FMT == MI355_W_BF16) ? 3 : 4;
     constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * TPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
-    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW>,
+    static hipError_t attr_err = hipFuncSetAttribute((const void*)gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW, ONCE>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr_err != hipSuccess) {
         mi355_set_error("hipFuncSetAttribute(gemm) failed: %s", hipGetErrorString(attr_err));
         return (int)attr_err;
     }
-    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE, TPW>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW>, kLds, p, s);
+    return launch_blocks<EPI, PAIR, kWaves, BM, FUSE, TPW>(gemm_deep_kernel<EPI, PAIR, FMT, kWaves, BM, FUSE, kDepth, GRP, RUNS, TPW, ONCE>, kLds, p, s);
 }
 template <int EPI, bool PAIR, int kWaves, int BM, int GRP = 0, bool FUSE = false>
 int launch_gemm_w(const GemmParams& p, hipStream_t s) {
@@ -2025,11 +2031,11 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
     const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE, p.slice_blocks != 0);
     if constexpr (FMT == MI355_W_BF16 && !FUSE) {
         if (sh.waves == 3) {
-            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 3, 64, FUSE>(p, s);
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 3, 64, FUSE, 0, kTPW, false, true>(p, s);
             return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
         }
         if (sh.waves == 2) {
-            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE, 0, kTPW, false, true>(p, s);
             return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
         }
     }

@@ -406,6 +406,18 @@ def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
+@pytest.mark.parametrize("M", [49, 64, 65])
+@pytest.mark.parametrize("N,K", [(128, 640), (33024, 384), (70000, 128)])
+def test_blocks_of_64_tokens_read_once_or_by_several(dev, N, K, M):
+    """BF16 blocks of 64 tokens by themselves (weights requested non-temporal) and side by side, of 2 to 8 waves: f32 sums of exact products (see test_tiled_product_against_64_bits)."""
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    got = ops.linear_gemm(x, ops.repack_bf16(w, None, 1), 1, N, K, out_dtype=torch.float32, fmt=nat.W_BF16).double()
+    ref = x.double() @ w.double().T
+    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+
+
 OPERAND_SLICES = [(9, 256, 9, 4096), (16, 512, 5, 4096), (24, 256, 22, 4096), (32, 256, 65, 128), (32, 3072, 2, 4096), (40, 256, 65, 256), (40, 256, 18, 4096), (64, 256, 66, 256), (64, 512, 11, 4096)]
 
 
