@@ -4,8 +4,9 @@
 // earlier layer.  A slot's cache is, per key head, `kept` rows for the first positions and a ring for the others.  A layer lends
 // its keys and values to later ones, which read its cache (and, in a prompt step, its prepared rows).
 //
-//   window_rows_kernel    one workgroup per (row, key head, split of the keys): decode steps of any size (q and the row's own k are
-//                         normalised and rotated here, the cache row is written here: one launch per layer), f32 models, odd head sizes
+//   window_keys_kernel    decode steps of bf16 models with heads of 64, 128 or 256: one workgroup per (row, up to four heads of a key head, split of the keys) on the matrix
+//                         cores (q and the row's own k are normalised and rotated here, the cache row is written here: one launch per layer)
+//   window_rows_kernel    one workgroup per (row, key head, split of the keys): other decode steps likewise, f32 models, odd head sizes
 //   window_tiles_kernel   128 queries of one head per workgroup on the matrix cores (bf16 prompt steps)
 //   prepare_keys_kernel   prompt steps: k rows normalised and rotated, v rows normalised in front of either kernel, in place or (a lender's)
 //                         to kv_rows
@@ -90,6 +91,86 @@ struct WinParams {
     int64_t ld_rows;
 };
 
+// What a row's attention starts from: the queries q [nh][dim] of heads h0 .. over the root mean square, rotated and scaled; with `owner` (a decode step) also the row's
+// own key kn [dim] and, where it is not the projection's, its value vn [vdim, padded to 8], as the cache takes them, and with `write` their cache rows kw, vw.
+// 32 lanes per head, a pair of values each; the row's own key is number nh
+template <typename T, int THREADS>
+__device__ __forceinline__ void make_queries(const mi355_window_attn_args& a, const T* prow, int row, int pos, int kvh, int h0, int nh, bool owner, bool made_v, bool write,
+                                             T* kw, T* vw, float* q, float* kn, float* vn) {
+    const int tid = threadIdx.x, dim = a.dim, vdim = a.vdim;
+    const int pairs = (dim + 1) / 2;  // (an odd size: the last pair is one value)
+    for (int h = tid >> 5; h < nh + (owner ? 1 : 0); h += THREADS / 32) {
+        const int lane = tid & 31;
+        const bool key = h == nh;
+        const T* src = key ? prow + a.off_k + (int64_t)kvh * dim : prow + a.off_q + (int64_t)(h0 + h) * dim;
+        auto at = [&](int d) { return d < dim ? to_f32<T>(src[d]) : 0.f; };
+        constexpr int kHeld = 2;  // pairs of a lane that are loaded once
+        float v[kHeld][2], ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) v[i][e] = at(2 * (lane + 32 * i) + e);
+        float f = key ? 1.f : a.head_scale != nullptr ? a.scale * a.head_scale[h0 + h] : a.scale;
+        if (a.unit_qk) {
+#pragma unroll
+            for (int i = 0; i < kHeld; ++i) ss += v[i][0] * v[i][0] + v[i][1] * v[i][1];
+            for (int d = 64 * kHeld + lane; d < dim; d += 32) ss += at(d) * at(d);
+            f /= sqrtf(group_sum(ss, 32) / (float)dim + a.unit_eps);
+        }
+        const float* by = key ? a.k_norm : a.q_norm;
+        auto put = [&](int pi, float u, float w) {
+            if (by != nullptr) {
+                u *= by[2 * pi];
+                if (2 * pi + 1 < dim) w *= by[2 * pi + 1];
+            }
+            if (const int ri = pi - a.rot_at / 2; ri >= 0 && 2 * ri < a.rot_dims) {
+                float c, s;
+                pair_cos_sin(pos, a.inv_freq[ri], c, s);
+                const float r = u * c - w * s;
+                w = w * c + u * s;
+                u = r;
+            }
+            u *= f, w *= f;
+            if (key) {
+                const T ru = from_f32<T>(u), rw = from_f32<T>(w);
+                kn[2 * pi] = to_f32<T>(ru);
+                if (write) kw[2 * pi] = ru;
+                if (2 * pi + 1 < dim) {
+                    kn[2 * pi + 1] = to_f32<T>(rw);
+                    if (write) kw[2 * pi + 1] = rw;
+                }
+            } else {
+                q[h * dim + 2 * pi] = u;
+                if (2 * pi + 1 < dim) q[h * dim + 2 * pi + 1] = w;
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i)
+            if (lane + 32 * i < pairs) put(lane + 32 * i, v[i][0], v[i][1]);
+        for (int pi = lane + 32 * kHeld; pi < pairs; pi += 32) put(pi, at(2 * pi), at(2 * pi + 1));
+    }
+    if (owner && write) {
+        const T* vs = prow + a.off_v + (int64_t)kvh * vdim;
+        if (!made_v)
+            for (int d = tid; d < vdim; d += THREADS) vw[d] = vs[d];
+    }
+    if (owner && made_v && tid < 64) {
+        const T* vs = prow + a.off_v + (int64_t)kvh * vdim;
+        float r = 1.f;
+        auto value = [&](int d) { return mixed_value<T>(a, row, kvh, d, to_f32<T>(vs[d])); };
+        if (a.unit_v) {
+            float ss = 0.f;
+            for (int d = tid; d < vdim; d += 64) ss += value(d) * value(d);
+            r = 1.0f / sqrtf(group_sum(ss, 64) / (float)vdim + a.unit_eps);
+        }
+        for (int d = tid; d < (vdim + 7) / 8 * 8; d += 64) {
+            const T o = from_f32<T>(d < vdim ? value(d) * r : 0.f);
+            vn[d] = to_f32<T>(o);
+            if (write && d < vdim) vw[d] = o;
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------ row kernel
 // HT query heads of one key head per workgroup, VE consecutive elements per load (8: 16-B loads of bf16; 1: any head size).  FRESH: a decode
 // step, whose keys all lie in the cache but a row's own
@@ -155,81 +236,7 @@ __global__ __launch_bounds__(kRowThreads, HT <= 4 ? 4 : 2) void window_rows_kern
     const bool owner = FRESH && p.own && k_begin < n_keys && k_end == n_keys;  // this split holds the row's own key
     const bool made_v = a.unit_v || a.v_first != nullptr;                      // ... whose value is not the projection's
 
-    // 32 lanes per head, a pair of values each: over the root mean square, rotated, scaled; a decode step's own key likewise (number nh)
-    T* kw = kcache + row_of(n_keys - 1) * (unsigned)dim;
-    const int pairs = (dim + 1) / 2;  // (an odd size: the last pair is one value)
-    for (int h = tid >> 5; h < nh + (owner ? 1 : 0); h += kRowThreads / 32) {
-        const int lane = tid & 31;
-        const bool key = h == nh;
-        const T* src = key ? prow + a.off_k + (int64_t)kvh * dim : prow + a.off_q + (int64_t)(h0 + h) * dim;
-        auto at = [&](int d) { return d < dim ? to_f32<T>(src[d]) : 0.f; };
-        constexpr int kHeld = 2;  // pairs of a lane that are loaded once
-        float v[kHeld][2], ss = 0.f;
-#pragma unroll
-        for (int i = 0; i < kHeld; ++i)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) v[i][e] = at(2 * (lane + 32 * i) + e);
-        float f = key ? 1.f : a.head_scale != nullptr ? a.scale * a.head_scale[h0 + h] : a.scale;
-        if (a.unit_qk) {
-#pragma unroll
-            for (int i = 0; i < kHeld; ++i) ss += v[i][0] * v[i][0] + v[i][1] * v[i][1];
-            for (int d = 64 * kHeld + lane; d < dim; d += 32) ss += at(d) * at(d);
-            f /= sqrtf(group_sum(ss, 32) / (float)dim + a.unit_eps);
-        }
-        const float* by = key ? a.k_norm : a.q_norm;
-        auto put = [&](int pi, float u, float w) {
-            if (by != nullptr) {
-                u *= by[2 * pi];
-                if (2 * pi + 1 < dim) w *= by[2 * pi + 1];
-            }
-            if (const int ri = pi - a.rot_at / 2; ri >= 0 && 2 * ri < a.rot_dims) {
-                float c, s;
-                pair_cos_sin(pos, a.inv_freq[ri], c, s);
-                const float r = u * c - w * s;
-                w = w * c + u * s;
-                u = r;
-            }
-            u *= f, w *= f;
-            if (key) {
-                const T ru = from_f32<T>(u), rw = from_f32<T>(w);
-                kn[2 * pi] = to_f32<T>(ru);
-                if (ht == 0) kw[2 * pi] = ru;
-                if (2 * pi + 1 < dim) {
-                    kn[2 * pi + 1] = to_f32<T>(rw);
-                    if (ht == 0) kw[2 * pi + 1] = rw;
-                }
-            } else {
-                q[h * dim + 2 * pi] = u;
-                if (2 * pi + 1 < dim) q[h * dim + 2 * pi + 1] = w;
-            }
-        };
-#pragma unroll
-        for (int i = 0; i < kHeld; ++i)
-            if (lane + 32 * i < pairs) put(lane + 32 * i, v[i][0], v[i][1]);
-        for (int pi = lane + 32 * kHeld; pi < pairs; pi += 32) put(pi, at(2 * pi), at(2 * pi + 1));
-    }
-    if (owner && ht == 0) {
-        T* vw = vcache + row_of(n_keys - 1) * (unsigned)vdim;
-        const T* vs = prow + a.off_v + (int64_t)kvh * vdim;
-        if (!made_v)
-            for (int d = tid; d < vdim; d += kRowThreads) vw[d] = vs[d];
-    }
-    if (owner && made_v && tid < 64) {
-        T* vw = vcache + row_of(n_keys - 1) * (unsigned)vdim;
-        const T* vs = prow + a.off_v + (int64_t)kvh * vdim;
-        float r = 1.f;
-        auto value = [&](int d) { return mixed_value<T>(a, row, kvh, d, to_f32<T>(vs[d])); };
-        if (a.unit_v) {
-            float ss = 0.f;
-            for (int d = tid; d < vdim; d += 64) ss += value(d) * value(d);
-            r = 1.0f / sqrtf(group_sum(ss, 64) / (float)vdim + a.unit_eps);
-        }
-        for (int d = tid; d < (vdim + 7) / 8 * 8; d += 64) {
-            const T o = from_f32<T>(d < vdim ? value(d) * r : 0.f);
-            vn[d] = to_f32<T>(o);
-            if (ht == 0 && d < vdim) vw[d] = o;
-        }
-    }
+    make_queries<T, kRowThreads>(a, prow, row, pos, kvh, h0, nh, owner, made_v, ht == 0, kcache + row_of(n_keys - 1) * (unsigned)dim, vcache + row_of(n_keys - 1) * (unsigned)vdim, q, kn, vn);
     if (tid < HT) {  // the sink is a key without a value: a score of its own in the first split
         const bool sink = a.sink != nullptr && split == 0 && tid < nh;
         stat[tid] = sink ? a.sink[h0 + tid] : -INFINITY;
@@ -384,6 +391,224 @@ __global__ __launch_bounds__(kRowThreads, HT <= 4 ? 4 : 2) void window_rows_kern
 #pragma unroll 4
         for (int k = 0; k < n_kl; ++k) o += red[k * HT * cols + i];
         if (d < vdim) put(h, d, o);
+    }
+}
+
+// ------------------------------------------------------------------------------------ decode steps on the matrix cores
+// A decode step's row over bf16 heads of 32 KS dimensions and values of up to 128 VB: one workgroup per (row, up to four heads of a key head, split of the keys).  What
+// bounds it are the cache rows' way from HBM and a chain of round trips, so every wave takes runs of 32 keys by itself, all keys and values of a run requested at once and
+// multiplied from the registers that they land in, without a barrier until the waves join.  (window_rows_kernel multiplies in f32 on the VALU, a pass of 64 keys, a softmax and
+// a pass of values one behind the other: 16 sequences of 96 to 1536 keys, 32 / 8 heads of 128, with the join 40 -> 23.5 us; 53 MB of cache are 9.)
+//   scores   D[key][column] = keys x queries: a query in f32 is three bf16 (limbs_of()), each a column: 4 heads x 3 of the 16 columns.  Products of bf16 are exact
+//            in f32, so the sum is that of f32 products
+//   weights  exp(score - maximum) in f32 per lane (its column's head, eight keys), split the same way
+//   values   D[dim][column] = values^T x weights.  The product's key number 8 g + j of lane group g is the key whose weight the group holds: key 4 g + j of the run
+//            (j < 4) or 16 + 4 g + j - 4; its row number i of product j is dimension 8 i + j, so a lane's loads are 16 B of a row and eight keys' values are turned by v_perm
+// Registers: three workgroups to a CU (two of 8 waves, the next run requested ahead: 26 us).  Error of the f32 sums against 64 bits 2.3e-7 to 6e-7 of a row (window_rows_kernel 1.5e-7 to
+// 4e-7), of the rows that leave, rounded to bf16, 1.7e-3 from both, equal to 1e-8.
+constexpr int kKeyHeads = 4, kRun = 32;
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr int kKeyWaves = 4, kKeyThreads = 64 * kKeyWaves;
+constexpr int key_occupancy(int ks, int vb) { return vb == 1 && ks <= 4 ? 3 : 2; }  // waves per SIMD
+
+// Limb 0, 1 or 2 of eight f32 as bf16: the upper 16 bits, of what is left the upper 16, and the rest (3: any)
+__device__ __forceinline__ u32x4 limbs_of(const float (&x)[8], int limb) {
+    uint32_t t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float r = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u), s = r - __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+        t[i] = __float_as_uint(limb == 0 ? x[i] : limb == 1 ? r : s);
+    }
+    return u32x4{__builtin_amdgcn_perm(t[1], t[0], 0x07060302u), __builtin_amdgcn_perm(t[3], t[2], 0x07060302u), __builtin_amdgcn_perm(t[5], t[4], 0x07060302u),
+                 __builtin_amdgcn_perm(t[7], t[6], 0x07060302u)};
+}
+// Sum over the limbs: columns c, c + 4, c + 8 and c + 12 of a row of 16 lanes.  All four get the same bits, (c + c8) + (c4 + c12) or the other way round: they split what follows from it,
+// and a weight whose limbs came from two roundings would lose all but its first eight bits now and then
+__device__ __forceinline__ float sum_limbs(float v) {
+    v = MI355_DPP_ADD(v, 0x128);     // row_ror:8
+    return MI355_DPP_ADD(v, 0x124);  // row_ror:4
+}
+
+template <int KS, int VB>
+__global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_keys_kernel(const WinParams p) {
+    constexpr int kDim = 32 * KS;
+    const mi355_window_attn_args& a = p.a;
+    __shared__ __attribute__((aligned(16))) float q[kKeyHeads * kDim], kn[kDim], vn[VB * 128], stat[2][kKeyWaves][kKeyHeads];
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    u32x4* qs = (u32x4*)smem;             // [KS][lane] the queries' limbs, then the row's own key and value
+    u32x4 *ks = qs + KS * 64, *vs = ks + kDim / 8;
+    float* red = (float*)(vs + VB * 16);  // [wave][head][128 VB]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15, head = c & 3, limb = c >> 2;
+    const int row = blockIdx.z, split = blockIdx.x;
+    const int kvh = blockIdx.y / p.head_tiles, ht = blockIdx.y - kvh * p.head_tiles;
+    const int per = a.heads / a.kv_heads, nh = min(kKeyHeads, per - ht * kKeyHeads), h0 = kvh * per + ht * kKeyHeads;
+    const int vdim = a.vdim, pos = p.b.pos[row];  // (a decode step: row = sequence)
+    const bf16_t* prow = (const bf16_t*)a.proj + (int64_t)row * a.ld;
+    const int64_t head_row = ((int64_t)p.b.slot[row] * a.kv_heads + kvh) * (a.kept + a.ring);
+    bf16_t* kcache = (bf16_t*)a.kring + head_row * kDim;
+    bf16_t* vcache = (bf16_t*)a.vring + head_row * vdim;
+    // numbers of the visible keys and their cache rows: see window_rows_kernel
+    const int n_first = min(a.keep, pos + 1), w0 = max(first_seen(a, pos), n_first), n_keys = n_first + pos - w0 + 1, w_shift = w0 - n_first;
+    const int w_row = w0 < a.kept ? w0 : a.kept + (w0 - a.kept) % a.ring, row_shift = w_row - n_first;
+    const int g_wrap = w0 < a.kept ? 0x7fffffff : n_first + a.kept + a.ring - w_row;
+    auto row_of = [&](int k) { return (unsigned)(k + (k < n_first ? 0 : row_shift) - (k < g_wrap ? 0 : a.ring)); };  // (n_first <= g_wrap)
+    const int step = max((n_keys + p.n_split - 1) / p.n_split, p.chunk), k_begin = split * step, k_end = min(n_keys, k_begin + step);
+    if (split > 0 && k_begin >= n_keys) {  // no keys: a record without weight
+        for (int i = tid; i < nh * (vdim + 2); i += kKeyThreads) {
+            const int h = i / (vdim + 2), d = i - h * (vdim + 2);
+            a.partials[(((int64_t)row * a.heads + h0 + h) * p.n_split + split) * (vdim + 2) + d] = d == 0 ? -INFINITY : 0.f;
+        }
+        return;
+    }
+    const bool owner = p.own && k_end == n_keys, made_v = a.unit_v || a.v_first != nullptr;
+    const int own = owner ? n_keys - 1 : -1;  // number of the row's own key
+
+    make_queries<bf16_t, kKeyThreads>(a, prow, row, pos, kvh, h0, nh, owner, made_v, ht == 0, kcache + row_of(n_keys - 1) * (unsigned)kDim,
+                                      vcache + row_of(n_keys - 1) * (unsigned)vdim, q, kn, vn);
+    __syncthreads();
+    for (int i = tid; i < KS * 64 + (owner ? kDim / 8 + VB * 16 : 0); i += kKeyThreads) {
+        const int at = i - KS * 64, d0 = at < 0 ? 0 : at < kDim / 8 ? 8 * at : 8 * at - kDim;
+        const int col = i & 15, h = col & 3;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (at < 0)
+                x[e] = h < nh && col < 12 ? q[h * kDim + 32 * (i >> 6) + 8 * ((i >> 4) & 3) + e] : 0.f;
+            else if (at < kDim / 8)
+                x[e] = kn[d0 + e];
+            else
+                x[e] = d0 + e >= vdim ? 0.f : made_v ? vn[d0 + e] : bf16_to_f32(prow[a.off_v + (int64_t)kvh * vdim + d0 + e]);
+        }
+        qs[i] = limbs_of(x, at < 0 ? col >> 2 : 0);
+    }
+    __syncthreads();
+
+    u32x4 kf[2][KS], vf[8][VB];
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    auto value_key = [&](int i) { return (i < 4 ? 0 : 12) + 4 * g + i; };  // this lane's value row i of a run
+    const float slope = a.slope != nullptr && head < nh ? a.slope[h0 + head] : 0.f;
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc[VB][8];
+#pragma unroll
+    for (int b = 0; b < VB; ++b)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = k_begin + kRun * wave; k0 < k_end; k0 += kRun * kKeyWaves) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const bf16_t* src = kcache + (row_of(min(k0 + 16 * t + c, k_end - 1)) * (unsigned)kDim + 8u * g);
+#pragma unroll
+            for (int s = 0; s < KS; ++s) kf[t][s] = __builtin_nontemporal_load((const u32x4*)(src + 32 * s));
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const bf16_t* src = vcache + (__umul24(row_of(min(k0 + value_key(i), k_end - 1)), (unsigned)vdim) + 8u * c);
+#pragma unroll
+            for (int b = 0; b < VB; ++b) vf[i][b] = 128 * b + 8 * c < vdim ? __builtin_nontemporal_load((const u32x4*)(src + 128 * b)) : zero;
+        }
+        const bool last = k0 + kRun >= k_end;
+        if (last) {  // the row's own key and value; rows past the end
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+                    if (k0 + 16 * t + c == own) kf[t][s] = ks[4 * s + g];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int b = 0; b < VB; ++b) {
+                    if (k0 + value_key(i) == own) vf[i][b] = vs[16 * b + c];
+                    if (k0 + value_key(i) >= k_end) vf[i][b] = zero;
+                }
+        }
+        float e[8], top = -INFINITY;
+        f32x4 d2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const bf16x8 b = __builtin_bit_cast(bf16x8, qs[s * 64 + lane]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) d2[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[t][s]), b, d2[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = k0 + 16 * t + 4 * g + r;
+                float v = cap_score(sum_limbs(d2[t][r]), a.softcap);
+                if (a.slope != nullptr) v -= slope * (float)(pos - (k < n_first ? k : k + w_shift));
+                e[4 * t + r] = k < k_end ? v : -INFINITY;
+                top = fmaxf(top, e[4 * t + r]);
+            }
+        top = fmaxf(top, lane_xor16(top));
+        top = fmaxf(top, lane_xor32(top));
+        if (__builtin_amdgcn_ballot_w64(top > m) != 0) {
+            const float m_new = fmaxf(m, top), corr = __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
+            m = m_new;
+            l *= corr;
+#pragma unroll
+            for (int b = 0; b < VB; ++b)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[b][j] *= corr;
+        }
+        const float base = m == -INFINITY ? 0.f : m;  // (no key with a weight so far)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[i] = __builtin_amdgcn_exp2f((e[i] - base) * kLog2e);  // (what the factor's rounding costs is the less the more a key weighs)
+            l += e[i];
+        }
+        const bf16x8 w = __builtin_bit_cast(bf16x8, limbs_of(e, limb));
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                u32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = __builtin_amdgcn_perm(vf[2 * i + 1][b][j >> 1], vf[2 * i][b][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
+                acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), w, acc[b][j], 0, 0, 0);
+            }
+    }
+    // ---- the waves join: lane (g, c) holds dimensions 8 (4 g + r) + j of head c & 3, and writes those of r = c >> 2
+    l += lane_xor16(l);
+    l += lane_xor32(l);
+    if (g == 0 && limb == 0) stat[0][wave][head] = m, stat[1][wave][head] = l;
+#pragma unroll
+    for (int b = 0; b < VB; ++b) {
+        float o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            f32x4 s = acc[b][j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] = sum_limbs(limb < 3 ? s[r] : 0.f);
+            o[j] = limb == 0 ? s[0] : limb == 1 ? s[1] : limb == 2 ? s[2] : s[3];
+        }
+        float* dst = red + (wave * kKeyHeads + head) * (128 * VB) + 128 * b + 32 * g + 8 * limb;
+        *(f32x4*)dst = f32x4{o[0], o[1], o[2], o[3]};
+        *(f32x4*)(dst + 4) = f32x4{o[4], o[5], o[6], o[7]};
+    }
+    __syncthreads();
+    for (int i = tid; i < nh * 128 * VB; i += kKeyThreads) {
+        const int h = i / (128 * VB), d = i - h * (128 * VB);
+        const bool sink = a.sink != nullptr && split == 0;  // (a key without a value)
+        float top = sink ? a.sink[h0 + h] : -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kKeyWaves; ++w) top = fmaxf(top, stat[0][w][h]);
+        float sum = sink ? expf(a.sink[h0 + h] - top) : 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < kKeyWaves; ++w) {
+            const float f = expf(stat[0][w][h] - top);
+            sum += f * stat[1][w][h];
+            o += f * red[(w * kKeyHeads + h) * (128 * VB) + d];
+        }
+        if (d >= vdim) continue;
+        if (p.n_split > 1) {
+            float* rec = a.partials + (((int64_t)row * a.heads + h0 + h) * p.n_split + split) * (vdim + 2);
+            rec[2 + d] = o;
+            if (d == 0) rec[0] = top, rec[1] = sum;
+        } else {
+            o /= sum;
+            if (a.off_g >= 0) o *= sigmoid_f32(bf16_to_f32(prow[a.off_g + (a.gate_values ? (h0 + h) * vdim + d : h0 + h)]));
+            ((bf16_t*)a.y)[(int64_t)row * a.ldy + (int64_t)(h0 + h) * vdim + d] = f32_to_bf16(o);
+        }
     }
 }
 
@@ -962,15 +1187,39 @@ int run_cache_write(const WinParams& p, hipStream_t s) {
     return 0;
 }
 
+template <int KS, int VB>
+int launch_keys(const WinParams& p, hipStream_t s) {
+    constexpr int kLds = (KS * 64 + 4 * KS + VB * 16) * 16 + kKeyWaves * kKeyHeads * 128 * VB * 4;
+    static hipError_t e = hipFuncSetAttribute((const void*)window_keys_kernel<KS, VB>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    MI355_CHECK_ARG(e == hipSuccess, (int)e, "window_attention: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+    hipLaunchKernelGGL((window_keys_kernel<KS, VB>), dim3(p.n_split, p.a.kv_heads * p.head_tiles, p.b.rows), dim3(kKeyThreads), kLds, s, p);
+    MI355_LAUNCH_CHECK();
+    return 0;
+}
+// Whether a decode step is one of window_keys_kernel(): bf16 rows and caches of whole 16-B vectors, head sizes that are whole products
+bool keys_fit(const WinParams& p) {
+    const mi355_window_attn_args& a = p.a;
+    const uintptr_t at = (uintptr_t)a.kring | (uintptr_t)a.vring | (uintptr_t)a.proj;
+    return p.fresh && a.path != 1 && a.dtype == MI355_BF16 && (a.dim == 64 || a.dim == 128 || a.dim == 256) && a.vdim % 8 == 0 && a.vdim <= 256 && at % 16 == 0 && a.kept + a.ring < 1 << 24;
+}
+int run_keys(WinParams p, hipStream_t s) {
+    const mi355_window_attn_args& a = p.a;
+    p.head_tiles = (a.heads / a.kv_heads + kKeyHeads - 1) / kKeyHeads;
+    if (a.vdim <= 128) return a.dim == 64 ? launch_keys<2, 1>(p, s) : a.dim == 128 ? launch_keys<4, 1>(p, s) : launch_keys<8, 1>(p, s);
+    return a.dim == 64 ? launch_keys<2, 2>(p, s) : a.dim == 128 ? launch_keys<4, 2>(p, s) : launch_keys<8, 2>(p, s);
+}
+
 template <typename T>
 int run(WinParams p, hipStream_t s) {
     const mi355_window_attn_args& a = p.a;
     if (p.fresh) {
         // splits: enough workgroups for the chip, at least 64 keys each, as far as the scratch goes.  A row of few keys has them in its first splits, a pass of keys each, and leaves the others
-        // empty: each split prepares the row's queries again (16 sequences of 32 to 512 keys, 4 layers, 4 steps: 2588 -> 2562 us, of 96 to 1536 2638 -> 2630)
-        const int per = a.heads / a.kv_heads, ht = per >= 5 ? 8 : per >= 2 ? 4 : 1;
+        // empty: each split prepares the row's queries again (16 sequences of 32 to 512 keys, 4 layers, 4 steps: 2588 -> 2562 us, of 96 to 1536 2638 -> 2630).  window_keys_kernel(), three
+        // workgroups to a CU, is best with about two for each (16 sequences of 96 to 1536 keys, 8 key heads, with the join: 1 / 2 / 3 / 4 / 6 / 8 splits 36 / 28 / 26 / 23.5 / 24 / 28 us)
+        const bool keys = keys_fit(p);
+        const int per = a.heads / a.kv_heads, ht = keys ? kKeyHeads : per >= 5 ? 8 : per >= 2 ? 4 : 1;
         const int groups = p.b.rows * a.kv_heads * ((per + ht - 1) / ht);
-        int n = 2048 / groups;
+        int n = (keys ? 512 : 2048) / groups;
         p.chunk = kPassKeys;
         const int most = (a.keep + (a.window < a.ring ? a.window : a.ring)) / 64;
         n = n < most ? n : most;
@@ -979,7 +1228,7 @@ int run(WinParams p, hipStream_t s) {
         if (a.partials == nullptr) n = 1;
         while (n > 1 && rec * n > a.partials_bytes) n /= 2;
         p.n_split = n < 1 ? 1 : n;
-        if (int rc = run_rows<T>(p, s)) return rc;
+        if (int rc = keys ? run_keys(p, s) : run_rows<T>(p, s)) return rc;
         if (p.n_split > 1) {
             hipLaunchKernelGGL(window_join_kernel<T>, dim3(a.heads, p.b.rows), dim3(128), 0, s, p);
             MI355_LAUNCH_CHECK();

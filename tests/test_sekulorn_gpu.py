@@ -96,6 +96,55 @@ def test_window_attention_split_decode_and_larger_ring(dev):
     assert rel(out, ref) < TOL[torch.float32]
 
 
+DECODE_FORMS = [  # heads, key heads, dim, vdim, window, ring, options
+    (8, 2, 128, 128, 1000, 1000, {}), (4, 4, 64, 64, 300, 320, dict(rot=64)), (10, 2, 64, 40, 77, 90, dict(keep=3, slope=True)), (16, 2, 256, 256, 200, 256, dict(rot=32, gate="values")),
+    (6, 2, 128, 200, 500, 500, dict(keep=40, sink=True, gate="heads")), (4, 1, 256, 64, 33, 33, dict(softcap=3.0, sink=True)), (8, 1, 64, 128, 600, 700, dict(chunked=True, head_scale=True)),
+    (3, 1, 128, 8, 1, 1, dict(gate="heads")), (8, 2, 128, 128, 400, 512, dict(unit=True, rot=64, unit_v=True, gate="heads")), (8, 8, 64, 128, 2000, 2000, dict(unit=True, rot=16, v_first=True, slope=True)),
+    (4, 1, 128, 128, 256, 256, dict(borrows=True, rot=128)),
+]
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("H,G,dim,vdim,window,ring,o", DECODE_FORMS)
+def test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, window, ring, o, split):
+    """window_keys_kernel takes what window_rows_kernel takes (path 1), wherever a run of keys ends: first positions, the ring's wrap, the row's own key.  Both sum f32 products in f32
+    (1e-4 of a head's size covers the order of up to 2000 terms), so what differs is a rounding of the result now and then: a step of bf16's 8 bits, 2^-7 of it at most.  The cache rows are the same bits."""
+    from lit_llama_amd import ops
+
+    gen = torch.Generator(device=dev).manual_seed(H * dim + vdim + window)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev)  # noqa: E731
+    keep, pos = o.get("keep", 0), [0, 1, 31, 32, 33, ring - 1, ring, ring + 5, 3 * ring + 17, 127, 1500]
+    kept, B = (keep + 3) // 4 * 4, len(pos)
+    off = [0, H * dim, (H + G) * dim, (H + G) * dim + G * vdim]
+    proj = rnd(B, off[3] + H * vdim).bfloat16()
+    rings = rnd(B, G, kept + ring, dim).bfloat16(), rnd(B, G, kept + ring, vdim).bfloat16()
+    rot = o.get("rot", 0)
+    kw = dict(heads=H, scale=1.5 * dim ** -0.5, window=window, off_q=off[0], off_k=off[1], off_v=off[2], off_g=off[3] if "gate" in o else -1, gate_values=o.get("gate") == "values",
+              keep=keep, kept=kept, softcap=o.get("softcap", 0.0), chunked=o.get("chunked", False), inv_freq=5000.0 ** (-torch.arange(rot // 2, device=dev).double() * 2 / rot) if rot else None,
+              partials=torch.zeros(1 << 22, device=dev) if split else None)
+    for name, size in (("sink", H), ("slope", H), ("head_scale", H)):
+        if name in o:
+            kw[name] = rnd(size).abs() * (0.02 if name == "slope" else 1)
+    if "unit" in o:
+        kw.update(unit_eps=1e-6, q_norm=rnd(dim).abs(), k_norm=rnd(dim).abs())
+    if "unit_v" in o:
+        kw["unit_v_eps"] = 1e-6
+    if "v_first" in o:
+        kw.update(v_first=rnd(B, G * vdim).bfloat16(), v_mix=0.3)
+    if "borrows" in o:
+        kw.update(role="borrows", kv_rows=rnd(B * G * (dim + vdim)).bfloat16())
+    b, got = ops.PackedBatch([1] * B, list(range(B))[::-1], pos, dev), []
+    for path in (0, 1):
+        kr, vr = rings[0].clone(), rings[1].clone()
+        got.append((ops.window_attention(proj, b, kr, vr, path=path, **kw).double(), kr, vr))
+    (y, kr, vr), (ref, kr1, vr1) = got
+    assert torch.isfinite(ref).all() and ref.abs().max() > 0.1
+    size = ref.view(B, H, vdim).square().mean(-1, keepdim=True).sqrt().expand(B, H, vdim).reshape(ref.shape)
+    bad = (y - ref).abs() > 2.0 ** -7 * ref.abs() + 1e-4 * size
+    assert not bad.any()
+    assert torch.equal(kr, kr1) and torch.equal(vr, vr1)
+
+
 def test_far_positions_keep_their_angle(dev):
     """Two rows a million positions in: rotation depends on the distance only."""
     from lit_llama_amd import ops
