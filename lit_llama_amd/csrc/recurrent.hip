@@ -12,9 +12,11 @@
 
 namespace {
 
-// state S [dim][vdim] of one (slot, head): column 64 * slice + lane, rows part * RMAX + r in registers
-template <typename T, int KIND, int RMAX>
-__global__ __launch_bounds__(1024) void rec_rows_kernel(const RecParams p) {
+// State S [dim][vdim] of one (slot, head): column 64 * slice + lane, rows part * RMAX + r in registers.  A decode step's time is the state's way from memory and back, and a chain of round
+// trips from the projections to the output: the state is requested in one go, without a branch, a vector or an address register per row, non-temporal.  16 sequences, 32 heads of 128 x
+// 128: delta rule 28.0 -> 18.2 us, GLA 20.2 -> 15; 64 sequences 103 -> 61, 72 -> 51 (268 MB read and written: 4.4 and 5.2 TB/s).
+template <typename T, int KIND, int RMAX, int THREADS>
+__global__ __launch_bounds__(THREADS, THREADS <= 512 ? 2 : 4) void rec_rows_kernel(const RecParams p) {
     const mi355_recurrent_args& a = p.a;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ float red[32];
@@ -41,11 +43,24 @@ __global__ __launch_bounds__(1024) void rec_rows_kernel(const RecParams p) {
     const bool col_ok = col < vdim;
 
     float S[RMAX];
+    // (a row of the state is a scalar offset, a column past the last one no address: nothing is read there, nothing written)
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(state, 0, dim * vdim * 4, 0x00020000);
+    const unsigned col_at = col_ok ? col * 4u : 0xFFFFFFF0u;
+    const int row_at = part * RMAX * vdim * 4;
+    const bool whole = (part + 1) * RMAX <= dim;  // (no branch between the rows)
+    auto request_state = [&]() __attribute__((always_inline)) {
+        auto row = [&](int r) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, col_at, row_at + r * vdim * 4, 2)); };
+        if (whole) {
 #pragma unroll
-    for (int r = 0; r < RMAX; ++r) {
-        const int i = part * RMAX + r;
-        S[r] = (col_ok && i < dim) ? state[(int64_t)i * vdim + col] : 0.f;
-    }
+            for (int r = 0; r < RMAX; ++r) S[r] = row(r);
+        } else {
+#pragma unroll
+            for (int r = 0; r < RMAX; ++r) S[r] = part * RMAX + r < dim ? row(r) : 0.f;
+        }
+    };
+    // the delta rule's chain is the longest: what it starts from is requested in front of the state (16 waves have no registers for both)
+    constexpr bool kAhead = KIND == MI355_REC_DELTA && THREADS < 1024;
+    if constexpr (!kAhead) request_state();
     for (int i = tid; i < p.parts * RMAX; i += nt) q[i] = k[i] = al[i] = uk[i] = 0.f;
     __syncthreads();
 
@@ -54,10 +69,74 @@ __global__ __launch_bounds__(1024) void rec_rows_kernel(const RecParams p) {
         // ---- the row's q, k (and decays) into LDS
         // (what needs no LDS is requested here, in front of the barriers: one memory latency instead of one per use)
         const bool out_ok = part == 0 && col_ok;
-        float gate = out_ok ? silu_f32(to_f32<T>(row[a.off_g + head * vdim + col])) : 0.f;
-        if constexpr (KIND != MI355_REC_SSD) gate *= out_ok ? a.head_norm[head * a.norm_ld + col] : 0.f;
+        float gate = 0.f;
+        if constexpr (!kAhead) {
+            gate = out_ok ? silu_f32(to_f32<T>(row[a.off_g + head * vdim + col])) : 0.f;
+            if constexpr (KIND != MI355_REC_SSD) gate *= out_ok ? a.head_norm[head * a.norm_ld + col] : 0.f;
+        }
         float g = 1.f, beta = 1.f, v = 0.f;
-        if constexpr (KIND == MI355_REC_DELTA) {
+        if constexpr (kAhead) {
+            const int c0 = col_ok ? col : vdim - 1, vcol = head * vdim + c0, d0 = tid < dim ? tid : dim - 1;  // (threads without a column or a dimension read the last one's)
+            const T a_in = row[a.off_a + head], b_in = row[a.off_b + head], gate_in = row[a.off_g + vcol];
+            const float bias_in = a.dt_bias[head], log_in = a.a_log[head], norm_in = a.head_norm[head * a.norm_ld + c0];
+            const int nqk = a.kv_heads * dim, cq = kvh * dim + d0;
+            const int off[3] = {a.off_v + vcol, a.off_q + cq, a.off_k + cq}, at[3] = {2 * nqk + vcol, cq, nqk + cq};
+            const float* const w[3] = {a.conv_v + (int64_t)vcol * a.taps, a.conv_q + (int64_t)cq * a.taps, a.conv_k + (int64_t)cq * a.taps};
+            float y[3] = {0.f, 0.f, 0.f};
+            T x[3][4];
+            float wj[3][4];
+            bool ok[3][4];
+            auto request_taps = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        ok[n][j] = j0 + j < a.taps;
+                        const int back = ok[n][j] ? j0 + j : 0;
+                        x[n][j] = *conv_input<T>(a, rows, ring, ring_ld, off[n], at[n], t - back, pos0, ok[n][j]);
+                        wj[n][j] = w[n][a.taps - 1 - back];
+                    }
+            };
+            auto add_taps = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int n = 0; n < 3; ++n)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) y[n] += ok[n][j] ? wj[n][j] * to_f32<T>(x[n][j]) : 0.f;
+            };
+            request_taps(0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t == 0) request_state();
+            __builtin_amdgcn_sched_barrier(0);
+            add_taps();
+            for (int j0 = 4; j0 < a.taps; j0 += 4) request_taps(j0), add_taps();
+            const float dt = softplus_f32(to_f32<T>(a_in) + bias_in);
+            g = expf(-expf(log_in) * dt);
+            if (col_ok) v = silu_f32(y[0]);
+            float sq = 0.f, sk = 0.f;
+            for (int d = tid; d < dim; d += nt) {
+                const int c = kvh * dim + d;
+                float qv, kv;
+                if (d == tid) {
+                    qv = silu_f32(y[1]), kv = silu_f32(y[2]);
+                } else {  // (more dimensions than threads)
+                    qv = conv_at<T>(a, rows, ring, ring_ld, a.off_q + c, c, a.conv_q + (int64_t)c * a.taps, t, pos0);
+                    kv = conv_at<T>(a, rows, ring, ring_ld, a.off_k + c, nqk + c, a.conv_k + (int64_t)c * a.taps, t, pos0);
+                }
+                q[d] = qv;
+                k[d] = kv;
+                sq += qv * qv;
+                sk += kv * kv;
+            }
+            beta = sigmoid_f32(to_f32<T>(b_in));
+            if (out_ok) gate = silu_f32(to_f32<T>(gate_in)) * norm_in;
+            sq = block_sum(sq, red);
+            sk = block_sum(sk, red);
+            const float iq = a.q_scale / sqrtf(sq + a.unit_eps), ik = 1.0f / sqrtf(sk + a.unit_eps);
+            for (int d = tid; d < dim; d += nt) {
+                q[d] *= iq;
+                k[d] *= ik;
+            }
+        } else if constexpr (KIND == MI355_REC_DELTA) {
             const float dt = softplus_f32(to_f32<T>(row[a.off_a + head]) + a.dt_bias[head]);
             g = expf(-expf(a.a_log[head]) * dt);
             beta = sigmoid_f32(to_f32<T>(row[a.off_b + head]));
@@ -177,10 +256,8 @@ __global__ __launch_bounds__(1024) void rec_rows_kernel(const RecParams p) {
         __syncthreads();
     }
 #pragma unroll
-    for (int r = 0; r < RMAX; ++r) {
-        const int i = part * RMAX + r;
-        if (col_ok && i < dim) state[(int64_t)i * vdim + col] = S[r];
-    }
+    for (int r = 0; r < RMAX; ++r)
+        if (whole || part * RMAX + r < dim) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[r]), rs, col_at, row_at + r * vdim * 4, 2);
     // ---- a decode step's own inputs enter the ring here (row pos0 % taps held position pos0 - taps: nobody reads it any more)
     if constexpr (has_conv(KIND)) {
         if (p.b.max_count == 1) {
@@ -211,7 +288,13 @@ __global__ __launch_bounds__(256) void conv_ring_kernel(const RecParams p) {
 template <typename T, int KIND, int RMAX>
 int launch_rows(const RecParams& p, hipStream_t s) {
     const size_t lds = ((size_t)4 * p.parts * RMAX + (size_t)2 * p.parts * p.slices * 64 + kMaxRank) * 4;
-    hipLaunchKernelGGL((rec_rows_kernel<T, KIND, RMAX>), dim3(p.a.heads, p.b.seqs), dim3(64 * p.parts * p.slices), lds, s, p);
+    const int threads = 64 * p.parts * p.slices;
+    if (threads <= 256)
+        hipLaunchKernelGGL((rec_rows_kernel<T, KIND, RMAX, 256>), dim3(p.a.heads, p.b.seqs), dim3(threads), lds, s, p);
+    else if (threads <= 512)
+        hipLaunchKernelGGL((rec_rows_kernel<T, KIND, RMAX, 512>), dim3(p.a.heads, p.b.seqs), dim3(threads), lds, s, p);
+    else
+        hipLaunchKernelGGL((rec_rows_kernel<T, KIND, RMAX, 1024>), dim3(p.a.heads, p.b.seqs), dim3(threads), lds, s, p);
     MI355_LAUNCH_CHECK();
     return 0;
 }
@@ -220,9 +303,14 @@ template <typename T, int KIND>
 int run_rows(RecParams p, hipStream_t s) {
     p.slices = (p.a.vdim + 63) / 64;
     MI355_CHECK_ARG(p.slices <= 16, MI355_E_SHAPE, "recurrent: value size %d exceeds 1024", p.a.vdim);
-    // waves: up to 16, rows per thread 64 at most
-    p.parts = 16 / p.slices;
+    // Waves of a workgroup, rows of a thread 64 at most: 8 where every workgroup has a CU to itself, else 4, whose state of 64 KB (128 x 128) lies in registers of which a CU has
+    // room for two, and whose barriers are fewer (delta rule, 32 heads of 128 x 128, 16 / 8 / 4 waves: one sequence 13.5 / 11.4 / 12.7 us, eight 14.9 / 13.0 / 13.7, 16 26.9 / 23.3 /
+    // 18.2, 64 93.6 / 84.8 / 61.5; a copy of 64 states takes 54).  Of 140 launches (four kinds, seven state sizes of 16 x 200 to 256 x 256, 1 to 64 sequences, 1 to 4 rows) none is slower than
+    // before with 16 waves wherever they fit
+    p.parts = (p.a.heads * p.b.seqs <= 256 ? 8 : 4) / p.slices;
+    if (p.parts < (p.a.dim + 63) / 64) p.parts = (p.a.dim + 63) / 64;
     if (p.parts > 8) p.parts = 8;
+    if (p.parts * p.slices > 16) p.parts = 16 / p.slices;
     int rmax = (p.a.dim + p.parts - 1) / p.parts;
     while (p.parts > 1 && (p.a.dim + p.parts / 2 - 1) / (p.parts / 2) <= 8) {  // short states: fewer waves
         p.parts /= 2;

@@ -234,6 +234,30 @@ def test_recurrences(dev, dtype, kind, H, G, dim, vdim, taps):
         assert rel(run_rec(*args, cuts, path=path, taps=taps or 4), ref) < tol, (path, cuts)
 
 
+@pytest.mark.parametrize("kind,H,G,dim,vdim", [("delta", 4, 2, 128, 128), ("delta", 6, 3, 130, 70), ("gla", 4, 4, 128, 128), ("gla", 4, 4, 40, 200), ("delta", 5, 5, 100, 300)])
+def test_decode_steps_of_many_sequences_give_those_of_few(dev, kind, H, G, dim, vdim):
+    """More workgroups than CUs have four waves, fewer eight: the same f32 sums in another order (300 terms, 2e-6 of their size; three steps of it)."""
+    from lit_llama_amd import ops
+
+    B, steps = 300 // H, 3
+    p, _, off, w = rec_case(kind, B * steps, H, G, dim, vdim, torch.float32)
+    kw = {k: (tuple(t.to(dev) for t in v) if isinstance(v, tuple) else v.to(dev) if torch.is_tensor(v) else v) for k, v in w.items()}
+    p = p.view(steps, B, -1).to(dev)
+    gen = torch.Generator().manual_seed(7)
+    state0, ring0 = torch.randn((B, H, dim, vdim), generator=gen).to(dev), torch.randn((B, 4, 2 * G * dim + H * vdim), generator=gen).to(dev)
+    got = []
+    for size in (B, 9):
+        state, ring, out = state0.clone(), ring0.clone(), []
+        for i in range(steps):
+            for at in range(0, B, size):
+                n = min(size, B - at)
+                b = ops.PackedBatch([1] * n, list(range(at, at + n)), [11 + i] * n, dev)
+                out.append(ops.recurrent(kind, p[i, at:at + n].contiguous(), b, state, off=off, kv_heads=G, conv_ring=ring, path=1, **kw))
+        got.append((torch.cat(out), state, ring))
+    assert rel(got[0][0], got[1][0].double().cpu()) < 1e-5 and rel(got[0][1], got[1][1].double().cpu()) < 1e-5
+    assert torch.equal(got[0][2], got[1][2])
+
+
 @pytest.mark.parametrize("kind,tau", [("delta", 1.0), ("gla", 1.0), ("gla", 16.0)])
 def test_recurrences_with_strong_decays_and_repeated_keys(dev, kind, tau):
     T, H, G, dim, vdim = 300, 2, 2, 48, 32
