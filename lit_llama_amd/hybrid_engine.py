@@ -635,13 +635,12 @@ class HybridEngine:
         this engine when one sub-step was enough: valid until the next step).  Work is queued on the current stream's behalf."""
         entries = [e for e in entries if len(e.tokens)]
         cur = torch.cuda.current_stream(self.device)
+        self.stream.wait_stream(cur)
         outs = []
         with torch.cuda.device(self.device), torch.cuda.stream(self.stream):
             subs = self._cut(entries)
             for sub in subs:
                 b, n_want = self._upload(sub)
-                if sub is subs[0]:
-                    self.stream.wait_stream(cur)  # (behind the upload, which only this engine's own steps read: 8 us of a step of 16 sequences)
                 self._run(b, n_want)
                 if n_want:
                     out = self.logits_buf[:n_want, : self.n_logits]
