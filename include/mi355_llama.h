@@ -996,6 +996,8 @@ int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq_batch* b, 
                          int n_want, float* logits, int run_end, mi355_stream_t stream);
 /* zero the state of `n` slots (device list) in every recurrent run and token shift */
 int mi355_hybrid_reset_slots(const mi355_hybrid_model* m, const int32_t* slots, int n, mi355_stream_t stream);
+/* the same for one slot whose number the host has */
+int mi355_hybrid_reset_slot(const mi355_hybrid_model* m, int slot, mi355_stream_t stream);
 /* greedy end of a decode step, one row per sequence: next[b] = tokens[b] = argmax(logits[b]), out[b * ld_out + pos[b] + 1] = it
  * (out may be NULL), pos[b] += 1 */
 int mi355_argmax_advance_rows(const float* logits, int64_t ld, int vocab, int seqs, int32_t* next, int32_t* tokens, int32_t* pos,

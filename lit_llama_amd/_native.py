@@ -325,6 +325,7 @@ PROTOTYPES = {
     "mi355_recurrent_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "mi355_hybrid_forward": (c_int, [C.POINTER(HybridModel), C.POINTER(SeqBatch), c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p]),
     "mi355_hybrid_reset_slots": (c_int, [C.POINTER(HybridModel), c_void_p, c_int, c_void_p]),
+    "mi355_hybrid_reset_slot": (c_int, [C.POINTER(HybridModel), c_int, c_void_p]),
     "mi355_argmax_advance_rows": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "mi355_gptq_row_params": (c_int, [c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "mi355_gptq_block": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_int64,

@@ -562,16 +562,11 @@ class HybridEngine:
         """A slot for a new sequence, its recurrent state zeroed."""
         with torch.cuda.stream(self.stream):
             slot = self.slots.acquire()
-            self._reset([slot])
+            check(lib().mi355_hybrid_reset_slot(C.byref(self.m), slot, self.stream.cuda_stream), "mi355_hybrid_reset_slot")
         return slot
 
     def release(self, slot: int) -> None:
         self.slots.release(slot)
-
-    def _reset(self, slots: List[int]) -> None:
-        t = torch.tensor(slots, dtype=torch.int32).to(self.device)
-        check(lib().mi355_hybrid_reset_slots(C.byref(self.m), ptr(t), len(slots), self.stream.cuda_stream), "mi355_hybrid_reset_slots")
-        self.stream.synchronize()  # (`t` may go)
 
     # ---- steps -----------------------------------------------------------------------------------------
     def _batch(self, rows: int, seqs: int, max_count: int, max_end: int = 0) -> SeqBatch:
@@ -588,7 +583,7 @@ class HybridEngine:
         for e in entries:
             t = e.tokens if isinstance(e.tokens, (list, tuple, range)) else torch.as_tensor(e.tokens).tolist()
             row0.append(len(tokens)), count.append(len(t)), slot.append(e.slot), pos.append(e.pos)
-            want.extend([len(tokens) + k for k in e.want])
+            want.extend([len(tokens) + int(k) for k in e.want])
             tokens.extend(t)
         self._meta_sent.synchronize()  # the previous upload has left the pinned buffer
         for row, numbers in zip(self._meta_rows, lists):

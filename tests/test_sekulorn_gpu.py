@@ -321,6 +321,34 @@ def test_model_layer_by_layer_and_logits(dev, name):
     eng.release(s)
 
 
+@pytest.mark.parametrize("runs", [3, 40])  # (one launch's regions, and more)
+def test_a_slot_is_cleared_in_every_run_and_no_other_slot_is(dev, runs):
+    import ctypes as C
+
+    from lit_llama_amd import _native as nat
+
+    sizes = [(3, 5, 7), (4, 128, 128), (1, 1, 1), (2, 64, 33)]
+    layers, states, shifts = (nat.HybridLayer * runs)(), [], []
+    for i in range(runs):
+        H, d, v = sizes[i % 4]
+        states.append(torch.ones((4, H, d, v), device=dev))
+        shifts.append(torch.ones((4, 30), device=dev))
+        l = layers[i]
+        l.mixer, l.n_mix, l.shift = 1, i % 2, shifts[i].data_ptr()
+        l.rec.heads, l.rec.dim, l.rec.vdim, l.rec.state = H, d, v, states[i].data_ptr()
+    m = nat.HybridModel()
+    m.n_runs, m.width, m.layers = runs, 30, layers
+    stream = torch.cuda.current_stream().cuda_stream
+    slots = torch.tensor([3, 0], dtype=torch.int32, device=dev)
+    nat.check(nat.lib().mi355_hybrid_reset_slot(C.byref(m), 1, stream), "reset_slot")
+    for live in ([0, 2, 3], [2]):
+        for i in range(runs):
+            for t, cleared in ((states[i], True), (shifts[i], i % 2 == 1)):
+                assert [bool((t[s] == 1).all()) for s in range(4)] == [s in live or not cleared for s in range(4)], (i, live)
+                assert not cleared or all(bool((t[s] == 0).all()) for s in range(4) if s not in live)
+        nat.check(nat.lib().mi355_hybrid_reset_slots(C.byref(m), slots.data_ptr(), 2, stream), "reset_slots")
+
+
 @pytest.mark.parametrize("name,dtype,tol", [("mixed", torch.float32, 1e-4), ("mixed", torch.bfloat16, 0.12), ("all looped", torch.bfloat16, 0.12)])
 def test_portions_batches_slots_and_decoding(dev, name, dtype, tol):
     """Unequal requests in one batch, cut differently, decoded together, their slots used again: the logits of each alone."""
