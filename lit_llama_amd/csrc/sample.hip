@@ -181,40 +181,55 @@ __device__ __forceinline__ float wave_incl_scan(float v, int lane) {
 // The code of this kernel is fetched cold on every token (the decode step before it streams 3.4 GB through the L2, and
 // ONE workgroup runs it): every loop below stays rolled (`unroll 1`) on purpose.  A fully unrolled, register-resident
 // version was 27 us back to back and 157 us behind a decode step: 10k straight-line instructions at instruction-miss
-// latency.  The scaled logits live in LDS with one pad word per 32, so that both the coalesced fill (consecutive
-// threads, consecutive words) and the thread-contiguous passes (thread t owns indices [t ch, (t + 1) ch): the CDF runs
-// in index order) are free of bank conflicts.
+// latency.  A rolled pass costs an LDS round trip per iteration and little else, so an iteration takes 16 bytes: a pass over 32 values of a thread is 8 of them
+// (one value at a time: a sampled token of 7B bf16 took 10 us more, of three int4 layers, whose code is warmer, 5.5).  The scaled logits live in LDS in chunks of four, the
+// eight chunks of a row of 32 permuted by the row, so that both the coalesced fill (consecutive threads, consecutive chunks) and the thread-contiguous passes
+// (thread t owns indices [t ch, (t + 1) ch): the CDF runs in index order) are free of bank conflicts.
 __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, float temperature, int top_k,
                                                     const float* uniforms, int32_t* next_token, int32_t* out_tokens,
                                                     int32_t* tokens, int32_t* pos, int advance, float* probs_out) {
-    extern __shared__ __attribute__((aligned(16))) float vals[];  // [V + V / 32]
+    extern __shared__ __attribute__((aligned(16))) float vals[];  // [V up to whole rows of 32]
     __shared__ unsigned hist[16][256];  // one histogram per wave: a shared one serialises on the hot bins
     __shared__ float red[32];
-    __shared__ float cand[kT];
+    __shared__ __attribute__((aligned(16))) float cand[kT];
     __shared__ unsigned sh_bin, sh_rank, sh_n, sh_cnt, sh_thr, sel_prefix, sel_rank;
     __shared__ int winner, lastk;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ps = pos[0];
     const float u = uniforms[ps];
-    const int ch = (V + kT - 1) / kT;  // <= kCH (host check)
+    const int ch = (V + 4 * kT - 1) / (4 * kT) * 4;  // whole chunks, <= kCH (host check)
     const int i0 = tid * ch;
     const int i1 = i0 + ch < V ? i0 + ch : V;  // this thread's indices: [i0, i1) (empty past the vocabulary)
-    auto at = [&](int i) -> float& { return vals[i + (i >> 5)]; };
-    // fill: 8 coalesced loads in flight per thread and round (the row was just written by another kernel: memory latency)
+    auto place = [](int q) { return (q & ~7) | ((q ^ (q >> 3)) & 7); };  // of chunk q (values 4 q .. 4 q + 3)
+    auto chunk = [&](int q) -> f32x4& { return ((f32x4*)vals)[place(q)]; };
+    auto at = [&](int i) -> float& { return vals[4 * place(i >> 2) + (i & 3)]; };
+    // f(value, its index) over this thread's indices, four per iteration; what lies past the vocabulary in the last chunk is left out
+    auto each = [&](auto&& f) __attribute__((always_inline)) {
 #pragma unroll 1
-    for (int b = 0; b < V; b += 8 * kT) {
-        float t[8];
+        for (int q = i0 >> 2; 4 * q < i1; ++q) {
+            const f32x4 x = chunk(q);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int i = b + q * kT + tid;
-            t[q] = i < V ? logits[i] : 0.f;
+            for (int e = 0; e < 4; ++e)
+                if (4 * q + e < i1) f(x[e], 4 * q + e);
+        }
+    };
+    // fill: four coalesced loads of four values in flight per thread and round (the row was just written by another kernel: memory latency)
+    struct __attribute__((packed, aligned(4))) Four { float v[4]; };
+#pragma unroll 1
+    for (int b = 0; b < V / 4; b += 4 * kT) {
+        Four t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int c = b + q * kT + tid;
+            t[q] = ((const Four*)logits)[c < V / 4 ? c : 0];
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int i = b + q * kT + tid;
-            if (i < V) at(i) = t[q] / temperature;  // IEEE division, as `logits / temperature`
+        for (int q = 0; q < 4; ++q) {
+            const int c = b + q * kT + tid;
+            if (c < V / 4) chunk(c) = f32x4{t[q].v[0] / temperature, t[q].v[1] / temperature, t[q].v[2] / temperature, t[q].v[3] / temperature};  // IEEE division, as `logits / temperature`
         }
     }
+    if (tid < V % 4) at(V / 4 * 4 + tid) = logits[V / 4 * 4 + tid] / temperature;
     if (tid == 0) {
         sh_bin = 255u;
         sh_cnt = 0u;
@@ -224,12 +239,7 @@ __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, 
     }
     __syncthreads();
     float mx = -INFINITY, sum = 0.f;
-#pragma unroll 1
-    for (int i = i0; i < i1; ++i) {
-        const float x = at(i);
-        mx = fmaxf(mx, x);
-        sum += x;
-    }
+    each([&](float x, int) { mx = fmaxf(mx, x), sum += x; });
     mx = block_max(mx, red);  // the maximum is kept by every top-k threshold: also the softmax maximum
 
     // ---- threshold = the k-th largest scaled logit (none when top_k covers the vocabulary)
@@ -243,15 +253,14 @@ __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, 
 #pragma unroll 1
             for (int b = tid; b < 16 * 256; b += kT) (&hist[0][0])[b] = 0u;
             __syncthreads();
-#pragma unroll 1
-            for (int i = i0; i < i1; ++i) {
-                const int b = (int)fminf((mx - at(i)) * sc, 255.f);  // monotone in the value; below the mean -> 255
+            each([&](float x, int) {
+                const int b = (int)fminf((mx - x) * sc, 255.f);  // monotone in the value; below the mean -> 255
                 if (b < 255) atomicAdd(&hist[wave][b], 1u);
-            }
+            });
             __syncthreads();
             unsigned t = 0, incl = 0;
             if (tid < 256) {
-#pragma unroll 1
+#pragma unroll 4
                 for (int w = 0; w < 16; ++w) t += hist[w][tid];
                 incl = t;
 #pragma unroll
@@ -275,20 +284,21 @@ __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, 
             const unsigned bsel = sh_bin, n = sh_n, r = sh_rank;
             fast = bsel < 255u && n <= (unsigned)kT;
             if (fast) {
-#pragma unroll 1
-                for (int i = i0; i < i1; ++i) {
-                    const float x = at(i);
+                each([&](float x, int) {
                     if ((int)fminf((mx - x) * sc, 255.f) == (int)bsel) cand[atomicAdd(&sh_cnt, 1u)] = x;
-                }
+                });
                 __syncthreads();
                 if ((unsigned)tid < n) {
                     const float c = cand[tid];
                     unsigned g = 0, ge = 0;
 #pragma unroll 1
-                    for (unsigned q = 0; q < n; ++q) {
-                        const float x = cand[q];
-                        g += x > c;
-                        ge += x >= c;
+                    for (unsigned q = 0; q < n; q += 4) {
+                        const f32x4 x = *(const f32x4*)(cand + q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            g += q + e < n && x[e] > c;
+                            ge += q + e < n && x[e] >= c;
+                        }
                     }
                     if (g < r && r <= ge) sh_thr = __float_as_uint(c);  // (ties write the same value)
                 }
@@ -341,11 +351,16 @@ __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, 
     // CONTIGUOUS index ranges, inclusive scan over the threads
     float local = 0.f;
 #pragma unroll 1
-    for (int i = i0; i < i1; ++i) {
-        const float x = at(i);
-        const float e = x >= thr ? expf(x - mx) : 0.f;
-        at(i) = x >= thr ? e : -1.f;  // -1: dropped (a kept entry may underflow to 0 and stays kept)
-        local += e;
+    for (int q = i0 >> 2; 4 * q < i1; ++q) {
+        f32x4 x = chunk(q);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool kept = x[r] >= thr && 4 * q + r < i1;
+            const float e = kept ? expf(x[r] - mx) : 0.f;
+            x[r] = kept ? e : -1.f;  // -1: dropped (a kept entry may underflow to 0 and stays kept)
+            local += e;
+        }
+        chunk(q) = x;
     }
     float after = wave_incl_scan(local, lane);
     __syncthreads();
@@ -371,24 +386,21 @@ __global__ __launch_bounds__(kT) void sample_kernel(const float* logits, int V, 
             // the walk re-adds this thread's terms in the order of its partial sum
             float acc = prev;
             int pick = -1;
-#pragma unroll 1
-            for (int i = i0; i < i1; ++i) {
-                const float e = at(i);
-                if (e >= 0.f) {
+            each([&](float e, int i) {
+                if (e >= 0.f && !(acc > target)) {
                     acc += e;
                     pick = i;
-                    if (acc > target) break;
                 }
-            }
+            });
             winner = pick;  // exactly one thread's interval contains the target
         }
     }
     __syncthreads();
     if (winner < 0) {  // target fell on / past the total: the last kept index
         int last = -1;
-#pragma unroll 1
-        for (int i = i0; i < i1; ++i)
-            if (at(i) >= 0.f) last = i;
+        each([&](float e, int i) {
+            if (e >= 0.f) last = i;
+        });
         if (last >= 0) atomicMax(&lastk, last);
         __syncthreads();
         if (tid == 0) winner = lastk < 0 ? 0 : lastk;
@@ -417,9 +429,9 @@ extern "C" int mi355_sample(const float* logits, int V, float temperature, int t
     if (V <= kT * kCH) {
         static hipError_t attr_err =
             hipFuncSetAttribute((const void*)sample_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (kT * kCH + kT * kCH / 32 + 1) * 4);  // = the request below at V = kT * kCH, the documented bound
+                                kT * kCH * 4);  // = the request below at V = kT * kCH, the documented bound
         MI355_CHECK_ARG(attr_err == hipSuccess, (int)attr_err, "sample: hipFuncSetAttribute failed: %s", hipGetErrorString(attr_err));
-        hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kT), (size_t)(V + V / 32 + 1) * 4, (hipStream_t)stream, logits, V,
+        hipLaunchKernelGGL(sample_kernel, dim3(1), dim3(kT), (size_t)(V + 31) / 32 * 128, (hipStream_t)stream, logits, V,
                            temperature, top_k, uniforms, next_token, out_tokens, tokens, pos, advance, probs_out);
     } else {
         const size_t lds = (size_t)V * sizeof(float);

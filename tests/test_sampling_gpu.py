@@ -15,7 +15,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("V,temperature,top_k", [(32000, 1.0, None), (32000, 0.8, 200), (32000, 0.7, 1), (32000, 1.3, 5),
-                                                 (1000, 0.5, 5000), (4099, 2.0, 37), (16, 1.0, 3)])
+                                                 (1000, 0.5, 5000), (4099, 2.0, 37), (16, 1.0, 3),
+                                                 # chunks of four: no whole one, a last one of 1 to 3 values, the last size in LDS and the first one past it
+                                                 (3, 1.0, 2), (4097, 0.9, 50), (8190, 1.1, 100), (12291, 0.8, 200), (32768, 1.0, 500), (32769, 1.0, 500)])
 def test_sample_kernel_matches_reference_arithmetic(dev, V, temperature, top_k):
     gen = torch.Generator().manual_seed(V + (top_k or 0))
     logits = torch.randn(V, generator=gen) * 3
