@@ -167,6 +167,16 @@ bool short_chunk_fits(const mi355_model* m, const mi355_weight& w, int M, int ep
     return w.R == (epi == MI355_EPI_SWIGLU ? 2 : 1) && (uintptr_t)m->gemm_ws % 16 == 0 && (size_t)m->gemm_ws_bytes >= mi355_linear_gemm_workspace_bytes(M, w.K) &&
            (!scale_groups || mi355_linear_gemm_tables_fit(M, w.N, w.K, w.R, w.group_cols));
 }
+// LLM.int8 likewise: from the second reading of the weights on (8 rows at K = 4096, 3 at 11008), and from 7 rows, which the row kernel multiplies one by one.  Prompts of two layers, all by rows
+// / all tiled: 4096 wide, 4 tokens 378 / 413 us (mlp.c_proj alone tiled 354), 6 407 / 406 (364), 7 424 / 385, 8 477 / 412, 16 804 / 419, 31 1348 / 455; 5120 wide, 4 466 / 475, 5 512 / 456, 16 1189 / 480; 8192 wide, 2 622 / 669, 3 705 / 673, 8 1470 /
+// 687, 31 5169 / 753.  Outlier columns are then those of the whole chunk, as in the reference, not of a launch's rows.
+int i8_rows(const mi355_weight& w) {
+    const int cap = row_cap(w);
+    return cap < 6 ? (cap < 1 ? 2 : cap + 1) : 7;
+}
+bool i8_chunk_fits(const mi355_model* m, const mi355_weight& w, int epi) {
+    return w.R == (epi == MI355_EPI_SWIGLU ? 2 : 1) && (uintptr_t)m->gemm_ws % 16 == 0 && (size_t)w.N * w.K * w.R < 0xF0000000ull;
+}
 // a linear the fused chain can run: int4 / bf16 stream, one scale per row or per group of whole units
 bool wide_plain(const mi355_weight& w) {
     const bool groups = in_groups(w);
@@ -238,7 +248,7 @@ FuseCtx plan_fusion(const mi355_model* m, int T) {
 // leaves the fused chain's partial sums alone, which are longer); no mask if the workspace was sized for less.
 mi355_i8_chain plan_i8_chain(const mi355_model* m, int T) {
     mi355_i8_chain c = {nullptr, 0, false};
-    if (T < 32 || m->gemm_ws == nullptr) return c;
+    if (T < 2 || m->gemm_ws == nullptr) return c;
     int K = m->lm_head.K;
     for (int l = 0; l < m->n_layer; ++l)
         for (const mi355_weight* w : {&m->layers[l].attn, &m->layers[l].proj, &m->layers[l].fc, &m->layers[l].mproj}) K = w->K > K ? w->K : K;
@@ -262,8 +272,8 @@ int run_linear(const mi355_model* m, const mi355_weight& w, const void* x, int x
         fill_linear_args(a, m, w, x, x_dtype, M, ldx, norm_scale, epi, y, y_dtype, ldy);
         return mi355_linear_gemm(&a, m->gemm_ws, (size_t)m->gemm_ws_bytes, s);
     }
-    if (w.fmt == MI355_W_I8 && M >= 32 && m->gemm_ws != nullptr && attn_partials == nullptr &&
-        (size_t)m->gemm_ws_bytes >= mi355_linear_int8_gemm_workspace_bytes(M, w.K)) {
+    if (w.fmt == MI355_W_I8 && M >= i8_rows(w) && m->gemm_ws != nullptr && attn_partials == nullptr &&
+        (size_t)m->gemm_ws_bytes >= mi355_linear_int8_gemm_workspace_bytes(M, w.K) && (M >= 32 || i8_chunk_fits(m, w, epi))) {
         // LLM.int8 prompt chunks: outlier columns over the whole chunk, int8 product on the MFMA (csrc/int8_gemm.hip)
         mi355_int8_args a;
         memset(&a, 0, sizeof(a));

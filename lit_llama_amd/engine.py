@@ -419,8 +419,8 @@ class DecodeEngine:
                 max_T = 0
             if max_T < 1:
                 raise EngineUnavailable("hidden size does not fit LDS")
-            # prompt chunks of >= 32 tokens go through the wide MFMA GEMM (csrc/gemm.hip, int8_gemm.hip; int4 and bf16 products from 8 to 32 rows on:
-            # engine.hip wide_rows) and flash attention (flash_prefill.hip), so the chunk is bounded by scratch memory only (0.6 GB at 2048 tokens
+            # prompt chunks of >= 32 tokens go through the wide MFMA GEMM (csrc/gemm.hip, int8_gemm.hip; int4 and bf16 products from 8 to 32 rows on, LLM.int8 from 2 to 7:
+            # engine.hip wide_rows, i8_rows) and flash attention (flash_prefill.hip), so the chunk is bounded by scratch memory only (0.6 GB at 2048 tokens
             # of a 7B model, 0.8 as LLM.int8: 262 MB of it f32 logits rows, which prefill() uses past the first for results off a 16-byte line).  Large chunks matter: the [n_embd]-wide outputs (c_proj, mlp.c_proj) are
             # 16 row blocks, so 512 tokens fill only a quarter of the chip (9 % vs 27-36 % of the MFMA peak at 2048)
             self.gemm_ws = None

@@ -30,6 +30,7 @@ def _reference(x, cb, scb):
     (33, 72, 200, 1), (64, 4096, 4096, 63), (200, 4096, 4096, 64), (130, 1000, 1024, 65), (257, 4096, 11008, 700), (48, 4096, 22016, 300),
     (1030, 4096, 640, 129), (2050, 1040, 512, 33), (40, 11008, 4096, 4096), (512, 4096, 1024, 0),
     (33, 1001, 4096, 3), (64, 1001, 4096, 5), (64, 4098, 4096, 70), (129, 1003, 2048, 0),  # K-slices whose rows are not whole vectors of four sums
+    (2, 4096, 11008, 40), (7, 1001, 4096, 3), (17, 12288, 4096, 70), (31, 260, 4100, 9),  # a few rows
     (100, 12292, 1152, 20), (200, 4100, 4096, 70), (257, 4096, 1030, 9), (65, 260, 12416, 2000),  # blocks of 64 tokens; rows staged element by element, up to 24 fours a thread
 ])
 @pytest.mark.parametrize("epi", ["store", "accum", "pair"])

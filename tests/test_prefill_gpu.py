@@ -159,6 +159,24 @@ def test_bf16_model_prompt_takes_the_wide_path_and_matches_oracle(dev):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("T", [2, 4, 6, 7, 12, 31])
+def test_short_llm_int8_prompts_match_oracle(dev, T):
+    """Up to where the row kernel takes a product (7B: 3 rows at K = 11008, 6 at 4096), one part of them tiled, all of them, up to the last length below 32: outlier columns over the whole prompt.
+    Band as below."""
+    cfg = LLaMAConfig(**W7B)
+    sd = synth.make_state_dict(cfg, seed=8, mode="llm.int8", dtype=torch.bfloat16, outlier_channels=8)
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode="llm.int8"):
+        model = LLaMA(cfg)
+    model.load_state_dict(sd)
+    model.eval()
+    om = oracle.Model(oracle.Config(**W7B), {k: v.float() for k, v in sd.items()}, mode="llm.int8")
+    toks = synth.make_prompt(T, seed=14 + T)
+    got = model(toks.view(1, -1).to(dev), 64, _pos(T, dev))[0].float().cpu()
+    ref = om(toks.view(1, -1), 64, torch.arange(T))[0].float()
+    assert (got - ref).abs().max().item() <= 0.15 * float(ref.std(-1).mean())
+
+
+@torch.no_grad()
 def test_llm_int8_prompt_takes_the_int8_gemm_and_matches_oracle(dev):
     """a 100-token prompt of a 7B-width llm.int8 layer through the engine — mi355_linear_int8_gemm (outlier
     columns over the whole prompt, as MatMul8bitLt determines them; the streaming kernel's <= 16-row chunks each had their own
