@@ -6,7 +6,7 @@
 // boolean causal mask (:230) — which the reference evaluates over all S cache rows; here only rows
 // [0, slot] are read.
 //
-// One workgroup per (head, query token, batch row).  K/V rows are streamed with 16-B lane loads
+// attn_kernel: one workgroup per (head, query token, batch row) (attn_tile_kernel: 16 tokens of a prompt).  K/V rows are streamed with 16-B lane loads
 // (LPR = row_bytes / 16 lanes per row, 64 / LPR rows per wave instruction), scores reduced with
 // wavefront shuffles, softmax in LDS, PV accumulated per lane and combined across waves in a fixed
 // order.  For the decode step (T == 1) the kernel also applies RoPE to the new key, writes the new
@@ -513,6 +513,182 @@ __global__ __launch_bounds__(512) void attn_kernel(const AttnParams p) {
 }
 
 // y[row, h*hs + d] = sum_j e^{m_j - M} o_j[d] / sum_j e^{m_j - M} l_j  over the n_split partial records
+
+// Several query tokens over a bf16 cache, queries in f32: a workgroup per (head, 16 tokens) on the matrix cores, its waves share out the keys in runs of 32.
+// attn_kernel reads all keys once per token, a workgroup each, and what it does per key on the VALU bounds it; here 16 tokens share a run, and queries and weights in f32 enter as three
+// bf16 each (limbs: products exact in f32, sums in f32).
+// attn_kernel -> this: 4 heads of 64, 512 tokens 45 -> 11 us, 2000 330 -> 29; 32 heads of 128, 24 tokens 15.4 -> 9.1, behind 1900 others 80 -> 32; 52 heads, 31 tokens 31 -> 9.7.
+// Error against 64 bits 1.2e-7 (1.4e-7) at 2000 tokens, 9e-8 (1e-7) at 31, behind 1900 others 2.1e-7 (2.3e-7).
+//   scores  D[key][token] = keys x queries' limbs;  weights exp(score - maximum) per lane (its column's token, eight keys), split the same way
+//   values  D[dim][token] = values^T x weights: key 8 g + j of a product is the key whose weight lane group g holds (4 g + j of the run, j < 4, or 16 + 4 g + j - 4), its row i of product
+//           j is dimension VD i + j, so a lane's loads are VD dimensions of a row and eight keys' values are turned by v_perm
+// A key that some token does not see may hold an infinity or NaN in its value, which a weight of 0 does not undo: runs that hold one take token by token.
+constexpr int kTileTokens = 16, kTileRun = 32, kTileWaves = 4;
+template <int HS>
+__global__ __launch_bounds__(64 * kTileWaves, 2) void attn_tile_kernel(const AttnParams p) {
+    constexpr int KS = HS / 32, VD = HS / 16;
+    __shared__ __attribute__((aligned(16))) float red[kTileWaves][kTileTokens][HS];
+    __shared__ float stat[2][kTileWaves][kTileTokens];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
+    const int h = blockIdx.x, t0 = blockIdx.y * kTileTokens, b = blockIdx.z;
+    const int t = t0 + c < p.T ? t0 + c : p.T - 1;  // (columns past the last token: a copy of it, never stored)
+    const int pos = p.pos ? p.pos[t] : t;
+    const int len = (pos < p.S - 1 ? pos : p.S - 1) + 1;
+    int most = len, least = len;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) most = max(most, __shfl_xor(most, o, 64)), least = min(least, __shfl_xor(least, o, 64));
+    most = __builtin_amdgcn_readfirstlane(most), least = __builtin_amdgcn_readfirstlane(least);
+    const bf16_t* kc = (const bf16_t*)p.kcache + ((int64_t)b * p.n_head + h) * p.S * HS;
+    const bf16_t* vc = (const bf16_t*)p.vcache + ((int64_t)b * p.n_head + h) * p.S * HS;
+    // limb 0, 1 or 2 of eight f32 as bf16: the upper 16 bits, of what is left the upper 16, and the rest
+    auto limbs = [](const float (&x)[8], u32x4 (&to)[3]) {
+        uint32_t r[3][8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float mid = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
+            r[0][i] = __float_as_uint(x[i]), r[1][i] = __float_as_uint(mid), r[2][i] = __float_as_uint(mid - __uint_as_float(__float_as_uint(mid) & 0xffff0000u));
+        }
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) to[l][i] = __builtin_amdgcn_perm(r[l][2 * i + 1], r[l][2 * i], 0x07060302u);
+    };
+    u32x4 q[KS][3];
+    {
+        const float* row = (const float*)p.qkv + ((int64_t)b * p.T + t) * p.ld_qkv + h * HS;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int d = 32 * s + 8 * g + 2 * i;
+                rope_pair(p.rope, p.rope_gathered ? t : pos, HS / 2, d / 2, row[d], row[d + 1], x[2 * i], x[2 * i + 1]);
+            }
+            limbs(x, q[s]);
+        }
+    }
+    constexpr float kNegBig = -1.0e30f;
+    float m = kNegBig, l = 0.f;
+    f32x4 acc[VD];
+#pragma unroll
+    for (int j = 0; j < VD; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = kTileRun * wave; k0 < most; k0 += kTileRun * kTileWaves) {
+        u32x4 kf[2][KS];
+        uint32_t vf[8][VD / 2];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const bf16_t* src = kc + (int64_t)min(k0 + 16 * half + c, most - 1) * HS + 8 * g;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) kf[half][s] = *(const u32x4*)(src + 32 * s);
+        }
+        auto value_key = [&](int i) { return k0 + (i < 4 ? 0 : 12) + 4 * g + i; };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const bf16_t* src = vc + (int64_t)min(value_key(i), most - 1) * HS + VD * c;
+            if constexpr (VD == 8) {
+                const u32x4 v = *(const u32x4*)src;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vf[i][e] = v[e];
+            } else {
+                const u32x2 v = *(const u32x2*)src;
+                vf[i][0] = v[0], vf[i][1] = v[1];
+            }
+        }
+        f32x4 d2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int limb = 2; limb >= 0; --limb)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+                    d2[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[half][s]), __builtin_bit_cast(bf16x8, q[s][limb]), d2[half], 0, 0, 0);
+        float e[8], top = kNegBig;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[i] = d2[i >> 2][i & 3] * p.scale;
+            if (value_key(i) < len) top = fmaxf(top, e[i]);
+        }
+        top = fmaxf(top, lane_xor16(top));
+        top = fmaxf(top, lane_xor32(top));
+        const float m_new = fmaxf(m, top), corr = __expf(m - m_new);
+        m = m_new;
+        l *= corr;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[i] = value_key(i) < len ? __expf(e[i] - m) : 0.f;
+            l += e[i];
+        }
+        u32x4 w[3];
+        limbs(e, w);
+        bool odd = false;
+        if (k0 + kTileRun > least) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int e2 = 0; e2 < VD / 2; ++e2) odd |= (vf[i][e2] & 0x7F80u) == 0x7F80u || (vf[i][e2] & 0x7F800000u) == 0x7F800000u;
+        }
+        // product j of the values of the keys below `end`
+        auto value = [&](int j, int end) __attribute__((always_inline)) {
+            u32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t lo = value_key(2 * i) < end ? vf[2 * i][j >> 1] : 0u, hi = value_key(2 * i + 1) < end ? vf[2 * i + 1][j >> 1] : 0u;
+                v[i] = __builtin_amdgcn_perm(hi, lo, j & 1 ? 0x07060302u : 0x05040100u);
+            }
+            return __builtin_bit_cast(bf16x8, v);
+        };
+        // (a run's products by themselves, the least first, then one rounding into the sum of the runs before)
+        auto weighted = [&](const bf16x8& v) __attribute__((always_inline)) {
+            f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int limb = 2; limb >= 0; --limb) sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8, w[limb]), sum, 0, 0, 0);
+            return sum;
+        };
+        if (__builtin_amdgcn_ballot_w64(odd) == 0) {
+#pragma unroll
+            for (int j = 0; j < VD; ++j) {
+                const f32x4 sum = weighted(value(j, 0x7fffffff));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[j][r] = __builtin_fmaf(acc[j][r], corr, sum[r]);
+            }
+        } else {
+#pragma unroll 1
+            for (int of = 0; of < kTileTokens; ++of) {
+                const int end = __builtin_amdgcn_readlane(len, of);
+#pragma unroll
+                for (int j = 0; j < VD; ++j) {
+                    const f32x4 sum = weighted(value(j, end));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[j][r] = c == of ? __builtin_fmaf(acc[j][r], corr, sum[r]) : acc[j][r];
+                }
+            }
+        }
+    }
+    // ---- the waves join: lane (g, c) holds dimensions VD (4 g + r) + j of token c
+    l += lane_xor16(l);
+    l += lane_xor32(l);
+    if (g == 0) stat[0][wave][c] = m, stat[1][wave][c] = l;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < VD; j += 4) *(f32x4*)&red[wave][c][VD * (4 * g + r) + j] = f32x4{acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r]};
+    __syncthreads();
+    for (int i = tid; i < kTileTokens * HS; i += 64 * kTileWaves) {
+        const int of = i / HS, d = i - of * HS;
+        if (t0 + of >= p.T) break;
+        float top = kNegBig, sum = 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) top = fmaxf(top, stat[0][w][of]);
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) {
+            const float f = __expf(stat[0][w][of] - top);
+            sum += f * stat[1][w][of];
+            o += f * red[w][of][d];
+        }
+        st_from_f32(p.y, ((int64_t)b * p.T + t0 + of) * p.ldy + h * HS + d, p.y_dtype, o / sum);
+    }
+}
+
 __global__ void attn_combine_kernel(const float* part, int n_split, int n_head, int hs, void* y, int y_dtype,
                                     int64_t ldy) {
     const int r = blockIdx.y, h = blockIdx.x;
@@ -632,6 +808,13 @@ extern "C" int mi355_attention(const mi355_attn_args* a, mi355_stream_t stream) 
         b.y = a->y;
         b.ldy = a->ldy;
         return mi355_adapter_prefix(&b, stream);
+    }
+    // Tokens that share their keys, where attn_kernel's workgroup per (head, token) no longer has a CU to itself (up to there 32 heads of 128, 8 tokens 7.6 us, shared 8.0; past it 12 tokens 11.2 / 8.7)
+    if (esz == 2 && (a->hs == 64 || a->hs == 128) && a->qkv_dtype == MI355_F32 && a->n_split <= 1 && !adapter && !p.fused && (int64_t)a->n_head * a->T * a->B > 256 &&
+        ((uintptr_t)p.kcache | (uintptr_t)p.vcache) % 16 == 0 && a->debug_stamps == nullptr) {
+        hipLaunchKernelGGL(a->hs == 64 ? attn_tile_kernel<64> : attn_tile_kernel<128>, dim3(a->n_head, (a->T + kTileTokens - 1) / kTileTokens, a->B), dim3(64 * kTileWaves), 0, s, p);
+        MI355_LAUNCH_CHECK();
+        return 0;
     }
     int ns = a->n_split > 1 ? a->n_split : 1;
     MI355_CHECK_ARG(ns == 1 || a->partials != nullptr, MI355_E_ARG, "attention: n_split > 1 needs a partials buffer");

@@ -491,6 +491,46 @@ def test_split_attention_equals_single_workgroup_and_feeds_the_projection(dev, n
     assert (got - ref).abs().max().item() <= 5e-3 * _rms(ref)
 
 
+@pytest.mark.parametrize("H,hs,T,first,S,B,out", [
+    (52, 128, 5, 0, 64, 1, torch.float32), (32, 128, 9, 300, 400, 1, torch.float32), (32, 128, 31, 0, 31, 1, torch.bfloat16), (24, 128, 17, 40, 50, 1, torch.float32),
+    (4, 64, 65, 0, 80, 1, torch.float32), (5, 64, 129, 7, 200, 1, torch.float32), (2, 64, 700, 0, 700, 1, torch.float32), (3, 64, 100, 30, 97, 1, torch.float32),
+    (4, 64, 48, 0, 48, 3, torch.float32), (6, 128, 33, 5, 60, 2, torch.float32),
+])
+@pytest.mark.parametrize("odd", [False, True])
+def test_attention_of_tokens_that_share_their_keys(dev, H, hs, T, first, S, B, out, odd):
+    """More (head, token) pairs than CUs, f32 queries over a bf16 cache, against 64 bits: positions in any order, past the cache's end (the last row), several batch rows, and an infinite value in the
+    last row, which only those that see it may take over.  f32 sums of up to 2048 terms and exponentials of |score| < 20: 1e-6 of the result; bf16 results 2^-8."""
+    g = torch.Generator().manual_seed(T)
+    qkv = torch.randn((B, T, 3 * H * hs), generator=g)
+    rope = oracle.build_rope_cache(1024, hs, dtype=torch.int64)
+    cs = rope.double()
+    pos = first + torch.randperm(T, generator=g)
+    last = pos.clamp(max=S - 1)
+    if odd:  # the value of one token whose row most of the others do not see
+        t_odd = int(pos.argmax())
+        qkv[:, t_odd, 2 * H * hs + 3] = float("inf")
+    cache = torch.randn((B, H, S, hs), generator=g).bfloat16().to(dev), torch.randn((B, H, S, hs), generator=g).bfloat16().to(dev)
+
+    def turn(x):  # [B, T, H, hs]
+        x = x.double().view(B, T, H, hs // 2, 2)
+        c, s = cs[pos][None, :, None, :, 0], cs[pos][None, :, None, :, 1]
+        return torch.stack([x[..., 0] * c - x[..., 1] * s, x[..., 1] * c + x[..., 0] * s], -1).reshape(B, T, H, hs)
+
+    q, k, v = qkv.view(B, T, 3, H, hs).unbind(2)
+    clash = int((last == S - 1).sum()) > 1  # several tokens write the last row: which of them stays is not said
+    y = ops.attention(qkv.to(dev), rope.to(dev), H, pos=pos.to(dev), kv_cache=cache, out_dtype=out).double().cpu()
+    kc, vc = cache[0].double().cpu(), cache[1].double().cpu()
+    score = turn(q).transpose(1, 2) @ kc.transpose(-1, -2) * hs ** -0.5
+    hide = torch.arange(S)[None, :] > last[:, None]
+    w = torch.softmax(score.masked_fill(hide, float("-inf")), -1)
+    ref = torch.stack([w[..., i, : int(last[i]) + 1][..., None, :] @ vc[..., : int(last[i]) + 1, :] for i in range(T)], 2)[..., 0, :]  # (an infinity times a weight of 0 is none of it)
+    ref = ref.transpose(1, 2).reshape(B, T, H * hs)
+    assert clash or torch.equal(cache[1][:, :, last].float().cpu(), v.bfloat16().float().transpose(1, 2))
+    assert torch.equal(torch.isfinite(y), torch.isfinite(ref)) and (odd or bool(torch.isfinite(y).all()))
+    y, ref = y.nan_to_num(0, 0, 0), ref.nan_to_num(0, 0, 0)
+    assert (y - ref).norm() <= (1e-6 if out == torch.float32 else 2.0 ** -8) * ref.norm()
+
+
 def test_attention_without_cache_batched(dev):
     B, T, n_head, hs = 3, 9, 4, 8
     C = n_head * hs
