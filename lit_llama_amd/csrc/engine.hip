@@ -149,17 +149,27 @@ int row_cap(const mi355_weight& w) {
     }
     return cap;
 }
-// Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per row_cap() rows (7B: 13 at K = 4096, 5 at
-// 11008): from the second reading on, and 8 rows (int4 of one scale per row, the cheapest to read again: 11).  Eight layers of a 7B model, all by rows / by
-// this rule: bf16 6 rows 896 / 896 us (926 with the tiled kernel from row 6 on), 8 1057 / 963, 12 1163 / 1056, 16 1614 / 1136, 31 2824 / 1236; int4 8 rows 652 / 652
-// (689), 11 802 / 737, 16 1146 / 839, 31 1877 / 965; groups of 128 columns 8 rows 752 / 749, 10 896 / 813, 16 1362 / 1030, 31 2318 / 1164.  Int4 scales that the
-// tiled kernel cannot apply unit by unit (mi355_linear_gemm): 32 rows, their sums over a whole K-slice in one accumulator cost a short chunk precision.
+// Rows from which a product takes the tiled kernel instead of the row kernel, which reads the weights once per row_cap() rows (7B: 13 at K = 4096, 5 at 11008): from the second reading on.
+// Tiled less by rows, us a layer, K = 13824 / 17920 / 22016 in front of 5120 / 6656 / 8192 rows: bf16 -29 / -37 / -58 there, groups of 128 columns -17 / -18 / -9, int4 of one scale per row, the
+// cheapest to read again, -4.5 / -1.7 / 0.  A tiled launch costs that one some 12 us more (staging, K-slices' sum), so what it reads again must be 30 MB at least (K = 11008, 4096 rows: second
+// reading +4.4 us, third -5.6), or the rows 11 (8192 wide, 8 rows: 702 us of two layers, all tiled 443; 4 rows 403 / 434).
+// bf16 from 11 rows in any case (7B, 10 rows 0.4, 12 rows -5 us a layer, 13B -8.5 and -11.5), and rows of 512 columns and less, which the row kernel multiplies one by one, from 8 (256 wide: -5
+// us a layer, 6 rows -0.4, 12 -12).  Int4 scales that the tiled kernel cannot apply unit by unit (mi355_linear_gemm): 32 rows, their sums over a whole K-slice in one accumulator cost a short
+// chunk precision.
 int wide_rows(const mi355_weight& w) {
     const bool by_unit = w.sz_dtype == MI355_BF16 && w.K % 128 == 0 && (w.group_cols == 0 || w.group_cols >= 128);
     if (w.fmt == MI355_W_Q4 && !by_unit) return 32;
-    const int cap = row_cap(w);
-    const int from = w.fmt == MI355_W_Q4 && (w.group_cols == 0 || w.group_cols >= w.K) ? 11 : 8;
-    return cap < from ? from : cap < 31 ? cap + 1 : 32;
+    if (w.K <= 512) return 8;
+    const int cap = row_cap(w) > 1 ? row_cap(w) : 1;
+    int from = cap + 1;
+    if (w.fmt == MI355_W_BF16) {
+        from = from < 11 ? from : 11;
+    } else if (!in_groups(w)) {
+        const double bytes = 0.5 * w.N * w.K * w.R;
+        const int cheap = cap * (bytes >= 30e6 ? 1 : bytes >= 15e6 ? 2 : 3) + 1, rows = cap < 11 ? 11 : cap + 1;
+        from = cheap < rows ? cheap : rows;
+    }
+    return from < 32 ? from : 32;
 }
 // Chunks of fewer than 32 rows were the row kernel's before they could be tiled: what the tiled kernel does not take stays there
 bool short_chunk_fits(const mi355_model* m, const mi355_weight& w, int M, int epi) {

@@ -159,6 +159,35 @@ def test_bf16_model_prompt_takes_the_wide_path_and_matches_oracle(dev):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("fmt,lengths", [("int4", [4, 5, 10, 12]), ("int4-g128", [3, 4, 8]), ("bf16", [5, 6, 11, 14])])
+def test_prompts_around_where_products_are_tiled_match_oracle(dev, fmt, lengths):
+    """13B width, a small vocabulary: one row below and at the second reading of the weights of mlp.c_proj (K = 13824: 4 rows int4, 3 with group tables, 5 bf16) and of the others, bf16 at 11 rows."""
+    from lit_llama_amd.quantization import ColBlockQuantizedLinear
+
+    width = dict(n_layer=1, n_head=40, n_embd=5120, vocab_size=1024)
+    cfg = LLaMAConfig(**width)
+    mode = None if fmt == "bf16" else "gptq.int4"
+    sd = synth.make_state_dict(cfg, seed=3, mode=mode, **({"group_cols": 128} if fmt == "int4-g128" else {"dtype": torch.bfloat16} if mode is None else {}))
+    with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16, quantization_mode=mode):
+        model = LLaMA(cfg)
+        if fmt == "int4-g128":
+            for m in list(model.modules()):
+                for name, child in list(m.named_children()):
+                    if isinstance(child, ColBlockQuantizedLinear):
+                        setattr(m, name, ColBlockQuantizedLinear(child.in_features, child.out_features, bias=False, bits=4, tile_cols=128))
+    model.load_state_dict(sd)
+    model.eval()
+    om = oracle.Model(oracle.Config(**width), {k: (v.float() if v.is_floating_point() else v) for k, v in sd.items()}, mode=mode)
+    for T in lengths:
+        toks = synth.make_prompt(T, seed=T) % 1024
+        got = model(toks.view(1, -1).to(dev), 32, _pos(T, dev))[0].float().cpu()
+        model.reset_cache()
+        ref = om(toks.view(1, -1), 32, torch.arange(T))[0].float()
+        om.reset_cache()
+        check(got, ref, f"{fmt}, {T} tokens")
+
+
+@torch.no_grad()
 @pytest.mark.parametrize("T", [2, 4, 6, 7, 12, 31])
 def test_short_llm_int8_prompts_match_oracle(dev, T):
     """Up to where the row kernel takes a product (7B: 3 rows at K = 11008, 6 at 4096), one part of them tiled, all of them, up to the last length below 32: outlier columns over the whole prompt.
