@@ -326,11 +326,25 @@ int run_rows(RecParams p, hipStream_t s) {
     return rc;
 }
 
+// Prompt rows one behind the other (run_rows) or in chunks of 64 (recurrent_chunks.hip): up to 8 rows a sequence by rows; states of about 128 x 128, whose times are known, by an estimate.  By
+// rows: a sequence's rows in turn, 4.0 us each (delta rule; GLA 2.05), or where the CUs have several workgroups each 12.5 ns (6.5) per head and row.  Chunks: 85 us + 0.2 a head and chunk or 40 + 0.28 (55 + 0.13 or
+// 30 + 0.2), whatever number of their 64 rows there are.  Of 354 launches (16 to 40 heads, 1 to 64 sequences of 9 to 128 rows, alike or from few rows to all; 9 % off) rows are taken where they are 0.9 (0.8) times the
+// estimate of chunks, and none of those is slower: 32 heads, 32 sequences of 16 rows delta rule 300 -> 174 us, GLA 214 -> 117; 40 heads, 64 sequences of 1 to 40 rows 801 -> 592 and 557 -> 294
+bool rows_in_turn(const RecParams& p) {
+    if (p.b.max_count <= 8) return true;
+    const bool delta = p.a.kind == MI355_REC_DELTA;
+    if ((!delta && p.a.kind != MI355_REC_GLA) || p.a.dim < 96 || p.a.dim > 128 || p.a.vdim < 96 || p.a.vdim > 128 || p.b.max_count > 64) return false;
+    const float heads = (float)p.a.heads, chunks = heads * (float)p.b.seqs;
+    const float turn = (delta ? 4.0f : 2.05f) * (float)p.b.max_count, all = (delta ? 0.0125f : 0.0065f) * heads * (float)p.b.rows;
+    const float few = delta ? 85.f + 0.2f * chunks : 55.f + 0.13f * chunks, many = delta ? 40.f + 0.28f * chunks : 30.f + 0.2f * chunks;
+    return (turn > all ? turn : all) + (delta ? 15.f : 10.f) < (delta ? 0.9f : 0.8f) * (few > many ? few : many);
+}
+
 template <typename T>
 int run(const RecParams& p, hipStream_t s) {
     const bool fit = mi355_recurrent_chunks_fit(p.a, p.b);
     MI355_CHECK_ARG(p.a.path != 2 || fit, MI355_E_SHAPE, "recurrent: chunks take states of up to 256 x 256 and their scratch");
-    const bool chunks = p.a.path == 2 || (p.a.path == 0 && fit && p.b.max_count > 8);
+    const bool chunks = p.a.path == 2 || (p.a.path == 0 && fit && !rows_in_turn(p));
     if (chunks) {
         if (int rc = mi355_recurrent_chunks(p, s)) return rc;
     } else if (int rc = p.a.kind == MI355_REC_DELTA ? run_rows<T, MI355_REC_DELTA>(p, s)
