@@ -406,6 +406,14 @@ def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
+@pytest.mark.parametrize("epi", ["store", "pair", "accum"])
+@pytest.mark.parametrize("M", [2, 17, 64])
+@pytest.mark.parametrize("N,K", [(100, 1024), (1000, 1900), (2048, 2048), (2052, 2200)])
+def test_few_bf16_rows_in_slices_of_2_and_3_units(dev, N, K, M, epi):
+    """Slices no longer than the buffers that are filled ahead, some of 2 and some of 3 units, the last one not whole.  The bound of longer slices."""
+    test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi)
+
+
 @pytest.mark.parametrize("M", [49, 64, 65])
 @pytest.mark.parametrize("N,K", [(128, 640), (33024, 384), (70000, 128)])
 def test_blocks_of_64_tokens_read_once_or_by_several(dev, N, K, M):
