@@ -1876,10 +1876,10 @@ void q4_whole(int M, int N, int K, bool pair, GemmCut* cut) {
 // slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, each unit of one `unit` us, `unit_wave`
 // more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Slices go down to 2 units: the weights are read past
 // the caches, so a short product is a wait for memory that more blocks share out (N = K = 2048, 16 / 24 / 32 tokens 8.2 / 9.1 / 9.5 us whole in 32 blocks -> 6.8 / 7.4 / 7.7 in 8 slices;
-// N = 6816, K = 4224, 32 tokens 21.9 -> 16.6).  Up to 8 tokens, and up to 16 of longer rows, the sums of more slices gave none of it back (N = 4672, K = 3456, 2 tokens 10.6 us in 3 slices,
-// 11.3 in 7; N = 5120, K = 20736, 16 tokens 36.7 in 2 waves x 3, 37.4 in 4 x 6), nor do pairs, whose sums are twice as long (25 products at 24 to 64 tokens 0.99-1.00 on average, the worst
-// 1.13): there slices keep 4 units.  50 products of 1024 to 32000 rows, against slices of 4 units and one line up to 32 tokens: 16 / 24 / 32 / 40 / 48 / 64 tokens 0.989 / 0.983 / 0.978 /
-// 0.991 / 0.989 / 0.995 times the time on average, the best 0.77, 5 of 300 2 to 4 % slower (profiles/product_cuts_bf16_few.txt).
+// N = 6256, K = 3328, 32 tokens 17.3 -> 14.1).  That holds for 512 to 4095 columns.  Longer rows have units enough (N = 2048, K = 8448, 16 tokens 11.1 us in 6 slices, 11.7 in 8; N = 5120,
+// K = 20736 36.7 in 2 waves x 3, 37.4 in 4 x 6), up to 8 tokens (N = 4672, K = 3456, 2 tokens 10.6 us in 3 slices, 11.3 in 7) and in pairs, whose sums are twice as long (25 products at
+// 24 to 64 tokens 0.99-1.00 on average, the worst 1.13), more sums cost what they give: there slices keep 4 units.  35 products of 1024 to 6176 rows and 1024 to 3072 columns, 16 to 64
+// tokens: 0.96 times as long as in slices of 4 units, the least 0.71, the most 1.03 (profiles/product_cuts_bf16_few.txt).
 GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced) {
     struct Cost {
         float wave, unit, unit_wave, crowd, slices, bytes;
@@ -1888,7 +1888,7 @@ GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced) {
                                      {0.494f, 0.0935f, 0.0402f, 0.17f, 1.56f, 2.33e6f}, {0.607f, 0.045f, 0.0371f, 0.0182f, 0.861f, 4.79e6f},  // of 2: up to 16, up to 32,
                                      {0.256f, 0.207f, 0.025f, 0.0058f, 0.576f, 2.31e6f}};                                                     // up to 64
     const int units = (K + 127) / 128;
-    const bool shorter = !pair && (M > 16 || (M > 8 && units <= 32));
+    const bool shorter = !pair && M > 8 && units >= 4 && units < 32;
     const int least = shorter ? 2 : 4, line = (M > 32) + (shorter ? 2 + (M > 16) : 0);
     const Cost& c = costs[line];
     GemmCut cut = {4, short_block(M, true), true, 1};
