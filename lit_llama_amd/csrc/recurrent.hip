@@ -26,6 +26,7 @@ __global__ __launch_bounds__(THREADS, THREADS <= 512 ? 2 : 4) void rec_rows_kern
     const int head = blockIdx.x, seq = blockIdx.y;
     const int dim = a.dim, vdim = a.vdim, kvh = head / (a.heads / a.kv_heads);
     const int pos0 = p.b.pos[seq], cnt = p.b.count[seq], slot = p.b.slot[seq];
+    if (cnt <= 0) return;  // (a sequence without rows: its state is requested with the first row's inputs below, so there would be nothing to store)
     const int cols = p.slices * 64;
     float* q = (float*)smem;           // [parts * RMAX], zero past dim
     float* k = q + p.parts * RMAX;

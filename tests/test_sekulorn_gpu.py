@@ -258,6 +258,28 @@ def test_decode_steps_of_many_sequences_give_those_of_few(dev, kind, H, G, dim, 
     assert torch.equal(got[0][2], got[1][2])
 
 
+@pytest.mark.parametrize("counts", [[3, 0, 2], [0, 2, 1], [0, 20, 0, 9]])
+@pytest.mark.parametrize("kind,H,dim,vdim", [("delta", 4, 128, 128), ("delta", 2, 16, 144), ("delta", 1, 64, 1000), ("gla", 4, 128, 128)])
+def test_sequences_without_rows_keep_their_state(dev, kind, H, dim, vdim, counts):
+    """An empty portion between others: its slot's state and ring keep their bits, the other sequences give the bits that they give without it."""
+    from lit_llama_amd import ops
+
+    p, _, off, w = rec_case(kind, sum(counts), H, H, dim, vdim, torch.float32)
+    kw = {k: (tuple(t.to(dev) for t in v) if isinstance(v, tuple) else v.to(dev) if torch.is_tensor(v) else v) for k, v in w.items()}
+    gen = torch.Generator().manual_seed(5)
+    state0, ring0 = torch.randn((len(counts), H, dim, vdim), generator=gen).to(dev), torch.randn((len(counts), 4, 2 * H * dim + H * vdim), generator=gen).to(dev)
+    for path in (0, 1) + ((2,) if vdim <= 256 else ()):
+        got = []
+        for keep in (range(len(counts)), [i for i, n in enumerate(counts) if n]):
+            state, ring = state0.clone(), ring0.clone()
+            b = ops.PackedBatch([counts[i] for i in keep], list(keep), [7] * len(keep), dev)
+            got.append((ops.recurrent(kind, p.to(dev), b, state, off=off, kv_heads=H, conv_ring=ring, path=path, **kw), state, ring))
+        for a, b in zip(*got):
+            assert torch.isfinite(a).all() and torch.equal(a, b), path
+        for i in [i for i, n in enumerate(counts) if n == 0]:
+            assert torch.equal(got[0][1][i], state0[i]) and torch.equal(got[0][2][i], ring0[i]), path
+
+
 @pytest.mark.parametrize("kind,H,dim,vdim,counts,rows", [
     ("delta", 32, 128, 128, list(range(1, 25)), True), ("gla", 32, 128, 128, list(range(9, 33)), True), ("delta", 16, 100, 120, [16], True), ("gla", 8, 128, 96, [17, 3], True),
     ("delta", 16, 128, 128, [40], False), ("gla", 4, 64, 128, [12, 12], False), ("delta", 4, 128, 200, [9], False), ("gla", 32, 128, 128, [65] * 8, False),
