@@ -12,7 +12,7 @@
 // order.  For the decode step (T == 1) the kernel also applies RoPE to the new key, writes the new
 // K/V row into the cache and uses its LDS copy for the current position, so no other kernel (and no
 // global round trip) sits between the qkv projection and the attention output.
-#include "common.h"
+#include "attend.h"
 
 // flash_prefill.hip: declared in gemm_fuse.h
 #include "gemm_fuse.h"
@@ -512,8 +512,6 @@ __global__ __launch_bounds__(512) void attn_kernel(const AttnParams p) {
 #undef MI355_STAMP
 }
 
-// y[row, h*hs + d] = sum_j e^{m_j - M} o_j[d] / sum_j e^{m_j - M} l_j  over the n_split partial records
-
 // Several query tokens over a bf16 cache, queries in f32: a workgroup per (head, 16 tokens) on the matrix cores, its waves share out the keys in runs of 32.
 // attn_kernel reads all keys once per token, a workgroup each, and what it does per key on the VALU bounds it; here 16 tokens share a run, and queries and weights in f32 enter as three
 // bf16 each (limbs: products exact in f32, sums in f32).
@@ -522,22 +520,23 @@ __global__ __launch_bounds__(512) void attn_kernel(const AttnParams p) {
 //   scores  D[key][token] = keys x queries' limbs;  weights exp(score - maximum) per lane (its column's token, eight keys), split the same way
 //   values  D[dim][token] = values^T x weights: key 8 g + j of a product is the key whose weight lane group g holds (4 g + j of the run, j < 4, or 16 + 4 g + j - 4), its row i of product
 //           j is dimension VD i + j, so a lane's loads are VD dimensions of a row and eight keys' values are turned by v_perm
-// A key that some token does not see may hold an infinity or NaN in its value, which a weight of 0 does not undo: runs that hold one take token by token.
+// Infinities and NaN: a token whose sums are not finite (its own, or a value that others see, which a weight of 0 does not undo) is made again by attend_plain().
 constexpr int kTileTokens = 16, kTileRun = 32, kTileWaves = 4;
 template <int HS>
 __global__ __launch_bounds__(64 * kTileWaves, 2) void attn_tile_kernel(const AttnParams p) {
     constexpr int KS = HS / 32, VD = HS / 16;
     __shared__ __attribute__((aligned(16))) float red[kTileWaves][kTileTokens][HS];
     __shared__ float stat[2][kTileWaves][kTileTokens];
+    __shared__ unsigned not_finite[kTileWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
     const int h = blockIdx.x, t0 = blockIdx.y * kTileTokens, b = blockIdx.z;
     const int t = t0 + c < p.T ? t0 + c : p.T - 1;  // (columns past the last token: a copy of it, never stored)
     const int pos = p.pos ? p.pos[t] : t;
     const int len = (pos < p.S - 1 ? pos : p.S - 1) + 1;
-    int most = len, least = len;
+    int most = len;
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) most = max(most, __shfl_xor(most, o, 64)), least = min(least, __shfl_xor(least, o, 64));
-    most = __builtin_amdgcn_readfirstlane(most), least = __builtin_amdgcn_readfirstlane(least);
+    for (int o = 1; o < 16; o <<= 1) most = max(most, __shfl_xor(most, o, 64));
+    most = __builtin_amdgcn_readfirstlane(most);
     const bf16_t* kc = (const bf16_t*)p.kcache + ((int64_t)b * p.n_head + h) * p.S * HS;
     const bf16_t* vc = (const bf16_t*)p.vcache + ((int64_t)b * p.n_head + h) * p.S * HS;
     // limb 0, 1 or 2 of eight f32 as bf16: the upper 16 bits, of what is left the upper 16, and the rest
@@ -545,13 +544,11 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void attn_tile_kernel(const Att
         uint32_t r[3][8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float mid = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
-            r[0][i] = __float_as_uint(x[i]), r[1][i] = __float_as_uint(mid), r[2][i] = __float_as_uint(mid - __uint_as_float(__float_as_uint(mid) & 0xffff0000u));
+            const float mid = below_limb(x[i]);
+            r[0][i] = __float_as_uint(x[i]), r[1][i] = __float_as_uint(mid), r[2][i] = __float_as_uint(below_limb(mid));
         }
 #pragma unroll
-        for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) to[l][i] = __builtin_amdgcn_perm(r[l][2 * i + 1], r[l][2 * i], 0x07060302u);
+        for (int l = 0; l < 3; ++l) to[l] = upper_halves(r[l]);
     };
     u32x4 q[KS][3];
     {
@@ -620,54 +617,30 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void attn_tile_kernel(const Att
         }
         u32x4 w[3];
         limbs(e, w);
-        bool odd = false;
-        if (k0 + kTileRun > least) {
+        // (a run's products by themselves, the least first, then one rounding into the sum of the runs before)
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int e2 = 0; e2 < VD / 2; ++e2) odd |= (vf[i][e2] & 0x7F80u) == 0x7F80u || (vf[i][e2] & 0x7F800000u) == 0x7F800000u;
-        }
-        // product j of the values of the keys below `end`
-        auto value = [&](int j, int end) __attribute__((always_inline)) {
+        for (int j = 0; j < VD; ++j) {
             u32x4 v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t lo = value_key(2 * i) < end ? vf[2 * i][j >> 1] : 0u, hi = value_key(2 * i + 1) < end ? vf[2 * i + 1][j >> 1] : 0u;
-                v[i] = __builtin_amdgcn_perm(hi, lo, j & 1 ? 0x07060302u : 0x05040100u);
-            }
-            return __builtin_bit_cast(bf16x8, v);
-        };
-        // (a run's products by themselves, the least first, then one rounding into the sum of the runs before)
-        auto weighted = [&](const bf16x8& v) __attribute__((always_inline)) {
+            for (int i = 0; i < 4; ++i) v[i] = __builtin_amdgcn_perm(vf[2 * i + 1][j >> 1], vf[2 * i][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
             f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int limb = 2; limb >= 0; --limb) sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, __builtin_bit_cast(bf16x8, w[limb]), sum, 0, 0, 0);
-            return sum;
-        };
-        if (__builtin_amdgcn_ballot_w64(odd) == 0) {
+            for (int limb = 2; limb >= 0; --limb) sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), __builtin_bit_cast(bf16x8, w[limb]), sum, 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < VD; ++j) {
-                const f32x4 sum = weighted(value(j, 0x7fffffff));
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[j][r] = __builtin_fmaf(acc[j][r], corr, sum[r]);
-            }
-        } else {
-#pragma unroll 1
-            for (int of = 0; of < kTileTokens; ++of) {
-                const int end = __builtin_amdgcn_readlane(len, of);
-#pragma unroll
-                for (int j = 0; j < VD; ++j) {
-                    const f32x4 sum = weighted(value(j, end));
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][r] = c == of ? __builtin_fmaf(acc[j][r], corr, sum[r]) : acc[j][r];
-                }
-            }
+            for (int r = 0; r < 4; ++r) acc[j][r] = __builtin_fmaf(acc[j][r], corr, sum[r]);
         }
     }
     // ---- the waves join: lane (g, c) holds dimensions VD (4 g + r) + j of token c
     l += lane_xor16(l);
     l += lane_xor32(l);
     if (g == 0) stat[0][wave][c] = m, stat[1][wave][c] = l;
+    float none = 0.f * l;  // 0, or NaN
+#pragma unroll
+    for (int j = 0; j < VD; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) none = __builtin_fmaf(0.f, acc[j][r], none);
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(!(none == 0.f));
+    if (lane == 0) not_finite[wave] = (unsigned)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -687,8 +660,28 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void attn_tile_kernel(const Att
         }
         st_from_f32(p.y, ((int64_t)b * p.T + t0 + of) * p.ldy + h * HS + d, p.y_dtype, o / sum);
     }
+    unsigned again = 0;
+#pragma unroll
+    for (int w = 0; w < kTileWaves; ++w) again |= not_finite[w];
+    for (again = __builtin_amdgcn_readfirstlane(again); again != 0; again &= again - 1) {
+        const int of = __builtin_ctz(again), token = t0 + of;
+        if (token >= p.T) break;
+        float* const row = &red[0][0][0];
+        const int at = p.pos ? p.pos[token] : token, keys = (at < p.S - 1 ? at : p.S - 1) + 1;
+        __syncthreads();
+        if (tid < HS / 2) {
+            const float* src = (const float*)p.qkv + ((int64_t)b * p.T + token) * p.ld_qkv + h * HS + 2 * tid;
+            rope_pair(p.rope, p.rope_gathered ? token : at, HS / 2, tid, src[0], src[1], row[2 * tid], row[2 * tid + 1]);
+        }
+        __syncthreads();
+        float top, sum, o;
+        attend_plain<64 * kTileWaves>(0, keys, HS, row + HS, [&](int k) { return dot_row(row, kc + (int64_t)k * HS, HS) * p.scale; }, [&](int k, int d) { return bf16_to_f32(vc[(int64_t)k * HS + d]); }, top,
+                                      sum, o);
+        if (tid < HS) st_from_f32(p.y, ((int64_t)b * p.T + token) * p.ldy + h * HS + tid, p.y_dtype, o / sum);
+    }
 }
 
+// y[row, h*hs + d] = sum_j e^{m_j - M} o_j[d] / sum_j e^{m_j - M} l_j  over the n_split partial records
 __global__ void attn_combine_kernel(const float* part, int n_split, int n_head, int hs, void* y, int y_dtype,
                                     int64_t ldy) {
     const int r = blockIdx.y, h = blockIdx.x;

@@ -496,20 +496,28 @@ def test_split_attention_equals_single_workgroup_and_feeds_the_projection(dev, n
     (4, 64, 65, 0, 80, 1, torch.float32), (5, 64, 129, 7, 200, 1, torch.float32), (2, 64, 700, 0, 700, 1, torch.float32), (3, 64, 100, 30, 97, 1, torch.float32),
     (4, 64, 48, 0, 48, 3, torch.float32), (6, 128, 33, 5, 60, 2, torch.float32),
 ])
-@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("odd", ["", "value", "values", "key"])
 def test_attention_of_tokens_that_share_their_keys(dev, H, hs, T, first, S, B, out, odd):
-    """More (head, token) pairs than CUs, f32 queries over a bf16 cache, against 64 bits: positions in any order, past the cache's end (the last row), several batch rows, and an infinite value in the
-    last row, which only those that see it may take over.  f32 sums of up to 2048 terms and exponentials of |score| < 20: 1e-6 of the result; bf16 results 2^-8."""
+    """More (head, token) pairs than CUs, f32 queries over a bf16 cache, against 64 bits: positions in any order, past the cache's end (the last row), several batch rows; an infinite value in the
+    last row, which only those that see it take over; infinite values that all see, of one sign in a dimension and of both in another; an infinite key, whose weight is 0 or NaN.  f32 sums of up to
+    2048 terms and exponentials of |score| < 20: 1e-6 of the result; bf16 results 2^-8.  Infinities and NaN are where 64 bits have them."""
+    if odd in ("values", "key") and first == 0:
+        pytest.skip("no rows of earlier calls")
     g = torch.Generator().manual_seed(T)
     qkv = torch.randn((B, T, 3 * H * hs), generator=g)
     rope = oracle.build_rope_cache(1024, hs, dtype=torch.int64)
     cs = rope.double()
     pos = first + torch.randperm(T, generator=g)
     last = pos.clamp(max=S - 1)
-    if odd:  # the value of one token whose row most of the others do not see
+    if odd == "value":  # the value of one token whose row most of the others do not see
         t_odd = int(pos.argmax())
         qkv[:, t_odd, 2 * H * hs + 3] = float("inf")
     cache = torch.randn((B, H, S, hs), generator=g).bfloat16().to(dev), torch.randn((B, H, S, hs), generator=g).bfloat16().to(dev)
+    if odd == "values":
+        cache[1][:, 1, 0, 5] = cache[1][:, 1, 2, 9] = float("inf")
+        cache[1][:, 1, 1, 9] = cache[1][:, 1, 3, 2] = -float("inf")
+    if odd == "key":
+        cache[0][:, 1, 2, 7] = float("inf")
 
     def turn(x):  # [B, T, H, hs]
         x = x.double().view(B, T, H, hs // 2, 2)
@@ -526,7 +534,9 @@ def test_attention_of_tokens_that_share_their_keys(dev, H, hs, T, first, S, B, o
     ref = torch.stack([w[..., i, : int(last[i]) + 1][..., None, :] @ vc[..., : int(last[i]) + 1, :] for i in range(T)], 2)[..., 0, :]  # (an infinity times a weight of 0 is none of it)
     ref = ref.transpose(1, 2).reshape(B, T, H * hs)
     assert clash or torch.equal(cache[1][:, :, last].float().cpu(), v.bfloat16().float().transpose(1, 2))
-    assert torch.equal(torch.isfinite(y), torch.isfinite(ref)) and (odd or bool(torch.isfinite(y).all()))
+    for kind in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(kind(y), kind(ref)), kind
+    assert bool(torch.isfinite(ref).all()) == (odd == "" or (odd == "value" and not bool(torch.isinf(vc).any())))
     y, ref = y.nan_to_num(0, 0, 0), ref.nan_to_num(0, 0, 0)
     assert (y - ref).norm() <= (1e-6 if out == torch.float32 else 2.0 ** -8) * ref.norm()
 
