@@ -14,7 +14,7 @@
 //                         the rows of earlier portions from it) and, of a lender, behind its last borrower
 //
 // Scores, softmax and weighted values are f32 (the tiles multiply bf16 operands into f32 accumulators).
-#include "common.h"
+#include "attend.h"
 
 namespace {
 
@@ -416,11 +416,10 @@ __device__ __forceinline__ u32x4 limbs_of(const float (&x)[8], int limb) {
     uint32_t t[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const float r = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u), s = r - __uint_as_float(__float_as_uint(r) & 0xffff0000u);
-        t[i] = __float_as_uint(limb == 0 ? x[i] : limb == 1 ? r : s);
+        const float r = below_limb(x[i]);
+        t[i] = __float_as_uint(limb == 0 ? x[i] : limb == 1 ? r : below_limb(r));
     }
-    return u32x4{__builtin_amdgcn_perm(t[1], t[0], 0x07060302u), __builtin_amdgcn_perm(t[3], t[2], 0x07060302u), __builtin_amdgcn_perm(t[5], t[4], 0x07060302u),
-                 __builtin_amdgcn_perm(t[7], t[6], 0x07060302u)};
+    return upper_halves(t);
 }
 // Sum over the limbs: columns c, c + 4, c + 8 and c + 12 of a row of 16 lanes.  All four get the same bits, (c + c8) + (c4 + c12) or the other way round: they split what follows from it,
 // and a weight whose limbs came from two roundings would lose all but its first eight bits now and then
@@ -434,6 +433,7 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
     constexpr int kDim = 32 * KS;
     const mi355_window_attn_args& a = p.a;
     __shared__ __attribute__((aligned(16))) float q[kKeyHeads * kDim], kn[kDim], vn[VB * 128], stat[2][kKeyWaves][kKeyHeads];
+    __shared__ int not_finite[kKeyWaves];
     extern __shared__ __attribute__((aligned(16))) char smem[];
     u32x4* qs = (u32x4*)smem;             // [KS][lane] the queries' limbs, then the row's own key and value
     u32x4 *ks = qs + KS * 64, *vs = ks + kDim / 8;
@@ -571,6 +571,15 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
     l += lane_xor16(l);
     l += lane_xor32(l);
     if (g == 0 && limb == 0) stat[0][wave][head] = m, stat[1][wave][head] = l;
+    float none = 0.f * l;  // 0, or NaN
+#pragma unroll
+    for (int b = 0; b < VB; ++b)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) none = __builtin_fmaf(0.f, acc[b][j][r], none);
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(!(none == 0.f));
+    if (lane == 0) not_finite[wave] = bad != 0;
 #pragma unroll
     for (int b = 0; b < VB; ++b) {
         float o[8];
@@ -586,6 +595,31 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
         *(f32x4*)(dst + 4) = f32x4{o[4], o[5], o[6], o[7]};
     }
     __syncthreads();
+    int again = 0;
+#pragma unroll
+    for (int w = 0; w < kKeyWaves; ++w) again |= not_finite[w];
+    if (__builtin_amdgcn_readfirstlane(again) != 0) {  // (the queries' limbs make room)
+        const bf16_t* own_v = prow + a.off_v + (int64_t)kvh * vdim;
+#pragma unroll 1
+        for (int h = 0; h < nh; ++h) {
+            const float bias = a.slope != nullptr ? a.slope[h0 + h] : 0.f, *qh = q + h * kDim;
+            auto score = [&](int k) {
+                float s = 0.f;
+                if (k == own)
+                    for (int d = 0; d < kDim; ++d) s += qh[d] * kn[d];
+                else
+                    s = dot_row(qh, kcache + row_of(k) * (unsigned)kDim, kDim);
+                return cap_score(s, a.softcap) - bias * (float)(pos - (k < n_first ? k : k + w_shift));
+            };
+            auto value = [&](int k, int d) { return k != own ? bf16_to_f32(vcache[row_of(k) * (unsigned)vdim + d]) : made_v ? vn[d] : bf16_to_f32(own_v[d]); };
+            float top, sum, o;
+            attend_plain<kKeyThreads>(k_begin, k_end, vdim, (float*)qs, score, value, top, sum, o);
+            if (tid < kKeyWaves) stat[0][tid][h] = tid == 0 ? top : -INFINITY, stat[1][tid][h] = tid == 0 ? sum : 0.f;
+            if (tid < vdim)
+                for (int w = 0; w < kKeyWaves; ++w) red[(w * kKeyHeads + h) * (128 * VB) + tid] = w == 0 ? o : 0.f;
+        }
+        __syncthreads();
+    }
     for (int i = tid; i < nh * 128 * VB; i += kKeyThreads) {
         const int h = i / (128 * VB), d = i - h * (128 * VB);
         const bool sink = a.sink != nullptr && split == 0;  // (a key without a value)
@@ -595,7 +629,7 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
         float sum = sink ? expf(a.sink[h0 + h] - top) : 0.f, o = 0.f;
 #pragma unroll
         for (int w = 0; w < kKeyWaves; ++w) {
-            const float f = expf(stat[0][w][h] - top);
+            const float f = stat[0][w][h] == -INFINITY ? 0.f : expf(stat[0][w][h] - top);  // (no key with a weight)
             sum += f * stat[1][w][h];
             o += f * red[(w * kKeyHeads + h) * (128 * VB) + d];
         }

@@ -106,7 +106,7 @@ DECODE_FORMS = [  # heads, key heads, dim, vdim, window, ring, options
 
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("H,G,dim,vdim,window,ring,o", DECODE_FORMS)
-def test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, window, ring, o, split):
+def test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, window, ring, o, split, odd=False):
     """window_keys_kernel takes what window_rows_kernel takes (path 1), wherever a run of keys ends: first positions, the ring's wrap, the row's own key.  Both sum f32 products in f32
     (1e-4 of a head's size covers the order of up to 2000 terms), so what differs is a rounding of the result now and then: a step of bf16's 8 bits, 2^-7 of it at most.  The cache rows are the same bits."""
     from lit_llama_amd import ops
@@ -118,6 +118,11 @@ def test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, wind
     off = [0, H * dim, (H + G) * dim, (H + G) * dim + G * vdim]
     proj = rnd(B, off[3] + H * vdim).bfloat16()
     rings = rnd(B, G, kept + ring, dim).bfloat16(), rnd(B, G, kept + ring, vdim).bfloat16()
+    if odd:  # of the last key head: an infinite value, one of each sign in one dimension, infinite keys; an infinite value of a row's own
+        for b in range(0, B, 2):
+            rings[1][b, -1, 0, 1], rings[1][b, -1, ring // 2, 5], rings[1][b, -1, ring // 3, 5] = float("inf"), float("inf"), -float("inf")
+        rings[0][2::3, -1, ring // 4, 3] = float("inf")
+        proj[1::4, off[3] - vdim + 2] = -float("inf")
     rot = o.get("rot", 0)
     kw = dict(heads=H, scale=1.5 * dim ** -0.5, window=window, off_q=off[0], off_k=off[1], off_v=off[2], off_g=off[3] if "gate" in o else -1, gate_values=o.get("gate") == "values",
               keep=keep, kept=kept, softcap=o.get("softcap", 0.0), chunked=o.get("chunked", False), inv_freq=5000.0 ** (-torch.arange(rot // 2, device=dev).double() * 2 / rot) if rot else None,
@@ -138,11 +143,21 @@ def test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, wind
         kr, vr = rings[0].clone(), rings[1].clone()
         got.append((ops.window_attention(proj, b, kr, vr, path=path, **kw).double(), kr, vr))
     (y, kr, vr), (ref, kr1, vr1) = got
-    assert torch.isfinite(ref).all() and ref.abs().max() > 0.1
+    for kind in (torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(kind(y), kind(ref)), kind
+    assert torch.isfinite(ref).all() != odd and ref.nan_to_num(0, 0, 0).abs().max() > 0.1
+    y, ref = y.nan_to_num(0, 0, 0), ref.nan_to_num(0, 0, 0)
     size = ref.view(B, H, vdim).square().mean(-1, keepdim=True).sqrt().expand(B, H, vdim).reshape(ref.shape)
     bad = (y - ref).abs() > 2.0 ** -7 * ref.abs() + 1e-4 * size
     assert not bad.any()
-    assert torch.equal(kr, kr1) and torch.equal(vr, vr1)
+    assert torch.equal(kr.view(torch.int16), kr1.view(torch.int16)) and torch.equal(vr.view(torch.int16), vr1.view(torch.int16))
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("H,G,dim,vdim,window,ring,o", [f for f in DECODE_FORMS if f[4] > 32 and not {"unit", "rot", "v_first", "borrows"} & set(f[6])] + [(16, 2, 128, 64, 400, 450, {})])
+def test_infinite_keys_and_values_of_decode_rows(dev, H, G, dim, vdim, window, ring, o, split):
+    """Three bf16 to a weight, one of them 0 as a rule: infinities stay infinities, a key whose score is -inf has no weight, and what is NaN over rows is NaN here."""
+    test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, window, ring, o, split, odd=True)
 
 
 def test_far_positions_keep_their_angle(dev):
