@@ -541,6 +541,28 @@ def test_attention_of_tokens_that_share_their_keys(dev, H, hs, T, first, S, B, o
     assert (y - ref).norm() <= (1e-6 if out == torch.float32 else 2.0 ** -8) * ref.norm()
 
 
+@pytest.mark.parametrize("sharp", [1.0, 4.0])
+@pytest.mark.parametrize("H,hs,T,first", [(32, 128, 24, 0), (32, 128, 31, 1900), (8, 128, 600, 0), (4, 64, 512, 0), (32, 64, 20, 500)])
+def test_shared_keys_cost_no_precision(dev, H, hs, T, first, sharp):
+    """The error of f32 results against 64 bits, four inputs together, is no larger than that of the workgroup per token (which n_split = 2 takes)."""
+    rope = oracle.build_rope_cache(first + T, hs, dtype=torch.int64).to(dev)
+    pos = first + torch.arange(T, device=dev)
+    turn = torch.view_as_complex(rope.double().view(-1, hs // 2, 2))[pos][:, None]
+    errors = [0.0, 0.0]
+    for seed in range(4):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        qkv = torch.randn((1, T, 3 * H * hs), generator=g, device=dev)
+        qkv[..., : H * hs] *= sharp
+        cache = [torch.randn((1, H, first + T, hs), generator=g, device=dev).bfloat16() for _ in range(2)]
+        got = [ops.attention(qkv, rope, H, pos=pos, kv_cache=tuple(cache), out_dtype=torch.float32, n_split=n).double() for n in (1, 2)]
+        q = torch.view_as_real(torch.view_as_complex(qkv[0, :, : H * hs].double().view(T, H, hs // 2, 2)) * turn).view(T, H, hs).transpose(0, 1)
+        score = (q @ cache[0][0].double().transpose(-1, -2).contiguous() * hs ** -0.5).masked_fill(torch.arange(first + T, device=dev) > pos[:, None], float("-inf"))
+        ref = (torch.softmax(score, -1) @ cache[1][0].double()).transpose(0, 1).reshape(1, T, H * hs)
+        for i, y in enumerate(got):
+            errors[i] += float((y - ref).square().sum() / ref.square().sum())
+    assert errors[0] <= errors[1]
+
+
 def test_attention_without_cache_batched(dev):
     B, T, n_head, hs = 3, 9, 4, 8
     C = n_head * hs
