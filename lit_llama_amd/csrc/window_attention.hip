@@ -400,18 +400,22 @@ __global__ __launch_bounds__(kRowThreads, HT <= 4 ? 4 : 2) void window_rows_kern
 // multiplied from the registers that they land in, without a barrier until the waves join.  (window_rows_kernel multiplies in f32 on the VALU, a pass of 64 keys, a softmax and
 // a pass of values one behind the other: 16 sequences of 96 to 1536 keys, 32 / 8 heads of 128, with the join 40 -> 23.5 us; 53 MB of cache are 9.)
 //   scores   D[key][column] = keys x queries: a query in f32 is three bf16 (limbs_of()), each a column: 4 heads x 3 of the 16 columns.  Products of bf16 are exact
-//            in f32, so the sum is that of f32 products
+//            in f32, so the sum is that of f32 products; 32 dimensions at a time, summed in pairs (dot_tree())
 //   weights  exp(score - maximum) in f32 per lane (its column's head, eight keys), split the same way
 //   values   D[dim][column] = values^T x weights.  The product's key number 8 g + j of lane group g is the key whose weight the group holds: key 4 g + j of the run
 //            (j < 4) or 16 + 4 g + j - 4; its row number i of product j is dimension 8 i + j, so a lane's loads are 16 B of a row and eight keys' values are turned by v_perm
-// Registers: three workgroups to a CU (two of 8 waves, the next run requested ahead: 26 us).  Error of the f32 sums against 64 bits 2.3e-7 to 6e-7 of a row (window_rows_kernel 1.5e-7 to
-// 4e-7), of the rows that leave, rounded to bf16, 1.7e-3 from both, equal to 1e-8.
+// Registers: three workgroups to a CU (two of 8 waves, the next run requested ahead: 26 us).
+// Error of the f32 sums against 64 bits, times window_rows_kernel's (18 forms of 64 to 256 dimensions x 5 lengths of 130 to 6000 keys, 16 to 32 rows each): scores of spread 0.3 0.58-0.70, 1 0.77-0.93 (1.0e-7
+// to 1.9e-7 of a row), 4 0.97-1.09.  (With a score's dimensions in one chain of products, limbs c + c8 first: 0.63-0.79, 0.85-1.45, 1.06-2.03.)
+// 587 launches against window_rows_kernel, caches from HBM (values and keys of 64 to 256, 1 to 64 sequences of 96 to 2048 keys): 1 query head to a key head 0.81 times as long, 2 0.64, 4 0.67, 5 and more,
+// which two or more workgroups read, 0.50; the most 0.99 (32 heads of 256 x 128, 16 sequences).  Caches that stay in the 256-MB cache likewise, but for a few hundred keys of a sequence or two without shared key heads: 1.04.
 constexpr int kKeyHeads = 4, kRun = 32;
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr int kKeyWaves = 4, kKeyThreads = 64 * kKeyWaves;
 constexpr int key_occupancy(int ks, int vb) { return vb == 1 && ks <= 4 ? 3 : 2; }  // waves per SIMD
 
-// Limb 0, 1 or 2 of eight f32 as bf16: the upper 16 bits, of what is left the upper 16, and the rest (3: any)
+// Limb 0, 1 or 3 of eight f32 as bf16: the upper 16 bits, of what is left the upper 16, and the rest (kNoLimb: any)
+constexpr int kNoLimb = 2;
 __device__ __forceinline__ u32x4 limbs_of(const float (&x)[8], int limb) {
     uint32_t t[8];
 #pragma unroll
@@ -422,10 +426,22 @@ __device__ __forceinline__ u32x4 limbs_of(const float (&x)[8], int limb) {
     return upper_halves(t);
 }
 // Sum over the limbs: columns c, c + 4, c + 8 and c + 12 of a row of 16 lanes.  All four get the same bits, (c + c8) + (c4 + c12) or the other way round: they split what follows from it,
-// and a weight whose limbs came from two roundings would lose all but its first eight bits now and then
+// and a weight whose limbs came from two roundings would lose all but its first eight bits now and then.  (c8 is kNoLimb's, 0: the two small limbs, c4 and c12, meet first)
 __device__ __forceinline__ float sum_limbs(float v) {
     v = MI355_DPP_ADD(v, 0x128);     // row_ror:8
     return MI355_DPP_ADD(v, 0x124);  // row_ror:4
+}
+
+// Products of 32 N dimensions from 32 S0 on, summed in pairs: one chain of them rounds the whole sum N times.  FEW: a pair at a time (as many registers as there are go to what is in flight)
+template <int S0, int N, bool FEW, int KS>
+__device__ __forceinline__ f32x4 dot_tree(const u32x4 (&k)[KS], const u32x4* q) {
+    if constexpr (N == 1) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[S0]), __builtin_bit_cast(bf16x8, q[S0 * 64]), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    } else {
+        const f32x4 a = dot_tree<S0, N / 2, FEW>(k, q), b = dot_tree<S0 + N / 2, N / 2, FEW>(k, q), sum = a + b;
+        if constexpr (FEW && N == 2) __builtin_amdgcn_sched_barrier(0);
+        return sum;
+    }
 }
 
 template <int KS, int VB>
@@ -473,7 +489,7 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (at < 0)
-                x[e] = h < nh && col < 12 ? q[h * kDim + 32 * (i >> 6) + 8 * ((i >> 4) & 3) + e] : 0.f;
+                x[e] = h < nh && col >> 2 != kNoLimb ? q[h * kDim + 32 * (i >> 6) + 8 * ((i >> 4) & 3) + e] : 0.f;
             else if (at < kDim / 8)
                 x[e] = kn[d0 + e];
             else
@@ -522,13 +538,9 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
                 }
         }
         float e[8], top = -INFINITY;
-        f32x4 d2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        f32x4 d2[2];
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const bf16x8 b = __builtin_bit_cast(bf16x8, qs[s * 64 + lane]);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) d2[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[t][s]), b, d2[t], 0, 0, 0);
-        }
+        for (int t = 0; t < 2; ++t) d2[t] = dot_tree<0, KS, KS == 8 && VB == 2>(kf[t], qs + lane);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -553,7 +565,7 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
         const float base = m == -INFINITY ? 0.f : m;  // (no key with a weight so far)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            e[i] = __builtin_amdgcn_exp2f((e[i] - base) * kLog2e);  // (what the factor's rounding costs is the less the more a key weighs)
+            e[i] = __builtin_amdgcn_exp2f((e[i] - base) * kLog2e);  // (what the factor's rounding costs is the less the more a key weighs: expf() takes 1 % off the error)
             l += e[i];
         }
         const bf16x8 w = __builtin_bit_cast(bf16x8, limbs_of(e, limb));
@@ -587,7 +599,7 @@ __global__ __launch_bounds__(kKeyThreads, key_occupancy(KS, VB)) void window_key
         for (int j = 0; j < 8; ++j) {
             f32x4 s = acc[b][j];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s[r] = sum_limbs(limb < 3 ? s[r] : 0.f);
+            for (int r = 0; r < 4; ++r) s[r] = sum_limbs(limb != kNoLimb ? s[r] : 0.f);
             o[j] = limb == 0 ? s[0] : limb == 1 ? s[1] : limb == 2 ? s[2] : s[3];
         }
         float* dst = red + (wave * kKeyHeads + head) * (128 * VB) + 128 * b + 32 * g + 8 * limb;

@@ -160,6 +160,31 @@ def test_infinite_keys_and_values_of_decode_rows(dev, H, G, dim, vdim, window, r
     test_decode_rows_on_the_matrix_cores_against_rows(dev, H, G, dim, vdim, window, ring, o, split, odd=True)
 
 
+@pytest.mark.parametrize("H,G,dim,vdim", [(32, 8, 128, 128), (8, 8, 64, 64), (16, 4, 256, 256), (32, 2, 64, 128), (4, 4, 128, 256), (8, 2, 256, 128)])
+def test_decode_rows_on_the_matrix_cores_cost_no_precision(dev, H, G, dim, vdim):
+    """The f32 sums of the splits, joined in 64 bits: their error is no larger than window_rows_kernel's (path 1), three lengths and inputs together."""
+    from lit_llama_amd import ops
+
+    errors = [0.0, 0.0]
+    for seed, (B, keys) in enumerate([(4, 1900), (8, 512), (8, 200)]):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        rnd = lambda *s: torch.randn(s, generator=g, device=dev).bfloat16()  # noqa: E731
+        off = [0, H * dim, (H + G) * dim, (H + G) * dim + G * vdim]
+        proj, kr, vr = rnd(B, off[3]), rnd(B, G, keys, dim), rnd(B, G, keys, vdim)
+        b = ops.PackedBatch([1] * B, list(range(B)), [keys - 1] * B, dev)
+        for path in (0, 1):
+            part = torch.full((1 << 21,), float("nan"), device=dev)
+            ops.window_attention(proj, b, kr, vr, heads=H, scale=dim ** -0.5, window=keys, off_q=off[0], off_k=off[1], off_v=off[2], path=path, partials=part)
+            rec = part[~part.isnan()].view(B, H, -1, vdim + 2).double()
+            assert rec.shape[2] > 1
+            w = torch.exp(rec[..., 0] - rec[..., 0].amax(-1, keepdim=True))
+            y = (rec[..., 2:] * w[..., None]).sum(2) / (rec[..., 1] * w).sum(-1, keepdim=True)
+            score = (proj[:, : H * dim].float() * dim ** -0.5).double().view(B, G, H // G, dim) @ kr.double().transpose(-1, -2).contiguous()
+            ref = (torch.softmax(score, -1) @ vr.double()).view(B, H, vdim)
+            errors[path] += float((y - ref).square().sum() / ref.square().sum())
+    assert errors[0] <= errors[1]
+
+
 def test_far_positions_keep_their_angle(dev):
     """Two rows a million positions in: rotation depends on the distance only."""
     from lit_llama_amd import ops
