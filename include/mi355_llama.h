@@ -36,8 +36,9 @@ enum { MI355_W_Q4 = 0, MI355_W_BF16 = 1, MI355_W_I8 = 2 };
 /* epilogues of the fast linear */
 /* (GEGLU: the pair stream with the tanh form of GELU instead of SiLU; BF16 streams only) */
 enum { MI355_EPI_STORE = 0, MI355_EPI_ACCUM = 1, MI355_EPI_SWIGLU = 2, MI355_EPI_GEGLU = 3, MI355_EPI_CLAMPGLU = 4 };
-/* bits of mi355_linear_args.flags: STORE writes max(y, 0)^2; the norm's scale is 1 + norm_scale */
-enum { MI355_LF_RELU2 = 1, MI355_LF_NORM_ONE = 2 };
+/* bits of mi355_linear_args.flags: STORE writes max(y, 0)^2; the norm's scale is 1 + norm_scale; the weights come from HBM at every use, more than the 256-MB cache
+ * holds being read between two (mi355_linear_gemm of few rows reads them past the caches and may cut a product otherwise; any value is right) */
+enum { MI355_LF_RELU2 = 1, MI355_LF_NORM_ONE = 2, MI355_LF_STREAMED = 4 };
 
 typedef void* mi355_stream_t; /* hipStream_t */
 
@@ -386,7 +387,7 @@ typedef struct mi355_weight {
     int32_t waves;
     int32_t grid;
     int32_t prefetch;
-    int32_t flags;      /* as mi355_linear_args.flags */
+    int32_t flags;      /* as mi355_linear_args.flags (of prompts' tiled products MI355_LF_STREAMED alone) */
     int32_t group_cols; /* Q4: as mi355_linear_args.group_cols (0: one scale / zero per output row) */
 } mi355_weight;
 
@@ -839,7 +840,7 @@ typedef struct mi355_latent_args {
     void* gemm_ws;
     uint64_t gemm_ws_bytes;
     int32_t path;          /* 0: by shape; 1: one workgroup per row and head; 2: matrix cores on the latents; 3: expanded tiles */
-    int32_t reserved0;
+    int32_t linear_flags;  /* of the products: MI355_LF_STREAMED, or 0 */
 } mi355_latent_args;
 
 int mi355_latent_attention(const mi355_latent_args* a, const mi355_seq_batch* b, mi355_stream_t stream);
@@ -988,6 +989,8 @@ typedef struct mi355_hybrid_model {
     int64_t ld_side;
     float* mixed;          /* [max_rows, ld_mixed]: SSD outputs in front of their norm */
     int64_t ld_mixed;
+    int32_t linear_flags;  /* of every product: MI355_LF_STREAMED, or 0 */
+    int32_t reserved0;
 } mi355_hybrid_model;
 
 /* embedding, every layer run, and the logits (f32 [n_want, ld_logits]) of the rows want[0 .. n_want) (device; NULL: all rows).

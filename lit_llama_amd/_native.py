@@ -19,7 +19,7 @@ CORE_LIB_PATH = _PKG / "libmi355core.so"  # the part a layered hybrid model need
 F32, BF16, F16 = 0, 1, 2
 W_Q4, W_BF16, W_I8 = 0, 1, 2
 EPI_STORE, EPI_ACCUM, EPI_SWIGLU, EPI_GEGLU, EPI_CLAMPGLU = 0, 1, 2, 3, 4
-LF_RELU2, LF_NORM_ONE = 1, 2
+LF_RELU2, LF_NORM_ONE, LF_STREAMED = 1, 2, 4
 
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
@@ -28,6 +28,12 @@ c_void_p, c_int, c_int32, c_int64, c_float, c_size_t = C.c_void_p, C.c_int, C.c_
 
 class NativeError(RuntimeError):
     pass
+
+
+def streamed(weight_bytes: int) -> int:
+    """LF_STREAMED for a model whose products read this many bytes of weights in a pass, or 0: up to 300 MB stay in the 256-MB cache from one pass to the next, mostly (products of few
+    rows that read their weights past the caches take 1.02 times as long at 288 MB, 0.97 at 320)."""
+    return LF_STREAMED if weight_bytes > 300_000_000 else 0
 
 
 class LinearArgs(C.Structure):
@@ -210,7 +216,7 @@ class LatentArgs(C.Structure):
         ("uq", Proj), ("expand", Proj), ("uk_t", c_void_p), ("uv", c_void_p), ("cache", c_void_p), ("y", c_void_p), ("ldy", c_int64),
         ("cq", c_void_p), ("q", c_void_p), ("qa", c_void_p), ("partials", c_void_p), ("partials_bytes", C.c_uint64),
         ("rows_c", c_void_p), ("kv_rows", c_void_p), ("expand_rows", c_int64), ("gemm_ws", c_void_p), ("gemm_ws_bytes", C.c_uint64),
-        ("path", c_int32), ("reserved0", c_int32),
+        ("path", c_int32), ("linear_flags", c_int32),
     ]
 
 
@@ -246,6 +252,7 @@ class HybridModel(C.Structure):
         ("partials", c_void_p), ("partials_bytes", C.c_uint64), ("rec_scratch", c_void_p), ("rec_scratch_bytes", C.c_uint64),
         ("moe_scratch", c_void_p), ("moe_scratch_bytes", C.c_uint64),
         ("embed_norm", c_void_p), ("stream", c_void_p), ("side", c_void_p), ("ld_side", c_int64), ("mixed", c_void_p), ("ld_mixed", c_int64),
+        ("linear_flags", c_int32), ("reserved0", c_int32),
     ]
 
 

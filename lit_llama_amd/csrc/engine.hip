@@ -115,6 +115,7 @@ void fill_linear_args(mi355_linear_args& a, const mi355_model* m, const mi355_we
     memset(&a, 0, sizeof(a));
     a.fmt = w.fmt;
     a.R = w.R;
+    a.flags = w.flags & MI355_LF_STREAMED;
     a.w = w.w;
     a.N = w.N;
     a.K = w.K;

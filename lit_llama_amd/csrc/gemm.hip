@@ -95,6 +95,7 @@ struct GemmParams {
     const float* bias;     // STORE: [N], or NULL
     mi355_reduce_norm rn;  // rn.done: the sum of the K-slices also leaves the rows' norm
     bool squares;          // BF16 blocks that may_run_in_squares(): an XCD's blocks are kSquare row blocks by some token blocks (square_blocks())
+    bool streamed;         // MI355_LF_STREAMED
     int slice_blocks;      // != 0: row blocks [i slice_blocks, (i + 1) slice_blocks) read the operand at xb + i slice_stride
     int64_t slice_stride;
     // grouped scales (GRP kernels): gtab[group 0..n_groups][r][tab_ld rows] = bf16 scale | bf16 zero << 16 (row n_groups
@@ -1104,10 +1105,12 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // units / 4 of their own on the f32 MFMA in front of the loop.
 // RUNS (Q4): a slice of several runs (gemm_runs()).  The second set of sums is 32 registers, with which two workgroups of 8 waves no longer share a CU: kernels of
 // their own.
-// ONCE: one token block (BM tokens at most), so nothing reads a piece of the weights again: they are requested non-temporal and push no activations out of the L2 caches.
-// BF16, 16 products of 2048 to 32000 rows, weights in no cache: 16 tokens 0.89 times as long (0.86 to 0.94; N = 4096, K = 16512 30.9 -> 26.8 us, N = 32000, K = 4096 52.0 -> 46.0), 24 tokens
-// 0.91, 40 0.93, 64 0.95 (two of 16 up to 1.01).  Int4 of one scale per row, which its own work bounds, the same either way; groups of 128 columns, 16 and 24 tokens, 0.95.
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW, bool ONCE = BM <= 48>
+// ONCE: one token block (BM tokens at most) and weights that come from HBM (MI355_LF_STREAMED), so nothing reads a piece of them again: they are requested non-temporal and push no activations
+// out of the L2 caches.  BF16, 16 products of 2048 to 32000 rows, weights in no cache: 16 tokens 0.89 times as long (0.86 to 0.94; N = 4096, K = 16512 30.9 -> 26.8 us, N = 32000, K = 4096 52.0 ->
+// 46.0), 24 tokens 0.91, 40 0.93, 64 0.95 (two of 16 up to 1.01).  Int4 of one scale per row, which its own work bounds, the same either way; groups of 128 columns, 16 and 24 tokens, 0.95.
+// Weights that a cache holds it costs: ten BF16 products of 1024 to 8192 rows, all copies read in turn 100 / 200 / 256 / 288 / 320 / 352 / 600 MB, 16 tokens 1.07 / 1.08 / 1.05 / 1.02 / 0.97 / 0.95 / 0.92 times
+// as long (100 MB: N = 6144, K = 2048 1.28), one copy again and again 1.12 (1.54).
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW, bool ONCE = false>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_deep_kernel(const GemmParams p) {
     static_assert(GRP == 0 || (FMT == MI355_W_Q4 && GRP == 1), "grouped scales are a Q4 feature");
     static_assert(!RUNS || (FMT == MI355_W_Q4 && GRP == 0), "runs: int4 sums, one scale per row");
@@ -1679,13 +1682,13 @@ int launch_blocks(Kernel kernel, int lds, const GemmParams& p, hipStream_t s) { 
     }
     return 0;
 }
-template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false, bool ONCE = BM <= 48>
+template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int GRP = 0, int TPW = kTPW, bool RUNS = false, bool ONCE = false>
 int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM <= 64 && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, true>(p, s);
     }
-    if constexpr (FMT == MI355_W_BF16 && BM == 64 && !ONCE) {
-        if (p.M <= BM) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, RUNS, true>(p, s);
+    if constexpr (!ONCE && ((FMT == MI355_W_BF16 && BM <= 64) || (GRP == 1 && BM <= 48))) {
+        if (p.streamed && p.M <= BM) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, RUNS, true>(p, s);
     }
     constexpr int kDepth = BM > 192 ? 2 : BM > kBM || (BM >= 96 && FMT == MI355_W_BF16) ? 3 : 4;
     constexpr int kLds = kRowAt<BM, FUSE, kDepth> + 3 * kWaves * TPW * 64 + (RUNS ? kMaxRuns * BM * 4 : 0) + (FMT == MI355_W_BF16 ? 256 : 0);
@@ -1874,22 +1877,24 @@ void q4_whole(int M, int N, int K, bool pair, GemmCut* cut) {
 // asks for no more than its memory pipeline holds, so 129 blocks of 128 rows leave half of what HBM gives, and a slice that would fill the other CUs costs a launch; smaller
 // blocks cost their activations again.  16 tokens, 4 / 3 / 2 waves without slices: N = 16512, K = 4096 29.7 / 26.1 / 35.0 us (129, 172, 258 blocks), 12416 33.2 (24.9 in two
 // slices) / 27.4 / 21.4; K = 16384, N = 4096 28.8 in 4-wave blocks x 6 slices, 27.9 in 2-wave blocks x 3.  The estimate is the rounds of the chip, each unit of one `unit` us, `unit_wave`
-// more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Slices go down to 2 units: the weights are read past
-// the caches, so a short product is a wait for memory that more blocks share out (N = K = 2048, 16 / 24 / 32 tokens 8.2 / 9.1 / 9.5 us whole in 32 blocks -> 6.8 / 7.4 / 7.7 in 8 slices;
-// N = 6256, K = 3328, 32 tokens 17.3 -> 14.1).  That holds for 512 to 4095 columns.  Longer rows have units enough (N = 2048, K = 8448, 16 tokens 11.1 us in 6 slices, 11.7 in 8; N = 5120,
-// K = 20736 36.7 in 2 waves x 3, 37.4 in 4 x 6), up to 8 tokens (N = 4672, K = 3456, 2 tokens 10.6 us in 3 slices, 11.3 in 7) and in pairs, whose sums are twice as long (25 products at
-// 24 to 64 tokens 0.99-1.00 on average, the worst 1.13), more sums cost what they give: there slices keep 4 units.  35 products of 1024 to 6176 rows and 1024 to 3072 columns, 16 to 64
-// tokens: 0.96 times as long as in slices of 4 units, the least 0.71, the most 1.03 (profiles/product_cuts_bf16_few.txt).
-GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced) {
+// more for each wave of a block and `crowd` more when every CU has one, `wave` for each wave's start, and a launch for the slices.  Slices go down to 2 units where a row is 4 to 31 of them (385 to
+// 3968 columns): a short product is a wait for memory that more blocks share out (N = K = 2048, weights from HBM, 16 / 24 / 32 tokens 8.2 / 9.3 / 9.6 us whole in 32 blocks, 6.8 / 7.5 / 7.8 in 8 slices).
+// Longer rows have units enough (N = 2048, K = 8448, 16 tokens 11.1 us in 6 slices, 11.7 in 8; N = 5120, K = 20736 36.7 in 2 waves x 3, 37.4 in 4 x 6), up to 8 tokens (N = 4672, K = 3456, 2 tokens
+// 10.6 us in 3 slices, 11.3 in 7) and in pairs, whose sums are twice as long (25 products at 24 to 64 tokens 0.99-1.00 on average, the worst 1.13), more sums cost what they give: there slices keep 4 units.
+// Weights that a cache holds (not MI355_LF_STREAMED) are asked for faster, so fewer blocks fill the chip: up to 32 tokens constants of their own (110 MB of copies, N = 5856, K = 3456, 16 tokens
+// 8.9 us in blocks of 2 waves, whole, 11.5 in 4 slices of blocks of 3).  Times of every cut: profiles/product_cuts_bf16_few.txt.  From HBM, 52 products of 1024 to 32000 rows and 512 to 20736 columns: up to 32 tokens 0.6 % behind the
+// fastest cut on average, 6 % at most, 40 and 64 tokens 1.1 % (9 %); from a cache, 56 products of 512 to 12288 rows and 512 to 3968 columns, 9 and 16 tokens 0.4 % (7 %), 24 and 32 0.7 % (9 %).
+GemmCut bf16_cut_few(int M, int N, int K, bool pair, bool sliced, bool streamed) {
     struct Cost {
         float wave, unit, unit_wave, crowd, slices, bytes;
     };
-    static constexpr Cost costs[] = {{0.f, 0.007f, 0.066f, 0.193f, 1.5f, 2.7e6f}, {0.25f, 0.21f, 0.023f, 0.041f, 0.3f, 2.3e6f},  // slices of 4 units: up to 32 tokens, up to 64
-                                     {0.494f, 0.0935f, 0.0402f, 0.17f, 1.56f, 2.33e6f}, {0.607f, 0.045f, 0.0371f, 0.0182f, 0.861f, 4.79e6f},  // of 2: up to 16, up to 32,
-                                     {0.256f, 0.207f, 0.025f, 0.0058f, 0.576f, 2.31e6f}};                                                     // up to 64
+    static constexpr Cost costs[] = {{0.f, 0.007f, 0.066f, 0.193f, 1.5f, 2.7e6f}, {0.25f, 0.21f, 0.023f, 0.041f, 0.3f, 2.3e6f},               // slices of 4 units: up to 32 tokens, up to 64
+                                     {0.494f, 0.0935f, 0.0402f, 0.17f, 1.56f, 2.33e6f}, {0.607f, 0.045f, 0.0371f, 0.0182f, 0.861f, 4.79e6f},  // of 2, from HBM: up to 16, up to 32
+                                     {0.516f, 0.066f, 0.0195f, 0.481f, 1.85f, 6.21e6f}, {0.57f, 0.0732f, 0.0415f, 0.153f, 1.36f, 1.44e6f},    // of 2, from a cache
+                                     {0.256f, 0.207f, 0.025f, 0.0058f, 0.576f, 2.31e6f}};                                                     // of 2, up to 64
     const int units = (K + 127) / 128;
     const bool shorter = !pair && M > 8 && units >= 4 && units < 32;
-    const int least = shorter ? 2 : 4, line = (M > 32) + (shorter ? 2 + (M > 16) : 0);
+    const int least = shorter ? 2 : 4, line = !shorter ? (M > 32) : M > 32 ? 6 : (streamed ? 2 : 4) + (M > 16);
     const Cost& c = costs[line];
     GemmCut cut = {4, short_block(M, true), true, 1};
     float best = 0.f;
@@ -1972,15 +1977,15 @@ GemmCut bf16_cut_long(int M, int N, int K, bool pair) {
         if (const float us = estimate(k, 1); us < best) best = us, cut = {k.waves, k.bm, true, 1};
     return cut;
 }
-GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced) {
+GemmCut bf16_cut(int M, int N, int K, bool pair, bool chain, bool sliced, bool streamed) {
     if (M > 64) return bf16_cut_long(M, N, K, pair);
     if (gemm_blocks(M, N, pair, 4, 64) > 256) return bf16_cut_many(M, N, K, pair);
-    return chain ? bf16_cut_few_chained(M, N, K, pair) : bf16_cut_few(M, N, K, pair, sliced);
+    return chain ? bf16_cut_few_chained(M, N, K, pair) : bf16_cut_few(M, N, K, pair, sliced, streamed);
 }
-// chain: a launch of the fused prompt chain (gemm_fuse.h); sliced: a launch of operand slices
-GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced) {
+// chain: a launch of the fused prompt chain (gemm_fuse.h); sliced: a launch of operand slices; streamed: weights that come from HBM
+GemmCut gemm_cut(int M, int N, int K, bool pair, bool bf16, bool chain, bool sliced, bool streamed) {
     const GemmForce fo = gemm_force();
-    const GemmCut first = bf16 ? bf16_cut(M, N, K, pair, chain, sliced) : q4_cut(M, N, K, pair);
+    const GemmCut first = bf16 ? bf16_cut(M, N, K, pair, chain, sliced, streamed) : q4_cut(M, N, K, pair);
     GemmCut cut = first;
     if (!bf16) q4_narrow(M, N, K, pair, chain, &cut), q4_whole(M, N, K, pair, &cut);
     const GemmCut& from = fo.deep >= 3 || (fo.waves == 0 && fo.bm == 0 && fo.deep == 0) ? cut : first;
@@ -2035,14 +2040,14 @@ GemmCut gemm_cut_grouped(int n_tiles, int M, bool pair, int units, int ksplit) {
 }
 template <int EPI, bool PAIR, int FMT, bool FUSE>
 int launch_gemm(const GemmParams& p, hipStream_t s) {
-    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE, p.slice_blocks != 0);
+    const GemmCut sh = gemm_cut(p.M, p.N, p.K, PAIR, FMT == MI355_W_BF16, FUSE, p.slice_blocks != 0, p.streamed);
     if constexpr (FMT == MI355_W_BF16 && !FUSE) {
         if (sh.waves == 3) {
-            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 3, 64, FUSE, 0, kTPW, false, true>(p, s);
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 3, 64, FUSE>(p, s);
             return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 3, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 3, 32, FUSE>(p, s);
         }
         if (sh.waves == 2) {
-            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE, 0, kTPW, false, true>(p, s);
+            if (sh.bm == 64) return launch_deep<EPI, PAIR, FMT, 2, 64, FUSE>(p, s);
             return sh.bm == 16 ? launch_deep<EPI, PAIR, FMT, 2, 16, FUSE>(p, s) : launch_deep<EPI, PAIR, FMT, 2, 32, FUSE>(p, s);
         }
     }
@@ -2179,14 +2184,18 @@ void plan_shares(const GemmCut& cut, int N, bool pair, int* ksplit, int* shares,
 }
 }  // namespace
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit) {
-    plan_shares(gemm_cut(M, N, K, R == 2, bf16, true, false), N, R == 2, ksplit, shares, shares_per_unit);
+    plan_shares(gemm_cut(M, N, K, R == 2, bf16, true, false, false), N, R == 2, ksplit, shares, shares_per_unit);
 }
 extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, bool sliced, int* waves, int* tokens, int* ksplit) {
-    const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain, sliced);
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, bf16, chain, sliced, false);
+    *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
+}
+extern "C" void mi355_linear_gemm_cut_streamed(int M, int N, int K, int R, bool sliced, int* waves, int* tokens, int* ksplit) {
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, true, false, sliced, true);
     *waves = cut.waves, *tokens = cut.bm, *ksplit = cut.ksplit;
 }
 extern "C" void mi355_linear_gemm_sums(int M, int N, int K, int R, bool chain, int* tiles, int* ksplit, int* runs, int* longest, int* longest_of_wide) {
-    const GemmCut cut = gemm_cut(M, N, K, R == 2, false, chain, false);
+    const GemmCut cut = gemm_cut(M, N, K, R == 2, false, chain, false, false);
     int run_units;
     gemm_runs(M, N, K, R == 2, cut, runs, &run_units);
     *tiles = cut.tiles, *ksplit = cut.ksplit, *longest = gemm_longest(M, N, K, R == 2, cut), *longest_of_wide = gemm_longest(M, N, K, R == 2, q4_cut(M, N, K, R == 2));
@@ -2250,7 +2259,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     MI355_CHECK_ARG(a != nullptr && workspace != nullptr, MI355_E_ARG, "linear_gemm: null argument");
     MI355_CHECK_ARG(a->fmt == MI355_W_Q4 || a->fmt == MI355_W_BF16, MI355_E_ARG,
                     "linear_gemm: the wide path handles the Q4 and BF16 streams (fmt %d)", a->fmt);
-    const bool q4 = a->fmt == MI355_W_Q4;
+    const bool q4 = a->fmt == MI355_W_Q4, streamed = (a->flags & MI355_LF_STREAMED) != 0;
     MI355_CHECK_ARG(a->w && a->x && a->y && (!q4 || (a->scales && a->zeros)), MI355_E_ARG, "linear_gemm: null w/x/y/scales/zeros");
     // grouped scales: group_cols = input columns per (scale, zero) pair; 0 or >= K: one pair per output row
     const bool scale_groups = q4 && a->group_cols > 0 && a->group_cols < a->K;
@@ -2306,7 +2315,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     }
     int runs = 1, run_units = units;
     if (!grouped) {
-        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr, a->slice_rows != 0);
+        const GemmCut cut = gemm_cut(a->M, a->N, a->K, swiglu, !q4, f != nullptr, a->slice_rows != 0, streamed);
         ksplit = cut.ksplit;
         if (q4) gemm_runs(a->M, a->N, a->K, swiglu, cut, &runs, &run_units);
         MI355_CHECK_ARG(runs <= kMaxRuns && ksplit * runs <= kMaxSums, MI355_E_STATE, "linear_gemm: %d slices of %d runs (M=%d N=%d K=%d)", ksplit, runs, a->M, a->N, a->K);
@@ -2398,6 +2407,7 @@ static int run_linear_gemm(const mi355_linear_args* a, const mi355_gemm_fuse* f,
     p.zeros = a->zeros;
     p.scales2 = a->scales2;
     p.zeros2 = a->zeros2;
+    p.streamed = streamed;
     p.relu2 = (a->flags & MI355_LF_RELU2) ? 1 : 0;
     MI355_CHECK_ARG(!p.relu2 || (a->epi == MI355_EPI_STORE && !fused), MI355_E_ARG, "linear_gemm: RELU2 belongs to the plain STORE epilogue");
     MI355_CHECK_ARG(!(grouped || f_in) || a->alpha == 0.f || a->alpha == 1.f, MI355_E_ARG, "linear_gemm: alpha needs the staging pass of per-row scales");

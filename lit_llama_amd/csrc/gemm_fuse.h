@@ -50,6 +50,8 @@ struct mi355_gemm_fuse {
 extern "C" void mi355_linear_gemm_plan(int M, int N, int K, int R, bool bf16, int* ksplit, int* shares, int* shares_per_unit);
 // how a launch of one scale per row is cut, in the chain or outside it, of operand slices or not: waves and tokens of a block, K-slices
 extern "C" void mi355_linear_gemm_cut(int M, int N, int K, int R, bool bf16, bool chain, bool sliced, int* waves, int* tokens, int* ksplit);
+// ... one of BF16 outside the chain, weights that come from HBM
+extern "C" void mi355_linear_gemm_cut_streamed(int M, int N, int K, int R, bool sliced, int* waves, int* tokens, int* ksplit);
 // int4, one scale per row: row tiles of a wave, K-slices, runs of a slice, the units that one accumulator sums, and those in the blocks of two row tiles a wave that the rule starts from
 extern "C" void mi355_linear_gemm_sums(int M, int N, int K, int R, bool chain, int* tiles, int* ksplit, int* runs, int* longest, int* longest_of_wide);
 // the plan for scales in groups of group_cols columns (whole units)

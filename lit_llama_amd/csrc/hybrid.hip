@@ -428,7 +428,7 @@ int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int6
     a.norm_dtype = m->norm_dtype;
     a.eps = m->eps;
     a.epi = what == kResidual ? MI355_EPI_ACCUM : what == kGeglu ? MI355_EPI_GEGLU : MI355_EPI_STORE;
-    a.flags = (what == kRelu2 ? MI355_LF_RELU2 : 0) | (m->norm_add != 0.f ? MI355_LF_NORM_ONE : 0);
+    a.flags = (what == kRelu2 ? MI355_LF_RELU2 : 0) | (m->norm_add != 0.f ? MI355_LF_NORM_ONE : 0) | m->linear_flags;
     a.alpha = what == kResidual ? m->residual_mult : what == kLogits ? m->logit_scale : 1.f;
     a.y_dtype = y_dtype;
     a.ldy = ldy;
@@ -485,6 +485,7 @@ mi355_product product_of(const mi355_hybrid_model* m, const void* x, int64_t ldx
     p.x = x, p.ldx = ldx, p.M = M;
     p.y = y, p.ldy = ldy, p.y_dtype = y_dtype, p.epi = epi;
     p.alpha = 1.f;
+    p.flags = m->linear_flags;
     p.ws = m->gemm_ws, p.ws_bytes = m->gemm_ws_bytes;
     return p;
 }
@@ -677,6 +678,7 @@ int mi355_product_run(const mi355_product& p, const mi355_proj& w, hipStream_t s
     a.ldy = p.ldy;
     a.slice_rows = p.slice_rows;
     a.slice_stride = p.slice_stride;
+    a.flags = p.flags;
     MI355_CHECK_ARG(p.ldx >= a.K && p.ldx % 8 == 0, MI355_E_SHAPE, "product: rows of pitch %lld hold no operand of %d columns", (long long)p.ldx, a.K);
     if (p.slice_rows != 0 || mi355_product_wide(w, p.M, a.R)) return mi355_linear_gemm(&a, p.ws, (size_t)p.ws_bytes, s);
     return mi355_linear_fast(&a, s);
@@ -761,6 +763,7 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
             }
         } else if (l.mixer == MI355_MIX_LATENT) {
             mi355_latent_args a = l.latent;
+            a.linear_flags = m->linear_flags;
             a.proj = m->proj;
             a.ld = ldp;
             a.dtype = m->dtype;

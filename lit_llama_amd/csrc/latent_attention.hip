@@ -676,7 +676,7 @@ int run_tiles(LatParams p, mi355_stream_t stream) {
         q.dtype = q.y_dtype = MI355_BF16;
         q.x = a.rows_c, q.ldx = ld_c, q.M = n * span;
         q.y = a.kv_rows, q.ldy = a.expand.N, q.epi = MI355_EPI_STORE, q.alpha = 1.f;
-        q.ws = a.gemm_ws, q.ws_bytes = a.gemm_ws_bytes;
+        q.ws = a.gemm_ws, q.ws_bytes = a.gemm_ws_bytes, q.flags = a.linear_flags;
         if (int rc = mi355_product_run(q, a.expand, s)) return rc;
         mi355_window_attn_args w;
         memset(&w, 0, sizeof(w));
@@ -731,7 +731,7 @@ extern "C" int mi355_latent_attention(const mi355_latent_args* a, const mi355_se
     q.dtype = q.y_dtype = a->dtype;
     q.x = a->cq, q.ldx = p.ld_cq, q.M = b->rows;
     q.y = a->q, q.ldy = a->uq.N, q.epi = MI355_EPI_STORE, q.alpha = 1.f;
-    q.ws = a->gemm_ws, q.ws_bytes = a->gemm_ws_bytes;
+    q.ws = a->gemm_ws, q.ws_bytes = a->gemm_ws_bytes, q.flags = a->linear_flags;
     if (int rc = mi355_product_run(q, a->uq, s)) return rc;
     const bool tiles = !p.fresh && tiles_fit(*a, *b), mfma = mfma_fits(*a);
     MI355_CHECK_ARG((a->path != 2 || mfma) && (a->path != 3 || tiles), MI355_E_SHAPE, "latent_attention: this shape does not take path %d", a->path);

@@ -14,6 +14,7 @@ struct mi355_product {
     float alpha, limit;
     int slice_rows;       // see mi355_linear_args
     int64_t slice_stride;
+    int flags;            // MI355_LF_STREAMED, or 0
     void* ws;             // of mi355_linear_gemm
     uint64_t ws_bytes;
 };

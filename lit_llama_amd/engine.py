@@ -407,6 +407,9 @@ class DecodeEngine:
                     self._keep += [ak, av, gate]
             head = pack_linear(model.lm_head, 1, tune=dflt("lm_head"))
             self.packed.append(head)
+            flags = nat.streamed(sum(p.stream_bytes for p in self.packed))
+            for w in [head.desc] + [w for L in layers for w in (L.attn, L.proj, L.fc, L.mproj)]:
+                w.flags |= flags
             self.layers = layers
 
             # LDS bound on the rows one launch can stage (see ops.fast_linear_max_m)

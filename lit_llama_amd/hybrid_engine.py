@@ -259,6 +259,7 @@ class HybridEngine:
         M.embed, M.final_norm = ptr(T["embed"]), self._norm("final.norm")
         M.head = self._proj(T["embed" if cfg.design.tied else "head"])
         M.ld_logits = M.head.N
+        M.linear_flags = nat.streamed(self.weight_bytes)
         M.layers = self.layers
         if cfg.design.sandwich:
             M.embed_norm = self._norm("embed.norm")

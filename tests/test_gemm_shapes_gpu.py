@@ -389,7 +389,7 @@ def test_fused_prompt_chain_over_layers_of_different_formats(dev, monkeypatch, T
 @pytest.mark.parametrize("epi", ["store", "pair", "accum"])
 @pytest.mark.parametrize("M", [5, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(64, 128), (68, 1000), (96, 4096), (100, 640), (4096, 2048), (8200, 384), (12352, 1024), (16512, 512)])
-def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
+def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi, flags=0):
     """Block edges at 64, 96 and 128 rows, slices, a last unit that is not whole.  The bound of the tiled product."""
     g = torch.Generator(device=dev).manual_seed(M * 31 + N + K)
     x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
@@ -397,33 +397,70 @@ def test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi):
     prods = [x.double() @ w.double().T for w in ws]
     if epi == "pair":
         ref = torch.nn.functional.silu(prods[0]) * prods[1]
-        got = ops.linear_gemm(x, ops.repack_bf16(ws[0], ws[1], 2), 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, fmt=nat.W_BF16).double()
+        got = ops.linear_gemm(x, ops.repack_bf16(ws[0], ws[1], 2), 2, N, K, epi=nat.EPI_SWIGLU, out_dtype=torch.bfloat16, fmt=nat.W_BF16, flags=flags).double()
         assert (got - ref).abs().max() <= 2.0 ** -8 * ref.abs().max() + 2e-3 * ref.square().mean().sqrt()
         return
     base = torch.randn((M, N), generator=g, device=dev) if epi == "accum" else torch.zeros((M, N), device=dev)
     ref = prods[0] + base.double()
-    got = ops.linear_gemm(x, ops.repack_bf16(ws[0], None, 1), 1, N, K, epi=nat.EPI_ACCUM if epi == "accum" else nat.EPI_STORE, out=base.clone(), fmt=nat.W_BF16).double()
+    got = ops.linear_gemm(x, ops.repack_bf16(ws[0], None, 1), 1, N, K, epi=nat.EPI_ACCUM if epi == "accum" else nat.EPI_STORE, out=base.clone(), fmt=nat.W_BF16, flags=flags).double()
     assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
 
 
-@pytest.mark.parametrize("epi", ["store", "pair", "accum"])
-@pytest.mark.parametrize("M", [2, 17, 64])
-@pytest.mark.parametrize("N,K", [(100, 1024), (1000, 1900), (2048, 2048), (2052, 2200)])
+@pytest.mark.parametrize("epi", ["store", "accum"])
+@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(1000, 1900), (1500, 2700), (2052, 2200), (640, 3968)])
 def test_few_bf16_rows_in_slices_of_2_and_3_units(dev, N, K, M, epi):
     """Slices no longer than the buffers that are filled ahead, some of 2 and some of 3 units, the last one not whole.  The bound of longer slices."""
-    test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi)
+    out = [C.c_int(0) for _ in range(3)]
+    nat.lib().mi355_linear_gemm_cut_streamed(M, N, K, 1, C.c_bool(False), *[C.byref(v) for v in out])
+    assert -(-K // 128) // out[2].value in (2, 3)
+    test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi, flags=nat.LF_STREAMED)
 
 
-@pytest.mark.parametrize("M", [49, 64, 65])
-@pytest.mark.parametrize("N,K", [(128, 640), (33024, 384), (70000, 128)])
-def test_blocks_of_64_tokens_read_once_or_by_several(dev, N, K, M):
-    """BF16 blocks of 64 tokens by themselves (weights requested non-temporal) and side by side, of 2 to 8 waves: f32 sums of exact products (see test_tiled_product_against_64_bits)."""
+@pytest.mark.parametrize("M", [2, 16, 24, 40, 48, 49, 64, 65])
+@pytest.mark.parametrize("N,K,fmt", [(128, 640, "bf16"), (33024, 384, "bf16"), (70000, 128, "bf16"), (4096, 4096, "bf16"), (640, 1024, "g128"), (4096, 1152, "q4")])
+def test_weights_past_the_caches_or_through_them(dev, N, K, fmt, M):
+    """Weights requested non-temporal (one token block) or not, of 2 to 8 waves: f32 sums of exact products (see test_tiled_product_against_64_bits), the same bits where the cut is the same."""
     g = torch.Generator(device=dev).manual_seed(M + N)
     x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
-    w = (torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16)
-    got = ops.linear_gemm(x, ops.repack_bf16(w, None, 1), 1, N, K, out_dtype=torch.float32, fmt=nat.W_BF16).double()
-    ref = x.double() @ w.double().T
-    assert (got - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+    if fmt == "bf16":
+        w = (torch.randn((N, K), generator=g, device=dev) * 0.05).to(torch.bfloat16)
+        kw, ref = dict(fmt=nat.W_BF16), x.double() @ w.double().T
+        stream = ops.repack_bf16(w, None, 1)
+    else:
+        groups = K // 128 if fmt == "g128" else 1
+        q = torch.randint(0, 16, (N, K), generator=g, device=dev, dtype=torch.uint8)
+        scales, zeros = (torch.rand((N, groups), generator=g, device=dev) * 0.01 + 0.01).bfloat16(), torch.full((N, groups), 8.0, device=dev).bfloat16()
+        stream = ops.repack_q4(synth.pack_colblock(q, 4), None, N, K, 1)
+        kw = dict(scales=scales if groups > 1 else scales.view(-1), zeros=zeros if groups > 1 else zeros.view(-1), **({"group_cols": 128} if groups > 1 else {}))
+        wide = lambda t: t.double().repeat_interleave(K // groups, 1)  # noqa: E731
+        ref = x.double() @ ((q.double() - wide(zeros)) * wide(scales)).T
+    got = [ops.linear_gemm(x, stream, 1, N, K, out_dtype=torch.float32, flags=f, **kw).double() for f in (0, nat.LF_STREAMED)]
+    for y in got:
+        assert (y - ref).abs().max() <= 1e-3 * ref.square().mean().sqrt()
+    assert torch.equal(*got)
+
+
+def test_engines_say_which_weights_are_streamed(dev, monkeypatch):
+    """Every product of a model, or none (a model of this size)."""
+    from lit_llama_amd import synth
+    from lit_llama_amd.model import LLaMA, LLaMAConfig
+    from lit_llama_amd.utils import EmptyInitOnDevice
+
+    cfg = LLaMAConfig(n_layer=2, n_head=4, n_embd=256, vocab_size=512)
+    for want in (0, nat.LF_STREAMED):
+        if want:
+            monkeypatch.setattr(nat, "streamed", lambda n: nat.LF_STREAMED if n == bytes_of else 0)
+        with EmptyInitOnDevice(device=dev, dtype=torch.bfloat16):
+            model = LLaMA(cfg)
+        model.load_state_dict(synth.make_state_dict(cfg, seed=1, dtype=torch.bfloat16))
+        model.eval()
+        with torch.no_grad():
+            model(torch.arange(9, device=dev).view(1, -1), 32, torch.arange(9, device=dev))
+        eng = model.engine()
+        bytes_of = sum(p.stream_bytes for p in eng.packed)
+        assert bytes_of == sum(p.numel() * 2 for n, p in model.named_parameters() if n == "lm_head.weight" or (p.dim() == 2 and "wte" not in n))
+        assert {w.flags for L in eng.layers for w in (L.attn, L.proj, L.fc, L.mproj)} | {eng.m.lm_head.flags} == {want}
 
 
 OPERAND_SLICES = [(9, 256, 9, 4096), (16, 512, 5, 4096), (24, 256, 22, 4096), (32, 256, 65, 128), (32, 3072, 2, 4096), (40, 256, 65, 256), (40, 256, 18, 4096), (64, 256, 66, 256), (64, 512, 11, 4096)]

@@ -685,6 +685,32 @@ def test_bf16_blocks_of_160_and_208_tokens_are_whole_rows():
     assert [_gemm_cut(M, N, K, 1, False)[1] for M, N, K in ((777, 12288, 4096), (777, 15360, 5120), (2048, 12416, 4096))] == [160, 208, 208]
 
 
+def test_weights_are_streamed_from_what_the_cache_does_not_hold():
+    assert [nat.streamed(n) for n in (0, 7_000_000, 300_000_000, 300_000_001, 13_000_000_000)] == [0, 0, 0, nat.LF_STREAMED, nat.LF_STREAMED]
+
+
+def _streamed_cut(M, N, K, R):
+    out = [C.c_int(0) for _ in range(3)]
+    nat.lib().mi355_linear_gemm_cut_streamed(M, N, K, R, C.c_bool(False), *[C.byref(v) for v in out])
+    return tuple(v.value for v in out)
+
+
+def test_few_bf16_rows_are_cut_by_where_their_weights_are():
+    """Slices of fewer than 4 units for 9 to 64 rows of 4 to 31 units only, and up to 32 rows fewer of them where a cache holds the weights (N = 5856, K = 3456, 16 rows 8.9 us whole, 11.5 in 4)."""
+    short, fewer = set(), 0
+    for N in (512, 1024, 2048, 2052, 4096, 5856, 6144, 8192):
+        for K in (300, 385, 1024, 1792, 2048, 3456, 2200, 3072, 3968, 3969, 4096, 8192):
+            for M in (1, 5, 8, 9, 16, 17, 24, 32, 33, 64):
+                cut, streamed = _gemm_cut(M, N, K, 1, False), _streamed_cut(M, N, K, 1)
+                assert cut == streamed or (8 < M <= 32 and 385 <= K <= 3968)
+                short |= {(M, K) for _, _, slices in (cut, streamed) if slices > 1 and -(-K // 128) < 4 * slices}
+                assert M > 16 or cut[2] <= streamed[2]
+                fewer += cut[2] < streamed[2]
+                assert _gemm_cut(M, N, K, 2, False) == _streamed_cut(M, N, K, 2)
+    assert {M for M, _ in short} == {9, 16, 17, 24, 32, 33, 64} and all(385 <= K <= 3968 for _, K in short) and fewer > 20
+    assert _gemm_cut(16, 5856, 3456, 1, False)[2] == 1 < _streamed_cut(16, 5856, 3456, 1)[2]
+
+
 def _gemm_shapes():
     import importlib.util
     import pathlib
