@@ -339,18 +339,18 @@ __global__ __launch_bounds__(256) void residual_kernel(float* x, const float* t,
 constexpr int kZeroRegions = 32;
 struct ZeroRegions {
     float* at[kZeroRegions];
-    int per[kZeroRegions];
+    int64_t per[kZeroRegions];
 };
-// grid (parts, regions, slots), 256 threads.  A server takes its slots one after another, so what counts is the launch: all runs in one, the slot's number by value (slots == NULL).  With a
+// grid (slots, regions, parts), 256 threads.  A server takes its slots one after another, so what counts is the launch: all runs in one, the slot's number by value (slots == NULL).  With a
 // launch per run, the number uploaded and waited for, 53 sequences of up to 73 tokens (four layers of 3072, a step each) took 4.53 ms from their slots on, now 3.72
 __global__ __launch_bounds__(256) void zero_slots_kernel(const ZeroRegions z, const int32_t* slots, int slot) {
-    const int n = z.per[blockIdx.y];
-    float* const s = z.at[blockIdx.y] + (int64_t)(slots != nullptr ? slots[blockIdx.z] : slot) * n;
-    const int at = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    const int64_t n = z.per[blockIdx.y];
+    float* const s = z.at[blockIdx.y] + (slots != nullptr ? slots[blockIdx.x] : slot) * n;
+    const int64_t at = blockIdx.z * 256 + threadIdx.x, step = gridDim.z * 256;
     if (((uintptr_t)s & 15) == 0 && n % 4 == 0) {
-        for (int i = at; i < n / 4; i += step) ((f32x4*)s)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int64_t i = at; i < n / 4; i += step) ((f32x4*)s)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     } else {
-        for (int i = at; i < n; i += step) s[i] = 0.f;
+        for (int64_t i = at; i < n; i += step) s[i] = 0.f;
     }
 }
 
@@ -832,19 +832,19 @@ extern "C" int mi355_hybrid_forward(const mi355_hybrid_model* m, const mi355_seq
 
 static int reset_slots(const mi355_hybrid_model* m, const int32_t* slots, int n, int slot, hipStream_t stream) {
     ZeroRegions z;
-    int regions = 0, most = 0;
+    int regions = 0;
+    int64_t most = 0;
     auto flush = [&]() -> int {
         if (regions == 0) return 0;
-        const int parts = (most + 4095) / 4096;  // (four stores of 16 bytes a thread: 2 MB are 128 blocks)
-        hipLaunchKernelGGL(zero_slots_kernel, dim3(parts < 128 ? parts : 128, regions, n), dim3(256), 0, stream, z, slots, slot);
+        const int64_t parts = (most + 4095) / 4096;  // (four stores of 16 bytes a thread: 2 MB are 128 blocks)
+        hipLaunchKernelGGL(zero_slots_kernel, dim3(n, regions, (unsigned)(parts < 128 ? parts : 128)), dim3(256), 0, stream, z, slots, slot);
         MI355_LAUNCH_CHECK();
-        regions = most = 0;
+        regions = 0, most = 0;
         return 0;
     };
     auto add = [&](float* at, int64_t per) -> int {
-        MI355_CHECK_ARG(per < (int64_t)1 << 31, MI355_E_SHAPE, "hybrid_reset_slots: a state of %lld numbers", (long long)per);
-        z.at[regions] = at, z.per[regions] = (int)per;
-        if (z.per[regions] > most) most = z.per[regions];
+        z.at[regions] = at, z.per[regions] = per;
+        if (per > most) most = per;
         return ++regions == kZeroRegions ? flush() : 0;
     };
     for (int r = 0; r < m->n_runs; ++r) {

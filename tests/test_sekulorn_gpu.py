@@ -435,6 +435,24 @@ def test_a_slot_is_cleared_in_every_run_and_no_other_slot_is(dev, runs):
         nat.check(nat.lib().mi355_hybrid_reset_slots(C.byref(m), slots.data_ptr(), 2, stream), "reset_slots")
 
 
+def test_more_slots_are_cleared_than_a_grid_is_high(dev):
+    import ctypes as C
+
+    from lit_llama_amd import _native as nat
+
+    states = [torch.ones((5, 2, 3, 4), device=dev), torch.ones((5, 1, 1, 3), device=dev)]
+    layers = (nat.HybridLayer * 2)()
+    for l, t in zip(layers, states):
+        l.mixer = 1
+        l.rec.heads, l.rec.dim, l.rec.vdim, l.rec.state = *t.shape[1:], t.data_ptr()
+    m = nat.HybridModel()
+    m.n_runs, m.width, m.layers = 2, 30, layers
+    slots = torch.tensor([1, 4], dtype=torch.int32, device=dev).repeat(40000)
+    nat.check(nat.lib().mi355_hybrid_reset_slots(C.byref(m), slots.data_ptr(), slots.numel(), torch.cuda.current_stream().cuda_stream), "reset_slots")
+    for t in states:
+        assert [bool((t[s] == (s not in (1, 4))).all()) for s in range(5)] == [True] * 5
+
+
 @pytest.mark.parametrize("name,dtype,tol", [("mixed", torch.float32, 1e-4), ("mixed", torch.bfloat16, 0.12), ("all looped", torch.bfloat16, 0.12)])
 def test_portions_batches_slots_and_decoding(dev, name, dtype, tol):
     """Unequal requests in one batch, cut differently, decoded together, their slots used again: the logits of each alone."""
