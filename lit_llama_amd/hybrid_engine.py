@@ -588,7 +588,10 @@ class HybridEngine:
             tokens.extend(t)
         self._meta_sent.synchronize()  # the previous upload has left the pinned buffer
         for row, numbers in zip(self._meta_rows, lists):
-            row[:len(numbers)] = numbers
+            try:
+                row[:len(numbers)] = numbers
+            except (TypeError, ValueError):  # (scalars on the device among them)
+                row[:len(numbers)] = [int(k) for k in numbers]
         self.meta.copy_(self.meta_host, non_blocking=True)
         self._meta_sent.record(self.stream)
         return self._batch(len(tokens), len(entries), max(count), max(p + n for p, n in zip(pos, count))), len(want)

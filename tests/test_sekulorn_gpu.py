@@ -453,6 +453,24 @@ def test_more_slots_are_cleared_than_a_grid_is_high(dev):
         assert [bool((t[s] == (s not in (1, 4))).all()) for s in range(5)] == [True] * 5
 
 
+def test_tokens_in_any_form(dev):
+    """Lists of numbers, of scalars on the device or the host, arrays, tensors: the same step."""
+    from lit_llama_amd.hybrid_engine import Entry
+
+    m, _ = build(CONFIGS["mixed"], torch.float32, dev)
+    eng = m.engine()
+    eng.ensure(2, 64)
+    toks, got = tokens_of(7), []
+    for form in (list, tuple, torch.tensor, lambda t: torch.tensor(t, device=dev), lambda t: list(torch.tensor(t, device=dev)), lambda t: [torch.tensor(t[0]), *t[1:]], lambda t: torch.tensor(t).numpy()):
+        slots = [eng.acquire(), eng.acquire()]
+        out = [eng.step([Entry(slots[0], 0, form(toks[:5]), [1, 4]), Entry(slots[1], 0, form(toks[5:6]), [0])]).clone()]
+        out.append(eng.step([Entry(slots[0], 5, form(toks[5:6]), [0]), Entry(slots[1], 1, form(toks[6:]), [0])]).clone())
+        got.append(torch.cat(out))
+        for s in slots:
+            eng.release(s)
+    assert got[0].shape[0] == 5 and all(torch.equal(g, got[0]) for g in got[1:])
+
+
 @pytest.mark.parametrize("name,dtype,tol", [("mixed", torch.float32, 1e-4), ("mixed", torch.bfloat16, 0.12), ("all looped", torch.bfloat16, 0.12)])
 def test_portions_batches_slots_and_decoding(dev, name, dtype, tol):
     """Unequal requests in one batch, cut differently, decoded together, their slots used again: the logits of each alone."""
