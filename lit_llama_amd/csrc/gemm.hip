@@ -1107,7 +1107,7 @@ __device__ __forceinline__ void lds_touch(__amdgpu_buffer_rsrc_t r, char* lds, u
 // their own.
 // ONCE: one token block (BM tokens at most) and weights that come from HBM (MI355_LF_STREAMED), so nothing reads a piece of them again: they are requested non-temporal and push no activations
 // out of the L2 caches.  BF16, 16 products of 2048 to 32000 rows, weights in no cache: 16 tokens 0.89 times as long (0.86 to 0.94; N = 4096, K = 16512 30.9 -> 26.8 us, N = 32000, K = 4096 52.0 ->
-// 46.0), 24 tokens 0.91, 40 0.93, 64 0.95 (two of 16 up to 1.01).  Int4 of one scale per row, which its own work bounds, the same either way; groups of 128 columns, 16 and 24 tokens, 0.95.
+// 46.0), 24 tokens 0.91, 40 0.93, 64 0.95 (two of 16 up to 1.01).  Int4 of one scale per row, nine products, 600 MB of copies, 16 / 32 / 37 / 48 tokens 0.92 / 0.93 / 0.94 / 0.95, groups of 128 columns 0.92 / 0.95 / 0.96 / 0.98.
 // Weights that a cache holds it costs: ten BF16 products of 1024 to 8192 rows, all copies read in turn 100 / 200 / 256 / 288 / 320 / 352 / 600 MB, 16 tokens 1.07 / 1.08 / 1.05 / 1.02 / 0.97 / 0.95 / 0.92 times
 // as long (100 MB: N = 6144, K = 2048 1.28), one copy again and again 1.12 (1.54).
 template <int EPI, bool PAIR, int FMT, int kWaves, int BM, bool FUSE, int DEPTH, int GRP = 0, bool RUNS = false, int TPW = kTPW, bool ONCE = false>
@@ -1687,7 +1687,7 @@ int launch_deep(const GemmParams& p, hipStream_t s) {
     if constexpr (FMT == MI355_W_Q4 && GRP == 0 && BM <= 64 && !RUNS) {
         if (p.runs > 1) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, true>(p, s);
     }
-    if constexpr (!ONCE && ((FMT == MI355_W_BF16 && BM <= 64) || (GRP == 1 && BM <= 48))) {
+    if constexpr (!ONCE && (FMT == MI355_W_BF16 ? BM <= 64 : BM <= 48 && (GRP == 1 || BM >= 32))) {  // (int4 of one scale per row: fewer than 32 tokens are multiplied unit by unit, GRP 1)
         if (p.streamed && p.M <= BM) return launch_deep<EPI, PAIR, FMT, kWaves, BM, FUSE, GRP, TPW, RUNS, true>(p, s);
     }
     constexpr int kDepth = BM > 192 ? 2 : BM > kBM || (BM >= 96 && FMT == MI355_W_BF16) ? 3 : 4;

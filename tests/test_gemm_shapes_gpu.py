@@ -417,8 +417,8 @@ def test_few_bf16_rows_in_slices_of_2_and_3_units(dev, N, K, M, epi):
     test_few_bf16_rows_in_blocks_of_2_to_4_waves(dev, N, K, M, epi, flags=nat.LF_STREAMED)
 
 
-@pytest.mark.parametrize("M", [2, 16, 24, 40, 48, 49, 64, 65])
-@pytest.mark.parametrize("N,K,fmt", [(128, 640, "bf16"), (33024, 384, "bf16"), (70000, 128, "bf16"), (4096, 4096, "bf16"), (640, 1024, "g128"), (4096, 1152, "q4")])
+@pytest.mark.parametrize("M", [2, 16, 24, 32, 40, 48, 49, 64, 65])
+@pytest.mark.parametrize("N,K,fmt", [(128, 640, "bf16"), (33024, 384, "bf16"), (70000, 128, "bf16"), (4096, 4096, "bf16"), (640, 1024, "g128"), (4096, 1152, "q4"), (1000, 4096, "q4")])
 def test_weights_past_the_caches_or_through_them(dev, N, K, fmt, M):
     """Weights requested non-temporal (one token block) or not, of 2 to 8 waves: f32 sums of exact products (see test_tiled_product_against_64_bits), the same bits where the cut is the same."""
     g = torch.Generator(device=dev).manual_seed(M + N)
