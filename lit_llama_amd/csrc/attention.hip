@@ -815,7 +815,8 @@ extern "C" int mi355_attention(const mi355_attn_args* a, mi355_stream_t stream) 
         b.ldy = a->ldy;
         return mi355_adapter_prefix(&b, stream);
     }
-    // Tokens that share their keys, where attn_kernel's workgroup per (head, token) no longer has a CU to itself (up to there 32 heads of 128, 8 tokens 7.6 us, shared 8.0; past it 12 tokens 11.2 / 8.7)
+    // Tokens that share their keys, where attn_kernel's workgroup per (head, token) no longer has a CU to itself (up to there 32 heads of 128, 8 tokens 7.6 us, shared 8.0; past it 12 tokens 11.2 / 8.7).
+    // A tile that holds few tokens is no worse: 661 launches past it, heads of 64 and 128, batches of 1 to 128, 2 to 31 tokens behind none to 3000, took 0.05 to 0.84 times as long
     if (esz == 2 && (a->hs == 64 || a->hs == 128) && a->qkv_dtype == MI355_F32 && a->n_split <= 1 && !adapter && !p.fused && (int64_t)a->n_head * a->T * a->B > 256 &&
         ((uintptr_t)p.kcache | (uintptr_t)p.vcache) % 16 == 0 && a->debug_stamps == nullptr) {
         hipLaunchKernelGGL(a->hs == 64 ? attn_tile_kernel<64> : attn_tile_kernel<128>, dim3(a->n_head, (a->T + kTileTokens - 1) / kTileTokens, a->B), dim3(64 * kTileWaves), 0, s, p);
