@@ -603,7 +603,7 @@ class HybridEngine:
             if e.pos + len(e.tokens) > self.max_len:
                 raise nat.NativeError(f"hybrid engine: position {e.pos + len(e.tokens) - 1} is outside the cache of {self.max_len}")
             if len(e.tokens) == 1 and len(e.want) <= 1 and room > 0 and wants > 0 and 0 <= e.tokens[0] < self.cfg.vocab_size:  # (a decode step's: as below, without its searches)
-                cur.append(e if len(e.want) == 0 or e.want[0] == 0 else Entry(e.slot, e.pos, e.tokens, []))
+                cur.append(e if len(e.want) == 0 or 0 in e.want else Entry(e.slot, e.pos, e.tokens, []))
                 room, wants = room - 1, wants - len(cur[-1].want)
                 continue
             if min(e.tokens, default=0) < 0 or max(e.tokens, default=0) >= self.cfg.vocab_size:

@@ -685,6 +685,19 @@ def test_bf16_blocks_of_160_and_208_tokens_are_whole_rows():
     assert [_gemm_cut(M, N, K, 1, False)[1] for M, N, K in ((777, 12288, 4096), (777, 15360, 5120), (2048, 12416, 4096))] == [160, 208, 208]
 
 
+@pytest.mark.parametrize("form", [list, tuple, set, frozenset, torch.tensor, lambda w: {k: None for k in w}.keys()])
+def test_a_steps_wanted_places_in_any_form(form):
+    """One token, whose places go by a shorter way, as several: what is asked for outside a portion is left out."""
+    from types import SimpleNamespace
+
+    from lit_llama_amd.hybrid_engine import Entry, HybridEngine
+
+    eng = SimpleNamespace(max_rows=8, max_logits_rows=8, max_len=64, cfg=SimpleNamespace(vocab_size=10))
+    for tokens, want, left in (([5], [0], [0]), ([5], [], []), ([5], [1], []), ([5], [-1], []), ([5, 6, 7], [0, 2], [0, 2]), ([5, 6], [1], [1])):
+        (e,), = HybridEngine._cut(eng, [Entry(3, 4, tokens, form(want))])
+        assert (e.slot, e.pos, e.tokens, [int(k) for k in e.want]) == (3, 4, tokens, left)
+
+
 def test_weights_are_streamed_from_what_the_cache_does_not_hold():
     assert [nat.streamed(n) for n in (0, 7_000_000, 300_000_000, 300_000_001, 13_000_000_000)] == [0, 0, 0, nat.LF_STREAMED, nat.LF_STREAMED]
 
