@@ -428,7 +428,7 @@ int linear(const mi355_hybrid_model* m, const mi355_proj& w, const void* x, int6
     a.norm_dtype = m->norm_dtype;
     a.eps = m->eps;
     a.epi = what == kResidual ? MI355_EPI_ACCUM : what == kGeglu ? MI355_EPI_GEGLU : MI355_EPI_STORE;
-    a.flags = (what == kRelu2 ? MI355_LF_RELU2 : 0) | (m->norm_add != 0.f ? MI355_LF_NORM_ONE : 0) | m->linear_flags;
+    a.flags = (what == kRelu2 ? MI355_LF_RELU2 : 0) | (m->norm_add != 0.f ? MI355_LF_NORM_ONE : 0) | (m->linear_flags & MI355_LF_STREAMED);
     a.alpha = what == kResidual ? m->residual_mult : what == kLogits ? m->logit_scale : 1.f;
     a.y_dtype = y_dtype;
     a.ldy = ldy;
@@ -678,7 +678,7 @@ int mi355_product_run(const mi355_product& p, const mi355_proj& w, hipStream_t s
     a.ldy = p.ldy;
     a.slice_rows = p.slice_rows;
     a.slice_stride = p.slice_stride;
-    a.flags = p.flags;
+    a.flags = p.flags & MI355_LF_STREAMED;  // (callers of mi355_latent_attention may have left its word, reserved before, as it was)
     MI355_CHECK_ARG(p.ldx >= a.K && p.ldx % 8 == 0, MI355_E_SHAPE, "product: rows of pitch %lld hold no operand of %d columns", (long long)p.ldx, a.K);
     if (p.slice_rows != 0 || mi355_product_wide(w, p.M, a.R)) return mi355_linear_gemm(&a, p.ws, (size_t)p.ws_bytes, s);
     return mi355_linear_fast(&a, s);

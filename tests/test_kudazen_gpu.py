@@ -521,6 +521,23 @@ def test_a_step_larger_than_the_scratch_is_cut(dev, dtype):
     assert close(out, ref, dtype)
 
 
+def test_bits_of_the_products_flags_that_are_not_theirs(dev):
+    """Of a model's word for its products LF_STREAMED alone is read: a caller may have left the rest as it was."""
+    from lit_llama_amd import _native as nat
+    from lit_llama_amd.hybrid_engine import Entry
+
+    config = CONFIGS["whole tiles"]
+    eng = build(config, torch.bfloat16, dev)[0].engine()
+    eng.ensure(1, 128)
+    toks, got = tokens_of(61, config["vocab"]), []
+    for flags in (0, ~nat.LF_STREAMED):
+        eng.m.linear_flags = flags
+        s = eng.acquire()
+        got.append(torch.cat([eng.step([Entry(s, at, toks[at:to], range(to - at))]).clone() for at, to in ((0, 40), (40, 60), (60, 61))]))
+        eng.release(s)
+    assert torch.equal(*got)
+
+
 def greedy_reference(config, sd, prompt, n, margin):
     """Greedy continuation by the oracle, up to the first near tie."""
     seq = list(prompt)
