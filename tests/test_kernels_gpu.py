@@ -491,18 +491,18 @@ def test_split_attention_equals_single_workgroup_and_feeds_the_projection(dev, n
     assert (got - ref).abs().max().item() <= 5e-3 * _rms(ref)
 
 
-@pytest.mark.parametrize("H,hs,T,first,S,B,out", [
+SHARED_KEYS = [
     (52, 128, 5, 0, 64, 1, torch.float32), (32, 128, 9, 300, 400, 1, torch.float32), (32, 128, 31, 0, 31, 1, torch.bfloat16), (24, 128, 17, 40, 50, 1, torch.float32),
     (4, 64, 65, 0, 80, 1, torch.float32), (5, 64, 129, 7, 200, 1, torch.float32), (2, 64, 700, 0, 700, 1, torch.float32), (3, 64, 100, 30, 97, 1, torch.float32),
     (4, 64, 48, 0, 48, 3, torch.float32), (6, 128, 33, 5, 60, 2, torch.float32),
-])
-@pytest.mark.parametrize("odd", ["", "value", "values", "key"])
+]
+
+
+@pytest.mark.parametrize("H,hs,T,first,S,B,out,odd", [(*c, odd) for odd in ("", "value", "values", "key") for c in SHARED_KEYS if odd in ("", "value") or c[3] > 0])  # (rows of earlier calls)
 def test_attention_of_tokens_that_share_their_keys(dev, H, hs, T, first, S, B, out, odd):
     """More (head, token) pairs than CUs, f32 queries over a bf16 cache, against 64 bits: positions in any order, past the cache's end (the last row), several batch rows; an infinite value in the
     last row, which only those that see it take over; infinite values that all see, of one sign in a dimension and of both in another; an infinite key, whose weight is 0 or NaN.  f32 sums of up to
     2048 terms and exponentials of |score| < 20: 1e-6 of the result; bf16 results 2^-8.  Infinities and NaN are where 64 bits have them."""
-    if odd in ("values", "key") and first == 0:
-        pytest.skip("no rows of earlier calls")
     g = torch.Generator().manual_seed(T)
     qkv = torch.randn((B, T, 3 * H * hs), generator=g)
     rope = oracle.build_rope_cache(1024, hs, dtype=torch.int64)
